@@ -40,7 +40,7 @@ const char* nd_app_name(int index);
  * with every change of the engine's interface, combined with the sizes of the structs the two
  * sides share, so that a forgotten raise is caught as well.  nd_engine_abi() is the library's own
  * value.  Returns 0, or a negative value (-2 ABI mismatch, -3 name taken). */
-#define ND_ENGINE_ABI 3
+#define ND_ENGINE_ABI 4
 int nd_engine_abi(void);
 int nd_register_app(const char* name, void* (*make)(const char* name), int engine_abi);
 
@@ -94,9 +94,8 @@ int nd_sampler_do_sample_parallel(nd_sampler* s);
  * The samples do not depend on the period.  Apps other than walks always invert. */
 int nd_sampler_set_inversion_period(nd_sampler* s, int period);
 /* getFinalSamples(data), src/nextdoor.cu:3211-3237: copies device -> host and returns the
- * host array (num_samples * final_sample_size int32, INVALID = n_vertices).  The array is
- * page-locked memory of the library's (the copy runs at the bus rate: 57 GB/s measured for
- * 1.68 GB, against 18 GB/s into pageable memory). */
+ * host array (num_samples * final_sample_size int32, INVALID = n_vertices).  More than a few
+ * megabytes cross the bus packed and are unpacked by up to eight host threads on the way. */
 int nd_sampler_get_final_samples(nd_sampler* s, const int32_t** data, int64_t* length);
 /* getFinalSampleSize<App>(), src/nextdoor.cu:1913-1929. */
 int nd_sampler_final_sample_size(const nd_sampler* s);
@@ -116,6 +115,16 @@ int nd_sampler_sampling_type(const nd_sampler* s);
  * SampleType structs.  nd_sampler_sample_state_bytes is 0 for an empty SampleType. */
 int64_t nd_sampler_sample_state_bytes(const nd_sampler* s);
 int nd_sampler_get_sample_states(nd_sampler* s, void* dst, int64_t bytes);
+/* The same into an array of the library's. */
+int nd_sampler_fetch_sample_states(nd_sampler* s, const void** data, int64_t* bytes);
+/* No counterpart in the reference.  Makes the array at `data` - final samples, rows or columns
+ * of the edge lists, or sample states, as the last call for them returned it - the caller's: the
+ * library neither writes to it nor frees it any more, and the next call for the same result
+ * returns another array.  *owner stands for it until nd_release_array(owner), after which its
+ * memory is used for a later result of the same sampler, or freed if that is gone.  Instead of
+ * a copy, for callers that keep what they are given. */
+int nd_sampler_detach_array(nd_sampler* s, const void* data, void** owner);
+void nd_release_array(void* owner);
 /* No counterpart in the reference (whose step loop waits for the host several times per step,
  * src/nextdoor.cu:2498-2636).  A pass here is a fixed sequence of launches with all varying
  * sizes in device memory, so it can be recorded once as a HIP graph and replayed: mode 1 on,

@@ -75,6 +75,21 @@ def _ptr(arr, ctype):
     return arr.ctypes.data_as(C.POINTER(ctype))
 
 
+class _Lease:
+    """Host memory of the library's that a numpy array stands on; given back with the array."""
+
+    def __init__(self, sampler_handle, address, shape, typestr):
+        owner = C.c_void_p()
+        check(lib().nd_sampler_detach_array(sampler_handle, address, C.byref(owner)))
+        self._release, self._owner = lib().nd_release_array, owner
+        self.__array_interface__ = {"version": 3, "data": (address, False), "shape": shape, "typestr": typestr}
+
+    def __del__(self):
+        owner, self._owner = getattr(self, "_owner", None), None
+        if owner:
+            self._release(owner)
+
+
 class Graph:
     """Host CSR graph (the reference's ``CSR*``)."""
 
@@ -225,8 +240,11 @@ class Sampler:
         """(num_samples, final_sample_size) int32 array; INVALID entries equal n_vertices."""
         p, n = C.POINTER(C.c_int32)(), C.c_int64()
         check(lib().nd_sampler_get_final_samples(self._h, C.byref(p), C.byref(n)))
-        flat = np.ctypeslib.as_array(p, shape=(n.value,)).copy()
-        return flat.reshape(self.num_samples, self.final_sample_size)
+        return self._own(p, (self.num_samples, self.final_sample_size), "<i4")
+
+    def _own(self, pointer, shape, typestr):
+        """The array a fetch has just returned, as the caller's own (no copy)."""
+        return np.asarray(_Lease(self._h, C.cast(pointer, C.c_void_p).value, shape, typestr))
 
     def adjacency(self):
         """Edge lists of the apps with AdjacencyMatrix output on per-transit sampling (MVS,
@@ -236,9 +254,8 @@ class Sampler:
         n_edges, n_samples = C.c_int64(), C.c_int64()
         check(lib().nd_sampler_get_adjacency(self._h, C.byref(rows), C.byref(cols), C.byref(n_edges), C.byref(start),
                                              C.byref(n_samples)))
-        take = lambda p, n, dt: (np.ctypeslib.as_array(p, shape=(n,)).copy() if n else np.zeros(0, dtype=dt))
-        return (take(rows, n_edges.value, np.int32), take(cols, n_edges.value, np.int32),
-                take(start, n_samples.value + 1, np.uint32))
+        take = lambda p: self._own(p, (n_edges.value,), "<i4") if n_edges.value else np.zeros(0, dtype=np.int32)
+        return take(rows), take(cols), np.ctypeslib.as_array(start, shape=(n_samples.value + 1,)).copy()
 
     def distinct(self):
         """Distinct post-pass on the device rows; returns counts[num_samples, steps]."""
@@ -248,12 +265,11 @@ class Sampler:
         return np.ctypeslib.as_array(p, shape=(n.value,)).copy().reshape(self.num_samples, self.steps)
 
     def sample_states(self):
-        nbytes = lib().nd_sampler_sample_state_bytes(self._h)
-        if nbytes <= 0:
+        if lib().nd_sampler_sample_state_bytes(self._h) <= 0:
             return None
-        buf = np.empty(nbytes, dtype=np.uint8)
-        check(lib().nd_sampler_get_sample_states(self._h, buf.ctypes.data_as(C.c_void_p), nbytes))
-        return buf
+        p, n = C.c_void_p(), C.c_int64()
+        check(lib().nd_sampler_fetch_sample_states(self._h, C.byref(p), C.byref(n)))
+        return self._own(p, (n.value,), "|u1")
 
     def set_inversion_period(self, period):
         """Walks: 1 inverts before every step (the reference's behaviour, default); p > 1 keeps

@@ -50,6 +50,9 @@ SIGNATURES = {
     "nd_sampler_sampling_type": (C.c_int, [C.c_void_p]),
     "nd_sampler_sample_state_bytes": (C.c_int64, [C.c_void_p]),
     "nd_sampler_get_sample_states": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int64]),
+    "nd_sampler_fetch_sample_states": (C.c_int, [C.c_void_p, C.POINTER(C.c_void_p), c_i64p]),
+    "nd_sampler_detach_array": (C.c_int, [C.c_void_p, C.c_void_p, C.POINTER(C.c_void_p)]),
+    "nd_release_array": (None, [C.c_void_p]),
     "nd_sampler_set_inversion_period": (C.c_int, [C.c_void_p, C.c_int]),
     "nd_sampler_set_launch_graph": (C.c_int, [C.c_void_p, C.c_int]),
     "nd_sampler_set_profiling": (C.c_int, [C.c_void_p, C.c_int]),

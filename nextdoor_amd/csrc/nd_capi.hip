@@ -443,6 +443,38 @@ int nd_sampler_get_sample_states(nd_sampler* s, void* dst, int64_t bytes) {
   });
 }
 
+int nd_sampler_fetch_sample_states(nd_sampler* s, const void** data, int64_t* bytes) {
+  return guarded([&]() -> int {
+    if (!s || !data || !bytes) return fail("null argument");
+    nd::EngineBase& e = *s->engine;
+    const size_t n = e.sample_state_bytes();
+    if (n == 0) return fail("no sample state");
+    e.hSampleStates.resize(n);
+    const int rc = e.fetch_sample_states(e.hSampleStates.data(), n);
+    if (rc != 0) return fail(e.last_error, rc);
+    *data = e.hSampleStates.data();
+    *bytes = (int64_t)n;
+    return 0;
+  });
+}
+
+int nd_sampler_detach_array(nd_sampler* s, const void* data, void** owner) {
+  return guarded([&]() -> int {
+    if (!s || !data || !owner) return fail("null argument");
+    nd::EngineBase& e = *s->engine;
+    nd::HostLease* lease = nullptr;
+    if (data == e.hFinalSamples.data()) lease = e.hFinalSamples.detach();
+    else if (data == e.hListRows.data()) lease = e.hListRows.detach();
+    else if (data == e.hListCols.data()) lease = e.hListCols.detach();
+    else if (data == e.hSampleStates.data()) lease = e.hSampleStates.detach();
+    if (!lease) return fail("not an array of this sampler");
+    *owner = lease;
+    return 0;
+  });
+}
+
+void nd_release_array(void* owner) { delete (nd::HostLease*)owner; }
+
 int nd_sampler_set_inversion_period(nd_sampler* s, int period) {
   if (!s) return fail("null sampler");
   if (period < 0) return fail("the inversion period is 0 (engine decides) or positive");
@@ -575,7 +607,9 @@ int nd_sampler_check_results(nd_sampler* s, int* ok) {
 }
 
 void nd_sampler_free_device(nd_sampler* s) {
-  if (s) s->engine->free_device();
+  if (!s) return;
+  s->engine->free_device();
+  s->engine->result_stream.release();
 }
 
 void nd_sampler_destroy(nd_sampler* s) { delete s; }

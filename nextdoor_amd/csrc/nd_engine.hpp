@@ -41,6 +41,7 @@
 #include "nd_contract.hpp"
 #include "nd_device_graph.hpp"
 #include "nd_distinct.hpp"
+#include "nd_host_results.hpp"
 #include "nd_radix_sort.hpp"
 #include "nd_transit_runs.hpp"
 
@@ -63,54 +64,6 @@ struct PhaseTimes {  // milliseconds, accumulated over one sample() call when pr
   int neighborhood_launches = 0;
 };
 
-// Host array the device copies results into.  Page-locked (hipHostMalloc) when a device is
-// there: the copy of 1.68 GB of walks takes 94 ms into pageable memory (17.8 GB/s) and about a
-// third of that into page-locked memory.  Falls back to ordinary memory (no device, or the
-// driver refuses).
-template <class T>
-class HostArray {
- public:
-  HostArray() = default;
-  HostArray(const HostArray&) = delete;
-  HostArray& operator=(const HostArray&) = delete;
-  ~HostArray() { clear(); }
-  T* data() { return data_; }
-  const T* data() const { return data_; }
-  size_t size() const { return size_; }
-  bool empty() const { return size_ == 0; }
-  // n elements, every one `value`
-  void assign(size_t n, T value) {
-    if (n != size_) {
-      clear();
-      if (n) {
-        void* p = nullptr;
-        if (hipHostMalloc(&p, n * sizeof(T), hipHostMallocDefault) == hipSuccess && p) {
-          pinned_ = true;
-        } else {
-          (void)hipGetLastError();  // the refusal is not an error of a later call
-          p = malloc(n * sizeof(T));
-          pinned_ = false;
-        }
-        data_ = (T*)p;
-        size_ = data_ ? n : 0;
-      }
-    }
-    std::fill_n(data_, size_, value);
-  }
-  void clear() {
-    if (data_) {
-      if (pinned_) (void)hipHostFree(data_); else free(data_);
-    }
-    data_ = nullptr;
-    size_ = 0;
-  }
-
- private:
-  T* data_ = nullptr;
-  size_t size_ = 0;
-  bool pinned_ = false;
-};
-
 // Roots index the row extents in the kernels: each must be a vertex, or the "no vertex" value
 // (the number of vertices).  The reference does not check (a root outside the graph reads past
 // its arrays there).
@@ -122,7 +75,7 @@ inline bool roots_are_vertices(const std::vector<VertexID_t>& roots, int32_t n_v
 
 class EngineBase {
  public:
-  virtual ~EngineBase() {}
+  virtual ~EngineBase() { host_pool->close(); }
   virtual const char* app_name() const = 0;
   virtual int set_graph(const CSR* graph) = 0;
   virtual int alloc(uint64_t seed) = 0;
@@ -162,13 +115,31 @@ class EngineBase {
     return -2;
   }
 
-  HostArray<VertexID_t> hFinalSamples;         // as NextDoorData::hFinalSamples (libNextDoor.hpp:17)
+  // Host memory of the results, and the way they take to it (nd_host_results.hpp)
+  const std::shared_ptr<HostPool> host_pool = std::make_shared<HostPool>();
+  ResultStream result_stream;
+  // Device memory to the host, complete on return.  bits, fill: what is known of its words (ResultStream::fetch).
+  int fetch_to_host(void* dst, const void* src, size_t bytes, uint32_t bits, int32_t fill, hipStream_t stream) {
+    hipError_t e;
+    if (bytes > kDirectResultBytes && bytes % sizeof(int32_t) == 0) {
+      e = result_stream.fetch((const int32_t*)src, bytes / sizeof(int32_t), bits, fill, (int32_t*)dst, stream);
+    } else {
+      e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream);
+      if (e == hipSuccess) e = hipStreamSynchronize(stream);
+    }
+    if (e == hipSuccess) return 0;
+    last_error = std::string("results to the host: ") + hipGetErrorString(e);
+    return -1;
+  }
+
+  HostArray<VertexID_t> hFinalSamples{host_pool};  // as NextDoorData::hFinalSamples (libNextDoor.hpp:17)
+  HostArray<unsigned char> hSampleStates{host_pool};
   std::vector<VertexID_t> initialContents;     // as NextDoorData::initialContents (libNextDoor.hpp:18)
   std::vector<int32_t> hDistinctCounts;        // [num_samples * steps] ids kept by distinct()
   // edge lists of all samples, packed in sample order: sample s owns entries
   // [hListStart[s], hListStart[s + 1]) of hListRows / hListCols
   std::vector<uint32_t> hListStart;
-  std::vector<VertexID_t> hListRows, hListCols;
+  HostArray<VertexID_t> hListRows{host_pool}, hListCols{host_pool};
   std::string last_error;
   bool profiling = false;
   PhaseTimes times;
@@ -2379,13 +2350,16 @@ class Engine : public EngineBase {
   }
 
   // getFinalSamples: device -> hFinalSamples
-  int fetch_final_samples() override { return fetch_final_samples_into(hFinalSamples.data()); }
+  int fetch_final_samples() override {
+    if (!allocated_) { last_error = "no device data"; return -1; }
+    hFinalSamples.resize((size_t)n_samples_ * (size_t)final_sample_size());
+    return fetch_final_samples_into(hFinalSamples.data());
+  }
 
   int fetch_final_samples_into(VertexID_t* dst) {
     if (!allocated_) { last_error = "no device data"; return -1; }
-    ND_HIP_TRY(hipMemcpy(dst, d_final_, sizeof(VertexID_t) * (size_t)n_samples_ * (size_t)final_sample_size(),
-                         hipMemcpyDeviceToHost));
-    return 0;
+    return fetch_to_host(dst, d_final_, sizeof(VertexID_t) * (size_t)n_samples_ * (size_t)final_sample_size(),
+                         (uint32_t)max_bits_, invalid_, stream_);
   }
 
   bool is_walk() const { return walk_mode_; }
@@ -2393,8 +2367,7 @@ class Engine : public EngineBase {
   int fetch_sample_states(void* dst, size_t bytes) override {
     if (!allocated_ || std::is_empty<SampleType>::value) { last_error = "no sample state"; return -1; }
     if (bytes != sample_state_bytes()) { last_error = "sample state size mismatch"; return -1; }
-    ND_HIP_TRY(hipMemcpy(dst, d_samples_, bytes, hipMemcpyDeviceToHost));
-    return 0;
+    return fetch_to_host(dst, d_samples_, bytes, 32, 0, stream_);
   }
 
   // Distinct post-pass over the device-resident result rows (see nd_distinct.hpp): every

@@ -1448,16 +1448,15 @@ class LayerEngine : public EngineBase {
 
   int fetch_final_samples() override {
     if (!allocated_) { last_error = "no device data"; return -1; }
-    ND_HIP_TRY(hipMemcpy(hFinalSamples.data(), d_final_, sizeof(VertexID_t) * hFinalSamples.size(),
-                         hipMemcpyDeviceToHost));
-    return 0;
+    hFinalSamples.resize((size_t)n_samples_ * (size_t)final_sample_size());
+    return fetch_to_host(hFinalSamples.data(), d_final_, sizeof(VertexID_t) * hFinalSamples.size(), (uint32_t)max_bits(),
+                         invalid_, stream_);
   }
 
   int fetch_sample_states(void* dst, size_t bytes) override {
     if (!allocated_ || std::is_empty<SampleType>::value) { last_error = "no sample state"; return -1; }
     if (bytes != sample_state_bytes()) { last_error = "sample state size mismatch"; return -1; }
-    ND_HIP_TRY(hipMemcpy(dst, d_samples_, bytes, hipMemcpyDeviceToHost));
-    return 0;
+    return fetch_to_host(dst, d_samples_, bytes, 32, 0, stream_);
   }
 
   int distinct() override {

@@ -123,6 +123,7 @@ class ShardedEngine : public EngineBase {
 
   int fetch_final_samples() override {
     size_t at = 0;
+    if (num_samples() > 0) hFinalSamples.resize((size_t)num_samples() * (size_t)final_sample_size());
     for (size_t i = 0; i < parts_.size(); ++i) {
       if (parts_[i]->fetch_final_samples_into(hFinalSamples.data() + at) != 0) return fail((int)i);
       at += (size_t)parts_[i]->num_samples() * (size_t)final_sample_size();

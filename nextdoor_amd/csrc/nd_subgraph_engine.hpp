@@ -437,16 +437,15 @@ class SubgraphEngine : public EngineBase {
 
   int fetch_final_samples() override {
     if (!allocated_) { last_error = "no device data"; return -1; }
-    ND_HIP_TRY(hipMemcpy(hFinalSamples.data(), d_final_, sizeof(VertexID_t) * hFinalSamples.size(),
-                         hipMemcpyDeviceToHost));
-    return 0;
+    hFinalSamples.resize((size_t)n_samples_ * (size_t)final_sample_size());
+    return fetch_to_host(hFinalSamples.data(), d_final_, sizeof(VertexID_t) * hFinalSamples.size(), (uint32_t)max_bits_,
+                         invalid_, stream_);
   }
 
   int fetch_sample_states(void* dst, size_t bytes) override {
     if (!allocated_) { last_error = "no device data"; return -1; }
     if (bytes != sample_state_bytes()) { last_error = "sample state buffer has the wrong size"; return -2; }
-    ND_HIP_TRY(hipMemcpy(dst, d_stored_, bytes, hipMemcpyDeviceToHost));
-    return 0;
+    return fetch_to_host(dst, d_stored_, bytes, 32, 0, stream_);
   }
 
   bool lists_edges() const override { return true; }
@@ -457,11 +456,10 @@ class SubgraphEngine : public EngineBase {
     hListRows.resize((size_t)n_edges_listed_);
     hListCols.resize((size_t)n_edges_listed_);
     ND_HIP_TRY(hipMemcpy(hListStart.data(), d_list_start_, sizeof(uint32_t) * hListStart.size(), hipMemcpyDeviceToHost));
-    if (n_edges_listed_ > 0) {
-      ND_HIP_TRY(hipMemcpy(hListRows.data(), d_rows_, sizeof(VertexID_t) * hListRows.size(), hipMemcpyDeviceToHost));
-      ND_HIP_TRY(hipMemcpy(hListCols.data(), d_cols_, sizeof(VertexID_t) * hListCols.size(), hipMemcpyDeviceToHost));
-    }
-    return 0;
+    if (n_edges_listed_ == 0) return 0;
+    const size_t bytes = sizeof(VertexID_t) * (size_t)n_edges_listed_;
+    const int rc = fetch_to_host(hListRows.data(), d_rows_, bytes, (uint32_t)max_bits_, invalid_, stream_);
+    return rc != 0 ? rc : fetch_to_host(hListCols.data(), d_cols_, bytes, (uint32_t)max_bits_, invalid_, stream_);
   }
 
   int distinct() override {

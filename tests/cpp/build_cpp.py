@@ -16,6 +16,8 @@ HOST_PROBE_SRC = os.path.join(HERE, "host_api_probe.cpp")
 HOST_PROBE = os.path.join(HERE, "host_api_probe")
 TEMPLATE_PROBE_SRC = os.path.join(HERE, "template_api_probe.hip")
 TEMPLATE_PROBE = os.path.join(HERE, "template_api_probe")
+RESULT_PROBE_SRC = os.path.join(HERE, "result_stream_probe.hip")
+RESULT_PROBE = os.path.join(HERE, "result_stream_probe")
 USER_APPS_SRC = os.path.join(HERE, "user_apps.hip")
 USER_APPS_LIB = os.path.join(HERE, "libuser_apps.so")
 
@@ -55,13 +57,18 @@ def build_template_probe():
     return TEMPLATE_PROBE
 
 
+def build_result_probe():
+    _run(_hipcc_flags() + [RESULT_PROBE_SRC, "-o", RESULT_PROBE, "-lpthread"])
+    return RESULT_PROBE
+
+
 def build_user_apps():
     _run(_hipcc_flags() + ["-shared", USER_APPS_SRC, "-o", USER_APPS_LIB] + _link_flags())
     return USER_APPS_LIB
 
 
 def build_all():
-    return [build_host_probe(), build_template_probe(), build_user_apps()]
+    return [build_host_probe(), build_template_probe(), build_result_probe(), build_user_apps()]
 
 
 if __name__ == "__main__":

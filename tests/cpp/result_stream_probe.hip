@@ -1,0 +1,46 @@
+// Results brought to the host by ResultStream (nd_host_results.hpp), against the words that were put on the device:
+// every width, sizes around a group, a chunk and a piece, dead groups, ids that do not fit their width, targets that
+// are no multiple of 32 bytes.  Prints the case before it runs, "all equal" at the end.
+#include "../../nextdoor_amd/csrc/nd_host_results.hpp"
+
+#include <stdio.h>
+
+#define TRY(expr)                                                              \
+  do {                                                                         \
+    hipError_t e_ = (expr);                                                    \
+    if (e_ != hipSuccess) { printf("%s\n", hipGetErrorString(e_)); return 1; } \
+  } while (0)
+
+int main() {
+  const size_t piece = (size_t)64 * nd::kPackChunk;  // the smallest piece
+  const size_t sizes[] = {1, 7, 8, 9, nd::kPackChunk - 1, nd::kPackChunk, nd::kPackChunk + 1, piece, piece + 9, 13 * piece + 4097};
+  nd::ResultStream stream;
+  for (size_t n : sizes) {
+    int32_t* d = nullptr;
+    TRY(hipMalloc(&d, n * sizeof(int32_t)));
+    for (uint32_t bits : {1u, 2u, 7u, 8u, 9u, 12u, 16u, 17u, 23u, 24u, 25u, 26u, 31u, 32u}) {
+      if (n > piece + 9 && bits != 12 && bits != 23 && bits != 32) continue;
+      for (int misfit = 0; misfit < 2; ++misfit) {
+        printf("n %zu bits %u misfit %d\n", n, bits, misfit);
+        fflush(stdout);
+        const uint32_t mask = bits == 32 ? 0xffffffffu : (1u << bits) - 1u;
+        const int32_t fill = (int32_t)mask;
+        std::vector<int32_t> want(n), got(n + 2, 77);
+        for (size_t i = 0; i < n; ++i)
+          want[i] = (i / 11) % 3 == 0 || (i / 700) % 4 == 1 ? fill : (int32_t)(((uint32_t)i * 2654435761u) & mask);
+        if (misfit) want[n / 2] = -5;
+        TRY(hipMemcpy(d, want.data(), n * sizeof(int32_t), hipMemcpyHostToDevice));
+        for (int shift = 0; shift < 2; ++shift) {
+          TRY(stream.fetch(d, n, bits, fill, got.data() + shift, nullptr));
+          if (memcmp(got.data() + shift, want.data(), n * sizeof(int32_t)) != 0 || got[n + 1] != 77) {
+            printf("differs at shift %d\n", shift);
+            return 1;
+          }
+        }
+      }
+    }
+    TRY(hipFree(d));
+  }
+  printf("all equal\n");
+  return 0;
+}
