@@ -272,9 +272,9 @@ class Sampler:
         return self._own(p, (n.value,), "|u1")
 
     def set_inversion_period(self, period):
-        """Walks: 1 inverts before every step (the reference's behaviour, default); p > 1 keeps
-        the walks out of transit order and only drops ended walks every p-th step; 0 lets the
-        engine decide.  The samples do not depend on it."""
+        """Walks: 1 inverts the (sample -> transit) map before every step, as the reference does; 0
+        (a new sampler's state) lets the engine decide, which keeps every walk on its lane; p > 1
+        does not invert either.  The samples do not depend on it."""
         check(lib().nd_sampler_set_inversion_period(self._h, int(period)))
 
     def set_launch_graph(self, mode):

@@ -50,6 +50,74 @@ __global__ void build_paired_edges(const CSR::Edge* col, const float* weight, si
   if (e < n) out[e] = EdgeRecord{col[e], weight[e]};
 }
 
+// An edge with what a walk needs of the vertex it leads to: one fetch per step instead of two dependent
+// ones (three, with the largest weight).  Aligned to its size, so that a record is never in two lines.
+struct alignas(16) WalkEdge {
+  VertexID dst;
+  EdgePos_t begin, n_edges;  // row extent of dst
+  float max_weight;          // and its largest weight
+};
+struct alignas(32) WeightedWalkEdge {
+  VertexID dst;
+  float weight;
+  EdgePos_t begin, n_edges;
+  float max_weight;
+  uint32_t unused[3];
+};
+
+// What a walk needs of the vertex it is at, in one 16-byte fetch.
+struct alignas(16) WalkVertex {
+  EdgePos_t begin, n_edges;
+  float max_weight;
+  uint32_t unused;
+};
+
+// The array views App::next() takes over such records.  `last` (the caller's register copy) holds the record
+// that was read last: most often the one of the vertex next() returns.
+template <class Record>
+struct WalkEdgeIds {
+  const Record* base;
+  Record* last;
+  __device__ __forceinline__ VertexID operator[](EdgePos_t i) const {
+    *last = base[i];
+    return last->dst;
+  }
+};
+struct WalkEdgeWeights {
+  const WeightedWalkEdge* base;
+  __device__ __forceinline__ float operator[](EdgePos_t i) const { return base[i].weight; }
+};
+
+__device__ __forceinline__ void set_weight_of(WalkEdge&, float) {}
+__device__ __forceinline__ void set_weight_of(WeightedWalkEdge& r, float weight) {
+  r.weight = weight;
+  r.unused[0] = r.unused[1] = r.unused[2] = 0;
+}
+
+template <class Record>
+__global__ void build_walk_edges(CSRPartition csr, Record* out) {
+  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= (size_t)csr.n_edges) return;
+  Record r;
+  r.dst = csr.edges[e];
+  r.begin = csr.row_ptr[r.dst];
+  r.n_edges = csr.row_ptr[r.dst + 1] - r.begin;
+  r.max_weight = csr.max_weights[r.dst];
+  set_weight_of(r, csr.weights[e]);
+  out[e] = r;
+}
+
+__global__ void build_walk_vertices(CSRPartition csr, WalkVertex* out) {
+  const size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (v >= (size_t)csr.n_vertices) return;
+  WalkVertex r;
+  r.begin = csr.row_ptr[v];
+  r.n_edges = csr.row_ptr[v + 1] - r.begin;
+  r.max_weight = csr.max_weights[v];
+  r.unused = 0;
+  out[v] = r;
+}
+
 class DeviceGraph {
  public:
   CSRPartition view{};
@@ -110,7 +178,37 @@ class DeviceGraph {
     return true;
   }
 
+  // The vertices as walk records, built when first asked for; nullptr: an error.
+  const WalkVertex* walk_vertices(hipStream_t stream) {
+    if (!walk_vertices_) {
+      if (hipMalloc(&walk_vertices_, sizeof(WalkVertex) * (size_t)view.n_vertices) != hipSuccess) return nullptr;
+      build_walk_vertices<<<dim3((unsigned)(((size_t)view.n_vertices + 255) / 256)), dim3(256), 0, stream>>>(view, walk_vertices_);
+      if (hipGetLastError() != hipSuccess || hipStreamSynchronize(stream) != hipSuccess) free_one(walk_vertices_);
+    }
+    return walk_vertices_;
+  }
+
+  // The edges as walk records, built when first asked for; nullptr where there is no memory for them.
+  template <class Record>
+  const Record* walk_edges(hipStream_t stream) {
+    if (walk_edges_ && walk_record_ != sizeof(Record)) free_one(walk_edges_);
+    if (!walk_edges_ && view.n_edges > 0) {
+      void* p = nullptr;
+      if (hipMalloc(&p, sizeof(Record) * (size_t)view.n_edges) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+      }
+      walk_edges_ = (char*)p;
+      walk_record_ = sizeof(Record);
+      build_walk_edges<Record><<<dim3((unsigned)(((size_t)view.n_edges + 255) / 256)), dim3(256), 0, stream>>>(view, (Record*)p);
+      if (hipGetLastError() != hipSuccess || hipStreamSynchronize(stream) != hipSuccess) free_one(walk_edges_);
+    }
+    return (const Record*)walk_edges_;
+  }
+
   void release() {
+    free_one(walk_edges_);
+    free_one(walk_vertices_);
     free_one(row_ptr_);
     free_one(col_);
     free_one(weight_);
@@ -138,6 +236,9 @@ class DeviceGraph {
   float* weight_ = nullptr;
   float* max_weight_ = nullptr;
   unsigned long long* edge_table_ = nullptr;
+  char* walk_edges_ = nullptr;
+  WalkVertex* walk_vertices_ = nullptr;
+  size_t walk_record_ = 0;
 };
 
 }  // namespace nd

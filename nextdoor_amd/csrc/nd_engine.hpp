@@ -80,12 +80,11 @@ class EngineBase {
   virtual int set_graph(const CSR* graph) = 0;
   virtual int alloc(uint64_t seed) = 0;
   virtual int sample(int mode) = 0;
-  // Walks: how often the (sample -> transit) map is inverted.  1: before every step, as the
-  // reference does.  p > 1: the walks are not brought into transit order at all; before step
-  // 1 and then every p-th step the walks that have ended are dropped from the list (a stable
-  // compaction in slot order), and there is no load balancing.  0: the engine decides from
-  // the walks-per-vertex ratio.  Results do not depend on it.  Other apps always invert.
-  int inversion_period = 1;
+  // Walks: whether the (sample -> transit) map is inverted.  1: before every step, as the
+  // reference does.  0 (default): the engine decides - it does not invert: over every graph
+  // and number of walks that was timed the order costs more than it saves (walk_rows_kernel).  p > 1: not inverted either.  Results do not depend on it.
+  // Other apps always invert.
+  int inversion_period = 0;
   // 1: replay a pass as a recorded HIP graph instead of enqueueing its launches one by one;
   // 0 (default): enqueue.  Layer-wise and edge-list apps have few, long launches and ignore it.
   int launch_graph = 0;
@@ -634,12 +633,6 @@ __device__ __forceinline__ void produce_groups_in_turn(const StepParams& P, CSRP
   }
 }
 
-// inversion_period == 0: walks are inverted before every step when there are at least this
-// many walks per vertex, else every kSparseInversionPeriod steps (measured on 4.2 M weighted
-// node2vec walks over 4.2 M vertices: 45.3 ms per 100 steps inverting every step, 38.0 every
-// 4th, 35.5 only once; the sorted order saves 3.4 ms in the step kernels and costs 13.7).
-constexpr double kWalksPerVertexForInversion = 4.0;
-constexpr int kSparseInversionPeriod = 32;
 
 // Lanes the flat kernel wants before it gives a lane all the outputs of a pair: enough to fill
 // the machine where the map is sorted by transit (neighbouring lanes then share their transit's
@@ -769,81 +762,253 @@ __global__ __launch_bounds__(kFlatThreads) void step_flat_kernel(StepParams P,
                                                      taken_stamp, stamp);
 }
 
-// Walks that are not re-inverted for a while: one lane keeps its walk for a whole stretch of
-// steps, with the current vertex and the sample state in registers.  Besides saving the
-// reads and writes of the pair list between steps, this evens out the rejection loops: a
-// wavefront waits for the SUM of its lanes' rounds over the stretch, not for the slowest
-// lane of every single step.  Step k of the stretch writes step_out[k * out_stride + slot].
-template <class SampleType, class App>
-__global__ __launch_bounds__(kFlatThreads) void walk_stretch_kernel(StepParams P, int stretch_steps, int last_step,
-                                                                    size_t out_stride) {
-  const uint32_t total = P.live_pairs ? *P.live_pairs : P.n_pairs;
-  const uint32_t i = blockIdx.x * kFlatThreads + threadIdx.x;
-  if (i >= total) return;
-  CSRPartition csr = P.csr;
-  VertexID transit = (VertexID)P.pair_keys[i];
-  const uint32_t slot = P.pair_slots ? P.pair_slots[i] : i;  // == the sample: one transit per sample
+// An App whose next() tries candidates until one is accepted may offer a single try as well
+// (kTriesOneCandidate): attempt() has next()'s arguments, whether this is the output's first
+// try, and where to put the result; it returns whether there is one.  next() is attempt()
+// until it does.
+template <class App, class = void>
+struct app_tries_one_candidate { static constexpr bool value = false; };
+template <class App>
+struct app_tries_one_candidate<App, decltype((void)App::kTriesOneCandidate)> {
+  static constexpr bool value = App::kTriesOneCandidate;
+};
+
+template <class SampleType, class App, class EdgeArray, class WeightArray>
+__device__ __forceinline__ bool attempt_output(int step, CSRPartition& csr, VertexID transit, VertexID sample_id,
+                                               SampleType* state, float max_weight, EdgeArray& edges,
+                                               WeightArray& weights, EdgePos_t n_edges, curandState* rng, bool first,
+                                               VertexID* result) {
+  if constexpr (app_tries_one_candidate<App>::value) {
+    return App().template attempt<SampleType, EdgeArray, WeightArray>(step, &csr, &transit, sample_id, state, max_weight,
+                                                                      edges, weights, n_edges, 0, rng, first, result);
+  } else {
+    *result = App().template next<SampleType, EdgeArray, WeightArray>(step, &csr, &transit, sample_id, state, max_weight,
+                                                                      edges, weights, n_edges, 0, rng);
+    return true;
+  }
+}
+
+template <class App>
+using walk_record = std::conditional_t<app_uses_weights<App>::value, WeightedWalkEdge, WalkEdge>;
+
+// What a walk needs of the vertex it has come to.  One 16-byte record where the largest weight is needed
+// (DeepWalk over 10 K vertices 1.71 -> 1.60 ms, over 1 M 3.84 -> 3.37, R-MAT 22 weighted node2vec 24.6 -> 24.1); the two
+// row positions alone are better off in their own array of 4 bytes a vertex (uniform walks over 1 M: 1.77, not 1.97 ms).
+template <class App>
+__device__ __forceinline__ void enter_vertex(const CSRPartition& csr, const WalkVertex* __restrict__ vertices, VertexID v,
+                                             EdgePos_t* begin, EdgePos_t* n_edges, float* max_weight) {
+  if constexpr (app_uses_weights<App>::value) {
+    const WalkVertex r = vertices[v];
+    *begin = r.begin;
+    *n_edges = r.n_edges;
+    *max_weight = r.max_weight;
+  } else {
+    *begin = csr.row_ptr[v];
+    *n_edges = csr.row_ptr[v + 1] - *begin;
+    *max_weight = csr.max_weights[v];
+  }
+}
+
+// Walks that are not inverted: one launch does all steps of all walks.  A lane keeps its walk, with
+// the current vertex, the random state and the sample state in registers, until it ends, and
+// then takes the next walk of its wavefront; results go straight into the rows, four to a store.
+//
+// What bounds it: the gathers.  Over a graph beyond the caches the requests past L2 (R-MAT 22 weighted
+// node2vec: 1.17e9 of them in 24.5 ms, 47.8 G/s of the 48-50 the gather probe reaches: row extent, 2.95
+// candidates and 0.9 tests a step), over one within them L2's own rate and, with few walks, the chain
+// of dependent loads.  A turn of the loop is therefore two CANDIDATES of every lane (they share a
+// Philox block), not one step: a wavefront that waits at every step for the slowest of 64 rejection
+// loops takes 12.7 rounds a step where its lanes need 2.95 on average; here a lane that has accepted goes on
+// while its neighbours still try (100 K node2vec walks 1.45 -> 0.77 ms).
+//
+// Against inverting before every step (ms a pass, sorted and balanced / this): uniform walks over 2.7 K vertices
+// 0.50 / 0.10, 57 K 0.83 / 0.12, 200 K 5.5 / 0.37, 1 M 10.1 / 1.5; DeepWalk, 100 walks a vertex, over 10 K vertices
+// 9.3 / 1.6 and over R-MAT 16 27.8 / 12.7; MultiRW 100 K 1.7 / 0.7; weighted node2vec 100 K 2.9 / 0.77, 700 K 13.6 /
+// 4.0, R-MAT 22 34.5 / 24.1, four walks a vertex over 700 K 27.6 / 14.5.  There is no case among them where
+// the order is worth what it costs.
+//
+// Walks are handed out in blocks of 64: block w to wavefront w, the rest from a counter.  (Every n_waves-th
+// block to a wavefront, without a counter: 38.6 ms on R-MAT 22 - whether a vertex has edges depends on the bits of
+// its id, and so do multiples of n_waves.)  queue[0] counts the blocks handed out after the first n_waves,
+// queue[1] the wavefronts that are done; the last one leaves both zero for the next pass.  Nobody waits for anybody.
+template <class SampleType, class App, bool kRecords>
+__global__ __launch_bounds__(kFlatThreads) void walk_rows_kernel(StepParams P, int n_steps, uint32_t n_waves,
+                                                                 uint32_t* queue,
+                                                                 const WalkVertex* __restrict__ vertices,
+                                                                 const walk_record<App>* __restrict__ records) {
+  typedef walk_record<App> Record;
+  static_assert(kFlatThreads == kWave, "a workgroup is a wavefront");
   constexpr bool kTravels = state_fits_pair<SampleType>::value;
+  const uint32_t lane = threadIdx.x;
+  const bool explicit_transits = App().hasExplicitTransits();
+  CSRPartition csr = P.csr;
+  const uint32_t n_walks = P.n_pairs;
+  // the walks [block, block_end) are this wavefront's to start; none and !more: nothing is left
+  uint32_t block = blockIdx.x * kWave;
+  uint32_t block_end = block + kWave < n_walks ? block + kWave : n_walks;
+  bool more = (uint64_t)n_waves * kWave < n_walks;
+  const bool queued = more;
+  bool busy = false, fresh = false, first = false;
+  uint32_t slot = 0;
+  int step = 0;
+  VertexID transit = P.invalid, r0 = P.invalid, r1 = P.invalid, r2 = P.invalid, r3 = P.invalid;  // the last four results
+  EdgePos_t begin = 0, n_edges = 0;
+  float max_weight = 0.0f;
+  curandState rng;
+  rng.reset(0, 0, 0);
   SampleType local_state;
   SampleType* state = &local_state;
-  if constexpr (kTravels) {
-    const uint32_t bits = P.pair_state ? P.pair_state[i] : ((const uint32_t*)P.samples)[slot];
-    __builtin_memcpy(&local_state, &bits, sizeof(uint32_t));
-  } else if (!std::is_empty<SampleType>::value) {
-    state = (SampleType*)P.samples + slot;
-  }
-  const bool explicit_transits = App().hasExplicitTransits();
-  int step = P.step;
-  for (int k = 0; k < stretch_steps && transit != P.invalid; ++k, ++step) {
-    const EdgePos_t begin = csr.row_ptr[transit];
-    const EdgePos_t n_edges = csr.row_ptr[transit + 1] - begin;
-    VertexID neighbor = P.invalid;
-    curandState rng;
-    if (n_edges != 0) {  // next() only runs for a transit that has edges (nextdoor.cu:250-262)
-      const float max_weight = csr.max_weights[transit];
-      rng.reset(P.seed, P.first_slot + slot, (uint32_t)step);
-      VertexID r;
-      if (app_uses_weights<App>::value) {
-        PairedEdgeIds edges{P.paired_edges + begin};
-        PairedEdgeWeights weights{P.paired_edges + begin};
-        r = App().template next<SampleType, PairedEdgeIds, PairedEdgeWeights>(
-            step, &csr, &transit, (VertexID)(P.first_sample + slot), state, max_weight, edges, weights, n_edges, 0, &rng);
-      } else {
-        const CSR::Edge* edges = csr.edges + begin;
-        const float* weights = csr.weights + begin;
-        r = App().template next<SampleType, const CSR::Edge*, const float*>(
-            step, &csr, &transit, (VertexID)(P.first_sample + slot), state, max_weight, edges, weights, n_edges, 0, &rng);
+  Record last;
+  last.dst = -1;
+  for (;;) {
+    const uint64_t idle = __ballot(!busy);
+    if (idle != 0 && (more || block < block_end)) {
+      if (block == block_end) {
+        uint32_t turn = 0;
+        if (lane == 0) turn = atomicAdd(queue, 1u);
+        const uint64_t at = ((uint64_t)n_waves + (uint32_t)__builtin_amdgcn_readfirstlane((int)turn)) * kWave;
+        more = at < n_walks;
+        block = more ? (uint32_t)at : 0u;
+        block_end = more ? (at + kWave < n_walks ? block + kWave : n_walks) : 0u;
       }
-      neighbor = r == -1 ? P.invalid : r;  // nextdoor.cu:288
+      const uint32_t walk = block + (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
+      if (!busy && walk < block_end) {
+        slot = walk;
+        transit = (VertexID)P.pair_keys[slot];
+        if constexpr (kTravels) {
+          const uint32_t bits = ((const uint32_t*)P.samples)[slot];
+          __builtin_memcpy(&local_state, &bits, sizeof(uint32_t));
+        } else if (!std::is_empty<SampleType>::value) {
+          state = (SampleType*)P.samples + slot;
+        }
+        step = 0;
+        busy = fresh = true;
+        n_edges = 0;
+        if (transit != P.invalid) enter_vertex<App>(csr, vertices, transit, &begin, &n_edges, &max_weight);
+      }
+      const uint32_t asked = (uint32_t)__popcll(idle);
+      block = block_end - block > asked ? block + asked : block_end;
     }
-    if (P.pair_cells) {
-      // the last step of all, or of this walk, or of the stretch may be an even one
-      int32_t* cell = P.pair_cells + ((size_t)(step >> 1) * P.pair_cell_samples + slot) * 2;
-      if (step & 1) *reinterpret_cast<int2*>(cell) = make_int2(transit, neighbor);
-      else if (step == last_step) cell[0] = neighbor;
-      if (P.walk_cells && (step == last_step || neighbor == P.invalid))
-        P.walk_cells[slot] = walk_cells_at_end(step, step == last_step);
-    } else {
-      P.step_out[(size_t)k * out_stride + slot] = neighbor;
+    if (__ballot(busy) == 0) {
+      if (more || block < block_end) continue;
+      break;
     }
-    transit = neighbor;
-    if (explicit_transits && step != last_step) {
-      if (n_edges == 0) rng.reset(P.seed, P.first_slot + slot, (uint32_t)step);
-      const VertexID_t t = App().stepTransits(step + 1, (VertexID)(P.first_sample + slot), *state, 0, &rng);
-      transit = t == -1 ? P.invalid : t;
+    bool ended = false;
+    if (busy) {
+      if (fresh) {
+        rng.reset(P.seed, P.first_slot + slot, (uint32_t)step);
+        first = true;
+      }
+      VertexID r = -1;
+      bool decided = true;
+      if (n_edges != 0) {  // next() only runs for a transit that has edges (nextdoor.cu:250-262)
+        const VertexID sample_id = (VertexID)(P.first_sample + slot);
+        decided = false;
+        // two tries a turn: they share a Philox block
+#pragma unroll
+        for (int t = 0; t < (app_tries_one_candidate<App>::value ? 2 : 1); ++t) {
+          if (decided) continue;
+          if constexpr (kRecords && app_uses_weights<App>::value) {
+            WalkEdgeIds<Record> edges{records + begin, &last};
+            WalkEdgeWeights weights{records + begin};
+            decided = attempt_output<SampleType, App, WalkEdgeIds<Record>, WalkEdgeWeights>(
+                step, csr, transit, sample_id, state, max_weight, edges, weights, n_edges, &rng, first, &r);
+          } else if constexpr (kRecords) {
+            WalkEdgeIds<Record> edges{records + begin, &last};
+            const float* weights = csr.weights + begin;
+            decided = attempt_output<SampleType, App, WalkEdgeIds<Record>, const float*>(
+                step, csr, transit, sample_id, state, max_weight, edges, weights, n_edges, &rng, first, &r);
+          } else if constexpr (app_uses_weights<App>::value) {
+            PairedEdgeIds edges{P.paired_edges + begin};
+            PairedEdgeWeights weights{P.paired_edges + begin};
+            decided = attempt_output<SampleType, App, PairedEdgeIds, PairedEdgeWeights>(
+                step, csr, transit, sample_id, state, max_weight, edges, weights, n_edges, &rng, first, &r);
+          } else {
+            const CSR::Edge* edges = csr.edges + begin;
+            const float* weights = csr.weights + begin;
+            decided = attempt_output<SampleType, App, const CSR::Edge*, const float*>(
+                step, csr, transit, sample_id, state, max_weight, edges, weights, n_edges, &rng, first, &r);
+          }
+          first = false;
+        }
+      }
+      fresh = decided;
+      if (decided) {
+        const VertexID neighbor = r == -1 ? P.invalid : r;  // nextdoor.cu:288
+        r0 = r1;
+        r1 = r2;
+        r2 = r3;
+        r3 = neighbor;
+        if ((step & 3) == 3)
+          *reinterpret_cast<FourIds*>(P.step_out + (size_t)slot * P.out_pitch + (step - 3)) = FourIds{r0, r1, r2, r3};
+        const bool had_transit = transit != P.invalid;
+        transit = neighbor;
+        if (explicit_transits && had_transit && step + 1 < n_steps) {
+          const VertexID t = App().stepTransits(step + 1, (VertexID)(P.first_sample + slot), *state, 0, &rng);
+          transit = t == -1 ? P.invalid : t;
+        }
+        step++;
+        ended = step == n_steps || transit == P.invalid;
+        if (!ended) {
+          if (kRecords && n_edges != 0 && last.dst == transit) {
+            begin = last.begin;
+            n_edges = last.n_edges;
+            max_weight = last.max_weight;
+          } else {
+            enter_vertex<App>(csr, vertices, transit, &begin, &n_edges, &max_weight);
+          }
+        }
+      }
+    }
+    const uint64_t ends = __ballot(ended);
+    if (ends != 0) {
+      int rest = n_steps;  // first slot of the row that is still to be written
+      if (ended) {
+        busy = false;
+        if constexpr (kTravels) {
+          uint32_t bits;
+          __builtin_memcpy(&bits, &local_state, sizeof(uint32_t));
+          ((uint32_t*)P.samples)[slot] = bits;
+        }
+        rest = step & ~3;
+        if ((step & 3) != 0) {
+          for (int k = step & 3; k < 4; ++k) {
+            r0 = r1;
+            r1 = r2;
+            r2 = r3;
+            r3 = P.invalid;
+          }
+          int32_t* dst = P.step_out + (size_t)slot * P.out_pitch + rest;
+          if (rest + 4 <= n_steps) {
+            *reinterpret_cast<FourIds*>(dst) = FourIds{r0, r1, r2, r3};
+          } else {
+            dst[0] = r0;
+            if (rest + 1 < n_steps) dst[1] = r1;
+            if (rest + 2 < n_steps) dst[2] = r2;
+          }
+          rest += 4;
+        }
+      }
+      // what is left of the rows of walks that ended early, by the whole wavefront: at most 128 slots
+      uint64_t todo = __ballot(rest < n_steps);
+      while (todo) {
+        const int src = __ffsll((unsigned long long)todo) - 1;
+        todo &= todo - 1;
+        const int from = __shfl(rest, src, kWave);
+        int32_t* row = P.step_out + (size_t)__shfl(slot, src, kWave) * P.out_pitch;
+        const int at = from + 4 * (int)lane;
+        if (at + 4 <= n_steps) {
+          *reinterpret_cast<FourIds*>(row + at) = FourIds{P.invalid, P.invalid, P.invalid, P.invalid};
+        } else {
+          for (int x = at; x < n_steps; ++x) row[x] = P.invalid;
+        }
+      }
     }
   }
-  // the walk as it stands after the stretch (INVALID: it has ended and the next compaction drops it)
-  const bool pass_over = step > last_step;
-  if (P.emit_keys && !pass_over) {
-    P.emit_keys[i] = (uint32_t)transit;
-    P.emit_slots[i] = slot;
-  }
-  if constexpr (kTravels) {
-    uint32_t bits;
-    __builtin_memcpy(&bits, &local_state, sizeof(uint32_t));
-    if (P.emit_state && !pass_over) P.emit_state[i] = bits;
-    if (pass_over || transit == P.invalid) ((uint32_t*)P.samples)[slot] = bits;  // the state goes home
+  if (queued && lane == 0 && atomicAdd(queue + 1, 1u) == n_waves - 1) {
+    // every wavefront has taken its last block
+    queue[0] = 0;
+    queue[1] = 0;
   }
 }
 
@@ -1790,6 +1955,7 @@ class Engine : public EngineBase {
     // Counters per vertex for the small-map inversion: the walks that step onto a vertex are
     // about its share of the edge ends; one counter per kSmallMapWalksPerCounter of them.
     small_map_ = false;
+    inversion_forced_ = getenv("ND_SMALL_MAP") != nullptr;  // chooses how the map is inverted: so it is
     if (walk_mode_ && max_pairs_ <= kSmallMapPairs && (uint64_t)invalid_ < kSmallMapCounters &&
         !(getenv("ND_SMALL_MAP") && atoi(getenv("ND_SMALL_MAP")) == 0)) {
       const size_t V = (size_t)graph_->get_n_vertices();
@@ -1899,6 +2065,25 @@ class Engine : public EngineBase {
     }
     paired_results_ = walk_mode_ && !rows_direct_ && rows_per_block_ > 0 && !App().hasExplicitTransits() &&
                       !(getenv("ND_PAIRED_RESULTS") && atoi(getenv("ND_PAIRED_RESULTS")) == 0);
+    if (walk_mode_) {
+      ND_HIP_TRY(hipMalloc(&d_walk_queue_, 2 * sizeof(uint32_t)));
+      ND_HIP_TRY(hipMemset(d_walk_queue_, 0, 2 * sizeof(uint32_t)));
+      int per_cu = 0, device = 0, cus = 0;
+      ND_HIP_TRY(hipGetDevice(&device));
+      ND_HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+      ND_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, walk_rows_kernel<SampleType, App, true>, kFlatThreads, 0));
+      if (app_uses_weights<App>::value) walk_vertices_ = dgraph_->walk_vertices(stream_);
+      if (app_uses_weights<App>::value && !walk_vertices_) { last_error = "no device memory for the walk vertices"; return -1; }
+      walk_records_ = nullptr;
+      // (not where stepTransits names another vertex than next() returned; nor for an app that looks edges up,
+      // whose tests are what its steps wait for: weighted node2vec over 1.07 GB of edges 24.1 ms, over records 26.4)
+      const size_t edge_bytes = (app_uses_weights<App>::value ? sizeof(EdgeRecord) : sizeof(CSR::Edge)) *
+                                (size_t)graph_->get_n_edges();
+      if (edge_bytes >= kWalkRecordsFromBytes && !app.hasExplicitTransits() && !app_uses_edge_lookup<App>::value)
+        walk_records_ = dgraph_->template walk_edges<walk_record<App>>(stream_);
+      walk_waves_at_once_ = (uint32_t)std::max(1, per_cu * cus);
+      walk_waves_queued_ = (uint32_t)std::max(1, (int)kQueuedWavesPerCu * cus);
+    }
     if (paired_results_) ND_HIP_TRY(hipMalloc(&d_walk_cells_, sizeof(uint32_t) * (size_t)n_samples_));
     allocated_ = true;
     return 0;
@@ -1973,25 +2158,61 @@ class Engine : public EngineBase {
     }
   }
 
+  // A pass of walks that are not inverted: one launch.
+  int enqueue_walks() {
+    balanced_this_pass_ = false;
+    if (mark_unwritten_) {
+      const size_t n = (size_t)n_samples_ * (size_t)final_sample_size();
+      fill_i32<<<dim3((unsigned)((n + 1023) / 1024)), dim3(1024), 0, stream_>>>(d_final_, n, invalid_ + 1);
+    }
+    StepParams P = {};
+    P.csr = view_;
+    P.step_size = 1;
+    P.transits_per_sample = 1;
+    P.final_size = P.out_pitch = (uint32_t)final_sample_size();
+    P.invalid = invalid_;
+    P.seed = seed_;
+    P.first_slot = (uint64_t)first_sample_;
+    P.first_sample = (uint32_t)first_sample_;
+    P.n_pairs = (uint32_t)n_samples_;
+    P.pair_keys = (const uint32_t*)d_initial_;
+    P.step_out = d_final_;
+    P.samples = d_samples_;
+    P.paired_edges = dgraph_->paired;
+    // Every walk at once where the device holds them all; else three wavefronts to a SIMD take them from a queue.
+    // That many keep the memory path past L2 as busy as more would (R-MAT 22 weighted node2vec: 24.1 ms with 12
+    // wavefronts to a compute unit, 23.9 with 20; 27 with 8), and the fewer walks are under way, the sooner each is
+    // done: shorter tails, more hits (DeepWalk over 1 M vertices 3.0 ms with 12, 3.4 with 20).
+    const uint64_t blocks = ((uint64_t)n_samples_ + kWave - 1) / kWave;
+    const uint32_t n_waves = (uint32_t)(blocks <= walk_waves_at_once_ ? blocks : std::min(walk_waves_at_once_, walk_waves_queued_));
+    tick();
+    if (walk_records_)
+      walk_rows_kernel<SampleType, App, true><<<dim3(n_waves), dim3(kFlatThreads), 0, stream_>>>(
+          P, App().steps(), n_waves, d_walk_queue_, walk_vertices_, walk_records_);
+    else
+      walk_rows_kernel<SampleType, App, false><<<dim3(n_waves), dim3(kFlatThreads), 0, stream_>>>(
+          P, App().steps(), n_waves, d_walk_queue_, walk_vertices_, nullptr);
+    tock(&times.flat_kernel);
+    times.flat_launches++;
+    ND_HIP_TRY(hipGetLastError());
+    return 0;
+  }
+
   // Every launch of one pass, in order, on stream_; no host wait in between.
   int enqueue_pass(int mode) {
     App app;
     const int n_steps = app.steps();
     const size_t F = (size_t)final_sample_size();
-    // With few walks per vertex hardly any two walks share a transit: the sorted order then
-    // saves less in the step kernels (shared lines) than the inversion costs.
-    int sort_period = inversion_period;
-    if (sort_period <= 0)
-      sort_period = (double)n_samples_ < kWalksPerVertexForInversion * (double)invalid_ ? kSparseInversionPeriod : 1;
     const bool sample_parallel = mode == kSampleParallel;
-    if (sample_parallel && sort_period <= 1) sort_period = kSparseInversionPeriod;
+    const bool inverts = inversion_period == 1 || (inversion_period == 0 && inversion_forced_);
+    if (walk_mode_ && (sample_parallel || !inverts)) return enqueue_walks();
     // A pass whose classifications found nothing at all for the workgroup kernel is followed by
     // passes that do not classify (nor launch the workgroup kernel); every kIdleLookEvery-th
     // pass looks again.  Results do not depend on it.
-    bool balance = mode == kTransitParallelLoadBalanced && n_steps > 1 && !(walk_mode_ && sort_period > 1);
+    bool balance = mode == kTransitParallelLoadBalanced && n_steps > 1;
     // small maps inverted at every step, the pairs placed by the kernel that emits them: one launch
     // per step, every pair with the flat lanes (what a hub's adjacency is, is in the caches)
-    const bool placed = small_placed_ && sort_period == 1 && !sample_parallel;
+    const bool placed = small_placed_;
     if (placed) {
       balance = false;
       if (placed_dirty_) {
@@ -2078,7 +2299,7 @@ class Engine : public EngineBase {
       P.emit_slots = emits ? d_emit_slots_ : nullptr;
       P.emit_state = emits && state_travels_ ? d_emit_state_ : nullptr;
       // small maps inverted at every step: the emitting kernels count the pairs per next transit
-      const bool counted = small_map_ && sort_period == 1 && !sample_parallel;
+      const bool counted = small_map_;
       P.emit_counts = emits && counted ? d_small_ : nullptr;
       P.emit_ranks = emits && counted ? d_emit_ranks_ : nullptr;
       P.emit_counter_base = d_counter_base_;
@@ -2169,7 +2390,7 @@ class Engine : public EngineBase {
           sorts_done++;
           if (launch_step(P, flat_lanes, balance, meta) != 0) return -1;
         } else {
-          const bool compact_only = sample_parallel || (walk_mode_ && sort_period > 1);
+          const bool compact_only = sample_parallel;
           const SortPlan plan = make_sort_plan(n_pairs, compact_only ? 0 : max_bits_);
           SortJob job;
           if (walk_mode_) {
@@ -2202,19 +2423,7 @@ class Engine : public EngineBase {
           P.live_pairs = live_now;
           live_last = live_now;
           sorts_done++;
-          if (compact_only && walk_mode_) {
-            // the walks keep their lanes until the next compaction
-            const int stretch = n_steps - step < sort_period ? n_steps - step : sort_period;
-            P.emit_keys = d_emit_keys_;
-            P.emit_slots = d_emit_slots_;
-            P.emit_state = state_travels_ ? d_emit_state_ : nullptr;
-            tick();
-            walk_stretch_kernel<SampleType, App><<<dim3((n_pairs + kFlatThreads - 1) / kFlatThreads), dim3(kFlatThreads), 0,
-                                                   stream_>>>(P, stretch, n_steps - 1, (size_t)n_samples_);
-            tock(&times.flat_kernel);
-            times.flat_launches++;
-            step += stretch - 1;
-          } else if (!balance || compact_only) {
+          if (!balance || compact_only) {
             if (launch_step(P, flat_lanes, false, nullptr) != 0) return -1;
           } else {
             tick();
@@ -2448,6 +2657,12 @@ class Engine : public EngineBase {
   // the step.  ND_STEP_SCHEDULE=serial|merged|forked forces one (read when the buffers are
   // allocated).  Results do not depend on it.
   enum { kScheduleAuto = -1, kScheduleSerial = 0, kScheduleMerged = 1, kScheduleForked = 2 };
+  static constexpr uint32_t kQueuedWavesPerCu = 12;
+  // Edge arrays (as the walk would read them otherwise) from this size on are read as walk records: 4 and 8 bytes an
+  // edge fit the caches then where 16 and 32 do not, and a step over a graph in the caches gains nothing from them
+  // (32 MB is the L2 of all eight XCDs).  Uniform walks over 48 MB: 1.77 -> 1.49 ms; DeepWalk over 120 MB 3.37 -> 2.96,
+  // over 17 MB 12.7 -> 14.4, over 2.4 MB 1.60 -> 2.16.
+  static constexpr size_t kWalkRecordsFromBytes = 32u << 20;
   static constexpr uint64_t kMergedLanesAtMost = 1ull << 19;
   static constexpr uint32_t kMergedWorkgroupBlocks = 16384;
 
@@ -2568,6 +2783,7 @@ class Engine : public EngineBase {
     release(d_final_);
     release(d_step_out_);
     release(d_walk_cells_);
+    release(d_walk_queue_);
     release(d_keys_a_);
     release(d_vals_a_);
     release(d_keys_b_);
@@ -2625,6 +2841,9 @@ class Engine : public EngineBase {
   uint32_t chunk_capacity_ = 0;
   uint32_t row_pitch_ = 0, rows_per_block_ = 0;
   bool paired_results_ = false;
+  const WalkVertex* walk_vertices_ = nullptr;
+  const walk_record<App>* walk_records_ = nullptr;  // dgraph_'s, where they pay
+  uint32_t walk_waves_at_once_ = 1, walk_waves_queued_ = 1;  // wavefronts of walk_rows_kernel
   StepLayout layout_{};
   bool allocated_ = false;
 
@@ -2637,6 +2856,7 @@ class Engine : public EngineBase {
   SampleType* d_samples_init_ = nullptr;
   VertexID_t* d_final_ = nullptr;
   VertexID_t* d_step_out_ = nullptr;
+  uint32_t* d_walk_queue_ = nullptr;  // of walk_rows_kernel
   uint32_t* d_walk_cells_ = nullptr;  // cells of every walk that hold results (StepParams::walk_cells)
   uint32_t *d_keys_a_ = nullptr, *d_vals_a_ = nullptr, *d_keys_b_ = nullptr, *d_vals_b_ = nullptr;
   uint32_t* d_hist_ = nullptr;
@@ -2647,7 +2867,7 @@ class Engine : public EngineBase {
   VertexID_t* d_explicit_ = nullptr;    // that map: the transit of every pair of the coming step
   uint32_t *d_emit_keys_ = nullptr, *d_emit_slots_ = nullptr, *d_emit_state_ = nullptr;  // next step's pairs
   // small maps: the inversion without a sort (small_map_scan, small_map_place)
-  bool small_map_ = false;
+  bool small_map_ = false, inversion_forced_ = false;
   size_t small_counters_ = 0;
   uint32_t* d_counter_base_ = nullptr;  // first counter of every vertex
   uint32_t* d_emit_ranks_ = nullptr;

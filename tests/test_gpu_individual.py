@@ -473,3 +473,36 @@ def test_small_map_inversion_classifies_every_run_by_the_rules(oracle, monkeypat
         assert [s.counter(i) for i in range(5)] == [looked, single, split, refused, items]
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("app,kind_name,state,n,mean_degree", [
+    # more walks than the device holds at once, so that lanes take walks from the queue; the edges of the first two
+    # are read as walk records (32 MB of them and more), MultiRW's transits are not what next() returned
+    ("UniformRandomWalk8", "UNIFORM_WALK", False, 600011, 15),
+    ("DeepWalkPerVertex", "DEEPWALK", False, 530003, 9),
+    ("WeightedNode2Vec8", "WEIGHTED_NODE2VEC", True, 600011, 3),
+    ("MultiRW4x6", "MULTIRW", False, 600011, 3),
+    # one walk more and one less than a wavefront holds
+    ("UniformRandomWalk8", "UNIFORM_WALK", False, 63, 3),
+    ("DeepWalkPerVertex", "DEEPWALK", False, 65, 3),
+])
+def test_walks_that_keep_their_lanes(oracle, app, kind_name, state, n, mean_degree):
+    g = graphs.random_graph(n=n, mean_degree=mean_degree, seed=n, isolated_every=5)
+    s = nd.Sampler(app, g, seed=SEED)  # as it comes: not inverted
+    try:
+        roots = s.initial_contents
+        if kind_name == "MULTIRW":
+            states = s.sample_states().view(np.int32).reshape(s.num_samples, -1)
+            want = oracle.sample_multirw(graphs.oracle_view(g), SEED, states[:, :-1], s.steps)[0]
+        else:
+            want, want_state = oracle.sample_individual(graphs.oracle_view(g), desc_for(oracle, s, getattr(oracle, kind_name), app),
+                                                        SEED, roots)
+        for turn in range(2):
+            print("app", app, "V", n, "turn", turn, flush=True)
+            s.do_transit_parallel()
+            assert np.array_equal(s.final_samples(), want)
+            if state:
+                alive = want_state != -1
+                assert np.array_equal(s.sample_states().view(np.int32)[alive], want_state[alive])
+    finally:
+        s.close()
