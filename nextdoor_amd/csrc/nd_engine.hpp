@@ -131,6 +131,14 @@ class EngineBase {
     return -1;
   }
 
+  // Sample states: what an App's struct holds is its own, but mostly it is vertices (and small numbers), which
+  // fit the ids' bits.  Where they do not once, no later transfer tries (100 K samples of MultiRW, 40 MB: 0.88 -> 0.52 ms).
+  int states_to_host(void* dst, const void* src, size_t bytes, hipStream_t stream) {
+    const int rc = fetch_to_host(dst, src, bytes, states_fit_ids_ ? (uint32_t)max_bits() : 32u, -1, stream);
+    if (result_stream.misfit()) states_fit_ids_ = false;
+    return rc;
+  }
+
   HostArray<VertexID_t> hFinalSamples{host_pool};  // as NextDoorData::hFinalSamples (libNextDoor.hpp:17)
   HostArray<unsigned char> hSampleStates{host_pool};
   std::vector<VertexID_t> initialContents;     // as NextDoorData::initialContents (libNextDoor.hpp:18)
@@ -142,6 +150,9 @@ class EngineBase {
   std::string last_error;
   bool profiling = false;
   PhaseTimes times;
+
+ private:
+  bool states_fit_ids_ = true;
 };
 
 #define ND_HIP_TRY(expr)                                                                  \
@@ -2066,8 +2077,8 @@ class Engine : public EngineBase {
     paired_results_ = walk_mode_ && !rows_direct_ && rows_per_block_ > 0 && !App().hasExplicitTransits() &&
                       !(getenv("ND_PAIRED_RESULTS") && atoi(getenv("ND_PAIRED_RESULTS")) == 0);
     if (walk_mode_) {
-      ND_HIP_TRY(hipMalloc(&d_walk_queue_, 2 * sizeof(uint32_t)));
-      ND_HIP_TRY(hipMemset(d_walk_queue_, 0, 2 * sizeof(uint32_t)));
+      ND_HIP_TRY(hipMalloc(&d_walk_queue_, 2 * kMostWalkRanges * sizeof(uint32_t)));
+      ND_HIP_TRY(hipMemset(d_walk_queue_, 0, 2 * kMostWalkRanges * sizeof(uint32_t)));
       int per_cu = 0, device = 0, cus = 0;
       ND_HIP_TRY(hipGetDevice(&device));
       ND_HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
@@ -2093,6 +2104,7 @@ class Engine : public EngineBase {
   // the only host wait is at the end.
   int sample(int mode) override {
     if (!allocated_) { last_error = "sample before alloc"; return -1; }
+    if (ahead_) (void)finish_rows_ahead();  // nobody asked for them
     times = PhaseTimes();
     if (!std::is_empty<SampleType>::value) {
       ND_HIP_TRY(hipMemcpyAsync(d_samples_, d_samples_init_, sizeof(SampleType) * (size_t)n_samples_,
@@ -2165,6 +2177,47 @@ class Engine : public EngineBase {
       const size_t n = (size_t)n_samples_ * (size_t)final_sample_size();
       fill_i32<<<dim3((unsigned)((n + 1023) / 1024)), dim3(1024), 0, stream_>>>(d_final_, n, invalid_ + 1);
     }
+    const uint32_t ranges = walk_ranges();
+    if (ranges == 1) return launch_walks(0, (uint32_t)n_samples_, d_walk_queue_);
+    const size_t F = (size_t)final_sample_size();
+    std::vector<ResultStream::Ready> ready;
+    while (range_ends_.size() < ranges) {
+      hipEvent_t ev = nullptr;
+      ND_HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+      range_ends_.push_back(ev);
+    }
+    uint32_t first = 0;
+    for (uint32_t r = 0; r < ranges; ++r) {
+      const uint32_t end = r + 1 == ranges ? (uint32_t)n_samples_ : (uint32_t)((uint64_t)n_samples_ * (r + 1) / ranges / kWave * kWave);
+      const int rc = launch_walks(first, end - first, d_walk_queue_ + 2 * r);
+      if (rc != 0) return rc;
+      ND_HIP_TRY(hipEventRecord(range_ends_[r], stream_));
+      ready.push_back({end * F, range_ends_[r]});
+      first = end;
+    }
+    const hipError_t e = result_stream.begin(d_final_, (size_t)n_samples_ * F, (uint32_t)max_bits_, invalid_, rows_ahead,
+                                             stream_, std::move(ready));
+    if (e != hipSuccess) { last_error = std::string("results to the host: ") + hipGetErrorString(e); return -1; }
+    ahead_ = true;
+    return 0;
+  }
+
+  // Launches a pass of walks is split into, where its rows are to leave early.  Every one of them ends with its longest
+  // walks alone on the device (0.1 ms of uniform ones, 0.45 of weighted node2vec over R-MAT 22), and the first row
+  // leaves at the end of the first.  Pass with its rows, in 1 / 2 / 4 / 6 of them (ms): PPR over 262 K vertices
+  // 1.83 / 1.37 / 1.48 / 1.96, DeepWalk over 100 K 0.93 / 1.12 / -, over 500 K 4.1 / 3.2 / 2.8 / 3.0, 100 a vertex over
+  // 10 K 5.3 / 5.1 / 4.8 / 4.6, weighted node2vec over 700 K 7.2 / 6.2 / 5.4 / 6.6, R-MAT 22 38.1 / 32.7 / 30.2 / 30.8.
+  // Walks with states in memory wait for those, not for each other: MultiRW over 100 K vertices 1.89 / 1.56 / 1.66.
+  uint32_t walk_ranges() const {
+    if (!rows_ahead || profiling || wants_launch_graph()) return 1;
+    if (sizeof(VertexID_t) * (size_t)n_samples_ * (size_t)final_sample_size() <= kDirectResultBytes) return 1;
+    constexpr int64_t least = std::is_empty<SampleType>::value || state_fits_pair<SampleType>::value ? 96 << 10 : 48 << 10;
+    if (n_samples_ >= 10 * least) return kMostWalkRanges;
+    return (uint32_t)std::max<int64_t>(1, std::min<int64_t>(4, n_samples_ / least));
+  }
+
+  // The walks [first, first + count).
+  int launch_walks(uint32_t first, uint32_t count, uint32_t* queue) {
     StepParams P = {};
     P.csr = view_;
     P.step_size = 1;
@@ -2172,26 +2225,26 @@ class Engine : public EngineBase {
     P.final_size = P.out_pitch = (uint32_t)final_sample_size();
     P.invalid = invalid_;
     P.seed = seed_;
-    P.first_slot = (uint64_t)first_sample_;
-    P.first_sample = (uint32_t)first_sample_;
-    P.n_pairs = (uint32_t)n_samples_;
-    P.pair_keys = (const uint32_t*)d_initial_;
-    P.step_out = d_final_;
-    P.samples = d_samples_;
+    P.first_slot = (uint64_t)first_sample_ + first;
+    P.first_sample = (uint32_t)first_sample_ + first;
+    P.n_pairs = count;
+    P.pair_keys = (const uint32_t*)d_initial_ + first;
+    P.step_out = d_final_ + (size_t)first * P.out_pitch;
+    P.samples = d_samples_ ? d_samples_ + first : nullptr;
     P.paired_edges = dgraph_->paired;
     // Every walk at once where the device holds them all; else three wavefronts to a SIMD take them from a queue.
     // That many keep the memory path past L2 as busy as more would (R-MAT 22 weighted node2vec: 24.1 ms with 12
     // wavefronts to a compute unit, 23.9 with 20; 27 with 8), and the fewer walks are under way, the sooner each is
     // done: shorter tails, more hits (DeepWalk over 1 M vertices 3.0 ms with 12, 3.4 with 20).
-    const uint64_t blocks = ((uint64_t)n_samples_ + kWave - 1) / kWave;
+    const uint64_t blocks = ((uint64_t)count + kWave - 1) / kWave;
     const uint32_t n_waves = (uint32_t)(blocks <= walk_waves_at_once_ ? blocks : std::min(walk_waves_at_once_, walk_waves_queued_));
     tick();
     if (walk_records_)
       walk_rows_kernel<SampleType, App, true><<<dim3(n_waves), dim3(kFlatThreads), 0, stream_>>>(
-          P, App().steps(), n_waves, d_walk_queue_, walk_vertices_, walk_records_);
+          P, App().steps(), n_waves, queue, walk_vertices_, walk_records_);
     else
       walk_rows_kernel<SampleType, App, false><<<dim3(n_waves), dim3(kFlatThreads), 0, stream_>>>(
-          P, App().steps(), n_waves, d_walk_queue_, walk_vertices_, nullptr);
+          P, App().steps(), n_waves, queue, walk_vertices_, nullptr);
     tock(&times.flat_kernel);
     times.flat_launches++;
     ND_HIP_TRY(hipGetLastError());
@@ -2571,18 +2624,32 @@ class Engine : public EngineBase {
                          (uint32_t)max_bits_, invalid_, stream_);
   }
 
+  // Walks: where the next pass's rows shall go, if the caller expects to fetch them.  Rows of the first walks then
+  // cross the bus while later walks are still under way; sample() returns when the sampling is done, as
+  // always, and the rest of the rows arrives until finish_rows_ahead().  Any pass may leave it be.
+  VertexID_t* rows_ahead = nullptr;
+  bool rows_are_ahead() const { return ahead_; }
+  int finish_rows_ahead() {
+    ahead_ = false;
+    const hipError_t e = result_stream.finish();
+    if (e == hipSuccess) return 0;
+    last_error = std::string("results to the host: ") + hipGetErrorString(e);
+    return -1;
+  }
+
   bool is_walk() const { return walk_mode_; }
 
   int fetch_sample_states(void* dst, size_t bytes) override {
     if (!allocated_ || std::is_empty<SampleType>::value) { last_error = "no sample state"; return -1; }
     if (bytes != sample_state_bytes()) { last_error = "sample state size mismatch"; return -1; }
-    return fetch_to_host(dst, d_samples_, bytes, 32, 0, stream_);
+    return states_to_host(dst, d_samples_, bytes, stream_);
   }
 
   // Distinct post-pass over the device-resident result rows (see nd_distinct.hpp): every
   // hop segment of every sample becomes its ascending unique valid ids, INVALID-padded.
   int distinct() override {
     if (!allocated_) { last_error = "distinct before alloc"; return -1; }
+    if (ahead_) (void)finish_rows_ahead();  // they are about to change
     App app;
     if (app.outputFormat() != SampledVertices) { last_error = "distinct needs SampledVertices output"; return -2; }
     const int n_steps = app.steps();
@@ -2622,6 +2689,7 @@ class Engine : public EngineBase {
   static constexpr int kBalanceWords =
       kMaxSteps + 2 + (int)(kCounterCopies * sizeof(ClassCounters) / sizeof(uint32_t));
   static constexpr int kIdleLookEvery = 8;
+  static constexpr uint32_t kMostWalkRanges = 6;
   ClassCounters* counters_dev() const { return (ClassCounters*)(d_balance_ + kMaxSteps + 2); }
   // Walks write their results in cells of two steps (StepParams::pair_cells) where a step's
   // transit is the previous step's result and the rows are regrouped by assemble_walk_rows.
@@ -2776,6 +2844,10 @@ class Engine : public EngineBase {
   }
 
   void free_run_buffers() {
+    if (ahead_) (void)finish_rows_ahead();
+    rows_ahead = nullptr;
+    for (hipEvent_t ev : range_ends_) (void)hipEventDestroy(ev);
+    range_ends_.clear();
     drop_recorded_passes();
     release(d_initial_);
     release(d_samples_);
@@ -2844,6 +2916,8 @@ class Engine : public EngineBase {
   const WalkVertex* walk_vertices_ = nullptr;
   const walk_record<App>* walk_records_ = nullptr;  // dgraph_'s, where they pay
   uint32_t walk_waves_at_once_ = 1, walk_waves_queued_ = 1;  // wavefronts of walk_rows_kernel
+  bool ahead_ = false;                    // rows are on their way to rows_ahead
+  std::vector<hipEvent_t> range_ends_;    // ends of the launches of such a pass
   StepLayout layout_{};
   bool allocated_ = false;
 

@@ -10,8 +10,10 @@
 //    ids that are all INVALID - walks that have ended, samples without neighbours - are left out.
 //    The kernel writes its output straight into page-locked memory (54.7 GB/s, as fast as the copy
 //    engine's 57, without a launch and a copy per piece), and host threads unpack a piece
-//    while the next one crosses.  The host side is not what bounds it: eight threads write 170 GB/s of
-//    unpacked ids on the 16-core share of a GPU's host, four 147.
+//    while the next one crosses.  Twelve threads write 220 GB/s of unpacked ids on the 16-core share of a
+//    GPU's host, eight 200.
+//  * Results whose first words are final while later ones are still being computed (walks) can leave then already
+//    (ResultStream::begin, with what to wait for).
 //  * The arrays results land in come from a small pool per sampler and keep their pages: a first
 //    touch costs 0.1-0.4 s per GB, more than the sampling.
 //  * Such an array can be given to the caller (HostLease) instead of being copied for them; it goes
@@ -47,45 +49,56 @@ namespace nd {
 // until the process ends (no destructor: a thread must not outlast what it waits on).
 class HostWorkers {
  public:
-  // More do not help: unpacking is bound by memory from four threads on.
-  static constexpr unsigned kMost = 7;
+  // PPR walks over 262 K vertices, most groups dead: 1.33 ms with seven, 1.18 with eleven.
+  static constexpr unsigned kMost = 11;
 
   static HostWorkers& get() {
     static HostWorkers* workers = new HostWorkers;
     return *workers;
   }
 
-  // Runs body() on this thread and, as far as threads are free, on up to `helpers` others.  Returns
-  // when every body() that started has returned.  body() has to be able to do all the work
-  // alone, and must not throw.
-  void run(unsigned helpers, const std::function<void()>& body, const std::function<void()>& caller_body) {
-    helpers = std::min(helpers, limit());
-    Job job{&body, helpers, 0};
-    if (helpers > 0) {
-      std::lock_guard<std::mutex> lock(mutex_);
-      grow(helpers);
-      jobs_.push_back(&job);
-    }
-    if (helpers > 0) wake_.notify_all();
-    caller_body();
-    if (helpers == 0) return;
-    std::unique_lock<std::mutex> lock(mutex_);
-    jobs_.remove(&job);  // nobody starts on it any more
-    ended_.wait(lock, [&] { return job.running == 0; });
-  }
-  void run(unsigned helpers, const std::function<void()>& body) { run(helpers, body, body); }
-
- private:
+  // Work that several threads may take part in: each calls body() once, and every body() has to be able to
+  // do all of it alone, and must not throw.  A Job stays where it is from start() to join().
   struct Job {
-    const std::function<void()>* body;
-    unsigned wanted, running;
+    std::function<void()> body;
+    unsigned wanted = 0, running = 0;
   };
 
+  // Has up to `helpers` threads call body(), as far as threads are free.
+  void start(Job& job, unsigned helpers) {
+    job.wanted = std::min(helpers, limit());
+    job.running = 0;
+    if (job.wanted == 0) return;
+    {
+      std::lock_guard<std::mutex> lock(mutex_);
+      grow(job.wanted);
+      jobs_.push_back(&job);
+    }
+    wake_.notify_all();
+  }
+
+  // Nobody starts on it any more; returns when every body() that started has returned.
+  void join(Job& job) {
+    std::unique_lock<std::mutex> lock(mutex_);
+    jobs_.remove(&job);
+    ended_.wait(lock, [&] { return job.running == 0; });
+  }
+
+  // body() on this thread and on up to `helpers` others.
+  void run(unsigned helpers, const std::function<void()>& body) {
+    Job job;
+    job.body = body;
+    start(job, helpers);
+    body();
+    join(job);
+  }
+
+ private:
   HostWorkers() = default;
 
   static unsigned limit() {
     const unsigned hw = std::thread::hardware_concurrency();
-    return hw > 1 ? std::min(hw / 2, kMost) : 0;
+    return hw > 1 ? std::min(hw * 3 / 4, kMost) : 0;
   }
 
   void grow(unsigned helpers) {
@@ -112,7 +125,7 @@ class HostWorkers {
       job->wanted--;
       job->running++;
       lock.unlock();
-      (*job->body)();
+      job->body();
       lock.lock();
       if (--job->running == 0) ended_.notify_all();
     }
@@ -284,6 +297,13 @@ class HostArray {
     block_ = HostBlock();
     return lease;
   }
+  // its memory was handed over, and not taken anew since
+  bool taken() const { return size_ != 0 && !block_.p; }
+  void swap(HostArray& other) {
+    std::swap(pool_, other.pool_);
+    std::swap(block_, other.block_);
+    std::swap(size_, other.size_);
+  }
   void clear() {
     if (block_.p) pool_->give(block_);
     block_ = HostBlock();
@@ -319,71 +339,77 @@ struct PackHeader {
 // consecutive lanes; nothing else here is tuned.
 __global__ __launch_bounds__(kPackThreads) void pack_results(const int32_t* __restrict__ src, size_t n, uint32_t bits,
                                                              int32_t fill, uint8_t* __restrict__ out,
-                                                             PackHeader* __restrict__ headers) {
+                                                             PackHeader* __restrict__ headers, uint32_t n_chunks) {
   __shared__ __align__(16) uint8_t s_packed[kPackChunk * sizeof(int32_t)];
   __shared__ uint64_t s_live[kPackChunkGroups / 64];
   constexpr uint32_t kRounds = kPackChunkGroups / kPackThreads;
-  const size_t first = (size_t)blockIdx.x * kPackChunk;
   const uint32_t lane = threadIdx.x & 63u;
-  int32_t ids[kRounds][kPackGroup];
-  bool live[kRounds];
-  bool overflow = false;
+  for (uint32_t chunk = blockIdx.x; chunk < n_chunks; chunk += gridDim.x) {
+    const size_t first = (size_t)chunk * kPackChunk;
+    int32_t ids[kRounds][kPackGroup];
+    bool live[kRounds];
+    bool overflow = false;
 #pragma unroll
-  for (uint32_t r = 0; r < kRounds; ++r) {
-    const size_t at = first + (size_t)(r * kPackThreads + threadIdx.x) * kPackGroup;
-    if (at + kPackGroup <= n) {
-      const int4 lo = *reinterpret_cast<const int4*>(src + at), hi = *reinterpret_cast<const int4*>(src + at + 4);
-      ids[r][0] = lo.x; ids[r][1] = lo.y; ids[r][2] = lo.z; ids[r][3] = lo.w;
-      ids[r][4] = hi.x; ids[r][5] = hi.y; ids[r][6] = hi.z; ids[r][7] = hi.w;
-    } else {
+    for (uint32_t r = 0; r < kRounds; ++r) {
+      const size_t at = first + (size_t)(r * kPackThreads + threadIdx.x) * kPackGroup;
+      if (at + kPackGroup <= n) {
+        const int4 lo = *reinterpret_cast<const int4*>(src + at), hi = *reinterpret_cast<const int4*>(src + at + 4);
+        ids[r][0] = lo.x; ids[r][1] = lo.y; ids[r][2] = lo.z; ids[r][3] = lo.w;
+        ids[r][4] = hi.x; ids[r][5] = hi.y; ids[r][6] = hi.z; ids[r][7] = hi.w;
+      } else {
 #pragma unroll
-      for (uint32_t i = 0; i < kPackGroup; ++i) ids[r][i] = at + i < n ? src[at + i] : fill;
-    }
-    live[r] = false;
+        for (uint32_t i = 0; i < kPackGroup; ++i) ids[r][i] = at + i < n ? src[at + i] : fill;
+      }
+      live[r] = false;
 #pragma unroll
-    for (uint32_t i = 0; i < kPackGroup; ++i) live[r] = live[r] || ids[r][i] != fill;
-    const uint64_t mask = __ballot(live[r]);
-    if (lane == 0) s_live[(r * kPackThreads + threadIdx.x) / 64u] = mask;
-    if (bits < 32 && live[r]) {
+      for (uint32_t i = 0; i < kPackGroup; ++i) live[r] = live[r] || ids[r][i] != fill;
+      const uint64_t mask = __ballot(live[r]);
+      if (lane == 0) s_live[(r * kPackThreads + threadIdx.x) / 64u] = mask;
+      if (bits < 32 && live[r]) {
+        if (at + kPackGroup > n)  // what fills the last group up need not fit
 #pragma unroll
-      for (uint32_t i = 0; i < kPackGroup; ++i) overflow = overflow || ((uint32_t)ids[r][i] >> bits) != 0;
-    }
-  }
-  const int any_overflow = __syncthreads_or(overflow ? 1 : 0);
-  uint32_t total = 0;
+          for (uint32_t i = 0; i < kPackGroup; ++i) ids[r][i] = at + i < n ? ids[r][i] : 0;
 #pragma unroll
-  for (uint32_t r = 0; r < kRounds; ++r) {
-    const uint32_t word = (r * kPackThreads + threadIdx.x) / 64u;
-    uint32_t before = 0;
-    total = 0;
-    for (uint32_t w = 0; w < kPackChunkGroups / 64; ++w) {
-      const uint32_t here = (uint32_t)__popcll(s_live[w]);
-      if (w < word) before += here;
-      total += here;
-    }
-    if (!live[r]) continue;
-    before += (uint32_t)__popcll(s_live[word] & ((1ull << lane) - 1ull));
-    uint8_t* dst = s_packed + before * bits;
-    uint64_t acc = 0;
-    uint32_t held = 0;
-#pragma unroll
-    for (uint32_t i = 0; i < kPackGroup; ++i) {
-      acc |= (uint64_t)(uint32_t)ids[r][i] << held;
-      held += bits;
-      while (held >= 8) {
-        *dst++ = (uint8_t)acc;
-        acc >>= 8;
-        held -= 8;
+        for (uint32_t i = 0; i < kPackGroup; ++i) overflow = overflow || ((uint32_t)ids[r][i] >> bits) != 0;
       }
     }
+    const int any_overflow = __syncthreads_or(overflow ? 1 : 0);
+    uint32_t total = 0;
+#pragma unroll
+    for (uint32_t r = 0; r < kRounds; ++r) {
+      const uint32_t word = (r * kPackThreads + threadIdx.x) / 64u;
+      uint32_t before = 0;
+      total = 0;
+      for (uint32_t w = 0; w < kPackChunkGroups / 64; ++w) {
+        const uint32_t here = (uint32_t)__popcll(s_live[w]);
+        if (w < word) before += here;
+        total += here;
+      }
+      if (!live[r]) continue;
+      before += (uint32_t)__popcll(s_live[word] & ((1ull << lane) - 1ull));
+      uint8_t* dst = s_packed + before * bits;
+      uint64_t acc = 0;
+      uint32_t held = 0;
+#pragma unroll
+      for (uint32_t i = 0; i < kPackGroup; ++i) {
+        acc |= (uint64_t)(uint32_t)ids[r][i] << held;
+        held += bits;
+        while (held >= 8) {
+          *dst++ = (uint8_t)acc;
+          acc >>= 8;
+          held -= 8;
+        }
+      }
+    }
+    __syncthreads();
+    uint8_t* chunk_out = out + (size_t)chunk * kPackChunkGroups * bits;
+    const uint32_t words = (total * bits + 15u) / 16u;
+    for (uint32_t i = threadIdx.x; i < words; i += kPackThreads)
+      reinterpret_cast<uint4*>(chunk_out)[i] = reinterpret_cast<const uint4*>(s_packed)[i];
+    if (threadIdx.x < kPackChunkGroups / 64) headers[chunk].live[threadIdx.x] = s_live[threadIdx.x];
+    if (threadIdx.x == kPackChunkGroups / 64) headers[chunk].overflow = (uint64_t)any_overflow;
+    __syncthreads();  // the next chunk overwrites what has just been read
   }
-  __syncthreads();
-  uint8_t* chunk_out = out + (size_t)blockIdx.x * kPackChunkGroups * bits;
-  const uint32_t words = (total * bits + 15u) / 16u;
-  for (uint32_t i = threadIdx.x; i < words; i += kPackThreads)
-    reinterpret_cast<uint4*>(chunk_out)[i] = reinterpret_cast<const uint4*>(s_packed)[i];
-  if (threadIdx.x < kPackChunkGroups / 64) headers[blockIdx.x].live[threadIdx.x] = s_live[threadIdx.x];
-  if (threadIdx.x == kPackChunkGroups / 64) headers[blockIdx.x].overflow = (uint64_t)any_overflow;
 }
 
 // ---- unpacking -----------------------------------------------------------------------------
@@ -412,86 +438,110 @@ struct UnpackPlan {
 // Bytes the unpacking may read past the last group of a chunk.
 constexpr size_t kUnpackOverread = 32;
 
-inline void unpack_groups_plain(const UnpackPlan& plan, const uint8_t* src, int32_t* dst, size_t groups) {
-  for (size_t g = 0; g < groups; ++g, src += plan.bits, dst += kPackGroup) {
-    if (plan.bits > kPackMostBits) {
-      memcpy(dst, src, kPackGroup * sizeof(int32_t));
+// One chunk to dst (kPackChunk ids).
+inline void unpack_chunk_plain(const UnpackPlan& plan, const PackHeader& header, const uint8_t* src, int32_t fill,
+                               int32_t* dst) {
+  for (uint32_t g = 0; g < kPackChunkGroups; ++g, dst += kPackGroup) {
+    if (!(header.live[g / 64] >> (g % 64) & 1u)) {
+      std::fill_n(dst, kPackGroup, fill);
       continue;
     }
     for (uint32_t i = 0; i < kPackGroup; ++i) {
-      uint64_t word;
-      memcpy(&word, src + ((i * plan.bits) >> 3), sizeof(word));
+      uint64_t word = 0;
+      memcpy(&word, src + ((i * plan.bits) >> 3), plan.bits > kPackMostBits ? sizeof(uint32_t) : sizeof(word));
       dst[i] = (int32_t)((uint32_t)(word >> ((i * plan.bits) & 7u)) & plan.mask);
     }
+    src += plan.bits;
   }
 }
 
 #if defined(__x86_64__) && !defined(__HIP_DEVICE_COMPILE__)
-// Streaming stores (dst is a multiple of 32 bytes): the result is written once and read by nobody here, and a line
-// that is not fetched before it is overwritten is half the memory traffic.
-__attribute__((target("avx2"))) inline void unpack_groups_avx2(const UnpackPlan& plan, const uint8_t* src, int32_t* dst,
-                                                               size_t groups) {
-  if (plan.bits > kPackMostBits) {
-    for (size_t g = 0; g < groups; ++g)
-      _mm256_stream_si256((__m256i*)(dst + g * kPackGroup), _mm256_loadu_si256((const __m256i*)(src + g * 32)));
-    return;
-  }
+// The same with dst a multiple of 32 bytes.  Streaming stores: the result is written once and read by nobody here, and
+// a line that is not fetched before it is overwritten is half the memory traffic.  Words of 64 live groups, and of 64
+// dead ones, have loops of their own; in a mixed word every group is unpacked from where the next live one
+// starts and replaced by `fill` if it is not live itself - no branch to mispredict where walks end at random.
+// Eight threads: 200 GB/s of ids (76-100 with a call for every run of groups of one kind).
+__attribute__((target("avx2"))) inline void unpack_chunk_avx2(const UnpackPlan& plan, const PackHeader& header,
+                                                              const uint8_t* src, int32_t fill, int32_t* dst) {
+  const bool whole = plan.bits > kPackMostBits;
+  const size_t bits = plan.bits;
   const __m256i shuffle = _mm256_loadu_si256((const __m256i*)plan.shuffle);
   const __m256i shift = _mm256_loadu_si256((const __m256i*)plan.shift);
-  const __m256i mask = _mm256_set1_epi32((int)plan.mask);
-  for (size_t g = 0; g < groups; ++g, src += plan.bits) {
-    const __m128i lo = _mm_loadu_si128((const __m128i*)src);
-    const __m128i hi = _mm_loadu_si128((const __m128i*)(src + plan.high_at));
-    const __m256i both = _mm256_inserti128_si256(_mm256_castsi128_si256(lo), hi, 1);
-    const __m256i ids = _mm256_and_si256(_mm256_srlv_epi32(_mm256_shuffle_epi8(both, shuffle), shift), mask);
-    _mm256_stream_si256((__m256i*)(dst + g * kPackGroup), ids);
+  const __m256i mask = _mm256_set1_epi32((int)plan.mask), dead = _mm256_set1_epi32(fill);
+  const size_t high_at = plan.high_at;
+#define ND_UNPACKED_GROUP                                                                                          \
+  _mm256_and_si256(                                                                                                \
+      _mm256_srlv_epi32(_mm256_shuffle_epi8(_mm256_inserti128_si256(                                               \
+                                                _mm256_castsi128_si256(_mm_loadu_si128((const __m128i*)src)),      \
+                                                _mm_loadu_si128((const __m128i*)(src + high_at)), 1),              \
+                                            shuffle),                                                              \
+                        shift),                                                                                    \
+      mask)
+  for (uint32_t w = 0; w < kPackChunkGroups / 64; ++w) {
+    uint64_t live = header.live[w];
+    if (live == 0) {
+      for (uint32_t g = 0; g < 64; ++g, dst += kPackGroup) _mm256_stream_si256((__m256i*)dst, dead);
+    } else if (whole) {
+      for (uint32_t g = 0; g < 64; ++g, dst += kPackGroup, live >>= 1) {
+        const __m256i here = _mm256_set1_epi32(-(int)(live & 1u));
+        _mm256_stream_si256((__m256i*)dst, _mm256_blendv_epi8(dead, _mm256_loadu_si256((const __m256i*)src), here));
+        src += bits & (0 - (size_t)(live & 1u));
+      }
+    } else if (~live == 0) {
+      for (uint32_t g = 0; g < 64; ++g, dst += kPackGroup, src += bits)
+        _mm256_stream_si256((__m256i*)dst, ND_UNPACKED_GROUP);
+    } else {
+      for (uint32_t g = 0; g < 64; ++g, dst += kPackGroup, live >>= 1) {
+        const __m256i here = _mm256_set1_epi32(-(int)(live & 1u));
+        _mm256_stream_si256((__m256i*)dst, _mm256_blendv_epi8(dead, ND_UNPACKED_GROUP, here));
+        src += bits & (0 - (size_t)(live & 1u));
+      }
+    }
   }
-}
-__attribute__((target("avx2"))) inline void fill_groups_avx2(int32_t fill, int32_t* dst, size_t groups) {
-  const __m256i ids = _mm256_set1_epi32(fill);
-  for (size_t g = 0; g < groups; ++g) _mm256_stream_si256((__m256i*)(dst + g * kPackGroup), ids);
+#undef ND_UNPACKED_GROUP
 }
 inline bool unpack_has_avx2() { return __builtin_cpu_supports("avx2"); }
 inline void unpack_fence() { _mm_sfence(); }
 inline void spin_pause() { _mm_pause(); }
 #else
-inline void unpack_groups_avx2(const UnpackPlan&, const uint8_t*, int32_t*, size_t) {}
-inline void fill_groups_avx2(int32_t, int32_t*, size_t) {}
+inline void unpack_chunk_avx2(const UnpackPlan&, const PackHeader&, const uint8_t*, int32_t, int32_t*) {}
 inline bool unpack_has_avx2() { return false; }
 inline void unpack_fence() {}
 inline void spin_pause() {}
 #endif
 
-// One chunk: count ids (at most kPackChunk) to dst.
+// The first count ids (at most kPackChunk) of a chunk to dst.
 inline void unpack_chunk(const UnpackPlan& plan, const PackHeader& header, const uint8_t* src, int32_t fill,
                          int32_t* dst, size_t count) {
-  alignas(32) int32_t whole[kPackChunk];
-  const bool direct = count == kPackChunk;
-  int32_t* at = direct ? dst : whole;
-  const bool streams = ((uintptr_t)at & 31u) == 0 && unpack_has_avx2();
-  for (uint32_t w = 0; w < kPackChunkGroups / 64; ++w) {
-    uint64_t live = header.live[w];
-    for (uint32_t g = 0; g < 64;) {
-      // a run of groups of one kind
-      const bool is_live = live & 1u;
-      const uint64_t ends = is_live ? ~live : live;
-      uint32_t run = ends ? (uint32_t)__builtin_ctzll(ends) : 64u;
-      run = std::min(run, 64u - g);
-      if (is_live) {
-        if (streams) unpack_groups_avx2(plan, src, at, run);
-        else unpack_groups_plain(plan, src, at, run);
-        src += (size_t)run * plan.bits;
-      } else if (streams) {
-        fill_groups_avx2(fill, at, run);
-      } else {
-        std::fill_n(at, (size_t)run * kPackGroup, fill);
-      }
-      at += (size_t)run * kPackGroup;
-      g += run;
-      live = run < 64 ? live >> run : 0;
+  alignas(32) int32_t part[kPackChunk];
+  int32_t* at = count == kPackChunk ? dst : part;
+  if (((uintptr_t)at & 31u) == 0 && unpack_has_avx2()) unpack_chunk_avx2(plan, header, src, fill, at);
+  else unpack_chunk_plain(plan, header, src, fill, at);
+  if (at == part) memcpy(dst, part, count * sizeof(int32_t));
+}
+
+// The stream results cross the bus on while something else is computed: one per device and process, on a hardware
+// queue of its own, which a stream with a mask of compute units (here: all) gets.  (Ordinary streams share four;
+// where the computation's lands on the same one, nothing overlaps.)
+inline hipStream_t transfer_stream() {
+  static std::mutex mutex;
+  static std::vector<hipStream_t>* streams = new std::vector<hipStream_t>;
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess) return nullptr;
+  std::lock_guard<std::mutex> lock(mutex);
+  if (streams->size() <= (size_t)device) streams->resize((size_t)device + 1, nullptr);
+  hipStream_t& stream = (*streams)[(size_t)device];
+  if (!stream) {
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus <= 0) return nullptr;
+    std::vector<uint32_t> every_cu((size_t)(cus + 31) / 32, 0xffffffffu);
+    if (cus % 32 != 0) every_cu.back() = (1u << (cus % 32)) - 1u;
+    if (hipExtStreamCreateWithCUMask(&stream, (uint32_t)every_cu.size(), every_cu.data()) != hipSuccess) {
+      (void)hipGetLastError();
+      stream = nullptr;
     }
   }
-  if (!direct) memcpy(dst, whole, count * sizeof(int32_t));
+  return stream;
 }
 
 // ---- the stream ----------------------------------------------------------------------------
@@ -504,46 +554,102 @@ class ResultStream {
   ResultStream& operator=(const ResultStream&) = delete;
   ~ResultStream() { release(); }
 
+  // The first `words` words of a result are on the device once `event` has happened.
+  struct Ready {
+    size_t words;
+    hipEvent_t event;
+  };
+
   // n words at src (aligned to 16 bytes) to dst, in stream order.  Words that are `fill` in groups of eight cost
   // nothing; words are expected to fit `bits` bits (one that does not makes the whole transfer start again with
   // 32).  Large transfers only: it pays from a few megabytes on.
   hipError_t fetch(const int32_t* src, size_t n, uint32_t bits, int32_t fill, int32_t* dst, hipStream_t stream) {
-    if (bits > kPackMostBits) bits = 32;
-    bool overflow = false;
-    hipError_t e = transfer(src, n, bits, fill, dst, stream, &overflow);
-    if (e == hipSuccess && overflow) e = transfer(src, n, 32, fill, dst, stream, &overflow);
-    return e;
+    const hipError_t e = begin(src, n, bits, fill, dst, stream, {});
+    return e == hipSuccess ? finish() : e;
   }
 
-  void release() {
-    for (Slot& s : slots_) {
-      if (s.done) (void)hipEventDestroy(s.done);
-      s.done = nullptr;
+  // The same as a begin() that returns at once, other threads taking it from there, and a finish() that takes part
+  // and returns when the words are at dst.  `ready` (words ascending, the last n): what has to have
+  // happened before words may be read, while other work of the caller's is still going on; empty: stream order.  What is given has to stay until finish().
+  hipError_t begin(const int32_t* src, size_t n, uint32_t bits, int32_t fill, int32_t* dst, hipStream_t stream,
+                   std::vector<Ready> ready) {
+    hipError_t e = finish();  // an earlier one that nobody waited for
+    if (e != hipSuccess || n == 0) return e;
+    if (!transfer_) transfer_.reset(new Transfer);
+    Transfer& t = *transfer_;
+    e = hipGetDevice(&t.device);
+    if (e != hipSuccess) return e;
+    t.set(src, n, bits > kPackMostBits ? 32 : bits, fill, dst, std::move(ready));
+    e = prepare(t.slot_bytes);
+    if (e != hipSuccess) return e;
+    t.streams[0] = t.streams[1] = transfer_stream();
+    if (t.ready.empty()) {
+      // pieces alternate between two streams, so that the bus is not idle between two launches
+      t.streams[0] = stream;
+      e = hipEventRecord(begun_, stream);
+      if (e == hipSuccess) e = hipStreamWaitEvent(t.streams[1], begun_, 0);
+      if (e != hipSuccess) return e;
     }
+    job_.body = [this] { take_part(); };
+    under_way_ = true;
+    HostWorkers::get().start(job_, HostWorkers::kMost);
+    return hipSuccess;
+  }
+
+  hipError_t finish() {
+    if (!under_way_) return hipSuccess;
+    Transfer& t = *transfer_;
+    take_part();
+    HostWorkers::get().join(job_);
+    under_way_ = false;
+    if (t.error != hipSuccess) {
+      for (hipStream_t s : t.streams) (void)hipStreamSynchronize(s);  // nothing writes to the ring after this
+      return t.error;
+    }
+    if (!t.overflow.load()) return hipSuccess;
+    misfit_ = true;
+    return fetch(t.src, t.n, 32, t.fill, t.dst, t.streams[0]);
+  }
+
+  // whether a word has ever not fitted
+  bool misfit() const { return misfit_; }
+
+  void release() {
+    (void)finish();
+    for (hipEvent_t& ev : packed_)
+      if (ev) (void)hipEventDestroy(ev), ev = nullptr;
+    if (begun_) (void)hipEventDestroy(begun_);
+    begun_ = nullptr;
     if (ring_) (void)hipHostFree(ring_);
     ring_ = nullptr;
     ring_bytes_ = 0;
   }
 
  private:
-  static constexpr int kSlots = 8;
+  static constexpr size_t kSlots = 8;
   // Chunks of a piece: at most 8 MB of results (0.1 ms on the bus, long against a launch and an event; with pieces of
   // 16 MB the ring no longer stays in the last-level cache between the bus and the threads: 1.68 GB in 16 instead of 14
-  // ms), at least 1 MB, else a sixth of the whole (23 MB: 265 us, with a sixteenth 352).
-  static constexpr size_t kMostChunks = 512, kLeastChunks = 64, kPieces = 6;
-  static constexpr size_t kChunksAtOnce = 4;  // what a thread takes
+  // ms).  The first one is 1 MB and each of the next twice as long, so that the threads have something to do soon, and
+  // none is more than a third of what is left, so that little is left to do when the last one arrives.
+  static constexpr size_t kMostChunks = 512, kLeastChunks = 64;
+  static constexpr size_t kChunksAtOnce = 4;  // what a thread takes; kLeastChunks is a multiple
+  // Workgroups of a launch of pack_results, and launches under way, while something else is computed: stores that wait
+  // for the bus stand in the way of that something's own.  R-MAT 22 walks in four ranges, sampling / with their
+  // rows here: 512 workgroups 34.1 / 38.6 ms, 64 30.5 / 35.2, 48 29.0 / 33.1, 32 26.9 / 31.0, 24 26.9 / 32.2.
+  static constexpr uint32_t kGentleBlocks = 32;
+  static constexpr size_t kGentleAhead = 2;
   static constexpr int kSpins = 4000;  // tens of microseconds; none: 1.68 GB in 19 instead of 13 ms, 23 MB in 527 instead of 290 us
 
-  struct Slot {
-    hipEvent_t done = nullptr;
-  };
-
   hipError_t prepare(size_t slot_bytes) {
-    for (Slot& s : slots_)
-      if (!s.done) {
-        const hipError_t e = hipEventCreateWithFlags(&s.done, hipEventDisableTiming | hipEventReleaseToSystem);
+    for (hipEvent_t& ev : packed_)
+      if (!ev) {
+        const hipError_t e = hipEventCreateWithFlags(&ev, hipEventDisableTiming | hipEventReleaseToSystem);
         if (e != hipSuccess) return e;
       }
+    if (!begun_) {
+      const hipError_t e = hipEventCreateWithFlags(&begun_, hipEventDisableTiming);
+      if (e != hipSuccess) return e;
+    }
     if (ring_bytes_ >= slot_bytes * kSlots) return hipSuccess;
     if (ring_) (void)hipHostFree(ring_);
     ring_ = nullptr;
@@ -553,131 +659,187 @@ class ResultStream {
     return e;
   }
 
-  hipError_t transfer(const int32_t* src, size_t n, uint32_t bits, int32_t fill, int32_t* dst, hipStream_t stream,
-                      bool* overflow) {
-    *overflow = false;
-    if (n == 0) return hipSuccess;
-    const size_t chunks = (n + kPackChunk - 1) / kPackChunk;
-    size_t per_piece = (chunks + kPieces - 1) / kPieces;
-    per_piece = std::min(kMostChunks, std::max(kLeastChunks, per_piece));
-    per_piece = (per_piece + kChunksAtOnce - 1) / kChunksAtOnce * kChunksAtOnce;
-    const size_t pieces = (chunks + per_piece - 1) / per_piece;
-    const size_t chunk_bytes = (size_t)kPackChunkGroups * bits;
-    const size_t packed_at = sizeof(PackHeader) * per_piece;
-    const size_t slot_bytes = (packed_at + chunk_bytes * per_piece + kUnpackOverread + 255) / 256 * 256;
-    hipError_t error = prepare(slot_bytes);
-    if (error != hipSuccess) return error;
-    const UnpackPlan plan(bits);
+  struct Transfer {
+    const int32_t* src;
+    size_t n;
+    uint32_t bits;
+    int32_t fill;
+    int32_t* dst;
+    hipStream_t streams[2];
+    std::vector<Ready> ready;
+    int device = 0;
 
-    struct Shared {
-      std::atomic<size_t> next{0};       // chunk to take
-      std::atomic<size_t> arrived{0};    // pieces whose bytes are here
-      std::atomic<bool> stop{false}, overflow{false};
-      std::mutex mutex;
-      std::condition_variable more;
-      unsigned sleepers = 0;
-    } shared;
+    size_t chunks, pieces, chunk_bytes, packed_at, slot_bytes;
+    std::vector<size_t> begins;        // first chunk of every piece, and the end of the last
+    std::vector<uint32_t> piece_of;    // of every kLeastChunks chunks
+    size_t happened;                   // of `ready`
+    UnpackPlan plan{32};
+    std::atomic<bool> driven{false};   // a thread has taken the launching on
+    std::atomic<size_t> next{0};       // chunk to take
+    std::atomic<size_t> arrived{0};    // pieces whose bytes are here
+    std::atomic<bool> stop{false}, overflow{false};
+    hipError_t error = hipSuccess;     // the driving thread's
+    std::mutex mutex;
+    std::condition_variable more;
+    unsigned sleepers = 0;
+    std::vector<std::atomic<size_t>> left;  // chunks of a piece that are not unpacked yet
+
+    void set(const int32_t* src_, size_t n_, uint32_t bits_, int32_t fill_, int32_t* dst_, std::vector<Ready> ready_) {
+      src = src_, n = n_, bits = bits_, fill = fill_, dst = dst_, ready = std::move(ready_);
+      happened = 0;
+      chunks = (n + kPackChunk - 1) / kPackChunk;
+      begins.clear();
+      piece_of.clear();
+      size_t most = kLeastChunks, longest = 0;
+      for (size_t at = 0; at < chunks; most = std::min(kMostChunks, most * 2)) {
+        const size_t third = ((chunks - at) / 3 + kLeastChunks - 1) / kLeastChunks * kLeastChunks;
+        const size_t here = std::max(kLeastChunks, std::min(most, third));
+        piece_of.insert(piece_of.end(), here / kLeastChunks, (uint32_t)begins.size());
+        begins.push_back(at);
+        longest = std::max(longest, here);
+        at += here;
+      }
+      pieces = begins.size();
+      begins.push_back(chunks);
+      chunk_bytes = (size_t)kPackChunkGroups * bits;
+      packed_at = sizeof(PackHeader) * longest;
+      slot_bytes = (packed_at + chunk_bytes * longest + kUnpackOverread + 255) / 256 * 256;
+      plan = UnpackPlan(bits);
+      driven = false, next = 0, arrived = 0, stop = false, overflow = false, error = hipSuccess;
+      left = std::vector<std::atomic<size_t>>(pieces);
+      for (size_t p = 0; p < pieces; ++p) left[p].store(begins[p + 1] - begins[p]);
+    }
+
     // A piece comes every 20-200 us: worth a short wait awake (a thread that sleeps is back 50 us later, and
     // waking all of them costs the driving thread as much), but not more than that.
-    auto await = [&](size_t piece) {
+    void await(size_t piece) {
       for (int spin = 0; spin < kSpins; ++spin) {
-        if (shared.arrived.load(std::memory_order_acquire) > piece || shared.stop.load()) return;
+        if (arrived.load(std::memory_order_acquire) > piece || stop.load()) return;
         spin_pause();
       }
-      std::unique_lock<std::mutex> lock(shared.mutex);
-      shared.sleepers++;
-      shared.more.wait(lock, [&] { return shared.arrived.load(std::memory_order_acquire) > piece || shared.stop.load(); });
-      shared.sleepers--;
-    };
-    auto announce = [&](size_t arrived, bool stop) {
+      std::unique_lock<std::mutex> lock(mutex);
+      sleepers++;
+      more.wait(lock, [&] { return arrived.load(std::memory_order_acquire) > piece || stop.load(); });
+      sleepers--;
+    }
+    void announce(size_t pieces_here, bool stops) {
       bool asleep;
       {
-        std::lock_guard<std::mutex> lock(shared.mutex);
-        if (stop) shared.stop.store(true);
-        else shared.arrived.store(arrived, std::memory_order_release);
-        asleep = shared.sleepers > 0;
+        std::lock_guard<std::mutex> lock(mutex);
+        if (stops) stop.store(true);
+        else arrived.store(pieces_here, std::memory_order_release);
+        asleep = sleepers > 0;
       }
-      if (asleep) shared.more.notify_all();
-    };
-    std::vector<std::atomic<size_t>> left(pieces);  // chunks of a piece that are not unpacked yet
-    for (size_t p = 0; p < pieces; ++p) left[p].store(std::min(per_piece, chunks - p * per_piece));
-
-    auto slot = [&](size_t piece) { return ring_ + (piece % kSlots) * slot_bytes; };
-    auto launch = [&](size_t piece) -> hipError_t {
-      const size_t first = piece * per_piece * kPackChunk;
-      const size_t here = std::min(n - first, per_piece * kPackChunk);
-      uint8_t* at = slot(piece);
-      pack_results<<<dim3((unsigned)((here + kPackChunk - 1) / kPackChunk)), dim3(kPackThreads), 0, stream>>>(
-          src + first, here, bits, fill, at + packed_at, (PackHeader*)at);
-      const hipError_t e = hipGetLastError();
-      return e != hipSuccess ? e : hipEventRecord(slots_[piece % kSlots].done, stream);
-    };
-    // unpacks the chunks [c, end) of a piece that is here
-    auto unpack = [&](size_t c, size_t end) {
-      const size_t piece = c / per_piece;
-      const uint8_t* at = slot(piece);
-      for (size_t i = c; i < end; ++i) {
-        const size_t in_piece = i - piece * per_piece;
-        const PackHeader& header = ((const PackHeader*)at)[in_piece];
-        if (header.overflow) shared.overflow.store(true, std::memory_order_relaxed);
-        const size_t first = i * kPackChunk;
-        unpack_chunk(plan, header, at + packed_at + in_piece * chunk_bytes, fill, dst + first,
-                     std::min<size_t>(kPackChunk, n - first));
-      }
-      unpack_fence();
-      left[piece].fetch_sub(end - c, std::memory_order_release);
-    };
-    auto work = [&] {
-      for (;;) {
-        const size_t c = shared.next.fetch_add(kChunksAtOnce);
-        if (c >= chunks) return;
-        const size_t piece = c / per_piece;
-        await(piece);
-        if (shared.stop.load()) return;
-        unpack(c, std::min(c + kChunksAtOnce, std::min(chunks, (piece + 1) * per_piece)));
-      }
-    };
-    auto drive = [&] {
-      size_t launched = 0;
-      for (; launched < pieces && launched < kSlots && error == hipSuccess; ++launched) error = launch(launched);
-      for (size_t p = 0; p < pieces && error == hipSuccess; ++p) {
-        // the slot of piece p - 1 is free for piece p - 1 + kSlots once it is unpacked; kSlots - 1 pieces are
-        // under way meanwhile
-        if (p > 0 && launched < pieces) {
-          while (left[p - 1].load(std::memory_order_acquire) != 0) {
-            const size_t c = shared.next.load();
-            size_t mine = c;
-            if (c < p * per_piece && shared.next.compare_exchange_strong(mine, c + kChunksAtOnce))
-              unpack(c, std::min(c + kChunksAtOnce, std::min(chunks, (c / per_piece + 1) * per_piece)));
-            else
-              std::this_thread::yield();
-          }
-          error = launch(launched);
-          if (error != hipSuccess) break;
-          launched++;
-        }
-        error = hipEventSynchronize(slots_[p % kSlots].done);
-        if (error != hipSuccess) break;
-        announce(p + 1, false);
-      }
-      if (error != hipSuccess) {
-        announce(0, true);
-        return;
-      }
-      work();
-    };
-    HostWorkers::get().run(HostWorkers::kMost, work, drive);
-    if (error != hipSuccess) {
-      (void)hipStreamSynchronize(stream);  // nothing writes to the ring after this
-      return error;
+      if (asleep) more.notify_all();
     }
-    *overflow = shared.overflow.load();
-    return hipSuccess;
+  };
+
+  uint8_t* slot(size_t piece) const { return ring_ + (piece % kSlots) * transfer_->slot_bytes; }
+  size_t piece_end(size_t piece) const {
+    return std::min(transfer_->n, transfer_->begins[piece + 1] * kPackChunk);
   }
 
+  // Whether piece may be read, or, with `waits`, until it may.
+  bool readable(size_t piece, bool waits, hipError_t* error) {
+    Transfer& t = *transfer_;
+    while (t.happened < t.ready.size() && (t.happened == 0 || t.ready[t.happened - 1].words < piece_end(piece))) {
+      const hipEvent_t ev = t.ready[t.happened].event;
+      const hipError_t e = waits ? hipEventSynchronize(ev) : hipEventQuery(ev);
+      if (e == hipErrorNotReady) return false;
+      if (e != hipSuccess) {
+        *error = e;
+        return false;
+      }
+      t.happened++;
+    }
+    return true;
+  }
+
+  // Whether nothing is being computed any more that the transfer could be in the way of.
+  bool alone() const {
+    const Transfer& t = *transfer_;
+    return t.happened == t.ready.size() || hipEventQuery(t.ready.back().event) == hipSuccess;
+  }
+
+  hipError_t launch(size_t piece, bool gently) {
+    const Transfer& t = *transfer_;
+    const size_t first = t.begins[piece] * kPackChunk;
+    const size_t here = piece_end(piece) - first;
+    uint8_t* at = slot(piece);
+    const uint32_t n_chunks = (uint32_t)((here + kPackChunk - 1) / kPackChunk);
+    const hipStream_t stream = t.streams[piece % 2];
+    pack_results<<<dim3(gently ? std::min(n_chunks, kGentleBlocks) : n_chunks), dim3(kPackThreads), 0, stream>>>(
+        t.src + first, here, t.bits, t.fill, at + t.packed_at, (PackHeader*)at, n_chunks);
+    const hipError_t e = hipGetLastError();
+    return e != hipSuccess ? e : hipEventRecord(packed_[piece % kSlots], stream);
+  }
+
+  // unpacks the chunks [c, end) of a piece that is here
+  void unpack(size_t c, size_t end) {
+    Transfer& t = *transfer_;
+    const size_t piece = t.piece_of[c / kLeastChunks];
+    const uint8_t* at = slot(piece);
+    for (size_t i = c; i < end; ++i) {
+      const size_t in_piece = i - t.begins[piece];
+      const PackHeader& header = ((const PackHeader*)at)[in_piece];
+      if (header.overflow) t.overflow.store(true, std::memory_order_relaxed);
+      const size_t first = i * kPackChunk;
+      unpack_chunk(t.plan, header, at + t.packed_at + in_piece * t.chunk_bytes, t.fill, t.dst + first,
+                   std::min<size_t>(kPackChunk, t.n - first));
+    }
+    unpack_fence();
+    t.left[piece].fetch_sub(end - c, std::memory_order_release);
+  }
+
+  void take_part() {
+    Transfer& t = *transfer_;
+    if (!t.driven.exchange(true)) drive();
+    for (;;) {
+      const size_t c = t.next.fetch_add(kChunksAtOnce);
+      if (c >= t.chunks) return;
+      const size_t piece = t.piece_of[c / kLeastChunks];
+      t.await(piece);
+      if (t.stop.load()) return;
+      unpack(c, std::min(c + kChunksAtOnce, t.chunks));
+    }
+  }
+
+  // Launches the packing of pieces, up to kSlots of them under way at a time, and announces them as they arrive.
+  void drive() {
+    Transfer& t = *transfer_;
+    hipError_t error = hipSetDevice(t.device);  // a worker's device is whatever it served last
+    size_t launched = 0;
+    bool gently = true;
+    for (size_t p = 0; p < t.pieces && error == hipSuccess; ++p) {
+      while (launched < t.pieces && error == hipSuccess && readable(launched, /*waits=*/launched == p, &error)) {
+        gently = gently && !alone();
+        if (launched >= p + (gently ? kGentleAhead : kSlots)) break;
+        // its slot is free once the piece before it there is unpacked
+        while (launched >= kSlots && t.left[launched - kSlots].load(std::memory_order_acquire) != 0) {
+          const size_t c = t.next.load();
+          size_t mine = c;
+          if (c < t.begins[p] && t.next.compare_exchange_strong(mine, c + kChunksAtOnce))
+            unpack(c, std::min(c + kChunksAtOnce, t.chunks));
+          else
+            std::this_thread::yield();
+        }
+        error = launch(launched++, gently);
+      }
+      if (error == hipSuccess) error = hipEventSynchronize(packed_[p % kSlots]);
+      if (error == hipSuccess) t.announce(p + 1, false);
+    }
+    if (error != hipSuccess) {
+      t.error = error;
+      t.announce(0, true);
+    }
+  }
+
+  std::unique_ptr<Transfer> transfer_;
+  HostWorkers::Job job_;
+  bool under_way_ = false, misfit_ = false;
   uint8_t* ring_ = nullptr;
   size_t ring_bytes_ = 0;
-  Slot slots_[kSlots];
+  hipEvent_t packed_[kSlots] = {}, begun_ = nullptr;
 };
 
 }  // namespace nd

@@ -1456,7 +1456,7 @@ class LayerEngine : public EngineBase {
   int fetch_sample_states(void* dst, size_t bytes) override {
     if (!allocated_ || std::is_empty<SampleType>::value) { last_error = "no sample state"; return -1; }
     if (bytes != sample_state_bytes()) { last_error = "sample state size mismatch"; return -1; }
-    return fetch_to_host(dst, d_samples_, bytes, 32, 0, stream_);
+    return states_to_host(dst, d_samples_, bytes, stream_);
   }
 
   int distinct() override {

@@ -90,6 +90,13 @@ class ShardedEngine : public EngineBase {
       p->launch_graph = launch_graph;
       p->profiling = profiling;
     }
+    // A caller who took the last pass's rows, array and all, is expected to take this one's as well.
+    parts_[0]->rows_ahead = nullptr;
+    if (parts_.size() == 1 && parts_[0]->is_walk() && rows_fetched_ && hFinalSamples.taken()) {
+      rows_ahead_.resize(hFinalSamples.size());
+      parts_[0]->rows_ahead = rows_ahead_.data();
+    }
+    rows_fetched_ = false;
     times = PhaseTimes();
     const auto t0 = std::chrono::steady_clock::now();
     std::vector<int> rc(parts_.size(), 0);
@@ -123,6 +130,17 @@ class ShardedEngine : public EngineBase {
 
   int fetch_final_samples() override {
     size_t at = 0;
+    rows_fetched_ = true;
+    if (parts_.size() == 1 && parts_[0]->rows_are_ahead()) {
+      if (parts_[0]->finish_rows_ahead() != 0) return fail(0);
+      hFinalSamples.swap(rows_ahead_);
+      rows_ahead_.clear();
+      return 0;
+    }
+    if (!rows_ahead_.empty()) {  // taken for a pass that did without
+      hFinalSamples.swap(rows_ahead_);
+      rows_ahead_.clear();
+    }
     if (num_samples() > 0) hFinalSamples.resize((size_t)num_samples() * (size_t)final_sample_size());
     for (size_t i = 0; i < parts_.size(); ++i) {
       if (parts_[i]->fetch_final_samples_into(hFinalSamples.data() + at) != 0) return fail((int)i);
@@ -174,6 +192,8 @@ class ShardedEngine : public EngineBase {
 
   const char* name_;
   const CSR* graph_ = nullptr;
+  HostArray<VertexID_t> rows_ahead_{host_pool};  // of a pass whose rows are on their way while it runs
+  bool rows_fetched_ = false;                    // since the last pass
   std::vector<std::unique_ptr<Part>> parts_;
 };
 

@@ -445,7 +445,7 @@ class SubgraphEngine : public EngineBase {
   int fetch_sample_states(void* dst, size_t bytes) override {
     if (!allocated_) { last_error = "no device data"; return -1; }
     if (bytes != sample_state_bytes()) { last_error = "sample state buffer has the wrong size"; return -2; }
-    return fetch_to_host(dst, d_stored_, bytes, 32, 0, stream_);
+    return states_to_host(dst, d_stored_, bytes, stream_);
   }
 
   bool lists_edges() const override { return true; }

@@ -39,3 +39,33 @@ def test_arrays_stay_the_callers(oracle, n):
     s.close()
     for turn, got in held:
         assert np.all(got == -turn)
+
+
+# fewer walks than are split into ranges, two ranges, and more than the device holds at once
+@pytest.mark.parametrize("n", [98303, 196609, 1000003])
+def test_rows_that_leave_before_the_pass_is_over(oracle, n):
+    g = graphs.random_graph(n=n, mean_degree=4, seed=n, isolated_every=3)
+    s = nd.Sampler("UniformRandomWalk8", g, seed=42)
+    d = oracle.app_desc(oracle.UNIFORM_WALK, s.steps, [s.step_size(k) for k in range(s.steps)])
+    want, _ = oracle.sample_individual(graphs.oracle_view(g), d, 42, s.initial_contents)
+    step = lambda name: print("n", n, name, flush=True)
+    rows = []
+    for turn in range(3):  # from the second pass on the engine expects the rows to be fetched
+        step("pass")
+        s.do_transit_parallel()
+        rows.append(s.final_samples())
+        assert np.array_equal(rows[-1], want)
+    step("a pass whose rows nobody fetches, and one more")
+    s.do_transit_parallel()
+    s.do_transit_parallel()
+    assert np.array_equal(s.final_samples(), want)
+    assert all(np.array_equal(r, want) for r in rows)
+    step("rows changed after the pass")
+    s.do_transit_parallel()
+    s.distinct()
+    changed = s.final_samples()
+    assert np.array_equal(changed, want)  # one id a segment: each is distinct
+    step("closed with rows on their way")
+    s.do_transit_parallel()
+    s.close()
+    assert all(np.array_equal(r, want) for r in rows)
