@@ -48,17 +48,9 @@
 #include "nd_device_graph.hpp"
 #include "nd_engine.hpp"
 #include "nd_radix_sort.hpp"
+#include "nd_union_sums.hpp"
 
 namespace nd {
-
-constexpr uint32_t kMaxLayerTransits = 1024;  // transits of one sample the build kernel stages in LDS
-
-// transits of sample s: base[s * stride + i], i < count
-struct TransitView {
-  const int32_t* base;
-  uint32_t stride;
-  uint32_t count;
-};
 
 // One wave per sample: sum of the degrees of its valid transits.
 __global__ __launch_bounds__(256) void collective_sizes(CSRPartition csr, TransitView tv, uint32_t n_samples,
@@ -314,7 +306,6 @@ constexpr uint32_t kBinVerticesSums = 7168;   // LADIES form: 56 KB of 64-bit su
 constexpr uint32_t kDensePieceEntries = 1024;
 constexpr uint32_t kDensePieceEntriesSums = 2048;  // LADIES form: a piece is 7168 64-bit sums
 constexpr size_t kDensePieceBudgetBytes = (size_t)2 << 30;
-constexpr uint32_t kNoPiece = 0xFFFFFFFFu;
 struct DensePieces {
   const int32_t* hub_row = nullptr;  // nullptr: the graph has none
   const uint32_t* piece_of = nullptr;
@@ -823,143 +814,6 @@ __global__ __launch_bounds__(kBinThreads, 8) __attribute__((amdgpu_num_vgpr(56))
   }
 }
 
-// ---- FastGCN form: the marked vertices of a sample weighted by degree^2, without a list ----
-//
-// The app draws "the first marked vertex, ascending, whose running sum of degree^2 exceeds a
-// target".  Listing the marked vertices with their running sums costs 20 bytes for each of
-// the 2.0e9 distinct pairs of a full-size pass; instead the bitmap is kept and summed at two
-// levels - groups of 256 vertices (8 words) and parts of 64 groups - so that a draw searches
-// the parts of its sample, then the groups of one part, then walks one group's set bits.
-constexpr uint32_t kGroupWords = 8;
-constexpr uint32_t kGroupsPerPart = 64;
-constexpr uint32_t kPartWords = kGroupWords * kGroupsPerPart;  // 16384 vertices
-
-// The degrees of a part's 16,384 vertices do not depend on the sample, so a workgroup keeps
-// them in LDS and runs its samples past them: fetching the row extents of every marked vertex
-// of every sample from the caches instead (2.0e9 gathers a pass at full size, a lane waiting
-// for each) took as long as the marking itself.
-constexpr uint32_t kSumThreads = 1024;
-constexpr uint32_t kSumSamplesPerBlock = 128;
-constexpr uint32_t kGroupVertices = kGroupWords * 32u;
-constexpr uint32_t kGroupPitch = kGroupVertices + 1u;  // lanes walk different groups: the odd pitch spreads them over the banks
-
-// One workgroup per (part, block of 128 samples), a wavefront per sample, a lane per group:
-// group_through[(s * parts + part) * 64 + g] = degree^2 of the marked vertices of groups 0..g
-// of the part; part_total[s * parts + part]; marked[s] += marked vertices.  Workgroups of the
-// low parts (where the hubs of a skewed graph sit, marked in nearly every sample) come first.
-__global__ __launch_bounds__(kSumThreads) void bitmap_group_sums(const uint32_t* __restrict__ bitmap,
-                                                                 uint32_t words_per_sample, uint32_t n_samples,
-                                                                 uint32_t n_vertices,
-                                                                 const EdgePos_t* __restrict__ row_ptr,
-                                                                 uint64_t* __restrict__ group_through,
-                                                                 uint64_t* __restrict__ part_total,
-                                                                 uint32_t* __restrict__ marked) {
-  __shared__ uint32_t s_degree[kGroupsPerPart * kGroupPitch];
-  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-  const uint32_t parts_per_sample = words_per_sample / kPartWords;
-  const uint32_t sample_blocks = (n_samples + kSumSamplesPerBlock - 1) / kSumSamplesPerBlock;
-  const uint32_t part = blockIdx.x / sample_blocks;
-  const uint32_t first_sample = (blockIdx.x - part * sample_blocks) * kSumSamplesPerBlock;
-  const uint32_t first_vertex = part * (kPartWords * 32u);
-  for (uint32_t i = threadIdx.x; i < kPartWords * 32u; i += kSumThreads) {
-    const uint32_t v = first_vertex + i;
-    s_degree[(i / kGroupVertices) * kGroupPitch + i % kGroupVertices] =
-        v < n_vertices ? (uint32_t)(row_ptr[v + 1] - row_ptr[v]) : 0u;
-  }
-  __syncthreads();
-  const uint32_t end_sample = first_sample + kSumSamplesPerBlock < n_samples ? first_sample + kSumSamplesPerBlock : n_samples;
-  const uint32_t* mine = s_degree + lane * kGroupPitch;
-  for (uint32_t s = first_sample + wave; s < end_sample; s += kSumThreads / kWave) {
-    const uint4* words = (const uint4*)(bitmap + (size_t)s * words_per_sample + (size_t)part * kPartWords + lane * kGroupWords);
-    const uint4 a = words[0], b = words[1];
-    // word by word: finding and clearing the lowest set bit of a 32-bit word is three vector
-    // instructions, of a 64-bit one eight, and the launch is bound by instruction issue
-    const uint32_t w[kGroupWords] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-    uint64_t sum = 0;
-    uint32_t count = 0;
-#pragma unroll
-    for (uint32_t k = 0; k < kGroupWords; ++k) {
-      uint32_t bits = w[k];
-      count += (uint32_t)__popc(bits);
-      const uint32_t* from = mine + k * 32u;
-      while (bits) {
-        const uint32_t i0 = (uint32_t)__ffs((int)bits) - 1u;
-        bits &= bits - 1u;
-        const uint64_t d0 = from[i0];
-        sum += d0 * d0;
-      }
-    }
-    const uint64_t through = wave_inclusive_scan_u64(sum);
-    const size_t at = (size_t)s * parts_per_sample + part;
-    group_through[at * kGroupsPerPart + lane] = through;
-    if (lane == 63) part_total[at] = through;
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) count += __shfl_xor(count, d, kWave);
-    if (lane == 0 && count) atomicAdd(&marked[s], count);
-  }
-}
-
-// One wavefront per sample: part_before[s * (parts + 1) + p] = degree^2 of the marked vertices
-// of the sample's parts before p; entry `parts` is the sample's total.
-__global__ __launch_bounds__(64) void sample_part_sums(const uint64_t* __restrict__ part_total, uint32_t parts,
-                                                       uint64_t* __restrict__ part_before) {
-  const uint32_t s = blockIdx.x, lane = threadIdx.x;
-  uint64_t carry = 0;
-  for (uint32_t p0 = 0; p0 < parts; p0 += 64) {
-    const uint32_t p = p0 + lane;
-    const uint64_t mine = p < parts ? part_total[(size_t)s * parts + p] : 0ull;
-    const uint64_t through = wave_inclusive_scan_u64(mine);
-    if (p < parts) part_before[(size_t)s * (parts + 1) + p] = carry + through - mine;
-    const uint32_t lo = __shfl((uint32_t)through, 63, kWave), hi = __shfl((uint32_t)(through >> 32), 63, kWave);
-    carry += ((uint64_t)hi << 32) | lo;
-  }
-  if (lane == 0) part_before[(size_t)s * (parts + 1) + parts] = carry;
-}
-
-// What next() of a kDistinctByDegreeSquared app receives as transitEdges.
-struct DistinctByDegreeSquared {
-  const uint32_t* bits;           // the sample's bitmap
-  const uint64_t* part_before;    // the sample's parts + 1 entries
-  const uint64_t* group_through;  // the sample's parts * 64 entries
-  const EdgePos_t* row_ptr;
-  uint32_t parts;
-
-  __device__ __forceinline__ uint64_t total() const { return part_before[parts]; }
-
-  // the smallest marked vertex whose running sum of degree^2 (marked vertices ascending)
-  // exceeds target; target < total()
-  __device__ inline VertexID first_exceeding(uint64_t target) const {
-    uint32_t lo = 0, hi = parts;  // last part whose sum-before is <= target
-    while (hi - lo > 1) {
-      const uint32_t mid = lo + (hi - lo) / 2;
-      if (part_before[mid] <= target) lo = mid; else hi = mid;
-    }
-    const uint32_t part = lo;
-    target -= part_before[part];
-    const uint64_t* through = group_through + (size_t)part * kGroupsPerPart;
-    uint32_t first = 0, last = kGroupsPerPart - 1;  // first group whose sum-through exceeds target
-    while (first < last) {
-      const uint32_t mid = first + (last - first) / 2;
-      if (through[mid] > target) last = mid; else first = mid + 1;
-    }
-    if (first) target -= through[first - 1];
-    const uint32_t first_word = part * kPartWords + first * kGroupWords;
-    uint64_t running = 0;
-    VertexID found = -1;
-    for (uint32_t k = 0; k < kGroupWords && found < 0; ++k) {
-      uint32_t word = bits[first_word + k];
-      while (word) {
-        const uint32_t v = (first_word + k) * 32u + (uint32_t)__ffs((int)word) - 1u;
-        const uint64_t d = (uint64_t)(row_ptr[v + 1] - row_ptr[v]);
-        running += d * d;
-        if (running > target) { found = (VertexID)v; break; }
-        word &= word - 1u;
-      }
-    }
-    return found;
-  }
-};
-
 // item_count[s] = work items of sample s (at least one, so that row offsets get written)
 __global__ void build_item_counts(const uint32_t* __restrict__ sizes, uint32_t n, uint32_t* __restrict__ item_count) {
   const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1173,12 +1027,6 @@ struct LayerParams {
   // ranked_ids[ranked_start[ls] .. ranked_start[ls + 1])
   const uint32_t* ranked_start;
   const int32_t* ranked_ids;
-  // kDistinctByDegreeSquared: bitmaps and their two levels of degree^2 sums
-  const uint32_t* bitmap;
-  uint32_t words_per_sample;
-  const uint64_t* part_before;
-  const uint64_t* group_through;
-  const uint32_t* marked;        // marked vertices per sample
 };
 
 template <class SampleType, class App>
@@ -1207,16 +1055,6 @@ __global__ __launch_bounds__(256) void layer_execute_kernel(LayerParams P) {
           (VertexID_t)nbr, &rng);
       neighbor = r == -1 ? P.invalid : r;
     }
-  } else if constexpr (apps::neighborhood_form_of<App>::value == apps::kDistinctByDegreeSquared) {
-    const uint32_t parts = P.words_per_sample / kPartWords;
-    DistinctByDegreeSquared distinct{P.bitmap + (size_t)ls * P.words_per_sample,
-                                     P.part_before + (size_t)ls * (parts + 1),
-                                     P.group_through + (size_t)ls * parts * kGroupsPerPart, csr.row_ptr, parts};
-    const float* no_weights = nullptr;
-    const VertexID r = App().template next<SampleType, DistinctByDegreeSquared, const float*>(
-        P.step, &csr, transits, sample_id, state, 0.0f, distinct, no_weights, (EdgePos_t)P.marked[ls],
-        (VertexID_t)nbr, &rng);
-    neighbor = r == -1 ? P.invalid : r;
   } else {
     const uint32_t begin = P.ranked_start[ls];
     const CSR::Edge* ranked = P.ranked_ids + begin;
@@ -1227,6 +1065,52 @@ __global__ __launch_bounds__(256) void layer_execute_kernel(LayerParams P) {
     neighbor = r == -1 ? P.invalid : r;
   }
   P.final_samples[(size_t)s * P.final_size + P.out_base + nbr] = neighbor;
+}
+
+// kDistinctByDegreeSquared (nd_union_sums.hpp): next() for output nbr of sample ls of the chunk.
+template <class SampleType, class App, class Distinct>
+__device__ __forceinline__ void draw_by_degree(const LayerParams& P, uint32_t ls, uint32_t nbr, Distinct& distinct,
+                                               uint32_t n_distinct) {
+  const uint32_t s = P.sample_begin + ls;
+  CSRPartition csr = P.csr;
+  SampleType local_state;
+  SampleType* state = std::is_empty<SampleType>::value ? &local_state : (SampleType*)P.samples + s;
+  curandState rng;
+  rng.reset(P.seed, (P.first_sample + s) * P.step_size + nbr, (uint32_t)P.step);
+  const float* no_weights = nullptr;
+  const VertexID r = App().template next<SampleType, Distinct, const float*>(
+      P.step, &csr, P.transits.base + (size_t)ls * P.transits.stride, (VertexID)(P.first_sample + s), state, 0.0f, distinct,
+      no_weights, (EdgePos_t)n_distinct, (VertexID_t)nbr, &rng);
+  P.final_samples[(size_t)s * P.final_size + P.out_base + nbr] = r == -1 ? P.invalid : r;
+}
+
+template <class SampleType, class App>
+__global__ __launch_bounds__(kSortedThreads) void sorted_layer_kernel(LayerParams P, const uint32_t* __restrict__ sizes,
+                                                                      uint32_t* __restrict__ distinct) {
+  const uint32_t ls = blockIdx.x, size = sizes[ls];
+  if (size > kSortedEntries) return;
+  sorted_layer(P.csr, P.transits.base + (size_t)ls * P.transits.stride, P.transits.count, P.invalid, size, distinct + ls,
+               [&](SortedByDegreeSquared& view, uint32_t n_distinct) {
+                 for (uint32_t nbr = threadIdx.x; nbr < P.step_size; nbr += kSortedThreads)
+                   draw_by_degree<SampleType, App>(P, ls, nbr, view, n_distinct);
+               });
+}
+
+// The draws of the marked samples, a lane each, the workgroups of the grid in turn.
+template <class SampleType, class App>
+__global__ __launch_bounds__(256) void marked_layer_kernel(LayerParams P, MarkedSamples marked,
+                                                           const uint32_t* __restrict__ distinct,
+                                                           const uint32_t* __restrict__ bitmap, uint32_t words_per_sample,
+                                                           const uint64_t* __restrict__ part_before,
+                                                           const uint64_t* __restrict__ group_through, uint32_t parts) {
+  const uint64_t draws = (uint64_t)*marked.count * P.step_size;
+  for (uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x; i < draws; i += gridDim.x * 256ull) {
+    const uint32_t at = (uint32_t)(i / P.step_size), nbr = (uint32_t)(i - (uint64_t)at * P.step_size);
+    const uint32_t ls = marked.sample[at];
+    MarkedByDegreeSquared mine{bitmap + (size_t)at * words_per_sample, part_before + (size_t)at * (parts + 1),
+                               group_through + (size_t)at * parts * kGroupsPerPart, P.csr.row_ptr, parts};
+    draw_by_degree<SampleType, App>(P, ls, nbr, mine, distinct[ls]);
+  }
 }
 
 // Entries of concatenated neighbourhood one chunk of samples may hold (about 70 bytes of
@@ -1276,8 +1160,8 @@ class LayerEngine : public EngineBase {
       if (rc != 0) return rc;
     }
     if (apps::neighborhood_form_of<App>::value == apps::kDistinctByDegreeSquared) {
-      const int rc = build_dense_pieces(graph, nullptr);
-      if (rc != 0) return rc;
+      ND_HIP_TRY(union_.build(dgraph_.view, bitmap_words_for((uint32_t)graph->get_n_vertices())));
+      dense_pieces_ = union_.pieces;
     }
     graph_ = graph;
     return 0;
@@ -1375,6 +1259,16 @@ class LayerEngine : public EngineBase {
     ND_HIP_TRY(hipMalloc(&d_item_start_, sizeof(uint32_t) * ((size_t)n_samples_ + 1)));
     ND_HIP_TRY(hipMalloc(&d_row_offsets_, sizeof(uint32_t) * (size_t)n_samples_ * widest));
     ND_HIP_TRY(hipMalloc(&d_small_scratch_, sizeof(uint32_t) * scan_scratch_elems((size_t)n_samples_ + 1)));
+    if (apps::neighborhood_form_of<App>::value == apps::kDistinctByDegreeSquared) {
+      ND_HIP_TRY(hipMalloc(&d_layer_counts_, sizeof(uint32_t) * 2 * (size_t)n_samples_ * n_steps));
+      ND_HIP_TRY(hipHostMalloc((void**)&h_too_long_, sizeof(uint32_t), hipHostMallocDefault));
+      *h_too_long_ = 0;
+      marked_.stride = widest;
+      ND_HIP_TRY(hipMalloc(&marked_.count, sizeof(uint32_t)));
+      ND_HIP_TRY(hipMalloc(&marked_.sample, sizeof(uint32_t) * (size_t)n_samples_));
+      ND_HIP_TRY(hipMalloc(&marked_.transits, sizeof(int32_t) * (size_t)n_samples_ * widest));
+      ND_HIP_TRY(hipMalloc(&marked_.transit_count, sizeof(uint2) * (size_t)n_samples_));
+    }
     if (apps::neighborhood_form_of<App>::value == apps::kRankedByLadiesImportance) {
       const size_t per_sample = sizeof(uint32_t) * ((size_t)n_samples_ + 1);
       ND_HIP_TRY(hipMalloc(&d_ranked_start_, per_sample));
@@ -1394,6 +1288,8 @@ class LayerEngine : public EngineBase {
     neighborhood_total_ = 0;
     distinct_total_ = 0;
     chunks_run_ = 0;
+    counted_ = true;
+    if (h_too_long_) *h_too_long_ = 0;
     if (!std::is_empty<SampleType>::value) {
       ND_HIP_TRY(hipMemcpyAsync(d_samples_, d_samples_init_, sizeof(SampleType) * (size_t)n_samples_,
                                 hipMemcpyDeviceToDevice, stream_));
@@ -1412,17 +1308,24 @@ class LayerEngine : public EngineBase {
         all.stride = (uint32_t)F;
         all.count = (uint32_t)app.stepSize(step - 1);
       }
+      constexpr int form = apps::neighborhood_form_of<App>::value;
+      if (form == apps::kDistinctByDegreeSquared && bitmap_chunk_entries_ == kBitmapChunkEntries) {
+        // chunks of as many samples as there is memory for bitmaps of: nothing the host has to know first
+        for (uint32_t s0 = 0; s0 < S; s0 += bitmap_chunk_samples_, chunks_run_++)
+          if (run_chunk(step, all, s0, std::min(S, s0 + bitmap_chunk_samples_), 0) != 0) return -1;
+        continue;
+      }
       // size of every sample's collective neighbourhood, then chunks of samples that fit the budget
       collective_sizes<<<dim3((S + 3) / 4), dim3(256), 0, stream_>>>(dgraph_.view, all, S, invalid_, d_sizes_);
       ND_HIP_TRY(hipMemcpyAsync(h_sizes_.data(), d_sizes_, sizeof(uint32_t) * S, hipMemcpyDeviceToHost, stream_));
       ND_HIP_TRY(hipStreamSynchronize(stream_));
       // chunk limits: entries of concatenation the work arrays hold, or (bitmap form) bitmaps
       // that fit the budget and a grid of marking work items that fits 31 bits
-      constexpr bool by_bitmap = apps::neighborhood_form_of<App>::value != apps::kConcatenated;
+      constexpr bool by_bitmap = form != apps::kConcatenated;
       const uint64_t entry_budget = by_bitmap ? bitmap_chunk_entries_ : chunk_entries_;
       const uint32_t sample_budget = by_bitmap ? bitmap_chunk_samples_ : S;
       for (uint32_t s = 0; s < S; ++s)
-        if (h_sizes_[s] >= (1u << 31)) { last_error = "collective neighbourhood of one sample has 2^31 or more entries"; return -2; }
+        if (h_sizes_[s] >= (1u << 31)) { last_error = kTooLong; return -2; }
       uint32_t s0 = 0;
       while (s0 < S) {
         uint64_t total = h_sizes_[s0];
@@ -1443,6 +1346,8 @@ class LayerEngine : public EngineBase {
     ND_HIP_TRY(hipEventRecord(ev_end_, stream_));
     ND_HIP_TRY(hipStreamSynchronize(stream_));
     ND_HIP_TRY(hipEventElapsedTime(&times.end_to_end, ev_begin_, ev_end_));
+    if (h_too_long_ && *h_too_long_) { last_error = kTooLong; return -2; }
+    counted_ = apps::neighborhood_form_of<App>::value != apps::kDistinctByDegreeSquared;
     return 0;
   }
 
@@ -1466,6 +1371,13 @@ class LayerEngine : public EngineBase {
 
   // sizes of the last run, for the algorithmic-bytes figure
   int64_t counter(int which) const override {
+    if (!counted_ && (which == 0 || which == 1)) {  // the last pass left them on the device
+      std::vector<uint32_t> all(2 * (size_t)n_samples_ * (size_t)App().steps());
+      if (hipMemcpy(all.data(), d_layer_counts_, sizeof(uint32_t) * all.size(), hipMemcpyDeviceToHost) != hipSuccess) return 0;
+      neighborhood_total_ = distinct_total_ = 0;
+      for (size_t i = 0; i < all.size(); ++i) (i < all.size() / 2 ? neighborhood_total_ : distinct_total_) += all[i];
+      counted_ = true;
+    }
     return which == 0 ? (int64_t)neighborhood_total_ : which == 1 ? (int64_t)distinct_total_
            : which == 2 ? (int64_t)chunks_run_ : which == 3 ? (int64_t)dense_pieces_ : 0;
   }
@@ -1474,6 +1386,7 @@ class LayerEngine : public EngineBase {
     free_run_buffers();
     release(d_row_sums_);
     release_dense_pieces();
+    union_.release();
     dgraph_.release();
     graph_ = nullptr;
   }
@@ -1566,6 +1479,9 @@ class LayerEngine : public EngineBase {
   }
 
 
+  static constexpr uint32_t kDrawBlocks = 4096;
+  static constexpr const char* kTooLong = "collective neighbourhood of one sample has 2^31 or more entries";
+
   // events around the neighbourhood kernel when profiling is on
   void tick() {
     if (profiling) (void)hipEventRecord(ev_a_, stream_);
@@ -1589,9 +1505,9 @@ class LayerEngine : public EngineBase {
     constexpr int form = apps::neighborhood_form_of<App>::value;
     TransitView tv = all;
     tv.base = all.base + (size_t)s0 * all.stride;
-    if (form != apps::kConcatenated) {
+    if (form == apps::kRankedByLadiesImportance) {
       if (build_distinct_by_bitmap(step, s0, tv, n) != 0) return -1;
-    } else {
+    } else if (form == apps::kConcatenated) {
       // work items of the build: long neighbourhoods are spread over several workgroups
       uint64_t n_items = 0;
       for (uint32_t s = s0; s < s1; ++s) {
@@ -1629,65 +1545,58 @@ class LayerEngine : public EngineBase {
     P.offsets = d_offsets_;
     P.nbr_cols = d_nbr_cols_;
     P.nbr_weights = d_nbr_weights_;
-    if (form != apps::kConcatenated) {
+    if constexpr (form == apps::kDistinctByDegreeSquared) {
+      return run_by_degree(P, step);
+    } else {
       P.ranked_start = d_ranked_start_;
       P.ranked_ids = d_ranked_ids_;
-      P.bitmap = d_bitmap_;
-      P.words_per_sample = bitmap_words_;
-      P.part_before = d_part_before_;
-      P.group_through = d_group_through_;
-      P.marked = d_marked_;
+      const uint64_t outputs = (uint64_t)n * P.step_size;
+      layer_execute_kernel<SampleType, App><<<dim3((unsigned)((outputs + 255) / 256)), dim3(256), 0, stream_>>>(P);
+      ND_HIP_TRY(hipGetLastError());
+      return 0;
     }
-    const uint64_t outputs = (uint64_t)n * P.step_size;
-    layer_execute_kernel<SampleType, App><<<dim3((unsigned)((outputs + 255) / 256)), dim3(256), 0, stream_>>>(P);
+  }
+
+  // kDistinctByDegreeSquared: the samples of the chunk by the size of their neighbourhoods, and their draws.
+  int run_by_degree(const LayerParams& P, int step) {
+    const uint32_t n = P.chunk_samples, parts = union_.parts;
+    const size_t n_parts = (size_t)n * parts;
+    if (n > bitmap_samples_) {
+      release(d_bitmap_); release(d_group_through_); release(d_part_total_); release(d_part_before_);
+      ND_HIP_TRY(hipMalloc(&d_bitmap_, sizeof(uint32_t) * (size_t)n * bitmap_words_));
+      ND_HIP_TRY(hipMalloc(&d_group_through_, sizeof(uint64_t) * n_parts * kGroupsPerPart));
+      ND_HIP_TRY(hipMalloc(&d_part_total_, sizeof(uint64_t) * n_parts));
+      ND_HIP_TRY(hipMalloc(&d_part_before_, sizeof(uint64_t) * (size_t)n * (parts + 1)));
+      bitmap_samples_ = n;
+    }
+    const size_t S = (size_t)n_samples_;
+    uint32_t* sizes = d_layer_counts_ + S * step + P.sample_begin;
+    uint32_t* distinct = sizes + S * App().steps();
+    ND_HIP_TRY(hipMemsetAsync(marked_.count, 0, sizeof(uint32_t), stream_));
+    sort_out_samples<<<dim3((n + 15) / 16), dim3(kSortOutThreads), 0, stream_>>>(P.csr, P.transits, n, invalid_, union_.hubs.row_of, sizes,
+                                                                   distinct, marked_, h_too_long_);
+    tick();
+    sorted_layer_kernel<SampleType, App><<<dim3(n), dim3(kSortedThreads), 0, stream_>>>(P, sizes, distinct);
+    const uint32_t turns = (parts + kXcdCount - 1) / kXcdCount * kUnionSlices;
+    union_parts<<<dim3(turns * kXcdCount), dim3(kUnionThreads), 0, stream_>>>(P.csr, union_.hubs, parts, marked_, bitmap_words_,
+                                                                              d_bitmap_);
+    union_sums<<<dim3(parts * kSumSlices), dim3(kSumThreads), 0, stream_>>>(
+        union_.squares, union_.square_rows, parts, marked_, bitmap_words_, d_bitmap_, d_group_through_, d_part_total_, distinct);
+    tock();
+    sample_part_sums<<<dim3(n), dim3(64), 0, stream_>>>(d_part_total_, parts, marked_.count, d_part_before_);
+    marked_layer_kernel<SampleType, App><<<dim3(kDrawBlocks), dim3(256), 0, stream_>>>(
+        P, marked_, distinct, d_bitmap_, bitmap_words_, d_part_before_, d_group_through_, parts);
     ND_HIP_TRY(hipGetLastError());
     return 0;
   }
 
-  // What next() of the importance forms is handed, for every sample of the chunk.
+  // What next() of the LADIES form is handed, for every sample of the chunk.
   int build_distinct_by_bitmap(int step, uint32_t s0, const TransitView& tv, uint32_t n) {
-    constexpr bool ladies = apps::neighborhood_form_of<App>::value == apps::kRankedByLadiesImportance;
-    constexpr uint32_t bin_words = ladies ? kBinVerticesSums / 32u : kBinWordsBits;
+    constexpr uint32_t bin_words = kBinVerticesSums / 32u;
     const uint32_t bins = (bitmap_words_ + bin_words - 1) / bin_words;
-    constexpr uint32_t per_group = ladies ? kBinsPerGroupSums : kBinsPerGroupBits;
-    const uint32_t groups = (bins + per_group - 1) / per_group;
+    const uint32_t groups = (bins + kBinsPerGroupSums - 1) / kBinsPerGroupSums;
     if ((uint64_t)n * groups >= (1ull << 31)) { last_error = "a chunk needs 2^31 or more workgroups"; return -1; }
-    if constexpr (ladies) {
-      return rank_by_keys(step, s0, tv, n, bins, groups);
-    } else {
-      return list_distinct(tv, n, bins, groups);
-    }
-  }
-
-  // FastGCN form: mark the vertices of every sample's neighbourhood in its bitmap and add up
-  // degree^2 over the marked vertices at two levels (groups of 256 vertices, parts of 64 groups).
-  int list_distinct(const TransitView& tv, uint32_t n, uint32_t bins, uint32_t groups) {
-    const uint32_t parts_per_sample = bitmap_words_ / kPartWords;
-    const size_t n_parts = (size_t)n * parts_per_sample;
-    if (n_parts >= (1ull << 32)) { last_error = "a chunk needs 2^32 or more bitmap parts"; return -1; }
-    if (n > bitmap_samples_) {
-      release(d_bitmap_); release(d_group_through_); release(d_part_total_); release(d_part_before_); release(d_marked_);
-      ND_HIP_TRY(hipMalloc(&d_bitmap_, sizeof(uint32_t) * (size_t)n * bitmap_words_));
-      ND_HIP_TRY(hipMalloc(&d_group_through_, sizeof(uint64_t) * n_parts * kGroupsPerPart));
-      ND_HIP_TRY(hipMalloc(&d_part_total_, sizeof(uint64_t) * n_parts));
-      ND_HIP_TRY(hipMalloc(&d_part_before_, sizeof(uint64_t) * (size_t)n * (parts_per_sample + 1)));
-      ND_HIP_TRY(hipMalloc(&d_marked_, sizeof(uint32_t) * (size_t)n));
-      bitmap_samples_ = n;
-    }
-    tick();
-    collective_mark_binned<false><<<dim3(n * groups), dim3(kBinThreads), 0, stream_>>>(
-        dgraph_.view, tv, invalid_, n, bins, d_bitmap_, bitmap_words_, nullptr, 0u, dense_, KeysOnTheWayOut());
-    tock();
-    ND_HIP_TRY(hipMemsetAsync(d_marked_, 0, sizeof(uint32_t) * (size_t)n, stream_));
-    const uint32_t sample_blocks = (n + kSumSamplesPerBlock - 1) / kSumSamplesPerBlock;
-    bitmap_group_sums<<<dim3(parts_per_sample * sample_blocks), dim3(kSumThreads), 0, stream_>>>(
-        d_bitmap_, bitmap_words_, n, (uint32_t)invalid_, dgraph_.row_ptr(), d_group_through_, d_part_total_, d_marked_);
-    sample_part_sums<<<dim3(n), dim3(64), 0, stream_>>>(d_part_total_, parts_per_sample, d_part_before_);
-    std::vector<uint32_t> marked(n);
-    ND_HIP_TRY(hipMemcpyAsync(marked.data(), d_marked_, sizeof(uint32_t) * n, hipMemcpyDeviceToHost, stream_));
-    ND_HIP_TRY(hipStreamSynchronize(stream_));
-    for (uint32_t c : marked) distinct_total_ += c;
-    return hipGetLastError() == hipSuccess ? 0 : -1;
+    return rank_by_keys(step, s0, tv, n, bins, groups);
   }
 
   // LADIES form: the marking leaves one sampling key per (sample, vertex); per sample, the
@@ -1805,7 +1714,7 @@ class LayerEngine : public EngineBase {
   void release_neighborhood_buffers() {
     release(d_nbr_cols_); release(d_nbr_weights_);
     release(d_bitmap_); release(d_keys_dense_); release(d_stretch_best_);
-    release(d_group_through_); release(d_part_total_); release(d_part_before_); release(d_marked_);
+    release(d_group_through_); release(d_part_total_); release(d_part_before_);
     release_distinct_buffers();
     capacity_ = 0;
     bitmap_samples_ = 0;
@@ -1815,6 +1724,10 @@ class LayerEngine : public EngineBase {
     release(d_initial_); release(d_samples_); release(d_samples_init_); release(d_final_);
     release(d_sizes_); release(d_offsets_); release(d_row_offsets_); release(d_small_scratch_);
     release(d_item_count_); release(d_item_start_);
+    release(d_layer_counts_);
+    if (h_too_long_) (void)hipHostFree(h_too_long_);
+    h_too_long_ = nullptr;
+    release(marked_.count); release(marked_.sample); release(marked_.transits); release(marked_.transit_count);
     release(d_ranked_start_); release(d_select_kept_);
     release(d_select_threshold_); release(d_select_present_);
     release_neighborhood_buffers();
@@ -1855,7 +1768,9 @@ class LayerEngine : public EngineBase {
   // LADIES form: importance sums and sampling keys, [sample][vertex, padded to whole stretches]
   uint32_t* d_keys_dense_ = nullptr;
   uint16_t* d_stretch_best_ = nullptr;  // LADIES form: best key prefix of every 256 keys of every sample
-  uint64_t neighborhood_total_ = 0, distinct_total_ = 0, chunks_run_ = 0;
+  mutable uint64_t neighborhood_total_ = 0, distinct_total_ = 0;
+  uint64_t chunks_run_ = 0;
+  mutable bool counted_ = true;  // those two are the last pass's
   uint64_t chunk_entries_ = kLayerChunkEntries;
   bool progress_ = false;
 
@@ -1878,7 +1793,10 @@ class LayerEngine : public EngineBase {
   uint32_t *d_key2_ = nullptr, *d_index2_ = nullptr, *d_hist_ = nullptr, *d_scratch_ = nullptr;
   // FastGCN form: degree^2 of the marked vertices, by group inside a part, by part, by sample
   uint64_t *d_group_through_ = nullptr, *d_part_total_ = nullptr, *d_part_before_ = nullptr;
-  uint32_t* d_marked_ = nullptr;
+  UnionTables union_;                  // of the graph
+  MarkedSamples marked_{};
+  uint32_t* d_layer_counts_ = nullptr;  // entries of every layer and sample's neighbourhood, then its distinct vertices
+  uint32_t* h_too_long_ = nullptr;      // a neighbourhood was too long
   int32_t* d_ranked_ids_ = nullptr;
 };
 
