@@ -155,17 +155,59 @@ __host__ __device__ __forceinline__ unsigned long long importance_term_fixed(flo
   return shift > -24 ? (unsigned long long)(mantissa >> -shift) : 0ull;
 }
 
-// ---- the distinct vertices of a collective neighbourhood, marked stretch by stretch ----
+// ---- LADIES form: the importance sums of a collective neighbourhood, stretch by stretch ----
 //
-// collective_mark_binned walks the neighbourhood as collective_build does, but instead of
-// copying an entry it marks the entry's vertex; nothing of the concatenation is stored.  A
-// neighbourhood that sits on hubs repeats its vertices many times over (3.8e10 entries hold
-// 2.0e9 distinct pairs at FastGCN's full size).  FastGCN form: the result is a bitmap per
-// sample (words_per_sample 32-bit words, a multiple of the tile below).  LADIES form
-// (kWithImportance): every entry also adds (weight * inverse_row_sum[transit])^2, as a 2^53
-// fixed-point integer, to the 64-bit sum of (sample, vertex) in LDS; the result is the sampling
-// key formed from that sum for every vertex of every sample, kAbsentKey where the sample's
-// neighbourhood does not hold the vertex.
+// What an entry (u, v) contributes to v does not depend on the sample: (weight * inverse_row_sum[u])^2 as a 2^53
+// fixed-point integer.  So the terms are worked out once per graph, and parallel edges (hub pairs are joined by
+// thousands: 4.5 M entries of a sample's second layer over 500 K vertices are 1.5 M pairs) are one entry with the sum of
+// theirs - integers, to which the order of the additions does not matter.
+struct MergedEdges {
+  const EdgePos_t* row_ptr;          // [vertices + 1]
+  const VertexID* ids;               // ascending and without repeats in every row
+  const unsigned long long* terms;
+  bool zero_terms;                   // some are 0: a vertex can be there with the sum 0
+  // Vertices with kCutDegree neighbours or more: where their rows pass from stretch to stretch (a search of a hub's row
+  // is twenty dependent loads, and a workgroup waits for its slowest lane's in every stretch).
+  const int32_t* cut_row_of;         // [vertices], -1: none
+  const HubCut* cuts;                // [rows][stretches + 1]; no pieces in it
+};
+constexpr uint32_t kCutDegree = 32;
+
+__global__ __launch_bounds__(256) void first_of_parallel_edges(CSRPartition csr, uint32_t* __restrict__ is_first) {
+  const size_t e = (size_t)blockIdx.x * 256u + threadIdx.x;
+  if (e > (size_t)csr.n_edges) return;
+  if (e == (size_t)csr.n_edges) {
+    is_first[e] = 0;
+    return;
+  }
+  const VertexID u = source_of_edge(csr.row_ptr, csr.n_vertices, (EdgePos_t)e);
+  is_first[e] = (EdgePos_t)e == csr.row_ptr[u] || csr.edges[e - 1] != csr.edges[e] ? 1u : 0u;
+}
+
+// at[e] = how many first edges there are before e
+__global__ __launch_bounds__(256) void merge_rows(CSRPartition csr, const uint32_t* __restrict__ at, EdgePos_t* __restrict__ row_ptr) {
+  const size_t v = (size_t)blockIdx.x * 256u + threadIdx.x;
+  if (v <= (size_t)csr.n_vertices) row_ptr[v] = (EdgePos_t)at[csr.row_ptr[v]];
+}
+
+__global__ __launch_bounds__(256) void merge_edges(CSRPartition csr, const float* __restrict__ inverse_row_sums,
+                                                   const uint32_t* __restrict__ at, VertexID* __restrict__ ids,
+                                                   unsigned long long* __restrict__ terms, uint32_t* zero_terms) {
+  const size_t e = (size_t)blockIdx.x * 256u + threadIdx.x;
+  if (e >= (size_t)csr.n_edges || at[e + 1] == at[e]) return;
+  const float inverse = inverse_row_sums[source_of_edge(csr.row_ptr, csr.n_vertices, (EdgePos_t)e)];
+  unsigned long long sum = 0;
+  for (size_t i = e;;) {  // to the next first edge
+    const float p = csr.weights[i] * inverse;
+    sum += importance_term_fixed(p * p);
+    ++i;
+    if (i >= (size_t)csr.n_edges || at[i + 1] != at[i]) break;
+  }
+  ids[at[e]] = csr.edges[e];
+  terms[at[e]] = sum;
+  if (sum == 0) *zero_terms = 1;
+}
+
 constexpr uint32_t kBitmapTileWords = 2048;  // bitmaps are padded to whole tiles of 65536 vertices (4 parts)
 
 // log2 of a positive normal float from exponent extraction and an atanh series; every step
@@ -245,72 +287,31 @@ template <int kShift>
 __device__ __forceinline__ uint32_t row_shift_up(uint32_t fill, uint32_t x) {
   return (uint32_t)__builtin_amdgcn_update_dpp((int)fill, (int)x, 0x110 | kShift, 0xF, 0xF, false);
 }
-// The value of lane - 1 / lane + 1 across the whole wavefront; the end lanes get `fill`.
-__device__ __forceinline__ uint32_t wave_from_below(uint32_t fill, uint32_t x) {
-  return (uint32_t)__builtin_amdgcn_update_dpp((int)fill, (int)x, 0x138, 0xF, 0xF, false);  // wave_shr:1
-}
-__device__ __forceinline__ uint32_t wave_from_above(uint32_t fill, uint32_t x) {
-  return (uint32_t)__builtin_amdgcn_update_dpp((int)fill, (int)x, 0x130, 0xF, 0xF, false);  // wave_shl:1
-}
-
-// One step of a segmented inclusive sum along a row of 16 lanes: (closed, term) of this lane
-// takes in (up_closed, up_term) of a lane further down.  A lane is closed once its sum has
-// reached the start of its segment.
-__device__ __forceinline__ void take_in(uint32_t up_closed, uint32_t up_lo, uint32_t up_hi, uint32_t& closed,
-                                        unsigned long long& term) {
-  if (!closed) term += ((unsigned long long)up_hi << 32) | up_lo;
-  closed |= up_closed;
-}
-
-template <int kShift>
-__device__ __forceinline__ void segmented_row_step(uint32_t& closed, unsigned long long& term) {
-  // lanes without a source take in the neutral element (open, 0)
-  const uint32_t c = row_shift_up<kShift>(0u, closed);
-  const uint32_t lo = row_shift_up<kShift>(0u, (uint32_t)term);
-  const uint32_t hi = row_shift_up<kShift>(0u, (uint32_t)(term >> 32));
-  take_in(c, lo, hi, closed, term);
-}
-
-// The same marking with the presence map (and the importance sums) of one stretch of the vertex
-// range held in LDS: one workgroup per (sample, stretch).  Adjacencies are sorted by
-// destination, so the part of a transit's adjacency that falls into the stretch is one
-// sub-range, found by two binary searches; the workgroup streams the sub-ranges of all the
-// sample's transits, marks and adds in LDS, and writes the stretch out once - plain stores
-// that cover the whole map, so nothing is cleared beforehand and no atomic reaches memory
-// (global atomics stop at ~24 G/s on this part; the LADIES form needs 4.2e9 of them).
-// The LDS pipeline is what this kernel runs out of (counters: a wavefront waits for LDS a
-// third of its time), so it is kept for the map itself: every wavefront walks a contiguous
-// part of the stretch's entries, which lets a lane step from one sub-range to the next instead
-// of searching the table for every entry, and the sums along the wavefront move through DPP.
+// One workgroup per (sample, some consecutive stretches of 7168 vertices), the sums of one stretch in LDS at a time.
+// Adjacencies are sorted by destination, so the part of a transit's adjacency that falls into a stretch is one
+// sub-range; the workgroup streams the sub-ranges of all the sample's transits, adds in LDS, and writes the stretch
+// out once - plain stores that cover the whole map, so nothing is cleared beforehand and no atomic reaches memory
+// (global atomics stop at ~24 G/s on this part).  Every wavefront walks a contiguous part of the stretch's entries,
+// which lets a lane step from one sub-range to the next instead of searching the table for every entry.
 constexpr uint32_t kBinThreads = 1024;
 constexpr uint32_t kBinWaves = kBinThreads / 64;
 constexpr uint32_t kBinAhead = 4;             // entries a lane fetches before it works on the first
-constexpr EdgePos_t kShortRest = 16;          // edges left of an adjacency that are stepped through one by one
-// consecutive stretches of a sample one workgroup takes (FastGCN form: few, large stretches per
-// sample, and the low ones hold most entries; LADIES form: hundreds of small ones)
-constexpr uint32_t kBinsPerGroupBits = 8;
-constexpr uint32_t kBinsPerGroupSums = 16;
-constexpr uint32_t kBinWordsBits = 2048;      // FastGCN form: 65,536 vertices, one byte each in LDS (64 KB)
-constexpr uint32_t kBinVerticesSums = 7168;   // LADIES form: 56 KB of 64-bit sums + 896 B of bits
+constexpr uint32_t kBinsPerGroup = 16;        // consecutive stretches of a sample one workgroup takes
+constexpr uint32_t kBinVertices = 7168;       // 56 KB of 64-bit sums + 896 B of bits
+constexpr uint32_t kBinWords = kBinVertices / 32u;
 
-// Dense pieces.  What a hub contributes to a stretch can be thousands of entries (a layer
-// drawn by degree^2 sits on the hubs: 144 K entries per transit at FastGCN's full size), and
-// it is the same for every sample that holds the hub.  Where a vertex has kDensePieceEntries
-// (LADIES form: kDensePieceEntriesSums) or more edges into one stretch, the stretch's piece of
-// that vertex is built once per graph - FastGCN form: its bitmap (2048 words); LADIES form:
-// the importance sum of every vertex of the stretch (7168 64-bit integers, kAbsentSum where
-// there is no edge; the sums are integers, so adding a piece gives the bits that adding its
-// edges one by one gives) - and a sample ORs / adds the piece on the stretch's way out of LDS
-// instead of going through the entries.  hub_row[v] = row of v in piece_of or -1;
+// Dense pieces.  What a hub contributes to a stretch can be thousands of entries (a layer drawn by importance sits on
+// the hubs), and it is the same for every sample that holds the hub.  Where a vertex has kDensePieceEntries or more
+// neighbours in one stretch, the stretch's piece of that vertex is built once per graph - the importance sum of every
+// vertex of the stretch (7168 64-bit integers, kAbsentSum where there is no edge) - and a sample adds the piece on the
+// stretch's way out of LDS instead of going through the entries.  hub_row[v] = row of v in piece_of or -1;
 // piece_of[row * stretches + stretch] = piece index or kNoPiece.
-constexpr uint32_t kDensePieceEntries = 1024;
-constexpr uint32_t kDensePieceEntriesSums = 2048;  // LADIES form: a piece is 7168 64-bit sums
+constexpr uint32_t kDensePieceEntries = 2048;
 constexpr size_t kDensePieceBudgetBytes = (size_t)2 << 30;
 struct DensePieces {
   const int32_t* hub_row = nullptr;  // nullptr: the graph has none
   const uint32_t* piece_of = nullptr;
-  const uint32_t* words = nullptr;            // FastGCN form: 2048 words of bits per piece
-  const unsigned long long* sums = nullptr;  // LADIES form: 7168 importance sums per piece (kAbsentSum: no edge)
+  const unsigned long long* sums = nullptr;
 };
 
 // LADIES form: the marking kernel turns the importance sums into sampling keys itself where a
@@ -331,198 +332,112 @@ inline uint32_t bitmap_words_for(uint32_t n_vertices) {
   return ((n_vertices + 31u) / 32u + kBitmapTileWords - 1) / kBitmapTileWords * kBitmapTileWords;
 }
 
-// First edge of the sorted adjacency [from, end) whose destination is >= v_hi, given that the
-// destination of `from` is below it; *next = that edge's destination (0xFFFFFFFF: none left).
-// A workgroup waits for the slowest of these searches and each probe is a trip to the caches:
-// a short rest is stepped through edge by edge, a long one galloped and bisected.
-__device__ __forceinline__ EdgePos_t first_edge_at_or_above(const VertexID* __restrict__ edges, EdgePos_t from,
-                                                            EdgePos_t end, uint32_t v_hi, uint32_t* next) {
-  EdgePos_t lo = from;
-  if (end - from <= kShortRest) {
-    uint32_t dst;
-    do {
-      ++lo;
-      dst = lo < end ? (uint32_t)edges[lo] : 0xFFFFFFFFu;
-    } while (dst < v_hi);
-    *next = dst;
-    return lo;
-  }
-  EdgePos_t width = 64;
-  while (lo < end) {
-    const EdgePos_t probe = lo + width < end ? lo + width : end;
-    if ((uint32_t)edges[probe - 1] >= v_hi) break;
-    lo = probe;
-    width <<= 1;
-  }
-  EdgePos_t hi = lo + width < end ? lo + width : end;
-  while (lo < hi) {
-    const EdgePos_t mid = lo + (hi - lo) / 2;
-    if ((uint32_t)edges[mid] < v_hi) lo = mid + 1; else hi = mid;
-  }
-  *next = lo < end ? (uint32_t)edges[lo] : 0xFFFFFFFFu;
-  return lo;
-}
-
-// One wavefront: drops the empty sub-ranges of the per-transit tables (length, first edge,
-// row sum) and turns lengths into starts: starts[k] = first entry of kept sub-range k,
-// starts[kept] = all entries; *ranges = kept.  A length with kPieceFlag set stands for a
-// transit whose entries reach the stretch as a ready-made piece: no sub-range, and the piece
-// index joins the list that takes the place of the lengths, *pieces = how many.  The tables
-// are rewritten in place: an entry moves down or stays, and a round only writes below what it
-// has read.
+// The workgroup's sub-ranges, a lane each (lanes of a wavefront without a transit: length 0), into the tables: those that
+// hold entries in lane order, starts[k] = first entry of sub-range k, starts[kept] = all entries, edge[k] its first edge.
+// A length with kPieceFlag set stands for a transit whose entries reach the stretch as a ready-made piece: its index
+// joins the list `pieces`.  Two barriers; every lane gets the three counts.
 constexpr uint32_t kPieceFlag = 0x80000000u;
-template <bool kWithImportance>
-__device__ __forceinline__ void keep_filled_subranges(uint32_t n_transits, uint32_t lane, uint32_t* lengths,
-                                                      EdgePos_t* edge, float* row_sum, uint32_t* starts,
-                                                      uint32_t* ranges, uint32_t* pieces) {
-  uint32_t kept = 0, entries = 0, listed = 0;
-  for (uint32_t c = 0; c < n_transits; c += 64) {
-    const uint32_t i = c + lane;
-    const uint32_t raw = i < n_transits ? lengths[i] : 0u;
-    const bool is_piece = (raw & kPieceFlag) != 0;
-    const uint32_t len = is_piece ? 0u : raw;
-    const EdgePos_t first = i < n_transits ? edge[i] : 0;
-    const float sum = kWithImportance && i < n_transits ? row_sum[i] : 1.0f;
-    const uint64_t holds = __ballot(len != 0), ready = __ballot(is_piece);
-    const uint64_t below = (1ull << lane) - 1ull;
-    const uint32_t through = wave_inclusive_scan(len);
-    if (len != 0) {
-      const uint32_t k = kept + (uint32_t)__popcll(holds & below);
-      starts[k] = entries + through - len;
-      edge[k] = first;
-      if (kWithImportance) row_sum[k] = sum;
-    }
-    if (is_piece) lengths[listed + (uint32_t)__popcll(ready & below)] = raw & ~kPieceFlag;
-    kept += (uint32_t)__popcll(holds);
-    listed += (uint32_t)__popcll(ready);
-    entries += __shfl(through, 63, kWave);
+struct Subranges {
+  uint32_t ranges, pieces, entries;
+};
+__device__ __forceinline__ Subranges list_subranges(uint32_t raw, EdgePos_t first, uint32_t n_transits, uint32_t* starts,
+                                                    EdgePos_t* edge, uint32_t* pieces, uint4* s_wave) {
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, waves = (n_transits + 63u) / 64u;
+  const bool is_piece = (raw & kPieceFlag) != 0;
+  const uint32_t len = is_piece ? 0u : raw;
+  const uint64_t holds = __ballot(len != 0), ready = __ballot(is_piece), below = (1ull << lane) - 1ull;
+  const uint32_t through = wave < waves ? wave_inclusive_scan(len) : 0u;
+  if (lane == 63 && wave < waves) s_wave[wave] = make_uint4((uint32_t)__popcll(holds), (uint32_t)__popcll(ready), through, 0u);
+  __syncthreads();
+  Subranges all{0, 0, 0}, mine{0, 0, 0};
+  for (uint32_t w = 0; w < waves; ++w) {
+    const uint4 t = s_wave[w];
+    if (w == wave) mine = all;
+    all.ranges += t.x;
+    all.pieces += t.y;
+    all.entries += t.z;
   }
-  if (lane == 0) {
-    starts[kept] = entries;
-    *ranges = kept;
-    *pieces = listed;
+  if (len != 0) {
+    const uint32_t k = mine.ranges + (uint32_t)__popcll(holds & below);
+    starts[k] = mine.entries + through - len;
+    edge[k] = first;
   }
+  if (is_piece) pieces[mine.pieces + (uint32_t)__popcll(ready & below)] = raw & ~kPieceFlag;
+  if (threadIdx.x == 0) starts[all.ranges] = all.entries;
+  __syncthreads();
+  return all;
 }
 
-// A sample without hubs among its transits and with at most this many entries in a
-// workgroup's stretches (a layer whose transits are drawn uniformly) marks them all at once.
-constexpr uint32_t kSparseGroupEntries = 32768;
-constexpr uint32_t kSparseGroupEntriesSums = 2048;  // LADIES form: sums in an LDS table of twice as many slots
+// A sample without hubs among its transits and with at most this many entries in a workgroup's stretches (a layer whose
+// transits are drawn uniformly) adds them all up at once, in an LDS table of twice as many slots.
+constexpr uint32_t kSparseGroupEntries = 2048;
 
-// Two workgroups of 16 wavefronts share a compute unit only at 8 wavefronts per SIMD, which the
-// kernel's attributes ask the compiler for.  Measured without them: 63 (LADIES form) and 66
-// registers per lane, 7 wavefronts per SIMD, one workgroup resident, and the LADIES form takes
-// 1.6 times as long; the LDS size (tried: 62 to 70 KB) makes no difference.
-template <bool kWithImportance>
+// The samples that are not ranked in LDS (ranked_layer): the keys of sample `at` of them go to keys + at * keys_per_sample.
+// Two workgroups of 16 wavefronts share a compute unit only at 8 wavefronts per SIMD, which the kernel's attributes ask
+// the compiler for.
+// 500 K vertices, 12 M edges, second layer of 1024 samples of 512 (1.5 M pairs a sample): see the engine's rank_by_keys.
 __global__ __launch_bounds__(kBinThreads, 8) __attribute__((amdgpu_num_vgpr(56))) void collective_mark_binned(
-    CSRPartition csr, TransitView tv, int32_t invalid, uint32_t n_samples, uint32_t bins_per_sample,
-    uint32_t* __restrict__ bitmap,
-    uint32_t words_per_sample, const float* __restrict__ inverse_row_sums,
-    uint32_t keys_per_sample, DensePieces dense, KeysOnTheWayOut keys_out) {
-  constexpr uint32_t kBinWords = kWithImportance ? kBinVerticesSums / 32u : kBinWordsBits;
-  constexpr uint32_t kBinVertices = kBinWords * 32u;
-  // FastGCN form: a byte per vertex, set with plain LDS stores (every writer stores 1) and
-  // packed into bits on the way out; LADIES form: bits and 64-bit sums, LDS atomics
-  __shared__ __align__(16) uint32_t s_bits[kWithImportance ? kBinWords : kBinVertices / 4u];
-  __shared__ __align__(16) unsigned long long s_acc[kWithImportance ? kBinVerticesSums : 1];
-  uint8_t* s_bytes = (uint8_t*)s_bits;
+    MergedEdges merged, TransitView tv, int32_t invalid, uint32_t n_samples, const uint32_t* __restrict__ n_marked,
+    const uint32_t* __restrict__ marked, uint32_t bins_per_sample, uint32_t keys_per_sample, DensePieces dense,
+    KeysOnTheWayOut keys_out) {
+  __shared__ __align__(16) uint32_t s_bits[kBinWords];  // where some terms are 0
+  __shared__ __align__(16) unsigned long long s_acc[kBinVertices];
   // the sub-ranges that hold entries, in transit order
   __shared__ uint32_t s_start[kMaxLayerTransits + 1];  // first entry of sub-range k among the stretch's entries
   __shared__ EdgePos_t s_edge[kMaxLayerTransits];      // its first edge
-  __shared__ float s_row_sum[kWithImportance ? kMaxLayerTransits : 1];  // 1 / (the weights of its transit added up)
-  __shared__ uint32_t s_length[kMaxLayerTransits];     // length of every transit's sub-range, then the stretch's dense pieces
-  __shared__ uint32_t s_ranges;                        // sub-ranges kept
-  __shared__ uint32_t s_pieces;                        // dense pieces listed
-  // A workgroup takes kBinsPerGroup consecutive stretches of one sample, one after the other:
-  // where a transit's sub-range ends in one stretch it begins in the next, and the end is
-  // then only a short gallop away instead of a search of the whole adjacency.
-  constexpr uint32_t kBinsPerGroup = kWithImportance ? kBinsPerGroupSums : kBinsPerGroupBits;
-  // the low stretches hold the hubs and take longest: all samples' first groups start first
+  __shared__ uint32_t s_piece[kMaxLayerTransits];      // the stretch's dense pieces
+  __shared__ uint4 s_wave[kBinWaves];
+  // A workgroup takes kBinsPerGroup consecutive stretches of one sample, one after the other: where a transit's sub-range
+  // ends in one stretch it begins in the next, and the end is then only a short gallop away instead of a search of the
+  // whole adjacency.  The low stretches hold the hubs and take longest: all samples' first groups start first.
   const uint32_t group = blockIdx.x / n_samples;
-  const uint32_t s = blockIdx.x - group * n_samples;
+  const uint32_t at = blockIdx.x - group * n_samples;
+  if (at >= *n_marked) return;
+  const uint32_t s = marked[at];
   const uint32_t first_bin = group * kBinsPerGroup;
   const int32_t* transits = tv.base + (size_t)s * tv.stride;
+  uint32_t* my_keys = keys_out.keys + (size_t)at * keys_per_sample;
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wave = threadIdx.x >> 6;
-  // tv.count <= kBinThreads: lane i keeps transit i's adjacency and how far the stretches
-  // before this one reach into it
+  // tv.count <= kBinThreads: lane i keeps transit i's adjacency and how far the stretches before this one reach into it
   EdgePos_t my_end = 0, my_reach = 0;
   uint32_t my_next = 0xFFFFFFFFu;  // destination of edge my_reach; none left: above every vertex
-  float my_row_sum = 1.0f;
-  int32_t my_hub = -1;
+  int32_t my_hub = -1, my_cut_row = -1;
   int32_t my_transit = -1;
   if (threadIdx.x < tv.count) {
     my_transit = transits[threadIdx.x];
     if (my_transit == invalid) my_transit = -1;
     if (my_transit != -1 && dense.hub_row) my_hub = dense.hub_row[my_transit];
+    if (my_transit != -1 && merged.cut_row_of) my_cut_row = merged.cut_row_of[my_transit];
   }
-  bool hubs_among_transits = false;
-  if (!kWithImportance) {
-    // the byte map starts out clear and every stretch leaves it clear: what it reads on the
-    // way out it sets back to zero, so no stretch spends a pass on clearing
-    for (uint32_t i = threadIdx.x; i < kBinVertices / 4u; i += kBinThreads) s_bits[i] = 0;
-    if (threadIdx.x < tv.count) s_start[threadIdx.x] = (uint32_t)my_transit;  // the table is free until the first stretch
-    hubs_among_transits = __syncthreads_or(my_hub >= 0) != 0;
-    // A vertex marks the same bits however often it is among the transits, and a layer drawn
-    // with replacement by degree^2 repeats its hubs: 29 distinct transits of 64 at full size,
-    // four fifths of all entries belong to repeats.  Only a vertex's first occurrence counts.
-    if (my_transit != -1) {
-      bool repeated = false;
-      for (uint32_t j = 0; j < threadIdx.x; ++j) repeated |= s_start[j] == (uint32_t)my_transit;
-      if (repeated) {
-        my_transit = -1;
-        my_hub = -1;
-      }
-    }
-    __syncthreads();  // the table is written next
-  } else {
-    hubs_among_transits = __syncthreads_or(my_hub >= 0) != 0;
+  const bool hubs_among_transits = __syncthreads_or(my_hub >= 0) != 0;
+  const HubCut* my_cuts = merged.cuts + (my_cut_row < 0 ? 0 : (size_t)my_cut_row * (bins_per_sample + 1));
+  if (my_transit != -1) {
+    my_end = merged.row_ptr[my_transit + 1];
+    my_reach = my_cut_row >= 0 ? my_cuts[first_bin].from
+                               : first_edge_from(merged.ids, merged.row_ptr[my_transit], my_end, first_bin * kBinVertices);
+    if (my_cut_row < 0 && my_reach < my_end) my_next = (uint32_t)merged.ids[my_reach];
   }
-  if (threadIdx.x < tv.count) {
-    const int32_t t = my_transit;
-    if (t != -1) {
-      my_end = csr.row_ptr[t + 1];
-      EdgePos_t lo = csr.row_ptr[t], hi = my_end;  // first edge whose destination is in the first stretch or above
-      const uint32_t v_first = first_bin * kBinVertices;
-      while (lo < hi) {
-        const EdgePos_t mid = lo + (hi - lo) / 2;
-        if ((uint32_t)csr.edges[mid] < v_first) lo = mid + 1; else hi = mid;
-      }
-      my_reach = lo;
-      if (lo < my_end) my_next = (uint32_t)csr.edges[lo];
-      if (kWithImportance) my_row_sum = inverse_row_sums[t];
-    }
-  }
-  if (kWithImportance && !hubs_among_transits) {
-    // LADIES form, a sample without hubs: the stretches of the workgroup as one.  At most kSparseGroupEntriesSums entries: their sums are
-    // gathered in an LDS table hashed by vertex (in the room of the per-vertex sums), the
-    // keys of the whole range are written as absent, and the table's vertices then get theirs.
-    // Stretch by stretch, 16 chains of searches, tables and barriers cost a workgroup 130 us
-    // for a few hundred entries.
+  if (!hubs_among_transits) {
+    // The stretches of the workgroup as one: the sums are gathered in an LDS table hashed by vertex (in the room of the
+    // per-vertex sums), the keys of the whole range are written as absent, and the table's vertices then get theirs.
+    // Stretch by stretch, 16 chains of searches, tables and barriers cost a workgroup 130 us for a few hundred entries.
     const uint32_t group_bins = first_bin + kBinsPerGroup < bins_per_sample ? kBinsPerGroup : bins_per_sample - first_bin;
     const uint32_t v_lo = first_bin * kBinVertices, v_hi = v_lo + group_bins * kBinVertices;
-    if (threadIdx.x < tv.count) {
-      uint32_t unused;
-      const EdgePos_t stop =
-          my_next < v_hi ? first_edge_at_or_above(csr.edges, my_reach, my_end, v_hi, &unused) : my_reach;
-      s_length[threadIdx.x] = (uint32_t)(stop - my_reach);
-      s_edge[threadIdx.x] = my_reach;
-      s_row_sum[threadIdx.x] = my_row_sum;
-    }
-    __syncthreads();
-    if (wave == 0) keep_filled_subranges<true>(tv.count, lane, s_length, s_edge, s_row_sum, s_start, &s_ranges, &s_pieces);
-    __syncthreads();
-    const uint32_t ranges = s_ranges;
-    const uint32_t size = s_start[ranges];
-    if (size <= kSparseGroupEntriesSums) {
-      constexpr uint32_t kSlots = 2u * kSparseGroupEntriesSums;  // a power of two
+    EdgePos_t stop = my_reach;
+    if (my_cut_row >= 0) stop = my_cuts[first_bin + group_bins].from;
+    else if (my_next < v_hi) stop = first_edge_from(merged.ids, my_reach, my_end, v_hi);
+    const Subranges all = list_subranges((uint32_t)(stop - my_reach), my_reach, tv.count, s_start, s_edge, s_piece, s_wave);
+    const uint32_t ranges = all.ranges, size = all.entries;
+    if (size <= kSparseGroupEntries) {
+      constexpr uint32_t kSlots = 2u * kSparseGroupEntries;  // a power of two
       unsigned long long* slot_sum = s_acc;
       uint32_t* slot_vertex = (uint32_t*)(s_acc + kSlots);
       for (uint32_t i = threadIdx.x; i < kSlots; i += kBinThreads) {
         slot_vertex[i] = 0xFFFFFFFFu;
         slot_sum[i] = 0;
       }
-      uint32_t* out_keys = keys_out.keys + (size_t)s * keys_per_sample + v_lo;
+      uint32_t* out_keys = my_keys + v_lo;
       for (uint32_t i = threadIdx.x; i < group_bins * kBinVertices; i += kBinThreads) out_keys[i] = kAbsentKey;
       __syncthreads();
       for (uint32_t e = threadIdx.x; e < size; e += kBinThreads) {
@@ -532,229 +447,116 @@ __global__ __launch_bounds__(kBinThreads, 8) __attribute__((amdgpu_num_vgpr(56))
           if (s_start[mid] <= e) lo = mid; else hi = mid;
         }
         const EdgePos_t src = s_edge[lo] + (EdgePos_t)(e - s_start[lo]);
-        const uint32_t local = (uint32_t)csr.edges[src] - v_lo;
-        const float p = csr.weights[src] * s_row_sum[lo];
-        const unsigned long long term = importance_term_fixed(p * p);
+        const uint32_t local = (uint32_t)merged.ids[src] - v_lo;
         uint32_t slot = (local * 2654435761u) >> 20 & (kSlots - 1u);
         for (;;) {  // at most half of the slots are ever taken
           const uint32_t before = atomicCAS(&slot_vertex[slot], 0xFFFFFFFFu, local);
           if (before == 0xFFFFFFFFu || before == local) break;
           slot = (slot + 1u) & (kSlots - 1u);
         }
-        if (term != 0) atomicAdd(&slot_sum[slot], term);
+        atomicAdd(&slot_sum[slot], merged.terms[src]);
       }
       __syncthreads();  // the table is complete, and the absent keys have been written
       for (uint32_t i = threadIdx.x; i < kSlots; i += kBinThreads) {
         const uint32_t local = slot_vertex[i];
         if (local == 0xFFFFFFFFu) continue;
-        const uint32_t v = v_lo + local;
-        out_keys[local] = ladies_key_bits(slot_sum[i], ladies_pair_index(keys_out.first_sample + s, keys_out.n_vertices, v),
+        out_keys[local] = ladies_key_bits(slot_sum[i], ladies_pair_index(keys_out.first_sample + s, keys_out.n_vertices, v_lo + local),
                                           keys_out.step, keys_out.seed);
       }
       return;
     }
-    // too many entries for that: stretch by stretch (the tables are next written after every
-    // lane has read the size above)
-  }
-  if (!kWithImportance && !hubs_among_transits) {
-    // The stretches of the workgroup as one: a bit per vertex fits the same LDS, and the few
-    // entries can afford LDS atomics.  Per stretch, the searches, the table and the way out
-    // are chains of dependent trips (to the caches, to LDS, through barriers) that cost the
-    // same however few entries there are: 3.5 ms a layer at full size for 2 K entries a sample.
-    const uint32_t group_bins = first_bin + kBinsPerGroup < bins_per_sample ? kBinsPerGroup : bins_per_sample - first_bin;
-    const uint32_t v_lo = first_bin * kBinVertices, v_hi = v_lo + group_bins * kBinVertices;
-    if (threadIdx.x < tv.count) {
-      uint32_t unused;
-      const EdgePos_t stop =
-          my_next < v_hi ? first_edge_at_or_above(csr.edges, my_reach, my_end, v_hi, &unused) : my_reach;
-      s_length[threadIdx.x] = (uint32_t)(stop - my_reach);
-      s_edge[threadIdx.x] = my_reach;
-    }
+    // too many entries for that: stretch by stretch
     __syncthreads();
-    if (wave == 0) keep_filled_subranges<false>(tv.count, lane, s_length, s_edge, nullptr, s_start, &s_ranges, &s_pieces);
-    __syncthreads();
-    const uint32_t ranges = s_ranges;
-    const uint32_t size = s_start[ranges];
-    if (size <= kSparseGroupEntries) {
-      for (uint32_t e = threadIdx.x; e < size; e += kBinThreads) {
-        uint32_t lo = 0, hi = ranges;  // the sub-range that holds entry e
-        while (hi - lo > 1) {
-          const uint32_t mid = lo + (hi - lo) / 2;
-          if (s_start[mid] <= e) lo = mid; else hi = mid;
-        }
-        const uint32_t local = (uint32_t)csr.edges[s_edge[lo] + (EdgePos_t)(e - s_start[lo])] - v_lo;
-        atomicOr(&s_bits[local >> 5], 1u << (local & 31u));
-      }
-      __syncthreads();
-      const uint32_t first_word = first_bin * kBinWords;
-      uint32_t* out = bitmap + (size_t)s * words_per_sample + first_word;
-      for (uint32_t i = threadIdx.x; i < group_bins * kBinWords && first_word + i < words_per_sample; i += kBinThreads)
-        out[i] = s_bits[i];
-      return;
-    }
-    // too many entries for that: stretch by stretch (nothing has been marked, and the tables
-    // are next written after every lane has read the size above)
   }
+  EdgePos_t cut_after = my_cut_row >= 0 ? my_cuts[first_bin + 1].from : 0;  // the end of the coming stretch, fetched one stretch ahead
   for (uint32_t bin = first_bin; bin < first_bin + kBinsPerGroup && bin < bins_per_sample; ++bin) {
-  const uint32_t v_lo = bin * kBinVertices;
-  if (kWithImportance) {
-    for (uint32_t i = threadIdx.x; i < kBinWords; i += kBinThreads) s_bits[i] = 0;
-    for (uint32_t i = threadIdx.x; i < kBinVerticesSums; i += kBinThreads) s_acc[i] = 0;
-  }
-  if (threadIdx.x < tv.count) {
+    const uint32_t v_lo = bin * kBinVertices;
+    if (merged.zero_terms)
+      for (uint32_t i = threadIdx.x; i < kBinWords; i += kBinThreads) s_bits[i] = 0;
+    for (uint32_t i = threadIdx.x; i < kBinVertices; i += kBinThreads) s_acc[i] = 0;
+    uint32_t length = 0;
     const EdgePos_t my_from = my_reach;
-    const uint32_t v_hi = v_lo + kBinVertices;
-    // nothing is fetched where the next edge already lies beyond the stretch (a short
-    // adjacency misses most stretches)
-    if (my_next < v_hi) my_reach = first_edge_at_or_above(csr.edges, my_from, my_end, v_hi, &my_next);
-    uint32_t length = (uint32_t)(my_reach - my_from);
-    if (my_hub >= 0 && length != 0) {
-      const uint32_t piece = dense.piece_of[(size_t)my_hub * bins_per_sample + bin];
-      if (piece != kNoPiece) length = kPieceFlag | piece;  // these entries reach the stretch ready-made
-    }
-    s_length[threadIdx.x] = length;
-    s_edge[threadIdx.x] = my_from;  // by transit for now
-    if (kWithImportance) s_row_sum[threadIdx.x] = my_row_sum;
-  }
-  __syncthreads();
-  if (wave == 0)
-    keep_filled_subranges<kWithImportance>(tv.count, lane, s_length, s_edge, s_row_sum, s_start, &s_ranges, &s_pieces);
-  __syncthreads();
-  const uint32_t ranges = s_ranges;
-  const uint32_t size = s_start[ranges];
-  // every wavefront walks a contiguous part of the entries, 64 * kBinAhead per round
-  constexpr uint32_t kRound = 64u * kBinAhead;
-  const uint32_t part = (size + kBinWaves * kRound - 1) / (kBinWaves * kRound) * kRound;
-  const uint32_t part_begin = wave * part;
-  const uint32_t part_end = part_begin + part < size ? part_begin + part : size;
-  uint32_t cur = 0, cur_begin = 0, cur_end = 0;
-  EdgePos_t cur_edges = 0;
-  float cur_row_sum = 1.0f;
-  if (part_begin + lane < part_end) {  // the sub-range of the lane's first entry
-    const uint32_t e = part_begin + lane;
-    uint32_t lo = 0, hi = ranges;
-    while (hi - lo > 1) {
-      const uint32_t mid = lo + (hi - lo) / 2;
-      if (s_start[mid] <= e) lo = mid; else hi = mid;
-    }
-    cur = lo;
-    cur_begin = s_start[lo];
-    cur_end = s_start[lo + 1];
-    cur_edges = s_edge[lo];
-    if (kWithImportance) cur_row_sum = s_row_sum[lo];
-  }
-  if (!kWithImportance) {
-    // FastGCN form: nothing is shared between neighbouring entries, so a lane takes four
-    // consecutive entries per round - one 16-byte load and one round of index arithmetic for
-    // four marks (the kernel is bound by instruction issue: its edge stream comes from the
-    // caches) - unless its four entries straddle the end of a sub-range or of the part.
-    struct __attribute__((packed, aligned(4))) FourIds { uint32_t id[4]; };
-    for (uint32_t e0 = part_begin; e0 < part_end; e0 += kRound) {
-      const uint32_t e = e0 + lane * kBinAhead;
-      if (e >= part_end) continue;
-      if (e >= cur_end) {
-        do {
-          ++cur;
-          cur_begin = cur_end;
-          cur_end = s_start[cur + 1];
-        } while (e >= cur_end);
-        cur_edges = s_edge[cur];
+    if (my_transit != -1) {
+      const uint32_t v_hi = v_lo + kBinVertices;
+      if (my_cut_row >= 0) {
+        my_reach = cut_after;
+        if (bin + 2 <= bins_per_sample) cut_after = my_cuts[bin + 2].from;
+      } else if (my_next < v_hi) {  // nothing is fetched where the next edge already lies beyond the stretch
+        my_reach = first_edge_from(merged.ids, my_from, my_end, v_hi);
+        my_next = my_reach < my_end ? (uint32_t)merged.ids[my_reach] : 0xFFFFFFFFu;
       }
-      if (e + kBinAhead <= cur_end && e + kBinAhead <= part_end) {
-        FourIds four;
-        __builtin_memcpy(&four, csr.edges + cur_edges + (EdgePos_t)(e - cur_begin), sizeof(four));
+      length = (uint32_t)(my_reach - my_from);
+      if (my_hub >= 0 && length != 0) {
+        const uint32_t piece = dense.piece_of[(size_t)my_hub * bins_per_sample + bin];
+        if (piece != kNoPiece) length = kPieceFlag | piece;  // these entries reach the stretch ready-made
+      }
+    }
+    const Subranges all = list_subranges(length, my_from, tv.count, s_start, s_edge, s_piece, s_wave);
+    const uint32_t ranges = all.ranges, size = all.entries;
+    // every wavefront walks a contiguous part of the entries, 64 * kBinAhead per round
+    constexpr uint32_t kRound = 64u * kBinAhead;
+    const uint32_t part = (size + kBinWaves * kRound - 1) / (kBinWaves * kRound) * kRound;
+    const uint32_t part_begin = wave * part;
+    const uint32_t part_end = part_begin + part < size ? part_begin + part : size;
+    uint32_t cur = 0, cur_begin = 0, cur_end = 0;
+    EdgePos_t cur_edges = 0;
+    if (part_begin + lane < part_end) {  // the sub-range of the lane's first entry
+      const uint32_t e = part_begin + lane;
+      uint32_t lo = 0, hi = ranges;
+      while (hi - lo > 1) {
+        const uint32_t mid = lo + (hi - lo) / 2;
+        if (s_start[mid] <= e) lo = mid; else hi = mid;
+      }
+      cur = lo;
+      cur_begin = s_start[lo];
+      cur_end = s_start[lo + 1];
+      cur_edges = s_edge[lo];
+    }
+    for (uint32_t e0 = part_begin; e0 < part_end; e0 += kRound) {
+      uint32_t locals[kBinAhead];  // vertex - v_lo
+      unsigned long long terms[kBinAhead];
 #pragma unroll
-        for (uint32_t a = 0; a < kBinAhead; ++a) s_bytes[four.id[a] - v_lo] = 1;
-      } else {
-        for (uint32_t a = 0; a < kBinAhead && e + a < part_end; ++a) {
-          while (e + a >= cur_end) {
-            ++cur;
-            cur_begin = cur_end;
-            cur_end = s_start[cur + 1];
+      for (uint32_t a = 0; a < kBinAhead; ++a) {
+        const uint32_t e = e0 + a * 64u + lane;
+        locals[a] = 0xFFFFFFFFu;
+        terms[a] = 0;
+        if (e < part_end) {
+          if (e >= cur_end) {
+            do {  // no sub-range is empty
+              ++cur;
+              cur_begin = cur_end;
+              cur_end = s_start[cur + 1];
+            } while (e >= cur_end);
             cur_edges = s_edge[cur];
           }
-          s_bytes[(uint32_t)csr.edges[cur_edges + (EdgePos_t)(e + a - cur_begin)] - v_lo] = 1;
+          const EdgePos_t src = cur_edges + (EdgePos_t)(e - cur_begin);
+          locals[a] = (uint32_t)merged.ids[src] - v_lo;
+          terms[a] = merged.terms[src];
         }
       }
-    }
-  }
-  for (uint32_t e0 = part_begin; kWithImportance && e0 < part_end; e0 += kRound) {  // the same trip count for every lane of a wave
-    uint32_t locals[kBinAhead];  // vertex - v_lo
-    float weights[kBinAhead], sums_of_row[kBinAhead];
 #pragma unroll
-    for (uint32_t a = 0; a < kBinAhead; ++a) {
-      const uint32_t e = e0 + a * 64u + lane;
-      locals[a] = 0xFFFFFFFFu;
-      weights[a] = 0.0f;
-      sums_of_row[a] = 1.0f;
-      if (e < part_end) {
-        if (e >= cur_end) {
-          do {  // no sub-range is empty: at most a few steps
-            ++cur;
-            cur_begin = cur_end;
-            cur_end = s_start[cur + 1];
-          } while (e >= cur_end);
-          cur_edges = s_edge[cur];
-          if (kWithImportance) cur_row_sum = s_row_sum[cur];
-        }
-        const EdgePos_t src = cur_edges + (EdgePos_t)(e - cur_begin);
-        locals[a] = (uint32_t)csr.edges[src] - v_lo;
-        if (kWithImportance) {
-          weights[a] = csr.weights[src];
-          sums_of_row[a] = cur_row_sum;
-        }
+      for (uint32_t a = 0; a < kBinAhead; ++a) {
+        if (locals[a] == 0xFFFFFFFFu) continue;
+        atomicAdd(&s_acc[locals[a]], terms[a]);
+        if (merged.zero_terms) atomicOr(&s_bits[locals[a] >> 5], 1u << (locals[a] & 31u));
       }
     }
-#pragma unroll
-    for (uint32_t a = 0; a < kBinAhead; ++a) {
-      const uint32_t local = locals[a];
-      if (kWithImportance) {
-        unsigned long long term = 0;
-        if (local != 0xFFFFFFFFu) {
-          const float p = weights[a] * sums_of_row[a];
-          term = importance_term_fixed(p * p);
-        }
-        // Parallel edges sit in neighbouring lanes.  A few of them may as well hit the same
-        // LDS word one after the other; a run of four or more somewhere in the wave (hub pairs
-        // are joined by thousands of edges) is added up first, inside the rows of 16 lanes.
-        // 0xFFFFFFFE: no lane holds it, so lane 0 always starts a segment.
-        const uint32_t left = wave_from_below(0xFFFFFFFEu, local);
-        uint32_t closed = (left != local || (lane & 15u) == 0) ? 1u : 0u;
-        const uint64_t repeats = __ballot(left == local && local != 0xFFFFFFFFu);
-        bool adds = true;  // this lane adds its term to the vertex's sum
-        if ((repeats & (repeats >> 1) & (repeats >> 2)) != 0) {
-          segmented_row_step<1>(closed, term);
-          segmented_row_step<2>(closed, term);
-          segmented_row_step<4>(closed, term);
-          segmented_row_step<8>(closed, term);
-          const uint32_t right = wave_from_above(0xFFFFFFFEu, local);
-          adds = right != local || (lane & 15u) == 15u;
-        }
-        if (local != 0xFFFFFFFFu && adds) {
-          if (term != 0) atomicAdd(&s_acc[local], term);
-          atomicOr(&s_bits[local >> 5], 1u << (local & 31u));
-        }
-      } else if (local != 0xFFFFFFFFu) {
-        s_bytes[local] = 1;
-      }
-    }
-  }
-  __syncthreads();
-  if (kWithImportance) {
-    // LADIES form: what leaves the workgroup is the sampling key of every vertex of the
-    // stretch (kAbsentKey where the neighbourhood does not hold the vertex); no bitmap.
-    // A lane takes four consecutive vertices: 16-byte accesses to LDS, to the pieces and to
+    __syncthreads();
+    // What leaves the workgroup is the sampling key of every vertex of the stretch (kAbsentKey where the neighbourhood
+    // does not hold the vertex).  A lane takes four consecutive vertices: 16-byte accesses to LDS, to the pieces and to
     // the output, and one Philox block where it forms keys.
-    const uint32_t n_pieces = s_pieces;
-    for (uint32_t q = threadIdx.x; q < kBinVerticesSums / 4u; q += kBinThreads) {
+    const uint32_t n_pieces = all.pieces;
+    for (uint32_t q = threadIdx.x; q < kBinVertices / 4u; q += kBinThreads) {
       const uint32_t i = 4u * q;
-      const uint32_t bits = (s_bits[i >> 5] >> (i & 31u)) & 15u;
       const ulonglong2 low = ((const ulonglong2*)s_acc)[2u * q], high = ((const ulonglong2*)s_acc)[2u * q + 1u];
       unsigned long long sum[4] = {low.x, low.y, high.x, high.y};  // 0 where nothing was added
-      bool present[4] = {(bits & 1u) != 0, (bits & 2u) != 0, (bits & 4u) != 0, (bits & 8u) != 0};
+      const uint32_t bits = merged.zero_terms ? (s_bits[i >> 5] >> (i & 31u)) & 15u : 0u;
+      bool present[4];
+#pragma unroll
+      for (uint32_t k = 0; k < 4; ++k) present[k] = sum[k] != 0 || (bits >> k & 1u) != 0;
 #pragma unroll 4
-      for (uint32_t p = 0; p < n_pieces; ++p) {  // integer sums: the order of the additions does not matter
-        const ulonglong2* piece = (const ulonglong2*)(dense.sums + (size_t)s_length[p] * kBinVerticesSums + i);
+      for (uint32_t p = 0; p < n_pieces; ++p) {
+        const ulonglong2* piece = (const ulonglong2*)(dense.sums + (size_t)s_piece[p] * kBinVertices + i);
         const ulonglong2 a = piece[0], b = piece[1];
         const unsigned long long ready[4] = {a.x, a.y, b.x, b.y};
 #pragma unroll
@@ -772,46 +574,163 @@ __global__ __launch_bounds__(kBinThreads, 8) __attribute__((amdgpu_num_vgpr(56))
         for (uint32_t k = 0; k < 4; ++k)
           if (present[k]) key[k] = ladies_key_from_word(sum[k], blk.w[k]);
       }
-      *(uint4*)(keys_out.keys + (size_t)s * keys_per_sample + v_lo + i) = make_uint4(key[0], key[1], key[2], key[3]);
+      *(uint4*)(my_keys + v_lo + i) = make_uint4(key[0], key[1], key[2], key[3]);
     }
-  } else {
-    const uint32_t first_word = bin * kBinWords;
-    uint32_t* out = bitmap + (size_t)s * words_per_sample + first_word;
-    const uint32_t n_pieces = s_pieces;
-    // two words per lane (stretches and bitmaps hold even numbers of words): eight bytes per
-    // load of a piece, several pieces under way
-    const uint32_t i = 2u * threadIdx.x;
-    if (i < kBinWords && first_word + i < words_per_sample) {
-      uint2 words = make_uint2(0u, 0u);
-      if (size != 0) {  // 2 x 32 bytes, each 0 or 1 -> 2 x 32 bits
-        uint4* bytes = (uint4*)s_bits + i * 2u;
-        const uint4 q0 = bytes[0], q1 = bytes[1], q2 = bytes[2], q3 = bytes[3];
-        const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
-        bytes[0] = zero;
-        bytes[1] = zero;
-        bytes[2] = zero;
-        bytes[3] = zero;
-        const uint32_t low[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
-        const uint32_t high[8] = {q2.x, q2.y, q2.z, q2.w, q3.x, q3.y, q3.z, q3.w};
+    __syncthreads();  // the next stretch clears what this one has just read
+  }
+}
+
+// ---- LADIES form: small neighbourhoods, ranked in LDS -------------------------------------
+
+// Entries (pairs) of a sample's neighbourhood up to which it is ranked by one workgroup in LDS; the others, in whatever
+// order they are found, are listed.
+constexpr uint32_t kRankedEntries = 8192;
+constexpr uint32_t kRankedThreads = 1024;
+
+// A wavefront per sample: sizes[s] = entries of its neighbourhood, parallel edges and all (saturated).
+__global__ __launch_bounds__(kSortOutThreads) void sort_out_ranked(CSRPartition csr, MergedEdges merged, TransitView tv,
+                                                                   uint32_t n_samples, int32_t invalid,
+                                                                   uint32_t* __restrict__ sizes,
+                                                                   uint32_t* __restrict__ merged_sizes,
+                                                                   uint32_t* __restrict__ n_marked,
+                                                                   uint32_t* __restrict__ marked,
+                                                                   uint32_t* __restrict__ too_long) {
+  __shared__ uint32_t s_taken, s_base;
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t s = blockIdx.x * (kSortOutThreads / 64u) + (threadIdx.x >> 6);
+  if (threadIdx.x == 0) s_taken = 0;
+  __syncthreads();
+  uint64_t both = 0, pairs = 0;
+  for (uint32_t i = lane; i < tv.count && s < n_samples; i += 64u) {
+    const int32_t t = tv.base[(size_t)s * tv.stride + i];
+    if (t == invalid || t == -1) continue;
+    both += (uint64_t)(csr.row_ptr[t + 1] - csr.row_ptr[t]);
+    pairs += (uint64_t)(merged.row_ptr[t + 1] - merged.row_ptr[t]);
+  }
+  both = __shfl(wave_inclusive_scan_u64(both), 63, kWave);
+  pairs = __shfl(wave_inclusive_scan_u64(pairs), 63, kWave);
+  uint32_t at = 0;
+  if (lane == 0 && s < n_samples) {
+    sizes[s] = both > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)both;
+    merged_sizes[s] = pairs > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)pairs;
+    if (both >= (1ull << 31)) *too_long = 1;
+    if (pairs > kRankedEntries) at = atomicAdd(&s_taken, 1u);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0 && s_taken) s_base = atomicAdd(n_marked, s_taken);
+  __syncthreads();
+  if (lane == 0 && s < n_samples && pairs > kRankedEntries) marked[s_base + at] = s;
+}
+
+// A workgroup per sample: fetches the entries, sorts them by vertex, adds their terms up, forms the keys and sorts the
+// vertices by them (equal keys by vertex, as the sorts are stable).  Marked stretch by stretch, a layer of 1024 such samples
+// over 500 K vertices wrote and read 4 GB of keys, most of them absent.
+template <class Draw>
+__device__ __forceinline__ void ranked_layer(const MergedEdges& merged, uint32_t n_vertices, const int32_t* transits,
+                                             uint32_t n_transits, int32_t invalid, uint32_t size, uint64_t sample,
+                                             uint32_t step, uint64_t seed, uint32_t* __restrict__ distinct_out, Draw draw) {
+  constexpr uint32_t kEach = kRankedEntries / kRankedThreads;
+  // two buffers of ids with one for the kept ids between them: next to whichever the sort leaves free it makes the sums' room
+  __shared__ __align__(16) uint32_t s_words[3 * kRankedEntries];
+  __shared__ uint16_t s_payload[2][kRankedEntries];
+  __shared__ uint32_t s_start[kMaxLayerTransits];
+  __shared__ EdgePos_t s_edge[kMaxLayerTransits];
+  __shared__ uint32_t s_count[kRankedThreads / 64][kSortedDigits];
+  __shared__ uint32_t s_wave_count[kRankedThreads / 64];
+  static_assert(kMaxLayerTransits <= kRankedThreads && kRankedEntries <= 65536, "a lane a transit; 16 bits an entry");
+  uint32_t* const kept = s_words + kRankedEntries;
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  auto before_wave = [&](uint32_t through, uint32_t* all) {  // exclusive prefix of a wavefront's total
+    if (lane == 63) s_wave_count[wave] = through;
+    __syncthreads();
+    uint32_t before = 0, total = 0;
+    for (uint32_t w = 0; w < kRankedThreads / 64; ++w) {
+      if (w < wave) before += s_wave_count[w];
+      total += s_wave_count[w];
+    }
+    __syncthreads();
+    *all = total;
+    return before;
+  };
+  uint32_t total;
+  {
+    const int32_t t = threadIdx.x < n_transits ? transits[threadIdx.x] : -1;
+    EdgePos_t begin = 0;
+    uint32_t degree = 0;
+    if (t != invalid && t != -1) {
+      begin = merged.row_ptr[t];
+      degree = (uint32_t)(merged.row_ptr[t + 1] - begin);
+    }
+    const uint32_t through = wave_inclusive_scan(degree);
+    const uint32_t before = before_wave(through, &total);
+    if (threadIdx.x < n_transits) {
+      s_start[threadIdx.x] = before + through - degree;
+      s_edge[threadIdx.x] = begin;
+    }
+    __syncthreads();
+  }
+  auto edge_of = [&](uint32_t e) {
+    uint32_t lo = 0, hi = n_transits;  // the last transit that starts at e or before (empty ones start where the next does)
+    while (hi - lo > 1) {
+      const uint32_t mid = lo + (hi - lo) / 2;
+      if (s_start[mid] <= e) lo = mid; else hi = mid;
+    }
+    return s_edge[lo] + (EdgePos_t)(e - s_start[lo]);
+  };
+  for (uint32_t e = threadIdx.x; e < size; e += kRankedThreads) {
+    s_words[e] = (uint32_t)merged.ids[edge_of(e)];
+    s_payload[0][e] = (uint16_t)e;
+  }
+  __syncthreads();
+  SortedIds sorted{s_words, s_words + 2 * kRankedEntries, s_payload[0], s_payload[1]};
+  sorted = sort_ids<kRankedThreads, true>(sorted, s_count, s_wave_count, size, 32u - (uint32_t)__clz((int)n_vertices));
+  // which of a lane's entries are a vertex's first, and how many vertices come before
+  unsigned long long* sums = (unsigned long long*)(sorted.other == s_words ? s_words : kept);
+  for (uint32_t i = threadIdx.x; i < kRankedEntries; i += kRankedThreads) sums[i] = 0;
+  uint32_t id[kEach], firsts = 0;
+  uint32_t last = threadIdx.x != 0 && threadIdx.x * kEach <= size ? sorted.ids[threadIdx.x * kEach - 1] : 0xFFFFFFFFu;
 #pragma unroll
-        for (uint32_t q = 0; q < 8; ++q) {
-          const uint32_t four = low[q], next_four = high[q];
-          words.x |= ((four & 1u) | ((four >> 7) & 2u) | ((four >> 14) & 4u) | ((four >> 21) & 8u)) << (4u * q);
-          words.y |= ((next_four & 1u) | ((next_four >> 7) & 2u) | ((next_four >> 14) & 4u) | ((next_four >> 21) & 8u))
-                     << (4u * q);
-        }
-      }
-#pragma unroll 8
-      for (uint32_t p = 0; p < n_pieces; ++p) {
-        const uint2 piece = *(const uint2*)(dense.words + (size_t)s_length[p] * kBinWords + i);
-        words.x |= piece.x;
-        words.y |= piece.y;
-      }
-      *(uint2*)(out + i) = words;
-    }
+  for (uint32_t k = 0; k < kEach; ++k) {
+    const uint32_t i = threadIdx.x * kEach + k;
+    id[k] = i < size ? sorted.ids[i] : 0xFFFFFFFFu;
+    if (i < size && id[k] != last) firsts |= 1u << k;
+    last = id[k];
   }
-  __syncthreads();  // the next stretch clears what this one has just read
+  const uint32_t through = wave_inclusive_scan((uint32_t)__popc(firsts));
+  uint32_t distinct;
+  const uint32_t rank0 = before_wave(through, &distinct) + through - (uint32_t)__popc(firsts);  // the sums are clear now
+#pragma unroll
+  for (uint32_t k = 0; k < kEach; ++k) {
+    const uint32_t i = threadIdx.x * kEach + k;
+    if (i >= size) continue;
+    const uint32_t rank = rank0 + (uint32_t)__popc(firsts & ((2u << k) - 1u)) - 1u;
+    atomicAdd(&sums[rank], merged.terms[edge_of(sorted.payload[i])]);
   }
+  __syncthreads();
+  uint32_t key[kEach];
+#pragma unroll
+  for (uint32_t k = 0; k < kEach; ++k) {
+    key[k] = 0;
+    if (firsts >> k & 1u)
+      key[k] = ladies_key_bits(sums[rank0 + (uint32_t)__popc(firsts & ((1u << k) - 1u))], ladies_pair_index(sample, n_vertices, id[k]),
+                               step, seed);
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t k = 0; k < kEach; ++k) {
+    if (!(firsts >> k & 1u)) continue;
+    const uint32_t rank = rank0 + (uint32_t)__popc(firsts & ((1u << k) - 1u));
+    s_words[rank] = key[k];
+    kept[rank] = id[k];
+    s_payload[0][rank] = (uint16_t)rank;
+  }
+  __syncthreads();
+  sorted = SortedIds{s_words, s_words + 2 * kRankedEntries, s_payload[0], s_payload[1]};
+  sorted = sort_ids<kRankedThreads, true>(sorted, s_count, s_wave_count, distinct, 32);
+  for (uint32_t i = threadIdx.x; i < distinct; i += kRankedThreads) sorted.other[i] = kept[sorted.payload[i]];
+  __syncthreads();
+  if (threadIdx.x == 0) *distinct_out = distinct;
+  draw((const CSR::Edge*)sorted.other, distinct);
 }
 
 // item_count[s] = work items of sample s (at least one, so that row offsets get written)
@@ -853,7 +772,7 @@ __global__ void fill_u32(uint32_t* dst, size_t n, uint32_t value) {
 // kSelectBits bits in an LDS
 // histogram and picks the bin that holds the wanted-th smallest key: threshold[s] = that bin,
 // kept[s] = keys up to and including it (a sample with fewer keys than wanted keeps them all),
-// present[s] = all its keys.  A sample's whole histogram stays in the workgroup: no atomic
+// distinct[its number] = all its keys.  A sample's whole histogram stays in the workgroup: no atomic
 // reaches memory, and no second pass over the keys refines the threshold (two levels of 8 bits,
 // counted by a workgroup per tile of 8192 keys, read every key twice).
 constexpr uint32_t kSelectBits = 14;
@@ -885,13 +804,18 @@ __device__ __forceinline__ void note_best_of_stretch(const uint32_t (&key)[4], u
   if (lane == 63) best_of[quad / 64u] = (uint16_t)best;
 }
 __global__ __launch_bounds__(kSelectThreads, 8) __attribute__((amdgpu_num_vgpr(56))) void select_threshold(
-    const uint32_t* __restrict__ keys, uint32_t keys_per_sample, uint32_t wanted,
-    uint32_t* __restrict__ threshold, uint32_t* __restrict__ kept, uint32_t* __restrict__ present,
-    uint16_t* __restrict__ stretch_best) {
+    const uint32_t* __restrict__ keys, uint32_t keys_per_sample, uint32_t wanted, const uint32_t* __restrict__ n_marked,
+    const uint32_t* __restrict__ marked, uint32_t* __restrict__ threshold, uint32_t* __restrict__ kept,
+    uint32_t* __restrict__ claimed, uint32_t* __restrict__ distinct, uint16_t* __restrict__ stretch_best) {
   __shared__ uint32_t s_hist[kSelectBins];
   __shared__ uint32_t s_wave_total[kSelectThreads / 64];
   const uint32_t s = blockIdx.x;
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  if (threadIdx.x == 0) claimed[s] = 0;  // for select_collect
+  if (s >= *n_marked) {
+    if (threadIdx.x == 0) kept[s] = 0;
+    return;
+  }
   for (uint32_t i = threadIdx.x; i < kSelectBins; i += kSelectThreads) s_hist[i] = 0;
   __syncthreads();
   const uint32_t* mine = keys + (size_t)s * keys_per_sample;
@@ -933,7 +857,7 @@ __global__ __launch_bounds__(kSelectThreads, 8) __attribute__((amdgpu_num_vgpr(5
     if (w < wave) before += t;
     total += t;
   }
-  if (threadIdx.x == 0) present[s] = total;
+  if (threadIdx.x == 0) distinct[marked[s]] = total;
   if (total < wanted) {  // everything stays
     if (threadIdx.x == 0) {
       threshold[s] = kSelectBins - 1u;
@@ -1024,17 +948,21 @@ struct LayerParams {
   const int32_t* nbr_cols;
   const float* nbr_weights;
   // kRankedByLadiesImportance: the kept ids of sample ls in descending key order are
-  // ranked_ids[ranked_start[ls] .. ranked_start[ls + 1])
+  // ranked_ids[ranked_start[at] .. ranked_start[at + 1]) for marked[at] == ls, at < n_marked
   const uint32_t* ranked_start;
   const int32_t* ranked_ids;
+  const uint32_t* marked;
+  uint32_t n_marked;
 };
 
 template <class SampleType, class App>
 __global__ __launch_bounds__(256) void layer_execute_kernel(LayerParams P) {
   const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= (uint64_t)P.chunk_samples * P.step_size) return;
-  const uint32_t ls = (uint32_t)(i / P.step_size);  // sample inside the chunk
-  const uint32_t nbr = (uint32_t)(i - (uint64_t)ls * P.step_size);
+  constexpr bool ranked_form = apps::neighborhood_form_of<App>::value == apps::kRankedByLadiesImportance;
+  if (i >= (uint64_t)(ranked_form ? P.n_marked : P.chunk_samples) * P.step_size) return;
+  const uint32_t at = (uint32_t)(i / P.step_size);
+  const uint32_t nbr = (uint32_t)(i - (uint64_t)at * P.step_size);
+  const uint32_t ls = ranked_form ? P.marked[at] : at;  // sample inside the chunk
   const uint32_t s = P.sample_begin + ls;
   CSRPartition csr = P.csr;
   const int32_t* transits = P.transits.base + (size_t)ls * P.transits.stride;
@@ -1056,20 +984,20 @@ __global__ __launch_bounds__(256) void layer_execute_kernel(LayerParams P) {
       neighbor = r == -1 ? P.invalid : r;
     }
   } else {
-    const uint32_t begin = P.ranked_start[ls];
+    const uint32_t begin = P.ranked_start[at];
     const CSR::Edge* ranked = P.ranked_ids + begin;
     const float* no_weights = nullptr;
     const VertexID r = App().template next<SampleType, const CSR::Edge*, const float*>(
         P.step, &csr, transits, sample_id, state, 0.0f, ranked, no_weights,
-        (EdgePos_t)(P.ranked_start[ls + 1] - begin), (VertexID_t)nbr, &rng);
+        (EdgePos_t)(P.ranked_start[at + 1] - begin), (VertexID_t)nbr, &rng);
     neighbor = r == -1 ? P.invalid : r;
   }
   P.final_samples[(size_t)s * P.final_size + P.out_base + nbr] = neighbor;
 }
 
-// kDistinctByDegreeSquared (nd_union_sums.hpp): next() for output nbr of sample ls of the chunk.
+// next() for output nbr of sample ls of the chunk, with what it takes for transitEdges.
 template <class SampleType, class App, class Distinct>
-__device__ __forceinline__ void draw_by_degree(const LayerParams& P, uint32_t ls, uint32_t nbr, Distinct& distinct,
+__device__ __forceinline__ void draw_from(const LayerParams& P, uint32_t ls, uint32_t nbr, Distinct& distinct,
                                                uint32_t n_distinct) {
   const uint32_t s = P.sample_begin + ls;
   CSRPartition csr = P.csr;
@@ -1092,7 +1020,21 @@ __global__ __launch_bounds__(kSortedThreads) void sorted_layer_kernel(LayerParam
   sorted_layer(P.csr, P.transits.base + (size_t)ls * P.transits.stride, P.transits.count, P.invalid, size, distinct + ls,
                [&](SortedByDegreeSquared& view, uint32_t n_distinct) {
                  for (uint32_t nbr = threadIdx.x; nbr < P.step_size; nbr += kSortedThreads)
-                   draw_by_degree<SampleType, App>(P, ls, nbr, view, n_distinct);
+                   draw_from<SampleType, App>(P, ls, nbr, view, n_distinct);
+               });
+}
+
+template <class SampleType, class App>
+__global__ __launch_bounds__(kRankedThreads) void ranked_layer_kernel(LayerParams P, MergedEdges merged,
+                                                                      const uint32_t* __restrict__ merged_sizes,
+                                                                      uint32_t* __restrict__ distinct) {
+  const uint32_t ls = blockIdx.x, size = merged_sizes[ls];
+  if (size > kRankedEntries) return;
+  ranked_layer(merged, (uint32_t)P.csr.n_vertices, P.transits.base + (size_t)ls * P.transits.stride, P.transits.count, P.invalid,
+               size, P.first_sample + P.sample_begin + ls, (uint32_t)P.step, P.seed, distinct + ls,
+               [&](const CSR::Edge* ranked, uint32_t n_distinct) {
+                 for (uint32_t nbr = threadIdx.x; nbr < P.step_size; nbr += kRankedThreads)
+                   draw_from<SampleType, App>(P, ls, nbr, ranked, n_distinct);
                });
 }
 
@@ -1109,7 +1051,7 @@ __global__ __launch_bounds__(256) void marked_layer_kernel(LayerParams P, Marked
     const uint32_t ls = marked.sample[at];
     MarkedByDegreeSquared mine{bitmap + (size_t)at * words_per_sample, part_before + (size_t)at * (parts + 1),
                                group_through + (size_t)at * parts * kGroupsPerPart, P.csr.row_ptr, parts};
-    draw_by_degree<SampleType, App>(P, ls, nbr, mine, distinct[ls]);
+    draw_from<SampleType, App>(P, ls, nbr, mine, distinct[ls]);
   }
 }
 
@@ -1143,7 +1085,6 @@ class LayerEngine : public EngineBase {
   int set_graph(const CSR* graph) override {
     free_run_buffers();  // sized against the previous graph: alloc() is due again
     graph_ = nullptr;
-    release(d_row_sums_);
     if (!dgraph_.upload(graph, false, app_uses_edge_lookup<App>::value, &last_error)) return -1;
     if (apps::neighborhood_form_of<App>::value == apps::kRankedByLadiesImportance) {
       // 1 / (weights of every vertex summed in edge order, sequential float adds)
@@ -1154,9 +1095,8 @@ class LayerEngine : public EngineBase {
         for (EdgePos_t x = graph->row_ptr[v]; x < graph->row_ptr[v + 1]; ++x) acc = acc + graph->weight[x];
         sums[v] = 1.0f / acc;  // the kernels multiply by the inverse
       }
-      ND_HIP_TRY(hipMalloc(&d_row_sums_, sizeof(float) * V));
-      ND_HIP_TRY(hipMemcpy(d_row_sums_, sums.data(), sizeof(float) * V, hipMemcpyHostToDevice));
-      const int rc = build_dense_pieces(graph, sums.data());
+      int rc = merge_parallel_edges(sums);
+      if (rc == 0) rc = build_dense_pieces(graph, sums.data());
       if (rc != 0) return rc;
     }
     if (apps::neighborhood_form_of<App>::value == apps::kDistinctByDegreeSquared) {
@@ -1223,8 +1163,7 @@ class LayerEngine : public EngineBase {
     // to whole stretches (LADIES form)
     uint64_t bytes_per_sample = (uint64_t)bitmap_words_ * sizeof(uint32_t);
     if (apps::neighborhood_form_of<App>::value == apps::kRankedByLadiesImportance) {
-      const uint32_t bin_words = kBinVerticesSums / 32u;
-      bytes_per_sample = (uint64_t)((bitmap_words_ + bin_words - 1) / bin_words) * kBinVerticesSums * sizeof(uint32_t);
+      bytes_per_sample = (uint64_t)((bitmap_words_ + kBinWords - 1) / kBinWords) * kBinVertices * sizeof(uint32_t);
     }
     const uint64_t fit = kBitmapBudgetBytes / bytes_per_sample;
     bitmap_chunk_samples_ = fit < 1 ? 1u : fit > (uint64_t)n_samples_ ? (uint32_t)n_samples_ : (uint32_t)fit;
@@ -1259,13 +1198,15 @@ class LayerEngine : public EngineBase {
     ND_HIP_TRY(hipMalloc(&d_item_start_, sizeof(uint32_t) * ((size_t)n_samples_ + 1)));
     ND_HIP_TRY(hipMalloc(&d_row_offsets_, sizeof(uint32_t) * (size_t)n_samples_ * widest));
     ND_HIP_TRY(hipMalloc(&d_small_scratch_, sizeof(uint32_t) * scan_scratch_elems((size_t)n_samples_ + 1)));
-    if (apps::neighborhood_form_of<App>::value == apps::kDistinctByDegreeSquared) {
+    if (apps::neighborhood_form_of<App>::value != apps::kConcatenated) {
       ND_HIP_TRY(hipMalloc(&d_layer_counts_, sizeof(uint32_t) * 2 * (size_t)n_samples_ * n_steps));
-      ND_HIP_TRY(hipHostMalloc((void**)&h_too_long_, sizeof(uint32_t), hipHostMallocDefault));
+      ND_HIP_TRY(hipHostMalloc((void**)&h_too_long_, 3 * sizeof(uint32_t), hipHostMallocDefault));
       *h_too_long_ = 0;
-      marked_.stride = widest;
       ND_HIP_TRY(hipMalloc(&marked_.count, sizeof(uint32_t)));
       ND_HIP_TRY(hipMalloc(&marked_.sample, sizeof(uint32_t) * (size_t)n_samples_));
+    }
+    if (apps::neighborhood_form_of<App>::value == apps::kDistinctByDegreeSquared) {
+      marked_.stride = widest;
       ND_HIP_TRY(hipMalloc(&marked_.transits, sizeof(int32_t) * (size_t)n_samples_ * widest));
       ND_HIP_TRY(hipMalloc(&marked_.transit_count, sizeof(uint2) * (size_t)n_samples_));
     }
@@ -1274,7 +1215,8 @@ class LayerEngine : public EngineBase {
       ND_HIP_TRY(hipMalloc(&d_ranked_start_, per_sample));
       ND_HIP_TRY(hipMalloc(&d_select_kept_, per_sample));
       ND_HIP_TRY(hipMalloc(&d_select_threshold_, per_sample));
-      ND_HIP_TRY(hipMalloc(&d_select_present_, per_sample));
+      ND_HIP_TRY(hipMalloc(&d_select_claimed_, per_sample));
+      ND_HIP_TRY(hipMalloc(&d_merged_sizes_, per_sample));
     }
     return 0;
   }
@@ -1309,7 +1251,7 @@ class LayerEngine : public EngineBase {
         all.count = (uint32_t)app.stepSize(step - 1);
       }
       constexpr int form = apps::neighborhood_form_of<App>::value;
-      if (form == apps::kDistinctByDegreeSquared && bitmap_chunk_entries_ == kBitmapChunkEntries) {
+      if (form != apps::kConcatenated && bitmap_chunk_entries_ == kBitmapChunkEntries) {
         // chunks of as many samples as there is memory for bitmaps of: nothing the host has to know first
         for (uint32_t s0 = 0; s0 < S; s0 += bitmap_chunk_samples_, chunks_run_++)
           if (run_chunk(step, all, s0, std::min(S, s0 + bitmap_chunk_samples_), 0) != 0) return -1;
@@ -1347,7 +1289,7 @@ class LayerEngine : public EngineBase {
     ND_HIP_TRY(hipStreamSynchronize(stream_));
     ND_HIP_TRY(hipEventElapsedTime(&times.end_to_end, ev_begin_, ev_end_));
     if (h_too_long_ && *h_too_long_) { last_error = kTooLong; return -2; }
-    counted_ = apps::neighborhood_form_of<App>::value != apps::kDistinctByDegreeSquared;
+    counted_ = apps::neighborhood_form_of<App>::value == apps::kConcatenated;
     return 0;
   }
 
@@ -1384,7 +1326,7 @@ class LayerEngine : public EngineBase {
 
   void free_device() override {
     free_run_buffers();
-    release(d_row_sums_);
+    release_merged();
     release_dense_pieces();
     union_.release();
     dgraph_.release();
@@ -1398,26 +1340,104 @@ class LayerEngine : public EngineBase {
     p = nullptr;
   }
 
-  // What the vertices with many edges into one stretch contribute to it, built once per graph
-  // (see DensePieces).  inverse_row_sums: the LADIES form's 1 / rowsum per vertex, else nullptr.
+  // The graph's edges with their terms, parallel ones as one (MergedEdges).
+  int merge_parallel_edges(const std::vector<float>& inverse_row_sums) {
+    release_merged();
+    const size_t E = (size_t)graph_edges(), V = inverse_row_sums.size();
+    float* d_inverse = nullptr;
+    uint32_t *d_at = nullptr, *d_zero = nullptr, *d_scratch = nullptr;
+    uint32_t pairs = 0, zero = 0;
+    hipError_t e = hipMalloc(&d_inverse, sizeof(float) * V);
+    if (e == hipSuccess) e = hipMemcpy(d_inverse, inverse_row_sums.data(), sizeof(float) * V, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMalloc(&d_at, sizeof(uint32_t) * (E + 1));
+    if (e == hipSuccess) e = hipMalloc(&d_scratch, sizeof(uint32_t) * scan_scratch_elems(E + 1));
+    if (e == hipSuccess) e = hipMalloc(&d_zero, sizeof(uint32_t));
+    if (e == hipSuccess) e = hipMemset(d_zero, 0, sizeof(uint32_t));
+    const dim3 over_edges((unsigned)((E + 256) / 256));
+    if (e == hipSuccess) {
+      first_of_parallel_edges<<<over_edges, dim3(256)>>>(dgraph_.view, d_at);
+      e = exclusive_scan_u32(d_at, d_at, E + 1, d_scratch, nullptr);
+    }
+    if (e == hipSuccess) e = hipMemcpy(&pairs, d_at + E, sizeof(pairs), hipMemcpyDeviceToHost);
+    if (e == hipSuccess) e = hipMalloc(&d_merged_rows_, sizeof(EdgePos_t) * (V + 1));
+    if (e == hipSuccess) e = hipMalloc(&d_merged_ids_, sizeof(VertexID) * std::max<size_t>(1, pairs));
+    if (e == hipSuccess) e = hipMalloc(&d_merged_terms_, sizeof(unsigned long long) * std::max<size_t>(1, pairs));
+    if (e == hipSuccess) {
+      merge_rows<<<dim3((unsigned)((V + 256) / 256)), dim3(256)>>>(dgraph_.view, d_at, d_merged_rows_);
+      merge_edges<<<over_edges, dim3(256)>>>(dgraph_.view, d_inverse, d_at, d_merged_ids_, d_merged_terms_, d_zero);
+      e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipMemcpy(&zero, d_zero, sizeof(zero), hipMemcpyDeviceToHost);
+    release(d_inverse); release(d_at); release(d_zero); release(d_scratch);
+    if (e != hipSuccess) {
+      release_merged();
+      last_error = std::string("merging parallel edges: ") + hipGetErrorString(e);
+      return -1;
+    }
+    merged_ = MergedEdges{d_merged_rows_, d_merged_ids_, d_merged_terms_, zero != 0, nullptr, nullptr};
+    return cut_merged_rows();
+  }
+  int cut_merged_rows() {
+    CSRPartition view = dgraph_.view;
+    view.row_ptr = d_merged_rows_;
+    view.edges = d_merged_ids_;
+    const uint32_t V = (uint32_t)view.n_vertices, stretches = (bitmap_words_for(V) + kBinWords - 1) / kBinWords;
+    uint32_t *d_rows = nullptr, rows = 0;
+    int32_t* d_vertex_of = nullptr;
+    const dim3 over_vertices((V + 255u) / 256u);
+    hipError_t e = hipMalloc(&d_rows, sizeof(uint32_t));
+    uint32_t from_degree = kCutDegree;
+    for (; e == hipSuccess; from_degree *= 2) {  // fewer rows where the cuts of all of them would take too much
+      e = hipMemset(d_rows, 0, sizeof(uint32_t));
+      if (e != hipSuccess) break;
+      number_hubs<<<over_vertices, dim3(256)>>>(view, from_degree, nullptr, nullptr, d_rows);
+      e = hipMemcpy(&rows, d_rows, sizeof(rows), hipMemcpyDeviceToHost);
+      if (e != hipSuccess || (size_t)rows * (stretches + 1) * sizeof(HubCut) <= kCutBudgetBytes) break;
+    }
+    if (e == hipSuccess && rows > 0) {
+      e = hipMalloc(&d_cut_row_of_, sizeof(int32_t) * V);
+      if (e == hipSuccess) e = hipMalloc(&d_vertex_of, sizeof(int32_t) * rows);
+      if (e == hipSuccess) e = hipMalloc(&d_cuts_, sizeof(HubCut) * (size_t)rows * (stretches + 1));
+      if (e == hipSuccess) e = hipMemset(d_rows, 0, sizeof(uint32_t));
+      if (e == hipSuccess) {
+        number_hubs<<<over_vertices, dim3(256)>>>(view, from_degree, d_cut_row_of_, d_vertex_of, d_rows);
+        cut_hubs<<<dim3((rows + 255) / 256, stretches + 1), dim3(256)>>>(view, d_vertex_of, rows, stretches, kBinVertices, d_cuts_);
+        e = hipGetLastError();
+      }
+      if (e == hipSuccess) e = hipDeviceSynchronize();
+    }
+    release(d_rows); release(d_vertex_of);
+    if (e != hipSuccess) {
+      release_merged();
+      last_error = std::string("cutting rows: ") + hipGetErrorString(e);
+      return -1;
+    }
+    merged_.cut_row_of = d_cut_row_of_;
+    merged_.cuts = d_cuts_;
+    return 0;
+  }
+  size_t graph_edges() const { return (size_t)dgraph_.view.n_edges; }
+  void release_merged() {
+    release(d_merged_rows_); release(d_merged_ids_); release(d_merged_terms_);
+    release(d_cut_row_of_); release(d_cuts_);
+    merged_ = MergedEdges{};
+  }
+
+  // What the vertices with many neighbours in one stretch contribute to it, built once per graph (see DensePieces).
   int build_dense_pieces(const CSR* graph, const float* inverse_row_sums) {
     release_dense_pieces();
-    constexpr bool ladies = apps::neighborhood_form_of<App>::value == apps::kRankedByLadiesImportance;
-    uint32_t threshold = ladies ? kDensePieceEntriesSums : kDensePieceEntries;
+    uint32_t threshold = kDensePieceEntries;
     if (const char* env = getenv("ND_DENSE_PIECE_ENTRIES")) {  // 0: no pieces; small: to exercise them on small graphs
       const long long v = atoll(env);
       if (v <= 0) return 0;
       threshold = (uint32_t)v;
     }
-    constexpr uint32_t stretch_words = ladies ? kBinVerticesSums / 32u : kBinWordsBits;
-    constexpr uint32_t stretch = stretch_words * 32u;
-    // a piece: a bit per vertex of the stretch, or a 64-bit importance sum (kAbsentSum: no edge)
-    constexpr size_t piece_words = ladies ? (size_t)stretch * 2u : (size_t)stretch_words;
     const uint32_t V = (uint32_t)graph->get_n_vertices();
-    const uint32_t stretches = (bitmap_words_for(V) + stretch_words - 1) / stretch_words;
-    const size_t most_pieces = kDensePieceBudgetBytes / (sizeof(uint32_t) * piece_words);
+    const uint32_t stretches = (bitmap_words_for(V) + kBinWords - 1) / kBinWords;
+    const size_t most_pieces = kDensePieceBudgetBytes / (sizeof(uint64_t) * kBinVertices);
     std::vector<int32_t> hub_row(V, -1);
-    std::vector<uint32_t> piece_of, words;
+    std::vector<uint32_t> piece_of;
+    std::vector<unsigned long long> sums;
     size_t n_hubs = 0, n_pieces = 0;
     for (uint32_t v = 0; v < V; ++v) {
       const int32_t* const row = graph->col.data() + graph->row_ptr[v];
@@ -1425,30 +1445,27 @@ class LayerEngine : public EngineBase {
       const int32_t* last = graph->col.data() + graph->row_ptr[v + 1];
       if ((size_t)(last - first) < threshold) continue;
       while (first < last) {  // one sub-range of the sorted adjacency per stretch
-        const uint32_t b = (uint32_t)*first / stretch;
-        const uint32_t limit = (b + 1) * stretch;
+        const uint32_t b = (uint32_t)*first / kBinVertices;
+        const uint32_t limit = (b + 1) * kBinVertices;
         const int32_t* stop = std::partition_point(first, last, [limit](int32_t c) { return (uint32_t)c < limit; });
-        if ((size_t)(stop - first) >= threshold && n_pieces < most_pieces) {
+        size_t neighbours = (size_t)(stop - first);
+        if (neighbours >= threshold) {  // without the repeats
+          neighbours = 1;
+          for (const int32_t* c = first + 1; c < stop; ++c) neighbours += c[0] != c[-1];
+        }
+        if (neighbours >= threshold && n_pieces < most_pieces) {
           if (hub_row[v] < 0) {
             hub_row[v] = (int32_t)n_hubs++;
             piece_of.resize(n_hubs * stretches, kNoPiece);
           }
           piece_of[(size_t)hub_row[v] * stretches + b] = (uint32_t)n_pieces;
-          words.resize((n_pieces + 1) * piece_words, ladies ? 0xFFFFFFFFu : 0u);
-          uint32_t* w = words.data() + n_pieces * piece_words;
+          sums.resize((n_pieces + 1) * kBinVertices, kAbsentSum);
+          unsigned long long* of = sums.data() + n_pieces * kBinVertices;
           for (const int32_t* c = first; c < stop; ++c) {
-            const uint32_t local = (uint32_t)*c - b * stretch;
-            if (ladies) {
-              // the term the marking kernel adds for this edge, in the same arithmetic
-              const float p = graph->weight[(size_t)graph->row_ptr[v] + (size_t)(c - row)] * inverse_row_sums[v];
-              unsigned long long sum;
-              memcpy(&sum, w + 2u * local, sizeof(sum));
-              if (sum == kAbsentSum) sum = 0;
-              sum += importance_term_fixed(p * p);
-              memcpy(w + 2u * local, &sum, sizeof(sum));
-            } else {
-              w[local >> 5] |= 1u << (local & 31u);
-            }
+            // the term of this edge, in the arithmetic of merge_edges
+            const float p = graph->weight[(size_t)graph->row_ptr[v] + (size_t)(c - row)] * inverse_row_sums[v];
+            unsigned long long& sum = of[(uint32_t)*c - b * kBinVertices];
+            sum = (sum == kAbsentSum ? 0 : sum) + importance_term_fixed(p * p);
           }
           ++n_pieces;
         }
@@ -1458,14 +1475,13 @@ class LayerEngine : public EngineBase {
     if (n_pieces == 0) return 0;
     ND_HIP_TRY(hipMalloc(&d_hub_row_, sizeof(int32_t) * V));
     ND_HIP_TRY(hipMalloc(&d_piece_of_, sizeof(uint32_t) * piece_of.size()));
-    ND_HIP_TRY(hipMalloc(&d_piece_words_, sizeof(uint32_t) * words.size()));
+    ND_HIP_TRY(hipMalloc(&d_piece_sums_, sizeof(uint64_t) * sums.size()));
     ND_HIP_TRY(hipMemcpy(d_hub_row_, hub_row.data(), sizeof(int32_t) * V, hipMemcpyHostToDevice));
     ND_HIP_TRY(hipMemcpy(d_piece_of_, piece_of.data(), sizeof(uint32_t) * piece_of.size(), hipMemcpyHostToDevice));
-    ND_HIP_TRY(hipMemcpy(d_piece_words_, words.data(), sizeof(uint32_t) * words.size(), hipMemcpyHostToDevice));
+    ND_HIP_TRY(hipMemcpy(d_piece_sums_, sums.data(), sizeof(uint64_t) * sums.size(), hipMemcpyHostToDevice));
     dense_.hub_row = d_hub_row_;
     dense_.piece_of = d_piece_of_;
-    dense_.words = d_piece_words_;
-    dense_.sums = (const unsigned long long*)d_piece_words_;
+    dense_.sums = d_piece_sums_;
     dense_pieces_ = n_pieces;
     return 0;
   }
@@ -1473,7 +1489,7 @@ class LayerEngine : public EngineBase {
   void release_dense_pieces() {
     release(d_hub_row_);
     release(d_piece_of_);
-    release(d_piece_words_);
+    release(d_piece_sums_);
     dense_ = DensePieces();
     dense_pieces_ = 0;
   }
@@ -1505,9 +1521,7 @@ class LayerEngine : public EngineBase {
     constexpr int form = apps::neighborhood_form_of<App>::value;
     TransitView tv = all;
     tv.base = all.base + (size_t)s0 * all.stride;
-    if (form == apps::kRankedByLadiesImportance) {
-      if (build_distinct_by_bitmap(step, s0, tv, n) != 0) return -1;
-    } else if (form == apps::kConcatenated) {
+    if (form == apps::kConcatenated) {
       // work items of the build: long neighbourhoods are spread over several workgroups
       uint64_t n_items = 0;
       for (uint32_t s = s0; s < s1; ++s) {
@@ -1547,9 +1561,9 @@ class LayerEngine : public EngineBase {
     P.nbr_weights = d_nbr_weights_;
     if constexpr (form == apps::kDistinctByDegreeSquared) {
       return run_by_degree(P, step);
+    } else if constexpr (form == apps::kRankedByLadiesImportance) {
+      return run_ranked(P, step);
     } else {
-      P.ranked_start = d_ranked_start_;
-      P.ranked_ids = d_ranked_ids_;
       const uint64_t outputs = (uint64_t)n * P.step_size;
       layer_execute_kernel<SampleType, App><<<dim3((unsigned)((outputs + 255) / 256)), dim3(256), 0, stream_>>>(P);
       ND_HIP_TRY(hipGetLastError());
@@ -1590,56 +1604,55 @@ class LayerEngine : public EngineBase {
     return 0;
   }
 
-  // What next() of the LADIES form is handed, for every sample of the chunk.
-  int build_distinct_by_bitmap(int step, uint32_t s0, const TransitView& tv, uint32_t n) {
-    constexpr uint32_t bin_words = kBinVerticesSums / 32u;
-    const uint32_t bins = (bitmap_words_ + bin_words - 1) / bin_words;
-    const uint32_t groups = (bins + kBinsPerGroupSums - 1) / kBinsPerGroupSums;
+  // LADIES form: small neighbourhoods are ranked by a workgroup each.  The others leave one sampling key per (sample,
+  // vertex); per sample, the vertices that can be among its first `wanted` in key order are picked by a radix select on the
+  // upper 14 bits of the key and ordered by descending key.  Their distinct pairs (2.4 M per batch at full size) are
+  // never listed.
+  int run_ranked(LayerParams P, int step) {
+    const uint32_t n = P.chunk_samples;
+    const uint32_t bins = (bitmap_words_ + kBinWords - 1) / kBinWords, groups = (bins + kBinsPerGroup - 1) / kBinsPerGroup;
     if ((uint64_t)n * groups >= (1ull << 31)) { last_error = "a chunk needs 2^31 or more workgroups"; return -1; }
-    return rank_by_keys(step, s0, tv, n, bins, groups);
-  }
-
-  // LADIES form: the marking leaves one sampling key per (sample, vertex); per sample, the
-  // vertices that can be among its first `wanted` in key order are picked by a radix select on
-  // the upper 14 bits of the key and ordered by descending key.  The distinct pairs of a
-  // sample (2.4 M per batch at full size) are never listed.
-  int rank_by_keys(int step, uint32_t s0, const TransitView& tv, uint32_t n, uint32_t bins, uint32_t groups) {
-    const uint32_t keys_per_sample = bins * kBinVerticesSums;
+    const uint32_t keys_per_sample = bins * kBinVertices;
     if (n > bitmap_samples_) {
       release(d_keys_dense_); release(d_stretch_best_);
       ND_HIP_TRY(hipMalloc(&d_keys_dense_, sizeof(uint32_t) * (size_t)n * keys_per_sample));
       ND_HIP_TRY(hipMalloc(&d_stretch_best_, sizeof(uint16_t) * (size_t)n * (keys_per_sample / kCollectStretch)));
       bitmap_samples_ = n;
     }
+    const size_t S = (size_t)n_samples_;
+    uint32_t* sizes = d_layer_counts_ + S * step + P.sample_begin;
+    uint32_t* distinct = sizes + S * App().steps();
+    ND_HIP_TRY(hipMemsetAsync(marked_.count, 0, sizeof(uint32_t), stream_));
+    sort_out_ranked<<<dim3((n + 15) / 16), dim3(kSortOutThreads), 0, stream_>>>(
+        P.csr, merged_, P.transits, n, invalid_, sizes, d_merged_sizes_, marked_.count, marked_.sample, h_too_long_);
+    tick();
+    ranked_layer_kernel<SampleType, App><<<dim3(n), dim3(kRankedThreads), 0, stream_>>>(P, merged_, d_merged_sizes_, distinct);
     KeysOnTheWayOut keys_out;
     keys_out.keys = d_keys_dense_;
     keys_out.seed = seed_;
-    keys_out.first_sample = s0;
+    keys_out.first_sample = P.first_sample + P.sample_begin;
     keys_out.step = (uint32_t)step;
     keys_out.n_vertices = (uint32_t)invalid_;
-    tick();
-    collective_mark_binned<true><<<dim3(n * groups), dim3(kBinThreads), 0, stream_>>>(
-        dgraph_.view, tv, invalid_, n, bins, nullptr, 0u, d_row_sums_, keys_per_sample, dense_, keys_out);
+    collective_mark_binned<<<dim3(n * groups), dim3(kBinThreads), 0, stream_>>>(
+        merged_, P.transits, invalid_, n, marked_.count, marked_.sample, bins, keys_per_sample, dense_, keys_out);
     tock();
     const uint32_t wanted = (uint32_t)App().stepSize(step);
-    select_threshold<<<dim3(n), dim3(kSelectThreads), 0, stream_>>>(d_keys_dense_, keys_per_sample, wanted,
-                                                                    d_select_threshold_, d_select_kept_,
-                                                                    d_select_present_, d_stretch_best_);
+    select_threshold<<<dim3(n), dim3(kSelectThreads), 0, stream_>>>(d_keys_dense_, keys_per_sample, wanted, marked_.count,
+                                                                    marked_.sample, d_select_threshold_, d_select_kept_,
+                                                                    d_select_claimed_, distinct, d_stretch_best_);
     // where every sample's ranked list starts: exclusive scan of the kept counts
     fill_u32<<<dim3(1), dim3(1), 0, stream_>>>(d_select_kept_ + n, 1, 0u);
     ND_HIP_TRY(exclusive_scan_u32(d_select_kept_, d_ranked_start_, (size_t)n + 1, d_small_scratch_, stream_));
-    uint32_t n_kept = 0;
-    ND_HIP_TRY(hipMemcpyAsync(&n_kept, d_small_scratch_ + scan_num_tiles((size_t)n + 1), sizeof(uint32_t),
+    ND_HIP_TRY(hipMemcpyAsync(h_too_long_ + 1, marked_.count, sizeof(uint32_t), hipMemcpyDeviceToHost, stream_));
+    ND_HIP_TRY(hipMemcpyAsync(h_too_long_ + 2, d_small_scratch_ + scan_num_tiles((size_t)n + 1), sizeof(uint32_t),
                               hipMemcpyDeviceToHost, stream_));
-    std::vector<uint32_t> present(n);
-    ND_HIP_TRY(hipMemcpyAsync(present.data(), d_select_present_, sizeof(uint32_t) * n, hipMemcpyDeviceToHost, stream_));
     ND_HIP_TRY(hipStreamSynchronize(stream_));
-    for (uint32_t c : present) distinct_total_ += c;
+    const uint32_t n_marked = h_too_long_[1], n_kept = h_too_long_[2];
+    if (n_marked == 0) return 0;
     if (ensure_distinct_capacity(n_kept) != 0) return -1;
-    ND_HIP_TRY(hipMemsetAsync(d_select_present_, 0, sizeof(uint32_t) * (size_t)n, stream_));  // now: room claimed
-    select_collect<<<dim3(n), dim3(kSelectThreads), 0, stream_>>>(d_keys_dense_, keys_per_sample, d_stretch_best_, d_select_threshold_,
-                                                     d_ranked_start_, d_select_present_, d_kept_key_, d_kept_sample_,
-                                                     d_kept_id_);
+    select_collect<<<dim3(n_marked), dim3(kSelectThreads), 0, stream_>>>(
+        d_keys_dense_, keys_per_sample, d_stretch_best_, d_select_threshold_, d_ranked_start_, d_select_claimed_, d_kept_key_,
+        d_kept_sample_, d_kept_id_);
     // order the kept vertices of every sample by descending key, equal keys by ascending
     // vertex id: stable sorts by vertex, then by key, then by sample
     if (n_kept > 0) {
@@ -1663,7 +1676,14 @@ class LayerEngine : public EngineBase {
       gather_u32<<<dim3(blocks), dim3(256), 0, stream_>>>((const uint32_t*)d_kept_id_, j4, n_kept,
                                                           (uint32_t*)d_ranked_ids_, nullptr);
     }
-    return hipGetLastError() == hipSuccess ? 0 : -1;
+    P.ranked_start = d_ranked_start_;
+    P.ranked_ids = d_ranked_ids_;
+    P.marked = marked_.sample;
+    P.n_marked = n_marked;
+    const uint64_t outputs = (uint64_t)n_marked * P.step_size;
+    layer_execute_kernel<SampleType, App><<<dim3((unsigned)((outputs + 255) / 256)), dim3(256), 0, stream_>>>(P);
+    ND_HIP_TRY(hipGetLastError());
+    return 0;
   }
 
   // Arrays with one entry per listed (sample, vertex) pair of a chunk: the distinct pairs
@@ -1729,7 +1749,7 @@ class LayerEngine : public EngineBase {
     h_too_long_ = nullptr;
     release(marked_.count); release(marked_.sample); release(marked_.transits); release(marked_.transit_count);
     release(d_ranked_start_); release(d_select_kept_);
-    release(d_select_threshold_); release(d_select_present_);
+    release(d_select_threshold_); release(d_select_claimed_); release(d_merged_sizes_);
     release_neighborhood_buffers();
     // whatever exists, also after an alloc that failed half way
     for (hipEvent_t* ev : {&ev_a_, &ev_b_, &ev_begin_, &ev_end_}) {
@@ -1744,10 +1764,9 @@ class LayerEngine : public EngineBase {
   const char* name_;
   const CSR* graph_ = nullptr;
   DeviceGraph dgraph_;
-  float* d_row_sums_ = nullptr;
-  int32_t* d_hub_row_ = nullptr;       // dense pieces of the graph (FastGCN form)
+  int32_t* d_hub_row_ = nullptr;       // dense pieces of the graph (LADIES form)
   uint32_t* d_piece_of_ = nullptr;
-  uint32_t* d_piece_words_ = nullptr;
+  unsigned long long* d_piece_sums_ = nullptr;
   DensePieces dense_;
   size_t dense_pieces_ = 0;
   std::vector<SampleType> samples_;
@@ -1784,7 +1803,14 @@ class LayerEngine : public EngineBase {
   uint32_t *d_item_count_ = nullptr, *d_item_start_ = nullptr;
   // LADIES form: the selection of the best keys per sample
   uint32_t *d_ranked_start_ = nullptr, *d_select_kept_ = nullptr, *d_select_threshold_ = nullptr;
-  uint32_t* d_select_present_ = nullptr;  // present[s]: distinct vertices of sample s's neighbourhood
+  uint32_t* d_select_claimed_ = nullptr;  // entries of a sample that have been given room
+  uint32_t* d_merged_sizes_ = nullptr;    // pairs of a sample's neighbourhood
+  EdgePos_t* d_merged_rows_ = nullptr;    // the graph without parallel edges
+  VertexID* d_merged_ids_ = nullptr;
+  unsigned long long* d_merged_terms_ = nullptr;
+  int32_t* d_cut_row_of_ = nullptr;
+  HubCut* d_cuts_ = nullptr;
+  MergedEdges merged_{};
   uint32_t *d_kept_key_ = nullptr, *d_kept_sample_ = nullptr;
   int32_t* d_kept_id_ = nullptr;
   int32_t* d_nbr_cols_ = nullptr;
@@ -1796,7 +1822,7 @@ class LayerEngine : public EngineBase {
   UnionTables union_;                  // of the graph
   MarkedSamples marked_{};
   uint32_t* d_layer_counts_ = nullptr;  // entries of every layer and sample's neighbourhood, then its distinct vertices
-  uint32_t* h_too_long_ = nullptr;      // a neighbourhood was too long
+  uint32_t* h_too_long_ = nullptr;      // whether a neighbourhood was too long, and two counts the LADIES form waits for
   int32_t* d_ranked_ids_ = nullptr;
 };
 

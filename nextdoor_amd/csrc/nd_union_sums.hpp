@@ -89,13 +89,13 @@ __global__ __launch_bounds__(256) void number_hubs(CSRPartition csr, uint32_t fr
 }
 
 __global__ __launch_bounds__(256) void cut_hubs(CSRPartition csr, const int32_t* vertex_of, uint32_t rows,
-                                                uint32_t parts, HubCut* cuts) {
+                                                uint32_t parts, uint32_t part_vertices, HubCut* cuts) {
   const uint32_t row = blockIdx.x * 256u + threadIdx.x, part = blockIdx.y;
   if (row >= rows) return;
   const int32_t v = vertex_of[row];
   const EdgePos_t begin = csr.row_ptr[v], end = csr.row_ptr[v + 1];
   cuts[(size_t)row * (parts + 1) + part] =
-      HubCut{part == parts ? end : first_edge_from(csr.edges, begin, end, part * kPartVertices), kNoPiece};
+      HubCut{part == parts ? end : first_edge_from(csr.edges, begin, end, part * part_vertices), kNoPiece};
 }
 
 // Numbers the pieces (those beyond `most` are left out), or, without place_of, only counts them.
@@ -240,7 +240,7 @@ class UnionTables {
     if (e == hipSuccess) e = hipMemset(counts, 0, 2 * sizeof(uint32_t));
     if (e == hipSuccess) {
       number_hubs<<<over_vertices, dim3(256)>>>(csr, hub_degree, d_row_of_, vertex_of, counts);
-      cut_hubs<<<dim3((rows + 255) / 256, parts + 1), dim3(256)>>>(csr, vertex_of, rows, parts, d_cuts_);
+      cut_hubs<<<dim3((rows + 255) / 256, parts + 1), dim3(256)>>>(csr, vertex_of, rows, parts, kPartVertices, d_cuts_);
       number_pieces<<<dim3((rows + 255) / 256, parts), dim3(256)>>>(d_cuts_, rows, parts, piece_entries, 0u, nullptr, counts + 1);
       uint32_t found = 0;
       e = hipMemcpy(&found, counts + 1, sizeof(found), hipMemcpyDeviceToHost);
@@ -344,7 +344,7 @@ __global__ __launch_bounds__(kSortOutThreads) void sort_out_samples(CSRPartition
 
 // ---- small neighbourhoods: sorted in LDS ---------------------------------------------------
 
-constexpr uint32_t kSortedThreads = 512;
+constexpr uint32_t kSortedThreads = 512, kSortedWaves = kSortedThreads / 64;
 constexpr uint32_t kSortedChunk = 8;  // ids a running sum is kept for
 
 // What next() receives as transitEdges there.
@@ -379,23 +379,30 @@ struct SortedByDegreeSquared {
   }
 };
 
-// Ids [0, n) of `ids` in ascending order, by passes over 7 bits, least significant first; the result is in the returned
-// one of the two buffers.  A wavefront takes a stretch of the ids, 64 at a time: lanes with equal digits find each other by
+// The n ids at `at.ids` in ascending order, equal ones as they were, by passes over 7 bits, least significant first; the
+// result is where the returned `ids` points.  A wavefront takes a stretch of the ids, 64 at a time: lanes with equal digits find each other by
 // ballots, and what came before them is in the wavefront's counters.  (A bitonic sort, 78 stages of LDS reads and writes for
 // 4096 ids, took 0.36 ms for the 4096 samples of R-MAT 20's first layer.)
-constexpr uint32_t kSortedWaves = kSortedThreads / 64, kSortedDigitBits = 7, kSortedDigits = 1u << kSortedDigitBits;
-__device__ __forceinline__ uint32_t* sort_ids(uint32_t* ids, uint32_t* other, uint32_t (*s_count)[kSortedDigits],
-                                              uint32_t* s_wave_count, uint32_t n, uint32_t bits) {
+// With a payload, 16 bits go where the ids go.
+constexpr uint32_t kSortedDigitBits = 7, kSortedDigits = 1u << kSortedDigitBits;
+struct SortedIds {
+  uint32_t *ids, *other;
+  uint16_t *payload, *other_payload;
+};
+template <uint32_t kThreads, bool kPayload>
+__device__ __forceinline__ SortedIds sort_ids(SortedIds at, uint32_t (*s_count)[kSortedDigits], uint32_t* s_wave_count,
+                                              uint32_t n, uint32_t bits) {
+  constexpr uint32_t kWaves = kThreads / 64;
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-  const uint32_t stretch = ((n + kSortedWaves - 1) / kSortedWaves + 63u) & ~63u;
+  const uint32_t stretch = ((n + kWaves - 1) / kWaves + 63u) & ~63u;
   const uint32_t begin = wave * stretch, end = begin + stretch < n ? begin + stretch : n;
   for (uint32_t shift = 0; shift < bits; shift += kSortedDigitBits) {
-    for (uint32_t i = threadIdx.x; i < kSortedWaves * kSortedDigits; i += kSortedThreads) (&s_count[0][0])[i] = 0;
+    for (uint32_t i = threadIdx.x; i < kWaves * kSortedDigits; i += kThreads) (&s_count[0][0])[i] = 0;
     __syncthreads();
-    for (uint32_t i = begin + lane; i < end; i += 64u) atomicAdd(&s_count[wave][ids[i] >> shift & (kSortedDigits - 1u)], 1u);
+    for (uint32_t i = begin + lane; i < end; i += 64u) atomicAdd(&s_count[wave][at.ids[i] >> shift & (kSortedDigits - 1u)], 1u);
     __syncthreads();
     // starts: by digit, then by wavefront; lane t has two counters that follow each other in that order
-    const uint32_t digit = threadIdx.x / (kSortedWaves / 2u), of = threadIdx.x % (kSortedWaves / 2u) * 2u;
+    const uint32_t digit = threadIdx.x / (kWaves / 2u), of = threadIdx.x % (kWaves / 2u) * 2u;
     const uint32_t a = s_count[of][digit], b = s_count[of + 1u][digit];
     const uint32_t through = wave_inclusive_scan(a + b);
     if (lane == 63) s_wave_count[wave] = through;
@@ -407,7 +414,7 @@ __device__ __forceinline__ uint32_t* sort_ids(uint32_t* ids, uint32_t* other, ui
     __syncthreads();
     for (uint32_t i0 = begin; i0 < end; i0 += 64u) {
       const bool here = i0 + lane < end;
-      const uint32_t id = here ? ids[i0 + lane] : 0u, d = id >> shift & (kSortedDigits - 1u);
+      const uint32_t id = here ? at.ids[i0 + lane] : 0u, d = id >> shift & (kSortedDigits - 1u);
       uint64_t same = __ballot(here);
 #pragma unroll
       for (uint32_t bit = 0; bit < kSortedDigitBits; ++bit) {
@@ -417,18 +424,17 @@ __device__ __forceinline__ uint32_t* sort_ids(uint32_t* ids, uint32_t* other, ui
       }
       if (here) {
         const uint32_t rank = (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
-        const uint32_t at = s_count[wave][d] + rank;
-        other[at] = id;
-        if (rank == 0) s_count[wave][d] = at + (uint32_t)__popcll(same);
+        const uint32_t to = s_count[wave][d] + rank;
+        at.other[to] = id;
+        if (kPayload) at.other_payload[to] = at.payload[i0 + lane];
+        if (rank == 0) s_count[wave][d] = to + (uint32_t)__popcll(same);
       }
       __builtin_amdgcn_wave_barrier();
     }
     __syncthreads();
-    uint32_t* t = ids;
-    ids = other;
-    other = t;
+    at = SortedIds{at.other, at.ids, at.other_payload, at.payload};
   }
-  return ids;
+  return at;
 }
 
 // A workgroup per sample: fetches the entries, sorts them, adds degree^2 up over the distinct ones and draws.
@@ -477,7 +483,8 @@ __device__ __forceinline__ void sorted_layer(const CSRPartition& csr, const int3
     s_buffers[0][e] = (uint32_t)csr.edges[s_edge[lo] + (EdgePos_t)(e - s_start[lo])];
   }
   __syncthreads();
-  uint32_t* s_ids = sort_ids(s_buffers[0], s_buffers[1], s_count, s_wave_count, size, 32u - (uint32_t)__clz(csr.n_vertices));
+  uint32_t* s_ids = sort_ids<kSortedThreads, false>(SortedIds{s_buffers[0], s_buffers[1], nullptr, nullptr}, s_count, s_wave_count,
+                                                    size, 32u - (uint32_t)__clz(csr.n_vertices)).ids;
   const uint32_t chunks = size ? (size + kSortedChunk - 1) / kSortedChunk : 1u;
   if (size + threadIdx.x < chunks * kSortedChunk) s_ids[size + threadIdx.x] = 0xFFFFFFFFu;
   __syncthreads();
