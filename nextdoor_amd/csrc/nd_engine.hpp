@@ -1245,6 +1245,9 @@ constexpr int kClassifyItemsLarge = 16;
 // against 0.24 on 5.2e7 pairs - the launch waits for its slowest lanes, not for the atomics)
 constexpr int kClassifyThreadsLarge = 256;
 constexpr uint32_t kClassifyLargeFrom = 16u << 20;  // pairs
+// Apps that are not walks classify once a pass, and most of their wavefronts find a run: one atomic each on the
+// counter of work items, 10 ns after the other (1.5 M pairs of 60 K k-hop samples: 0.10 ms with one pair a lane).
+constexpr uint32_t kClassifyManyFrom = 64u << 10;
 
 // A run of `count` pairs on `transit` that starts at pair `start`: should the workgroup kernel
 // take it?  Gives the run and the number of work items it needs.  refused_out (nullable): set to
@@ -2484,7 +2487,7 @@ class Engine : public EngineBase {
             RunsMeta* meta = d_meta_ + (balanced_steps_ & 1);
             RunsMeta* meta_next = d_meta_ + ((balanced_steps_ + 1) & 1);
             balanced_steps_++;
-            if (n_pairs >= kClassifyLargeFrom) {
+            if (n_pairs >= (walk_mode_ ? kClassifyLargeFrom : kClassifyManyFrom)) {
               const unsigned per_block = kClassifyThreadsLarge * kClassifyItemsLarge;
               const unsigned tail_blocks = (n_pairs + per_block - 1) / per_block;
               classify_run_tails<kClassifyItemsLarge, kClassifyThreadsLarge>
