@@ -2107,7 +2107,7 @@ class Engine : public EngineBase {
   // the only host wait is at the end.
   int sample(int mode) override {
     if (!allocated_) { last_error = "sample before alloc"; return -1; }
-    if (ahead_) (void)finish_rows_ahead();  // nobody asked for them
+    (void)finish_rows_ahead();  // nobody asked for them
     times = PhaseTimes();
     if (!std::is_empty<SampleType>::value) {
       ND_HIP_TRY(hipMemcpyAsync(d_samples_, d_samples_init_, sizeof(SampleType) * (size_t)n_samples_,
@@ -2623,6 +2623,7 @@ class Engine : public EngineBase {
 
   int fetch_final_samples_into(VertexID_t* dst) {
     if (!allocated_) { last_error = "no device data"; return -1; }
+    settle_rows_ahead();
     return fetch_to_host(dst, d_final_, sizeof(VertexID_t) * (size_t)n_samples_ * (size_t)final_sample_size(),
                          (uint32_t)max_bits_, invalid_, stream_);
   }
@@ -2631,13 +2632,13 @@ class Engine : public EngineBase {
   // cross the bus while later walks are still under way; sample() returns when the sampling is done, as
   // always, and the rest of the rows arrives until finish_rows_ahead().  Any pass may leave it be.
   VertexID_t* rows_ahead = nullptr;
-  bool rows_are_ahead() const { return ahead_; }
-  int finish_rows_ahead() {
+  // Waits for rows on their way; whether they are at rows_ahead.  Where not (no pass sent them, the transfer failed) they
+  // are to be fetched like any others.
+  bool finish_rows_ahead() {
+    settle_rows_ahead();
+    const bool there = ahead_;
     ahead_ = false;
-    const hipError_t e = result_stream.finish();
-    if (e == hipSuccess) return 0;
-    last_error = std::string("results to the host: ") + hipGetErrorString(e);
-    return -1;
+    return there;
   }
 
   bool is_walk() const { return walk_mode_; }
@@ -2645,6 +2646,7 @@ class Engine : public EngineBase {
   int fetch_sample_states(void* dst, size_t bytes) override {
     if (!allocated_ || std::is_empty<SampleType>::value) { last_error = "no sample state"; return -1; }
     if (bytes != sample_state_bytes()) { last_error = "sample state size mismatch"; return -1; }
+    settle_rows_ahead();
     return states_to_host(dst, d_samples_, bytes, stream_);
   }
 
@@ -2652,7 +2654,7 @@ class Engine : public EngineBase {
   // hop segment of every sample becomes its ascending unique valid ids, INVALID-padded.
   int distinct() override {
     if (!allocated_) { last_error = "distinct before alloc"; return -1; }
-    if (ahead_) (void)finish_rows_ahead();  // they are about to change
+    (void)finish_rows_ahead();  // they are about to change
     App app;
     if (app.outputFormat() != SampledVertices) { last_error = "distinct needs SampledVertices output"; return -2; }
     const int n_steps = app.steps();
@@ -2697,6 +2699,11 @@ class Engine : public EngineBase {
   // Walks write their results in cells of two steps (StepParams::pair_cells) where a step's
   // transit is the previous step's result and the rows are regrouped by assemble_walk_rows.
   bool paired_results() const { return paired_results_; }
+  // The result stream carries one transfer at a time, and whoever begins another waits for the one before: rows on their way
+  // are waited for here first, where it is known whose they are and what has become of them.
+  void settle_rows_ahead() {
+    if (ahead_ && result_stream.finish() != hipSuccess) ahead_ = false;
+  }
 
   void launch_workgroup(const StepParams& P, unsigned grid, const RunsMeta* meta) {
     if (P.step_size == 1)
@@ -2847,7 +2854,7 @@ class Engine : public EngineBase {
   }
 
   void free_run_buffers() {
-    if (ahead_) (void)finish_rows_ahead();
+    (void)finish_rows_ahead();
     rows_ahead = nullptr;
     for (hipEvent_t ev : range_ends_) (void)hipEventDestroy(ev);
     range_ends_.clear();

@@ -830,6 +830,7 @@ class ResultStream {
     }
     if (error != hipSuccess) {
       t.error = error;
+      (void)hipGetLastError();  // reported by finish(), not to this thread's next launch
       t.announce(0, true);
     }
   }

@@ -131,16 +131,12 @@ class ShardedEngine : public EngineBase {
   int fetch_final_samples() override {
     size_t at = 0;
     rows_fetched_ = true;
-    if (parts_.size() == 1 && parts_[0]->rows_are_ahead()) {
-      if (parts_[0]->finish_rows_ahead() != 0) return fail(0);
-      hFinalSamples.swap(rows_ahead_);
-      rows_ahead_.clear();
-      return 0;
-    }
-    if (!rows_ahead_.empty()) {  // taken for a pass that did without
+    const bool there = parts_.size() == 1 && parts_[0]->finish_rows_ahead();
+    if (!rows_ahead_.empty()) {  // of a pass that sent its rows, or that did without
       hFinalSamples.swap(rows_ahead_);
       rows_ahead_.clear();
     }
+    if (there) return 0;
     if (num_samples() > 0) hFinalSamples.resize((size_t)num_samples() * (size_t)final_sample_size());
     for (size_t i = 0; i < parts_.size(); ++i) {
       if (parts_[i]->fetch_final_samples_into(hFinalSamples.data() + at) != 0) return fail((int)i);

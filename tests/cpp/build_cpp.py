@@ -18,6 +18,8 @@ TEMPLATE_PROBE_SRC = os.path.join(HERE, "template_api_probe.hip")
 TEMPLATE_PROBE = os.path.join(HERE, "template_api_probe")
 RESULT_PROBE_SRC = os.path.join(HERE, "result_stream_probe.hip")
 RESULT_PROBE = os.path.join(HERE, "result_stream_probe")
+ROWS_AHEAD_PROBE_SRC = os.path.join(HERE, "rows_ahead_probe.hip")
+ROWS_AHEAD_PROBE = os.path.join(HERE, "rows_ahead_probe")
 USER_APPS_SRC = os.path.join(HERE, "user_apps.hip")
 USER_APPS_LIB = os.path.join(HERE, "libuser_apps.so")
 
@@ -62,13 +64,21 @@ def build_result_probe():
     return RESULT_PROBE
 
 
+def build_rows_ahead_probe():
+    from nextdoor_amd.build import CSRC
+    _run(_hipcc_flags() + ["-I", INCLUDE, ROWS_AHEAD_PROBE_SRC, os.path.join(CSRC, "nd_graph.cpp"), "-o", ROWS_AHEAD_PROBE,
+                           "-lpthread"])
+    return ROWS_AHEAD_PROBE
+
+
 def build_user_apps():
     _run(_hipcc_flags() + ["-shared", USER_APPS_SRC, "-o", USER_APPS_LIB] + _link_flags())
     return USER_APPS_LIB
 
 
 def build_all():
-    return [build_host_probe(), build_template_probe(), build_result_probe(), build_user_apps()]
+    return [build_host_probe(), build_template_probe(), build_result_probe(), build_rows_ahead_probe(),
+            build_user_apps()]
 
 
 if __name__ == "__main__":

@@ -8,7 +8,7 @@ import pytest
 
 import nextdoor_amd as nd
 from tests import graphs
-from tests.cpp.build_cpp import RESULT_PROBE
+from tests.cpp.build_cpp import RESULT_PROBE, ROWS_AHEAD_PROBE
 
 pytestmark = pytest.mark.gpu
 
@@ -17,6 +17,14 @@ def test_packed_transfer_gives_back_the_words_on_the_device():
     assert os.path.exists(RESULT_PROBE), "tests/cpp/result_stream_probe is built by __graft_entry__.build()"
     out = subprocess.run([RESULT_PROBE], capture_output=True, text=True, timeout=100)
     assert out.returncode == 0 and out.stdout.endswith("all equal\n"), out.stdout[-300:] + out.stderr[-300:]
+
+
+def test_what_is_asked_for_before_rows_that_are_on_their_way():
+    """States fetched while rows are on their way do not take the news of a failed transfer with them: the rows are
+    then fetched anew, not given out unfilled."""
+    assert os.path.exists(ROWS_AHEAD_PROBE), "tests/cpp/rows_ahead_probe is built by __graft_entry__.build()"
+    out = subprocess.run([ROWS_AHEAD_PROBE], capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0 and out.stdout.endswith("all as they should be\n"), out.stdout[-300:] + out.stderr[-300:]
 
 
 # 1.1 MB: copied as it is; 8.8 MB: packed (12 bits, the ids and INVALID); 36 MB of 16 and 17 bits
