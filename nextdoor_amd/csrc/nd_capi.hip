@@ -609,7 +609,7 @@ int nd_sampler_check_results(nd_sampler* s, int* ok) {
 void nd_sampler_free_device(nd_sampler* s) {
   if (!s) return;
   s->engine->free_device();
-  s->engine->result_stream.release();
+  s->engine->result_stream->release();
 }
 
 void nd_sampler_destroy(nd_sampler* s) { delete s; }

@@ -116,12 +116,13 @@ class EngineBase {
 
   // Host memory of the results, and the way they take to it (nd_host_results.hpp)
   const std::shared_ptr<HostPool> host_pool = std::make_shared<HostPool>();
-  ResultStream result_stream;
+  // (engines that are parts of another one use that one's, so that there is one ring a sampler, and one to give back)
+  std::shared_ptr<ResultStream> result_stream = std::make_shared<ResultStream>();
   // Device memory to the host, complete on return.  bits, fill: what is known of its words (ResultStream::fetch).
   int fetch_to_host(void* dst, const void* src, size_t bytes, uint32_t bits, int32_t fill, hipStream_t stream) {
     hipError_t e;
     if (bytes > kDirectResultBytes && bytes % sizeof(int32_t) == 0) {
-      e = result_stream.fetch((const int32_t*)src, bytes / sizeof(int32_t), bits, fill, (int32_t*)dst, stream);
+      e = result_stream->fetch((const int32_t*)src, bytes / sizeof(int32_t), bits, fill, (int32_t*)dst, stream);
     } else {
       e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream);
       if (e == hipSuccess) e = hipStreamSynchronize(stream);
@@ -135,7 +136,7 @@ class EngineBase {
   // fit the ids' bits.  Where they do not once, no later transfer tries (100 K samples of MultiRW, 40 MB: 0.88 -> 0.52 ms).
   int states_to_host(void* dst, const void* src, size_t bytes, hipStream_t stream) {
     const int rc = fetch_to_host(dst, src, bytes, states_fit_ids_ ? (uint32_t)max_bits() : 32u, -1, stream);
-    if (result_stream.misfit()) states_fit_ids_ = false;
+    if (result_stream->misfit()) states_fit_ids_ = false;
     return rc;
   }
 
@@ -2198,7 +2199,7 @@ class Engine : public EngineBase {
       ready.push_back({end * F, range_ends_[r]});
       first = end;
     }
-    const hipError_t e = result_stream.begin(d_final_, (size_t)n_samples_ * F, (uint32_t)max_bits_, invalid_, rows_ahead,
+    const hipError_t e = result_stream->begin(d_final_, (size_t)n_samples_ * F, (uint32_t)max_bits_, invalid_, rows_ahead,
                                              stream_, std::move(ready));
     if (e != hipSuccess) { last_error = std::string("results to the host: ") + hipGetErrorString(e); return -1; }
     ahead_ = true;
@@ -2702,7 +2703,7 @@ class Engine : public EngineBase {
   // The result stream carries one transfer at a time, and whoever begins another waits for the one before: rows on their way
   // are waited for here first, where it is known whose they are and what has become of them.
   void settle_rows_ahead() {
-    if (ahead_ && result_stream.finish() != hipSuccess) ahead_ = false;
+    if (ahead_ && result_stream->finish() != hipSuccess) ahead_ = false;
   }
 
   void launch_workgroup(const StepParams& P, unsigned grid, const RunsMeta* meta) {

@@ -613,6 +613,8 @@ class ResultStream {
 
   // whether a word has ever not fitted
   bool misfit() const { return misfit_; }
+  // page-locked memory it holds until release()
+  size_t page_locked_bytes() const { return ring_bytes_; }
 
   void release() {
     (void)finish();

@@ -25,7 +25,7 @@ class ShardedEngine : public EngineBase {
   typedef Engine<SampleType, App> Part;
 
  public:
-  explicit ShardedEngine(const char* name) : name_(name) { parts_.emplace_back(new Part(name)); }
+  explicit ShardedEngine(const char* name) : name_(name) { add_part(); }
 
   const char* app_name() const override { return name_; }
   int64_t num_samples() const override {
@@ -67,7 +67,7 @@ class ShardedEngine : public EngineBase {
       if (atoi(env) == 2 && walk && n >= 2) n_parts = 2;
     }
     while ((int)parts_.size() < n_parts) {
-      parts_.emplace_back(new Part(name_));
+      add_part();
       parts_.back()->share_graph(*parts_[0]);
     }
     initialContents.clear();
@@ -181,6 +181,10 @@ class ShardedEngine : public EngineBase {
   }
 
  private:
+  void add_part() {
+    parts_.emplace_back(new Part(name_));
+    parts_.back()->result_stream = result_stream;
+  }
   int fail(int part, int rc = -1) {
     last_error = parts_[(size_t)part]->last_error;
     return rc;

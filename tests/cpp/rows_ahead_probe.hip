@@ -58,11 +58,11 @@ int main() {
     std::fill(got.begin(), got.end(), -7);
     CHECK(engine.sample(nd::kTransitParallelLoadBalanced) == 0);
     // in the place of the rows' transfer one that waits for no event at all, which the runtime refuses
-    CHECK(engine.result_stream.finish() == hipSuccess);
+    CHECK(engine.result_stream->finish() == hipSuccess);
     std::fill(got.begin(), got.end(), -7);
     int32_t* words = nullptr;
     CHECK(hipMalloc(&words, n * sizeof(int32_t)) == hipSuccess);
-    CHECK(engine.result_stream.begin(words, n, 32, 0, got.data(), nullptr, {{n, nullptr}}) == hipSuccess);
+    CHECK(engine.result_stream->begin(words, n, 32, 0, got.data(), nullptr, {{n, nullptr}}) == hipSuccess);
     if (with_states) {
       std::fill(states.begin(), states.end(), 0);
       CHECK(engine.fetch_sample_states(states.data(), states.size()) == 0 && states == want_states);
@@ -78,6 +78,22 @@ int main() {
   STEP("freed with rows on their way");
   CHECK(engine.sample(nd::kTransitParallelLoadBalanced) == 0);
   engine.free_device();
+  STEP("what a sampler holds, given back");
+  for (const char* ranges : {"1", "2"}) {
+    setenv("ND_SAMPLE_RANGES", ranges, 1);
+    nd::ShardedEngine<Node2VecSample, WeightedNode2VecAppT<8>> sampler("walks");
+    nd::EngineBase& base = sampler;
+    CHECK(base.set_graph(&graph) == 0 && base.alloc(42) == 0);
+    for (int pass = 0; pass < 2; ++pass) {
+      CHECK(base.sample(nd::kTransitParallelLoadBalanced) == 0 && base.fetch_final_samples() == 0);
+      CHECK(memcmp(base.hFinalSamples.data(), want.data(), n * sizeof(VertexID_t)) == 0);
+      delete base.hFinalSamples.detach();  // so that the next pass sends its rows ahead
+    }
+    CHECK(base.result_stream->page_locked_bytes() > 0);
+    base.free_device();  // what nd_sampler_free_device does
+    base.result_stream->release();
+    CHECK(base.result_stream->page_locked_bytes() == 0);
+  }
   printf("all as they should be\n");
   return 0;
 }
