@@ -520,14 +520,36 @@ inline void unpack_chunk(const UnpackPlan& plan, const PackHeader& header, const
   if (at == part) memcpy(dst, part, count * sizeof(int32_t));
 }
 
-// The stream results cross the bus on while something else is computed: one per device and process, on a hardware
-// queue of its own, which a stream with a mask of compute units (here: all) gets.  (Ordinary streams share four;
-// where the computation's lands on the same one, nothing overlaps.)
-inline hipStream_t transfer_stream() {
+// Makes a device this thread's current one for as long as it lives.
+class OnDevice {
+ public:
+  explicit OnDevice(int device) {
+    error = hipGetDevice(&before_);
+    if (error != hipSuccess || before_ == device) return;
+    error = hipSetDevice(device);
+    moved_ = error == hipSuccess;
+  }
+  OnDevice(const OnDevice&) = delete;
+  OnDevice& operator=(const OnDevice&) = delete;
+  ~OnDevice() { if (moved_) (void)hipSetDevice(before_); }
+  hipError_t error;
+
+ private:
+  int before_ = 0;
+  bool moved_ = false;
+};
+
+// The device of a stream; of the default stream: the current one.
+inline hipError_t device_of(hipStream_t stream, int* device) {
+  return stream ? hipStreamGetDevice(stream, device) : hipGetDevice(device);
+}
+
+// The stream results cross the bus on while something else is computed: one per device (the current one) and process, on
+// a hardware queue of its own, which a stream with a mask of compute units (here: all) gets.  (Ordinary streams share
+// four; where the computation's lands on the same one, nothing overlaps.)
+inline hipStream_t transfer_stream(int device) {
   static std::mutex mutex;
   static std::vector<hipStream_t>* streams = new std::vector<hipStream_t>;
-  int device = 0;
-  if (hipGetDevice(&device) != hipSuccess) return nullptr;
   std::lock_guard<std::mutex> lock(mutex);
   if (streams->size() <= (size_t)device) streams->resize((size_t)device + 1, nullptr);
   hipStream_t& stream = (*streams)[(size_t)device];
@@ -546,7 +568,8 @@ inline hipStream_t transfer_stream() {
 
 // ---- the stream ----------------------------------------------------------------------------
 
-// Brings words of device memory to the host, packed on the way.  One caller at a time.
+// Brings words of device memory to the host, packed on the way.  One caller at a time.  Everything happens on the device of the
+// stream that is given, whatever the calling thread's current device is, and leaves that as it was.
 class ResultStream {
  public:
   ResultStream() = default;
@@ -577,12 +600,16 @@ class ResultStream {
     if (e != hipSuccess || n == 0) return e;
     if (!transfer_) transfer_.reset(new Transfer);
     Transfer& t = *transfer_;
-    e = hipGetDevice(&t.device);
+    e = device_of(stream, &t.device);
     if (e != hipSuccess) return e;
+    const OnDevice on(t.device);
+    if (on.error != hipSuccess) return on.error;
     t.set(src, n, bits > kPackMostBits ? 32 : bits, fill, dst, std::move(ready));
+    if (t.device != device_) release_device();  // events of one device are not recorded on another's streams
+    device_ = t.device;
     e = prepare(t.slot_bytes);
     if (e != hipSuccess) return e;
-    t.streams[0] = t.streams[1] = transfer_stream();
+    t.streams[0] = t.streams[1] = transfer_stream(t.device);
     if (t.ready.empty()) {
       // pieces alternate between two streams, so that the bus is not idle between two launches
       t.streams[0] = stream;
@@ -603,11 +630,13 @@ class ResultStream {
     HostWorkers::get().join(job_);
     under_way_ = false;
     if (t.error != hipSuccess) {
+      const OnDevice on(t.device);
       for (hipStream_t s : t.streams) (void)hipStreamSynchronize(s);  // nothing writes to the ring after this
       return t.error;
     }
     if (!t.overflow.load()) return hipSuccess;
     misfit_ = true;
+    const OnDevice on(t.device);  // the stream may be the default one
     return fetch(t.src, t.n, 32, t.fill, t.dst, t.streams[0]);
   }
 
@@ -618,6 +647,11 @@ class ResultStream {
 
   void release() {
     (void)finish();
+    release_device();
+  }
+
+ private:
+  void release_device() {
     for (hipEvent_t& ev : packed_)
       if (ev) (void)hipEventDestroy(ev), ev = nullptr;
     if (begun_) (void)hipEventDestroy(begun_);
@@ -627,7 +661,6 @@ class ResultStream {
     ring_bytes_ = 0;
   }
 
- private:
   static constexpr size_t kSlots = 8;
   // Chunks of a piece: at most 8 MB of results (0.1 ms on the bus, long against a launch and an event; with pieces of
   // 16 MB the ring no longer stays in the last-level cache between the bus and the threads: 1.68 GB in 16 instead of 14
@@ -809,7 +842,8 @@ class ResultStream {
   // Launches the packing of pieces, up to kSlots of them under way at a time, and announces them as they arrive.
   void drive() {
     Transfer& t = *transfer_;
-    hipError_t error = hipSetDevice(t.device);  // a worker's device is whatever it served last
+    const OnDevice on(t.device);
+    hipError_t error = on.error;
     size_t launched = 0;
     bool gently = true;
     for (size_t p = 0; p < t.pieces && error == hipSuccess; ++p) {
@@ -840,6 +874,7 @@ class ResultStream {
   std::unique_ptr<Transfer> transfer_;
   HostWorkers::Job job_;
   bool under_way_ = false, misfit_ = false;
+  int device_ = -1;  // of the events and the ring
   uint8_t* ring_ = nullptr;
   size_t ring_bytes_ = 0;
   hipEvent_t packed_[kSlots] = {}, begun_ = nullptr;

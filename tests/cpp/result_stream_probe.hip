@@ -11,7 +11,51 @@
     if (e_ != hipSuccess) { printf("%s\n", hipGetErrorString(e_)); return 1; } \
   } while (0)
 
+// Words on one device brought home by a thread whose current device is another (or, where there is only one, the same):
+// the words are right and the thread's device stays what it was.
+static int on_other_devices() {
+  int devices = 0;
+  TRY(hipGetDeviceCount(&devices));
+  const size_t n = (size_t)70 * nd::kPackChunk;
+  std::vector<int32_t> want(n), got(n);
+  for (size_t i = 0; i < n; ++i) want[i] = (int32_t)(i & 0xfff);
+  nd::ResultStream results;
+  for (int home = 0; home < std::min(devices, 2); ++home) {
+    TRY(hipSetDevice(home));
+    int32_t* d = nullptr;
+    hipStream_t stream;
+    hipEvent_t done;
+    TRY(hipMalloc(&d, n * sizeof(int32_t)));
+    TRY(hipStreamCreate(&stream));
+    TRY(hipEventCreateWithFlags(&done, hipEventDisableTiming));
+    TRY(hipMemcpyAsync(d, want.data(), n * sizeof(int32_t), hipMemcpyHostToDevice, stream));
+    TRY(hipEventRecord(done, stream));
+    for (int away = 0; away < std::min(devices, 2); ++away) {
+      for (int ahead = 0; ahead < 2; ++ahead) {
+        printf("words on device %d, thread on %d, ahead %d\n", home, away, ahead);
+        fflush(stdout);
+        TRY(hipSetDevice(away));
+        std::fill(got.begin(), got.end(), -1);
+        std::vector<nd::ResultStream::Ready> ready;
+        if (ahead) ready.push_back({n, done});
+        TRY(results.begin(d, n, 12, 0, got.data(), stream, ready));
+        TRY(results.finish());
+        int now = -1;
+        TRY(hipGetDevice(&now));
+        if (now != away || got != want) { printf("device %d, or other words\n", now); return 1; }
+      }
+    }
+    TRY(hipSetDevice(home));
+    TRY(hipEventDestroy(done));
+    TRY(hipStreamDestroy(stream));
+    TRY(hipFree(d));
+  }
+  TRY(hipSetDevice(0));
+  return 0;
+}
+
 int main() {
+  if (on_other_devices() != 0) return 1;
   const size_t piece = (size_t)64 * nd::kPackChunk;  // the smallest piece
   const size_t sizes[] = {1, 7, 8, 9, nd::kPackChunk - 1, nd::kPackChunk, nd::kPackChunk + 1, piece, piece + 9, 13 * piece + 4097};
   nd::ResultStream stream;
