@@ -2199,10 +2199,14 @@ class Engine : public EngineBase {
       ready.push_back({end * F, range_ends_[r]});
       first = end;
     }
-    const hipError_t e = result_stream->begin(d_final_, (size_t)n_samples_ * F, (uint32_t)max_bits_, invalid_, rows_ahead,
-                                             stream_, std::move(ready));
-    if (e != hipSuccess) { last_error = std::string("results to the host: ") + hipGetErrorString(e); return -1; }
-    ahead_ = true;
+    // rows that cannot be sent now are fetched when they are asked for
+    try {
+      ahead_ = result_stream->begin(d_final_, (size_t)n_samples_ * F, (uint32_t)max_bits_, invalid_, rows_ahead, stream_,
+                                   std::move(ready)) == hipSuccess;
+    } catch (const std::bad_alloc&) {
+      ahead_ = false;
+    }
+    if (!ahead_) (void)hipGetLastError();
     return 0;
   }
 

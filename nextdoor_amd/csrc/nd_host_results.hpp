@@ -279,6 +279,15 @@ class HostArray {
     if (n) block_ = pool_->take(n * sizeof(T));
     size_ = n;
   }
+  // The same where the memory is only good to have: false, and empty, if there is none.
+  bool try_resize(size_t n) {
+    try {
+      resize(n);
+      return true;
+    } catch (const std::bad_alloc&) {
+      return false;
+    }
+  }
   // n elements, every one `value` (and every page touched: by several threads where there are many)
   void assign(size_t n, T value) {
     resize(n);
@@ -618,8 +627,8 @@ class ResultStream {
       if (e != hipSuccess) return e;
     }
     job_.body = [this] { take_part(); };
-    under_way_ = true;
     HostWorkers::get().start(job_, HostWorkers::kMost);
+    under_way_ = true;  // (not if start() throws: nobody has begun on it then)
     return hipSuccess;
   }
 

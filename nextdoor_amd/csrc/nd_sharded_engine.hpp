@@ -90,12 +90,12 @@ class ShardedEngine : public EngineBase {
       p->launch_graph = launch_graph;
       p->profiling = profiling;
     }
-    // A caller who took the last pass's rows, array and all, is expected to take this one's as well.
+    // A caller who took the last pass's rows, array and all, is expected to take this one's as well.  The pass does
+    // without where that fails, whatever it is.
     parts_[0]->rows_ahead = nullptr;
-    if (parts_.size() == 1 && parts_[0]->is_walk() && rows_fetched_ && hFinalSamples.taken()) {
-      rows_ahead_.resize(hFinalSamples.size());
+    if (parts_.size() == 1 && parts_[0]->is_walk() && rows_fetched_ && hFinalSamples.taken() &&
+        rows_ahead_.try_resize(hFinalSamples.size()))
       parts_[0]->rows_ahead = rows_ahead_.data();
-    }
     rows_fetched_ = false;
     times = PhaseTimes();
     const auto t0 = std::chrono::steady_clock::now();

@@ -6,12 +6,34 @@
 #include "../../nextdoor_amd/csrc/nd_sharded_engine.hpp"
 
 #include <stdio.h>
+#include <sys/resource.h>
 
 #define CHECK(expr)                                           \
   do {                                                        \
     if (!(expr)) { printf("not so: %s\n", #expr); return 1; } \
   } while (0)
 #define STEP(text) printf("%s\n", text), fflush(stdout)
+
+// Leaves the process `bytes` of private memory more than it has, or lifts that again (0).
+static bool leave_memory(size_t bytes) {
+  static rlim_t before = 0;
+  rlimit limit;
+  if (getrlimit(RLIMIT_DATA, &limit) != 0) return false;
+  if (bytes) {
+    size_t used_kb = 0;
+    char line[256];
+    FILE* f = fopen("/proc/self/status", "r");
+    if (!f) return false;
+    while (fgets(line, sizeof(line), f))
+      if (sscanf(line, "VmData: %zu kB", &used_kb) == 1) break;
+    fclose(f);
+    before = limit.rlim_cur;
+    limit.rlim_cur = used_kb * 1024 + bytes;
+  } else {
+    limit.rlim_cur = before;
+  }
+  return setrlimit(RLIMIT_DATA, &limit) == 0;
+}
 
 // more states than are copied without the result stream, and two ranges of walks
 static const int32_t kVertices = 1200007;
@@ -93,6 +115,24 @@ int main() {
     base.free_device();  // what nd_sampler_free_device does
     base.result_stream->release();
     CHECK(base.result_stream->page_locked_bytes() == 0);
+  }
+  STEP("no host memory for rows that nobody has asked for yet");
+  {
+    nd::ShardedEngine<Node2VecSample, WeightedNode2VecAppT<8>> sampler("walks");
+    nd::EngineBase& base = sampler;
+    CHECK(base.set_graph(&graph) == 0 && base.alloc(42) == 0);
+    CHECK(base.sample(nd::kTransitParallelLoadBalanced) == 0 && base.fetch_final_samples() == 0);
+    nd::HostLease* held = base.hFinalSamples.detach();
+    CHECK(leave_memory(n * sizeof(VertexID_t) / 2));
+    int rc = -1;
+    try {
+      rc = base.sample(nd::kTransitParallelLoadBalanced);
+    } catch (const std::bad_alloc&) {
+    }
+    CHECK(leave_memory(0));
+    CHECK(rc == 0 && base.fetch_final_samples() == 0);
+    CHECK(memcmp(base.hFinalSamples.data(), want.data(), n * sizeof(VertexID_t)) == 0);
+    delete held;
   }
   printf("all as they should be\n");
   return 0;
