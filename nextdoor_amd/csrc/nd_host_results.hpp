@@ -31,6 +31,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <condition_variable>
 #include <functional>
 #include <list>
@@ -46,14 +47,20 @@ namespace nd {
 // ---- host threads ------------------------------------------------------------------------
 
 // A few threads of the process that help whoever calls run(); they sleep otherwise.  They live
-// until the process ends (no destructor: a thread must not outlast what it waits on).
+// until the process ends (no destructor: a thread must not outlast what it waits on), and the process does not
+// end while one of them is at work: a thread inside the HIP runtime while that is being taken down does not come to a good end.
 class HostWorkers {
  public:
   // PPR walks over 262 K vertices, most groups dead: 1.33 ms with seven, 1.18 with eleven.
   static constexpr unsigned kMost = 11;
 
   static HostWorkers& get() {
-    static HostWorkers* workers = new HostWorkers;
+    static HostWorkers* workers = [] {
+      HostWorkers* w = new HostWorkers;
+      // what was registered last is done first: the runtime, which was there before any work for these threads, is still whole
+      (void)std::atexit([] { get().rest(); });
+      return w;
+    }();
     return *workers;
   }
 
@@ -96,6 +103,14 @@ class HostWorkers {
  private:
   HostWorkers() = default;
 
+  // No thread starts on anything any more; returns when none is at work.  What they work on ends by itself, within
+  // tens of milliseconds; if something else is amiss the process still ends.
+  void rest() {
+    std::unique_lock<std::mutex> lock(mutex_);
+    resting_ = true;
+    ended_.wait_for(lock, std::chrono::seconds(10), [&] { return at_work_ == 0; });
+  }
+
   static unsigned limit() {
     const unsigned hw = std::thread::hardware_concurrency();
     return hw > 1 ? std::min(hw * 3 / 4, kMost) : 0;
@@ -117,16 +132,18 @@ class HostWorkers {
     for (;;) {
       Job* job = nullptr;
       for (Job* j : jobs_)
-        if (j->wanted > 0) { job = j; break; }
+        if (j->wanted > 0 && !resting_) { job = j; break; }
       if (!job) {
         wake_.wait(lock);
         continue;
       }
       job->wanted--;
       job->running++;
+      at_work_++;
       lock.unlock();
       job->body();
       lock.lock();
+      at_work_--;
       if (--job->running == 0) ended_.notify_all();
     }
   }
@@ -134,7 +151,8 @@ class HostWorkers {
   std::mutex mutex_;
   std::condition_variable wake_, ended_;
   std::list<Job*> jobs_;
-  unsigned threads_ = 0;
+  unsigned threads_ = 0, at_work_ = 0;
+  bool resting_ = false;
 };
 
 // ---- host memory ---------------------------------------------------------------------------

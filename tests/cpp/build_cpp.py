@@ -20,6 +20,8 @@ RESULT_PROBE_SRC = os.path.join(HERE, "result_stream_probe.hip")
 RESULT_PROBE = os.path.join(HERE, "result_stream_probe")
 ROWS_AHEAD_PROBE_SRC = os.path.join(HERE, "rows_ahead_probe.hip")
 ROWS_AHEAD_PROBE = os.path.join(HERE, "rows_ahead_probe")
+HOST_RESULTS_PROBE_SRC = os.path.join(HERE, "host_results_probe.hip")
+HOST_RESULTS_PROBE = os.path.join(HERE, "host_results_probe")
 USER_APPS_SRC = os.path.join(HERE, "user_apps.hip")
 USER_APPS_LIB = os.path.join(HERE, "libuser_apps.so")
 
@@ -71,6 +73,11 @@ def build_rows_ahead_probe():
     return ROWS_AHEAD_PROBE
 
 
+def build_host_results_probe():
+    _run(_hipcc_flags() + [HOST_RESULTS_PROBE_SRC, "-o", HOST_RESULTS_PROBE, "-lpthread"])
+    return HOST_RESULTS_PROBE
+
+
 def build_user_apps():
     _run(_hipcc_flags() + ["-shared", USER_APPS_SRC, "-o", USER_APPS_LIB] + _link_flags())
     return USER_APPS_LIB
@@ -78,7 +85,7 @@ def build_user_apps():
 
 def build_all():
     return [build_host_probe(), build_template_probe(), build_result_probe(), build_rows_ahead_probe(),
-            build_user_apps()]
+            build_host_results_probe(), build_user_apps()]
 
 
 if __name__ == "__main__":
