@@ -7,6 +7,8 @@
 #include <sstream>
 #include <thread>
 
+#include "nd_host_threads.hpp"
+
 namespace nd {
 namespace {
 
@@ -38,8 +40,7 @@ class Verdict {
 
 template <class Fn>
 void for_each_sample(int64_t n_samples, Verdict& verdict, Fn fn) {
-  unsigned workers = std::min(std::thread::hardware_concurrency(), 16u);
-  if (workers == 0) workers = 4;
+  unsigned workers = host_threads(16);
   const int64_t block = 256;
   if (n_samples <= block) workers = 1;
   std::atomic<int64_t> next(0);

@@ -12,18 +12,12 @@
 #include <unordered_map>
 #include <vector>
 
+#include "nd_host_threads.hpp"
+
 namespace nd {
 namespace {
 
-int worker_count() {
-  unsigned hw = std::thread::hardware_concurrency();
-  if (hw == 0) hw = 4;
-  if (const char* env = getenv("ND_HOST_THREADS")) {
-    int v = atoi(env);
-    if (v > 0) return v;
-  }
-  return (int)std::min(hw, 16u);
-}
+int worker_count() { return (int)host_threads(16); }
 
 // Runs fn(begin, end) over [0, n) split into contiguous blocks handed out dynamically.
 void parallel_blocks(size_t n, size_t block, const std::function<void(size_t, size_t)>& fn) {

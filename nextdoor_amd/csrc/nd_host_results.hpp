@@ -42,6 +42,8 @@
 #include <thread>
 #include <vector>
 
+#include "nd_host_threads.hpp"
+
 namespace nd {
 
 // ---- host threads ------------------------------------------------------------------------
@@ -111,9 +113,11 @@ class HostWorkers {
     ended_.wait_for(lock, std::chrono::seconds(10), [&] { return at_work_ == 0; });
   }
 
+  // besides the thread that calls
   static unsigned limit() {
-    const unsigned hw = std::thread::hardware_concurrency();
-    return hw > 1 ? std::min(hw * 3 / 4, kMost) : 0;
+    if (const unsigned wanted = host_threads_wanted()) return std::min(wanted - 1, kMost);
+    const unsigned cpus = host_cpus();
+    return cpus > 1 ? std::min(cpus * 3 / 4, kMost) : 0;
   }
 
   void grow(unsigned helpers) {

@@ -1,5 +1,7 @@
 // The host side of results on their way (nd_host_results.hpp), on a machine without a GPU: what is asked for is the first argument.
 //   exit     the process ends while one of the threads is at work: prints "ended 1" if that work was waited for
+//   cpus     CPUs that the control groups under a folder give a process whose groups a file lists (two more arguments)
+//   threads  threads that took part in something
 #include "../../nextdoor_amd/csrc/nd_host_results.hpp"
 
 #include <stdio.h>
@@ -20,8 +22,24 @@ static int exit_while_at_work() {
   return 0;
 }
 
+static int threads_that_take_part() {
+  std::mutex mutex;
+  std::vector<std::thread::id> seen;
+  nd::HostWorkers::get().run(nd::HostWorkers::kMost, [&] {
+    {
+      std::lock_guard<std::mutex> lock(mutex);
+      seen.push_back(std::this_thread::get_id());
+    }
+    std::this_thread::sleep_for(std::chrono::milliseconds(300));
+  });
+  printf("%zu\n", seen.size());
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "exit") return exit_while_at_work();
+  if (what == "cpus" && argc > 3) return printf("%g\n", nd::cpus_of_groups(argv[2], argv[3])) < 0;
+  if (what == "threads") return threads_that_take_part();
   return 2;
 }
