@@ -124,8 +124,7 @@ class EngineBase {
     if (bytes > kDirectResultBytes && bytes % sizeof(int32_t) == 0) {
       e = result_stream->fetch((const int32_t*)src, bytes / sizeof(int32_t), bits, fill, (int32_t*)dst, stream);
     } else {
-      e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream);
-      if (e == hipSuccess) e = hipStreamSynchronize(stream);
+      e = result_stream->copy(src, bytes, dst, stream);
     }
     if (e == hipSuccess) return 0;
     last_error = std::string("results to the host: ") + hipGetErrorString(e);

@@ -162,18 +162,21 @@ class HostWorkers {
 // ---- host memory ---------------------------------------------------------------------------
 
 struct HostBlock {
-  enum Kind { kNone, kPinned, kPages, kHeap };
   void* p = nullptr;
   size_t bytes = 0;
-  Kind kind = kNone;
+  bool mapped = false;  // by mmap, else from the heap
 };
 
-// Results up to this size are copied by the copy engine straight into page-locked memory; above it
-// they are packed and streamed (ResultStream).
-constexpr size_t kDirectResultBytes = 4u << 20;
+// Results up to this size go through page-locked memory by the copy engine and one thread, above it they are packed and
+// streamed by several.  Copied / streamed with ids of 12 and of 32 bits, us: 0.5 MB 31 / 75, 82; 1.1 MB 67 / 95, 105;
+// 1.5 MB 92 / 100, 116; 2 MB 118 / 110, 128; 3 MB 169 / 121, 155; 4 MB 220 / 113, 158.
+constexpr size_t kDirectResultBytes = 2u << 20;
 
 // The host arrays of one sampler.  At most kKeep of them wait for their next use; all of those are
 // freed when the sampler goes, the others when their holders let go of them.
+// They are ordinary private memory, since callers do with them what they do with any array: page-locked memory
+// of the runtime's is not there in a forked child (a data loader's worker that touches it dies), nor may system calls
+// that pin pages use it.  (The copy engine writing into it directly would save 1.1 MB of results 39 of 67 us.)
 class HostPool {
  public:
   HostPool() = default;
@@ -182,7 +185,6 @@ class HostPool {
   ~HostPool() { close(); }
 
   HostBlock take(size_t bytes) {
-    bool pinned = bytes <= kDirectResultBytes;
     {
       std::lock_guard<std::mutex> lock(mutex_);
       for (size_t i = 0; i < free_.size(); ++i)
@@ -191,22 +193,8 @@ class HostPool {
           free_.erase(free_.begin() + (ptrdiff_t)i);
           return b;
         }
-      // page-locked memory is for what is in use, not for arrays a caller collects
-      pinned = pinned && pinned_ < kMostPinned;
-      if (pinned) pinned_++;
     }
     HostBlock b;
-    if (pinned) {
-      if (hipHostMalloc(&b.p, bytes, hipHostMallocDefault) == hipSuccess && b.p) {
-        b.bytes = bytes;
-        b.kind = HostBlock::kPinned;
-        return b;
-      }
-      (void)hipGetLastError();  // the refusal is not an error of a later call
-      b.p = nullptr;
-      std::lock_guard<std::mutex> lock(mutex_);
-      pinned_--;
-    }
     if (bytes > kDirectResultBytes) {
       // 2 MB pages: a two-thousandth of the faults
       const size_t whole = (bytes + kPage - 1) / kPage * kPage;
@@ -218,14 +206,13 @@ class HostPool {
         (void)madvise(at, whole, MADV_HUGEPAGE);
         b.p = at;
         b.bytes = whole;
-        b.kind = HostBlock::kPages;
+        b.mapped = true;
         return b;
       }
     }
     b.p = malloc(bytes);
     if (!b.p) throw std::bad_alloc();
     b.bytes = bytes;
-    b.kind = HostBlock::kHeap;
     return b;
   }
 
@@ -233,7 +220,7 @@ class HostPool {
     HostBlock drop = b;
     {
       std::lock_guard<std::mutex> lock(mutex_);
-      if (open_ && b.kind != HostBlock::kHeap) {
+      if (open_) {
         free_.push_back(b);
         drop = HostBlock();
         if (free_.size() > kKeep) {
@@ -241,7 +228,6 @@ class HostPool {
           free_.erase(free_.begin());
         }
       }
-      if (drop.kind == HostBlock::kPinned) pinned_--;
     }
     release(drop);
   }
@@ -259,18 +245,15 @@ class HostPool {
  private:
   // two arrays of a loop that holds the last result while it makes the next, for each of two results
   static constexpr size_t kKeep = 4;
-  static constexpr int kMostPinned = 8;
   static constexpr size_t kPage = 2u << 20;
 
   static void release(const HostBlock& b) {
-    if (b.kind == HostBlock::kPinned) (void)hipHostFree(b.p);
-    else if (b.kind == HostBlock::kPages) munmap(b.p, b.bytes);
-    else if (b.kind == HostBlock::kHeap) free(b.p);
+    if (b.mapped) munmap(b.p, b.bytes);
+    else free(b.p);
   }
 
   std::mutex mutex_;
   std::vector<HostBlock> free_;
-  int pinned_ = 0;
   bool open_ = true;
 };
 
@@ -293,7 +276,6 @@ class HostArray {
   const T* data() const { return (const T*)block_.p; }
   size_t size() const { return size_; }
   bool empty() const { return size_ == 0; }
-  bool page_locked() const { return block_.kind == HostBlock::kPinned; }
 
   void resize(size_t n) {
     if (n == size_ && (n == 0 || block_.p)) return;
@@ -614,6 +596,22 @@ class ResultStream {
     hipEvent_t event;
   };
 
+  // bytes at src to dst as they are, in stream order, complete on return.  For few of them, and for what is not words.
+  hipError_t copy(const void* src, size_t bytes, void* dst, hipStream_t stream) {
+    hipError_t e = finish();  // an earlier one that nobody waited for
+    if (e == hipSuccess) e = come_to_device_of(stream);
+    if (e != hipSuccess || bytes == 0) return e;
+    const OnDevice on(device_);
+    e = on.error != hipSuccess ? on.error : make_ring(kDirectResultBytes);
+    for (size_t at = 0; at < bytes && e == hipSuccess; at += kDirectResultBytes) {
+      const size_t here = std::min(bytes - at, kDirectResultBytes);
+      e = hipMemcpyAsync(ring_, (const char*)src + at, here, hipMemcpyDeviceToHost, stream);
+      if (e == hipSuccess) e = hipStreamSynchronize(stream);
+      if (e == hipSuccess) memcpy((char*)dst + at, ring_, here);
+    }
+    return e;
+  }
+
   // n words at src (aligned to 16 bytes) to dst, in stream order.  Words that are `fill` in groups of eight cost
   // nothing; words are expected to fit `bits` bits (one that does not makes the whole transfer start again with
   // 32).  Large transfers only: it pays from a few megabytes on.
@@ -631,13 +629,12 @@ class ResultStream {
     if (e != hipSuccess || n == 0) return e;
     if (!transfer_) transfer_.reset(new Transfer);
     Transfer& t = *transfer_;
-    e = device_of(stream, &t.device);
+    e = come_to_device_of(stream);
     if (e != hipSuccess) return e;
+    t.device = device_;
     const OnDevice on(t.device);
     if (on.error != hipSuccess) return on.error;
     t.set(src, n, bits > kPackMostBits ? 32 : bits, fill, dst, std::move(ready));
-    if (t.device != device_) release_device();  // events of one device are not recorded on another's streams
-    device_ = t.device;
     e = prepare(t.slot_bytes);
     if (e != hipSuccess) return e;
     t.streams[0] = t.streams[1] = transfer_stream(t.device);
@@ -706,6 +703,25 @@ class ResultStream {
   static constexpr size_t kGentleAhead = 2;
   static constexpr int kSpins = 4000;  // tens of microseconds; none: 1.68 GB in 19 instead of 13 ms, 23 MB in 527 instead of 290 us
 
+  hipError_t come_to_device_of(hipStream_t stream) {
+    int device = 0;
+    const hipError_t e = device_of(stream, &device);
+    if (e != hipSuccess || device == device_) return e;
+    release_device();  // events of one device are not recorded on another's streams
+    device_ = device;
+    return hipSuccess;
+  }
+
+  hipError_t make_ring(size_t bytes) {
+    if (ring_bytes_ >= bytes) return hipSuccess;
+    if (ring_) (void)hipHostFree(ring_);
+    ring_ = nullptr;
+    ring_bytes_ = 0;
+    const hipError_t e = hipHostMalloc((void**)&ring_, bytes, hipHostMallocDefault);
+    if (e == hipSuccess) ring_bytes_ = bytes;
+    return e;
+  }
+
   hipError_t prepare(size_t slot_bytes) {
     for (hipEvent_t& ev : packed_)
       if (!ev) {
@@ -716,13 +732,7 @@ class ResultStream {
       const hipError_t e = hipEventCreateWithFlags(&begun_, hipEventDisableTiming);
       if (e != hipSuccess) return e;
     }
-    if (ring_bytes_ >= slot_bytes * kSlots) return hipSuccess;
-    if (ring_) (void)hipHostFree(ring_);
-    ring_ = nullptr;
-    ring_bytes_ = 0;
-    const hipError_t e = hipHostMalloc((void**)&ring_, slot_bytes * kSlots, hipHostMallocDefault);
-    if (e == hipSuccess) ring_bytes_ = slot_bytes * kSlots;
-    return e;
+    return make_ring(slot_bytes * kSlots);
   }
 
   struct Transfer {

@@ -75,6 +75,11 @@ int main() {
         if (misfit) want[n / 2] = -5;
         TRY(hipMemcpy(d, want.data(), n * sizeof(int32_t), hipMemcpyHostToDevice));
         for (int shift = 0; shift < 2; ++shift) {
+          if (bits == 32) {  // as bytes, the last word not whole
+            const size_t bytes = n * sizeof(int32_t) - (size_t)shift;
+            TRY(stream.copy(d, bytes, got.data() + shift, nullptr));
+            if (memcmp(got.data() + shift, want.data(), bytes) != 0) { printf("bytes differ\n"); return 1; }
+          }
           TRY(stream.fetch(d, n, bits, fill, got.data() + shift, nullptr));
           if (memcmp(got.data() + shift, want.data(), n * sizeof(int32_t)) != 0 || got[n + 1] != 77) {
             printf("differs at shift %d\n", shift);

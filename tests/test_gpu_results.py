@@ -27,7 +27,7 @@ def test_what_is_asked_for_before_rows_that_are_on_their_way():
     assert out.returncode == 0 and out.stdout.endswith("all as they should be\n"), out.stdout[-300:] + out.stderr[-300:]
 
 
-# 1.1 MB: copied as it is; 8.8 MB: packed (12 bits, the ids and INVALID); 36 MB of 16 and 17 bits
+# 1.1 MB: copied as it is; 4.5 MB: packed (12 bits, the ids and INVALID); 36 MB of 15 and 16 bits
 @pytest.mark.parametrize("n", [1000, 4095, 32767, 32768])
 def test_arrays_stay_the_callers(oracle, n):
     g = graphs.random_graph(n=n, mean_degree=6, seed=n, isolated_every=3)
@@ -47,6 +47,32 @@ def test_arrays_stay_the_callers(oracle, n):
     s.close()
     for turn, got in held:
         assert np.all(got == -turn)
+
+
+def mapping_flags(address):
+    """The kernel's flags of the mapping an address is in (/proc/self/smaps)."""
+    inside = False
+    for line in open("/proc/self/smaps"):
+        first = line.split()[0]
+        if not first.endswith(":"):
+            lo, hi = (int(x, 16) for x in first.split("-"))
+            inside = lo <= address < hi
+        elif inside and first == "VmFlags:":
+            return line.split()[1:]
+
+
+@pytest.mark.parametrize("n", [300, 2711, 4095, 9000])  # 0.3 and 3 MB, 4.5 MB, 9.9 MB
+def test_arrays_are_ordinary_memory(n):
+    """What a forked child inherits and system calls may pin, as any other array of the caller's."""
+    s = nd.Sampler("KHop", graphs.random_graph(n=n, mean_degree=6, seed=n), seed=42)
+    for _ in range(3):
+        s.do_transit_parallel()
+        got = s.final_samples()
+        for address in (got.ctypes.data, got.ctypes.data + got.nbytes - 1):
+            flags = mapping_flags(address)
+            # dc: left out in a child; io, pf: a device's pages; sh: shared with a child that writes to it
+            assert flags and not {"dc", "io", "pf", "sh"} & set(flags), flags
+    s.close()
 
 
 # fewer walks than are split into ranges, two ranges, and more than the device holds at once
