@@ -610,6 +610,7 @@ void nd_sampler_free_device(nd_sampler* s) {
   if (!s) return;
   s->engine->free_device();
   s->engine->result_stream->release();
+  s->engine->host_pool->trim();
 }
 
 void nd_sampler_destroy(nd_sampler* s) { delete s; }

@@ -172,8 +172,8 @@ struct HostBlock {
 // 1.5 MB 92 / 100, 116; 2 MB 118 / 110, 128; 3 MB 169 / 121, 155; 4 MB 220 / 113, 158.
 constexpr size_t kDirectResultBytes = 2u << 20;
 
-// The host arrays of one sampler.  At most kKeep of them wait for their next use; all of those are
-// freed when the sampler goes, the others when their holders let go of them.
+// The host arrays of one sampler.  At most kKeep of them wait for their next use; all of those are freed with the
+// sampler's device memory and when it goes, the others when their holders let go of them.
 // They are ordinary private memory, since callers do with them what they do with any array: page-locked memory
 // of the runtime's is not there in a forked child (a data loader's worker that touches it dies), nor may system calls
 // that pin pages use it.  (The copy engine writing into it directly would save 1.1 MB of results 39 of 67 us.)
@@ -232,19 +232,32 @@ class HostPool {
     release(drop);
   }
 
-  void close() {
+  // frees those that wait
+  void trim() { drop_waiting(true); }
+  // ... and keeps none from here on
+  void close() { drop_waiting(false); }
+
+  size_t waiting_bytes() {
+    std::lock_guard<std::mutex> lock(mutex_);
+    size_t sum = 0;
+    for (const HostBlock& b : free_) sum += b.bytes;
+    return sum;
+  }
+
+ private:
+  // A loop that holds its last results while it makes the next leaves one array of each kind waiting at a time, and
+  // no sampler has more than two kinds (rows and states; rows and columns).
+  static constexpr size_t kKeep = 2;
+
+  void drop_waiting(bool open) {
     std::vector<HostBlock> all;
     {
       std::lock_guard<std::mutex> lock(mutex_);
-      open_ = false;
+      open_ = open_ && open;
       all.swap(free_);
     }
     for (const HostBlock& b : all) release(b);
   }
-
- private:
-  // two arrays of a loop that holds the last result while it makes the next, for each of two results
-  static constexpr size_t kKeep = 4;
   static constexpr size_t kPage = 2u << 20;
 
   static void release(const HostBlock& b) {

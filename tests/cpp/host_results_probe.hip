@@ -2,6 +2,7 @@
 //   exit     the process ends while one of the threads is at work: prints "ended 1" if that work was waited for
 //   cpus     CPUs that the control groups under a folder give a process whose groups a file lists (two more arguments)
 //   threads  threads that took part in something
+//   pool     bytes that wait for their next use after arrays were given back, after a trim, and at the end
 #include "../../nextdoor_amd/csrc/nd_host_results.hpp"
 
 #include <stdio.h>
@@ -36,10 +37,29 @@ static int threads_that_take_part() {
   return 0;
 }
 
+static int arrays_that_wait() {
+  auto pool = std::make_shared<nd::HostPool>();
+  std::vector<nd::HostBlock> held;
+  for (int i = 0; i < 5; ++i) held.push_back(pool->take(16u << 20));
+  for (const nd::HostBlock& b : held) pool->give(b);
+  printf("%zu\n", pool->waiting_bytes());
+  pool->trim();
+  printf("%zu\n", pool->waiting_bytes());
+  nd::HostBlock last = pool->take(1000);
+  pool->give(last);
+  printf("%zu\n", pool->waiting_bytes());
+  last = pool->take(1000);
+  pool->close();
+  pool->give(last);
+  printf("%zu\n", pool->waiting_bytes());
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "exit") return exit_while_at_work();
   if (what == "cpus" && argc > 3) return printf("%g\n", nd::cpus_of_groups(argv[2], argv[3])) < 0;
+  if (what == "pool") return arrays_that_wait();
   if (what == "threads") return threads_that_take_part();
   return 2;
 }

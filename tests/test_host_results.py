@@ -46,3 +46,7 @@ def test_the_control_groups_share_is_counted(probe, tmp_path, files, groups, cpu
         (root / name).write_text(text + "\n")
     (tmp_path / "groups").write_text(groups)
     assert probe("cpus", root, tmp_path / "groups").strip() == cpus
+
+
+def test_two_arrays_at_most_wait_for_their_next_use(probe):
+    assert [int(x) for x in probe("pool").split()] == [2 * (16 << 20), 0, 1000, 0]
