@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <mutex>
 #include <string>
 
 #include "nd_contract.hpp"
@@ -178,22 +179,34 @@ class DeviceGraph {
     return true;
   }
 
-  // The vertices as walk records, built when first asked for; nullptr: an error.
+  // The vertices as walk records, built when first asked for (engines that share the graph ask from their own threads);
+  // nullptr: an error.
   const WalkVertex* walk_vertices(hipStream_t stream) {
+    std::lock_guard<std::mutex> lock(tables_);
     if (!walk_vertices_) {
-      if (hipMalloc(&walk_vertices_, sizeof(WalkVertex) * (size_t)view.n_vertices) != hipSuccess) return nullptr;
+      if (hipMalloc(&walk_vertices_, sizeof(WalkVertex) * (size_t)view.n_vertices) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+      }
       build_walk_vertices<<<dim3((unsigned)(((size_t)view.n_vertices + 255) / 256)), dim3(256), 0, stream>>>(view, walk_vertices_);
       if (hipGetLastError() != hipSuccess || hipStreamSynchronize(stream) != hipSuccess) free_one(walk_vertices_);
     }
     return walk_vertices_;
   }
 
-  // The edges as walk records, built when first asked for; nullptr where there is no memory for them.
+  // The edges as walk records, built when first asked for; nullptr where they would take more than half of the memory that
+  // is left: they save a walk a fetch a step, and what else the program has to put on the device comes first.
   template <class Record>
   const Record* walk_edges(hipStream_t stream) {
+    std::lock_guard<std::mutex> lock(tables_);
     if (walk_edges_ && walk_record_ != sizeof(Record)) free_one(walk_edges_);
     if (!walk_edges_ && view.n_edges > 0) {
       void* p = nullptr;
+      size_t left = 0, all = 0;
+      if (hipMemGetInfo(&left, &all) != hipSuccess || sizeof(Record) * (size_t)view.n_edges > left / 2) {
+        (void)hipGetLastError();
+        return nullptr;
+      }
       if (hipMalloc(&p, sizeof(Record) * (size_t)view.n_edges) != hipSuccess) {
         (void)hipGetLastError();
         return nullptr;
@@ -239,6 +252,7 @@ class DeviceGraph {
   char* walk_edges_ = nullptr;
   WalkVertex* walk_vertices_ = nullptr;
   size_t walk_record_ = 0;
+  std::mutex tables_;
 };
 
 }  // namespace nd

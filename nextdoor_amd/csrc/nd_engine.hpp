@@ -1944,16 +1944,6 @@ class Engine : public EngineBase {
     // the result per output, so they go to one array per step and are regrouped at the end.
     rows_direct_ = true;
     for (int k = 0; k < n_steps; ++k) rows_direct_ = rows_direct_ && layout_.seg_len[k] >= kDirectSegment;
-    // (one more column where the steps of a walk are odd in number: its results go in cells of two)
-    if (!rows_direct_) ND_HIP_TRY(hipMalloc(&d_step_out_, sizeof(VertexID_t) * (size_t)n_samples_ * (F + 1)));
-    ND_HIP_TRY(hipMalloc(&d_keys_a_, sizeof(uint32_t) * max_pairs_));
-    ND_HIP_TRY(hipMalloc(&d_vals_a_, sizeof(uint32_t) * max_pairs_));
-    ND_HIP_TRY(hipMalloc(&d_keys_b_, sizeof(uint32_t) * max_pairs_));
-    ND_HIP_TRY(hipMalloc(&d_vals_b_, sizeof(uint32_t) * max_pairs_));
-    const SortPlan plan = make_sort_plan(max_pairs_, max_bits_);
-    ND_HIP_TRY(hipMalloc(&d_hist_, sizeof(uint32_t) * sort_hist_capacity(max_pairs_)));
-    ND_HIP_TRY(hipMalloc(&d_scratch_, sizeof(uint32_t) * plan.scratch_elems));
-    ND_HIP_TRY(hipMalloc(&d_live_, sizeof(uint32_t) * 2));
     // walks: every step has one pair per sample and one output per pair
     walk_mode_ = init_size_ == 1 && n_steps > 1;
     for (int k = 0; k < n_steps; ++k) walk_mode_ = walk_mode_ && app.stepSize(k) == 1;
@@ -1961,93 +1951,12 @@ class Engine : public EngineBase {
     // apps that choose their transits themselves and are not walks: the next step's map is an
     // array of its own, written next to the step's outputs
     explicit_map_ = app.hasExplicitTransits() && !walk_mode_;
-    if (explicit_map_) ND_HIP_TRY(hipMalloc(&d_explicit_, sizeof(VertexID_t) * max_pairs_));
-    if (walk_mode_) {
-      ND_HIP_TRY(hipMalloc(&d_emit_keys_, sizeof(uint32_t) * max_pairs_));
-      ND_HIP_TRY(hipMalloc(&d_emit_slots_, sizeof(uint32_t) * max_pairs_));
-    }
-    // Counters per vertex for the small-map inversion: the walks that step onto a vertex are
-    // about its share of the edge ends; one counter per kSmallMapWalksPerCounter of them.
-    small_map_ = false;
-    inversion_forced_ = getenv("ND_SMALL_MAP") != nullptr;  // chooses how the map is inverted: so it is
-    if (walk_mode_ && max_pairs_ <= kSmallMapPairs && (uint64_t)invalid_ < kSmallMapCounters &&
-        !(getenv("ND_SMALL_MAP") && atoi(getenv("ND_SMALL_MAP")) == 0)) {
-      const size_t V = (size_t)graph_->get_n_vertices();
-      const double per_edge = graph_->col.empty() ? 0.0 : (double)max_pairs_ / (double)graph_->col.size();
-      std::vector<uint32_t> base(V + 1), edges_into(V, 0), place_start(1, 0u);
-      for (const CSR::Edge dst : graph_->col) edges_into[(size_t)dst]++;
-      uint64_t at = 0;
-      for (size_t v = 0; v < V; ++v) {
-        base[v] = (uint32_t)at;
-        const double walks = per_edge * (double)edges_into[v];
-        uint32_t copies = 1;
-        while (copies < kSmallMapMaxCopies && (double)(copies * kSmallMapWalksPerCounter) < walks) copies <<= 1;
-        at += copies;
-        // places of each of its counters when the pairs are placed as they are emitted: twice
-        // the walks it expects and a few more
-        const uint32_t places = (uint32_t)(2.0 * walks / copies) + kSmallMapSparePlaces;
-        for (uint32_t c = 0; c < copies; ++c) place_start.push_back(place_start.back() + places);
-      }
-      base[V] = (uint32_t)at;
-      small_counters_ = (size_t)at + 1;  // one more, so that every run has an end to read
-      place_start.push_back(place_start.back());  // ... which owns no place
-      small_map_ = small_counters_ < kSmallMapCounters;
-      if (small_map_) {
-        ND_HIP_TRY(hipMalloc(&d_counter_base_, sizeof(uint32_t) * base.size()));
-        ND_HIP_TRY(hipMemcpy(d_counter_base_, base.data(), sizeof(uint32_t) * base.size(), hipMemcpyHostToDevice));
-      }
-      // Placing at emission walks every place at every step: only where the places are not many
-      // times the pairs (ND_SMALL_MAP=1 keeps the two placing launches).
-      small_placed_ = small_map_ && (size_t)place_start.back() <= kSmallMapPlacesPerPair * max_pairs_ &&
-                      !(getenv("ND_SMALL_MAP") && atoi(getenv("ND_SMALL_MAP")) == 1);
-      if (small_placed_) {
-        placed_spill_first_ = place_start.back();
-        placed_places_ = (size_t)placed_spill_first_ + max_pairs_;  // every pair could spill
-        ND_HIP_TRY(hipMalloc(&d_place_start_, sizeof(uint32_t) * place_start.size()));
-        ND_HIP_TRY(hipMemcpy(d_place_start_, place_start.data(), sizeof(uint32_t) * place_start.size(),
-                             hipMemcpyHostToDevice));
-        for (int b = 0; b < 2; ++b) {
-          ND_HIP_TRY(hipMalloc(&d_placed_keys_[b], sizeof(uint32_t) * placed_places_));
-          ND_HIP_TRY(hipMalloc(&d_placed_slots_[b], sizeof(uint32_t) * placed_places_));
-          ND_HIP_TRY(hipMemset(d_placed_slots_[b], 0, sizeof(uint32_t) * placed_places_));
-          if (state_fits_pair<SampleType>::value) {
-            ND_HIP_TRY(hipMalloc(&d_placed_state_[b], sizeof(uint32_t) * placed_places_));
-            ND_HIP_TRY(hipMemset(d_placed_state_[b], 0, sizeof(uint32_t) * placed_places_));
-          }
-          ND_HIP_TRY(hipMalloc(&d_placed_counts_[b], sizeof(uint32_t) * (small_counters_ + 1)));
-        }
-        placed_dirty_ = true;  // cleared by the first pass that uses them
-      }
-    }
-    if (small_map_) {
-      // counters, their starts inside a chunk, chunk totals
-      const size_t counters = small_counters_, chunks = (counters + kSmallMapChunk - 1) / kSmallMapChunk;
-      ND_HIP_TRY(hipMalloc(&d_small_, sizeof(uint32_t) * (2 * counters + chunks)));
-      ND_HIP_TRY(hipMemset(d_small_, 0, sizeof(uint32_t) * (2 * counters + chunks)));
-      ND_HIP_TRY(hipMalloc(&d_emit_ranks_, sizeof(uint32_t) * max_pairs_));
-    }
-    if (state_travels_) {
-      ND_HIP_TRY(hipMalloc(&d_emit_state_, sizeof(uint32_t) * max_pairs_));
-      ND_HIP_TRY(hipMalloc(&d_aux_a_, sizeof(uint32_t) * max_pairs_));
-      ND_HIP_TRY(hipMalloc(&d_aux_b_, sizeof(uint32_t) * max_pairs_));
-    }
-    ND_HIP_TRY(hipMalloc(&d_meta_, sizeof(RunsMeta) * 2));
-    {
-      RunsMeta fresh[2] = {};
-      fresh[0].stamp = 1;  // the first load-balanced step; every classification hands the next one its stamp
-      ND_HIP_TRY(hipMemcpy(d_meta_, fresh, sizeof(fresh), hipMemcpyHostToDevice));
-    }
-    ND_HIP_TRY(hipMalloc(&d_balance_, sizeof(uint32_t) * kBalanceWords));
-    ND_HIP_TRY(hipMemset(d_balance_, 0, sizeof(uint32_t) * kBalanceWords));
     class_counters_ = ClassCounters();
     idle_passes_ = 0;
     balanced_steps_ = 0;
     markers_cleared_at_ = 0;
     schedule_counts_ = ScheduleCounts();
     items_seen_ = false;
-    ND_HIP_TRY(hipMalloc(&d_chunks_, sizeof(WorkItem) * (size_t)chunk_capacity_));
-    ND_HIP_TRY(hipMalloc(&d_taken_stamp_, sizeof(uint32_t) * ((size_t)invalid_ + 1)));
-    ND_HIP_TRY(hipMemset(d_taken_stamp_, 0, sizeof(uint32_t) * ((size_t)invalid_ + 1)));
     ND_HIP_TRY(hipStreamCreate(&side_stream_));
     ND_HIP_TRY(hipEventCreate(&ev_a_));
     ND_HIP_TRY(hipEventCreate(&ev_b_));
@@ -2086,19 +1995,13 @@ class Engine : public EngineBase {
       ND_HIP_TRY(hipGetDevice(&device));
       ND_HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
       ND_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, walk_rows_kernel<SampleType, App, true>, kFlatThreads, 0));
-      if (app_uses_weights<App>::value) walk_vertices_ = dgraph_->walk_vertices(stream_);
-      if (app_uses_weights<App>::value && !walk_vertices_) { last_error = "no device memory for the walk vertices"; return -1; }
-      walk_records_ = nullptr;
-      // (not where stepTransits names another vertex than next() returned; nor for an app that looks edges up,
-      // whose tests are what its steps wait for: weighted node2vec over 1.07 GB of edges 24.1 ms, over records 26.4)
-      const size_t edge_bytes = (app_uses_weights<App>::value ? sizeof(EdgeRecord) : sizeof(CSR::Edge)) *
-                                (size_t)graph_->get_n_edges();
-      if (edge_bytes >= kWalkRecordsFromBytes && !app.hasExplicitTransits() && !app_uses_edge_lookup<App>::value)
-        walk_records_ = dgraph_->template walk_edges<walk_record<App>>(stream_);
       walk_waves_at_once_ = (uint32_t)std::max(1, per_cu * cus);
       walk_waves_queued_ = (uint32_t)std::max(1, (int)kQueuedWavesPerCu * cus);
     }
-    if (paired_results_) ND_HIP_TRY(hipMalloc(&d_walk_cells_, sizeof(uint32_t) * (size_t)n_samples_));
+    const char* small_map = getenv("ND_SMALL_MAP");
+    inversion_forced_ = small_map != nullptr;  // chooses how the map is inverted: so it is
+    small_map_switch_ = small_map ? atoi(small_map) : -1;
+    if (!walk_mode_ && alloc_inversion() != 0) return -1;  // walks: by the first pass that inverts
     allocated_ = true;
     return 0;
   }
@@ -2108,6 +2011,7 @@ class Engine : public EngineBase {
   int sample(int mode) override {
     if (!allocated_) { last_error = "sample before alloc"; return -1; }
     (void)finish_rows_ahead();  // nobody asked for them
+    if ((inverts(mode) ? alloc_inversion() : build_walk_tables()) != 0) return -1;  // what an earlier pass has not
     times = PhaseTimes();
     if (!std::is_empty<SampleType>::value) {
       ND_HIP_TRY(hipMemcpyAsync(d_samples_, d_samples_init_, sizeof(SampleType) * (size_t)n_samples_,
@@ -2264,8 +2168,7 @@ class Engine : public EngineBase {
     const int n_steps = app.steps();
     const size_t F = (size_t)final_sample_size();
     const bool sample_parallel = mode == kSampleParallel;
-    const bool inverts = inversion_period == 1 || (inversion_period == 0 && inversion_forced_);
-    if (walk_mode_ && (sample_parallel || !inverts)) return enqueue_walks();
+    if (!inverts(mode)) return enqueue_walks();
     // A pass whose classifications found nothing at all for the workgroup kernel is followed by
     // passes that do not classify (nor launch the workgroup kernel); every kIdleLookEvery-th
     // pass looks again.  Results do not depend on it.
@@ -2699,6 +2602,135 @@ class Engine : public EngineBase {
       kMaxSteps + 2 + (int)(kCounterCopies * sizeof(ClassCounters) / sizeof(uint32_t));
   static constexpr int kIdleLookEvery = 8;
   static constexpr uint32_t kMostWalkRanges = 6;
+
+  // Whether a pass brings the pairs into transit order (or, sample-parallel and no walk, only drops the dead ones).
+  bool inverts(int mode) const {
+    return !walk_mode_ || (mode != kSampleParallel && (inversion_period == 1 || (inversion_period == 0 && inversion_forced_)));
+  }
+
+  // What only passes that invert use: 410 bytes a walk of 100 steps for its results step by step, and the pairs to
+  // be sorted.  Walks that keep their lanes need none of it, so a sampler of walks takes it when a pass first inverts.
+  int alloc_inversion() {
+    if (inversion_ready_) return 0;
+    const int rc = alloc_inversion_buffers();
+    if (rc != 0) free_inversion_buffers();
+    inversion_ready_ = rc == 0;
+    return rc;
+  }
+  int alloc_inversion_buffers() {
+    const size_t F = (size_t)final_sample_size();
+    // (one more column where the steps of a walk are odd in number: its results go in cells of two)
+    if (!rows_direct_) ND_HIP_TRY(hipMalloc(&d_step_out_, sizeof(VertexID_t) * (size_t)n_samples_ * (F + 1)));
+    ND_HIP_TRY(hipMalloc(&d_keys_a_, sizeof(uint32_t) * max_pairs_));
+    ND_HIP_TRY(hipMalloc(&d_vals_a_, sizeof(uint32_t) * max_pairs_));
+    ND_HIP_TRY(hipMalloc(&d_keys_b_, sizeof(uint32_t) * max_pairs_));
+    ND_HIP_TRY(hipMalloc(&d_vals_b_, sizeof(uint32_t) * max_pairs_));
+    const SortPlan plan = make_sort_plan(max_pairs_, max_bits_);
+    ND_HIP_TRY(hipMalloc(&d_hist_, sizeof(uint32_t) * sort_hist_capacity(max_pairs_)));
+    ND_HIP_TRY(hipMalloc(&d_scratch_, sizeof(uint32_t) * plan.scratch_elems));
+    ND_HIP_TRY(hipMalloc(&d_live_, sizeof(uint32_t) * 2));
+    if (explicit_map_) ND_HIP_TRY(hipMalloc(&d_explicit_, sizeof(VertexID_t) * max_pairs_));
+    if (walk_mode_) {
+      ND_HIP_TRY(hipMalloc(&d_emit_keys_, sizeof(uint32_t) * max_pairs_));
+      ND_HIP_TRY(hipMalloc(&d_emit_slots_, sizeof(uint32_t) * max_pairs_));
+    }
+    // Counters per vertex for the small-map inversion: the walks that step onto a vertex are
+    // about its share of the edge ends; one counter per kSmallMapWalksPerCounter of them.
+    small_map_ = false;
+    if (walk_mode_ && max_pairs_ <= kSmallMapPairs && (uint64_t)invalid_ < kSmallMapCounters &&
+        small_map_switch_ != 0) {
+      const size_t V = (size_t)graph_->get_n_vertices();
+      const double per_edge = graph_->col.empty() ? 0.0 : (double)max_pairs_ / (double)graph_->col.size();
+      std::vector<uint32_t> base(V + 1), edges_into(V, 0), place_start(1, 0u);
+      for (const CSR::Edge dst : graph_->col) edges_into[(size_t)dst]++;
+      uint64_t at = 0;
+      for (size_t v = 0; v < V; ++v) {
+        base[v] = (uint32_t)at;
+        const double walks = per_edge * (double)edges_into[v];
+        uint32_t copies = 1;
+        while (copies < kSmallMapMaxCopies && (double)(copies * kSmallMapWalksPerCounter) < walks) copies <<= 1;
+        at += copies;
+        // places of each of its counters when the pairs are placed as they are emitted: twice
+        // the walks it expects and a few more
+        const uint32_t places = (uint32_t)(2.0 * walks / copies) + kSmallMapSparePlaces;
+        for (uint32_t c = 0; c < copies; ++c) place_start.push_back(place_start.back() + places);
+      }
+      base[V] = (uint32_t)at;
+      small_counters_ = (size_t)at + 1;  // one more, so that every run has an end to read
+      place_start.push_back(place_start.back());  // ... which owns no place
+      small_map_ = small_counters_ < kSmallMapCounters;
+      if (small_map_) {
+        ND_HIP_TRY(hipMalloc(&d_counter_base_, sizeof(uint32_t) * base.size()));
+        ND_HIP_TRY(hipMemcpy(d_counter_base_, base.data(), sizeof(uint32_t) * base.size(), hipMemcpyHostToDevice));
+      }
+      // Placing at emission walks every place at every step: only where the places are not many
+      // times the pairs (ND_SMALL_MAP=1 keeps the two placing launches).
+      small_placed_ = small_map_ && (size_t)place_start.back() <= kSmallMapPlacesPerPair * max_pairs_ &&
+                      small_map_switch_ != 1;
+      if (small_placed_) {
+        placed_spill_first_ = place_start.back();
+        placed_places_ = (size_t)placed_spill_first_ + max_pairs_;  // every pair could spill
+        ND_HIP_TRY(hipMalloc(&d_place_start_, sizeof(uint32_t) * place_start.size()));
+        ND_HIP_TRY(hipMemcpy(d_place_start_, place_start.data(), sizeof(uint32_t) * place_start.size(),
+                             hipMemcpyHostToDevice));
+        for (int b = 0; b < 2; ++b) {
+          ND_HIP_TRY(hipMalloc(&d_placed_keys_[b], sizeof(uint32_t) * placed_places_));
+          ND_HIP_TRY(hipMalloc(&d_placed_slots_[b], sizeof(uint32_t) * placed_places_));
+          ND_HIP_TRY(hipMemset(d_placed_slots_[b], 0, sizeof(uint32_t) * placed_places_));
+          if (state_fits_pair<SampleType>::value) {
+            ND_HIP_TRY(hipMalloc(&d_placed_state_[b], sizeof(uint32_t) * placed_places_));
+            ND_HIP_TRY(hipMemset(d_placed_state_[b], 0, sizeof(uint32_t) * placed_places_));
+          }
+          ND_HIP_TRY(hipMalloc(&d_placed_counts_[b], sizeof(uint32_t) * (small_counters_ + 1)));
+        }
+        placed_dirty_ = true;  // cleared by the first pass that uses them
+      }
+    }
+    if (small_map_) {
+      // counters, their starts inside a chunk, chunk totals
+      const size_t counters = small_counters_, chunks = (counters + kSmallMapChunk - 1) / kSmallMapChunk;
+      ND_HIP_TRY(hipMalloc(&d_small_, sizeof(uint32_t) * (2 * counters + chunks)));
+      ND_HIP_TRY(hipMemset(d_small_, 0, sizeof(uint32_t) * (2 * counters + chunks)));
+      ND_HIP_TRY(hipMalloc(&d_emit_ranks_, sizeof(uint32_t) * max_pairs_));
+    }
+    if (state_travels_) {
+      ND_HIP_TRY(hipMalloc(&d_emit_state_, sizeof(uint32_t) * max_pairs_));
+      ND_HIP_TRY(hipMalloc(&d_aux_a_, sizeof(uint32_t) * max_pairs_));
+      ND_HIP_TRY(hipMalloc(&d_aux_b_, sizeof(uint32_t) * max_pairs_));
+    }
+    ND_HIP_TRY(hipMalloc(&d_meta_, sizeof(RunsMeta) * 2));
+    {
+      RunsMeta fresh[2] = {};
+      fresh[0].stamp = 1;  // the first load-balanced step; every classification hands the next one its stamp
+      ND_HIP_TRY(hipMemcpy(d_meta_, fresh, sizeof(fresh), hipMemcpyHostToDevice));
+    }
+    ND_HIP_TRY(hipMalloc(&d_balance_, sizeof(uint32_t) * kBalanceWords));
+    ND_HIP_TRY(hipMemset(d_balance_, 0, sizeof(uint32_t) * kBalanceWords));
+    ND_HIP_TRY(hipMalloc(&d_chunks_, sizeof(WorkItem) * (size_t)chunk_capacity_));
+    ND_HIP_TRY(hipMalloc(&d_taken_stamp_, sizeof(uint32_t) * ((size_t)invalid_ + 1)));
+    ND_HIP_TRY(hipMemset(d_taken_stamp_, 0, sizeof(uint32_t) * ((size_t)invalid_ + 1)));
+    if (paired_results_) ND_HIP_TRY(hipMalloc(&d_walk_cells_, sizeof(uint32_t) * (size_t)n_samples_));
+    // the copies and fills of this function, on the default stream, before anything of stream_
+    ND_HIP_TRY(hipDeviceSynchronize());
+    return 0;
+  }
+
+  // What only walks that keep their lanes use, of the graph: the vertices they come to and, where they pay, the edges with
+  // the vertices they lead to.
+  int build_walk_tables() {
+    if (walk_tables_ready_) return 0;
+    if (app_uses_weights<App>::value) walk_vertices_ = dgraph_->walk_vertices(stream_);
+    if (app_uses_weights<App>::value && !walk_vertices_) { last_error = "no device memory for the walk vertices"; return -1; }
+    walk_records_ = nullptr;
+    // (not where stepTransits names another vertex than next() returned; nor for an app that looks edges up,
+    // whose tests are what its steps wait for: weighted node2vec over 1.07 GB of edges 24.1 ms, over records 26.4)
+    const size_t edge_bytes = (app_uses_weights<App>::value ? sizeof(EdgeRecord) : sizeof(CSR::Edge)) *
+                              (size_t)graph_->get_n_edges();
+    if (edge_bytes >= kWalkRecordsFromBytes && !App().hasExplicitTransits() && !app_uses_edge_lookup<App>::value)
+      walk_records_ = dgraph_->template walk_edges<walk_record<App>>(stream_);
+    walk_tables_ready_ = true;
+    return 0;
+  }
   ClassCounters* counters_dev() const { return (ClassCounters*)(d_balance_ + kMaxSteps + 2); }
   // Walks write their results in cells of two steps (StepParams::pair_cells) where a step's
   // transit is the previous step's result and the rows are regrouped by assemble_walk_rows.
@@ -2867,9 +2899,26 @@ class Engine : public EngineBase {
     release(d_samples_);
     release(d_samples_init_);
     release(d_final_);
+    release(d_walk_queue_);
+    free_inversion_buffers();
+    walk_tables_ready_ = false;
+    release(d_distinct_counts_);
+    // whatever exists, also after an alloc that failed half way
+    for (hipEvent_t* ev : {&ev_a_, &ev_b_, &ev_begin_, &ev_end_, &ev_fork_, &ev_join_}) {
+      if (*ev) (void)hipEventDestroy(*ev);
+      *ev = nullptr;
+    }
+    if (side_stream_) (void)hipStreamDestroy(side_stream_);
+    side_stream_ = nullptr;
+    if (stream_) (void)hipStreamDestroy(stream_);
+    stream_ = nullptr;
+    allocated_ = false;
+  }
+
+  void free_inversion_buffers() {
+    inversion_ready_ = false;
     release(d_step_out_);
     release(d_walk_cells_);
-    release(d_walk_queue_);
     release(d_keys_a_);
     release(d_vals_a_);
     release(d_keys_b_);
@@ -2887,7 +2936,7 @@ class Engine : public EngineBase {
       release(d_placed_state_[b]);
       release(d_placed_counts_[b]);
     }
-    small_placed_ = false;
+    small_map_ = small_placed_ = false;
     release(d_small_);
     release(d_counter_base_);
     release(d_emit_state_);
@@ -2898,17 +2947,6 @@ class Engine : public EngineBase {
     release(d_chunks_);
     release(d_taken_stamp_);
     release(d_explicit_);
-    release(d_distinct_counts_);
-    // whatever exists, also after an alloc that failed half way
-    for (hipEvent_t* ev : {&ev_a_, &ev_b_, &ev_begin_, &ev_end_, &ev_fork_, &ev_join_}) {
-      if (*ev) (void)hipEventDestroy(*ev);
-      *ev = nullptr;
-    }
-    if (side_stream_) (void)hipStreamDestroy(side_stream_);
-    side_stream_ = nullptr;
-    if (stream_) (void)hipStreamDestroy(stream_);
-    stream_ = nullptr;
-    allocated_ = false;
   }
 
   const char* name_;
@@ -2927,6 +2965,7 @@ class Engine : public EngineBase {
   uint32_t chunk_capacity_ = 0;
   uint32_t row_pitch_ = 0, rows_per_block_ = 0;
   bool paired_results_ = false;
+  bool inversion_ready_ = false, walk_tables_ready_ = false;
   const WalkVertex* walk_vertices_ = nullptr;
   const walk_record<App>* walk_records_ = nullptr;  // dgraph_'s, where they pay
   uint32_t walk_waves_at_once_ = 1, walk_waves_queued_ = 1;  // wavefronts of walk_rows_kernel
@@ -2956,6 +2995,7 @@ class Engine : public EngineBase {
   uint32_t *d_emit_keys_ = nullptr, *d_emit_slots_ = nullptr, *d_emit_state_ = nullptr;  // next step's pairs
   // small maps: the inversion without a sort (small_map_scan, small_map_place)
   bool small_map_ = false, inversion_forced_ = false;
+  int small_map_switch_ = -1;  // ND_SMALL_MAP when the buffers were allocated
   size_t small_counters_ = 0;
   uint32_t* d_counter_base_ = nullptr;  // first counter of every vertex
   uint32_t* d_emit_ranks_ = nullptr;

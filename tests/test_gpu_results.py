@@ -1,5 +1,6 @@
 """Results on their way to the host: the packed transfer against the words it starts from, and the arrays
 a caller is given, which stay what they were when later results are fetched."""
+import ctypes
 import os
 import subprocess
 
@@ -103,3 +104,47 @@ def test_rows_that_leave_before_the_pass_is_over(oracle, n):
     s.do_transit_parallel()
     s.close()
     assert all(np.array_equal(r, want) for r in rows)
+
+
+def device_memory_left():
+    hip = ctypes.CDLL("libamdhip64.so")
+    left, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert hip.hipMemGetInfo(ctypes.byref(left), ctypes.byref(total)) == 0
+    return left.value
+
+
+def test_walks_take_device_memory_for_what_they_run():
+    """Neither the buffers of an inversion nor the edges as walk records are there before a pass uses them."""
+    n, walk = 400009, 100
+    src = np.arange(n)
+    g = nd.Graph.from_edges(np.repeat(src, 22), (np.repeat(src, 22) * 31 + np.tile(np.arange(22), n)) % n, n_vertices=n)
+    rows, pairs, records = 4 * n * walk, 4 * n, 16 * g.n_edges
+    assert 4 * g.n_edges > 32 << 20  # enough for the records to pay
+    before = device_memory_left()
+    step = lambda name: print(name, before - device_memory_left(), flush=True)
+    s = nd.Sampler("UniformRandomWalk", g, seed=42)
+    try:
+        step("allocated")
+        s.set_inversion_period(1)
+        s.do_transit_parallel()
+        step("inverted")
+        want = s.final_samples()
+        inverted = device_memory_left()
+        assert before - inverted >= 2 * rows
+        s.set_inversion_period(0)
+        s.do_transit_parallel()
+        step("with records")
+        assert inverted - device_memory_left() >= records  # no sampler that only inverts has them
+        assert np.array_equal(s.final_samples(), want)
+        s.close()
+        s = nd.Sampler("UniformRandomWalk", g, seed=42)
+        s.do_transit_parallel()
+        step("not inverted")
+        # the graph, the rows, the records: and neither the results by step nor pairs to sort (allocations round up)
+        assert before - device_memory_left() <= 8 * g.n_edges + 8 * n + rows + records + 8 * pairs + (64 << 20)
+        assert np.array_equal(s.final_samples(), want)
+        s.set_inversion_period(1)
+        s.do_transit_parallel()
+        assert np.array_equal(s.final_samples(), want)
+    finally:
+        s.close()
