@@ -2114,16 +2114,31 @@ class Engine : public EngineBase {
   }
 
   // Launches a pass of walks is split into, where its rows are to leave early.  Every one of them ends with its longest
-  // walks alone on the device (0.1 ms of uniform ones, 0.45 of weighted node2vec over R-MAT 22), and the first row
-  // leaves at the end of the first.  Pass with its rows, in 1 / 2 / 4 / 6 of them (ms): PPR over 262 K vertices
-  // 1.83 / 1.37 / 1.48 / 1.96, DeepWalk over 100 K 0.93 / 1.12 / -, over 500 K 4.1 / 3.2 / 2.8 / 3.0, 100 a vertex over
-  // 10 K 5.3 / 5.1 / 4.8 / 4.6, weighted node2vec over 700 K 7.2 / 6.2 / 5.4 / 6.6, R-MAT 22 38.1 / 32.7 / 30.2 / 30.8.
-  // Walks with states in memory wait for those, not for each other: MultiRW over 100 K vertices 1.89 / 1.56 / 1.66.
+  // walks alone on the device, and the first row leaves at the end of the first; what there is to hide is the rows' time on
+  // the bus, 4.3 ms for a million walks of 100 steps.  An end costs 0.07 ms of uniform walks, 0.15-0.25 of DeepWalk and PPR,
+  // 0.6 of second-order walks (a state that travels; the most tries a step).  Passes with their rows, ms, by launches, over
+  // Chung-Lu graphs unless another is named:
+  //    no state                   1     2     3     4     6     8     a state that travels     1     2     3     4     6
+  //    uniform         100 K   0.68  0.64  0.66  0.77  0.94  1.13    weighted n2v  200 K    1.94  2.12  2.62  3.18  4.26
+  //                    200 K   1.20  1.12  1.11  1.09  1.25  1.49                  300 K    2.94  2.63  3.12  3.75  4.82
+  //                    400 K   2.35  2.22  2.05  1.99  2.06  2.07                  350 K    3.57  2.90  3.33  3.95  5.14
+  //                    800 K   4.70  4.71  4.57  4.43  4.27  4.13                  500 K    4.98  3.98  3.99  4.51  5.84
+  //                    1.2 M   7.04  6.94  7.07  6.98  6.71  6.50                  700 K    6.78  6.06  5.27  5.34  6.60
+  //    PPR             262 K   1.53  1.43  1.36  1.47  1.92  2.38                    1 M    9.54  8.58  8.39  7.45  7.89
+  //                    600 K   3.39  3.10  2.95  2.91  2.87  3.06                  1.5 M    14.5  12.3  12.1  11.8  10.9
+  //                    800 K   4.42  4.21  3.90  3.78  3.72  3.71                    3 M    28.8  24.1  23.0  22.3  23.5
+  //    DeepWalk        200 K   1.45  1.29  1.41  1.60  2.00  2.45             R-MAT 22      38.4  32.2  30.8  30.2  30.9
+  //                    400 K   3.02  2.40  2.27  2.30  2.63  3.04    a state in memory
+  //                    700 K   4.86  4.91  4.05  3.73  3.93  4.25    MultiRW        50 K    0.89  0.90  1.02  1.16  1.46
+  //                    800 K   5.54  5.83  4.79  4.36  4.38  4.60                   90 K    1.58  1.36  1.44  1.61  1.84
+  //                    1.2 M   8.48  7.65  8.59  7.40  6.44  6.42                  125 K    2.25  1.79  1.81  1.94  2.24
+  //             R-MAT 22       26.4  23.9  23.2  22.4  22.3  22.1                  300 K    5.42  4.97  4.38  4.07  4.30
   uint32_t walk_ranges() const {
     if (!rows_ahead || profiling || wants_launch_graph()) return 1;
     if (sizeof(VertexID_t) * (size_t)n_samples_ * (size_t)final_sample_size() <= kDirectResultBytes) return 1;
-    constexpr int64_t least = std::is_empty<SampleType>::value || state_fits_pair<SampleType>::value ? 96 << 10 : 48 << 10;
-    if (n_samples_ >= 10 * least) return kMostWalkRanges;
+    constexpr bool stateless = std::is_empty<SampleType>::value;
+    constexpr int64_t least = stateless ? 96 << 10 : state_fits_pair<SampleType>::value ? 160 << 10 : 40 << 10;
+    if (stateless && n_samples_ >= 8 * least) return kMostWalkRanges;
     return (uint32_t)std::max<int64_t>(1, std::min<int64_t>(4, n_samples_ / least));
   }
 
