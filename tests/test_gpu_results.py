@@ -120,6 +120,9 @@ def test_walks_take_device_memory_for_what_they_run():
     g = nd.Graph.from_edges(np.repeat(src, 22), (np.repeat(src, 22) * 31 + np.tile(np.arange(22), n)) % n, n_vertices=n)
     rows, pairs, records = 4 * n * walk, 4 * n, 16 * g.n_edges
     assert 4 * g.n_edges > 32 << 20  # enough for the records to pay
+    # What is left counts whole pages, and the runtime keeps blocks that earlier samplers of the process gave back: small
+    # allocations may come from those.  32 MB is several times all small ones of a sampler, a fifth of any that matters here.
+    held = 32 << 20
     before = device_memory_left()
     step = lambda name: print(name, before - device_memory_left(), flush=True)
     s = nd.Sampler("UniformRandomWalk", g, seed=42)
@@ -130,11 +133,11 @@ def test_walks_take_device_memory_for_what_they_run():
         step("inverted")
         want = s.final_samples()
         inverted = device_memory_left()
-        assert before - inverted >= 2 * rows
+        assert before - inverted >= 2 * rows - held
         s.set_inversion_period(0)
         s.do_transit_parallel()
         step("with records")
-        assert inverted - device_memory_left() >= records  # no sampler that only inverts has them
+        assert inverted - device_memory_left() >= records - held  # no sampler that only inverts has them
         assert np.array_equal(s.final_samples(), want)
         s.close()
         s = nd.Sampler("UniformRandomWalk", g, seed=42)
@@ -146,5 +149,46 @@ def test_walks_take_device_memory_for_what_they_run():
         s.set_inversion_period(1)
         s.do_transit_parallel()
         assert np.array_equal(s.final_samples(), want)
+    finally:
+        s.close()
+
+
+# the forms a walk has: its state in registers, in memory (and transits of its own), the edges as walk records
+@pytest.mark.parametrize("app,kind,n,mean_degree", [
+    ("WeightedNode2Vec8", "WEIGHTED_NODE2VEC", 360007, 3),
+    ("MultiRW4x6", "MULTIRW", 300007, 3),
+    ("UniformRandomWalk8", "UNIFORM_WALK", 600011, 15),
+    ("DeepWalkPerVertex", "DEEPWALK", 500009, 9),
+])
+@pytest.mark.parametrize("mode", ["transit", "sample"])
+def test_rows_of_every_kind_of_walk_leave_before_the_pass_is_over(oracle, app, kind, n, mean_degree, mode):
+    g = graphs.random_graph(n=n, mean_degree=mean_degree, seed=n, isolated_every=5)
+    og = graphs.oracle_view(g)
+    s = nd.Sampler(app, g, seed=42)
+    try:
+        states_of = lambda: s.sample_states().view(np.int32).reshape(s.num_samples, -1)
+        alive = slice(None)
+        if kind == "MULTIRW":
+            want, walkers, last, _ = oracle.sample_multirw(og, 42, states_of()[:, :-1], s.steps)
+            want_states = np.concatenate([walkers, last[:, None]], axis=1)
+        else:
+            d = oracle.app_desc(getattr(oracle, kind), s.steps, [s.step_size(k) for k in range(s.steps)], p=2.0, q=0.5)
+            want, want_states = oracle.sample_individual(og, d, 42, s.initial_contents)
+            if kind == "WEIGHTED_NODE2VEC":
+                alive = want_states != -1
+                want_states = want_states.reshape(s.num_samples, -1)
+            else:
+                want_states = None
+        run = s.do_transit_parallel if mode == "transit" else s.do_sample_parallel
+        for turn, states_first in enumerate([False, False, True, True]):
+            print("app", app, "mode", mode, "turn", turn, flush=True)
+            run()
+            # from the second pass on: one launch for every part of the rows that leaves by itself
+            assert (s.phase_times()["flat_launches"] > 1) == (turn > 0)
+            if states_first and want_states is not None:
+                assert np.array_equal(states_of()[alive], want_states[alive])
+            assert np.array_equal(s.final_samples(), want)
+            if want_states is not None:
+                assert np.array_equal(states_of()[alive], want_states[alive])
     finally:
         s.close()
