@@ -1152,7 +1152,7 @@ class LayerEngine : public EngineBase {
     h_sizes_.resize((size_t)n_samples_);
     chunk_entries_ = kLayerChunkEntries;
     bitmap_chunk_entries_ = kBitmapChunkEntries;
-    progress_ = getenv("ND_PROGRESS") != nullptr;  // long layers report on stderr every 16 chunks
+    progress_ = getenv("ND_PROGRESS") != nullptr;  // a line on stderr per chunk
     if (const char* env = getenv("ND_LAYER_CHUNK_ENTRIES")) {  // smaller chunks, e.g. to exercise chunking
       const long long v = atoll(env);
       if (v > 0) chunk_entries_ = bitmap_chunk_entries_ = (uint64_t)v;
@@ -1253,8 +1253,12 @@ class LayerEngine : public EngineBase {
       constexpr int form = apps::neighborhood_form_of<App>::value;
       if (form != apps::kConcatenated && bitmap_chunk_entries_ == kBitmapChunkEntries) {
         // chunks of as many samples as there is memory for bitmaps of: nothing the host has to know first
-        for (uint32_t s0 = 0; s0 < S; s0 += bitmap_chunk_samples_, chunks_run_++)
-          if (run_chunk(step, all, s0, std::min(S, s0 + bitmap_chunk_samples_), 0) != 0) return -1;
+        for (uint32_t s0 = 0, s1; s0 < S; s0 = s1) {
+          s1 = std::min(S, s0 + bitmap_chunk_samples_);
+          if (run_chunk(step, all, s0, s1, 0) != 0) return -1;
+          chunks_run_++;
+          if (progress_ && report_progress(step, s1, /*on_device=*/true) != 0) return -1;
+        }
         continue;
       }
       // size of every sample's collective neighbourhood, then chunks of samples that fit the budget
@@ -1276,12 +1280,7 @@ class LayerEngine : public EngineBase {
         if (run_chunk(step, all, s0, s1, total) != 0) return -1;
         neighborhood_total_ += total;
         chunks_run_++;
-        if (progress_ && chunks_run_ % 16 == 0) {
-          ND_HIP_TRY(hipStreamSynchronize(stream_));
-          fprintf(stderr, "[nextdoor] layer %d: samples %u of %u done, %llu neighbourhood entries so far\n", step, s1,
-                  S, (unsigned long long)neighborhood_total_);
-          fflush(stderr);
-        }
+        if (progress_ && report_progress(step, s1, /*on_device=*/false) != 0) return -1;
         s0 = s1;
       }
     }
@@ -1497,6 +1496,22 @@ class LayerEngine : public EngineBase {
 
   static constexpr uint32_t kDrawBlocks = 4096;
   static constexpr const char* kTooLong = "collective neighbourhood of one sample has 2^31 or more entries";
+
+  // A line on stderr when a chunk of a layer is done.  on_device: the sizes of its neighbourhoods were not needed here, and are
+  // there, layer after layer.
+  int report_progress(int step, uint32_t samples_done, bool on_device) {
+    ND_HIP_TRY(hipStreamSynchronize(stream_));
+    uint64_t entries = neighborhood_total_;
+    if (on_device) {
+      std::vector<uint32_t> sizes((size_t)n_samples_ * step + samples_done);
+      ND_HIP_TRY(hipMemcpy(sizes.data(), d_layer_counts_, sizeof(uint32_t) * sizes.size(), hipMemcpyDeviceToHost));
+      for (uint32_t n : sizes) entries += n;
+    }
+    fprintf(stderr, "[nextdoor] layer %d: samples %u of %u done, %llu neighbourhood entries so far\n", step, samples_done,
+            (uint32_t)n_samples_, (unsigned long long)entries);
+    fflush(stderr);
+    return 0;
+  }
 
   // events around the neighbourhood kernel when profiling is on
   void tick() {

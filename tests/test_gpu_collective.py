@@ -1,6 +1,8 @@
 """GPU parity of the layer-wise (CollectiveNeighborhood) engine against the CPU oracle:
 collective-neighbourhood build, the reference's FastGCN/LADIES app (vertices, recorded
 adjacency-matrix entries, the reference's validator) and the importance sampler."""
+import re
+
 import numpy as np
 import pytest
 
@@ -199,3 +201,19 @@ def test_chunked_processing_gives_the_same_samples(oracle, app, kind_name, monke
     assert s.counter(2) > 3 * s.steps
     assert np.array_equal(s.final_samples(), whole)
     s.close()
+
+
+@pytest.mark.parametrize("app", ["FastGCNImportance2x8", "LADIESImportance2x8", "LayerLiteral2x8"])
+def test_progress_is_reported_for_every_layer(app, monkeypatch, capfd):
+    monkeypatch.setenv("ND_PROGRESS", "1")
+    s = nd.Sampler(app, graphs.random_graph(n=400, mean_degree=8, seed=3, hub=2), seed=SEED)
+    try:
+        for _ in range(2):
+            capfd.readouterr()
+            s.do_transit_parallel()
+            lines = re.findall(r"\[nextdoor\] layer (\d+): samples (\d+) of (\d+) done, (\d+) ", capfd.readouterr().err)
+            assert [int(l[0]) for l in lines] == list(range(s.steps))  # a chunk a layer
+            assert all(int(l[1]) == int(l[2]) == s.num_samples for l in lines)
+            assert int(lines[-1][3]) == s.counter(0) > int(lines[0][3]) > 0
+    finally:
+        s.close()
