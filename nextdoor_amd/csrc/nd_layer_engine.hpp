@@ -587,13 +587,12 @@ __global__ __launch_bounds__(kBinThreads, 8) __attribute__((amdgpu_num_vgpr(56))
 constexpr uint32_t kRankedEntries = 8192;
 constexpr uint32_t kRankedThreads = 1024;
 
-// A wavefront per sample: sizes[s] = entries of its neighbourhood, parallel edges and all (saturated).
+// A wavefront per sample: sizes[s] = entries of its neighbourhood, parallel edges and all, merged_sizes[s] = without.
 __global__ __launch_bounds__(kSortOutThreads) void sort_out_ranked(CSRPartition csr, MergedEdges merged, TransitView tv,
                                                                    uint32_t n_samples, int32_t invalid,
                                                                    uint32_t* __restrict__ sizes,
                                                                    uint32_t* __restrict__ merged_sizes,
-                                                                   uint32_t* __restrict__ n_marked,
-                                                                   uint32_t* __restrict__ marked,
+                                                                   uint32_t* n_marked, uint32_t* __restrict__ marked,
                                                                    uint32_t* __restrict__ too_long) {
   __shared__ uint32_t s_taken, s_base;
   const uint32_t lane = threadIdx.x & 63u;
@@ -611,9 +610,10 @@ __global__ __launch_bounds__(kSortOutThreads) void sort_out_ranked(CSRPartition 
   pairs = __shfl(wave_inclusive_scan_u64(pairs), 63, kWave);
   uint32_t at = 0;
   if (lane == 0 && s < n_samples) {
-    sizes[s] = both > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)both;
-    merged_sizes[s] = pairs > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)pairs;
-    if (both >= (1ull << 31)) *too_long = 1;
+    const uint32_t size = entries_or_refused(both, n_marked + 1, too_long);
+    if (size == 0) pairs = 0;
+    sizes[s] = size;
+    merged_sizes[s] = (uint32_t)pairs;
     if (pairs > kRankedEntries) at = atomicAdd(&s_taken, 1u);
   }
   __syncthreads();
@@ -1202,7 +1202,7 @@ class LayerEngine : public EngineBase {
       ND_HIP_TRY(hipMalloc(&d_layer_counts_, sizeof(uint32_t) * 2 * (size_t)n_samples_ * n_steps));
       ND_HIP_TRY(hipHostMalloc((void**)&h_too_long_, 3 * sizeof(uint32_t), hipHostMallocDefault));
       *h_too_long_ = 0;
-      ND_HIP_TRY(hipMalloc(&marked_.count, sizeof(uint32_t)));
+      ND_HIP_TRY(hipMalloc(&marked_.count, 2 * sizeof(uint32_t)));
       ND_HIP_TRY(hipMalloc(&marked_.sample, sizeof(uint32_t) * (size_t)n_samples_));
     }
     if (apps::neighborhood_form_of<App>::value == apps::kDistinctByDegreeSquared) {
@@ -1231,7 +1231,10 @@ class LayerEngine : public EngineBase {
     distinct_total_ = 0;
     chunks_run_ = 0;
     counted_ = true;
-    if (h_too_long_) *h_too_long_ = 0;
+    if (h_too_long_) {
+      *h_too_long_ = 0;
+      ND_HIP_TRY(hipMemsetAsync(marked_.count + 1, 0, sizeof(uint32_t), stream_));
+    }
     if (!std::is_empty<SampleType>::value) {
       ND_HIP_TRY(hipMemcpyAsync(d_samples_, d_samples_init_, sizeof(SampleType) * (size_t)n_samples_,
                                 hipMemcpyDeviceToDevice, stream_));

@@ -277,14 +277,26 @@ constexpr uint32_t kSortedEntries = 4096;
 // A layer drawn with replacement by degree^2 repeats its hubs (34 distinct transits of 64 over R-MAT 20), and a vertex
 // marks the same bits however often it is there.
 struct MarkedSamples {
-  uint32_t* count;
+  uint32_t* count;      // and, next to it, whether a neighbourhood of this pass was too long (entries_or_refused)
   uint32_t* sample;     // [n]
   int32_t* transits;    // [n][stride]
   uint2* transit_count; // [n]: hubs, others
   uint32_t stride;
 };
 
-// A wavefront per sample: sizes[s] = entries of its neighbourhood (saturated), and which way it goes.  One atomic for the
+// What a sample's neighbourhood of `entries` counts for.  One of 2^31 entries or more is refused, and the pass with it: the host
+// hears of it at the end (*too_long, host memory), and until then nobody works on it - it counts as empty, and so does
+// every neighbourhood of the layers that follow (*refused).
+__device__ __forceinline__ uint32_t entries_or_refused(uint64_t entries, uint32_t* refused, uint32_t* too_long) {
+  const bool before = __hip_atomic_load(refused, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+  if (entries >= (1ull << 31)) {
+    *too_long = 1;
+    __hip_atomic_store(refused, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  return before || entries >= (1ull << 31) ? 0u : (uint32_t)entries;
+}
+
+// A wavefront per sample: sizes[s] = entries of its neighbourhood, and which way it goes.  One atomic for the
 // 16 samples of a workgroup: atomics on one address follow each other at 10 ns (4096 of them 41 us).
 constexpr uint32_t kSortOutThreads = 1024;
 __global__ __launch_bounds__(kSortOutThreads) void sort_out_samples(CSRPartition csr, TransitView tv, uint32_t n_samples,
@@ -307,17 +319,18 @@ __global__ __launch_bounds__(kSortOutThreads) void sort_out_samples(CSRPartition
     const uint32_t lo = __shfl_xor((uint32_t)sum, d, kWave), hi = __shfl_xor((uint32_t)(sum >> 32), d, kWave);
     sum += ((uint64_t)hi << 32) | lo;
   }
+  // one lane asks, since the answer may change meanwhile
+  const uint32_t size = (uint32_t)__shfl((int)(lane == 0 ? entries_or_refused(sum, marked.count + 1, too_long) : 0u), 0, kWave);
   uint32_t at = 0;
   if (lane == 0 && s < n_samples) {
-    sizes[s] = sum > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)sum;
+    sizes[s] = size;
     distinct[s] = 0;
-    if (sum >= (1ull << 31)) *too_long = 1;
-    if (sum > kSortedEntries) at = atomicAdd(&s_taken, 1u);
+    if (size > kSortedEntries) at = atomicAdd(&s_taken, 1u);
   }
   __syncthreads();
   if (threadIdx.x == 0 && s_taken) s_base = atomicAdd(marked.count, s_taken);
   __syncthreads();
-  if (sum <= kSortedEntries) return;  // the same for the whole wavefront
+  if (size <= kSortedEntries) return;  // the same for the whole wavefront
   at = s_base + __shfl(at, 0, kWave);
   if (lane == 0) marked.sample[at] = s;
   int32_t* mine = marked.transits + (size_t)at * marked.stride;

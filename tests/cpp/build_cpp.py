@@ -22,6 +22,8 @@ ROWS_AHEAD_PROBE_SRC = os.path.join(HERE, "rows_ahead_probe.hip")
 ROWS_AHEAD_PROBE = os.path.join(HERE, "rows_ahead_probe")
 HOST_RESULTS_PROBE_SRC = os.path.join(HERE, "host_results_probe.hip")
 HOST_RESULTS_PROBE = os.path.join(HERE, "host_results_probe")
+LONG_NEIGHBOURHOOD_PROBE_SRC = os.path.join(HERE, "long_neighbourhood_probe.hip")
+LONG_NEIGHBOURHOOD_PROBE = os.path.join(HERE, "long_neighbourhood_probe")
 USER_APPS_SRC = os.path.join(HERE, "user_apps.hip")
 USER_APPS_LIB = os.path.join(HERE, "libuser_apps.so")
 
@@ -78,6 +80,11 @@ def build_host_results_probe():
     return HOST_RESULTS_PROBE
 
 
+def build_long_neighbourhood_probe():
+    _run(_hipcc_flags() + ["-I", INCLUDE, LONG_NEIGHBOURHOOD_PROBE_SRC, "-o", LONG_NEIGHBOURHOOD_PROBE, "-lpthread"])
+    return LONG_NEIGHBOURHOOD_PROBE
+
+
 def build_user_apps():
     _run(_hipcc_flags() + ["-shared", USER_APPS_SRC, "-o", USER_APPS_LIB] + _link_flags())
     return USER_APPS_LIB
@@ -85,7 +92,7 @@ def build_user_apps():
 
 def build_all():
     return [build_host_probe(), build_template_probe(), build_result_probe(), build_rows_ahead_probe(),
-            build_host_results_probe(), build_user_apps()]
+            build_host_results_probe(), build_long_neighbourhood_probe(), build_user_apps()]
 
 
 if __name__ == "__main__":

@@ -1,13 +1,16 @@
 """GPU parity of the layer-wise (CollectiveNeighborhood) engine against the CPU oracle:
 collective-neighbourhood build, the reference's FastGCN/LADIES app (vertices, recorded
 adjacency-matrix entries, the reference's validator) and the importance sampler."""
+import os
 import re
+import subprocess
 
 import numpy as np
 import pytest
 
 import nextdoor_amd as nd
 from tests import graphs
+from tests.cpp.build_cpp import LONG_NEIGHBOURHOOD_PROBE
 
 pytestmark = pytest.mark.gpu
 
@@ -217,3 +220,11 @@ def test_progress_is_reported_for_every_layer(app, monkeypatch, capfd):
             assert int(lines[-1][3]) == s.counter(0) > int(lines[0][3]) > 0
     finally:
         s.close()
+
+
+def test_neighbourhoods_that_are_too_long_are_worked_on_by_nobody():
+    """A neighbourhood of 2^31 entries is refused before its layer, as far as any kernel is concerned, and the layers after
+    it work on none; the pass reports it when it is over."""
+    assert os.path.exists(LONG_NEIGHBOURHOOD_PROBE), "tests/cpp/long_neighbourhood_probe is built by __graft_entry__.build()"
+    out = subprocess.run([LONG_NEIGHBOURHOOD_PROBE], capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0 and out.stdout.endswith("all as they should be\n"), out.stdout[-300:] + out.stderr[-300:]
