@@ -77,7 +77,10 @@ int nd_sampler_set_graph(nd_sampler* s, const nd_graph* g);
 /* allocNextDoorDataOnGPU(csr, data), src/nextdoor.cu:1931-2086.  seed keys the Philox
  * stream that replaces init_curand_states (src/nextdoor.cu:1838-1843). */
 int nd_sampler_alloc(nd_sampler* s, uint64_t seed);
-/* doTransitParallelSampling(csr, data, enableLoadBalancing), src/nextdoor.cu:2191-3006. */
+/* doTransitParallelSampling(csr, data, enableLoadBalancing), src/nextdoor.cu:2191-3006.  Walks are only
+ * brought into transit order, and their transits only balanced and counted (nd_sampler_counter), where they are
+ * inverted: nd_sampler_set_inversion_period(s, 1).  On a new sampler they keep their lanes instead, with or
+ * without load balancing, and the counters of the kernel classes stay 0. */
 int nd_sampler_do_transit_parallel(nd_sampler* s, int enable_load_balancing);
 /* doSampleParallelSampling(csr, data), src/nextdoor.cu:3009-3209: the reference's baseline
  * mode.  The (sample -> transit) map is never sorted by transit: before a step the pairs whose
@@ -96,7 +99,7 @@ int nd_sampler_do_sample_parallel(nd_sampler* s);
 int nd_sampler_set_inversion_period(nd_sampler* s, int period);
 /* getFinalSamples(data), src/nextdoor.cu:3211-3237: copies device -> host and returns the
  * host array (num_samples * final_sample_size int32, INVALID = n_vertices).  More than a few
- * megabytes cross the bus packed and are unpacked by up to eight host threads on the way. */
+ * megabytes cross the bus packed and are unpacked by the caller and up to eleven host threads on the way. */
 int nd_sampler_get_final_samples(nd_sampler* s, const int32_t** data, int64_t* length);
 /* getFinalSampleSize<App>(), src/nextdoor.cu:1913-1929. */
 int nd_sampler_final_sample_size(const nd_sampler* s);

@@ -223,6 +223,9 @@ class Sampler:
         return np.ctypeslib.as_array(p, shape=(n.value,)).copy()
 
     def do_transit_parallel(self, load_balancing=True):
+        """One pass.  Walks are ordered by transit, balanced and counted per kernel class only where they are
+        inverted (``set_inversion_period(1)``); on a new sampler they keep their lanes, and ``load_balancing``
+        changes nothing.  Other apps: ``load_balancing`` chooses the kernel class of every transit."""
         check(lib().nd_sampler_do_transit_parallel(self._h, int(load_balancing)))
 
     def do_sample_parallel(self):

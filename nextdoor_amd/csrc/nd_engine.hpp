@@ -2325,9 +2325,6 @@ class Engine : public EngineBase {
         // inversion: sort (transit, slot) by transit.  Walks sort the pairs the previous
         // step emitted (only those still alive); other apps sort the previous step's
         // output array, whose index is the slot.
-        // Walks that invert only now and then gain nothing from the transit order (few of them
-        // share a transit, and the order is stale one step later): they only drop the walks
-        // that have ended, keeping slot order, in which the writes of a step's results coalesce.
         if (placed) {
           // small map, placed by the previous step's kernel: every place is a lane
           const int from = (step - 1) & 1;

@@ -17,16 +17,16 @@
 //    nullptr, nextdoor.cu:1441-1446).  Here offsets are an exclusive scan over samples
 //    (deterministic), the buffers are grown once and reused, and next() receives the
 //    neighbourhood in the form the app declares (nd::apps::NeighborhoodForm).
-//  * For kDistinctByDegreeSquared the concatenation is never stored, nor a list of its distinct
-//    vertices: every entry marks its vertex in a per-sample bitmap, built stretch by stretch
-//    in LDS; degree^2 of the marked vertices is summed over groups and parts of the bitmap,
-//    and a draw searches those sums.
-//  * For kRankedByLadiesImportance each entry also carries (weight * (1 / rowsum(transit)))^2;
-//    the terms of a vertex are summed as 2^53 fixed-point integers (in LDS) into one sum per
-//    (sample, vertex), its Efraimidis-Spirakis key is formed from the sum as it leaves LDS (the
-//    only thing stored per sample and vertex), a radix select keeps
-//    the few entries that can be among a sample's first picks, and stable sorts order those by
-//    descending key.
+//  * The importance forms never store the concatenation.  kDistinctByDegreeSquared (nd_union_sums.hpp): small
+//    neighbourhoods are sorted in LDS; of the others every part of the vertex range becomes bits, OR-ed from the
+//    hubs' ready-made pieces and marked entry by entry, whose degree^2 the matrix cores sum by group; a draw searches
+//    the sums.
+//  * kRankedByLadiesImportance: each entry carries (weight * (1 / rowsum(transit)))^2 as a 2^53 fixed-point integer,
+//    worked out once per graph with parallel edges merged.  Small neighbourhoods are summed, keyed
+//    (Efraimidis-Spirakis) and sorted in LDS by one workgroup.  Of the others the terms of a vertex are summed in LDS
+//    stretch by stretch, its key is formed from the sum as it leaves LDS (the only thing stored per sample and
+//    vertex), a radix select keeps the few entries that can be among the sample's first picks, and stable sorts
+//    order those by descending key.
 //  * Samples are processed in chunks whose concatenated neighbourhoods fit a fixed budget
 //    of entries, so a layer whose frontier sits on hubs cannot outgrow memory.
 //  * Random numbers: Philox keyed by the output slot s * stepSize(k) + nbr and the layer.
