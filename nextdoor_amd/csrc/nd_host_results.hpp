@@ -60,7 +60,7 @@ class HostWorkers {
     static HostWorkers* workers = [] {
       HostWorkers* w = new HostWorkers;
       // what was registered last is done first: the runtime, which was there before any work for these threads, is still whole
-      (void)std::atexit([] { get().rest(); });
+      (void)std::atexit([] { (void)get().rest(); });
       return w;
     }();
     return *workers;
@@ -93,6 +93,14 @@ class HostWorkers {
     ended_.wait(lock, [&] { return job.running == 0; });
   }
 
+  // For the end of the process: no thread starts on anything any more; returns whether none is at work.  What they work on
+  // ends by itself, within tens of milliseconds; if something else is amiss the process still ends.
+  bool rest() {
+    std::unique_lock<std::mutex> lock(mutex_);
+    resting_ = true;
+    return ended_.wait_for(lock, std::chrono::seconds(10), [&] { return at_work_ == 0; });
+  }
+
   // body() on this thread and on up to `helpers` others.
   void run(unsigned helpers, const std::function<void()>& body) {
     Job job;
@@ -104,14 +112,6 @@ class HostWorkers {
 
  private:
   HostWorkers() = default;
-
-  // No thread starts on anything any more; returns when none is at work.  What they work on ends by itself, within
-  // tens of milliseconds; if something else is amiss the process still ends.
-  void rest() {
-    std::unique_lock<std::mutex> lock(mutex_);
-    resting_ = true;
-    ended_.wait_for(lock, std::chrono::seconds(10), [&] { return at_work_ == 0; });
-  }
 
   // besides the thread that calls
   static unsigned limit() {
@@ -572,10 +572,24 @@ inline hipError_t device_of(hipStream_t stream, int* device) {
 
 // The stream results cross the bus on while something else is computed: one per device (the current one) and process, on
 // a hardware queue of its own, which a stream with a mask of compute units (here: all) gets.  (Ordinary streams share
-// four; where the computation's lands on the same one, nothing overlaps.)
+// four; where the computation's lands on the same one, nothing overlaps.)  They are destroyed when the process ends, while
+// the runtime and whatever watches it are still there: left to the runtime, their queues outlive a profiler's
+// bookkeeping of them, and a profiled process ended in a segmentation fault.
+inline std::vector<hipStream_t>& transfer_streams() {
+  static std::vector<hipStream_t>* streams = [] {
+    auto* made = new std::vector<hipStream_t>;
+    (void)std::atexit([] {
+      if (!HostWorkers::get().rest()) return;  // somebody may still use them
+      for (hipStream_t& s : transfer_streams())
+        if (s) (void)hipStreamDestroy(s), s = nullptr;
+    });
+    return made;
+  }();
+  return *streams;
+}
 inline hipStream_t transfer_stream(int device) {
   static std::mutex mutex;
-  static std::vector<hipStream_t>* streams = new std::vector<hipStream_t>;
+  std::vector<hipStream_t>* streams = &transfer_streams();
   std::lock_guard<std::mutex> lock(mutex);
   if (streams->size() <= (size_t)device) streams->resize((size_t)device + 1, nullptr);
   hipStream_t& stream = (*streams)[(size_t)device];
