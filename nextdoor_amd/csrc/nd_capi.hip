@@ -383,7 +383,13 @@ int nd_sampler_alloc(nd_sampler* s, uint64_t seed) {
   return guarded([&]() -> int {
     if (!s) return fail("null sampler");
     const int rc = s->engine->alloc(seed);
-    return rc == 0 ? 0 : fail(s->engine->last_error, rc);
+    if (rc != 0) return fail(s->engine->last_error, rc);
+    // small results' page-locked memory with the other buffers (0.5 ms, several passes' worth); if there is none, the
+    // first fetch says so
+    const uint64_t words = (uint64_t)s->engine->num_samples() * (uint64_t)s->engine->final_sample_size();
+    if (words * sizeof(int32_t) <= nd::kDirectResultBytes && s->engine->result_stream->reserve() != hipSuccess)
+      (void)hipGetLastError();
+    return 0;
   });
 }
 

@@ -623,6 +623,15 @@ class ResultStream {
     hipEvent_t event;
   };
 
+  // Takes the page-locked memory that copy() needs, on the current device, ahead of the first.
+  hipError_t reserve() {
+    hipError_t e = finish();
+    if (e == hipSuccess) e = come_to_device_of(nullptr);
+    if (e == hipSuccess) e = make_ring(kDirectResultBytes);
+    if (e == hipSuccess) memset(ring_, 0, kDirectResultBytes);  // its pages are mapped when they are first touched: 0.8 ms
+    return e;
+  }
+
   // bytes at src to dst as they are, in stream order, complete on return.  For few of them, and for what is not words.
   hipError_t copy(const void* src, size_t bytes, void* dst, hipStream_t stream) {
     hipError_t e = finish();  // an earlier one that nobody waited for
