@@ -25,6 +25,7 @@
 #include <stdlib.h>
 #include <string.h>
 #include <sys/mman.h>
+#include <unistd.h>
 #if defined(__x86_64__)
 #include <immintrin.h>
 #endif
@@ -94,8 +95,10 @@ class HostWorkers {
   }
 
   // For the end of the process: no thread starts on anything any more; returns whether none is at work.  What they work on
-  // ends by itself, within tens of milliseconds; if something else is amiss the process still ends.
+  // ends by itself, within tens of milliseconds; if something else is amiss the process still ends.  (A forked child
+  // has none of the threads, but a copy of what they were at, and of who held the lock.)
   bool rest() {
+    if (getpid() != process_) return false;
     std::unique_lock<std::mutex> lock(mutex_);
     resting_ = true;
     return ended_.wait_for(lock, std::chrono::seconds(10), [&] { return at_work_ == 0; });
@@ -155,6 +158,7 @@ class HostWorkers {
   std::mutex mutex_;
   std::condition_variable wake_, ended_;
   std::list<Job*> jobs_;
+  const pid_t process_ = getpid();
   unsigned threads_ = 0, at_work_ = 0;
   bool resting_ = false;
 };

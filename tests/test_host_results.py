@@ -50,3 +50,7 @@ def test_the_control_groups_share_is_counted(probe, tmp_path, files, groups, cpu
 
 def test_two_arrays_at_most_wait_for_their_next_use(probe):
     assert [int(x) for x in probe("pool").split()] == [2 * (16 << 20), 0, 1000, 0]
+
+
+def test_a_forked_child_does_not_wait_for_threads_it_does_not_have(probe):
+    assert "child ended 1\n" in probe("fork")
