@@ -34,19 +34,23 @@ HBM_PEAK_GBS = 8000.0
 # them 128 bytes - and TCC_EA0_WRREQ_sum: profiles/step_kernels_<profile>_l2_requests.md).
 MEASURED = {
     "weighted_node2vec_rmat22": {
-        "kernels": {"nd::step_flat_kernel": 1.123e9}, "bytes_per_pass": 145.38e9,
-        "read_requests": {"nd::step_flat_kernel": 8.235e6}, "write_requests": {"nd::step_flat_kernel": 1.698e6}},
+        "kernels": {"nd::step_flat_kernel": 1.122e9}, "bytes_per_pass": 145.24e9,
+        "read_requests": {"nd::step_flat_kernel": 8.224e6}, "write_requests": {"nd::step_flat_kernel": 1.698e6}},
     # the same workload with --inversion-period 0 (the engine's choice: walks keep their lanes)
     "weighted_node2vec_rmat22_period0": {
-        "kernels": {"nd::walk_stretch_kernel": 3.676e10}, "bytes_per_pass": 150.95e9,
-        "read_requests": {"nd::walk_stretch_kernel": 2.843e8}, "write_requests": {"nd::walk_stretch_kernel": 6.536e6}},
+        "kernels": {"nd::walk_rows_kernel": 1.408e11}, "bytes_per_pass": 140.79e9,
+        "read_requests": {"nd::walk_rows_kernel": 1.078e9}, "write_requests": {"nd::walk_rows_kernel": 7.506e7}},
     "uniform_walk_chunglu57k": {"kernels": {"nd::step_flat_kernel": 1.224e7}, "bytes_per_pass": 1.27e9},
+    "uniform_walk_chunglu57k_period0": {"kernels": {"nd::walk_rows_kernel": 1.329e8}, "bytes_per_pass": 0.13e9},
     # both kernel classes of a hop; the flat kernel is launched for both hops, the workgroup kernel for the second
     "khop_rmat21": {"kernels": {"nd::step_flat_kernel": 1.088e9, "nd::step_workgroup_kernel": 2.385e9},
-                    "bytes_per_pass": 8.45e9},
-    # collective_mark_binned, average over its 2 launches per pass
-    "fastgcn_importance_rmat22": {"kernels": {"nd::collective_mark_binned": 5.268e9}, "bytes_per_pass": 16.41e9},
-    "ladies_importance_chunglu3m": {"kernels": {"nd::collective_mark_binned": 6.752e10}, "bytes_per_pass": 161.61e9},
+                    "bytes_per_pass": 7.45e9},
+    # the kernels of a layer, average over a pass's 2 layers
+    "fastgcn_importance_rmat22": {
+        "kernels": {"nd::sorted_layer_kernel": 8.169e7, "nd::union_parts": 2.063e9, "nd::union_sums": 1.737e9},
+        "bytes_per_pass": 7.88e9},
+    "ladies_importance_chunglu3m": {
+        "kernels": {"nd::ranked_layer_kernel": 6.241e7, "nd::collective_mark_binned": 6.523e10}, "bytes_per_pass": 151.78e9},
 }
 
 
@@ -59,6 +63,9 @@ def _one(values):
 MEASURED_TRAFFIC_BYTES_PER_LAUNCH = {name: _one(m["kernels"]) for name, m in MEASURED.items() if len(m["kernels"]) == 1}
 MEASURED_TRAFFIC_BYTES_PER_LAUNCH["khop_rmat21"] = (2 * MEASURED["khop_rmat21"]["kernels"]["nd::step_flat_kernel"] +
                                                      MEASURED["khop_rmat21"]["kernels"]["nd::step_workgroup_kernel"]) / 2
+# layer-wise: the kernels of one layer together
+for _name in ("fastgcn_importance_rmat22", "ladies_importance_chunglu3m"):
+    MEASURED_TRAFFIC_BYTES_PER_LAUNCH[_name] = sum(MEASURED[_name]["kernels"].values())
 MEASURED_TRAFFIC_BYTES_PER_PASS = {name: m["bytes_per_pass"] for name, m in MEASURED.items()}
 MEASURED_L2_MISS_REQUESTS_PER_LAUNCH = {name: _one(m["read_requests"]) for name, m in MEASURED.items() if "read_requests" in m}
 MEASURED_L2_WRITE_REQUESTS_PER_LAUNCH = {name: _one(m["write_requests"]) for name, m in MEASURED.items() if "write_requests" in m}
@@ -157,50 +164,79 @@ def cpu_baseline_layers(graph, sampler, kind_name, budget_s, seed):
     }
 
 
-def marking_bytes_per_pass(graph, sampler, final, ladies):
-    """Bytes the marking kernel (collective_mark_binned) has to move in one pass, counted on
-    the host from the transits of every layer.  A transit with fewer edges into a stretch of the
-    vertex range than the library's threshold contributes those entries (id 4 B, + weight 4 B
-    for LADIES); with more, the stretch's ready-made piece (a bit per vertex, or a 64-bit sum
-    per vertex).  Every layer writes its whole per-sample map (bits, or 32-bit sampling keys).
-    FastGCN: a vertex that is among a sample's transits more than once counts once."""
-    stretch = 7168 if ladies else 65536
-    threshold = int(os.environ.get("ND_DENSE_PIECE_ENTRIES", 2048 if ladies else 1024))
-    piece_bytes = stretch * 8 if ladies else stretch // 8
-    entry_bytes = 8 if ladies else 4
-    rp, col = np.asarray(graph.row_ptr), np.asarray(graph.col)
-    degree = np.diff(rp).astype(np.int64)
-    n_samples, batch = sampler.num_samples, sampler.step_size(0)
-    layers = [sampler.initial_contents.reshape(-1)]
-    layers += [final[:, k * batch:(k + 1) * batch].reshape(-1) for k in range(sampler.steps - 1)]
-    if not ladies:
-        # the bitmap form marks a vertex once however often it is among a sample's transits
-        firsts = []
-        for layer in layers:
-            rows = np.sort(layer.reshape(n_samples, -1), axis=1)
-            keep = np.ones(rows.shape, bool)
-            keep[:, 1:] = rows[:, 1:] != rows[:, :-1]
-            firsts.append(rows[keep])
-        layers = firsts
-    transits = np.concatenate(layers)
-    transits = transits[(transits != sampler.invalid_vertex) & (transits >= 0)]
-    vertices, uses = np.unique(transits, return_counts=True)
-    big = degree[vertices] >= threshold if threshold > 0 else np.zeros(len(vertices), bool)
-    entries = int((uses[~big] * degree[vertices[~big]]).sum())
-    pieces, distinct_pieces = 0, 0
-    for v, c in zip(vertices[big], uses[big]):
-        per_stretch = np.bincount(col[rp[v]:rp[v + 1]] // stretch)
-        ready = per_stretch >= threshold
-        pieces += int(c) * int(ready.sum())
-        distinct_pieces += int(ready.sum())
-        entries += int(c) * int(per_stretch[~ready].sum())
-    words = ((graph.n_vertices + 31) // 32 + 2047) // 2048 * 2048  # a bit per vertex, padded to 2048 words
-    per_sample_out = (words + 223) // 224 * 7168 * 4 if ladies else words * 4  # LADIES: a 32-bit key per vertex
-    written = sampler.steps * n_samples * per_sample_out
-    # from_memory: every entry and every written map once, every piece that is used at all once
-    # per layer (the pieces are a few thousand per graph and stay in the caches between uses)
-    from_memory = entries * entry_bytes + sampler.steps * distinct_pieces * piece_bytes + written
-    return entries * entry_bytes + pieces * piece_bytes + written, entries, pieces, from_memory
+def _layers_of_transits(sampler, final):
+    """The transits of every layer of the last pass, [samples, transits of a sample] each."""
+    batch = sampler.step_size(0)
+    layers = [sampler.initial_contents.reshape(sampler.num_samples, -1)]
+    return layers + [final[:, k * batch:(k + 1) * batch] for k in range(sampler.steps - 1)]
+
+
+def _real(transits, invalid):
+    return (transits != invalid) & (transits >= 0)
+
+
+def union_bytes_per_pass(graph, sampler, final):
+    """FastGCN form: bytes the kernels that build and weigh a layer's neighbourhoods (sorted_layer_kernel, union_parts,
+    union_sums) have to move in one pass, counted on the host from the transits of every layer.  Every adjacency
+    that a layer touches comes from memory once (4 B an edge); a sample of more than 4096 entries has its bitmap written
+    and read (a bit per vertex, whole parts of 16,384 vertices) and its sums written (8 B a group of 256 vertices).
+    Returns (bytes, the same with every sample's distinct transits read anew, entries read once, samples with a bitmap)."""
+    degree = np.diff(np.asarray(graph.row_ptr)).astype(np.int64)
+    degree = np.append(degree, 0)  # of no vertex
+    parts = -(-graph.n_vertices // 16384)
+    per_sample = parts * (2 * 2048 + 64 * 8)
+    once, every, marked = 0, 0, 0
+    for layer in _layers_of_transits(sampler, final):
+        layer = np.where(_real(layer, sampler.invalid_vertex), layer, graph.n_vertices)
+        marked += int((degree[layer].sum(axis=1) > 4096).sum())
+        rows = np.sort(layer, axis=1)
+        firsts = np.ones(rows.shape, bool)
+        firsts[:, 1:] = rows[:, 1:] != rows[:, :-1]
+        every += int(degree[rows][firsts].sum())
+        once += int(degree[np.unique(rows)].sum())
+    return 4 * once + marked * per_sample, 4 * every + marked * per_sample, once, marked
+
+
+def marking_bytes_per_pass(graph, sampler, final):
+    """LADIES form: bytes the kernels that rank small neighbourhoods and mark the others (ranked_layer_kernel,
+    collective_mark_binned) have to move in one pass, counted on the host from the transits of every layer.  Parallel
+    edges are one pair of 12 B (id and term).  A transit with fewer pairs into a stretch of 7168 vertices than the
+    library's threshold contributes those pairs; with more, the stretch's ready-made piece of 64-bit sums.  Every
+    sample of more than 8192 pairs writes a 32-bit key per vertex, padded to whole stretches.
+    Returns (bytes with every use, pairs read one by one, pieces read, bytes with every piece once per layer)."""
+    stretch, threshold = 7168, int(os.environ.get("ND_DENSE_PIECE_ENTRIES", 2048))
+    rp, col = np.asarray(graph.row_ptr).astype(np.int64), np.asarray(graph.col)
+    is_first = np.ones(len(col), bool)
+    is_first[1:] = col[1:] != col[:-1]
+    is_first[rp[:-1][np.diff(rp) > 0]] = True
+    before = np.concatenate([[0], np.cumsum(is_first)])
+    pairs_of = np.append(before[rp[1:]] - before[rp[:-1]], 0)
+    stretches = -(-graph.n_vertices // stretch)
+    piece_bytes, keys_of_sample = 8 * stretch, 4 * stretch * stretches
+    pairs, pieces, distinct_pieces, marked = 0, 0, 0, 0
+    ready_of = {}  # vertex: (pieces, pairs outside of them)
+    for layer in _layers_of_transits(sampler, final):
+        layer = np.where(_real(layer, sampler.invalid_vertex), layer, graph.n_vertices)
+        sizes = pairs_of[layer].sum(axis=1)
+        large = sizes > 8192
+        marked += int(large.sum())
+        pairs += int(sizes[~large].sum())
+        vertices, uses = np.unique(layer[large], return_counts=True)
+        big = pairs_of[vertices] >= threshold if threshold > 0 else np.zeros(len(vertices), bool)
+        pairs += int((uses[~big] * pairs_of[vertices[~big]]).sum())
+        for v, c in zip(vertices[big].tolist(), uses[big].tolist()):
+            if v not in ready_of:
+                row = slice(rp[v], rp[v + 1])
+                per_stretch = np.bincount(col[row][is_first[row]] // stretch)
+                ready = per_stretch >= threshold
+                ready_of[v] = int(ready.sum()), int(per_stretch[~ready].sum())
+            n_ready, rest = ready_of[v]
+            pieces += c * n_ready
+            distinct_pieces += n_ready
+            pairs += c * rest
+    written = marked * keys_of_sample
+    return (pairs * 12 + pieces * piece_bytes + written, pairs, pieces,
+            pairs * 12 + distinct_pieces * piece_bytes + written)
 
 
 def pairs_reaching_the_step_kernels(sampler, final):
@@ -317,6 +353,9 @@ def measure(args, workload, steps, warmup, cpu_seconds, graphs, engine_choice=Tr
     adaptive = None
     if sampler.step_size(0) == 1 and sampler.steps > 1 and args.inversion_period == 1 and engine_choice:
         sampler.set_inversion_period(0)
+        # the first pass after a fetch sends its rows ahead, for the caller who fetches every pass's; the next one
+        # does without, as the timed ones do
+        sampler.do_transit_parallel(lb)
         sampler.do_transit_parallel(lb)
         t0 = time.perf_counter()
         for _ in range(steps):
@@ -361,37 +400,40 @@ def measure(args, workload, steps, warmup, cpu_seconds, graphs, engine_choice=Tr
         result["config"]["chunks"] = sampler.counter(2)
         result["config"]["hub_bitmaps"] = sampler.counter(3)
         result["config"]["neighbourhood_entries_per_s"] = entries / (ms_per_step / 1000.0)
-        # dominant kernel: collective_mark_binned accounts for every entry of every collective
-        # neighbourhood once, one by one or through the ready-made pieces of the hubs
+        # the kernels that build every neighbourhood and weigh its vertices: what runs between the library's
+        # neighbourhood events
         ladies = w["kind"] == "LADIES_IMPORTANCE"
-        mark_bytes, read_entries, read_pieces, from_memory = marking_bytes_per_pass(graph, sampler, final, ladies)
-        result["config"]["entries_read_one_by_one"] = read_entries
-        result["config"]["hub_pieces_read"] = read_pieces
         launches = max(prof["neighbourhood_launches"], 1)
-        # `achieved` prices what has to come from or go to HBM: entries read one by one, the
-        # maps written, and every ready-made piece once per layer; the repeated uses of the few
-        # thousand pieces are served by the caches and are reported apart, not as HBM bytes
+        if ladies:
+            kernels = "ranked_layer_kernel + collective_mark_binned"
+            every_use, read_pairs, read_pieces, from_memory = marking_bytes_per_pass(graph, sampler, final)
+            result["config"]["pairs_read_one_by_one"] = read_pairs
+            result["config"]["hub_pieces_read"] = read_pieces
+        else:
+            kernels = "sorted_layer_kernel + union_parts + union_sums"
+            from_memory, every_use, read_once, marked = union_bytes_per_pass(graph, sampler, final)
+            result["config"]["edges_read_once_per_layer"] = read_once
+            result["config"]["neighbourhoods_as_bitmaps"] = marked
+        # `achieved` prices what has to come from or go to HBM: what is read by many samples of a layer counts
+        # once, the uses beyond that are served by the caches and are reported apart, not as HBM bytes
         achieved = from_memory / (prof["neighbourhood_ms"] / 1000.0) / 1e9
-        all_uses = mark_bytes / (prof["neighbourhood_ms"] / 1000.0) / 1e9
-        # what the recorded counters say the launch is bound by: its measured HBM traffic over this
-        # run's launch time.  The LADIES form streams (entries in, keys out: near half of the HBM
-        # peak); the FastGCN form moves a fifth of the peak - its hubs' pieces and adjacencies come
-        # from the caches, and a workgroup spends its time in the chain of searches, LDS table and
-        # barriers it goes through per stretch of the vertex range
+        every_use_gbps = every_use / (prof["neighbourhood_ms"] / 1000.0) / 1e9
+        # what the recorded counters say the launches are bound by: their measured HBM traffic over this run's time
         recorded = MEASURED_TRAFFIC_BYTES_PER_LAUNCH.get(workload)
         traffic_gbps = recorded / (prof["neighbourhood_ms"] / launches / 1000.0) / 1e9 if recorded else None
-        bound = "hbm" if traffic_gbps is None or traffic_gbps / HBM_PEAK_GBS >= 0.3 else \
-            "latency (dependent steps per stretch of the vertex range; the caches serve the hubs)"
+        # (LADIES: 5 TB/s, and 63 % of the vector issue slots; FastGCN: union_parts takes its pieces and entries from L2, at
+        # 2.2 TB/s from memory, union_sums reads the bitmaps at 3.1 TB/s)
+        bound = "hbm" if ladies else "L2 (pieces and entries of union_parts), hbm (bitmaps of union_sums)"
         result["roofline"] = {
-            "bound": bound, "kernel": "collective_mark_binned", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+            "bound": bound, "kernel": kernels, "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS, "traffic": recorded,
             "measured_traffic_GBps": traffic_gbps,
             "measured_traffic_frac": traffic_gbps / HBM_PEAK_GBS if traffic_gbps else None,
             "algorithmic_bytes_per_launch": from_memory / launches,
             "avg_launch_ms": prof["neighbourhood_ms"] / launches,
-            "cache_served": {"bytes_per_launch_with_every_piece_use": mark_bytes / launches,
-                             "GBps_with_every_piece_use": all_uses,
-                             "note": "piece uses beyond the first per layer come from L2 / Infinity Cache: a cache "
+            "cache_served": {"bytes_per_launch_with_every_use": every_use / launches,
+                             "GBps_with_every_use": every_use_gbps,
+                             "note": "uses beyond the first per layer come from L2 / Infinity Cache: a cache "
                                      "throughput figure, not an HBM roofline fraction"},
             "whole_pass": {"measured_traffic": MEASURED_TRAFFIC_BYTES_PER_PASS.get(workload)},
         }
@@ -460,7 +502,7 @@ def measure(args, workload, steps, warmup, cpu_seconds, graphs, engine_choice=Tr
             chosen_launches = max(adaptive["phases_ms"]["flat_launches"], 1)
             period0 = MEASURED.get(workload + "_period0")
             adaptive["roofline"] = {
-                "bound": "hbm", "kernel": "walk_stretch_kernel (and step_flat_kernel for step 0)",
+                "bound": "hbm", "kernel": "walk_rows_kernel",
                 "achieved": step_bytes / (chosen_ms / 1000.0) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": step_bytes / (chosen_ms / 1000.0) / 1e9 / HBM_PEAK_GBS,
                 "algorithmic_bytes_per_launch": step_bytes / chosen_launches,
@@ -503,14 +545,11 @@ def measure(args, workload, steps, warmup, cpu_seconds, graphs, engine_choice=Tr
             }
             period0 = MEASURED.get(workload + "_period0")
             if adaptive and "roofline" in adaptive and period0 and "read_requests" in period0:
-                # the stretch kernel against the same ceiling: its recorded requests per launch (the
-                # average over a pass's stretches) times the stretches of this pass, over the time
-                # of the pass's step kernels (which includes the one flat launch of step 0)
-                stretches = max(adaptive["phases_ms"]["flat_launches"] - 1, 1)
-                reads = _one(period0["read_requests"]) * stretches
+                # walks that keep their lanes against the same ceiling: one launch a pass
+                reads = _one(period0["read_requests"])
                 chosen_s = adaptive["phases_ms"]["flat_kernel_ms"] / 1000.0
                 adaptive["roofline"]["l2_miss_path"] = {
-                    "read_requests_per_pass": reads, "write_requests_per_pass": _one(period0["write_requests"]) * stretches,
+                    "read_requests_per_pass": reads, "write_requests_per_pass": _one(period0["write_requests"]),
                     "achieved_read_requests_per_s": reads / chosen_s, "ceiling_requests_per_s": ceiling,
                     "frac_of_ceiling": reads / chosen_s / ceiling}
     del final
