@@ -125,8 +125,9 @@ int nd_sampler_fetch_sample_states(nd_sampler* s, const void** data, int64_t* by
  * of the edge lists, or sample states, as the last call for them returned it - the caller's: the
  * library neither writes to it nor frees it any more, and the next call for the same result
  * returns another array.  *owner stands for it until nd_release_array(owner), after which its
- * memory is used for a later result of the same sampler, or freed if that is gone.  (At most two
- * such arrays' memory is kept, until nd_sampler_free_device or nd_sampler_destroy.)  Instead of
+ * memory is used for a later result of the same sampler, or freed if that is gone.  (At most one
+ * such array's memory is kept for each kind of result the sampler has, until nd_sampler_free_device or
+ * nd_sampler_destroy.)  Instead of
  * a copy, for callers that keep what they are given. */
 int nd_sampler_detach_array(nd_sampler* s, const void* data, void** owner);
 void nd_release_array(void* owner);

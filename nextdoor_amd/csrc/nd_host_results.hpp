@@ -176,7 +176,7 @@ struct HostBlock {
 // 1.5 MB 92 / 100, 116; 2 MB 118 / 110, 128; 3 MB 169 / 121, 155; 4 MB 220 / 113, 158.
 constexpr size_t kDirectResultBytes = 2u << 20;
 
-// The host arrays of one sampler.  At most kKeep of them wait for their next use; all of those are freed with the
+// The host arrays of one sampler.  A few of them (keep()) wait for their next use; all of those are freed with the
 // sampler's device memory and when it goes, the others when their holders let go of them.
 // They are ordinary private memory, since callers do with them what they do with any array: page-locked memory
 // of the runtime's is not there in a forked child (a data loader's worker that touches it dies), nor may system calls
@@ -227,7 +227,7 @@ class HostPool {
       if (open_) {
         free_.push_back(b);
         drop = HostBlock();
-        if (free_.size() > kKeep) {
+        if (free_.size() > keep_) {
           drop = free_.front();  // the one that has waited longest
           free_.erase(free_.begin());
         }
@@ -236,6 +236,13 @@ class HostPool {
     release(drop);
   }
 
+  // How many wait at most.  A loop that holds its last results while it makes the next leaves one array of each kind
+  // of result waiting at a time.
+  void keep(size_t kinds) {
+    trim();
+    std::lock_guard<std::mutex> lock(mutex_);
+    keep_ = kinds;
+  }
   // frees those that wait
   void trim() { drop_waiting(true); }
   // ... and keeps none from here on
@@ -249,10 +256,6 @@ class HostPool {
   }
 
  private:
-  // A loop that holds its last results while it makes the next leaves one array of each kind waiting at a time, and
-  // no sampler has more than two kinds (rows and states; rows and columns).
-  static constexpr size_t kKeep = 2;
-
   void drop_waiting(bool open) {
     std::vector<HostBlock> all;
     {
@@ -271,6 +274,7 @@ class HostPool {
 
   std::mutex mutex_;
   std::vector<HostBlock> free_;
+  size_t keep_ = 2;
   bool open_ = true;
 };
 

@@ -58,6 +58,12 @@ static int arrays_that_wait() {
   for (int i = 0; i < 5; ++i) held.push_back(pool->take(16u << 20));
   for (const nd::HostBlock& b : held) pool->give(b);
   printf("%zu\n", pool->waiting_bytes());
+  for (size_t kinds = 1; kinds <= 4; ++kinds) {  // of a walk without states; of edge lists with all there is
+    pool->keep(kinds);
+    for (nd::HostBlock& b : held) b = pool->take(16u << 20);
+    for (const nd::HostBlock& b : held) pool->give(b);
+    printf("%zu\n", pool->waiting_bytes());
+  }
   pool->trim();
   printf("%zu\n", pool->waiting_bytes());
   nd::HostBlock last = pool->take(1000);

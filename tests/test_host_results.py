@@ -48,8 +48,9 @@ def test_the_control_groups_share_is_counted(probe, tmp_path, files, groups, cpu
     assert probe("cpus", root, tmp_path / "groups").strip() == cpus
 
 
-def test_two_arrays_at_most_wait_for_their_next_use(probe):
-    assert [int(x) for x in probe("pool").split()] == [2 * (16 << 20), 0, 1000, 0]
+def test_as_many_arrays_wait_for_their_next_use_as_there_are_kinds_of_result(probe):
+    mb16 = 16 << 20
+    assert [int(x) for x in probe("pool").split()] == [2 * mb16, mb16, 2 * mb16, 3 * mb16, 4 * mb16, 0, 1000, 0]
 
 
 def test_a_forked_child_does_not_wait_for_threads_it_does_not_have(probe):
