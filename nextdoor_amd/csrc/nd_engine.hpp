@@ -825,7 +825,7 @@ __device__ __forceinline__ void enter_vertex(const CSRPartition& csr, const Walk
 // then takes the next walk of its wavefront; results go straight into the rows, four to a store.
 //
 // What bounds it: the gathers.  Over a graph beyond the caches the requests past L2 (R-MAT 22 weighted
-// node2vec: 1.17e9 of them in 24.5 ms, 47.8 G/s of the 48-50 the gather probe reaches: row extent, 2.95
+// node2vec: 1.15e9 of them in 24.1 ms, 47.9 G/s of the 48-50 the gather probe reaches: row extent, 2.95
 // candidates and 0.9 tests a step), over one within them L2's own rate and, with few walks, the chain
 // of dependent loads.  A turn of the loop is therefore two CANDIDATES of every lane (they share a
 // Philox block), not one step: a wavefront that waits at every step for the slowest of 64 rejection

@@ -2,7 +2,7 @@
 //
 // A pass leaves gigabytes of 4-byte vertex ids in device memory and the caller wants them in
 // host memory: of 4.2 M node2vec walks (1.68 GB, 34 ms to sample) the copy took 29 ms at the bus's
-// 57 GB/s, and another 118 ms went into handing the caller an array of their own.  Three things
+// 57 GB/s, and another 118 ms went into handing the caller an array of their own.  Four things
 // are done about it here:
 //
 //  * What crosses the bus is packed (pack_results): ids take as many bits as the largest one, the
@@ -578,7 +578,7 @@ inline hipError_t device_of(hipStream_t stream, int* device) {
   return stream ? hipStreamGetDevice(stream, device) : hipGetDevice(device);
 }
 
-// The stream results cross the bus on while something else is computed: one per device (the current one) and process, on
+// The stream results cross the bus on while something else is computed: one per device (which has to be the current one) and process, on
 // a hardware queue of its own, which a stream with a mask of compute units (here: all) gets.  (Ordinary streams share
 // four; where the computation's lands on the same one, nothing overlaps.)  They are destroyed when the process ends, while
 // the runtime and whatever watches it are still there: left to the runtime, their queues outlive a profiler's
