@@ -386,10 +386,11 @@ int nd_sampler_alloc(nd_sampler* s, uint64_t seed) {
     if (rc != 0) return fail(s->engine->last_error, rc);
     nd::EngineBase& e = *s->engine;
     e.host_pool->keep(1 + (e.sample_state_bytes() > 0 ? 1 : 0) + (e.lists_edges() ? 2 : 0));
-    // small results' page-locked memory with the other buffers (0.5 ms, several passes' worth); if there is none, the
-    // first fetch says so
+    // small results' page-locked memory with the other buffers (a millisecond: the longer part of a first pass); larger
+    // ones' with their first fetch.  If there is none, the first fetch says so.
     const uint64_t words = (uint64_t)e.num_samples() * (uint64_t)e.final_sample_size();
-    if (words * sizeof(int32_t) <= nd::kDirectResultBytes && e.result_stream->reserve() != hipSuccess)
+    if (words * sizeof(int32_t) <= 2 * nd::kDirectResultBytes &&
+        e.result_stream->reserve((size_t)words, (uint32_t)e.max_bits()) != hipSuccess)
       (void)hipGetLastError();
     return 0;
   });

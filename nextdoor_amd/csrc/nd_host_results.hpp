@@ -631,12 +631,19 @@ class ResultStream {
     hipEvent_t event;
   };
 
-  // Takes the page-locked memory that copy() needs, on the current device, ahead of the first.
-  hipError_t reserve() {
+  // Takes, on the current device and ahead of the first, what a copy() or a fetch() of n words needs.
+  hipError_t reserve(size_t n, uint32_t bits) {
     hipError_t e = finish();
     if (e == hipSuccess) e = come_to_device_of(nullptr);
-    if (e == hipSuccess) e = make_ring(kDirectResultBytes);
-    if (e == hipSuccess) memset(ring_, 0, kDirectResultBytes);  // its pages are mapped when they are first touched: 0.8 ms
+    if (e != hipSuccess) return e;
+    if (n * sizeof(int32_t) <= kDirectResultBytes) {
+      e = make_ring(kDirectResultBytes);
+    } else {
+      if (!transfer_) transfer_.reset(new Transfer);
+      transfer_->set(nullptr, n, bits > kPackMostBits ? 32 : bits, 0, nullptr, {});
+      e = prepare(transfer_->slot_bytes);
+    }
+    if (e == hipSuccess) memset(ring_, 0, ring_bytes_);  // its pages are mapped when they are first touched: 0.8 ms of 2 MB
     return e;
   }
 
