@@ -24,9 +24,8 @@
 //  * kRankedByLadiesImportance: each entry carries (weight * (1 / rowsum(transit)))^2 as a 2^53 fixed-point integer,
 //    worked out once per graph with parallel edges merged.  Small neighbourhoods are summed, keyed
 //    (Efraimidis-Spirakis) and sorted in LDS by one workgroup.  Of the others the terms of a vertex are summed in LDS
-//    stretch by stretch, its key is formed from the sum as it leaves LDS (the only thing stored per sample and
-//    vertex), a radix select keeps the few entries that can be among the sample's first picks, and stable sorts
-//    order those by descending key.
+//    stretch by stretch, and of the keys formed from the sums as they leave LDS those that can be among the sample's
+//    first picks are kept (the only thing stored); one more workgroup a sample puts them in order.
 //  * Samples are processed in chunks whose concatenated neighbourhoods fit a fixed budget
 //    of entries, so a layer whose frontier sits on hubs cannot outgrow memory.
 //  * Random numbers: Philox keyed by the output slot s * stepSize(k) + nbr and the layer.
@@ -47,7 +46,6 @@
 #include "nd_contract.hpp"
 #include "nd_device_graph.hpp"
 #include "nd_engine.hpp"
-#include "nd_radix_sort.hpp"
 #include "nd_union_sums.hpp"
 
 namespace nd {
@@ -251,14 +249,15 @@ __host__ __device__ __forceinline__ float det_log2(float x) {
 // 0xFFFFFFFF (it would be a negative NaN): kAbsentKey marks the vertices a sample's
 // neighbourhood does not hold.
 constexpr uint32_t kAbsentKey = 0xFFFFFFFFu;
-// importance sums stay below 2^63 (at most 1024 transits, each adding at most 2^53)
-constexpr unsigned long long kAbsentSum = ~0ull;
 __host__ __device__ __forceinline__ uint64_t ladies_pair_index(uint64_t sample, uint32_t n_vertices, uint32_t v) {
   return sample * (uint64_t)((n_vertices + 3u) & ~3u) + v;
 }
 __device__ __forceinline__ PhiloxBlock ladies_block(uint64_t pair, uint32_t step, uint64_t seed) {
   const uint64_t block = pair >> 2;
-  return philox4x32_10((uint32_t)block, (uint32_t)(block >> 32), step, 0, (uint32_t)seed, (uint32_t)(seed >> 32));
+  // (the key opaque, as in grouped_first_block_scalar_seed: the round keys as they come, not twenty of them in registers)
+  uint32_t k0 = __builtin_amdgcn_readfirstlane((uint32_t)seed), k1 = __builtin_amdgcn_readfirstlane((uint32_t)(seed >> 32));
+  asm volatile("" : "+s"(k0), "+s"(k1));
+  return philox4x32_10((uint32_t)block, (uint32_t)(block >> 32), step, 0, k0, k1);
 }
 __device__ __forceinline__ uint32_t ladies_key_from_word(unsigned long long importance_fixed, uint32_t word) {
   const float importance = (float)importance_fixed;
@@ -268,6 +267,12 @@ __device__ __forceinline__ uint32_t ladies_key_from_word(unsigned long long impo
   uint32_t b = __float_as_uint(key);
   b = (b & 0x80000000u) ? ~b : (b | 0x80000000u);
   return ~b;
+}
+// Whether ladies_key_from_word of the same can be at or below the bound that `reach` belongs to (Keeper::reach): the word's
+// upper 24 bits against the least that can be, with 4 for what the float of 2^24 and the uniform itself are rounded by.
+__device__ __forceinline__ bool key_may_be_within(float reach, unsigned long long importance_fixed, uint32_t word) {
+  const float least = __builtin_fmaf((float)((uint32_t)(importance_fixed >> 32) + 1u), -reach, 16777212.0f);
+  return (word >> 8) >= (uint32_t)least;  // (negative and NaN: 0)
 }
 // one pair on its own
 __device__ __forceinline__ uint32_t ladies_key_bits(unsigned long long importance_fixed, uint64_t pair, uint32_t step,
@@ -281,17 +286,10 @@ __device__ __forceinline__ uint32_t ladies_key_bits(unsigned long long importanc
   return ladies_key_from_word(importance_fixed, word);
 }
 
-// ---- wave-wide data movement on the VALU (DPP), no LDS traffic ----
-// The value of the lane `shift` below inside the lane's row of 16; lanes without one get `fill`.
-template <int kShift>
-__device__ __forceinline__ uint32_t row_shift_up(uint32_t fill, uint32_t x) {
-  return (uint32_t)__builtin_amdgcn_update_dpp((int)fill, (int)x, 0x110 | kShift, 0xF, 0xF, false);
-}
 // One workgroup per (sample, some consecutive stretches of 7168 vertices), the sums of one stretch in LDS at a time.
 // Adjacencies are sorted by destination, so the part of a transit's adjacency that falls into a stretch is one
 // sub-range; the workgroup streams the sub-ranges of all the sample's transits, adds in LDS, and writes the stretch
-// out once - plain stores that cover the whole map, so nothing is cleared beforehand and no atomic reaches memory
-// (global atomics stop at ~24 G/s on this part).  Every wavefront walks a contiguous part of the stretch's entries,
+// over once, and no atomic reaches memory (global atomics stop at ~24 G/s on this part).  Every wavefront walks a contiguous part of the stretch's entries,
 // which lets a lane step from one sub-range to the next instead of searching the table for every entry.
 constexpr uint32_t kBinThreads = 1024;
 constexpr uint32_t kBinWaves = kBinThreads / 64;
@@ -303,8 +301,8 @@ constexpr uint32_t kBinWords = kBinVertices / 32u;
 // Dense pieces.  What a hub contributes to a stretch can be thousands of entries (a layer drawn by importance sits on
 // the hubs), and it is the same for every sample that holds the hub.  Where a vertex has kDensePieceEntries or more
 // neighbours in one stretch, the stretch's piece of that vertex is built once per graph - the importance sum of every
-// vertex of the stretch (7168 64-bit integers, kAbsentSum where there is no edge) - and a sample adds the piece on the
-// stretch's way out of LDS instead of going through the entries.  hub_row[v] = row of v in piece_of or -1;
+// vertex of the stretch (7168 64-bit integers, 0 where there is no edge; there is no piece where an edge's sum is 0) - and a
+// sample adds the piece on the stretch's way out of LDS instead of going through the entries.  hub_row[v] = row of v in piece_of or -1;
 // piece_of[row * stretches + stretch] = piece index or kNoPiece.
 constexpr uint32_t kDensePieceEntries = 2048;
 constexpr size_t kDensePieceBudgetBytes = (size_t)2 << 30;
@@ -314,17 +312,33 @@ struct DensePieces {
   const unsigned long long* sums = nullptr;
 };
 
-// LADIES form: the marking kernel turns the importance sums into sampling keys itself where a
-// stretch leaves LDS (a lane takes four consecutive vertices and pays for one Philox block) and
-// writes those, 4 bytes per vertex and sample.  Writing the sums instead and forming the keys in
-// the selection's pass cost 8 + 8 + 4 bytes per vertex and sample of traffic, and 3.4 ms more
-// per pass at full size.
-struct KeysOnTheWayOut {
-  uint32_t* keys = nullptr;
-  uint64_t seed = 0;
-  uint64_t first_sample = 0;
-  uint32_t step = 0;
-  uint32_t n_vertices = 0;
+// ---- the best keys of a sample ----
+//
+// Only the first stepSize vertices of a sample in key order are ever read, out of up to millions: `wanted` of them.  A
+// workgroup forms the keys of its stretches where the sums leave LDS and keeps those that can still be among them: it
+// counts what it has kept by the upper bits of the keys, and once `wanted` keys lie at or below an edge between two counts
+// (the bound) nothing above that edge can be.  A bound is good for the whole sample, and workgroups that start later begin
+// with it.  (One key for every vertex of a sample, written to memory, selected from and sorted by the radix sort's launches:
+// 2 GB written and read and 50 launches a layer over 500 K vertices.)
+// By float exponent and two bits of the mantissa: an edge lets at most a quarter too many through.
+constexpr uint32_t kBoundBins = 1024;
+constexpr uint32_t kNoBound = 0xFFFFFFFEu;  // below kAbsentKey
+// a key is the bit pattern of a negative float, or of +0 (the best there is) as 0x7FFFFFFF
+__device__ __forceinline__ uint32_t bin_of_key(uint32_t key) { return (int32_t)key >= 0 ? 0u : key >> 21 & (kBoundBins - 1u); }
+__device__ __forceinline__ uint32_t last_key_of_bin(uint32_t bin) { return 0x80000000u | bin << 21 | 0x1FFFFFu; }
+
+// What a workgroup keeps at most: room for everything a stretch can add to what it may begin the stretch with.
+constexpr uint32_t kKeptEntries = 12288;
+struct KeptKeys {
+  uint2* kept;          // (key, vertex), [workgroup of the chunk][kKeptEntries]
+  uint32_t* n_kept;     // [workgroup of the chunk]
+  uint32_t* bound;      // [marked sample]; kNoBound before the layer
+  uint32_t* distinct;   // [sample of the chunk]; 0 before the layer
+  uint64_t seed;
+  uint64_t first_sample;
+  uint32_t step;
+  uint32_t n_vertices;
+  uint32_t wanted;
 };
 
 // 32-bit words of one sample's presence map: a bit per vertex, padded to whole tiles.
@@ -333,7 +347,8 @@ inline uint32_t bitmap_words_for(uint32_t n_vertices) {
 }
 
 // The workgroup's sub-ranges, a lane each (lanes of a wavefront without a transit: length 0), into the tables: those that
-// hold entries in lane order, starts[k] = first entry of sub-range k, starts[kept] = all entries, edge[k] its first edge.
+// hold entries in lane order, starts[k] = first entry of sub-range k, starts[kept] = all entries, shift[k] = its first edge
+// less that (entry e of it is edge e + shift[k]).
 // A length with kPieceFlag set stands for a transit whose entries reach the stretch as a ready-made piece: its index
 // joins the list `pieces`.  Two barriers; every lane gets the three counts.
 constexpr uint32_t kPieceFlag = 0x80000000u;
@@ -341,7 +356,7 @@ struct Subranges {
   uint32_t ranges, pieces, entries;
 };
 __device__ __forceinline__ Subranges list_subranges(uint32_t raw, EdgePos_t first, uint32_t n_transits, uint32_t* starts,
-                                                    EdgePos_t* edge, uint32_t* pieces, uint4* s_wave) {
+                                                    EdgePos_t* shift, uint32_t* pieces, uint4* s_wave) {
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, waves = (n_transits + 63u) / 64u;
   const bool is_piece = (raw & kPieceFlag) != 0;
   const uint32_t len = is_piece ? 0u : raw;
@@ -360,7 +375,7 @@ __device__ __forceinline__ Subranges list_subranges(uint32_t raw, EdgePos_t firs
   if (len != 0) {
     const uint32_t k = mine.ranges + (uint32_t)__popcll(holds & below);
     starts[k] = mine.entries + through - len;
-    edge[k] = first;
+    shift[k] = first - (EdgePos_t)starts[k];
   }
   if (is_piece) pieces[mine.pieces + (uint32_t)__popcll(ready & below)] = raw & ~kPieceFlag;
   if (threadIdx.x == 0) starts[all.ranges] = all.entries;
@@ -368,25 +383,154 @@ __device__ __forceinline__ Subranges list_subranges(uint32_t raw, EdgePos_t firs
   return all;
 }
 
+// The rank-th smallest (from 1) of the values each(f) hands to f, all of them different; each() is called by the whole
+// workgroup, every value handed out by one lane, and there are at least `rank`.  Eight bits a turn.
+struct PickScratch {
+  uint32_t count[256];
+  uint32_t digit, rank;
+};
+template <class Each>
+__device__ __forceinline__ uint64_t nth_smallest(Each each, uint32_t rank, PickScratch& scratch) {
+  uint64_t prefix = 0, known = 0;
+  for (int shift = 56; shift >= 0; shift -= 8) {
+    __syncthreads();
+    if (threadIdx.x < 256) scratch.count[threadIdx.x] = 0;
+    __syncthreads();
+    each([&](uint64_t value) {
+      if ((value & known) == prefix) atomicAdd(&scratch.count[value >> shift & 255u], 1u);
+    });
+    __syncthreads();
+    if (threadIdx.x < 64) {
+      uint32_t own = 0;
+      for (uint32_t d = 0; d < 4; ++d) own += scratch.count[threadIdx.x * 4u + d];
+      const uint32_t through = wave_inclusive_scan(own);
+      uint32_t before = through - own;
+      if (before < rank && through >= rank) {  // one lane
+        uint32_t d = threadIdx.x * 4u;
+        while (before + scratch.count[d] < rank) before += scratch.count[d++];
+        scratch.digit = d;
+        scratch.rank = rank - before;
+      }
+    }
+    __syncthreads();
+    prefix |= (uint64_t)scratch.digit << shift;
+    known |= 255ull << shift;
+    rank = scratch.rank;
+  }
+  return prefix;
+}
+// keys in ascending order, equal ones by vertex
+__device__ __forceinline__ uint64_t rank_value(uint2 kept) { return (uint64_t)kept.x << 32 | kept.y; }
+
+// What a workgroup of collective_mark_binned knows of the keys it has kept; in LDS, set before use by begin().
+struct Keeper {
+  uint32_t counts[kBoundBins];  // of the keys at or below the bound of their time
+  uint32_t wave_total[kBinThreads / 64];
+  uint32_t bound, fresh, n;     // no key above it is wanted; keys since it was looked for; keys kept
+  PickScratch pick;
+
+  __device__ __forceinline__ void begin(uint32_t sample_bound) {  // the caller's next barrier ends it
+    for (uint32_t i = threadIdx.x; i < kBoundBins; i += kBinThreads) counts[i] = 0;
+    if (threadIdx.x == 0) {
+      bound = sample_bound;
+      fresh = n = 0;
+    }
+  }
+  // How far from 1 a uniform may be without its key being above the bound for certain, in units of 2^-24, for an importance of
+  // 2^32: -log2(u) is at least (1 - u) / ln 2, and 0.69325 for ln 2 leaves 1.5e-4 to what the two sides are rounded by (every
+  // operation by 6e-8).  NaN, and then everything may, without a bound.
+  __device__ __forceinline__ float reach() const {
+    return __uint_as_float(bound & 0x7FFFFFFFu) * (0.69325f * 4294967296.0f * 16777216.0f);
+  }
+  // A key that was formed: kAbsentKey where it is above the bound, else counted.
+  __device__ __forceinline__ uint32_t count(uint32_t key) {
+    if (key > bound) return kAbsentKey;
+    atomicAdd(&counts[bin_of_key(key)], 1u);
+    return key;
+  }
+  // When every lane has counted what it has of a stretch, `here` keys a wavefront: lowers the bound as far as it goes.
+  __device__ __forceinline__ void lower_bound_to(uint32_t wanted, uint32_t here, uint32_t* sample_bound) {
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    if (lane == 0 && here != 0) atomicAdd(&fresh, here);
+    __syncthreads();
+    if (fresh * 4u < wanted) return;  // not worth another look yet
+    static_assert(kBoundBins == kBinThreads, "a lane per count");
+    const uint32_t own = counts[threadIdx.x], through = wave_inclusive_scan(own);
+    if (lane == 63) wave_total[wave] = through;
+    __syncthreads();
+    uint32_t before = through - own;
+    for (uint32_t w = 0; w < wave; ++w) before += wave_total[w];
+    if (before < wanted && before + own >= wanted) {  // at most one lane
+      const uint32_t edge = last_key_of_bin(threadIdx.x);
+      if (edge < bound) {
+        bound = edge;
+        atomicMin(sample_bound, edge);
+      }
+    }
+    if (threadIdx.x == 0) fresh = 0;
+    __syncthreads();
+  }
+  // Then: a key of the lane's, if it is within the bound.  kept has room.
+  __device__ __forceinline__ void keep(uint32_t key, uint32_t vertex, uint2* kept) {
+    const bool stays = key <= bound;
+    const uint64_t mask = __ballot(stays);
+    if (mask == 0) return;
+    const uint32_t below = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+    uint32_t base = 0;
+    if (stays && below == 0) base = atomicAdd(&n, (uint32_t)__popcll(mask));
+    base = __shfl(base, __ffsll((unsigned long long)mask) - 1, kWave);
+    if (stays) kept[base + below] = make_uint2(key, vertex);
+  }
+  // Only the best `wanted` stay (there are more).  For the whole workgroup, between barriers.
+  __device__ __forceinline__ void drop_all_but(uint32_t wanted, uint2* kept, uint32_t* sample_bound) {
+    const uint32_t had = n;
+    const uint64_t last = nth_smallest(
+        [&](auto f) {
+          for (uint32_t i = threadIdx.x; i < had; i += kBinThreads) f(rank_value(kept[i]));
+        },
+        wanted, pick);
+    if (threadIdx.x == 0) {
+      n = 0;
+      const uint32_t edge = (uint32_t)(last >> 32);
+      if (edge < bound) {
+        bound = edge;
+        atomicMin(sample_bound, edge);
+      }
+    }
+    for (uint32_t from = 0; from < had; from += kBinThreads) {
+      const uint32_t i = from + threadIdx.x;
+      const uint2 mine = i < had ? kept[i] : make_uint2(0xFFFFFFFFu, 0xFFFFFFFFu);
+      __syncthreads();  // what is written goes where everything has been read
+      if (rank_value(mine) <= last) kept[atomicAdd(&n, 1u)] = mine;
+    }
+    __syncthreads();
+  }
+};
+
 // A sample without hubs among its transits and with at most this many entries in a workgroup's stretches (a layer whose
 // transits are drawn uniformly) adds them all up at once, in an LDS table of twice as many slots.
 constexpr uint32_t kSparseGroupEntries = 2048;
 
-// The samples that are not ranked in LDS (ranked_layer): the keys of sample `at` of them go to keys + at * keys_per_sample.
+// The samples that are not ranked in LDS (ranked_layer).
 // Two workgroups of 16 wavefronts share a compute unit only at 8 wavefronts per SIMD, which the kernel's attributes ask
 // the compiler for.
-// 500 K vertices, 12 M edges, second layer of 1024 samples of 512 (1.5 M pairs a sample): see the engine's rank_by_keys.
+// 500 K vertices, 12 M edges, second layer of 1024 samples of 512 (1.5 M pairs and 136 pieces a sample): 2.59 ms.  Writing a
+// key for every vertex it took 3.42, and the selection, the collecting and the sorts 1.1 more, where kept_layer_kernel takes
+// 0.04; forming only keys that may be within the bound 3.17, the ids of all of a round's entries under way before the first
+// is used 2.86, starts as bits 2.59.  What bounds it now: the vector ALU is at work 65 % of the time, the rest is the phases of a
+// stretch waiting for each other.
 __global__ __launch_bounds__(kBinThreads, 8) __attribute__((amdgpu_num_vgpr(56))) void collective_mark_binned(
     MergedEdges merged, TransitView tv, int32_t invalid, uint32_t n_samples, const uint32_t* __restrict__ n_marked,
-    const uint32_t* __restrict__ marked, uint32_t bins_per_sample, uint32_t keys_per_sample, DensePieces dense,
-    KeysOnTheWayOut keys_out) {
+    const uint32_t* __restrict__ marked, uint32_t bins_per_sample, DensePieces dense, KeptKeys out) {
   __shared__ __align__(16) uint32_t s_bits[kBinWords];  // where some terms are 0
   __shared__ __align__(16) unsigned long long s_acc[kBinVertices];
   // the sub-ranges that hold entries, in transit order
   __shared__ uint32_t s_start[kMaxLayerTransits + 1];  // first entry of sub-range k among the stretch's entries
-  __shared__ EdgePos_t s_edge[kMaxLayerTransits];      // its first edge
+  __shared__ EdgePos_t s_shift[kMaxLayerTransits];     // its first edge less that
   __shared__ uint32_t s_piece[kMaxLayerTransits];      // the stretch's dense pieces
   __shared__ uint4 s_wave[kBinWaves];
+  __shared__ uint32_t s_starts_here[kBinWaves][2 * kBinAhead];  // where sub-ranges start among a round's entries
+  __shared__ Keeper s_keeper;
   // A workgroup takes kBinsPerGroup consecutive stretches of one sample, one after the other: where a transit's sub-range
   // ends in one stretch it begins in the next, and the end is then only a short gallop away instead of a search of the
   // whole adjacency.  The low stretches hold the hubs and take longest: all samples' first groups start first.
@@ -396,14 +540,22 @@ __global__ __launch_bounds__(kBinThreads, 8) __attribute__((amdgpu_num_vgpr(56))
   const uint32_t s = marked[at];
   const uint32_t first_bin = group * kBinsPerGroup;
   const int32_t* transits = tv.base + (size_t)s * tv.stride;
-  uint32_t* my_keys = keys_out.keys + (size_t)at * keys_per_sample;
+  const uint32_t listing = at * (gridDim.x / n_samples) + group;
+  uint2* const kept = out.kept + (size_t)listing * kKeptEntries;
+  uint32_t* const sample_bound = out.bound + at;
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wave = threadIdx.x >> 6;
-  // tv.count <= kBinThreads: lane i keeps transit i's adjacency and how far the stretches before this one reach into it
-  EdgePos_t my_end = 0, my_reach = 0;
-  uint32_t my_next = 0xFFFFFFFFu;  // destination of edge my_reach; none left: above every vertex
-  int32_t my_hub = -1, my_cut_row = -1;
-  int32_t my_transit = -1;
+  s_keeper.begin(__hip_atomic_load(sample_bound, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  uint32_t n_present = 0;  // of the wavefront
+  // the bits of a lane and those below it, of 64
+  const uint32_t up_to_low = lane < 31u ? (2u << lane) - 1u : 0xFFFFFFFFu;
+  const uint32_t up_to_high = lane < 32u ? 0u : lane < 63u ? (2u << (lane - 32u)) - 1u : 0xFFFFFFFFu;
+  // tv.count <= kBinThreads: lane i keeps transit i and how far the stretches before this one reach into its adjacency
+  int32_t my_transit = -1, my_hub = -1, my_cut_row = -1;
+  EdgePos_t my_reach = 0;
+  // rows that are cut: the end of the coming stretch, fetched one stretch ahead; the others: the destination of edge
+  // my_reach, none left: above every vertex
+  uint32_t my_next = 0xFFFFFFFFu;
   if (threadIdx.x < tv.count) {
     my_transit = transits[threadIdx.x];
     if (my_transit == invalid) my_transit = -1;
@@ -411,23 +563,26 @@ __global__ __launch_bounds__(kBinThreads, 8) __attribute__((amdgpu_num_vgpr(56))
     if (my_transit != -1 && merged.cut_row_of) my_cut_row = merged.cut_row_of[my_transit];
   }
   const bool hubs_among_transits = __syncthreads_or(my_hub >= 0) != 0;
-  const HubCut* my_cuts = merged.cuts + (my_cut_row < 0 ? 0 : (size_t)my_cut_row * (bins_per_sample + 1));
+  auto my_cut = [&](uint32_t bin) { return merged.cuts[(size_t)my_cut_row * (bins_per_sample + 1) + bin].from; };
   if (my_transit != -1) {
-    my_end = merged.row_ptr[my_transit + 1];
-    my_reach = my_cut_row >= 0 ? my_cuts[first_bin].from
-                               : first_edge_from(merged.ids, merged.row_ptr[my_transit], my_end, first_bin * kBinVertices);
-    if (my_cut_row < 0 && my_reach < my_end) my_next = (uint32_t)merged.ids[my_reach];
+    if (my_cut_row >= 0) {
+      my_reach = my_cut(first_bin);
+    } else {
+      const EdgePos_t end = merged.row_ptr[my_transit + 1];
+      my_reach = first_edge_from(merged.ids, merged.row_ptr[my_transit], end, first_bin * kBinVertices);
+      if (my_reach < end) my_next = (uint32_t)merged.ids[my_reach];
+    }
   }
   if (!hubs_among_transits) {
     // The stretches of the workgroup as one: the sums are gathered in an LDS table hashed by vertex (in the room of the
-    // per-vertex sums), the keys of the whole range are written as absent, and the table's vertices then get theirs.
-    // Stretch by stretch, 16 chains of searches, tables and barriers cost a workgroup 130 us for a few hundred entries.
+    // per-vertex sums).  Stretch by stretch, 16 chains of searches, tables and barriers cost a workgroup 130 us for a few
+    // hundred entries.
     const uint32_t group_bins = first_bin + kBinsPerGroup < bins_per_sample ? kBinsPerGroup : bins_per_sample - first_bin;
     const uint32_t v_lo = first_bin * kBinVertices, v_hi = v_lo + group_bins * kBinVertices;
     EdgePos_t stop = my_reach;
-    if (my_cut_row >= 0) stop = my_cuts[first_bin + group_bins].from;
-    else if (my_next < v_hi) stop = first_edge_from(merged.ids, my_reach, my_end, v_hi);
-    const Subranges all = list_subranges((uint32_t)(stop - my_reach), my_reach, tv.count, s_start, s_edge, s_piece, s_wave);
+    if (my_cut_row >= 0) stop = my_cut(first_bin + group_bins);
+    else if (my_next < v_hi) stop = first_edge_from(merged.ids, my_reach, merged.row_ptr[my_transit + 1], v_hi);
+    const Subranges all = list_subranges((uint32_t)(stop - my_reach), my_reach, tv.count, s_start, s_shift, s_piece, s_wave);
     const uint32_t ranges = all.ranges, size = all.entries;
     if (size <= kSparseGroupEntries) {
       constexpr uint32_t kSlots = 2u * kSparseGroupEntries;  // a power of two
@@ -437,8 +592,6 @@ __global__ __launch_bounds__(kBinThreads, 8) __attribute__((amdgpu_num_vgpr(56))
         slot_vertex[i] = 0xFFFFFFFFu;
         slot_sum[i] = 0;
       }
-      uint32_t* out_keys = my_keys + v_lo;
-      for (uint32_t i = threadIdx.x; i < group_bins * kBinVertices; i += kBinThreads) out_keys[i] = kAbsentKey;
       __syncthreads();
       for (uint32_t e = threadIdx.x; e < size; e += kBinThreads) {
         uint32_t lo = 0, hi = ranges;  // the sub-range that holds entry e
@@ -446,7 +599,7 @@ __global__ __launch_bounds__(kBinThreads, 8) __attribute__((amdgpu_num_vgpr(56))
           const uint32_t mid = lo + (hi - lo) / 2;
           if (s_start[mid] <= e) lo = mid; else hi = mid;
         }
-        const EdgePos_t src = s_edge[lo] + (EdgePos_t)(e - s_start[lo]);
+        const EdgePos_t src = (EdgePos_t)e + s_shift[lo];
         const uint32_t local = (uint32_t)merged.ids[src] - v_lo;
         uint32_t slot = (local * 2654435761u) >> 20 & (kSlots - 1u);
         for (;;) {  // at most half of the slots are ever taken
@@ -456,19 +609,31 @@ __global__ __launch_bounds__(kBinThreads, 8) __attribute__((amdgpu_num_vgpr(56))
         }
         atomicAdd(&slot_sum[slot], merged.terms[src]);
       }
-      __syncthreads();  // the table is complete, and the absent keys have been written
+      __syncthreads();  // the table is complete
+      uint32_t here = 0;
       for (uint32_t i = threadIdx.x; i < kSlots; i += kBinThreads) {
         const uint32_t local = slot_vertex[i];
-        if (local == 0xFFFFFFFFu) continue;
-        out_keys[local] = ladies_key_bits(slot_sum[i], ladies_pair_index(keys_out.first_sample + s, keys_out.n_vertices, v_lo + local),
-                                          keys_out.step, keys_out.seed);
+        n_present += (uint32_t)__popcll(__ballot(local != 0xFFFFFFFFu));
+        uint32_t key = kAbsentKey;
+        if (local != 0xFFFFFFFFu)
+          key = s_keeper.count(ladies_key_bits(slot_sum[i], ladies_pair_index(out.first_sample + s, out.n_vertices, v_lo + local),
+                                               out.step, out.seed));
+        here += (uint32_t)__popcll(__ballot(key != kAbsentKey));
+        slot_sum[i] = key;
       }
+      s_keeper.lower_bound_to(out.wanted, here, sample_bound);
+      for (uint32_t i = threadIdx.x; i < kSlots; i += kBinThreads)
+        s_keeper.keep((uint32_t)slot_sum[i], v_lo + slot_vertex[i], kept);
+      if (lane == 0 && n_present != 0) atomicAdd(out.distinct + s, n_present);
+      __syncthreads();
+      if (threadIdx.x == 0) out.n_kept[listing] = s_keeper.n;
       return;
     }
     // too many entries for that: stretch by stretch
     __syncthreads();
   }
-  EdgePos_t cut_after = my_cut_row >= 0 ? my_cuts[first_bin + 1].from : 0;  // the end of the coming stretch, fetched one stretch ahead
+  if (my_cut_row >= 0) my_next = (uint32_t)my_cut(first_bin + 1);
+  uint32_t my_piece = my_hub >= 0 ? dense.piece_of[(size_t)my_hub * bins_per_sample + first_bin] : kNoPiece;
   for (uint32_t bin = first_bin; bin < first_bin + kBinsPerGroup && bin < bins_per_sample; ++bin) {
     const uint32_t v_lo = bin * kBinVertices;
     if (merged.zero_terms)
@@ -479,105 +644,146 @@ __global__ __launch_bounds__(kBinThreads, 8) __attribute__((amdgpu_num_vgpr(56))
     if (my_transit != -1) {
       const uint32_t v_hi = v_lo + kBinVertices;
       if (my_cut_row >= 0) {
-        my_reach = cut_after;
-        if (bin + 2 <= bins_per_sample) cut_after = my_cuts[bin + 2].from;
+        my_reach = (EdgePos_t)my_next;
+        if (bin + 2 <= bins_per_sample) my_next = (uint32_t)my_cut(bin + 2);
       } else if (my_next < v_hi) {  // nothing is fetched where the next edge already lies beyond the stretch
-        my_reach = first_edge_from(merged.ids, my_from, my_end, v_hi);
-        my_next = my_reach < my_end ? (uint32_t)merged.ids[my_reach] : 0xFFFFFFFFu;
+        const EdgePos_t end = merged.row_ptr[my_transit + 1];
+        my_reach = first_edge_from(merged.ids, my_from, end, v_hi);
+        my_next = my_reach < end ? (uint32_t)merged.ids[my_reach] : 0xFFFFFFFFu;
       }
       length = (uint32_t)(my_reach - my_from);
-      if (my_hub >= 0 && length != 0) {
-        const uint32_t piece = dense.piece_of[(size_t)my_hub * bins_per_sample + bin];
-        if (piece != kNoPiece) length = kPieceFlag | piece;  // these entries reach the stretch ready-made
+      // (fetched one stretch ahead)
+      if (my_hub >= 0) {
+        if (length != 0 && my_piece != kNoPiece) length = kPieceFlag | my_piece;  // these entries reach the stretch ready-made
+        if (bin + 1 < bins_per_sample) my_piece = dense.piece_of[(size_t)my_hub * bins_per_sample + bin + 1];
       }
     }
-    const Subranges all = list_subranges(length, my_from, tv.count, s_start, s_edge, s_piece, s_wave);
+    const Subranges all = list_subranges(length, my_from, tv.count, s_start, s_shift, s_piece, s_wave);
+    if (s_keeper.n > kKeptEntries - kBinVertices) s_keeper.drop_all_but(out.wanted, kept, sample_bound);
     const uint32_t ranges = all.ranges, size = all.entries;
-    // every wavefront walks a contiguous part of the entries, 64 * kBinAhead per round
+    // Every wavefront walks a contiguous part of the entries, 64 * kBinAhead per round.  Which sub-range an entry is in: the
+    // starts that fall into a round, at most 63 (a round ends early for more), become bits, and the bits up to an entry are
+    // counted.  (A lane that stepped from sub-range to sub-range for itself took five turns an entry for the slowest of 64, each
+    // a trip to LDS: 2.80 ms instead of 2.59 where collective_mark_binned gives its figures.)
     constexpr uint32_t kRound = 64u * kBinAhead;
+    const uint32_t uniform_wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave);
     const uint32_t part = (size + kBinWaves * kRound - 1) / (kBinWaves * kRound) * kRound;
-    const uint32_t part_begin = wave * part;
-    const uint32_t part_end = part_begin + part < size ? part_begin + part : size;
-    uint32_t cur = 0, cur_begin = 0, cur_end = 0;
-    EdgePos_t cur_edges = 0;
-    if (part_begin + lane < part_end) {  // the sub-range of the lane's first entry
-      const uint32_t e = part_begin + lane;
-      uint32_t lo = 0, hi = ranges;
-      while (hi - lo > 1) {
-        const uint32_t mid = lo + (hi - lo) / 2;
-        if (s_start[mid] <= e) lo = mid; else hi = mid;
+    uint32_t e0 = uniform_wave * part;
+    const uint32_t part_end = e0 + part < size ? e0 + part : size;
+    uint32_t before = 0;  // the sub-range that holds e0, or the one before it where one starts there
+    if (e0 < part_end) {
+      uint32_t hi = ranges;
+      while (hi - before > 1) {
+        const uint32_t mid = before + (hi - before) / 2;
+        if (s_start[mid] <= e0) before = mid; else hi = mid;
       }
-      cur = lo;
-      cur_begin = s_start[lo];
-      cur_end = s_start[lo + 1];
-      cur_edges = s_edge[lo];
+      before = (uint32_t)__builtin_amdgcn_readfirstlane((int)before);
     }
-    for (uint32_t e0 = part_begin; e0 < part_end; e0 += kRound) {
-      uint32_t locals[kBinAhead];  // vertex - v_lo
+    while (e0 < part_end) {
+      const uint32_t start = before + 1u + lane < ranges ? s_start[before + 1u + lane] : 0xFFFFFFFFu;
+      uint32_t end = e0 + kRound < part_end ? e0 + kRound : part_end;
+      const uint32_t last = (uint32_t)__builtin_amdgcn_readlane((int)start, 63);
+      end = last < end ? last : end;
+      const bool falls_here = start < end;
+      if (lane < kRound / 32u) s_starts_here[wave][lane] = 0;
+      __builtin_amdgcn_wave_barrier();
+      if (falls_here) atomicOr(&s_starts_here[wave][(start - e0) >> 5], 1u << ((start - e0) & 31u));
+      __builtin_amdgcn_wave_barrier();
+      // (nothing may be worked out from an id before the last is asked for: the compiler waits for it where that is done)
+      uint32_t ids[kBinAhead];
       unsigned long long terms[kBinAhead];
+      uint32_t of = before;
 #pragma unroll
       for (uint32_t a = 0; a < kBinAhead; ++a) {
+        const uint32_t low = s_starts_here[wave][2u * a], high = s_starts_here[wave][2u * a + 1u];
         const uint32_t e = e0 + a * 64u + lane;
-        locals[a] = 0xFFFFFFFFu;
+        const uint32_t mine = of + (uint32_t)__popc(low & up_to_low) + (uint32_t)__popc(high & up_to_high);
+        of += (uint32_t)__popc(low) + (uint32_t)__popc(high);
+        ids[a] = 0;
         terms[a] = 0;
-        if (e < part_end) {
-          if (e >= cur_end) {
-            do {  // no sub-range is empty
-              ++cur;
-              cur_begin = cur_end;
-              cur_end = s_start[cur + 1];
-            } while (e >= cur_end);
-            cur_edges = s_edge[cur];
-          }
-          const EdgePos_t src = cur_edges + (EdgePos_t)(e - cur_begin);
-          locals[a] = (uint32_t)merged.ids[src] - v_lo;
+        if (e < end) {
+          const EdgePos_t src = (EdgePos_t)e + s_shift[mine];
+          ids[a] = (uint32_t)merged.ids[src];
           terms[a] = merged.terms[src];
         }
       }
 #pragma unroll
       for (uint32_t a = 0; a < kBinAhead; ++a) {
-        if (locals[a] == 0xFFFFFFFFu) continue;
-        atomicAdd(&s_acc[locals[a]], terms[a]);
-        if (merged.zero_terms) atomicOr(&s_bits[locals[a] >> 5], 1u << (locals[a] & 31u));
+        if (e0 + a * 64u + lane >= end) continue;
+        const uint32_t local = ids[a] - v_lo;
+        atomicAdd(&s_acc[local], terms[a]);
+        if (merged.zero_terms) atomicOr(&s_bits[local >> 5], 1u << (local & 31u));
       }
+      before += (uint32_t)__popcll(__ballot(falls_here));
+      e0 = end;
     }
     __syncthreads();
-    // What leaves the workgroup is the sampling key of every vertex of the stretch (kAbsentKey where the neighbourhood
-    // does not hold the vertex).  A lane takes four consecutive vertices: 16-byte accesses to LDS, to the pieces and to
-    // the output, and one Philox block where it forms keys.
+    // The keys of the stretch's vertices.  A lane takes four consecutive vertices: 16-byte accesses to LDS and to the pieces,
+    // and one Philox block where it forms keys.  Most vertices' uniforms are too far from 1 for any importance like theirs:
+    // the two divisions and the logarithm are for the few others.
     const uint32_t n_pieces = all.pieces;
-    for (uint32_t q = threadIdx.x; q < kBinVertices / 4u; q += kBinThreads) {
+    const float reach = s_keeper.reach();
+    uint32_t here = 0, with_keys = 0;  // keys of the wavefront, and in which turns there were any
+    for (uint32_t q = threadIdx.x; q < kBinVertices / 4u; q += kBinThreads) {  // whole wavefronts
       const uint32_t i = 4u * q;
       const ulonglong2 low = ((const ulonglong2*)s_acc)[2u * q], high = ((const ulonglong2*)s_acc)[2u * q + 1u];
       unsigned long long sum[4] = {low.x, low.y, high.x, high.y};  // 0 where nothing was added
       const uint32_t bits = merged.zero_terms ? (s_bits[i >> 5] >> (i & 31u)) & 15u : 0u;
-      bool present[4];
-#pragma unroll
-      for (uint32_t k = 0; k < 4; ++k) present[k] = sum[k] != 0 || (bits >> k & 1u) != 0;
-#pragma unroll 4
-      for (uint32_t p = 0; p < n_pieces; ++p) {
-        const ulonglong2* piece = (const ulonglong2*)(dense.sums + (size_t)s_piece[p] * kBinVertices + i);
-        const ulonglong2 a = piece[0], b = piece[1];
-        const unsigned long long ready[4] = {a.x, a.y, b.x, b.y};
-#pragma unroll
-        for (uint32_t k = 0; k < 4; ++k)
-          if (ready[k] != kAbsentSum) {
-            sum[k] += ready[k];
-            present[k] = true;
-          }
+      // two pieces under way before the first is used
+      const ulonglong2* const pieces = (const ulonglong2*)(dense.sums + i);
+      uint32_t p = 0;
+      for (; p + 1 < n_pieces; p += 2) {
+        const ulonglong2* one = pieces + (size_t)s_piece[p] * (kBinVertices / 2u);
+        const ulonglong2* two = pieces + (size_t)s_piece[p + 1] * (kBinVertices / 2u);
+        const ulonglong2 a = one[0], b = one[1], c = two[0], d = two[1];
+        sum[0] += a.x + c.x;
+        sum[1] += a.y + c.y;
+        sum[2] += b.x + d.x;
+        sum[3] += b.y + d.y;
       }
+      if (p < n_pieces) {
+        const ulonglong2* one = pieces + (size_t)s_piece[p] * (kBinVertices / 2u);
+        const ulonglong2 a = one[0], b = one[1];
+        sum[0] += a.x;
+        sum[1] += a.y;
+        sum[2] += b.x;
+        sum[3] += b.y;
+      }
+#pragma unroll
+      for (uint32_t k = 0; k < 4; ++k) n_present += (uint32_t)__popcll(__ballot(sum[k] != 0 || (bits >> k & 1u) != 0));
+      const PhiloxBlock blk = ladies_block(ladies_pair_index(out.first_sample + s, out.n_vertices, v_lo + i), out.step, out.seed);
+      bool may[4];
+#pragma unroll
+      for (uint32_t k = 0; k < 4; ++k) may[k] = key_may_be_within(reach, sum[k], blk.w[k]);
       uint32_t key[4] = {kAbsentKey, kAbsentKey, kAbsentKey, kAbsentKey};
-      if (present[0] || present[1] || present[2] || present[3]) {
-        const PhiloxBlock blk = ladies_block(ladies_pair_index(keys_out.first_sample + s, keys_out.n_vertices, v_lo + i),
-                                             keys_out.step, keys_out.seed);
+      if (may[0] || may[1] || may[2] || may[3]) {
 #pragma unroll
         for (uint32_t k = 0; k < 4; ++k)
-          if (present[k]) key[k] = ladies_key_from_word(sum[k], blk.w[k]);
+          if (may[k] && (sum[k] != 0 || (bits >> k & 1u) != 0)) key[k] = s_keeper.count(ladies_key_from_word(sum[k], blk.w[k]));
       }
-      *(uint4*)(my_keys + v_lo + i) = make_uint4(key[0], key[1], key[2], key[3]);
+      uint32_t keys_here = 0;
+#pragma unroll
+      for (uint32_t k = 0; k < 4; ++k) keys_here += (uint32_t)__popcll(__ballot(key[k] != kAbsentKey));
+      here += keys_here;
+      if (keys_here != 0) ((uint4*)s_acc)[2u * q] = make_uint4(key[0], key[1], key[2], key[3]);  // in the sums' room
+      with_keys |= (keys_here != 0 ? 1u : 0u) << q / kBinThreads;
     }
+    s_keeper.lower_bound_to(out.wanted, here, sample_bound);
+    if (with_keys != 0)
+      for (uint32_t q = threadIdx.x; q < kBinVertices / 4u; q += kBinThreads) {
+        if ((with_keys >> q / kBinThreads & 1u) == 0) continue;
+        const uint4 key = ((const uint4*)s_acc)[2u * q];
+        const uint32_t v = v_lo + 4u * q;
+        s_keeper.keep(key.x, v, kept);
+        s_keeper.keep(key.y, v + 1u, kept);
+        s_keeper.keep(key.z, v + 2u, kept);
+        s_keeper.keep(key.w, v + 3u, kept);
+      }
     __syncthreads();  // the next stretch clears what this one has just read
   }
+  if (lane == 0 && n_present != 0) atomicAdd(out.distinct + s, n_present);
+  __syncthreads();
+  if (threadIdx.x == 0) out.n_kept[listing] = s_keeper.n;
 }
 
 // ---- LADIES form: small neighbourhoods, ranked in LDS -------------------------------------
@@ -593,6 +799,7 @@ __global__ __launch_bounds__(kSortOutThreads) void sort_out_ranked(CSRPartition 
                                                                    uint32_t* __restrict__ sizes,
                                                                    uint32_t* __restrict__ merged_sizes,
                                                                    uint32_t* n_marked, uint32_t* __restrict__ marked,
+                                                                   uint32_t* __restrict__ distinct, uint32_t* __restrict__ bound,
                                                                    uint32_t* __restrict__ too_long) {
   __shared__ uint32_t s_taken, s_base;
   const uint32_t lane = threadIdx.x & 63u;
@@ -619,7 +826,11 @@ __global__ __launch_bounds__(kSortOutThreads) void sort_out_ranked(CSRPartition 
   __syncthreads();
   if (threadIdx.x == 0 && s_taken) s_base = atomicAdd(n_marked, s_taken);
   __syncthreads();
-  if (lane == 0 && s < n_samples && pairs > kRankedEntries) marked[s_base + at] = s;
+  if (lane == 0 && s < n_samples && pairs > kRankedEntries) {
+    marked[s_base + at] = s;
+    bound[s_base + at] = kNoBound;
+    distinct[s] = 0;
+  }
 }
 
 // A workgroup per sample: fetches the entries, sorts them by vertex, adds their terms up, forms the keys and sorts the
@@ -744,191 +955,6 @@ __global__ void build_item_counts(const uint32_t* __restrict__ sizes, uint32_t n
   }
 }
 
-__global__ void gather_u32(const uint32_t* __restrict__ table, const uint32_t* __restrict__ index, size_t n,
-                           uint32_t* __restrict__ out, uint32_t* __restrict__ index_copy) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t p = index[i];
-  out[i] = table[p];
-  if (index_copy) index_copy[i] = p;
-}
-
-__global__ void fill_u32(uint32_t* dst, size_t n, uint32_t value) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dst[i] = value;
-}
-
-// ---- the best m keys of every sample, without sorting everything ----
-//
-// Only the first stepSize ranked vertices of a sample are ever read, out of up to millions of
-// distinct ones.  A radix select on the upper 14 bits of the sort key finds, per sample, the
-// smallest prefix T such that at least m keys have a prefix <= T; the entries with a prefix
-// <= T (m and some more) are copied out and only those are sorted.
-// The keys of a chunk are dense: keys[s * keys_per_sample + v] for every vertex v (kAbsentKey
-// where sample s does not hold v), so position tells sample and vertex and no list of the
-// distinct pairs is ever written.
-
-// One workgroup per sample, one pass over its keys: counts the present ones by their upper
-// kSelectBits bits in an LDS
-// histogram and picks the bin that holds the wanted-th smallest key: threshold[s] = that bin,
-// kept[s] = keys up to and including it (a sample with fewer keys than wanted keeps them all),
-// distinct[its number] = all its keys.  A sample's whole histogram stays in the workgroup: no atomic
-// reaches memory, and no second pass over the keys refines the threshold (two levels of 8 bits,
-// counted by a workgroup per tile of 8192 keys, read every key twice).
-constexpr uint32_t kSelectBits = 14;
-constexpr uint32_t kSelectBins = 1u << kSelectBits;
-constexpr uint32_t kSelectThreads = 1024;
-// The pass also notes, for every stretch of 256 consecutive keys (what a wavefront handles at a
-// time, four keys per lane), the smallest prefix in it: the copying of the kept entries then
-// reads only the stretches that hold one (a few hundred of a sample's 12,000).
-constexpr uint32_t kCollectStretch = 256;
-__device__ __forceinline__ void note_best_of_stretch(const uint32_t (&key)[4], uint32_t quad, uint32_t lane,
-                                                     uint16_t* __restrict__ best_of) {
-  uint32_t a = key[0] < key[1] ? key[0] : key[1], b = key[2] < key[3] ? key[2] : key[3];
-  uint32_t best = (a < b ? a : b) >> (32u - kSelectBits);  // kAbsentKey: the largest prefix
-  // minimum of the wavefront into lane 63, on the VALU (DPP): along the rows of 16 lanes, then
-  // the last lane of a row into the next row, then lane 31 into the upper half
-  const uint32_t none = 0xFFFFFFFFu;
-  uint32_t other = row_shift_up<1>(none, best);
-  best = other < best ? other : best;
-  other = row_shift_up<2>(none, best);
-  best = other < best ? other : best;
-  other = row_shift_up<4>(none, best);
-  best = other < best ? other : best;
-  other = row_shift_up<8>(none, best);
-  best = other < best ? other : best;
-  other = (uint32_t)__builtin_amdgcn_update_dpp((int)none, (int)best, 0x142, 0xA, 0xF, false);  // row_bcast:15
-  best = other < best ? other : best;
-  other = (uint32_t)__builtin_amdgcn_update_dpp((int)none, (int)best, 0x143, 0xC, 0xF, false);  // row_bcast:31
-  best = other < best ? other : best;
-  if (lane == 63) best_of[quad / 64u] = (uint16_t)best;
-}
-__global__ __launch_bounds__(kSelectThreads, 8) __attribute__((amdgpu_num_vgpr(56))) void select_threshold(
-    const uint32_t* __restrict__ keys, uint32_t keys_per_sample, uint32_t wanted, const uint32_t* __restrict__ n_marked,
-    const uint32_t* __restrict__ marked, uint32_t* __restrict__ threshold, uint32_t* __restrict__ kept,
-    uint32_t* __restrict__ claimed, uint32_t* __restrict__ distinct, uint16_t* __restrict__ stretch_best) {
-  __shared__ uint32_t s_hist[kSelectBins];
-  __shared__ uint32_t s_wave_total[kSelectThreads / 64];
-  const uint32_t s = blockIdx.x;
-  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-  if (threadIdx.x == 0) claimed[s] = 0;  // for select_collect
-  if (s >= *n_marked) {
-    if (threadIdx.x == 0) kept[s] = 0;
-    return;
-  }
-  for (uint32_t i = threadIdx.x; i < kSelectBins; i += kSelectThreads) s_hist[i] = 0;
-  __syncthreads();
-  const uint32_t* mine = keys + (size_t)s * keys_per_sample;
-  uint16_t* my_best = stretch_best + (size_t)s * (keys_per_sample / kCollectStretch);
-  {
-    const uint4* my_keys = (const uint4*)mine;
-    for (uint32_t q0 = 0; q0 < keys_per_sample / 4u; q0 += 4 * kSelectThreads) {
-      uint4 batch[4];
-#pragma unroll
-      for (uint32_t k = 0; k < 4; ++k) {
-        const uint32_t q = q0 + k * kSelectThreads + threadIdx.x;
-        batch[k] = q < keys_per_sample / 4u ? my_keys[q] : make_uint4(kAbsentKey, kAbsentKey, kAbsentKey, kAbsentKey);
-      }
-#pragma unroll
-      for (uint32_t k = 0; k < 4; ++k) {
-        const uint32_t q = q0 + k * kSelectThreads + threadIdx.x;
-        if (q >= keys_per_sample / 4u) continue;  // whole wavefronts: the sample holds a multiple of 256 keys
-        const uint32_t key[4] = {batch[k].x, batch[k].y, batch[k].z, batch[k].w};
-#pragma unroll
-        for (uint32_t i = 0; i < 4; ++i)
-          if (key[i] != kAbsentKey) atomicAdd(&s_hist[key[i] >> (32u - kSelectBits)], 1u);
-        note_best_of_stretch(key, q, lane, my_best);
-      }
-    }
-  }
-  __syncthreads();
-  // lane t owns bins [16 t, 16 t + 16): the bin in which the running count reaches `wanted`
-  constexpr uint32_t kOwn = kSelectBins / kSelectThreads;
-  uint32_t own = 0;
-#pragma unroll
-  for (uint32_t b = 0; b < kOwn; ++b) own += s_hist[threadIdx.x * kOwn + b];
-  const uint32_t through_wave = wave_inclusive_scan(own);
-  if (lane == 63) s_wave_total[wave] = through_wave;
-  __syncthreads();
-  uint32_t before = through_wave - own, total = 0;
-#pragma unroll
-  for (uint32_t w = 0; w < kSelectThreads / 64; ++w) {
-    const uint32_t t = s_wave_total[w];
-    if (w < wave) before += t;
-    total += t;
-  }
-  if (threadIdx.x == 0) distinct[marked[s]] = total;
-  if (total < wanted) {  // everything stays
-    if (threadIdx.x == 0) {
-      threshold[s] = kSelectBins - 1u;
-      kept[s] = total;
-    }
-  } else if (before < wanted && before + own >= wanted) {  // exactly one lane
-    uint32_t running = before;
-    for (uint32_t b = 0; b < kOwn; ++b) {
-      running += s_hist[threadIdx.x * kOwn + b];
-      if (running >= wanted) {
-        threshold[s] = threadIdx.x * kOwn + b;
-        kept[s] = running;
-        break;
-      }
-    }
-  }
-}
-
-__device__ __forceinline__ bool select_keeps(uint32_t key, uint32_t threshold) {
-  return key != kAbsentKey && (key >> (32u - kSelectBits)) <= threshold;
-}
-
-// Copies the kept entries of sample s into its part [ranked_start[s], ranked_start[s + 1]) of
-// kept_key / kept_id, in whatever order the wavefronts get there (a wavefront claims room for
-// the entries of a round with one atomic).  A few hundred of a sample's millions of keys stay:
-// one workgroup per sample, whose wavefronts look at the best prefix of each stretch of 256 keys
-// first and read only those that hold a kept key.  The sorts that follow fix the order.
-__global__ __launch_bounds__(kSelectThreads) void select_collect(const uint32_t* __restrict__ keys,
-                                                                 uint32_t keys_per_sample,
-                                                                 const uint16_t* __restrict__ stretch_best,
-                                                      const uint32_t* __restrict__ threshold_of,
-                                                      const uint32_t* __restrict__ ranked_start,
-                                                      uint32_t* __restrict__ claimed, uint32_t* __restrict__ kept_key,
-                                                      uint32_t* __restrict__ kept_sample, int32_t* __restrict__ kept_id) {
-  const uint32_t s = blockIdx.x;
-  const uint32_t* mine = keys + (size_t)s * keys_per_sample;
-  const uint32_t stretches = keys_per_sample / kCollectStretch;
-  const uint16_t* best_of = stretch_best + (size_t)s * stretches;
-  const uint32_t threshold = threshold_of[s];
-  const uint32_t first = ranked_start[s];
-  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-  // a wavefront looks at 64 stretches at a time: lane i knows whether stretch i holds a kept key
-  for (uint32_t stretch_begin = wave * 64u; stretch_begin < stretches; stretch_begin += (kSelectThreads / 64u) * 64u) {
-    const uint32_t my_stretch = stretch_begin + lane;
-    const bool holds = my_stretch < stretches && best_of[my_stretch] <= threshold;
-    uint64_t todo = __ballot(holds);
-    while (todo) {  // the same for every lane
-      const uint32_t stretch = stretch_begin + (uint32_t)__ffsll((long long)todo) - 1u;
-      todo &= todo - 1ull;
-      const uint32_t v0 = stretch * kCollectStretch + lane * 4u;
-      const uint4 four = *(const uint4*)(mine + v0);
-      const uint32_t key[4] = {four.x, four.y, four.z, four.w};
-#pragma unroll
-      for (uint32_t i = 0; i < 4; ++i) {
-        const bool stays = select_keeps(key[i], threshold);
-        const uint64_t mask = __ballot(stays);
-        if (mask == 0) continue;
-        uint32_t base = 0;
-        if (lane == (uint32_t)__ffsll((long long)mask) - 1u) base = atomicAdd(&claimed[s], (uint32_t)__popcll(mask));
-        base = __shfl(base, __ffsll((long long)mask) - 1, kWave);
-        if (stays) {
-          const uint32_t at = first + base + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
-          kept_key[at] = key[i];
-          kept_sample[at] = s;
-          kept_id[at] = (int32_t)(v0 + i);
-        }
-      }
-    }
-  }
-}
-
 struct LayerParams {
   CSRPartition csr;
   TransitView transits;   // base already points at the first sample of the chunk
@@ -947,22 +973,15 @@ struct LayerParams {
   const uint32_t* offsets;
   const int32_t* nbr_cols;
   const float* nbr_weights;
-  // kRankedByLadiesImportance: the kept ids of sample ls in descending key order are
-  // ranked_ids[ranked_start[at] .. ranked_start[at + 1]) for marked[at] == ls, at < n_marked
-  const uint32_t* ranked_start;
-  const int32_t* ranked_ids;
-  const uint32_t* marked;
-  uint32_t n_marked;
 };
 
+// The draws of kConcatenated.
 template <class SampleType, class App>
 __global__ __launch_bounds__(256) void layer_execute_kernel(LayerParams P) {
   const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-  constexpr bool ranked_form = apps::neighborhood_form_of<App>::value == apps::kRankedByLadiesImportance;
-  if (i >= (uint64_t)(ranked_form ? P.n_marked : P.chunk_samples) * P.step_size) return;
-  const uint32_t at = (uint32_t)(i / P.step_size);
-  const uint32_t nbr = (uint32_t)(i - (uint64_t)at * P.step_size);
-  const uint32_t ls = ranked_form ? P.marked[at] : at;  // sample inside the chunk
+  if (i >= (uint64_t)P.chunk_samples * P.step_size) return;
+  const uint32_t ls = (uint32_t)(i / P.step_size);  // sample inside the chunk
+  const uint32_t nbr = (uint32_t)(i - (uint64_t)ls * P.step_size);
   const uint32_t s = P.sample_begin + ls;
   CSRPartition csr = P.csr;
   const int32_t* transits = P.transits.base + (size_t)ls * P.transits.stride;
@@ -972,24 +991,14 @@ __global__ __launch_bounds__(256) void layer_execute_kernel(LayerParams P) {
   rng.reset(P.seed, (P.first_sample + s) * P.step_size + nbr, (uint32_t)P.step);
   const VertexID sample_id = (VertexID)(P.first_sample + s);
   VertexID neighbor = P.invalid;
-  if constexpr (apps::neighborhood_form_of<App>::value == apps::kConcatenated) {
-    // only the first transit decides whether next() runs (nextdoor.cu:1421)
-    if (transits[0] != P.invalid && transits[0] != -1) {
-      const uint32_t begin = P.offsets[ls];
-      const CSR::Edge* edges = P.nbr_cols + begin;
-      const float* weights = P.nbr_weights + begin;
-      const VertexID r = App().template next<SampleType, const CSR::Edge*, const float*>(
-          P.step, &csr, transits, sample_id, state, 0.0f, edges, weights, (EdgePos_t)(P.offsets[ls + 1] - begin),
-          (VertexID_t)nbr, &rng);
-      neighbor = r == -1 ? P.invalid : r;
-    }
-  } else {
-    const uint32_t begin = P.ranked_start[at];
-    const CSR::Edge* ranked = P.ranked_ids + begin;
-    const float* no_weights = nullptr;
+  // only the first transit decides whether next() runs (nextdoor.cu:1421)
+  if (transits[0] != P.invalid && transits[0] != -1) {
+    const uint32_t begin = P.offsets[ls];
+    const CSR::Edge* edges = P.nbr_cols + begin;
+    const float* weights = P.nbr_weights + begin;
     const VertexID r = App().template next<SampleType, const CSR::Edge*, const float*>(
-        P.step, &csr, transits, sample_id, state, 0.0f, ranked, no_weights,
-        (EdgePos_t)(P.ranked_start[at + 1] - begin), (VertexID_t)nbr, &rng);
+        P.step, &csr, transits, sample_id, state, 0.0f, edges, weights, (EdgePos_t)(P.offsets[ls + 1] - begin),
+        (VertexID_t)nbr, &rng);
     neighbor = r == -1 ? P.invalid : r;
   }
   P.final_samples[(size_t)s * P.final_size + P.out_base + nbr] = neighbor;
@@ -1036,6 +1045,87 @@ __global__ __launch_bounds__(kRankedThreads) void ranked_layer_kernel(LayerParam
                  for (uint32_t nbr = threadIdx.x; nbr < P.step_size; nbr += kRankedThreads)
                    draw_from<SampleType, App>(P, ls, nbr, ranked, n_distinct);
                });
+}
+
+// A workgroup per marked sample: the best of what the workgroups of collective_mark_binned have kept of it, in order, and the
+// draws.  An edge between counts first, as there, over all of them together; where more are at or below it than there is room
+// for (many equal keys), the wanted ones are picked out exactly.  1024 samples of 512, five workgroups' keys each: 0.03 ms.
+constexpr uint32_t kBestEntries = 2048;
+template <class SampleType, class App>
+__global__ __launch_bounds__(kBinThreads) void kept_layer_kernel(LayerParams P, const uint32_t* __restrict__ n_marked,
+                                                                 const uint32_t* __restrict__ marked, uint32_t groups,
+                                                                 KeptKeys in) {
+  __shared__ uint64_t s_best[kBestEntries];
+  __shared__ int32_t s_ids[kBestEntries];
+  __shared__ uint32_t s_counts[kBoundBins];
+  __shared__ uint32_t s_wave_total[kBinWaves];
+  __shared__ uint64_t s_last;
+  __shared__ uint32_t s_through, s_n;
+  __shared__ PickScratch s_pick;
+  const uint32_t at = blockIdx.x;
+  if (at >= *n_marked) return;
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  const uint32_t bound = in.bound[at];
+  auto each = [&](auto f) {
+    for (uint32_t g = 0; g < groups; ++g) {
+      const uint32_t listing = at * groups + g, n = in.n_kept[listing];
+      const uint2* kept = in.kept + (size_t)listing * kKeptEntries;
+      for (uint32_t i = threadIdx.x; i < n; i += kBinThreads) {
+        const uint2 mine = kept[i];
+        if (mine.x <= bound) f(rank_value(mine));
+      }
+    }
+  };
+  s_counts[threadIdx.x] = 0;
+  if (threadIdx.x == 0) s_n = 0;
+  __syncthreads();
+  each([&](uint64_t value) { atomicAdd(&s_counts[bin_of_key((uint32_t)(value >> 32))], 1u); });
+  __syncthreads();
+  const uint32_t own = s_counts[threadIdx.x], through_wave = wave_inclusive_scan(own);
+  if (lane == 63) s_wave_total[wave] = through_wave;
+  __syncthreads();
+  uint32_t through = through_wave;
+  for (uint32_t w = 0; w < wave; ++w) through += s_wave_total[w];
+  if (threadIdx.x == kBinThreads - 1 && through < in.wanted) {  // all of them
+    s_last = ~0ull;
+    s_through = through;
+  }
+  if (through - own < in.wanted && through >= in.wanted) {  // else one lane
+    s_last = (uint64_t)last_key_of_bin(threadIdx.x) << 32 | 0xFFFFFFFFu;
+    s_through = through;
+  }
+  __syncthreads();
+  uint64_t last = s_last;
+  uint32_t n = s_through;
+  if (n > kBestEntries) {
+    last = nth_smallest(each, in.wanted, s_pick);
+    n = in.wanted;
+  }
+  each([&](uint64_t value) {
+    if (value <= last) s_best[atomicAdd(&s_n, 1u)] = value;
+  });
+  uint32_t padded = 64;
+  while (padded < n) padded *= 2u;
+  __syncthreads();
+  for (uint32_t i = n + threadIdx.x; i < padded; i += kBinThreads) s_best[i] = ~0ull;
+  __syncthreads();
+  for (uint32_t size = 2; size <= padded; size *= 2u) {
+    for (uint32_t stride = size / 2u; stride != 0; stride /= 2u) {
+      for (uint32_t i = threadIdx.x; i < padded / 2u; i += kBinThreads) {
+        const uint32_t a = (i / stride) * 2u * stride + i % stride, b = a + stride;
+        const uint64_t x = s_best[a], y = s_best[b];
+        if ((x > y) == ((a & size) == 0)) {
+          s_best[a] = y;
+          s_best[b] = x;
+        }
+      }
+      __syncthreads();
+    }
+  }
+  for (uint32_t i = threadIdx.x; i < n; i += kBinThreads) s_ids[i] = (int32_t)(uint32_t)s_best[i];
+  __syncthreads();
+  const CSR::Edge* ranked = (const CSR::Edge*)s_ids;
+  for (uint32_t nbr = threadIdx.x; nbr < P.step_size; nbr += kBinThreads) draw_from<SampleType, App>(P, marked[at], nbr, ranked, n);
 }
 
 // The draws of the marked samples, a lane each, the workgroups of the grid in turn.
@@ -1163,13 +1253,10 @@ class LayerEngine : public EngineBase {
     // to whole stretches (LADIES form)
     uint64_t bytes_per_sample = (uint64_t)bitmap_words_ * sizeof(uint32_t);
     if (apps::neighborhood_form_of<App>::value == apps::kRankedByLadiesImportance) {
-      bytes_per_sample = (uint64_t)((bitmap_words_ + kBinWords - 1) / kBinWords) * kBinVertices * sizeof(uint32_t);
+      bytes_per_sample = (uint64_t)ladies_groups() * kKeptEntries * sizeof(uint2);
     }
     const uint64_t fit = kBitmapBudgetBytes / bytes_per_sample;
     bitmap_chunk_samples_ = fit < 1 ? 1u : fit > (uint64_t)n_samples_ ? (uint32_t)n_samples_ : (uint32_t)fit;
-    // the selection kernels of the LADIES form index the samples of a chunk by blockIdx.y
-    if (apps::neighborhood_form_of<App>::value == apps::kRankedByLadiesImportance && bitmap_chunk_samples_ > 65535u)
-      bitmap_chunk_samples_ = 65535u;
 
     ND_HIP_TRY(hipStreamCreate(&stream_));
     ND_HIP_TRY(hipEventCreate(&ev_begin_));
@@ -1200,7 +1287,7 @@ class LayerEngine : public EngineBase {
     ND_HIP_TRY(hipMalloc(&d_small_scratch_, sizeof(uint32_t) * scan_scratch_elems((size_t)n_samples_ + 1)));
     if (apps::neighborhood_form_of<App>::value != apps::kConcatenated) {
       ND_HIP_TRY(hipMalloc(&d_layer_counts_, sizeof(uint32_t) * 2 * (size_t)n_samples_ * n_steps));
-      ND_HIP_TRY(hipHostMalloc((void**)&h_too_long_, 3 * sizeof(uint32_t), hipHostMallocDefault));
+      ND_HIP_TRY(hipHostMalloc((void**)&h_too_long_, sizeof(uint32_t), hipHostMallocDefault));
       *h_too_long_ = 0;
       ND_HIP_TRY(hipMalloc(&marked_.count, 2 * sizeof(uint32_t)));
       ND_HIP_TRY(hipMalloc(&marked_.sample, sizeof(uint32_t) * (size_t)n_samples_));
@@ -1212,10 +1299,6 @@ class LayerEngine : public EngineBase {
     }
     if (apps::neighborhood_form_of<App>::value == apps::kRankedByLadiesImportance) {
       const size_t per_sample = sizeof(uint32_t) * ((size_t)n_samples_ + 1);
-      ND_HIP_TRY(hipMalloc(&d_ranked_start_, per_sample));
-      ND_HIP_TRY(hipMalloc(&d_select_kept_, per_sample));
-      ND_HIP_TRY(hipMalloc(&d_select_threshold_, per_sample));
-      ND_HIP_TRY(hipMalloc(&d_select_claimed_, per_sample));
       ND_HIP_TRY(hipMalloc(&d_merged_sizes_, per_sample));
     }
     return 0;
@@ -1439,7 +1522,7 @@ class LayerEngine : public EngineBase {
     const size_t most_pieces = kDensePieceBudgetBytes / (sizeof(uint64_t) * kBinVertices);
     std::vector<int32_t> hub_row(V, -1);
     std::vector<uint32_t> piece_of;
-    std::vector<unsigned long long> sums;
+    std::vector<unsigned long long> sums, piece(kBinVertices);
     size_t n_hubs = 0, n_pieces = 0;
     for (uint32_t v = 0; v < V; ++v) {
       const int32_t* const row = graph->col.data() + graph->row_ptr[v];
@@ -1456,20 +1539,20 @@ class LayerEngine : public EngineBase {
           for (const int32_t* c = first + 1; c < stop; ++c) neighbours += c[0] != c[-1];
         }
         if (neighbours >= threshold && n_pieces < most_pieces) {
-          if (hub_row[v] < 0) {
-            hub_row[v] = (int32_t)n_hubs++;
-            piece_of.resize(n_hubs * stretches, kNoPiece);
-          }
-          piece_of[(size_t)hub_row[v] * stretches + b] = (uint32_t)n_pieces;
-          sums.resize((n_pieces + 1) * kBinVertices, kAbsentSum);
-          unsigned long long* of = sums.data() + n_pieces * kBinVertices;
+          std::fill(piece.begin(), piece.end(), 0ull);
           for (const int32_t* c = first; c < stop; ++c) {
             // the term of this edge, in the arithmetic of merge_edges
             const float p = graph->weight[(size_t)graph->row_ptr[v] + (size_t)(c - row)] * inverse_row_sums[v];
-            unsigned long long& sum = of[(uint32_t)*c - b * kBinVertices];
-            sum = (sum == kAbsentSum ? 0 : sum) + importance_term_fixed(p * p);
+            piece[(uint32_t)*c - b * kBinVertices] += importance_term_fixed(p * p);
           }
-          ++n_pieces;
+          if (std::all_of(first, stop, [&](int32_t c) { return piece[(uint32_t)c - b * kBinVertices] != 0; })) {
+            if (hub_row[v] < 0) {
+              hub_row[v] = (int32_t)n_hubs++;
+              piece_of.resize(n_hubs * stretches, kNoPiece);
+            }
+            piece_of[(size_t)hub_row[v] * stretches + b] = (uint32_t)n_pieces++;
+            sums.insert(sums.end(), piece.begin(), piece.end());
+          }
         }
         first = stop;
       }
@@ -1622,19 +1705,17 @@ class LayerEngine : public EngineBase {
     return 0;
   }
 
-  // LADIES form: small neighbourhoods are ranked by a workgroup each.  The others leave one sampling key per (sample,
-  // vertex); per sample, the vertices that can be among its first `wanted` in key order are picked by a radix select on the
-  // upper 14 bits of the key and ordered by descending key.  Their distinct pairs (2.4 M per batch at full size) are
-  // never listed.
+  // LADIES form: small neighbourhoods are ranked by a workgroup each, in LDS.  Of the others every workgroup of the marking
+  // keeps the keys that can be among the sample's first, and one more workgroup a sample puts those together.
   int run_ranked(LayerParams P, int step) {
     const uint32_t n = P.chunk_samples;
-    const uint32_t bins = (bitmap_words_ + kBinWords - 1) / kBinWords, groups = (bins + kBinsPerGroup - 1) / kBinsPerGroup;
+    const uint32_t bins = ladies_bins(), groups = ladies_groups();
     if ((uint64_t)n * groups >= (1ull << 31)) { last_error = "a chunk needs 2^31 or more workgroups"; return -1; }
-    const uint32_t keys_per_sample = bins * kBinVertices;
     if (n > bitmap_samples_) {
-      release(d_keys_dense_); release(d_stretch_best_);
-      ND_HIP_TRY(hipMalloc(&d_keys_dense_, sizeof(uint32_t) * (size_t)n * keys_per_sample));
-      ND_HIP_TRY(hipMalloc(&d_stretch_best_, sizeof(uint16_t) * (size_t)n * (keys_per_sample / kCollectStretch)));
+      release(d_kept_); release(d_n_kept_); release(d_bound_);
+      ND_HIP_TRY(hipMalloc(&d_kept_, sizeof(uint2) * kKeptEntries * (size_t)n * groups));
+      ND_HIP_TRY(hipMalloc(&d_n_kept_, sizeof(uint32_t) * (size_t)n * groups));
+      ND_HIP_TRY(hipMalloc(&d_bound_, sizeof(uint32_t) * (size_t)n));
       bitmap_samples_ = n;
     }
     const size_t S = (size_t)n_samples_;
@@ -1642,93 +1723,29 @@ class LayerEngine : public EngineBase {
     uint32_t* distinct = sizes + S * App().steps();
     ND_HIP_TRY(hipMemsetAsync(marked_.count, 0, sizeof(uint32_t), stream_));
     sort_out_ranked<<<dim3((n + 15) / 16), dim3(kSortOutThreads), 0, stream_>>>(
-        P.csr, merged_, P.transits, n, invalid_, sizes, d_merged_sizes_, marked_.count, marked_.sample, h_too_long_);
+        P.csr, merged_, P.transits, n, invalid_, sizes, d_merged_sizes_, marked_.count, marked_.sample, distinct, d_bound_,
+        h_too_long_);
     tick();
     ranked_layer_kernel<SampleType, App><<<dim3(n), dim3(kRankedThreads), 0, stream_>>>(P, merged_, d_merged_sizes_, distinct);
-    KeysOnTheWayOut keys_out;
-    keys_out.keys = d_keys_dense_;
-    keys_out.seed = seed_;
-    keys_out.first_sample = P.first_sample + P.sample_begin;
-    keys_out.step = (uint32_t)step;
-    keys_out.n_vertices = (uint32_t)invalid_;
+    KeptKeys kept;
+    kept.kept = d_kept_;
+    kept.n_kept = d_n_kept_;
+    kept.bound = d_bound_;
+    kept.distinct = distinct;
+    kept.seed = seed_;
+    kept.first_sample = P.first_sample + P.sample_begin;
+    kept.step = (uint32_t)step;
+    kept.n_vertices = (uint32_t)invalid_;
+    kept.wanted = P.step_size;
     collective_mark_binned<<<dim3(n * groups), dim3(kBinThreads), 0, stream_>>>(
-        merged_, P.transits, invalid_, n, marked_.count, marked_.sample, bins, keys_per_sample, dense_, keys_out);
+        merged_, P.transits, invalid_, n, marked_.count, marked_.sample, bins, dense_, kept);
     tock();
-    const uint32_t wanted = (uint32_t)App().stepSize(step);
-    select_threshold<<<dim3(n), dim3(kSelectThreads), 0, stream_>>>(d_keys_dense_, keys_per_sample, wanted, marked_.count,
-                                                                    marked_.sample, d_select_threshold_, d_select_kept_,
-                                                                    d_select_claimed_, distinct, d_stretch_best_);
-    // where every sample's ranked list starts: exclusive scan of the kept counts
-    fill_u32<<<dim3(1), dim3(1), 0, stream_>>>(d_select_kept_ + n, 1, 0u);
-    ND_HIP_TRY(exclusive_scan_u32(d_select_kept_, d_ranked_start_, (size_t)n + 1, d_small_scratch_, stream_));
-    ND_HIP_TRY(hipMemcpyAsync(h_too_long_ + 1, marked_.count, sizeof(uint32_t), hipMemcpyDeviceToHost, stream_));
-    ND_HIP_TRY(hipMemcpyAsync(h_too_long_ + 2, d_small_scratch_ + scan_num_tiles((size_t)n + 1), sizeof(uint32_t),
-                              hipMemcpyDeviceToHost, stream_));
-    ND_HIP_TRY(hipStreamSynchronize(stream_));
-    const uint32_t n_marked = h_too_long_[1], n_kept = h_too_long_[2];
-    if (n_marked == 0) return 0;
-    if (ensure_distinct_capacity(n_kept) != 0) return -1;
-    select_collect<<<dim3(n_marked), dim3(kSelectThreads), 0, stream_>>>(
-        d_keys_dense_, keys_per_sample, d_stretch_best_, d_select_threshold_, d_ranked_start_, d_select_claimed_, d_kept_key_,
-        d_kept_sample_, d_kept_id_);
-    // order the kept vertices of every sample by descending key, equal keys by ascending
-    // vertex id: stable sorts by vertex, then by key, then by sample
-    if (n_kept > 0) {
-      int chunk_bits = 1;
-      while (((uint64_t)n >> chunk_bits) != 0) chunk_bits++;
-      const unsigned blocks = (n_kept + 255) / 256;
-      const SortPlan by_vertex = make_sort_plan(n_kept, max_bits_);
-      uint32_t *k2 = nullptr, *j2 = nullptr;
-      ND_HIP_TRY(radix_sort_pairs(by_vertex, (const uint32_t*)d_kept_id_, nullptr, d_keys_a_, d_vals_a_, d_keys_b_,
-                                  d_vals_b_, d_hist_, d_scratch_, stream_, &k2, &j2));
-      gather_u32<<<dim3(blocks), dim3(256), 0, stream_>>>(d_kept_key_, j2, n_kept, d_key2_, d_index2_);
-      const SortPlan by_key = make_sort_plan(n_kept, 32);
-      uint32_t *k3 = nullptr, *j3 = nullptr;
-      ND_HIP_TRY(radix_sort_pairs(by_key, d_key2_, d_index2_, d_keys_a_, d_vals_a_, d_keys_b_, d_vals_b_, d_hist_,
-                                  d_scratch_, stream_, &k3, &j3));
-      gather_u32<<<dim3(blocks), dim3(256), 0, stream_>>>(d_kept_sample_, j3, n_kept, d_key2_, d_index2_);
-      const SortPlan by_sample = make_sort_plan(n_kept, chunk_bits);
-      uint32_t *k4 = nullptr, *j4 = nullptr;
-      ND_HIP_TRY(radix_sort_pairs(by_sample, d_key2_, d_index2_, d_keys_a_, d_vals_a_, d_keys_b_, d_vals_b_, d_hist_,
-                                  d_scratch_, stream_, &k4, &j4));
-      gather_u32<<<dim3(blocks), dim3(256), 0, stream_>>>((const uint32_t*)d_kept_id_, j4, n_kept,
-                                                          (uint32_t*)d_ranked_ids_, nullptr);
-    }
-    P.ranked_start = d_ranked_start_;
-    P.ranked_ids = d_ranked_ids_;
-    P.marked = marked_.sample;
-    P.n_marked = n_marked;
-    const uint64_t outputs = (uint64_t)n_marked * P.step_size;
-    layer_execute_kernel<SampleType, App><<<dim3((unsigned)((outputs + 255) / 256)), dim3(256), 0, stream_>>>(P);
+    kept_layer_kernel<SampleType, App><<<dim3(n), dim3(kBinThreads), 0, stream_>>>(P, marked_.count, marked_.sample, groups, kept);
     ND_HIP_TRY(hipGetLastError());
     return 0;
   }
-
-  // Arrays with one entry per listed (sample, vertex) pair of a chunk: the distinct pairs
-  // (FastGCN form) or the pairs the selection keeps (LADIES form).
-  int ensure_distinct_capacity(uint32_t n_distinct) {
-    if (n_distinct <= distinct_capacity_ && distinct_capacity_ > 0) return 0;
-    constexpr int form = apps::neighborhood_form_of<App>::value;
-    const size_t cap = (size_t)n_distinct + n_distinct / 8 + 1024;
-    release_distinct_buffers();
-    if (form == apps::kRankedByLadiesImportance) {
-      ND_HIP_TRY(hipMalloc(&d_ranked_ids_, sizeof(int32_t) * cap));
-      ND_HIP_TRY(hipMalloc(&d_kept_key_, sizeof(uint32_t) * cap));
-      ND_HIP_TRY(hipMalloc(&d_kept_sample_, sizeof(uint32_t) * cap));
-      ND_HIP_TRY(hipMalloc(&d_kept_id_, sizeof(int32_t) * cap));
-      ND_HIP_TRY(hipMalloc(&d_keys_a_, sizeof(uint32_t) * cap));
-      ND_HIP_TRY(hipMalloc(&d_vals_a_, sizeof(uint32_t) * cap));
-      ND_HIP_TRY(hipMalloc(&d_keys_b_, sizeof(uint32_t) * cap));
-      ND_HIP_TRY(hipMalloc(&d_vals_b_, sizeof(uint32_t) * cap));
-      ND_HIP_TRY(hipMalloc(&d_key2_, sizeof(uint32_t) * cap));
-      ND_HIP_TRY(hipMalloc(&d_index2_, sizeof(uint32_t) * cap));
-      ND_HIP_TRY(hipMalloc(&d_hist_, sizeof(uint32_t) * sort_hist_capacity(cap)));
-      size_t scratch = make_sort_plan(cap, 32).scratch_elems;
-      ND_HIP_TRY(hipMalloc(&d_scratch_, sizeof(uint32_t) * scratch));
-    }
-    distinct_capacity_ = cap;
-    return 0;
-  }
+  uint32_t ladies_bins() const { return (bitmap_words_ + kBinWords - 1) / kBinWords; }
+  uint32_t ladies_groups() const { return (ladies_bins() + kBinsPerGroup - 1) / kBinsPerGroup; }
 
   // The concatenated neighbourhood itself (kConcatenated form).
   int ensure_neighborhood_capacity(uint32_t total) {
@@ -1741,19 +1758,10 @@ class LayerEngine : public EngineBase {
     return 0;
   }
 
-  void release_distinct_buffers() {
-    release(d_ranked_ids_);
-    release(d_keys_a_); release(d_vals_a_); release(d_keys_b_); release(d_vals_b_);
-    release(d_key2_); release(d_index2_); release(d_hist_); release(d_scratch_);
-    release(d_kept_key_); release(d_kept_sample_); release(d_kept_id_);
-    distinct_capacity_ = 0;
-  }
-
   void release_neighborhood_buffers() {
     release(d_nbr_cols_); release(d_nbr_weights_);
-    release(d_bitmap_); release(d_keys_dense_); release(d_stretch_best_);
+    release(d_bitmap_); release(d_kept_); release(d_n_kept_); release(d_bound_);
     release(d_group_through_); release(d_part_total_); release(d_part_before_);
-    release_distinct_buffers();
     capacity_ = 0;
     bitmap_samples_ = 0;
   }
@@ -1766,8 +1774,7 @@ class LayerEngine : public EngineBase {
     if (h_too_long_) (void)hipHostFree(h_too_long_);
     h_too_long_ = nullptr;
     release(marked_.count); release(marked_.sample); release(marked_.transits); release(marked_.transit_count);
-    release(d_ranked_start_); release(d_select_kept_);
-    release(d_select_threshold_); release(d_select_claimed_); release(d_merged_sizes_);
+    release(d_merged_sizes_);
     release_neighborhood_buffers();
     // whatever exists, also after an alloc that failed half way
     for (hipEvent_t* ev : {&ev_a_, &ev_b_, &ev_begin_, &ev_end_}) {
@@ -1800,11 +1807,10 @@ class LayerEngine : public EngineBase {
   uint32_t bitmap_chunk_samples_ = 0;  // samples whose bitmaps fit the budget
   uint64_t bitmap_chunk_entries_ = 0;
   uint32_t bitmap_samples_ = 0;        // samples the allocated bitmaps hold
-  size_t distinct_capacity_ = 0;
   uint32_t* d_bitmap_ = nullptr;
-  // LADIES form: importance sums and sampling keys, [sample][vertex, padded to whole stretches]
-  uint32_t* d_keys_dense_ = nullptr;
-  uint16_t* d_stretch_best_ = nullptr;  // LADIES form: best key prefix of every 256 keys of every sample
+  // LADIES form: what the workgroups of the marking keep (KeptKeys)
+  uint2* d_kept_ = nullptr;
+  uint32_t *d_n_kept_ = nullptr, *d_bound_ = nullptr;
   mutable uint64_t neighborhood_total_ = 0, distinct_total_ = 0;
   uint64_t chunks_run_ = 0;
   mutable bool counted_ = true;  // those two are the last pass's
@@ -1819,9 +1825,6 @@ class LayerEngine : public EngineBase {
   VertexID_t* d_final_ = nullptr;
   uint32_t *d_sizes_ = nullptr, *d_offsets_ = nullptr, *d_row_offsets_ = nullptr, *d_small_scratch_ = nullptr;
   uint32_t *d_item_count_ = nullptr, *d_item_start_ = nullptr;
-  // LADIES form: the selection of the best keys per sample
-  uint32_t *d_ranked_start_ = nullptr, *d_select_kept_ = nullptr, *d_select_threshold_ = nullptr;
-  uint32_t* d_select_claimed_ = nullptr;  // entries of a sample that have been given room
   uint32_t* d_merged_sizes_ = nullptr;    // pairs of a sample's neighbourhood
   EdgePos_t* d_merged_rows_ = nullptr;    // the graph without parallel edges
   VertexID* d_merged_ids_ = nullptr;
@@ -1829,19 +1832,14 @@ class LayerEngine : public EngineBase {
   int32_t* d_cut_row_of_ = nullptr;
   HubCut* d_cuts_ = nullptr;
   MergedEdges merged_{};
-  uint32_t *d_kept_key_ = nullptr, *d_kept_sample_ = nullptr;
-  int32_t* d_kept_id_ = nullptr;
   int32_t* d_nbr_cols_ = nullptr;
   float* d_nbr_weights_ = nullptr;
-  uint32_t *d_keys_a_ = nullptr, *d_vals_a_ = nullptr, *d_keys_b_ = nullptr, *d_vals_b_ = nullptr;
-  uint32_t *d_key2_ = nullptr, *d_index2_ = nullptr, *d_hist_ = nullptr, *d_scratch_ = nullptr;
   // FastGCN form: degree^2 of the marked vertices, by group inside a part, by part, by sample
   uint64_t *d_group_through_ = nullptr, *d_part_total_ = nullptr, *d_part_before_ = nullptr;
   UnionTables union_;                  // of the graph
   MarkedSamples marked_{};
   uint32_t* d_layer_counts_ = nullptr;  // entries of every layer and sample's neighbourhood, then its distinct vertices
-  uint32_t* h_too_long_ = nullptr;      // whether a neighbourhood was too long, and two counts the LADIES form waits for
-  int32_t* d_ranked_ids_ = nullptr;
+  uint32_t* h_too_long_ = nullptr;      // whether a neighbourhood was too long
 };
 
 }  // namespace nd

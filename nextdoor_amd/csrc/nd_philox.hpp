@@ -47,6 +47,15 @@ ND_HD uint32_t mul_hi_u32(uint32_t a, uint32_t b) {
 #endif
 }
 
+// (three operands in one instruction, which the compiler does not find by itself)
+ND_HD uint32_t xor3_u32(uint32_t a, uint32_t b, uint32_t c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+#else
+  return a ^ b ^ c;
+#endif
+}
+
 ND_HD PhiloxBlock philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3,
                                 uint32_t k0, uint32_t k1) {
   constexpr uint32_t kMulA = 0xD2511F53u, kMulB = 0xCD9E8D57u;
@@ -55,9 +64,9 @@ ND_HD PhiloxBlock philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t 
   for (int r = 0; r < 10; ++r) {
     const uint32_t hi_a = mul_hi_u32(kMulA, c0), lo_a = kMulA * c0;
     const uint32_t hi_b = mul_hi_u32(kMulB, c2), lo_b = kMulB * c2;
-    c0 = hi_b ^ c1 ^ k0;
+    c0 = xor3_u32(hi_b, c1, k0);
     c1 = lo_b;
-    c2 = hi_a ^ c3 ^ k1;
+    c2 = xor3_u32(hi_a, c3, k1);
     c3 = lo_a;
     k0 += kWeylA;
     k1 += kWeylB;

@@ -188,6 +188,37 @@ def test_ladies_importance_matches_oracle(oracle, app, gname):
     s.close()
 
 
+@pytest.mark.parametrize("weights", ["equal_keys", "later_is_better", "one_of_all"])
+@pytest.mark.parametrize("pieces", ["0", "default"])
+def test_ladies_keys_that_are_hard_to_tell_apart(oracle, weights, pieces, monkeypatch):
+    """What a workgroup keeps of a sample: nearly all keys equal (terms below 2^-53: importance 0, told apart by vertex;
+    more of them in one stretch than a workgroup begins the next with), every stretch's keys better than the last one's,
+    and one vertex far better than all others."""
+    if pieces != "default":
+        monkeypatch.setenv("ND_DENSE_PIECE_ENTRIES", pieces)
+    n, hubs = 60000, 24
+    rng = np.random.default_rng(3)
+    src = np.concatenate([np.repeat(np.arange(hubs), n), np.arange(n)])  # the hubs know everyone, everyone knows a hub
+    dst = np.concatenate([np.tile(np.arange(n), hubs), rng.integers(0, hubs, n)])
+    w = np.ones(len(src), np.float32)
+    if weights == "equal_keys":
+        w[:hubs * n] = 1e-9
+        w[np.arange(hubs) * n + rng.integers(0, n, hubs)] = 1.0
+    elif weights == "later_is_better":
+        w[:hubs * n] = np.tile(np.exp2(np.arange(n) / 3000.0), hubs)
+    else:
+        w[np.arange(hubs) * n + 4321] = 1e6
+    g = nd.Graph.from_edges(src, dst, w, n_vertices=n)
+    s = nd.Sampler("LADIESImportance2x8", g, seed=SEED)
+    want = oracle.sample_ladies_importance(graphs.oracle_view(g), layer_desc(oracle, s, oracle.LADIES_IMPORTANCE), SEED,
+                                           s.initial_contents)
+    print("weights", weights, "pieces", pieces, "built", s.counter(3), flush=True)
+    for _ in range(2):
+        s.do_transit_parallel(True)
+        assert np.array_equal(s.final_samples(), want)
+    s.close()
+
+
 @pytest.mark.parametrize("app,kind_name", [("FastGCNImportance3x16", "FASTGCN_IMPORTANCE"),
                                            ("LADIESImportance3x16", "LADIES_IMPORTANCE"),
                                            ("LayerLiteral3x16", "LAYER_LITERAL")])
