@@ -799,8 +799,9 @@ __global__ __launch_bounds__(kSortOutThreads) void sort_out_ranked(CSRPartition 
                                                                    uint32_t* __restrict__ sizes,
                                                                    uint32_t* __restrict__ merged_sizes,
                                                                    uint32_t* n_marked, uint32_t* __restrict__ marked,
-                                                                   uint32_t* __restrict__ distinct, uint32_t* __restrict__ bound,
-                                                                   uint32_t* __restrict__ too_long) {
+                                                                   uint32_t* __restrict__ too_long,
+                                                                   uint32_t* __restrict__ distinct = nullptr,
+                                                                   uint32_t* __restrict__ bound = nullptr) {
   __shared__ uint32_t s_taken, s_base;
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t s = blockIdx.x * (kSortOutThreads / 64u) + (threadIdx.x >> 6);
@@ -828,8 +829,8 @@ __global__ __launch_bounds__(kSortOutThreads) void sort_out_ranked(CSRPartition 
   __syncthreads();
   if (lane == 0 && s < n_samples && pairs > kRankedEntries) {
     marked[s_base + at] = s;
-    bound[s_base + at] = kNoBound;
-    distinct[s] = 0;
+    if (bound) bound[s_base + at] = kNoBound;
+    if (distinct) distinct[s] = 0;
   }
 }
 
@@ -1723,8 +1724,8 @@ class LayerEngine : public EngineBase {
     uint32_t* distinct = sizes + S * App().steps();
     ND_HIP_TRY(hipMemsetAsync(marked_.count, 0, sizeof(uint32_t), stream_));
     sort_out_ranked<<<dim3((n + 15) / 16), dim3(kSortOutThreads), 0, stream_>>>(
-        P.csr, merged_, P.transits, n, invalid_, sizes, d_merged_sizes_, marked_.count, marked_.sample, distinct, d_bound_,
-        h_too_long_);
+        P.csr, merged_, P.transits, n, invalid_, sizes, d_merged_sizes_, marked_.count, marked_.sample, h_too_long_,
+        distinct, d_bound_);
     tick();
     ranked_layer_kernel<SampleType, App><<<dim3(n), dim3(kRankedThreads), 0, stream_>>>(P, merged_, d_merged_sizes_, distinct);
     KeptKeys kept;
