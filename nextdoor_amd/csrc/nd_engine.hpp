@@ -58,6 +58,7 @@ enum KernelMode { kTransitParallel = 0, kTransitParallelLoadBalanced = 1, kSampl
 
 struct PhaseTimes {  // milliseconds, accumulated over one sample() call when profiling is on
   float end_to_end = 0, inversion = 0, load_balancing = 0, flat_kernel = 0, workgroup_kernel = 0, assemble = 0, distinct = 0;
+  // (flat: a launch of walks whose rows leave while it runs counts once for every part of them that leaves by itself)
   int flat_launches = 0, workgroup_launches = 0, sort_launches = 0;
   // layer-wise apps: the kernel that walks the collective neighbourhoods (marking / building)
   float neighborhood = 0;
@@ -820,9 +821,37 @@ __device__ __forceinline__ void enter_vertex(const CSRPartition& csr, const Walk
   }
 }
 
+// Rows that leave while later ones are still being walked (stretch: 2^shift consecutive walks).  A stretch's rows are in
+// memory, for every compute unit to read, before `arrived` of it is written: they are stored past the L2 of the XCD the
+// wavefront is on, which nothing else would write back before the kernel ends, and a walk is counted when its
+// stores have been acknowledged.  The last one of a stretch clears the stretch's count for the next pass.
+// (One count to a line: atomics on one are served 10 ns apart, whichever of its words they are for.)
+constexpr uint32_t kWordsPerCount = 32;
+constexpr uint32_t kLineWords = 32;  // of memory
+struct EarlyRows {
+  uint32_t* walked = nullptr;   // [stretch * kWordsPerCount] walks of it that are done; all 0 between passes
+  uint32_t* arrived = nullptr;  // [stretch], page-locked host memory: the number of the pass that has all of its rows
+  uint32_t shift = 0, pass = 0;
+};
+
+__device__ __forceinline__ void store_four(int32_t* at, VertexID a, VertexID b, VertexID c, VertexID d, bool past_caches) {
+  if (past_caches) {
+    typedef int Four __attribute__((ext_vector_type(4)));
+    const Four v = {a, b, c, d};
+    // (two wait states before its registers are written again, as the compiler would have them)
+    asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" : : "v"(at), "v"(v) : "memory");
+  } else {
+    *reinterpret_cast<FourIds*>(at) = FourIds{a, b, c, d};
+  }
+}
+__device__ __forceinline__ void store_one(int32_t* at, VertexID v, bool past_caches) {
+  if (past_caches) __hip_atomic_store(at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  else *at = v;
+}
+
 // Walks that are not inverted: one launch does all steps of all walks.  A lane keeps its walk, with
 // the current vertex, the random state and the sample state in registers, until it ends, and
-// then takes the next walk of its wavefront; results go straight into the rows, four to a store.
+// then takes the next walk of its wavefront; results go straight into the rows.
 //
 // What bounds it: the gathers.  Over a graph beyond the caches the requests past L2 (R-MAT 22 weighted
 // node2vec: 1.15e9 of them in 24.1 ms, 47.9 G/s of the 48-50 the gather probe reaches: row extent, 2.95
@@ -838,15 +867,21 @@ __device__ __forceinline__ void enter_vertex(const CSRPartition& csr, const Walk
 // 4.0, R-MAT 22 34.5 / 24.1, four walks a vertex over 700 K 27.6 / 14.5.  There is no case among them where
 // the order is worth what it costs.
 //
+// Results go to the rows a line of memory at a time, or four at a time (Engine::kLinesFromWalks).  Where rows leave early they are
+// stored past the L2 (EarlyRows).
+//
 // Walks are handed out in blocks of 64: block w to wavefront w, the rest from a counter.  (Every n_waves-th
 // block to a wavefront, without a counter: 38.6 ms on R-MAT 22 - whether a vertex has edges depends on the bits of
 // its id, and so do multiples of n_waves.)  queue[0] counts the blocks handed out after the first n_waves,
 // queue[1] the wavefronts that are done; the last one leaves both zero for the next pass.  Nobody waits for anybody.
-template <class SampleType, class App, bool kRecords>
+// (kPlain: no rows that leave early and no lines.  The instantiation with both takes 2.7 K uniform walks from 0.093 to 0.098 ms
+// and 57 K from 0.113 to 0.128 where it uses neither.)
+template <class SampleType, class App, bool kRecords, bool kPlain>
 __global__ __launch_bounds__(kFlatThreads) void walk_rows_kernel(StepParams P, int n_steps, uint32_t n_waves,
                                                                  uint32_t* queue,
                                                                  const WalkVertex* __restrict__ vertices,
-                                                                 const walk_record<App>* __restrict__ records) {
+                                                                 const walk_record<App>* __restrict__ records,
+                                                                 EarlyRows early, bool lines) {
   typedef walk_record<App> Record;
   static_assert(kFlatThreads == kWave, "a workgroup is a wavefront");
   constexpr bool kTravels = state_fits_pair<SampleType>::value;
@@ -871,6 +906,34 @@ __global__ __launch_bounds__(kFlatThreads) void walk_rows_kernel(StepParams P, i
   SampleType* state = &local_state;
   Record last;
   last.dst = -1;
+  const bool past_caches = !kPlain && early.arrived != nullptr, by_lines = !kPlain && lines;
+  // by_lines: four results go to the lane's line in LDS (its eight fours in an order of the lane's own, for the banks), and
+  // eight lanes store a line that is full.
+  __shared__ __align__(16) int32_t s_lines[kPlain ? 1 : kWave][kLineWords];
+  auto in_line = [&](uint32_t of, uint32_t four) { return &s_lines[of][4u * ((four ^ of) & 7u)]; };
+  // A lane counts for all of the wavefront's walks that end in a turn: `counted` of stretch counted_of, where there were
+  // count_before.  That is looked at a turn or more later, when it has come with what the turn waits for anyway.
+  uint32_t counted = 0, counted_of = 0, count_before = 0;
+  auto count_in = [&](uint64_t ends) {  // those of the first one's stretch; returns the others
+    const int src = __ffsll((unsigned long long)ends) - 1;
+    const uint32_t stretch = (uint32_t)__builtin_amdgcn_readlane((int)slot, src) >> early.shift;
+    const uint64_t same = __ballot(slot >> early.shift == stretch) & ends;
+    if ((int)lane == src) {
+      counted = (uint32_t)__popcll(same);
+      counted_of = stretch;
+      count_before = atomicAdd(early.walked + (size_t)stretch * kWordsPerCount, counted);
+    }
+    return ends & ~same;
+  };
+  auto look_at_count = [&] {
+    if (counted == 0) return;
+    const uint32_t left = n_walks - (counted_of << early.shift);
+    if (count_before + counted == (left < 1u << early.shift ? left : 1u << early.shift)) {
+      early.walked[(size_t)counted_of * kWordsPerCount] = 0;
+      __hip_atomic_store(early.arrived + counted_of, early.pass, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    counted = 0;
+  };
   for (;;) {
     const uint64_t idle = __ballot(!busy);
     if (idle != 0 && (more || block < block_end)) {
@@ -904,7 +967,7 @@ __global__ __launch_bounds__(kFlatThreads) void walk_rows_kernel(StepParams P, i
       if (more || block < block_end) continue;
       break;
     }
-    bool ended = false;
+    bool ended = false, four_done = false;
     if (busy) {
       if (fresh) {
         rng.reset(P.seed, P.first_slot + slot, (uint32_t)step);
@@ -950,8 +1013,14 @@ __global__ __launch_bounds__(kFlatThreads) void walk_rows_kernel(StepParams P, i
         r1 = r2;
         r2 = r3;
         r3 = neighbor;
-        if ((step & 3) == 3)
-          *reinterpret_cast<FourIds*>(P.step_out + (size_t)slot * P.out_pitch + (step - 3)) = FourIds{r0, r1, r2, r3};
+        if ((step & 3) == 3) {
+          if (by_lines) {
+            *reinterpret_cast<int4*>(in_line(lane, (slot * P.out_pitch + (uint32_t)step) >> 2)) = make_int4(r0, r1, r2, r3);
+            four_done = true;
+          } else {
+            store_four(P.step_out + (size_t)slot * P.out_pitch + (step - 3), r0, r1, r2, r3, past_caches);
+          }
+        }
         const bool had_transit = transit != P.invalid;
         transit = neighbor;
         if (explicit_transits && had_transit && step + 1 < n_steps) {
@@ -971,7 +1040,30 @@ __global__ __launch_bounds__(kFlatThreads) void walk_rows_kernel(StepParams P, i
         }
       }
     }
+    // the lines that are full, or whose walk has ended
+    auto flush_lines = [&](bool has_ended) {
+      const size_t row = (size_t)slot * P.out_pitch, top = row + (((uint32_t)step + 3u) & ~3u);
+      const uint32_t line = (uint32_t)((top - 1) / kLineWords), last = (uint32_t)(top - 1) % kLineWords / 4u;
+      const uint32_t first = row / kLineWords == line ? (uint32_t)row % kLineWords / 4u : 0u;
+      uint64_t todo = __ballot(four_done && (has_ended || last == kLineWords / 4u - 1u));
+      while (todo) {
+        uint32_t of = kWave;  // whose line this lane helps with
+        for (uint32_t helpers = 0; helpers < kWave && todo; helpers += kLineWords / 4u) {
+          const uint32_t src = (uint32_t)__ffsll((unsigned long long)todo) - 1u;
+          todo &= todo - 1;
+          if (lane - helpers < kLineWords / 4u) of = src;
+        }
+        const uint32_t from = of % kWave;
+        const uint32_t its_line = __shfl(line, from, kWave), its_first = __shfl(first, from, kWave), its_last = __shfl(last, from, kWave);
+        const uint32_t four = lane % (kLineWords / 4u);
+        if (of < kWave && four >= its_first && four <= its_last) {
+          const int4 v = *reinterpret_cast<const int4*>(in_line(of, four));
+          store_four(P.step_out + (size_t)its_line * kLineWords + 4u * four, v.x, v.y, v.z, v.w, past_caches);
+        }
+      }
+    };
     const uint64_t ends = __ballot(ended);
+    if (ends == 0 && by_lines && __ballot(four_done) != 0) flush_lines(false);
     if (ends != 0) {
       int rest = n_steps;  // first slot of the row that is still to be written
       if (ended) {
@@ -990,16 +1082,20 @@ __global__ __launch_bounds__(kFlatThreads) void walk_rows_kernel(StepParams P, i
             r3 = P.invalid;
           }
           int32_t* dst = P.step_out + (size_t)slot * P.out_pitch + rest;
-          if (rest + 4 <= n_steps) {
-            *reinterpret_cast<FourIds*>(dst) = FourIds{r0, r1, r2, r3};
+          if (by_lines) {
+            *reinterpret_cast<int4*>(in_line(lane, (slot * P.out_pitch + (uint32_t)rest) >> 2)) = make_int4(r0, r1, r2, r3);
+            four_done = true;
+          } else if (rest + 4 <= n_steps) {
+            store_four(dst, r0, r1, r2, r3, past_caches);
           } else {
-            dst[0] = r0;
-            if (rest + 1 < n_steps) dst[1] = r1;
-            if (rest + 2 < n_steps) dst[2] = r2;
+            store_one(dst, r0, past_caches);
+            if (rest + 1 < n_steps) store_one(dst + 1, r1, past_caches);
+            if (rest + 2 < n_steps) store_one(dst + 2, r2, past_caches);
           }
           rest += 4;
         }
       }
+      if (by_lines) flush_lines(ended);
       // what is left of the rows of walks that ended early, by the whole wavefront: at most 128 slots
       uint64_t todo = __ballot(rest < n_steps);
       while (todo) {
@@ -1009,13 +1105,22 @@ __global__ __launch_bounds__(kFlatThreads) void walk_rows_kernel(StepParams P, i
         int32_t* row = P.step_out + (size_t)__shfl(slot, src, kWave) * P.out_pitch;
         const int at = from + 4 * (int)lane;
         if (at + 4 <= n_steps) {
-          *reinterpret_cast<FourIds*>(row + at) = FourIds{P.invalid, P.invalid, P.invalid, P.invalid};
+          store_four(row + at, P.invalid, P.invalid, P.invalid, P.invalid, past_caches);
         } else {
-          for (int x = at; x < n_steps; ++x) row[x] = P.invalid;
+          for (int x = at; x < n_steps; ++x) store_one(row + x, P.invalid, past_caches);
+        }
+      }
+      if (past_caches) {
+        look_at_count();  // of the turns before
+        asm volatile("s_waitcnt vmcnt(0)" : : : "memory");  // the rows of those that have ended are where they belong
+        for (uint64_t others = count_in(ends); others != 0;) {
+          look_at_count();
+          others = count_in(others);
         }
       }
     }
   }
+  look_at_count();
   if (queued && lane == 0 && atomicAdd(queue + 1, 1u) == n_waves - 1) {
     // every wavefront has taken its last block
     queue[0] = 0;
@@ -1994,9 +2099,9 @@ class Engine : public EngineBase {
       int per_cu = 0, device = 0, cus = 0;
       ND_HIP_TRY(hipGetDevice(&device));
       ND_HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
-      ND_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, walk_rows_kernel<SampleType, App, true>, kFlatThreads, 0));
+      ND_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, walk_rows_kernel<SampleType, App, true, true>, kFlatThreads, 0));
       walk_waves_at_once_ = (uint32_t)std::max(1, per_cu * cus);
-      walk_waves_queued_ = (uint32_t)std::max(1, (int)kQueuedWavesPerCu * cus);
+      cus_ = (uint32_t)std::max(1, cus);
     }
     const char* small_map = getenv("ND_SMALL_MAP");
     inversion_forced_ = small_map != nullptr;  // chooses how the map is inverted: so it is
@@ -2084,11 +2189,12 @@ class Engine : public EngineBase {
       const size_t n = (size_t)n_samples_ * (size_t)final_sample_size();
       fill_i32<<<dim3((unsigned)((n + 1023) / 1024)), dim3(1024), 0, stream_>>>(d_final_, n, invalid_ + 1);
     }
-    const uint32_t ranges = walk_ranges();
-    if (ranges == 1) return launch_walks(0, (uint32_t)n_samples_, d_walk_queue_);
+    EarlyRows early;
+    const EarlyForm form = early_form(&early);
+    const uint32_t ranges = form == kRowsByRange ? walk_ranges() : 1;
     const size_t F = (size_t)final_sample_size();
     std::vector<ResultStream::Ready> ready;
-    while (range_ends_.size() < ranges) {
+    while (form != kRowsStay && range_ends_.size() < ranges) {
       hipEvent_t ev = nullptr;
       ND_HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
       range_ends_.push_back(ev);
@@ -2096,11 +2202,18 @@ class Engine : public EngineBase {
     uint32_t first = 0;
     for (uint32_t r = 0; r < ranges; ++r) {
       const uint32_t end = r + 1 == ranges ? (uint32_t)n_samples_ : (uint32_t)((uint64_t)n_samples_ * (r + 1) / ranges / kWave * kWave);
-      const int rc = launch_walks(first, end - first, d_walk_queue_ + 2 * r);
-      if (rc != 0) return rc;
+      if (launch_walks(first, end - first, d_walk_queue_ + 2 * r, early) != 0) return -1;
+      if (form == kRowsStay) return 0;
       ND_HIP_TRY(hipEventRecord(range_ends_[r], stream_));
       ready.push_back({end * F, range_ends_[r]});
       first = end;
+    }
+    if (form == kRowsByStretch) {
+      times.flat_launches = (int)(((uint64_t)n_samples_ - 1) >> early.shift) + 1;
+      ready.clear();
+      for (uint64_t at = 0; at < (uint64_t)n_samples_; at += 1ull << early.shift)
+        ready.push_back({(size_t)std::min<uint64_t>((uint64_t)n_samples_, at + (1ull << early.shift)) * F, range_ends_[0],
+                         h_arrived_ + (at >> early.shift), early.pass});
     }
     // rows that cannot be sent now are fetched when they are asked for
     try {
@@ -2113,37 +2226,88 @@ class Engine : public EngineBase {
     return 0;
   }
 
-  // Launches a pass of walks is split into, where its rows are to leave early.  Every one of them ends with its longest
-  // walks alone on the device, and the first row leaves at the end of the first; what there is to hide is the rows' time on
-  // the bus, 4.3 ms for a million walks of 100 steps.  An end costs 0.07 ms of uniform walks, 0.15-0.25 of DeepWalk and PPR,
-  // 0.6 of second-order walks (a state that travels; the most tries a step).  Passes with their rows, ms, by launches, over
-  // Chung-Lu graphs unless another is named:
-  //    no state                   1     2     3     4     6     8     a state that travels     1     2     3     4     6
-  //    uniform         100 K   0.68  0.64  0.66  0.77  0.94  1.13    weighted n2v  200 K    1.94  2.12  2.62  3.18  4.26
-  //                    200 K   1.20  1.12  1.11  1.09  1.25  1.49                  300 K    2.94  2.63  3.12  3.75  4.82
-  //                    400 K   2.35  2.22  2.05  1.99  2.06  2.07                  350 K    3.57  2.90  3.33  3.95  5.14
-  //                    800 K   4.70  4.71  4.57  4.43  4.27  4.13                  500 K    4.98  3.98  3.99  4.51  5.84
-  //                    1.2 M   7.04  6.94  7.07  6.98  6.71  6.50                  700 K    6.78  6.06  5.27  5.34  6.60
-  //    PPR             262 K   1.53  1.43  1.36  1.47  1.92  2.38                    1 M    9.54  8.58  8.39  7.45  7.89
-  //                    600 K   3.39  3.10  2.95  2.91  2.87  3.06                  1.5 M    14.5  12.3  12.1  11.8  10.9
-  //                    800 K   4.42  4.21  3.90  3.78  3.72  3.71                    3 M    28.8  24.1  23.0  22.3  23.5
-  //    DeepWalk        200 K   1.45  1.29  1.41  1.60  2.00  2.45             R-MAT 22      38.4  32.2  30.8  30.2  30.9
-  //                    400 K   3.02  2.40  2.27  2.30  2.63  3.04    a state in memory
-  //                    700 K   4.86  4.91  4.05  3.73  3.93  4.25    MultiRW        50 K    0.89  0.90  1.02  1.16  1.46
-  //                    800 K   5.54  5.83  4.79  4.36  4.38  4.60                   90 K    1.58  1.36  1.44  1.61  1.84
-  //                    1.2 M   8.48  7.65  8.59  7.40  6.44  6.42                  125 K    2.25  1.79  1.81  1.94  2.24
-  //             R-MAT 22       26.4  23.9  23.2  22.4  22.3  22.1                  300 K    5.42  4.97  4.38  4.07  4.30
+  // How rows leave before the pass is over.  kRowsByStretch: one launch, whose wavefronts count the walks that are done by
+  // stretch (EarlyRows); rows leave as fast as they come, packed for the copy engine, and the walks are not slowed down.
+  // kRowsByRange: a few launches, one range of walks after another; rows leave from the end of the first on (one launch:
+  // when it has ended).  Every launch ends with its longest walks alone on the device (0.07 ms of uniform walks, 0.2 of
+  // DeepWalk and PPR, 0.6 of second-order walks), but all of a range's rows are there at once, and their way straight to
+  // the ring has no 8 us between two pieces.  Passes with their rows, ms, by launches and, one launch, by wavefronts a compute
+  // unit (Chung-Lu graphs, mean degree 10 to 12, unless another is named):
+  //                     launches  1     2     3     4      wavefronts  6     8    10    12    16
+  //    uniform         300 K   1.45  1.33  1.29  1.32           1.41  1.42  1.41  1.42  1.44
+  //                    550 K   2.59  2.31  2.26  2.19           2.39  2.28  2.32  2.37  2.49
+  //                    800 K   3.74  3.63  3.36  3.30           3.11  3.13  3.15  3.23  3.38
+  //                    1.1 M   4.95  4.80  4.79  4.69           4.14  4.13  4.15  4.23  4.42
+  //    DeepWalk        300 K   2.10  1.63  1.66  1.90           1.76  1.75  1.79  1.81  1.86
+  //                    400 K   2.52  2.09  2.03  2.05           2.12  2.08  2.14  2.22  2.31
+  //                    550 K   3.25  2.98  2.71  2.70           2.73  2.65  2.73  2.81  3.06
+  //                    1.1 M   6.45  5.93  5.61  5.54           4.99  4.90  4.93  5.00  5.20
+  //                  R-MAT 22                                  16.17 15.99 16.12 16.44 17.28
+  //    PPR             300 K   1.72  1.49  1.47  1.69           1.61  1.60  1.57  1.58  1.61
+  //                    550 K   2.71  2.59  2.49  2.49           2.46  2.44  2.46  2.47  2.60
+  //                    1.1 M   5.25  4.96  4.90  4.80           4.46  4.29  4.37  4.41  4.53
+  //    weighted n2v    100 K   1.26  1.72  2.25  2.84           1.43  1.27  1.27  1.27  1.28
+  //                    140 K   1.47  2.00  2.47  3.05           1.78  1.59  1.49  1.50  1.51
+  //                    300 K   2.98  2.56  3.16  3.81           2.86  2.59  2.56  2.51  2.55
+  //                    550 K   5.20  5.07  4.17  4.78           4.61  4.08  4.11  4.17  4.40
+  //                    1.1 M   9.89  8.65  8.42  9.72           8.60  7.29  6.78  6.87  7.97
+  //                  R-MAT 22  (30.1 by four launches)         33.7  28.8  26.2  25.2  24.4
+  //                                                    wavefronts  2     3     4     5     6
+  //    MultiRW         100 K   1.16  0.94  1.02  1.13           1.10  1.09  0.94  1.05  1.17
+  //                    200 K   2.51  2.04  1.83  1.80           1.84  1.72  1.93  2.19  2.33
+  //                    400 K   5.06  4.93  4.26  3.78           3.36  3.07  3.23  3.54  3.81
+  //                    1.1 M  14.72 14.09 13.35 14.24                 7.73  8.28  8.76  9.33
+  enum EarlyForm { kRowsStay, kRowsByRange, kRowsByStretch };
+  EarlyForm early_form(EarlyRows* early) {
+    if (!rows_ahead || profiling || wants_launch_graph()) return kRowsStay;
+    if (sizeof(VertexID_t) * (size_t)n_samples_ * (size_t)final_sample_size() <= kDirectResultBytes) return kRowsStay;
+    const bool many = n_samples_ >= (state_fits_pair<SampleType>::value ? 96 << 10 : std::is_empty<SampleType>::value ? 448 << 10 : 192 << 10);
+    return many && ready_for_early_rows(early) ? kRowsByStretch : kRowsByRange;
+  }
   uint32_t walk_ranges() const {
-    if (!rows_ahead || profiling || wants_launch_graph()) return 1;
-    if (sizeof(VertexID_t) * (size_t)n_samples_ * (size_t)final_sample_size() <= kDirectResultBytes) return 1;
-    constexpr bool stateless = std::is_empty<SampleType>::value;
-    constexpr int64_t least = stateless ? 96 << 10 : state_fits_pair<SampleType>::value ? 160 << 10 : 40 << 10;
-    if (stateless && n_samples_ >= 8 * least) return kMostWalkRanges;
-    return (uint32_t)std::max<int64_t>(1, std::min<int64_t>(4, n_samples_ / least));
+    const int64_t least = std::is_empty<SampleType>::value ? 96 << 10 : state_fits_pair<SampleType>::value ? 160 << 10 : 40 << 10;
+    return (uint32_t)std::max<int64_t>(1, std::min<int64_t>(kMostWalkRanges, n_samples_ / least));
+  }
+  // What that takes, and the stretches the walks are counted by; false: without.
+  bool ready_for_early_rows(EarlyRows* early) {
+    if (!h_arrived_) {
+      if (hipHostMalloc((void**)&h_arrived_, sizeof(uint32_t) * kMostStretches, hipHostMallocDefault) != hipSuccess ||
+          hipMalloc(&d_walked_, sizeof(uint32_t) * kMostStretches * kWordsPerCount) != hipSuccess ||
+          hipMemset(d_walked_, 0, sizeof(uint32_t) * kMostStretches * kWordsPerCount) != hipSuccess ||
+          hipStreamSynchronize(nullptr) != hipSuccess) {
+        (void)hipGetLastError();
+        free_early_rows();
+        return false;
+      }
+      memset(h_arrived_, 0, sizeof(uint32_t) * kMostStretches);
+      early_pass_ = 0;
+    }
+    if (++early_pass_ == 0) early_pass_ = 1;
+    early->walked = d_walked_;
+    early->arrived = h_arrived_;
+    early->pass = early_pass_;
+    early->shift = 12;
+    while (((uint64_t)n_samples_ - 1) >> early->shift >= kMostStretches) early->shift++;
+    return true;
+  }
+  void free_early_rows() {
+    if (h_arrived_) (void)hipHostFree(h_arrived_);
+    h_arrived_ = nullptr;
+    if (d_walked_) (void)hipFree(d_walked_);
+    d_walked_ = nullptr;
   }
 
+  template <bool kRecords>
+  void launch_walk_kernel(const StepParams& P, uint32_t n_waves, uint32_t* queue, const EarlyRows& early, bool lines) {
+    const walk_record<App>* records = kRecords ? walk_records_ : nullptr;
+    const dim3 grid(n_waves), block(kFlatThreads);
+    if (early.arrived || lines)
+      walk_rows_kernel<SampleType, App, kRecords, false><<<grid, block, 0, stream_>>>(P, App().steps(), n_waves, queue, walk_vertices_, records, early, lines);
+    else
+      walk_rows_kernel<SampleType, App, kRecords, true><<<grid, block, 0, stream_>>>(P, App().steps(), n_waves, queue, walk_vertices_, records, early, lines);
+  }
   // The walks [first, first + count).
-  int launch_walks(uint32_t first, uint32_t count, uint32_t* queue) {
+  int launch_walks(uint32_t first, uint32_t count, uint32_t* queue, const EarlyRows& early) {
     StepParams P = {};
     P.csr = view_;
     P.step_size = 1;
@@ -2162,15 +2326,24 @@ class Engine : public EngineBase {
     // That many keep the memory path past L2 as busy as more would (R-MAT 22 weighted node2vec: 24.1 ms with 12
     // wavefronts to a compute unit, 23.9 with 20; 27 with 8), and the fewer walks are under way, the sooner each is
     // done: shorter tails, more hits (DeepWalk over 1 M vertices 3.0 ms with 12, 3.4 with 20).
+    // Where rows leave by stretch the first of them should be there soon, and the fewer walks at a time the sooner: as many
+    // as keep the memory path busy (EarlyForm), second-order walks an eighth of the pass at a time if that is more, but no
+    // more than four wavefronts to a SIMD: the packing needs room in LDS beside them (R-MAT 22 node2vec with 20 to a
+    // compute unit: 34 ms).
+    constexpr bool kSecondOrder = state_fits_pair<SampleType>::value;
+    constexpr uint64_t kLeast = kSecondOrder ? 10 : std::is_empty<SampleType>::value ? 8 : 3;
     const uint64_t blocks = ((uint64_t)count + kWave - 1) / kWave;
-    const uint32_t n_waves = (uint32_t)(blocks <= walk_waves_at_once_ ? blocks : std::min(walk_waves_at_once_, walk_waves_queued_));
+    uint64_t n_waves = blocks;
+    if (early.arrived)
+      n_waves = std::min({blocks, std::max(kSecondOrder ? blocks / 8 : 0, kLeast * cus_), (uint64_t)std::min(16u * cus_, walk_waves_at_once_)});
+    else if (blocks > walk_waves_at_once_)
+      n_waves = std::min(walk_waves_at_once_, kQueuedWavesPerCu * cus_);
+    const bool lines = count == (uint32_t)n_samples_ && count > kLinesFromWalks && P.out_pitch % 4u == 0;
     tick();
     if (walk_records_)
-      walk_rows_kernel<SampleType, App, true><<<dim3(n_waves), dim3(kFlatThreads), 0, stream_>>>(
-          P, App().steps(), n_waves, queue, walk_vertices_, walk_records_);
+      launch_walk_kernel<true>(P, (uint32_t)n_waves, queue, early, lines);
     else
-      walk_rows_kernel<SampleType, App, false><<<dim3(n_waves), dim3(kFlatThreads), 0, stream_>>>(
-          P, App().steps(), n_waves, queue, walk_vertices_, nullptr);
+      launch_walk_kernel<false>(P, (uint32_t)n_waves, queue, early, lines);
     tock(&times.flat_kernel);
     times.flat_launches++;
     ND_HIP_TRY(hipGetLastError());
@@ -2613,7 +2786,8 @@ class Engine : public EngineBase {
   static constexpr int kBalanceWords =
       kMaxSteps + 2 + (int)(kCounterCopies * sizeof(ClassCounters) / sizeof(uint32_t));
   static constexpr int kIdleLookEvery = 8;
-  static constexpr uint32_t kMostWalkRanges = 6;
+  static constexpr uint32_t kMostWalkRanges = 4;
+  static constexpr uint32_t kMostStretches = 1024;  // of a pass whose rows leave early
 
   // Whether a pass brings the pairs into transit order (or, sample-parallel and no walk, only drops the dead ones).
   bool inverts(int mode) const {
@@ -2784,6 +2958,13 @@ class Engine : public EngineBase {
   // allocated).  Results do not depend on it.
   enum { kScheduleAuto = -1, kScheduleSerial = 0, kScheduleMerged = 1, kScheduleForked = 2 };
   static constexpr uint32_t kQueuedWavesPerCu = 12;
+  // Walks whose results are stored a line at a time (rows of whole fours of words only).  Four at a time, every one of them
+  // is a request of its own past L2 where the lines of all walks under way do not fit there: R-MAT 22 weighted node2vec 24.1 ->
+  // 22.7 ms, DeepWalk, a million walks over 10 K vertices, 1.63 -> 1.57, PPR over 262 K vertices 0.53 -> 0.49, MultiRW 100 K
+  // 0.65 -> 0.62.  Fewer walks wait for the chain of their steps, to which it adds: uniform walks 57 K 0.112 -> 0.126, 2.7 K
+  // 0.092 -> 0.112.  Ranges of a pass keep the fours too: stores straight to the host's memory are under way beside them, and
+  // PPR's two took 0.73 ms by lines instead of 0.67.
+  static constexpr uint32_t kLinesFromWalks = 64u << 10;
   // Edge arrays (as the walk would read them otherwise) from this size on are read as walk records: 4 and 8 bytes an
   // edge fit the caches then where 16 and 32 do not, and a step over a graph in the caches gains nothing from them
   // (32 MB is the L2 of all eight XCDs).  Uniform walks over 48 MB: 1.77 -> 1.49 ms; DeepWalk over 120 MB 3.37 -> 2.96,
@@ -2906,6 +3087,7 @@ class Engine : public EngineBase {
     rows_ahead = nullptr;
     for (hipEvent_t ev : range_ends_) (void)hipEventDestroy(ev);
     range_ends_.clear();
+    free_early_rows();
     drop_recorded_passes();
     release(d_initial_);
     release(d_samples_);
@@ -2980,9 +3162,12 @@ class Engine : public EngineBase {
   bool inversion_ready_ = false, walk_tables_ready_ = false;
   const WalkVertex* walk_vertices_ = nullptr;
   const walk_record<App>* walk_records_ = nullptr;  // dgraph_'s, where they pay
-  uint32_t walk_waves_at_once_ = 1, walk_waves_queued_ = 1;  // wavefronts of walk_rows_kernel
+  uint32_t walk_waves_at_once_ = 1, cus_ = 1;  // wavefronts of walk_rows_kernel the device holds, compute units
   bool ahead_ = false;                    // rows are on their way to rows_ahead
   std::vector<hipEvent_t> range_ends_;    // ends of the launches of such a pass
+  // of such a pass: EarlyRows::arrived and walked, and the number of the last
+  uint32_t *h_arrived_ = nullptr, *d_walked_ = nullptr;
+  uint32_t early_pass_ = 0;
   StepLayout layout_{};
   bool allocated_ = false;
 

@@ -11,9 +11,12 @@
 //    The kernel writes its output straight into page-locked memory (54.7 GB/s, as fast as the copy
 //    engine's 57, without a launch and a copy per piece), and host threads unpack a piece
 //    while the next one crosses.  Twelve threads write 220 GB/s of unpacked ids on the 16-core share of a
-//    GPU's host, eight 200.
+//    GPU's host, 140 while the bus writes to the same memory at its full rate.
 //  * Results whose first words are final while later ones are still being computed (walks) can leave then already
-//    (ResultStream::begin, with what to wait for).
+//    (ResultStream::begin, with what to wait for).  They are packed into device memory and the copy engine takes them
+//    from there: stores of a kernel that wait for the bus stand in the way of all others, and the computation took as much
+//    longer as the transfer saved (R-MAT 22 walks 24.1 ms alone, 26.9 with 32 such workgroups beside it, 34 with 512; 24.3
+//    with the copy engine at 55 GB/s).
 //  * The arrays results land in come from a small pool per sampler and keep their pages: a first
 //    touch costs 0.1-0.4 s per GB, more than the sampling.
 //  * Such an array can be given to the caller (HostLease) instead of being copied for them; it goes
@@ -363,19 +366,34 @@ constexpr uint32_t kPackMostBits = 25;                           // wider ids tr
 struct PackHeader {
   uint64_t live[kPackChunkGroups / 64];
   uint64_t overflow;
-  uint64_t pad[7];
+  uint64_t at;  // of its bytes among the piece's
+  uint64_t pad[6];
+};
+
+// Where the chunks' bytes go: chunk after chunk, each as far from the last as a whole one takes, or (staged) one directly
+// after another, in whatever order the workgroups get there, for a copy that is to take no more than there is.
+struct PackedOut {
+  uint8_t* bytes;
+  PackHeader* headers;
+  // staged
+  uint32_t* cursor = nullptr;    // 16 bytes each; 0 before the launch and after it
+  uint32_t* finished = nullptr;  // workgroups; likewise
+  uint32_t* total = nullptr;     // host memory: what cursor was at the end
 };
 
 // Packs ids [chunk * kPackChunk, ...) of src into out[chunk * kPackChunkGroups * bits ...): the groups of
-// eight that are not all `fill`, back to back, `bits` bytes each.  out and headers are host memory, and the
+// eight that are not all `fill`, back to back, `bits` bytes each.  Where out is host memory the
 // stores to it are what takes the time (54.7 GB/s of packed bytes; packing the 1.68 GB of R-MAT 22 walks into
-// device memory instead would take a twentieth of it), hence whole chunks through LDS and 16-byte stores by
-// consecutive lanes; nothing else here is tuned.
+// device memory instead takes a twentieth of it), hence whole chunks through LDS and 16-byte stores by
+// consecutive lanes; nothing else here is tuned.  (kStaged is the kernel's and not the launch's: with both forms' loads in one
+// kernel those of a chunk wait for each other, and MultiRW 100 K took 1.59 ms instead of 1.55, KHop over R-MAT 20 11.7 instead
+// of 11.4.)
+template <bool kStaged>
 __global__ __launch_bounds__(kPackThreads) void pack_results(const int32_t* __restrict__ src, size_t n, uint32_t bits,
-                                                             int32_t fill, uint8_t* __restrict__ out,
-                                                             PackHeader* __restrict__ headers, uint32_t n_chunks) {
+                                                             int32_t fill, PackedOut out, uint32_t n_chunks) {
   __shared__ __align__(16) uint8_t s_packed[kPackChunk * sizeof(int32_t)];
   __shared__ uint64_t s_live[kPackChunkGroups / 64];
+  __shared__ uint32_t s_at;
   constexpr uint32_t kRounds = kPackChunkGroups / kPackThreads;
   const uint32_t lane = threadIdx.x & 63u;
   for (uint32_t chunk = blockIdx.x; chunk < n_chunks; chunk += gridDim.x) {
@@ -387,12 +405,26 @@ __global__ __launch_bounds__(kPackThreads) void pack_results(const int32_t* __re
     for (uint32_t r = 0; r < kRounds; ++r) {
       const size_t at = first + (size_t)(r * kPackThreads + threadIdx.x) * kPackGroup;
       if (at + kPackGroup <= n) {
-        const int4 lo = *reinterpret_cast<const int4*>(src + at), hi = *reinterpret_cast<const int4*>(src + at + 4);
+        int4 lo, hi;
+        if (kStaged) {
+          // Words of a kernel that is still running, which stored them past its caches: they are read past this one's.  (A fence
+          // that empties the caches would empty them for that kernel too: DeepWalk, a million walks, 2.3 -> 3.1 ms.)
+          const uint64_t* from = reinterpret_cast<const uint64_t*>(src + at);
+          uint64_t two[4];
+#pragma unroll
+          for (uint32_t i = 0; i < 4; ++i) two[i] = __hip_atomic_load(from + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+          lo = make_int4((int)two[0], (int)(two[0] >> 32), (int)two[1], (int)(two[1] >> 32));
+          hi = make_int4((int)two[2], (int)(two[2] >> 32), (int)two[3], (int)(two[3] >> 32));
+        } else {
+          lo = *reinterpret_cast<const int4*>(src + at);
+          hi = *reinterpret_cast<const int4*>(src + at + 4);
+        }
         ids[r][0] = lo.x; ids[r][1] = lo.y; ids[r][2] = lo.z; ids[r][3] = lo.w;
         ids[r][4] = hi.x; ids[r][5] = hi.y; ids[r][6] = hi.z; ids[r][7] = hi.w;
       } else {
 #pragma unroll
-        for (uint32_t i = 0; i < kPackGroup; ++i) ids[r][i] = at + i < n ? src[at + i] : fill;
+        for (uint32_t i = 0; i < kPackGroup; ++i)
+          ids[r][i] = at + i >= n ? fill : kStaged ? __hip_atomic_load(src + at + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) : src[at + i];
       }
       live[r] = false;
 #pragma unroll
@@ -435,14 +467,25 @@ __global__ __launch_bounds__(kPackThreads) void pack_results(const int32_t* __re
         }
       }
     }
-    __syncthreads();
-    uint8_t* chunk_out = out + (size_t)chunk * kPackChunkGroups * bits;
     const uint32_t words = (total * bits + 15u) / 16u;
+    if (kStaged && threadIdx.x == 0) s_at = atomicAdd(out.cursor, words);
+    __syncthreads();
+    const size_t at = kStaged ? (size_t)s_at * 16u : (size_t)chunk * kPackChunkGroups * bits;
+    uint8_t* chunk_out = out.bytes + at;
     for (uint32_t i = threadIdx.x; i < words; i += kPackThreads)
       reinterpret_cast<uint4*>(chunk_out)[i] = reinterpret_cast<const uint4*>(s_packed)[i];
-    if (threadIdx.x < kPackChunkGroups / 64) headers[chunk].live[threadIdx.x] = s_live[threadIdx.x];
-    if (threadIdx.x == kPackChunkGroups / 64) headers[chunk].overflow = (uint64_t)any_overflow;
+    if (threadIdx.x < kPackChunkGroups / 64) out.headers[chunk].live[threadIdx.x] = s_live[threadIdx.x];
+    if (threadIdx.x == kPackChunkGroups / 64) {
+      out.headers[chunk].overflow = (uint64_t)any_overflow;
+      out.headers[chunk].at = at;
+    }
     __syncthreads();  // the next chunk overwrites what has just been read
+  }
+  if (kStaged && threadIdx.x == 0 && atomicAdd(out.finished, 1u) == gridDim.x - 1) {
+    // the last workgroup: the others' claims were answered before they counted themselves
+    __hip_atomic_store(out.total, atomicAdd(out.cursor, 0u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    *out.cursor = 0;
+    *out.finished = 0;
   }
 }
 
@@ -578,7 +621,7 @@ inline hipError_t device_of(hipStream_t stream, int* device) {
   return stream ? hipStreamGetDevice(stream, device) : hipGetDevice(device);
 }
 
-// The stream results cross the bus on while something else is computed: one per device (which has to be the current one) and process, on
+// The streams results cross the bus on while something else is computed: two per device (which has to be the current one) and process, each on
 // a hardware queue of its own, which a stream with a mask of compute units (here: all) gets.  (Ordinary streams share
 // four; where the computation's lands on the same one, nothing overlaps.)  They are destroyed when the process ends, while
 // the runtime and whatever watches it are still there: left to the runtime, their queues outlive a profiler's
@@ -595,12 +638,13 @@ inline std::vector<hipStream_t>& transfer_streams() {
   }();
   return *streams;
 }
-inline hipStream_t transfer_stream(int device) {
+inline hipStream_t transfer_stream(int device, size_t which) {
   static std::mutex mutex;
   std::vector<hipStream_t>* streams = &transfer_streams();
   std::lock_guard<std::mutex> lock(mutex);
-  if (streams->size() <= (size_t)device) streams->resize((size_t)device + 1, nullptr);
-  hipStream_t& stream = (*streams)[(size_t)device];
+  const size_t at = 2 * (size_t)device + which;
+  if (streams->size() <= at) streams->resize(at + 1, nullptr);
+  hipStream_t& stream = (*streams)[at];
   if (!stream) {
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus <= 0) return nullptr;
@@ -625,10 +669,14 @@ class ResultStream {
   ResultStream& operator=(const ResultStream&) = delete;
   ~ResultStream() { release(); }
 
-  // The first `words` words of a result are on the device once `event` has happened.
+  // The first `words` words of a result are on the device once `event` has happened, or, if there is a `sign` (all of a
+  // transfer's have one or none has; page-locked memory a kernel that is still running writes to, after the words), once that is
+  // `value`.
   struct Ready {
     size_t words;
     hipEvent_t event;
+    const uint32_t* sign = nullptr;
+    uint32_t value = 0;
   };
 
   // Takes, on the current device and ahead of the first, what a copy() or a fetch() of n words needs.
@@ -687,10 +735,11 @@ class ResultStream {
     if (on.error != hipSuccess) return on.error;
     t.set(src, n, bits > kPackMostBits ? 32 : bits, fill, dst, std::move(ready));
     e = prepare(t.slot_bytes);
+    if (e == hipSuccess && t.staged) e = prepare_staging(t.slot_bytes);
     if (e != hipSuccess) return e;
-    t.streams[0] = t.streams[1] = transfer_stream(t.device);
+    // pieces alternate between two streams, so that the bus is not idle between two of them
+    for (size_t which = 0; which < 2; ++which) t.streams[which] = transfer_stream(t.device, which);
     if (t.ready.empty()) {
-      // pieces alternate between two streams, so that the bus is not idle between two launches
       t.streams[0] = stream;
       e = hipEventRecord(begun_, stream);
       if (e == hipSuccess) e = hipStreamWaitEvent(t.streams[1], begun_, 0);
@@ -733,6 +782,7 @@ class ResultStream {
   void release_device() {
     for (hipEvent_t& ev : packed_)
       if (ev) (void)hipEventDestroy(ev), ev = nullptr;
+    release_staging();
     if (begun_) (void)hipEventDestroy(begun_);
     begun_ = nullptr;
     if (ring_) (void)hipHostFree(ring_);
@@ -743,15 +793,16 @@ class ResultStream {
   static constexpr size_t kSlots = 8;
   // Chunks of a piece: at most 8 MB of results (0.1 ms on the bus, long against a launch and an event; with pieces of
   // 16 MB the ring no longer stays in the last-level cache between the bus and the threads: 1.68 GB in 16 instead of 14
-  // ms).  The first one is 1 MB and each of the next twice as long, so that the threads have something to do soon, and
+  // ms; the copy engine, which rests 8 us between two copies, gets 16 MB all the same).  The first one is 1 MB and each of the next twice as long, so that the threads have something to do soon, and
   // none is more than a third of what is left, so that little is left to do when the last one arrives.
-  static constexpr size_t kMostChunks = 512, kLeastChunks = 64;
+  static constexpr size_t kMostChunks = 512, kMostStagedChunks = 1024, kLeastChunks = 64;
   static constexpr size_t kChunksAtOnce = 4;  // what a thread takes; kLeastChunks is a multiple
-  // Workgroups of a launch of pack_results, and launches under way, while something else is computed: stores that wait
-  // for the bus stand in the way of that something's own.  R-MAT 22 walks in four ranges, sampling / with their
-  // rows here: 512 workgroups 34.1 / 38.6 ms, 64 30.5 / 35.2, 48 29.0 / 33.1, 32 26.9 / 31.0, 24 26.9 / 32.2.
+  // Workgroups of a launch of pack_results that goes straight to the ring, and launches under way, while something else is
+  // computed: stores that wait for the bus stand in the way of that something's own.
   static constexpr uint32_t kGentleBlocks = 32;
   static constexpr size_t kGentleAhead = 2;
+  static constexpr size_t kPackedAhead = 3;     // pieces packed before the copy engine has come to them
+  static constexpr int kSignsPerQuery = 1024;   // looks at a sign for one at the event beside it: some 20 us
   static constexpr int kSpins = 4000;  // tens of microseconds; none: 1.68 GB in 19 instead of 13 ms, 23 MB in 527 instead of 290 us
 
   hipError_t come_to_device_of(hipStream_t stream) {
@@ -786,6 +837,44 @@ class ResultStream {
     return make_ring(slot_bytes * kSlots);
   }
 
+  // What pieces that are packed in device memory take.
+  hipError_t prepare_staging(size_t slot_bytes) {
+    for (hipEvent_t& ev : copied_)
+      if (!ev) {
+        const hipError_t e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+        if (e != hipSuccess) return e;
+      }
+    hipError_t e = hipSuccess;
+    if (!totals_) e = hipHostMalloc((void**)&totals_, kSlots * sizeof(uint32_t), hipHostMallocDefault);
+    if (e == hipSuccess && !counts_) {
+      e = hipMalloc(&counts_, 2 * kSlots * kWordsPerLine * sizeof(uint32_t));
+      // on a stream of their own: the computation is not waited for
+      const hipStream_t stream = transfer_stream(device_, 0);
+      if (e == hipSuccess) e = hipMemsetAsync(counts_, 0, 2 * kSlots * kWordsPerLine * sizeof(uint32_t), stream);
+      if (e == hipSuccess) e = hipStreamSynchronize(stream);
+    }
+    if (e == hipSuccess && staging_bytes_ < slot_bytes * kSlots) {
+      if (staging_) (void)hipFree(staging_);
+      staging_ = nullptr;
+      staging_bytes_ = 0;
+      e = hipMalloc(&staging_, slot_bytes * kSlots);
+      if (e == hipSuccess) staging_bytes_ = slot_bytes * kSlots;
+    }
+    if (e != hipSuccess) release_staging();
+    return e;
+  }
+  void release_staging() {
+    for (hipEvent_t& ev : copied_)
+      if (ev) (void)hipEventDestroy(ev), ev = nullptr;
+    if (totals_) (void)hipHostFree(totals_);
+    totals_ = nullptr;
+    if (counts_) (void)hipFree(counts_);
+    counts_ = nullptr;
+    if (staging_) (void)hipFree(staging_);
+    staging_ = nullptr;
+    staging_bytes_ = 0;
+  }
+
   struct Transfer {
     const int32_t* src;
     size_t n;
@@ -794,12 +883,14 @@ class ResultStream {
     int32_t* dst;
     hipStream_t streams[2];
     std::vector<Ready> ready;
+    bool staged = false;  // pieces are packed in device memory, for the copy engine, while something else is computed
     int device = 0;
 
     size_t chunks, pieces, chunk_bytes, packed_at, slot_bytes;
     std::vector<size_t> begins;        // first chunk of every piece, and the end of the last
     std::vector<uint32_t> piece_of;    // of every kLeastChunks chunks
     size_t happened;                   // of `ready`
+    bool computed;                     // all of it
     UnpackPlan plan{32};
     std::atomic<bool> driven{false};   // a thread has taken the launching on
     std::atomic<size_t> next{0};       // chunk to take
@@ -813,12 +904,14 @@ class ResultStream {
 
     void set(const int32_t* src_, size_t n_, uint32_t bits_, int32_t fill_, int32_t* dst_, std::vector<Ready> ready_) {
       src = src_, n = n_, bits = bits_, fill = fill_, dst = dst_, ready = std::move(ready_);
+      staged = !ready.empty() && ready.front().sign != nullptr;
       happened = 0;
+      computed = false;
       chunks = (n + kPackChunk - 1) / kPackChunk;
       begins.clear();
       piece_of.clear();
       size_t most = kLeastChunks, longest = 0;
-      for (size_t at = 0; at < chunks; most = std::min(kMostChunks, most * 2)) {
+      for (size_t at = 0; at < chunks; most = std::min(staged ? kMostStagedChunks : kMostChunks, most * 2)) {
         const size_t third = ((chunks - at) / 3 + kLeastChunks - 1) / kLeastChunks * kLeastChunks;
         const size_t here = std::max(kLeastChunks, std::min(most, third));
         piece_of.insert(piece_of.end(), here / kLeastChunks, (uint32_t)begins.size());
@@ -870,8 +963,18 @@ class ResultStream {
   bool readable(size_t piece, bool waits, hipError_t* error) {
     Transfer& t = *transfer_;
     while (t.happened < t.ready.size() && (t.happened == 0 || t.ready[t.happened - 1].words < piece_end(piece))) {
-      const hipEvent_t ev = t.ready[t.happened].event;
-      const hipError_t e = waits ? hipEventSynchronize(ev) : hipEventQuery(ev);
+      const Ready& next = t.ready[t.happened];
+      hipError_t e = hipErrorNotReady;
+      if (!next.sign) {
+        e = waits ? hipEventSynchronize(next.event) : hipEventQuery(next.event);
+      } else {
+        for (;;) {
+          if (__atomic_load_n(next.sign, __ATOMIC_ACQUIRE) == next.value) e = hipSuccess;
+          else if (looks_++ % kSignsPerQuery == 0) e = hipEventQuery(next.event);  // the kernel may have ended, or failed
+          if (e != hipErrorNotReady || !waits) break;
+          spin_pause();
+        }
+      }
       if (e == hipErrorNotReady) return false;
       if (e != hipSuccess) {
         *error = e;
@@ -883,22 +986,40 @@ class ResultStream {
   }
 
   // Whether nothing is being computed any more that the transfer could be in the way of.
-  bool alone() const {
-    const Transfer& t = *transfer_;
-    return t.happened == t.ready.size() || hipEventQuery(t.ready.back().event) == hipSuccess;
+  bool computed() {
+    Transfer& t = *transfer_;
+    if (!t.computed) t.computed = t.ready.empty() || hipEventQuery(t.ready.back().event) == hipSuccess;
+    return t.computed;
   }
 
-  hipError_t launch(size_t piece, bool gently) {
+  hipError_t launch(size_t piece, uint32_t most_blocks = UINT32_MAX) {
     const Transfer& t = *transfer_;
     const size_t first = t.begins[piece] * kPackChunk;
-    const size_t here = piece_end(piece) - first;
-    uint8_t* at = slot(piece);
+    const size_t here = piece_end(piece) - first, slot_of = piece % kSlots;
+    uint8_t* at = t.staged ? staging_ + slot_of * t.slot_bytes : slot(piece);
     const uint32_t n_chunks = (uint32_t)((here + kPackChunk - 1) / kPackChunk);
-    const hipStream_t stream = t.streams[piece % 2];
-    pack_results<<<dim3(gently ? std::min(n_chunks, kGentleBlocks) : n_chunks), dim3(kPackThreads), 0, stream>>>(
-        t.src + first, here, t.bits, t.fill, at + t.packed_at, (PackHeader*)at, n_chunks);
+    const hipStream_t stream = t.streams[t.staged ? 0 : piece % 2];  // (a copy on it would be waited for)
+    PackedOut out{at + t.packed_at, (PackHeader*)at};
+    if (t.staged) {
+      out.cursor = counts_ + 2 * slot_of * kWordsPerLine;
+      out.finished = out.cursor + kWordsPerLine;
+      out.total = totals_ + slot_of;
+    }
+    const dim3 grid(std::min(n_chunks, most_blocks)), block(kPackThreads);
+    if (t.staged) pack_results<true><<<grid, block, 0, stream>>>(t.src + first, here, t.bits, t.fill, out, n_chunks);
+    else pack_results<false><<<grid, block, 0, stream>>>(t.src + first, here, t.bits, t.fill, out, n_chunks);
     const hipError_t e = hipGetLastError();
-    return e != hipSuccess ? e : hipEventRecord(packed_[piece % kSlots], stream);
+    return e != hipSuccess ? e : hipEventRecord(packed_[slot_of], stream);
+  }
+
+  // Sends a piece that is packed in device memory on its way.
+  hipError_t copy_piece(size_t piece) {
+    const Transfer& t = *transfer_;
+    const size_t slot_of = piece % kSlots;
+    const hipStream_t stream = t.streams[1];
+    const size_t bytes = t.packed_at + 16 * (size_t)__atomic_load_n(totals_ + slot_of, __ATOMIC_RELAXED);
+    const hipError_t e = hipMemcpyAsync(slot(piece), staging_ + slot_of * t.slot_bytes, bytes, hipMemcpyDeviceToHost, stream);
+    return e != hipSuccess ? e : hipEventRecord(copied_[slot_of], stream);
   }
 
   // unpacks the chunks [c, end) of a piece that is here
@@ -911,7 +1032,7 @@ class ResultStream {
       const PackHeader& header = ((const PackHeader*)at)[in_piece];
       if (header.overflow) t.overflow.store(true, std::memory_order_relaxed);
       const size_t first = i * kPackChunk;
-      unpack_chunk(t.plan, header, at + t.packed_at + in_piece * t.chunk_bytes, t.fill, t.dst + first,
+      unpack_chunk(t.plan, header, at + t.packed_at + header.at, t.fill, t.dst + first,
                    std::min<size_t>(kPackChunk, t.n - first));
     }
     unpack_fence();
@@ -931,31 +1052,22 @@ class ResultStream {
     }
   }
 
-  // Launches the packing of pieces, up to kSlots of them under way at a time, and announces them as they arrive.
+  // Whether a piece's slot is free: the piece before it there is unpacked.  If not, does some of that (of pieces that are here).
+  bool slot_is_free(size_t piece, size_t here) {
+    Transfer& t = *transfer_;
+    if (piece < kSlots || t.left[piece - kSlots].load(std::memory_order_acquire) == 0) return true;
+    size_t c = t.next.load();
+    if (c < t.begins[here] && t.next.compare_exchange_strong(c, c + kChunksAtOnce)) unpack(c, std::min(c + kChunksAtOnce, t.chunks));
+    else std::this_thread::yield();
+    return false;
+  }
+
+  // Has all pieces packed and announces them as they arrive.
   void drive() {
     Transfer& t = *transfer_;
     const OnDevice on(t.device);
     hipError_t error = on.error;
-    size_t launched = 0;
-    bool gently = true;
-    for (size_t p = 0; p < t.pieces && error == hipSuccess; ++p) {
-      while (launched < t.pieces && error == hipSuccess && readable(launched, /*waits=*/launched == p, &error)) {
-        gently = gently && !alone();
-        if (launched >= p + (gently ? kGentleAhead : kSlots)) break;
-        // its slot is free once the piece before it there is unpacked
-        while (launched >= kSlots && t.left[launched - kSlots].load(std::memory_order_acquire) != 0) {
-          const size_t c = t.next.load();
-          size_t mine = c;
-          if (c < t.begins[p] && t.next.compare_exchange_strong(mine, c + kChunksAtOnce))
-            unpack(c, std::min(c + kChunksAtOnce, t.chunks));
-          else
-            std::this_thread::yield();
-        }
-        error = launch(launched++, gently);
-      }
-      if (error == hipSuccess) error = hipEventSynchronize(packed_[p % kSlots]);
-      if (error == hipSuccess) t.announce(p + 1, false);
-    }
+    if (error == hipSuccess) error = t.staged ? drive_staged() : drive_straight();
     if (error != hipSuccess) {
       t.error = error;
       (void)hipGetLastError();  // reported by finish(), not to this thread's next launch
@@ -963,13 +1075,76 @@ class ResultStream {
     }
   }
 
+  // Up to kSlots pieces under way at a time, straight to the ring; few, and of few workgroups, while something is computed.
+  hipError_t drive_straight() {
+    Transfer& t = *transfer_;
+    hipError_t error = hipSuccess;
+    size_t launched = 0;
+    bool gently = !t.ready.empty();
+    if (t.ready.size() == 1) {
+      // all of it at once: the device waits, without a way over this thread
+      for (hipStream_t stream : t.streams)
+        if (error == hipSuccess) error = hipStreamWaitEvent(stream, t.ready[0].event, 0);
+      t.happened = 1;
+      gently = false;
+    } else if (gently) {
+      t.streams[1] = t.streams[0];
+    }
+    for (size_t p = 0; p < t.pieces && error == hipSuccess; ++p) {
+      while (launched < t.pieces && error == hipSuccess && readable(launched, /*waits=*/launched == p, &error)) {
+        gently = gently && !computed();
+        if (launched >= p + (gently ? kGentleAhead : kSlots)) break;
+        while (!slot_is_free(launched, p)) {}
+        error = launch(launched++, gently ? kGentleBlocks : UINT32_MAX);
+      }
+      if (error == hipSuccess) error = hipEventSynchronize(packed_[p % kSlots]);
+      if (error == hipSuccess) t.announce(p + 1, false);
+    }
+    return error;
+  }
+
+  // A few pieces packed ahead of the copy engine, as they become readable and as slots become free.
+  hipError_t drive_staged() {
+    Transfer& t = *transfer_;
+    size_t launched = 0, sent = 0, here = 0;
+    while (here < t.pieces) {
+      hipError_t e = hipSuccess;
+      bool moved = false;
+      if (launched < t.pieces && launched < sent + kPackedAhead && readable(launched, /*waits=*/here == launched, &e) &&
+          slot_is_free(launched, here)) {
+        e = launch(launched++);
+        moved = true;
+      }
+      if (e != hipSuccess) return e;
+      if (sent < launched && (e = hipEventQuery(packed_[sent % kSlots])) != hipErrorNotReady) {
+        if (e == hipSuccess) e = copy_piece(sent++);
+        if (e != hipSuccess) return e;
+        moved = true;
+      }
+      if (here < sent && (e = hipEventQuery(copied_[here % kSlots])) != hipErrorNotReady) {
+        if (e != hipSuccess) return e;
+        t.announce(++here, false);
+        moved = true;
+      }
+      if (!moved) spin_pause();
+    }
+    return hipSuccess;
+  }
+
   std::unique_ptr<Transfer> transfer_;
   HostWorkers::Job job_;
   bool under_way_ = false, misfit_ = false;
   int device_ = -1;  // of the events and the ring
+  uint32_t looks_ = 0;
   uint8_t* ring_ = nullptr;
   size_t ring_bytes_ = 0;
   hipEvent_t packed_[kSlots] = {}, begun_ = nullptr;
+  // of pieces that are packed in device memory
+  static constexpr size_t kWordsPerLine = 32;
+  hipEvent_t copied_[kSlots] = {};
+  uint8_t* staging_ = nullptr;
+  size_t staging_bytes_ = 0;
+  uint32_t *counts_ = nullptr, *totals_ = nullptr;
 };
 
 }  // namespace nd

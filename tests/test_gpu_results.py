@@ -192,3 +192,26 @@ def test_rows_of_every_kind_of_walk_leave_before_the_pass_is_over(oracle, app, k
                 assert np.array_equal(states_of()[alive], want_states[alive])
     finally:
         s.close()
+
+
+# rows as lines of memory: one walk more than are stored by fours, rows that end within a line and share it with the next,
+# walks that end after a step, a stretch of one walk, and as many walks as leave by range or by stretch
+@pytest.mark.parametrize("app,kind,n,isolated_every", [
+    ("UniformRandomWalk", "UNIFORM_WALK", 65536, 7),
+    ("UniformRandomWalk", "UNIFORM_WALK", 65537, 2),
+    ("PPRPerVertex", "PPR", 458752, 3),
+    ("WeightedNode2Vec", "WEIGHTED_NODE2VEC", 98304, 0),
+    ("WeightedNode2Vec", "WEIGHTED_NODE2VEC", 98305, 3),
+])
+def test_rows_that_are_stored_by_lines(oracle, app, kind, n, isolated_every):
+    g = graphs.random_graph(n=n, mean_degree=3, seed=n, isolated_every=isolated_every)
+    s = nd.Sampler(app, g, seed=42)
+    try:
+        d = oracle.app_desc(getattr(oracle, kind), s.steps, [s.step_size(k) for k in range(s.steps)], p=2.0, q=0.5)
+        want, _ = oracle.sample_individual(graphs.oracle_view(g), d, 42, s.initial_contents)
+        for turn in range(3):
+            print("app", app, "n", n, "turn", turn, flush=True)
+            s.do_transit_parallel()
+            assert np.array_equal(s.final_samples(), want)
+    finally:
+        s.close()
