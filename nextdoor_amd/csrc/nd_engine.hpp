@@ -806,19 +806,24 @@ using walk_record = std::conditional_t<app_uses_weights<App>::value, WeightedWal
 // What a walk needs of the vertex it has come to.  One 16-byte record where the largest weight is needed
 // (DeepWalk over 10 K vertices 1.71 -> 1.60 ms, over 1 M 3.84 -> 3.37, R-MAT 22 weighted node2vec 24.6 -> 24.1); the two
 // row positions alone are better off in their own array of 4 bytes a vertex (uniform walks over 1 M: 1.77, not 1.97 ms).
+// (*end: where its edges end, or how many they are: vertex_degree(), once it is needed and not while it is loaded.)
 template <class App>
 __device__ __forceinline__ void enter_vertex(const CSRPartition& csr, const WalkVertex* __restrict__ vertices, VertexID v,
-                                             EdgePos_t* begin, EdgePos_t* n_edges, float* max_weight) {
+                                             EdgePos_t* begin, EdgePos_t* end, float* max_weight) {
   if constexpr (app_uses_weights<App>::value) {
     const WalkVertex r = vertices[v];
     *begin = r.begin;
-    *n_edges = r.n_edges;
+    *end = r.n_edges;
     *max_weight = r.max_weight;
   } else {
     *begin = csr.row_ptr[v];
-    *n_edges = csr.row_ptr[v + 1] - *begin;
+    *end = csr.row_ptr[v + 1];
     *max_weight = csr.max_weights[v];
   }
+}
+template <class App>
+__device__ __forceinline__ EdgePos_t vertex_degree(EdgePos_t begin, EdgePos_t end) {
+  return app_uses_weights<App>::value ? end : end - begin;
 }
 
 // Rows that leave while later ones are still being walked (stretch: 2^shift consecutive walks).  A stretch's rows are in
@@ -867,6 +872,11 @@ __device__ __forceinline__ void store_one(int32_t* at, VertexID v, bool past_cac
 // 4.0, R-MAT 22 34.5 / 24.1, four walks a vertex over 700 K 27.6 / 14.5.  There is no case among them where
 // the order is worth what it costs.
 //
+// Few walks are bound by the chain of a step: the vertex, a random number, the edge.  The random numbers of the next step depend on
+// neither load, and are computed while the edge is on its way (apps that never try again), or the vertex: uniform walks
+// 2.7 K 0.092 -> 0.065 ms, 57 K 0.113 -> 0.089, weighted node2vec 30 K 0.58 -> 0.565.  (While the vertex is on its way only: 0.084
+// and 0.102.  Half of the rounds with each of the two loads: 0.065 and 0.090.)
+//
 // Results go to the rows a line of memory at a time, or four at a time (Engine::kLinesFromWalks).  Where rows leave early they are
 // stored past the L2 (EarlyRows).
 //
@@ -894,11 +904,11 @@ __global__ __launch_bounds__(kFlatThreads) void walk_rows_kernel(StepParams P, i
   uint32_t block_end = block + kWave < n_walks ? block + kWave : n_walks;
   bool more = (uint64_t)n_waves * kWave < n_walks;
   const bool queued = more;
-  bool busy = false, fresh = false, first = false;
+  bool busy = false, first = false;
   uint32_t slot = 0;
   int step = 0;
   VertexID transit = P.invalid, r0 = P.invalid, r1 = P.invalid, r2 = P.invalid, r3 = P.invalid;  // the last four results
-  EdgePos_t begin = 0, n_edges = 0;
+  EdgePos_t begin = 0, end = 0;
   float max_weight = 0.0f;
   curandState rng;
   rng.reset(0, 0, 0);
@@ -956,9 +966,10 @@ __global__ __launch_bounds__(kFlatThreads) void walk_rows_kernel(StepParams P, i
           state = (SampleType*)P.samples + slot;
         }
         step = 0;
-        busy = fresh = true;
-        n_edges = 0;
-        if (transit != P.invalid) enter_vertex<App>(csr, vertices, transit, &begin, &n_edges, &max_weight);
+        busy = first = true;
+        rng.reset(P.seed, P.first_slot + slot, 0);
+        begin = end = 0;
+        if (transit != P.invalid) enter_vertex<App>(csr, vertices, transit, &begin, &end, &max_weight);
       }
       const uint32_t asked = (uint32_t)__popcll(idle);
       block = block_end - block > asked ? block + asked : block_end;
@@ -969,10 +980,7 @@ __global__ __launch_bounds__(kFlatThreads) void walk_rows_kernel(StepParams P, i
     }
     bool ended = false, four_done = false;
     if (busy) {
-      if (fresh) {
-        rng.reset(P.seed, P.first_slot + slot, (uint32_t)step);
-        first = true;
-      }
+      const EdgePos_t n_edges = vertex_degree<App>(begin, end);
       VertexID r = -1;
       bool decided = true;
       if (n_edges != 0) {  // next() only runs for a transit that has edges (nextdoor.cu:250-262)
@@ -1006,7 +1014,14 @@ __global__ __launch_bounds__(kFlatThreads) void walk_rows_kernel(StepParams P, i
           first = false;
         }
       }
-      fresh = decided;
+      // The random numbers of the next step, while the edge is loaded (ten rounds of multiplications), or, where it has still to
+      // be found out whether there is one, while its vertex or the next try's is.
+      constexpr bool kOneTry = !app_tries_one_candidate<App>::value;
+      if (kOneTry && !explicit_transits) {
+        rng.reset(P.seed, P.first_slot + slot, (uint32_t)step + 1u);
+        rng.compute_block();
+        asm volatile("" : "+v"(r), "+v"(rng.word0));  // (the compiler would do that when the edge is there)
+      }
       if (decided) {
         const VertexID neighbor = r == -1 ? P.invalid : r;  // nextdoor.cu:288
         r0 = r1;
@@ -1032,13 +1047,16 @@ __global__ __launch_bounds__(kFlatThreads) void walk_rows_kernel(StepParams P, i
         if (!ended) {
           if (kRecords && n_edges != 0 && last.dst == transit) {
             begin = last.begin;
-            n_edges = last.n_edges;
+            end = app_uses_weights<App>::value ? last.n_edges : begin + last.n_edges;
             max_weight = last.max_weight;
           } else {
-            enter_vertex<App>(csr, vertices, transit, &begin, &n_edges, &max_weight);
+            enter_vertex<App>(csr, vertices, transit, &begin, &end, &max_weight);
           }
+          if (!kOneTry || explicit_transits) rng.reset(P.seed, P.first_slot + slot, (uint32_t)step);
+          first = true;
         }
       }
+      if ((!kOneTry || explicit_transits) && rng.left == 0) rng.compute_block();
     }
     // the lines that are full, or whose walk has ended
     auto flush_lines = [&](bool has_ended) {

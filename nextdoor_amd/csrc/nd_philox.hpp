@@ -114,7 +114,8 @@ ND_HD uint32_t block_word(const PhiloxBlock& b, uint32_t i) {
 // Cursor over the draws of one (slot, step).  This is the object an App's next()
 // receives as its random-state handle.
 struct RandState {
-  uint32_t slot_lo, slot_hi, step, draw;  // draw: draws taken from the slot's own stream
+  uint32_t slot_lo, slot_hi, step;
+  uint32_t next_block, left;  // of the slot's own stream: the block after word0..3, and how many of those are there
   uint32_t key0, key1;
   uint32_t first_word;  // grouped form: the word of the shared block, until it is drawn
   uint32_t has_first;
@@ -128,7 +129,8 @@ struct RandState {
     slot_lo = (uint32_t)slot;
     slot_hi = (uint32_t)(slot >> 32);
     step = step_;
-    draw = 0;
+    next_block = 0;
+    left = 0;
     key0 = (uint32_t)seed;
     key1 = (uint32_t)(seed >> 32);
     word0 = word1 = word2 = word3 = 0;
@@ -148,19 +150,24 @@ struct RandState {
     reset_with_first(seed, slot, step_, block_word(grouped_first_block(seed, slot >> 2, step_), (uint32_t)slot & 3u));
   }
 
+  // What the next draw does if no word is left: a caller with nothing to do until a load returns does it then.
+  ND_HD void compute_block() {
+    const PhiloxBlock b = philox4x32_10(slot_lo, slot_hi, step, next_block, key0, key1);
+    word0 = b.w[0];
+    word1 = b.w[1];
+    word2 = b.w[2];
+    word3 = b.w[3];
+    ++next_block;
+    left = 4;
+  }
+
   ND_HD uint32_t next_word() {
     if (has_first) {
       has_first = 0;
       return first_word;
     }
-    if ((draw & 3u) == 0) {
-      const PhiloxBlock b = philox4x32_10(slot_lo, slot_hi, step, draw >> 2, key0, key1);
-      word0 = b.w[0];
-      word1 = b.w[1];
-      word2 = b.w[2];
-      word3 = b.w[3];
-    }
-    ++draw;
+    if (left == 0) compute_block();
+    --left;
     const uint32_t word = word0;
     word0 = word1;
     word1 = word2;
