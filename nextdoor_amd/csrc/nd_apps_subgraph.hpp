@@ -76,16 +76,31 @@ struct MVSSamplingAppT : nd::apps::SubgraphCommon<kBatch> {
                                   const VertexID_t neighbrID, curandState*) {
     const VertexID_t row = transits[0];
     EdgePos_t e = neighbrID;
-    // a hub keeps its lanes busy for thousands of rounds: fetch eight edges before handing
-    // them over, so that eight loads are under way instead of one
-    for (; e + 7 * kBatch < numEdges; e += 8 * kBatch) {
-      VertexID_t ahead[8];
+    // a hub keeps its lanes busy for hundreds of rounds: fetch eight edges before handing over the eight before them
+    if (e + 7 * kBatch < numEdges) {
+      VertexID_t now[8], ahead[8];
 #pragma unroll
-      for (int i = 0; i < 8; i++) ahead[i] = transitEdges[e + i * kBatch];
+      for (int i = 0; i < 8; i++) now[i] = transitEdges[e + i * kBatch];
+      for (e += 8 * kBatch; e + 7 * kBatch < numEdges; e += 8 * kBatch) {
 #pragma unroll
-      for (int i = 0; i < 8; i++) sample->emit(row, ahead[i]);
+        for (int i = 0; i < 8; i++) ahead[i] = transitEdges[e + i * kBatch];
+#pragma unroll
+        for (int i = 0; i < 8; i++) sample->emit(row, now[i]);
+#pragma unroll
+        for (int i = 0; i < 8; i++) now[i] = ahead[i];
+      }
+#pragma unroll
+      for (int i = 0; i < 8; i++) sample->emit(row, now[i]);
     }
-    for (; e < numEdges; e += kBatch) sample->emit(row, transitEdges[e]);
+    // the lane's last edges, four at a time (the last one again for those it does not have)
+    for (; e < numEdges; e += 4 * kBatch) {
+      VertexID_t ahead[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) ahead[i] = transitEdges[e + i * kBatch < numEdges ? e + i * kBatch : numEdges - 1];
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        if (e + i * kBatch < numEdges) sample->emit(row, ahead[i]);
+    }
     return -1;
   }
 

@@ -116,3 +116,30 @@ def test_other_apps_have_no_edge_lists():
     with pytest.raises(nd.NextDoorError):
         s.adjacency()
     s.close()
+
+
+# degrees beside each other in a unit: lanes without an edge, with the last one that is looked up ahead, with whole and broken
+# groups of four and eight, and with many more than their neighbours
+@pytest.mark.parametrize("degrees", [
+    [1, 0, 31, 32, 33, 127, 128, 129, 159, 160, 161],
+    [4 * 32, 4 * 32 + 1, 8 * 32 - 1, 8 * 32, 8 * 32 + 1, 12 * 32, 16 * 32 - 1, 16 * 32, 16 * 32 + 1],
+    [7, 20011, 64, 24 * 32, 24 * 32 + 31, 3, 9 * 32 + 5, 0],
+])
+def test_lists_of_neighbouring_lanes_of_unlike_lengths(oracle, degrees):
+    n = 64
+    rng = np.random.default_rng(len(degrees))
+    src = np.repeat(np.arange(len(degrees)) * 3 % n, degrees)
+    g = nd.Graph.from_edges(src, rng.integers(0, n, len(src)), n_vertices=n)
+    og = graphs.oracle_view(g)
+    for app, batch in (("MVS", 32), ("MVS5", 5)):
+        s = nd.Sampler(app, g, seed=42)
+        try:
+            verts = oracle.mvs_vertices(og, s.num_samples, batch)
+            want_rows, want_cols, want_start = oracle.sample_mvs(og, verts)
+            print("app", app, "degrees", degrees, flush=True)
+            s.do_transit_parallel()
+            rows, cols, start = s.adjacency()
+            assert np.array_equal(start, want_start)
+            assert np.array_equal(rows, want_rows) and np.array_equal(cols, want_cols)
+        finally:
+            s.close()
