@@ -38,10 +38,10 @@ MEASURED = {
         "read_requests": {"nd::step_flat_kernel": 8.224e6}, "write_requests": {"nd::step_flat_kernel": 1.698e6}},
     # the same workload with --inversion-period 0 (the engine's choice: walks keep their lanes)
     "weighted_node2vec_rmat22_period0": {
-        "kernels": {"nd::walk_rows_kernel": 1.408e11}, "bytes_per_pass": 140.79e9,
-        "read_requests": {"nd::walk_rows_kernel": 1.078e9}, "write_requests": {"nd::walk_rows_kernel": 7.506e7}},
+        "kernels": {"nd::walk_rows_kernel": 1.393e11}, "bytes_per_pass": 139.31e9,
+        "read_requests": {"nd::walk_rows_kernel": 1.074e9}, "write_requests": {"nd::walk_rows_kernel": 3.195e7}},
     "uniform_walk_chunglu57k": {"kernels": {"nd::step_flat_kernel": 1.224e7}, "bytes_per_pass": 1.27e9},
-    "uniform_walk_chunglu57k_period0": {"kernels": {"nd::walk_rows_kernel": 1.329e8}, "bytes_per_pass": 0.13e9},
+    "uniform_walk_chunglu57k_period0": {"kernels": {"nd::walk_rows_kernel": 1.320e8}, "bytes_per_pass": 0.13e9},
     # both kernel classes of a hop; the flat kernel is launched for both hops, the workgroup kernel for the second
     "khop_rmat21": {"kernels": {"nd::step_flat_kernel": 1.088e9, "nd::step_workgroup_kernel": 2.385e9},
                     "bytes_per_pass": 7.45e9},
@@ -50,7 +50,7 @@ MEASURED = {
         "kernels": {"nd::sorted_layer_kernel": 8.169e7, "nd::union_parts": 2.063e9, "nd::union_sums": 1.737e9},
         "bytes_per_pass": 7.88e9},
     "ladies_importance_chunglu3m": {
-        "kernels": {"nd::ranked_layer_kernel": 6.241e7, "nd::collective_mark_binned": 6.523e10}, "bytes_per_pass": 151.78e9},
+        "kernels": {"nd::ranked_layer_kernel": 6.243e7, "nd::collective_mark_binned": 6.172e10}, "bytes_per_pass": 123.74e9},
 }
 
 
@@ -201,8 +201,8 @@ def marking_bytes_per_pass(graph, sampler, final):
     """LADIES form: bytes the kernels that rank small neighbourhoods and mark the others (ranked_layer_kernel,
     collective_mark_binned) have to move in one pass, counted on the host from the transits of every layer.  Parallel
     edges are one pair of 12 B (id and term).  A transit with fewer pairs into a stretch of 7168 vertices than the
-    library's threshold contributes those pairs; with more, the stretch's ready-made piece of 64-bit sums.  Every
-    sample of more than 8192 pairs writes a 32-bit key per vertex, padded to whole stretches.
+    library's threshold contributes those pairs; with more, the stretch's ready-made piece of 64-bit sums.  (What is
+    written, the few thousand keys of a sample that can be among its first, is left out.)
     Returns (bytes with every use, pairs read one by one, pieces read, bytes with every piece once per layer)."""
     stretch, threshold = 7168, int(os.environ.get("ND_DENSE_PIECE_ENTRIES", 2048))
     rp, col = np.asarray(graph.row_ptr).astype(np.int64), np.asarray(graph.col)
@@ -211,15 +211,13 @@ def marking_bytes_per_pass(graph, sampler, final):
     is_first[rp[:-1][np.diff(rp) > 0]] = True
     before = np.concatenate([[0], np.cumsum(is_first)])
     pairs_of = np.append(before[rp[1:]] - before[rp[:-1]], 0)
-    stretches = -(-graph.n_vertices // stretch)
-    piece_bytes, keys_of_sample = 8 * stretch, 4 * stretch * stretches
-    pairs, pieces, distinct_pieces, marked = 0, 0, 0, 0
+    piece_bytes = 8 * stretch
+    pairs, pieces, distinct_pieces = 0, 0, 0
     ready_of = {}  # vertex: (pieces, pairs outside of them)
     for layer in _layers_of_transits(sampler, final):
         layer = np.where(_real(layer, sampler.invalid_vertex), layer, graph.n_vertices)
         sizes = pairs_of[layer].sum(axis=1)
         large = sizes > 8192
-        marked += int(large.sum())
         pairs += int(sizes[~large].sum())
         vertices, uses = np.unique(layer[large], return_counts=True)
         big = pairs_of[vertices] >= threshold if threshold > 0 else np.zeros(len(vertices), bool)
@@ -234,9 +232,7 @@ def marking_bytes_per_pass(graph, sampler, final):
             pieces += c * n_ready
             distinct_pieces += n_ready
             pairs += c * rest
-    written = marked * keys_of_sample
-    return (pairs * 12 + pieces * piece_bytes + written, pairs, pieces,
-            pairs * 12 + distinct_pieces * piece_bytes + written)
+    return pairs * 12 + pieces * piece_bytes, pairs, pieces, pairs * 12 + distinct_pieces * piece_bytes
 
 
 def pairs_reaching_the_step_kernels(sampler, final):
@@ -421,7 +417,7 @@ def measure(args, workload, steps, warmup, cpu_seconds, graphs, engine_choice=Tr
         # what the recorded counters say the launches are bound by: their measured HBM traffic over this run's time
         recorded = MEASURED_TRAFFIC_BYTES_PER_LAUNCH.get(workload)
         traffic_gbps = recorded / (prof["neighbourhood_ms"] / launches / 1000.0) / 1e9 if recorded else None
-        # (LADIES: 5 TB/s, and 63 % of the vector issue slots; FastGCN: union_parts takes its pieces and entries from L2, at
+        # (LADIES: 5.8 TB/s, and 52 % of the vector issue slots; FastGCN: union_parts takes its pieces and entries from L2, at
         # 2.2 TB/s from memory, union_sums reads the bitmaps at 3.1 TB/s)
         bound = "hbm" if ladies else "L2 (pieces and entries of union_parts), hbm (bitmaps of union_sums)"
         result["roofline"] = {

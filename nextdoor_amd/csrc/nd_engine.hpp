@@ -859,7 +859,7 @@ __device__ __forceinline__ void store_one(int32_t* at, VertexID v, bool past_cac
 // then takes the next walk of its wavefront; results go straight into the rows.
 //
 // What bounds it: the gathers.  Over a graph beyond the caches the requests past L2 (R-MAT 22 weighted
-// node2vec: 1.15e9 of them in 24.1 ms, 47.9 G/s of the 48-50 the gather probe reaches: row extent, 2.95
+// node2vec: 1.11e9 of them in 22.5 ms, 49.2 G/s of the 48-50 the gather probe reaches: row extent, 2.95
 // candidates and 0.9 tests a step), over one within them L2's own rate and, with few walks, the chain
 // of dependent loads.  A turn of the loop is therefore two CANDIDATES of every lane (they share a
 // Philox block), not one step: a wavefront that waits at every step for the slowest of 64 rejection
@@ -867,9 +867,9 @@ __device__ __forceinline__ void store_one(int32_t* at, VertexID v, bool past_cac
 // while its neighbours still try (100 K node2vec walks 1.45 -> 0.77 ms).
 //
 // Against inverting before every step (ms a pass, sorted and balanced / this): uniform walks over 2.7 K vertices
-// 0.50 / 0.10, 57 K 0.83 / 0.12, 200 K 5.5 / 0.37, 1 M 10.1 / 1.5; DeepWalk, 100 walks a vertex, over 10 K vertices
+// 0.50 / 0.07, 57 K 0.83 / 0.09, 200 K 5.5 / 0.37, 1 M 10.1 / 1.5; DeepWalk, 100 walks a vertex, over 10 K vertices
 // 9.3 / 1.6 and over R-MAT 16 27.8 / 12.7; MultiRW 100 K 1.7 / 0.7; weighted node2vec 100 K 2.9 / 0.77, 700 K 13.6 /
-// 4.0, R-MAT 22 34.5 / 24.1, four walks a vertex over 700 K 27.6 / 14.5.  There is no case among them where
+// 3.9, R-MAT 22 34.5 / 22.4, four walks a vertex over 700 K 27.6 / 14.5.  There is no case among them where
 // the order is worth what it costs.
 //
 // Few walks are bound by the chain of a step: the vertex, a random number, the edge.  The random numbers of the next step depend on
