@@ -57,11 +57,16 @@ void* make_app_engine(const char* name) {
   return engine;
 }
 
-// What nd_register_app compares: the hand-raised ND_ENGINE_ABI and the sizes of the structs a
-// shared object of apps and the library both lay out (the engine's base class, the kernel
-// parameters, the per-step bookkeeping).
+// What nd_register_app compares: the hand-raised ND_ENGINE_ABI and the sizes of what a shared object of apps and the library
+// both lay out: the engine's base class with all that it owns through a pointer (an engine made by one side brings its results
+// home with the other's code), the graph, the kernel parameters, the per-step bookkeeping.
+constexpr size_t kSharedLayouts[] = {sizeof(EngineBase),   sizeof(PhaseTimes), sizeof(ResultStream), ResultStream::transfer_bytes(),
+                                     sizeof(HostPool),     sizeof(HostLease),  sizeof(HostWorkers),  sizeof(HostWorkers::Job),
+                                     sizeof(CSR),          sizeof(StepParams), sizeof(RunsMeta)};
 constexpr int engine_abi() {
-  return ND_ENGINE_ABI * 65536 + (int)((sizeof(EngineBase) + sizeof(StepParams) + sizeof(RunsMeta) + sizeof(PhaseTimes)) % 65536);
+  uint32_t sizes = 0;
+  for (size_t bytes : kSharedLayouts) sizes = sizes * 31u + (uint32_t)bytes;  // two that change do not make up for each other
+  return ND_ENGINE_ABI * 65536 + (int)(sizes % 65536u);
 }
 
 // Registers <SampleType, App> under `name` when the object is constructed (a namespace-scope

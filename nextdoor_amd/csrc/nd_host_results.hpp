@@ -770,6 +770,8 @@ class ResultStream {
 
   // whether a word has ever not fitted
   bool misfit() const { return misfit_; }
+  // of what it owns through a pointer (nd::engine_abi)
+  static constexpr size_t transfer_bytes() { return sizeof(Transfer); }
   // page-locked memory it holds until release()
   size_t page_locked_bytes() const { return ring_bytes_; }
 

@@ -2,6 +2,8 @@
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -91,6 +93,31 @@ def test_app_registration_refuses_what_it_cannot_run():
     assert L.nd_register_app(b"HostSideProbeApp", fn, abi) == 0
     assert "HostSideProbeApp" in nextdoor_amd.app_names()
     assert L.nd_register_app(b"HostSideProbeApp", fn, abi) == -3
+
+
+def test_the_engine_layout_number_covers_what_an_engine_owns_through_a_pointer():
+    """An engine made by an app's shared object is handed to the library, with the stream that brings its results, its
+    pools and its threads: objects that do not show in sizeof(EngineBase).  A change of any one size changes the number."""
+    code = ("import ctypes as C, nextdoor_amd._capi as c\n"
+            "L = c.lib()\n"
+            "A = C.CDLL(%r, mode=C.RTLD_GLOBAL)\n"
+            "out = (C.c_uint64 * 64)()\n"
+            "n = A.user_apps_shared_layouts(out, 64)\n"
+            "print(L.nd_engine_abi(), *out[:n])\n" % os.path.join(ROOT, "tests", "cpp", "libuser_apps.so"))
+    done = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=100)
+    assert done.returncode == 0, done.stderr[-500:]
+    abi, *sizes = map(int, done.stdout.split())
+    assert len(sizes) >= 11 and "not registered" not in done.stderr
+
+    def number(of):
+        n = 0
+        for b in of:
+            n = (n * 31 + b) % (1 << 32)
+        return n % 65536
+    assert abi % 65536 == number(sizes)
+    for i in range(len(sizes)):
+        for by in (-64, -8, 8, 16, 256):
+            assert number(sizes[:i] + [sizes[i] + by] + sizes[i + 1:]) != number(sizes)
 
 
 keep_alive = []  # ctypes callbacks handed to the library must outlive the test
