@@ -58,7 +58,6 @@ enum KernelMode { kTransitParallel = 0, kTransitParallelLoadBalanced = 1, kSampl
 
 struct PhaseTimes {  // milliseconds, accumulated over one sample() call when profiling is on
   float end_to_end = 0, inversion = 0, load_balancing = 0, flat_kernel = 0, workgroup_kernel = 0, assemble = 0, distinct = 0;
-  // (flat: a launch of walks whose rows leave while it runs counts once for every part of them that leaves by itself)
   int flat_launches = 0, workgroup_launches = 0, sort_launches = 0;
   // layer-wise apps: the kernel that walks the collective neighbourhoods (marking / building)
   float neighborhood = 0;
@@ -2136,6 +2135,7 @@ class Engine : public EngineBase {
     (void)finish_rows_ahead();  // nobody asked for them
     if ((inverts(mode) ? alloc_inversion() : build_walk_tables()) != 0) return -1;  // what an earlier pass has not
     times = PhaseTimes();
+    sent_ahead_ = false;
     if (!std::is_empty<SampleType>::value) {
       ND_HIP_TRY(hipMemcpyAsync(d_samples_, d_samples_init_, sizeof(SampleType) * (size_t)n_samples_,
                                 hipMemcpyDeviceToDevice, stream_));
@@ -2184,6 +2184,7 @@ class Engine : public EngineBase {
   // pass after one that found nothing for the workgroup class is not), 7 = load-balanced steps
   // whose two classes ran as one launch, 8 = as two launches side by side on two streams,
   // 9 = one after the other.
+  // Walks: 10 = parts of the last pass's rows that were on their way to the host before its walks were done.
   int64_t counter(int which) const override {
     switch (which) {
       case 0: return (int64_t)class_counters_.sorted_pairs;
@@ -2196,6 +2197,7 @@ class Engine : public EngineBase {
       case 7: return (int64_t)schedule_counts_.merged_steps;
       case 8: return (int64_t)schedule_counts_.forked_steps;
       case 9: return (int64_t)schedule_counts_.serial_steps;
+      case 10: return sent_ahead_ ? (int64_t)result_stream->parts_ahead() : 0;
       default: return 0;
     }
   }
@@ -2227,7 +2229,6 @@ class Engine : public EngineBase {
       first = end;
     }
     if (form == kRowsByStretch) {
-      times.flat_launches = (int)(((uint64_t)n_samples_ - 1) >> early.shift) + 1;
       ready.clear();
       for (uint64_t at = 0; at < (uint64_t)n_samples_; at += 1ull << early.shift)
         ready.push_back({(size_t)std::min<uint64_t>((uint64_t)n_samples_, at + (1ull << early.shift)) * F, range_ends_[0],
@@ -2241,6 +2242,7 @@ class Engine : public EngineBase {
       ahead_ = false;
     }
     if (!ahead_) (void)hipGetLastError();
+    sent_ahead_ = ahead_;
     return 0;
   }
 
@@ -2942,7 +2944,7 @@ class Engine : public EngineBase {
   // The result stream carries one transfer at a time, and whoever begins another waits for the one before: rows on their way
   // are waited for here first, where it is known whose they are and what has become of them.
   void settle_rows_ahead() {
-    if (ahead_ && result_stream->finish() != hipSuccess) ahead_ = false;
+    if (ahead_ && result_stream->finish() != hipSuccess) ahead_ = sent_ahead_ = false;
   }
 
   void launch_workgroup(const StepParams& P, unsigned grid, const RunsMeta* meta) {
@@ -3182,6 +3184,7 @@ class Engine : public EngineBase {
   const walk_record<App>* walk_records_ = nullptr;  // dgraph_'s, where they pay
   uint32_t walk_waves_at_once_ = 1, cus_ = 1;  // wavefronts of walk_rows_kernel the device holds, compute units
   bool ahead_ = false;                    // rows are on their way to rows_ahead
+  bool sent_ahead_ = false;               // ... or have been, in the last pass
   std::vector<hipEvent_t> range_ends_;    // ends of the launches of such a pass
   // of such a pass: EarlyRows::arrived and walked, and the number of the last
   uint32_t *h_arrived_ = nullptr, *d_walked_ = nullptr;

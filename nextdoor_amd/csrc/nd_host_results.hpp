@@ -745,6 +745,7 @@ class ResultStream {
       if (e == hipSuccess) e = hipStreamWaitEvent(t.streams[1], begun_, 0);
       if (e != hipSuccess) return e;
     }
+    if (!t.ready.empty()) ahead_.store(0, std::memory_order_relaxed);
     job_.body = [this] { take_part(); };
     HostWorkers::get().start(job_, HostWorkers::kMost);
     under_way_ = true;  // (not if start() throws: nobody has begun on it then)
@@ -770,6 +771,8 @@ class ResultStream {
 
   // whether a word has ever not fitted
   bool misfit() const { return misfit_; }
+  // pieces of the last begin() that was given a `ready` which set out before all of that had happened
+  size_t parts_ahead() const { return ahead_.load(std::memory_order_relaxed); }
   // of what it owns through a pointer (nd::engine_abi)
   static constexpr size_t transfer_bytes() { return sizeof(Transfer); }
   // page-locked memory it holds until release()
@@ -987,7 +990,7 @@ class ResultStream {
     return true;
   }
 
-  // Whether nothing is being computed any more that the transfer could be in the way of.
+  // Whether nothing is being computed any more that the transfer could be in the way of, or ahead of.
   bool computed() {
     Transfer& t = *transfer_;
     if (!t.computed) t.computed = t.ready.empty() || hipEventQuery(t.ready.back().event) == hipSuccess;
@@ -1097,6 +1100,7 @@ class ResultStream {
         gently = gently && !computed();
         if (launched >= p + (gently ? kGentleAhead : kSlots)) break;
         while (!slot_is_free(launched, p)) {}
+        if (gently) ahead_.fetch_add(1, std::memory_order_relaxed);
         error = launch(launched++, gently ? kGentleBlocks : UINT32_MAX);
       }
       if (error == hipSuccess) error = hipEventSynchronize(packed_[p % kSlots]);
@@ -1114,6 +1118,7 @@ class ResultStream {
       bool moved = false;
       if (launched < t.pieces && launched < sent + kPackedAhead && readable(launched, /*waits=*/here == launched, &e) &&
           slot_is_free(launched, here)) {
+        if (!computed()) ahead_.fetch_add(1, std::memory_order_relaxed);
         e = launch(launched++);
         moved = true;
       }
@@ -1138,6 +1143,7 @@ class ResultStream {
   bool under_way_ = false, misfit_ = false;
   int device_ = -1;  // of the events and the ring
   uint32_t looks_ = 0;
+  std::atomic<size_t> ahead_{0};  // parts_ahead()
   uint8_t* ring_ = nullptr;
   size_t ring_bytes_ = 0;
   hipEvent_t packed_[kSlots] = {}, begun_ = nullptr;
