@@ -621,9 +621,9 @@ inline hipError_t device_of(hipStream_t stream, int* device) {
   return stream ? hipStreamGetDevice(stream, device) : hipGetDevice(device);
 }
 
-// The streams results cross the bus on while something else is computed: two per device (which has to be the current one) and process, each on
+// The streams results cross the bus on while something else is computed: two or three per device (which has to be the current one) and process, each on
 // a hardware queue of its own, which a stream with a mask of compute units (here: all) gets.  (Ordinary streams share
-// four; where the computation's lands on the same one, nothing overlaps.)  They are destroyed when the process ends, while
+// four; where the computation's lands on the same one, nothing overlaps.)  What each is for: StreamUse.  They are destroyed when the process ends, while
 // the runtime and whatever watches it are still there: left to the runtime, their queues outlive a profiler's
 // bookkeeping of them, and a profiled process ended in a segmentation fault.
 inline std::vector<hipStream_t>& transfer_streams() {
@@ -638,11 +638,12 @@ inline std::vector<hipStream_t>& transfer_streams() {
   }();
   return *streams;
 }
+constexpr size_t kTransferStreams = 3;  // of a device, at most
 inline hipStream_t transfer_stream(int device, size_t which) {
   static std::mutex mutex;
   std::vector<hipStream_t>* streams = &transfer_streams();
   std::lock_guard<std::mutex> lock(mutex);
-  const size_t at = 2 * (size_t)device + which;
+  const size_t at = kTransferStreams * (size_t)device + which;
   if (streams->size() <= at) streams->resize(at + 1, nullptr);
   hipStream_t& stream = (*streams)[at];
   if (!stream) {
@@ -659,6 +660,52 @@ inline hipStream_t transfer_stream(int device, size_t which) {
 }
 
 // ---- the stream ----------------------------------------------------------------------------
+
+// What a transfer may use besides the first of its device's streams, on which nothing ever waits for a computation: all the
+// samplers of the process share it, and what others put there would wait as well.  The second is either one transfer's that
+// has it wait for its computation, or packs pieces for any number that do not; who wants to pack while somebody waits
+// there does so on a third.  (Not a stream for each from the start: uniform walks 57 K, whose rows wait for them, 0.35 ms, 0.40
+// on the third such stream of a process.)
+class StreamUse {
+ public:
+  StreamUse() = default;
+  StreamUse(const StreamUse&) = delete;
+  StreamUse& operator=(const StreamUse&) = delete;
+  ~StreamUse() { give_back(); }
+
+  // the second one, for waiting: false if it is in use
+  bool wait(int device) {
+    give_back();
+    int nobody = 0;
+    if ((unsigned)device >= kDevices || !users(device).compare_exchange_strong(nobody, -1)) return false;
+    device_ = device, held_ = -1;
+    return true;
+  }
+  // the one to pack on
+  size_t pack(int device) {
+    give_back();
+    if ((unsigned)device >= kDevices) return 1;  // nobody waits there
+    for (int now = users(device).load();;) {
+      if (now < 0) return 2;
+      if (users(device).compare_exchange_weak(now, now + 1)) break;
+    }
+    device_ = device, held_ = 1;
+    return 1;
+  }
+  // nothing of the transfer is on it any more
+  void give_back() {
+    if (held_ != 0) users(device_).fetch_sub(held_);
+    held_ = 0;
+  }
+
+ private:
+  static constexpr unsigned kDevices = 64;
+  static std::atomic<int>& users(int device) {  // of the second stream; -1: one that waits
+    static std::atomic<int> all[kDevices] = {};
+    return all[device];
+  }
+  int device_ = 0, held_ = 0;
+};
 
 // Brings words of device memory to the host, packed on the way.  One caller at a time.  Everything happens on the device of the
 // stream that is given, whatever the calling thread's current device is, and leaves that as it was.
@@ -725,6 +772,7 @@ class ResultStream {
   hipError_t begin(const int32_t* src, size_t n, uint32_t bits, int32_t fill, int32_t* dst, hipStream_t stream,
                    std::vector<Ready> ready) {
     hipError_t e = finish();  // an earlier one that nobody waited for
+    use_.give_back();
     if (e != hipSuccess || n == 0) return e;
     if (!transfer_) transfer_.reset(new Transfer);
     Transfer& t = *transfer_;
@@ -737,10 +785,14 @@ class ResultStream {
     e = prepare(t.slot_bytes);
     if (e == hipSuccess && t.staged) e = prepare_staging(t.slot_bytes);
     if (e != hipSuccess) return e;
-    // pieces alternate between two streams, so that the bus is not idle between two of them
-    t.streams[1] = transfer_stream(t.device, 0);
-    t.streams[0] = t.ready.empty() ? stream : t.staged || t.ready.size() == 1 ? transfer_stream(t.device, 1) : t.streams[1];
+    t.streams[0] = t.streams[1] = transfer_stream(t.device, 0);
+    // all words at once: the device waits for them, without a way over a thread, if it can
+    t.device_waits = t.ready.size() == 1 && !t.staged && use_.wait(t.device);
+    if (t.device_waits) t.streams[0] = t.streams[1] = transfer_stream(t.device, 1);
+    if (t.staged) t.streams[0] = transfer_stream(t.device, use_.pack(t.device));
     if (t.ready.empty()) {
+      // pieces alternate between two streams, so that the bus is not idle between two of them
+      t.streams[0] = stream;
       e = hipEventRecord(begun_, stream);
       if (e == hipSuccess) e = hipStreamWaitEvent(t.streams[1], begun_, 0);
       if (e != hipSuccess) return e;
@@ -761,12 +813,13 @@ class ResultStream {
     if (t.error != hipSuccess) {
       const OnDevice on(t.device);
       for (hipStream_t s : t.streams) (void)hipStreamSynchronize(s);  // nothing writes to the ring after this
-      return t.error;
     }
+    use_.give_back();
+    if (t.error != hipSuccess) return t.error;
     if (!t.overflow.load()) return hipSuccess;
     misfit_ = true;
     const OnDevice on(t.device);  // the stream may be the default one
-    return fetch(t.src, t.n, 32, t.fill, t.dst, t.streams[0]);
+    return fetch(t.src, t.n, 32, t.fill, t.dst, t.ready.empty() ? t.streams[0] : transfer_stream(t.device, 0));
   }
 
   // whether a word has ever not fitted
@@ -853,7 +906,7 @@ class ResultStream {
     if (!totals_) e = hipHostMalloc((void**)&totals_, kSlots * sizeof(uint32_t), hipHostMallocDefault);
     if (e == hipSuccess && !counts_) {
       e = hipMalloc(&counts_, 2 * kSlots * kWordsPerLine * sizeof(uint32_t));
-      // on a stream of their own: the computation is not waited for
+      // on a stream that waits for no computation
       const hipStream_t stream = transfer_stream(device_, 0);
       if (e == hipSuccess) e = hipMemsetAsync(counts_, 0, 2 * kSlots * kWordsPerLine * sizeof(uint32_t), stream);
       if (e == hipSuccess) e = hipStreamSynchronize(stream);
@@ -889,6 +942,7 @@ class ResultStream {
     hipStream_t streams[2];
     std::vector<Ready> ready;
     bool staged = false;  // pieces are packed in device memory, for the copy engine, while something else is computed
+    bool device_waits = false;
     int device = 0;
 
     size_t chunks, pieces, chunk_bytes, packed_at, slot_bytes;
@@ -1088,10 +1142,8 @@ class ResultStream {
     hipError_t error = hipSuccess;
     size_t launched = 0;
     bool gently = !t.ready.empty();
-    if (t.ready.size() == 1) {
-      // all of it at once: the device waits, without a way over this thread
-      for (hipStream_t stream : t.streams)
-        if (error == hipSuccess) error = hipStreamWaitEvent(stream, t.ready[0].event, 0);
+    if (t.device_waits) {
+      error = hipStreamWaitEvent(t.streams[0], t.ready[0].event, 0);
       t.happened = 1;
       gently = false;
     }
@@ -1140,6 +1192,7 @@ class ResultStream {
 
   std::unique_ptr<Transfer> transfer_;
   HostWorkers::Job job_;
+  StreamUse use_;
   bool under_way_ = false, misfit_ = false;
   int device_ = -1;  // of the events and the ring
   uint32_t looks_ = 0;

@@ -5,6 +5,9 @@
 
 #include <stdio.h>
 
+#include <chrono>
+#include <thread>
+
 #define TRY(expr)                                                              \
   do {                                                                         \
     hipError_t e_ = (expr);                                                    \
@@ -54,8 +57,82 @@ static int on_other_devices() {
   return 0;
 }
 
+// Some 70 ms of one wavefront; it ends by itself.
+__global__ void take_a_while() {
+  for (uint32_t i = 0; i < 20000; ++i) __builtin_amdgcn_s_sleep(127);
+}
+__global__ void write_words(int32_t* words, size_t n) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) words[i] = (int32_t)(i & 0xfff);
+}
+
+// Two transfers whose words come at the end of a long computation, and others whose words are there: those do not wait for it.
+static int beside_one_that_waits() {
+  const size_t n = (size_t)300 * nd::kPackChunk;
+  std::vector<int32_t> want(n), late(n), later(n), got(n);
+  for (size_t i = 0; i < n; ++i) want[i] = (int32_t)(i & 0xfff);
+  int32_t *d = nullptr, *d_late = nullptr;
+  uint32_t* sign = nullptr;
+  hipStream_t busy, stream;
+  hipEvent_t there, computed;
+  TRY(hipMalloc(&d, n * sizeof(int32_t)));
+  TRY(hipMalloc(&d_late, n * sizeof(int32_t)));
+  TRY(hipHostMalloc((void**)&sign, sizeof(uint32_t), hipHostMallocDefault));
+  *sign = 7;
+  TRY(hipStreamCreate(&stream));
+  TRY(hipStreamCreate(&busy));
+  TRY(hipEventCreateWithFlags(&there, hipEventDisableTiming));
+  TRY(hipEventCreateWithFlags(&computed, hipEventDisableTiming));
+  TRY(hipMemcpyAsync(d, want.data(), n * sizeof(int32_t), hipMemcpyHostToDevice, stream));
+  TRY(hipEventRecord(there, stream));
+  TRY(hipStreamSynchronize(stream));
+  nd::ResultStream first, second, other;
+  for (int turn = 0; turn < 3; ++turn) {  // the first one takes the memory
+    TRY(hipMemset(d_late, 0, n * sizeof(int32_t)));
+    TRY(hipDeviceSynchronize());
+    if (turn) take_a_while<<<dim3(1), dim3(64), 0, busy>>>();
+    write_words<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, busy>>>(d_late, n);
+    TRY(hipGetLastError());
+    TRY(hipEventRecord(computed, busy));
+    std::fill(late.begin(), late.end(), -1);
+    std::fill(later.begin(), later.end(), -1);
+    TRY(first.begin(d_late, n, 12, 0, late.data(), busy, {{n, computed}}));
+    TRY(second.begin(d_late, n, 12, 0, later.data(), busy, {{n, computed}}));
+    std::this_thread::sleep_for(std::chrono::milliseconds(5));  // other threads take them on
+    for (int form = 0; form < 3; ++form) {
+      printf("beside one that waits: turn %d form %d\n", turn, form);
+      fflush(stdout);
+      std::vector<nd::ResultStream::Ready> ready{{n, there}};
+      if (form == 1) ready.insert(ready.begin(), {n / 2, there});
+      if (form == 2) ready = {{n / 3, there, sign, 7u}, {n, there, sign, 7u}};
+      std::fill(got.begin(), got.end(), -1);
+      TRY(other.begin(d, n, 12, 0, got.data(), stream, ready));
+      TRY(other.finish());
+      const bool before = hipEventQuery(computed) == hipErrorNotReady;
+      (void)hipGetLastError();
+      if (got != want) { printf("other words\n"); return 1; }
+      if (turn && !before) { printf("held up until the other computation was over\n"); return 1; }
+    }
+    TRY(first.finish());
+    TRY(second.finish());
+    if (late != want || later != want) { printf("words from before they were there\n"); return 1; }
+  }
+  first.release();
+  second.release();
+  other.release();
+  TRY(hipEventDestroy(there));
+  TRY(hipEventDestroy(computed));
+  TRY(hipStreamDestroy(stream));
+  TRY(hipStreamDestroy(busy));
+  TRY(hipHostFree(sign));
+  TRY(hipFree(d));
+  TRY(hipFree(d_late));
+  return 0;
+}
+
 int main() {
   if (on_other_devices() != 0) return 1;
+  if (beside_one_that_waits() != 0) return 1;
   const size_t piece = (size_t)64 * nd::kPackChunk;  // the smallest piece
   const size_t sizes[] = {1, 7, 8, 9, nd::kPackChunk - 1, nd::kPackChunk, nd::kPackChunk + 1, piece, piece + 9, 13 * piece + 4097};
   nd::ResultStream stream;
