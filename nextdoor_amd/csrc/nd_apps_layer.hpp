@@ -36,8 +36,8 @@ namespace apps {
 //                  numEdges = how many distinct ids there are; no weight array
 //   kRankedByLadiesImportance  the distinct ids ordered by descending Efraimidis-Spirakis key
 //                  for the LADIES importance (squared column norm of the row-normalised
-//                  adjacency restricted to the transits); no weights.  numEdges = how many of them are handed over: all
-//                  there are, or at least stepSize(k)
+//                  adjacency restricted to the transits): the first stepSize(k) of them, or all if there are fewer.
+//                  numEdges = how many that is; no weights
 enum NeighborhoodForm { kConcatenated = 0, kDistinctByDegreeSquared = 1, kRankedByLadiesImportance = 2 };
 
 // The form an App's next() takes the collective neighbourhood in: App::kNeighborhoodForm, or the

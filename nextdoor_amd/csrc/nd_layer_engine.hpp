@@ -1043,8 +1043,9 @@ __global__ __launch_bounds__(kRankedThreads) void ranked_layer_kernel(LayerParam
   ranked_layer(merged, (uint32_t)P.csr.n_vertices, P.transits.base + (size_t)ls * P.transits.stride, P.transits.count, P.invalid,
                size, P.first_sample + P.sample_begin + ls, (uint32_t)P.step, P.seed, distinct + ls,
                [&](const CSR::Edge* ranked, uint32_t n_distinct) {
+                 const uint32_t n_first = n_distinct < P.step_size ? n_distinct : P.step_size;
                  for (uint32_t nbr = threadIdx.x; nbr < P.step_size; nbr += kRankedThreads)
-                   draw_from<SampleType, App>(P, ls, nbr, ranked, n_distinct);
+                   draw_from<SampleType, App>(P, ls, nbr, ranked, n_first);
                });
 }
 
@@ -1126,7 +1127,9 @@ __global__ __launch_bounds__(kBinThreads) void kept_layer_kernel(LayerParams P, 
   for (uint32_t i = threadIdx.x; i < n; i += kBinThreads) s_ids[i] = (int32_t)(uint32_t)s_best[i];
   __syncthreads();
   const CSR::Edge* ranked = (const CSR::Edge*)s_ids;
-  for (uint32_t nbr = threadIdx.x; nbr < P.step_size; nbr += kBinThreads) draw_from<SampleType, App>(P, marked[at], nbr, ranked, n);
+  // (how many more there are here depends on what the workgroups knew of each other's bounds)
+  const uint32_t n_first = n < P.step_size ? n : P.step_size;
+  for (uint32_t nbr = threadIdx.x; nbr < P.step_size; nbr += kBinThreads) draw_from<SampleType, App>(P, marked[at], nbr, ranked, n_first);
 }
 
 // The draws of the marked samples, a lane each, the workgroups of the grid in turn.

@@ -152,6 +152,19 @@ struct UserAnchorHopApp {
   }
 };
 
+class UserRankedSample {};
+
+// LADIES importance sampling of one layer that tells in its first place how many vertices it was handed
+struct UserRankedCountApp : LadiesImportanceAppT<1, 16, 60> {
+  template <typename SampleType, typename EdgeArray, typename WeightArray>
+  __device__ inline VertexID next(int step, CSRPartition* csr, const VertexID* transits, const VertexID sampleIdx,
+                                  SampleType* sample, const float max_weight, EdgeArray& ranked, WeightArray& none,
+                                  const EdgePos_t numEdges, const VertexID_t neighbrID, curandState* state) {
+    if (neighbrID == 0) return numEdges < csr->get_n_vertices() ? numEdges : -1;
+    return neighbrID < numEdges ? ranked[neighbrID] : -1;
+  }
+};
+
 // The sizes this object was built with, for the test of what the library compares.
 extern "C" int user_apps_shared_layouts(uint64_t* out, int room) {
   const uint64_t sizes[] = {sizeof(nd::EngineBase), sizeof(nd::PhaseTimes), sizeof(nd::ResultStream), nd::ResultStream::transfer_bytes(),
@@ -162,6 +175,7 @@ extern "C" int user_apps_shared_layouts(uint64_t* out, int room) {
   return n;
 }
 
+ND_REGISTER_APP("UserRankedCount", UserRankedSample, UserRankedCountApp)
 ND_REGISTER_APP("UserAnchorHop", UserAnchorSample, UserAnchorHopApp)
 ND_REGISTER_APP("UserThreeHop", UserHopSample, UserThreeHopApp)
 ND_REGISTER_APP("UserShortDeepWalk", UserWalkSample, UserShortDeepWalkApp)

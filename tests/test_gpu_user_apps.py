@@ -74,6 +74,35 @@ def test_an_app_with_explicit_transits_and_several_transits_per_sample(gname):
         s.close()
 
 
+# neighbourhoods ranked in LDS (of fewer vertices than a layer takes, and of more), and larger ones, with keys that tell the
+# vertices apart and with equal ones
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,mean_degree,weight", [(2000, 0.5, "any"), (2000, 10, "any"), (6000, 700, "any"), (6000, 700, "tiny")])
+def test_a_ranked_layer_hands_over_as_many_vertices_as_it_takes(n, mean_degree, weight):
+    """numEdges of the LADIES form is a function of the graph and the roots: the layer's size, or all that there are."""
+    nd.load_app_library(USER_APPS_LIB)
+    rng = np.random.default_rng(5)
+    src, dst = rng.integers(0, n, (2, int(n * mean_degree)))
+    w = rng.uniform(1.0, 2.0, len(src)).astype(np.float32)
+    if weight == "tiny":  # terms of 0, but for one edge of each row
+        w[:] = 1e-9
+        src, dst, w = np.append(src, np.arange(n)), np.append(dst, rng.integers(0, n, n)), np.append(w, np.ones(n, np.float32))
+    g = nd.Graph.from_edges(src, dst, w, n_vertices=n)
+    s = nd.Sampler("UserRankedCount", g, seed=SEED)
+    try:
+        roots = s.initial_contents.reshape(s.num_samples, -1)
+        distinct = [len(np.unique(np.concatenate([g.col[g.row_ptr[r]:g.row_ptr[r + 1]] for r in row]))) for row in roots]
+        want = np.minimum(distinct, s.step_size(0))
+        print("UserRankedCount", n, mean_degree, weight, "least and most vertices", min(distinct), max(distinct), flush=True)
+        for _ in range(3):
+            s.do_transit_parallel()
+            got = s.final_samples()
+            assert np.array_equal(got[:, 0], want)
+            assert np.array_equal((got[:, 1:] != s.invalid_vertex).sum(axis=1), np.maximum(want - 1, 0))
+    finally:
+        s.close()
+
+
 def write_binary_edge_list(path, src, dst, weight):
     """The reference's binary edge list: 12-byte records (int32 src, int32 dst, float32 weight),
     src/graph.hpp:42-75."""
