@@ -2251,42 +2251,55 @@ class Engine : public EngineBase {
   // kRowsByRange: a few launches, one range of walks after another; rows leave from the end of the first on (one launch:
   // when it has ended).  Every launch ends with its longest walks alone on the device (0.07 ms of uniform walks, 0.2 of
   // DeepWalk and PPR, 0.6 of second-order walks), but all of a range's rows are there at once, and their way straight to
-  // the ring has no 8 us between two pieces.  Passes with their rows, ms, by launches and, one launch, by wavefronts a compute
-  // unit (Chung-Lu graphs, mean degree 10 to 12, unless another is named):
-  //                     launches  1     2     3     4      wavefronts  6     8    10    12    16
-  //    uniform         300 K   1.45  1.33  1.29  1.32           1.41  1.42  1.41  1.42  1.44
-  //                    550 K   2.59  2.31  2.26  2.19           2.39  2.28  2.32  2.37  2.49
-  //                    800 K   3.74  3.63  3.36  3.30           3.11  3.13  3.15  3.23  3.38
-  //                    1.1 M   4.95  4.80  4.79  4.69           4.14  4.13  4.15  4.23  4.42
-  //    DeepWalk        300 K   2.10  1.63  1.66  1.90           1.76  1.75  1.79  1.81  1.86
-  //                    400 K   2.52  2.09  2.03  2.05           2.12  2.08  2.14  2.22  2.31
-  //                    550 K   3.25  2.98  2.71  2.70           2.73  2.65  2.73  2.81  3.06
-  //                    1.1 M   6.45  5.93  5.61  5.54           4.99  4.90  4.93  5.00  5.20
-  //                  R-MAT 22                                  16.17 15.99 16.12 16.44 17.28
-  //    PPR             300 K   1.72  1.49  1.47  1.69           1.61  1.60  1.57  1.58  1.61
-  //                    550 K   2.71  2.59  2.49  2.49           2.46  2.44  2.46  2.47  2.60
-  //                    1.1 M   5.25  4.96  4.90  4.80           4.46  4.29  4.37  4.41  4.53
-  //    weighted n2v    100 K   1.26  1.72  2.25  2.84           1.43  1.27  1.27  1.27  1.28
-  //                    140 K   1.47  2.00  2.47  3.05           1.78  1.59  1.49  1.50  1.51
-  //                    300 K   2.98  2.56  3.16  3.81           2.86  2.59  2.56  2.51  2.55
-  //                    550 K   5.20  5.07  4.17  4.78           4.61  4.08  4.11  4.17  4.40
-  //                    1.1 M   9.89  8.65  8.42  9.72           8.60  7.29  6.78  6.87  7.97
-  //                  R-MAT 22  (30.1 by four launches)         33.7  28.8  26.2  25.2  24.4
-  //                                                    wavefronts  2     3     4     5     6
-  //    MultiRW         100 K   1.16  0.94  1.02  1.13           1.10  1.09  0.94  1.05  1.17
-  //                    200 K   2.51  2.04  1.83  1.80           1.84  1.72  1.93  2.19  2.33
-  //                    400 K   5.06  4.93  4.26  3.78           3.36  3.07  3.23  3.54  3.81
-  //                    1.1 M  14.72 14.09 13.35 14.24                 7.73  8.28  8.76  9.33
+  // the ring has no 8 us between two pieces.  Passes with their rows, ms, by launches and by stretch, over Chung-Lu graphs
+  // (exponent 2.2) of the mean degree that is named:
+  //                     launches   1     2     3     4     6   stretch
+  //    uniform     11   400 K         1.86  1.73  1.66          1.76      of 8 steps   8   300 K  0.21  0.21        0.22        0.29
+  //                     500 K         2.33  2.19  2.08          2.12                       500 K  0.31  0.32        0.30        0.38
+  //                     600 K         2.90  2.75  2.64          2.52                       800 K                    0.45  0.45  0.53
+  //                     800 K         3.83  3.64  3.54          3.15                       1.2 M                    0.68  0.66  0.69
+  //                 5   500 K               1.64  1.62          1.61                       1.6 M                    0.88  0.84  0.86
+  //                18   500 K               2.95  2.82          2.62                       2 M    1.30  1.24        1.09        1.02
+  //    DeepWalk    11   350 K         1.76  1.73  1.79          1.85
+  //                     450 K         2.29  2.15  2.10          2.18
+  //                     550 K         2.86  2.63  2.57          2.58
+  //                18   500 K                     3.08          2.81
+  //    PPR         11   250 K         1.24  1.26  1.41          1.34
+  //                     450 K         2.08  2.02  1.98          2.02
+  //                     550 K         2.55  2.40  2.44          2.36
+  //    weighted    11   100 K   1.13  1.53                      1.17      of 8 steps   8   120 K  0.22  0.28        0.43        0.26
+  //    node2vec         150 K   1.38  1.77                      1.46                       300 K  0.38  0.36        0.50        0.43
+  //                     200 K   1.64  1.87                      1.69                       500 K  0.57  0.48  0.51  0.59        0.58
+  //                     240 K   1.94  2.02  2.54                1.95                       900 K  0.92  0.95  0.80  0.83        0.85
+  //                     300 K   2.85  2.21                      2.34                       1.2 M  1.18  1.13  1.16  1.02        1.05
+  //                     400 K   3.54  2.74  2.98                2.93
+  //                 6   300 K   1.92  1.69  2.10                1.64
+  //                     400 K         2.22  2.30                2.09
+  //                20   300 K   4.04  3.07  3.45                2.98
+  //                     400 K         4.10  4.22                3.70
+  //       R-MAT 17 x 16         1.33  1.73                      1.39
+  //       R-MAT 18 x 12         2.10  2.06                      2.23
+  //       R-MAT 19 x 16               3.85  3.91                3.73
+  //    MultiRW     11   100 K         1.42  1.45  1.54          1.57      of 6 steps   8   200 K  0.15  0.16        0.17        0.20
+  //                     135 K         1.97  1.84                1.93                       500 K  0.39  0.29        0.29        0.33
+  //                     190 K         2.74  2.53  2.50          2.48                       850 K        0.51        0.46        0.46
+  //                                                                                        1 M    0.68  0.69        0.55        0.51
+  // Where the two meet moves with the graph (second-order walks of 400 K from 10 % for stretches to 6 % against them, by its
+  // degree), and with the walks' length as if a walk were 24 results longer.  Longer walks are not taken from fewer on: a pass whose
+  // walks are all under way at once has no first ones.
   enum EarlyForm { kRowsStay, kRowsByRange, kRowsByStretch };
   EarlyForm early_form(EarlyRows* early) {
     if (!rows_ahead || profiling || wants_launch_graph()) return kRowsStay;
-    if (sizeof(VertexID_t) * (size_t)n_samples_ * (size_t)final_sample_size() <= kDirectResultBytes) return kRowsStay;
-    const bool many = n_samples_ >= (state_fits_pair<SampleType>::value ? 96 << 10 : std::is_empty<SampleType>::value ? 448 << 10 : 192 << 10);
+    const uint64_t n = (uint64_t)n_samples_, results = (uint64_t)final_sample_size();
+    if (sizeof(VertexID_t) * n * results <= kDirectResultBytes) return kRowsStay;
+    constexpr uint64_t kOf100Steps = state_fits_pair<SampleType>::value ? 384 << 10 : std::is_empty<SampleType>::value ? 448 << 10 : 192 << 10;
+    const bool many = n * (std::min<uint64_t>(results, 100) + 24) >= kOf100Steps * (100 + 24);
     return many && ready_for_early_rows(early) ? kRowsByStretch : kRowsByRange;
   }
   uint32_t walk_ranges() const {
-    const int64_t least = std::is_empty<SampleType>::value ? 96 << 10 : state_fits_pair<SampleType>::value ? 160 << 10 : 40 << 10;
-    return (uint32_t)std::max<int64_t>(1, std::min<int64_t>(kMostWalkRanges, n_samples_ / least));
+    constexpr int64_t least = std::is_empty<SampleType>::value ? 96 << 10 : state_fits_pair<SampleType>::value ? 128 << 10 : 40 << 10;
+    if (std::is_empty<SampleType>::value && n_samples_ >= 8 * least) return kMostWalkRanges;  // short ones
+    return (uint32_t)std::max<int64_t>(1, std::min<int64_t>(4, n_samples_ / least));
   }
   // What that takes, and the stretches the walks are counted by; false: without.
   bool ready_for_early_rows(EarlyRows* early) {
@@ -2347,9 +2360,18 @@ class Engine : public EngineBase {
     // wavefronts to a compute unit, 23.9 with 20; 27 with 8), and the fewer walks are under way, the sooner each is
     // done: shorter tails, more hits (DeepWalk over 1 M vertices 3.0 ms with 12, 3.4 with 20).
     // Where rows leave by stretch the first of them should be there soon, and the fewer walks at a time the sooner: as many
-    // as keep the memory path busy (EarlyForm), second-order walks an eighth of the pass at a time if that is more, but no
-    // more than four wavefronts to a SIMD: the packing needs room in LDS beside them (R-MAT 22 node2vec with 20 to a
-    // compute unit: 34 ms).
+    // as keep the memory path busy, second-order walks an eighth of the pass at a time if that is more, but no more than four
+    // wavefronts to a SIMD: the packing needs room in LDS beside them (R-MAT 22 node2vec with 20 to a compute unit: 34
+    // ms).  Passes with their rows, ms, by wavefronts a compute unit (Chung-Lu graphs, mean degree 10 to 12):
+    //                            6     8    10    12    16                               2     3     4     5     6
+    //    uniform       800 K  3.11  3.13  3.15  3.23  3.38           MultiRW  200 K   1.84  1.72  1.93  2.19  2.33
+    //                  1.1 M  4.14  4.13  4.15  4.23  4.42                    400 K   3.36  3.07  3.23  3.54  3.81
+    //    DeepWalk      1.1 M  4.99  4.90  4.93  5.00  5.20                    1.1 M         7.73  8.28  8.76  9.33
+    //       R-MAT 22         16.17 15.99 16.12 16.44 17.28
+    //    PPR           1.1 M  4.46  4.29  4.37  4.41  4.53
+    //    weighted n2v  550 K  4.61  4.08  4.11  4.17  4.40
+    //                  1.1 M  8.60  7.29  6.78  6.87  7.97
+    //       R-MAT 22          33.7  28.8  26.2  25.2  24.4
     constexpr bool kSecondOrder = state_fits_pair<SampleType>::value;
     constexpr uint64_t kLeast = kSecondOrder ? 10 : std::is_empty<SampleType>::value ? 8 : 3;
     const uint64_t blocks = ((uint64_t)count + kWave - 1) / kWave;
@@ -2806,7 +2828,7 @@ class Engine : public EngineBase {
   static constexpr int kBalanceWords =
       kMaxSteps + 2 + (int)(kCounterCopies * sizeof(ClassCounters) / sizeof(uint32_t));
   static constexpr int kIdleLookEvery = 8;
-  static constexpr uint32_t kMostWalkRanges = 4;
+  static constexpr uint32_t kMostWalkRanges = 6;
   static constexpr uint32_t kMostStretches = 1024;  // of a pass whose rows leave early
 
   // Whether a pass brings the pairs into transit order (or, sample-parallel and no walk, only drops the dead ones).

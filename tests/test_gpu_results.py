@@ -153,15 +153,21 @@ def test_walks_take_device_memory_for_what_they_run():
         s.close()
 
 
-# the forms a walk has: its state in registers, in memory (and transits of its own), the edges as walk records
-@pytest.mark.parametrize("app,kind,n,mean_degree", [
-    ("WeightedNode2Vec8", "WEIGHTED_NODE2VEC", 360007, 3),
-    ("MultiRW4x6", "MULTIRW", 300007, 3),
-    ("UniformRandomWalk8", "UNIFORM_WALK", 600011, 15),
-    ("DeepWalkPerVertex", "DEEPWALK", 500009, 9),
+# the forms a walk has: its state in registers, in memory (and transits of its own), the edges as walk records; each in one launch
+# whose rows leave by stretch, from the least number of walks on (1), and below it by the range, in so many launches
+@pytest.mark.parametrize("app,kind,n,mean_degree,launches", [
+    ("WeightedNode2Vec8", "WEIGHTED_NODE2VEC", 360007, 3, 2),
+    ("WeightedNode2Vec8", "WEIGHTED_NODE2VEC", 1523713, 3, 1),
+    ("MultiRW4x6", "MULTIRW", 300007, 3, 4),
+    ("MultiRW4x6", "MULTIRW", 812647, 3, 1),
+    ("UniformRandomWalk8", "UNIFORM_WALK", 600011, 15, 4),
+    ("UniformRandomWalk8", "UNIFORM_WALK", 1777663, 2, 6),
+    ("UniformRandomWalk8", "UNIFORM_WALK", 1777664, 2, 1),
+    ("DeepWalkPerVertex", "DEEPWALK", 350003, 12, 3),
+    ("DeepWalkPerVertex", "DEEPWALK", 500009, 9, 1),
 ])
 @pytest.mark.parametrize("mode", ["transit", "sample"])
-def test_rows_of_every_kind_of_walk_leave_before_the_pass_is_over(oracle, app, kind, n, mean_degree, mode):
+def test_rows_of_every_kind_of_walk_leave_before_the_pass_is_over(oracle, app, kind, n, mean_degree, launches, mode):
     g = graphs.random_graph(n=n, mean_degree=mean_degree, seed=n, isolated_every=5)
     og = graphs.oracle_view(g)
     s = nd.Sampler(app, g, seed=42)
@@ -184,8 +190,7 @@ def test_rows_of_every_kind_of_walk_leave_before_the_pass_is_over(oracle, app, k
         for turn, states_first in enumerate([False, False, True, True]):
             print("app", app, "mode", mode, "turn", turn, flush=True)
             run()
-            # all walks in one launch, whatever has become of their rows
-            assert s.phase_times()["flat_launches"] == 1
+            assert s.phase_times()["flat_launches"] == (launches if turn else 1)
             if states_first and want_states is not None:
                 assert np.array_equal(states_of()[alive], want_states[alive])
             assert np.array_equal(s.final_samples(), want)
