@@ -1,6 +1,7 @@
 // Results brought to the host by ResultStream (nd_host_results.hpp), against the words that were put on the device:
 // every width, sizes around a group, a chunk and a piece, dead groups, ids that do not fit their width, targets that
-// are no multiple of 32 bytes.  Prints the case before it runs, "all equal" at the end.
+// are no multiple of 32 bytes; straight to the host, and packed on the device as words that come while others are still
+// computed are, with a sign that is there and with one that never comes.  Prints the case before it runs, "all equal" at the end.
 #include "../../nextdoor_amd/csrc/nd_host_results.hpp"
 
 #include <stdio.h>
@@ -136,6 +137,11 @@ int main() {
   const size_t piece = (size_t)64 * nd::kPackChunk;  // the smallest piece
   const size_t sizes[] = {1, 7, 8, 9, nd::kPackChunk - 1, nd::kPackChunk, nd::kPackChunk + 1, piece, piece + 9, 13 * piece + 4097};
   nd::ResultStream stream;
+  uint32_t* sign = nullptr;  // what has arrived, and what never does
+  hipEvent_t done;
+  TRY(hipHostMalloc((void**)&sign, 2 * sizeof(uint32_t), hipHostMallocDefault));
+  sign[0] = 3, sign[1] = 0;
+  TRY(hipEventCreateWithFlags(&done, hipEventDisableTiming));
   for (size_t n : sizes) {
     int32_t* d = nullptr;
     TRY(hipMalloc(&d, n * sizeof(int32_t)));
@@ -163,10 +169,27 @@ int main() {
             return 1;
           }
         }
+        TRY(hipEventRecord(done, nullptr));
+        TRY(hipEventSynchronize(done));
+        for (int comes = 0; comes < 2; ++comes) {
+          const uint32_t* word = sign + 1 - comes;
+          std::vector<nd::ResultStream::Ready> ready{{n, done, word, 3}};
+          if (n > 1) ready.insert(ready.begin(), {n / 2, done, word, 3});
+          std::fill(got.begin(), got.end(), 77);
+          TRY(stream.begin(d, n, bits, fill, got.data() + comes, nullptr, ready));
+          TRY(stream.finish());
+          if (memcmp(got.data() + comes, want.data(), n * sizeof(int32_t)) != 0 || got[n + 1] != 77) {
+            printf("differs where the sign comes %d\n", comes);
+            return 1;
+          }
+        }
       }
     }
     TRY(hipFree(d));
   }
+  stream.release();
+  TRY(hipHostFree(sign));
+  TRY(hipEventDestroy(done));
   printf("all equal\n");
   return 0;
 }

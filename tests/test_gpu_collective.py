@@ -216,6 +216,14 @@ def test_ladies_keys_that_are_hard_to_tell_apart(oracle, weights, pieces, monkey
     for _ in range(2):
         s.do_transit_parallel(True)
         assert np.array_equal(s.final_samples(), want)
+    assert s.counter(2) == s.steps  # one chunk a layer
+    s.close()
+    monkeypatch.setenv("ND_LAYER_CHUNK_ENTRIES", str(20 * n))
+    s = nd.Sampler("LADIESImportance2x8", g, seed=SEED)
+    for _ in range(2):
+        s.do_transit_parallel(True)
+        assert np.array_equal(s.final_samples(), want)
+    assert s.counter(2) > 3 * s.steps
     s.close()
 
 
