@@ -330,7 +330,8 @@ __device__ __forceinline__ uint32_t last_key_of_bin(uint32_t bin) { return 0x800
 // What a workgroup keeps at most: room for everything a stretch can add to what it may begin the stretch with.
 constexpr uint32_t kKeptEntries = 12288;
 struct KeptKeys {
-  uint2* kept;          // (key, vertex), [workgroup of the chunk][kKeptEntries]
+  uint2* kept;          // (key, vertex), [workgroup of the chunk][room]
+  uint32_t room;        // kKeptEntries, or as many as there are vertices
   uint32_t* n_kept;     // [workgroup of the chunk]
   uint32_t* bound;      // [marked sample]; kNoBound before the layer
   uint32_t* distinct;   // [sample of the chunk]; 0 before the layer
@@ -541,7 +542,7 @@ __global__ __launch_bounds__(kBinThreads, 8) __attribute__((amdgpu_num_vgpr(56))
   const uint32_t first_bin = group * kBinsPerGroup;
   const int32_t* transits = tv.base + (size_t)s * tv.stride;
   const uint32_t listing = at * (gridDim.x / n_samples) + group;
-  uint2* const kept = out.kept + (size_t)listing * kKeptEntries;
+  uint2* const kept = out.kept + (size_t)listing * out.room;
   uint32_t* const sample_bound = out.bound + at;
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wave = threadIdx.x >> 6;
@@ -1071,7 +1072,7 @@ __global__ __launch_bounds__(kBinThreads) void kept_layer_kernel(LayerParams P, 
   auto each = [&](auto f) {
     for (uint32_t g = 0; g < groups; ++g) {
       const uint32_t listing = at * groups + g, n = in.n_kept[listing];
-      const uint2* kept = in.kept + (size_t)listing * kKeptEntries;
+      const uint2* kept = in.kept + (size_t)listing * in.room;
       for (uint32_t i = threadIdx.x; i < n; i += kBinThreads) {
         const uint2 mine = kept[i];
         if (mine.x <= bound) f(rank_value(mine));
@@ -1257,7 +1258,7 @@ class LayerEngine : public EngineBase {
     // to whole stretches (LADIES form)
     uint64_t bytes_per_sample = (uint64_t)bitmap_words_ * sizeof(uint32_t);
     if (apps::neighborhood_form_of<App>::value == apps::kRankedByLadiesImportance) {
-      bytes_per_sample = (uint64_t)ladies_groups() * kKeptEntries * sizeof(uint2);
+      bytes_per_sample = (uint64_t)ladies_groups() * kept_room() * sizeof(uint2);
     }
     const uint64_t fit = kBitmapBudgetBytes / bytes_per_sample;
     bitmap_chunk_samples_ = fit < 1 ? 1u : fit > (uint64_t)n_samples_ ? (uint32_t)n_samples_ : (uint32_t)fit;
@@ -1717,7 +1718,7 @@ class LayerEngine : public EngineBase {
     if ((uint64_t)n * groups >= (1ull << 31)) { last_error = "a chunk needs 2^31 or more workgroups"; return -1; }
     if (n > bitmap_samples_) {
       release(d_kept_); release(d_n_kept_); release(d_bound_);
-      ND_HIP_TRY(hipMalloc(&d_kept_, sizeof(uint2) * kKeptEntries * (size_t)n * groups));
+      ND_HIP_TRY(hipMalloc(&d_kept_, sizeof(uint2) * kept_room() * (size_t)n * groups));
       ND_HIP_TRY(hipMalloc(&d_n_kept_, sizeof(uint32_t) * (size_t)n * groups));
       ND_HIP_TRY(hipMalloc(&d_bound_, sizeof(uint32_t) * (size_t)n));
       bitmap_samples_ = n;
@@ -1733,6 +1734,7 @@ class LayerEngine : public EngineBase {
     ranked_layer_kernel<SampleType, App><<<dim3(n), dim3(kRankedThreads), 0, stream_>>>(P, merged_, d_merged_sizes_, distinct);
     KeptKeys kept;
     kept.kept = d_kept_;
+    kept.room = kept_room();
     kept.n_kept = d_n_kept_;
     kept.bound = d_bound_;
     kept.distinct = distinct;
@@ -1750,6 +1752,7 @@ class LayerEngine : public EngineBase {
   }
   uint32_t ladies_bins() const { return (bitmap_words_ + kBinWords - 1) / kBinWords; }
   uint32_t ladies_groups() const { return (ladies_bins() + kBinsPerGroup - 1) / kBinsPerGroup; }
+  uint32_t kept_room() const { return std::max(1u, std::min(kKeptEntries, (uint32_t)invalid_)); }  // no vertex is kept twice
 
   // The concatenated neighbourhood itself (kConcatenated form).
   int ensure_neighborhood_capacity(uint32_t total) {

@@ -1,6 +1,7 @@
 """GPU parity of the layer-wise (CollectiveNeighborhood) engine against the CPU oracle:
 collective-neighbourhood build, the reference's FastGCN/LADIES app (vertices, recorded
 adjacency-matrix entries, the reference's validator) and the importance sampler."""
+import ctypes
 import os
 import re
 import subprocess
@@ -33,6 +34,13 @@ def test_collective_neighborhood_matches_oracle(oracle):
         assert np.array_equal(weights[offsets[s]:offsets[s + 1]], ww)
         assert np.array_equal(rows[s], wr)
     assert sizes[3] == 0
+
+
+def device_memory_left():
+    hip = ctypes.CDLL("libamdhip64.so")
+    left, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert hip.hipMemGetInfo(ctypes.byref(left), ctypes.byref(total)) == 0
+    return left.value
 
 
 def layer_desc(oracle, s, kind):
@@ -225,6 +233,23 @@ def test_ladies_keys_that_are_hard_to_tell_apart(oracle, weights, pieces, monkey
         assert np.array_equal(s.final_samples(), want)
     assert s.counter(2) > 3 * s.steps
     s.close()
+
+
+def test_what_is_kept_of_a_sample_is_no_more_than_there_are_vertices(oracle):
+    """1024 samples over 2000 vertices: 16 MB for what is kept of them, where room for a workgroup's stretches is 100."""
+    g = graphs.random_graph(n=2000, mean_degree=60, seed=6, hub=5)  # 512 roots have 30000 neighbours: ranked in parts
+    before = device_memory_left()
+    s = nd.Sampler("LADIESImportance", g, seed=SEED)
+    try:
+        s.do_transit_parallel(True)
+        taken = before - device_memory_left()
+        print("taken", taken, flush=True)
+        assert taken < 64 << 20
+        want = oracle.sample_ladies_importance(graphs.oracle_view(g), layer_desc(oracle, s, oracle.LADIES_IMPORTANCE), SEED,
+                                               s.initial_contents)
+        assert np.array_equal(s.final_samples(), want)
+    finally:
+        s.close()
 
 
 @pytest.mark.parametrize("app,kind_name", [("FastGCNImportance3x16", "FASTGCN_IMPORTANCE"),
