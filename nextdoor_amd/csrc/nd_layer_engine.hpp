@@ -288,9 +288,9 @@ __device__ __forceinline__ uint32_t ladies_key_bits(unsigned long long importanc
 
 // One workgroup per (sample, some consecutive stretches of 7168 vertices), the sums of one stretch in LDS at a time.
 // Adjacencies are sorted by destination, so the part of a transit's adjacency that falls into a stretch is one
-// sub-range; the workgroup streams the sub-ranges of all the sample's transits, adds in LDS, and writes the stretch
-// over once, and no atomic reaches memory (global atomics stop at ~24 G/s on this part).  Every wavefront walks a contiguous part of the stretch's entries,
-// which lets a lane step from one sub-range to the next instead of searching the table for every entry.
+// sub-range; the workgroup streams the sub-ranges of all the sample's transits and adds in LDS, and no atomic reaches
+// memory (global atomics stop at ~24 G/s on this part).  Every wavefront walks a contiguous part of the stretch's entries,
+// a few of each lane at a time, and finds the sub-range of each from bits that say where the next ones start.
 constexpr uint32_t kBinThreads = 1024;
 constexpr uint32_t kBinWaves = kBinThreads / 64;
 constexpr uint32_t kBinAhead = 4;             // entries a lane fetches before it works on the first
@@ -515,11 +515,11 @@ constexpr uint32_t kSparseGroupEntries = 2048;
 // The samples that are not ranked in LDS (ranked_layer).
 // Two workgroups of 16 wavefronts share a compute unit only at 8 wavefronts per SIMD, which the kernel's attributes ask
 // the compiler for.
-// 500 K vertices, 12 M edges, second layer of 1024 samples of 512 (1.5 M pairs and 136 pieces a sample): 2.59 ms.  Writing a
+// 500 K vertices, 12 M edges, second layer of 1024 samples of 512 (1.5 M pairs and 136 pieces a sample): 2.52 ms.  Writing a
 // key for every vertex it took 3.42, and the selection, the collecting and the sorts 1.1 more, where kept_layer_kernel takes
 // 0.04; forming only keys that may be within the bound 3.17, the ids of all of a round's entries under way before the first
-// is used 2.86, starts as bits 2.59.  What bounds it now: the vector ALU is at work 65 % of the time, the rest is the phases of a
-// stretch waiting for each other.
+// is used 2.86, starts as bits 2.59.  What bounds it now: vector instructions take 69 % of the issue slots (1.08 G of them at four
+// clocks), the rest is the phases of a stretch waiting for each other, and registers that do not fit.
 __global__ __launch_bounds__(kBinThreads, 8) __attribute__((amdgpu_num_vgpr(56))) void collective_mark_binned(
     MergedEdges merged, TransitView tv, int32_t invalid, uint32_t n_samples, const uint32_t* __restrict__ n_marked,
     const uint32_t* __restrict__ marked, uint32_t bins_per_sample, DensePieces dense, KeptKeys out) {
@@ -1052,7 +1052,8 @@ __global__ __launch_bounds__(kRankedThreads) void ranked_layer_kernel(LayerParam
 
 // A workgroup per marked sample: the best of what the workgroups of collective_mark_binned have kept of it, in order, and the
 // draws.  An edge between counts first, as there, over all of them together; where more are at or below it than there is room
-// for (many equal keys), the wanted ones are picked out exactly.  1024 samples of 512, five workgroups' keys each: 0.03 ms.
+// for (many equal keys), the wanted ones are picked out exactly.  1024 samples of 512, five workgroups' keys each (500 K
+// vertices): 0.044 ms; 27 workgroups' (3.07 M vertices): 0.08.
 constexpr uint32_t kBestEntries = 2048;
 template <class SampleType, class App>
 __global__ __launch_bounds__(kBinThreads) void kept_layer_kernel(LayerParams P, const uint32_t* __restrict__ n_marked,
@@ -1153,8 +1154,8 @@ __global__ __launch_bounds__(256) void marked_layer_kernel(LayerParams P, Marked
 // Entries of concatenated neighbourhood one chunk of samples may hold (about 70 bytes of
 // device memory per entry across all work arrays).
 constexpr uint64_t kLayerChunkEntries = 96ull << 20;
-// Importance forms: nothing is stored per entry, so a chunk is bounded by the memory of its
-// presence maps (and accumulators) and by the number of marking work items (entries / kBuildItemEntries) of one launch.
+// Importance forms: nothing is stored per entry, so a chunk is bounded by the memory of its presence maps or of the keys
+// that are kept.
 constexpr uint64_t kBitmapBudgetBytes = 48ull << 30;
 constexpr uint64_t kBitmapChunkEntries = 1ull << 40;
 
@@ -1252,10 +1253,8 @@ class LayerEngine : public EngineBase {
       const long long v = atoll(env);
       if (v > 0) chunk_entries_ = bitmap_chunk_entries_ = (uint64_t)v;
     }
-    // one byte per vertex for the LADIES form, one bit for the FastGCN form
     bitmap_words_ = bitmap_words_for((uint32_t)invalid_);
-    // bytes a sample of a chunk holds: its bitmap (FastGCN form) or one key per vertex, padded
-    // to whole stretches (LADIES form)
+    // bytes a sample of a chunk holds: its bitmap (FastGCN form), or what its workgroups keep (LADIES form)
     uint64_t bytes_per_sample = (uint64_t)bitmap_words_ * sizeof(uint32_t);
     if (apps::neighborhood_form_of<App>::value == apps::kRankedByLadiesImportance) {
       bytes_per_sample = (uint64_t)ladies_groups() * kept_room() * sizeof(uint2);
