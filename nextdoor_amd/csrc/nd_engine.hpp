@@ -121,7 +121,7 @@ class EngineBase {
   // Device memory to the host, complete on return.  bits, fill: what is known of its words (ResultStream::fetch).
   int fetch_to_host(void* dst, const void* src, size_t bytes, uint32_t bits, int32_t fill, hipStream_t stream) {
     hipError_t e;
-    if (bytes > kDirectResultBytes && bytes % sizeof(int32_t) == 0) {
+    if (bytes % sizeof(int32_t) == 0) {
       e = result_stream->fetch((const int32_t*)src, bytes / sizeof(int32_t), bits, fill, (int32_t*)dst, stream);
     } else {
       e = result_stream->copy(src, bytes, dst, stream);
@@ -2135,7 +2135,7 @@ class Engine : public EngineBase {
     (void)finish_rows_ahead();  // nobody asked for them
     if ((inverts(mode) ? alloc_inversion() : build_walk_tables()) != 0) return -1;  // what an earlier pass has not
     times = PhaseTimes();
-    sent_ahead_ = false;
+    sent_ahead_ = rows_follow_ = false;
     if (!std::is_empty<SampleType>::value) {
       ND_HIP_TRY(hipMemcpyAsync(d_samples_, d_samples_init_, sizeof(SampleType) * (size_t)n_samples_,
                                 hipMemcpyDeviceToDevice, stream_));
@@ -2153,7 +2153,8 @@ class Engine : public EngineBase {
     const int rc = wants_launch_graph() ? replay_pass(mode) : enqueue_pass(mode);
     if (rc != 0) return rc;
     ND_HIP_TRY(hipEventRecord(ev_end_, stream_));
-    ND_HIP_TRY(hipStreamSynchronize(stream_));
+    if (rows_follow_) send_rows({}, ev_end_);
+    ND_HIP_TRY(hipEventSynchronize(ev_end_));
     ND_HIP_TRY(hipEventElapsedTime(&times.end_to_end, ev_begin_, ev_end_));
     schedule_counts_.passes++;
     if (balanced_this_pass_) {
@@ -2214,7 +2215,8 @@ class Engine : public EngineBase {
     const uint32_t ranges = form == kRowsByRange ? walk_ranges() : 1;
     const size_t F = (size_t)final_sample_size();
     std::vector<ResultStream::Ready> ready;
-    while (form != kRowsStay && range_ends_.size() < ranges) {
+    rows_follow_ = form == kRowsFollow;
+    while (form != kRowsStay && form != kRowsFollow && range_ends_.size() < ranges) {
       hipEvent_t ev = nullptr;
       ND_HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
       range_ends_.push_back(ev);
@@ -2223,7 +2225,7 @@ class Engine : public EngineBase {
     for (uint32_t r = 0; r < ranges; ++r) {
       const uint32_t end = r + 1 == ranges ? (uint32_t)n_samples_ : (uint32_t)((uint64_t)n_samples_ * (r + 1) / ranges / kWave * kWave);
       if (launch_walks(first, end - first, d_walk_queue_ + 2 * r, early) != 0) return -1;
-      if (form == kRowsStay) return 0;
+      if (form == kRowsStay || form == kRowsFollow) return 0;
       ND_HIP_TRY(hipEventRecord(range_ends_[r], stream_));
       ready.push_back({end * F, range_ends_[r]});
       first = end;
@@ -2234,16 +2236,20 @@ class Engine : public EngineBase {
         ready.push_back({(size_t)std::min<uint64_t>((uint64_t)n_samples_, at + (1ull << early.shift)) * F, range_ends_[0],
                          h_arrived_ + (at >> early.shift), early.pass});
     }
-    // rows that cannot be sent now are fetched when they are asked for
+    send_rows(std::move(ready), nullptr);
+    sent_ahead_ = ahead_;
+    return 0;
+  }
+
+  // Has the rows leave for rows_ahead; those that cannot be sent now are fetched when they are asked for.
+  void send_rows(std::vector<ResultStream::Ready> ready, hipEvent_t computed) {
     try {
-      ahead_ = result_stream->begin(d_final_, (size_t)n_samples_ * F, (uint32_t)max_bits_, invalid_, rows_ahead, stream_,
-                                   std::move(ready)) == hipSuccess;
+      ahead_ = result_stream->begin(d_final_, (size_t)n_samples_ * (size_t)final_sample_size(), (uint32_t)max_bits_, invalid_,
+                                   rows_ahead, stream_, std::move(ready), computed) == hipSuccess;
     } catch (const std::bad_alloc&) {
       ahead_ = false;
     }
     if (!ahead_) (void)hipGetLastError();
-    sent_ahead_ = ahead_;
-    return 0;
   }
 
   // How rows leave before the pass is over.  kRowsByStretch: one launch, whose wavefronts count the walks that are done by
@@ -2287,14 +2293,15 @@ class Engine : public EngineBase {
   // Where the two meet moves with the graph (second-order walks of 400 K from 10 % for stretches to 6 % against them, by its
   // degree), and with the walks' length as if a walk were 24 results longer.  Longer walks are not taken from fewer on: a pass whose
   // walks are all under way at once has no first ones.
-  enum EarlyForm { kRowsStay, kRowsByRange, kRowsByStretch };
+  // kRowsFollow: one launch, and the rows' packing directly behind it.
+  enum EarlyForm { kRowsStay, kRowsFollow, kRowsByRange, kRowsByStretch };
   EarlyForm early_form(EarlyRows* early) {
     if (!rows_ahead || profiling || wants_launch_graph()) return kRowsStay;
     const uint64_t n = (uint64_t)n_samples_, results = (uint64_t)final_sample_size();
-    if (sizeof(VertexID_t) * n * results <= kDirectResultBytes) return kRowsStay;
     constexpr uint64_t kOf100Steps = state_fits_pair<SampleType>::value ? 384 << 10 : std::is_empty<SampleType>::value ? 448 << 10 : 192 << 10;
     const bool many = n * (std::min<uint64_t>(results, 100) + 24) >= kOf100Steps * (100 + 24);
-    return many && ready_for_early_rows(early) ? kRowsByStretch : kRowsByRange;
+    if (many && ready_for_early_rows(early)) return kRowsByStretch;
+    return walk_ranges() > 1 && sizeof(VertexID_t) * n * results > kDirectResultBytes ? kRowsByRange : kRowsFollow;
   }
   uint32_t walk_ranges() const {
     constexpr int64_t least = std::is_empty<SampleType>::value ? 96 << 10 : state_fits_pair<SampleType>::value ? 128 << 10 : 40 << 10;
@@ -2810,11 +2817,11 @@ class Engine : public EngineBase {
     }
     ND_HIP_TRY(hipGetLastError());
     ND_HIP_TRY(hipEventRecord(ev_end_, stream_));
-    ND_HIP_TRY(hipStreamSynchronize(stream_));
-    ND_HIP_TRY(hipEventElapsedTime(&times.distinct, ev_begin_, ev_end_));
     hDistinctCounts.resize((size_t)n_samples_ * n_steps);
-    ND_HIP_TRY(hipMemcpy(hDistinctCounts.data(), d_distinct_counts_, sizeof(int32_t) * hDistinctCounts.size(),
-                         hipMemcpyDeviceToHost));
+    if (fetch_to_host(hDistinctCounts.data(), d_distinct_counts_, sizeof(int32_t) * hDistinctCounts.size(), 32, -1, stream_) != 0)
+      return -1;
+    ND_HIP_TRY(hipEventSynchronize(ev_end_));
+    ND_HIP_TRY(hipEventElapsedTime(&times.distinct, ev_begin_, ev_end_));
     return 0;
   }
 
@@ -3206,7 +3213,8 @@ class Engine : public EngineBase {
   const walk_record<App>* walk_records_ = nullptr;  // dgraph_'s, where they pay
   uint32_t walk_waves_at_once_ = 1, cus_ = 1;  // wavefronts of walk_rows_kernel the device holds, compute units
   bool ahead_ = false;                    // rows are on their way to rows_ahead
-  bool sent_ahead_ = false;               // ... or have been, in the last pass
+  bool sent_ahead_ = false;               // ... or have been, in the last pass, while its walks were under way
+  bool rows_follow_ = false;              // the pass under way sends them directly behind its last launch
   std::vector<hipEvent_t> range_ends_;    // ends of the launches of such a pass
   // of such a pass: EarlyRows::arrived and walked, and the number of the last
   uint32_t *h_arrived_ = nullptr, *d_walked_ = nullptr;

@@ -9,8 +9,8 @@
 //    number of vertices, needs (23 instead of 32 for R-MAT 22), and groups of eight consecutive
 //    ids that are all INVALID - walks that have ended, samples without neighbours - are left out.
 //    The kernel writes its output straight into page-locked memory (54.7 GB/s, as fast as the copy
-//    engine's 57, without a launch and a copy per piece), and host threads unpack a piece
-//    while the next one crosses.  Twelve threads write 220 GB/s of unpacked ids on the 16-core share of a
+//    engine's 57, without a copy per piece) and stamps every chunk that is there, and host threads unpack
+//    a chunk while the next ones cross.  Twelve threads write 220 GB/s of unpacked ids on the 16-core share of a
 //    GPU's host, 140 while the bus writes to the same memory at its full rate.
 //  * Results whose first words are final while later ones are still being computed (walks) can leave then already
 //    (ResultStream::begin, with what to wait for).  They are packed into device memory and the copy engine takes them
@@ -174,9 +174,9 @@ struct HostBlock {
   bool mapped = false;  // by mmap, else from the heap
 };
 
-// Results up to this size go through page-locked memory by the copy engine and one thread, above it they are packed and
-// streamed by several.  Copied / streamed with ids of 12 and of 32 bits, us: 0.5 MB 31 / 75, 82; 1.1 MB 67 / 95, 105;
-// 1.5 MB 92 / 100, 116; 2 MB 118 / 110, 128; 3 MB 169 / 121, 155; 4 MB 220 / 113, 158.
+// Results up to this size are unpacked by the thread that asks for them, and into the caches: other threads are awake 50 us
+// later (64 KB to 2 MB in 31 to 118 us by the copy engine and memcpy(), which also waited for the bus before it began; walks
+// over 2.7 K vertices, 1.1 MB, whose packing follows them: 0.121 ms a pass instead of 0.147).
 constexpr size_t kDirectResultBytes = 2u << 20;
 
 // The host arrays of one sampler.  A few of them (keep()) wait for their next use; all of those are freed with the
@@ -361,38 +361,63 @@ constexpr uint32_t kPackChunkGroups = 512;                       // groups of a 
 constexpr uint32_t kPackChunk = kPackGroup * kPackChunkGroups;   // ids of a chunk: 16 KB of results
 constexpr uint32_t kPackMostBits = 25;                           // wider ids travel as whole words
 
-// What a chunk's groups are: which of them hold anything but `fill` (bit g of word g / 64), and whether an id
-// did not fit its bits.
+// What a chunk's groups are: which of them hold anything but `fill` (bit g of word g / 64), how many bits an id of
+// theirs takes, counted from the smallest (all ones: `fill`; 32: the words as they are), and whether that is more than there is room for.
 struct PackHeader {
   uint64_t live[kPackChunkGroups / 64];
   uint64_t overflow;
   uint64_t at;  // of its bytes among the piece's, if staged
-  uint64_t pad[6];
+  uint32_t bits, base;
+  uint64_t stamp;  // straight to the host: the transfer's number and the chunk's, once all else of the chunk is there
+  uint64_t pad[4];
 };
+static_assert(sizeof(PackHeader) == 128, "a line of memory");
 
-// Where the chunks' bytes go: chunk after chunk, each as far from the last as a whole one takes, or (staged) one directly
-// after another, in whatever order the workgroups get there, for a copy that is to take no more than there is.
+// Where the chunks' bytes go: chunk after chunk, each as far from the last as a whole one takes, round a ring (a power of two chunks, or
+// more than there are), or (staged) one directly after another, in whatever order the workgroups get there, for a copy that is to
+// take no more than there is.
 struct PackedOut {
   uint8_t* bytes;
   PackHeader* headers;
+  // straight
+  uint32_t first = 0, ring_mask = 0xffffffffu;  // of the launch's first chunk
+  uint64_t stamp = 0;                           // its
   // staged
   uint32_t* cursor = nullptr;    // 16 bytes each; 0 before the launch and after it
   uint32_t* finished = nullptr;  // workgroups; likewise
   uint32_t* total = nullptr;     // host memory: what cursor was at the end
 };
 
-// Packs ids [chunk * kPackChunk, ...) of src into out[chunk * kPackChunkGroups * bits ...): the groups of
-// eight that are not all `fill`, back to back, `bits` bytes each.  Where out is host memory the
-// stores to it are what takes the time (54.7 GB/s of packed bytes; packing the 1.68 GB of R-MAT 22 walks into
-// device memory instead takes a twentieth of it), hence whole chunks through LDS and 16-byte stores by
-// consecutive lanes; nothing else here is tuned.  (kStaged is the kernel's and not the launch's: with both forms' loads in one
-// kernel those of a chunk wait for each other, and MultiRW 100 K took 1.59 ms instead of 1.55, KHop over R-MAT 20 11.7 instead
-// of 11.4.)
+// Bits for the numbers 0 .. range and one more, all of them ones.
+__host__ __device__ inline uint32_t bits_for_range(uint32_t range) {
+  uint32_t bits = 1;
+  while (bits <= kPackMostBits && range >= (1u << bits) - 1u) bits++;
+  return bits <= kPackMostBits ? bits : 32u;
+}
+
+__device__ __forceinline__ void store_past_caches(uint4* at, uint4 v) {
+  typedef uint32_t Four __attribute__((ext_vector_type(4)));
+  const Four x = {v.x, v.y, v.z, v.w};
+  // (two wait states before its registers are written again, as the compiler would have them)
+  asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" : : "v"(at), "v"(x) : "memory");
+}
+
+// Packs ids [chunk * kPackChunk, ...) of src: the groups of eight that are not all `fill`, back to back, at most `bits` bits an
+// id.  Where out is host memory the stores to it are what takes the time (54.7 GB/s of packed bytes; packing the 1.68 GB of
+// R-MAT 22 walks into device memory instead takes a twentieth of it), hence whole chunks through LDS and 16-byte stores by
+// consecutive lanes.  Such a chunk is stamped when its bytes have been acknowledged: the threads that unpack it look for that,
+// so that any number of chunks is one launch (uniform walks 57 K, whose rows were nine launches with an event and
+// 5.6 us between each and the next: 225 us from the first to the last, now 180).  Ids are counted from the chunk's
+// smallest: two in five bits of what MVS lists (rows of 32 batches of consecutive vertices: 9 bits instead of 18) and, with
+// `fill` all ones, one of the 21 that 2^20 vertices and INVALID would take.  (kStaged is the kernel's and not the launch's: with both
+// forms' loads in one kernel those of a chunk wait for each other, and MultiRW 100 K took 1.59 ms instead of 1.55, KHop over
+// R-MAT 20 11.7 instead of 11.4.)
 template <bool kStaged>
-__global__ __launch_bounds__(kPackThreads) void pack_results(const int32_t* __restrict__ src, size_t n, uint32_t bits,
+__global__ __launch_bounds__(kPackThreads) void pack_results(const int32_t* __restrict__ src, size_t n, uint32_t most_bits,
                                                              int32_t fill, PackedOut out, uint32_t n_chunks) {
   __shared__ __align__(16) uint8_t s_packed[kPackChunk * sizeof(int32_t)];
   __shared__ uint64_t s_live[kPackChunkGroups / 64];
+  __shared__ uint32_t s_least[kPackThreads / 64], s_largest[kPackThreads / 64];
   __shared__ uint32_t s_at;
   constexpr uint32_t kRounds = kPackChunkGroups / kPackThreads;
   const uint32_t lane = threadIdx.x & 63u;
@@ -400,7 +425,7 @@ __global__ __launch_bounds__(kPackThreads) void pack_results(const int32_t* __re
     const size_t first = (size_t)chunk * kPackChunk;
     int32_t ids[kRounds][kPackGroup];
     bool live[kRounds];
-    bool overflow = false;
+    uint32_t least = 0xffffffffu, largest = 0;  // of those that are not `fill`
 #pragma unroll
     for (uint32_t r = 0; r < kRounds; ++r) {
       const size_t at = first + (size_t)(r * kPackThreads + threadIdx.x) * kPackGroup;
@@ -426,20 +451,36 @@ __global__ __launch_bounds__(kPackThreads) void pack_results(const int32_t* __re
         for (uint32_t i = 0; i < kPackGroup; ++i)
           ids[r][i] = at + i >= n ? fill : kStaged ? __hip_atomic_load(src + at + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) : src[at + i];
       }
+    }
+#pragma unroll
+    for (uint32_t r = 0; r < kRounds; ++r) {
       live[r] = false;
 #pragma unroll
-      for (uint32_t i = 0; i < kPackGroup; ++i) live[r] = live[r] || ids[r][i] != fill;
+      for (uint32_t i = 0; i < kPackGroup; ++i) {
+        const bool counts = ids[r][i] != fill;
+        live[r] = live[r] || counts;
+        least = counts && (uint32_t)ids[r][i] < least ? (uint32_t)ids[r][i] : least;
+        largest = counts && (uint32_t)ids[r][i] > largest ? (uint32_t)ids[r][i] : largest;
+      }
       const uint64_t mask = __ballot(live[r]);
       if (lane == 0) s_live[(r * kPackThreads + threadIdx.x) / 64u] = mask;
-      if (bits < 32 && live[r]) {
-        if (at + kPackGroup > n)  // what fills the last group up need not fit
-#pragma unroll
-          for (uint32_t i = 0; i < kPackGroup; ++i) ids[r][i] = at + i < n ? ids[r][i] : 0;
-#pragma unroll
-        for (uint32_t i = 0; i < kPackGroup; ++i) overflow = overflow || ((uint32_t)ids[r][i] >> bits) != 0;
-      }
     }
-    const int any_overflow = __syncthreads_or(overflow ? 1 : 0);
+    for (int d = 32; d > 0; d >>= 1) {
+      const uint32_t a = (uint32_t)__shfl_xor((int)least, d, 64), b = (uint32_t)__shfl_xor((int)largest, d, 64);
+      least = a < least ? a : least;
+      largest = b > largest ? b : largest;
+    }
+    if (lane == 0) s_least[threadIdx.x / 64u] = least, s_largest[threadIdx.x / 64u] = largest;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t w = 0; w < kPackThreads / 64; ++w) {
+      least = s_least[w] < least ? s_least[w] : least;
+      largest = s_largest[w] > largest ? s_largest[w] : largest;
+    }
+    const bool any = least <= largest;
+    const uint32_t bits = any ? bits_for_range(largest - least) : 1u;
+    const bool overflow = bits > most_bits;
+    const uint32_t base = bits == 32 || !any ? 0u : least, none = bits == 32 ? (uint32_t)fill : (1u << bits) - 1u;
     uint32_t total = 0;
 #pragma unroll
     for (uint32_t r = 0; r < kRounds; ++r) {
@@ -458,7 +499,7 @@ __global__ __launch_bounds__(kPackThreads) void pack_results(const int32_t* __re
       uint32_t held = 0;
 #pragma unroll
       for (uint32_t i = 0; i < kPackGroup; ++i) {
-        acc |= (uint64_t)(uint32_t)ids[r][i] << held;
+        acc |= (uint64_t)(ids[r][i] == fill ? none : (uint32_t)ids[r][i] - base) << held;
         held += bits;
         while (held >= 8) {
           *dst++ = (uint8_t)acc;
@@ -467,19 +508,29 @@ __global__ __launch_bounds__(kPackThreads) void pack_results(const int32_t* __re
         }
       }
     }
-    const uint32_t words = (total * bits + 15u) / 16u;
+    const uint32_t words = overflow ? 0u : (total * bits + 15u) / 16u;
     if (kStaged && threadIdx.x == 0) s_at = atomicAdd(out.cursor, words);
     __syncthreads();
-    const size_t at = kStaged ? (size_t)s_at * 16u : (size_t)chunk * kPackChunkGroups * bits;
-    uint8_t* chunk_out = out.bytes + at;
-    for (uint32_t i = threadIdx.x; i < words; i += kPackThreads)
-      reinterpret_cast<uint4*>(chunk_out)[i] = reinterpret_cast<const uint4*>(s_packed)[i];
-    if (threadIdx.x < kPackChunkGroups / 64) out.headers[chunk].live[threadIdx.x] = s_live[threadIdx.x];
-    if (threadIdx.x == kPackChunkGroups / 64) {
-      out.headers[chunk].overflow = (uint64_t)any_overflow;
-      if (kStaged) out.headers[chunk].at = at;
+    const uint32_t place = kStaged ? chunk : (out.first + chunk) & out.ring_mask;
+    const size_t at = kStaged ? (size_t)s_at * 16u : (size_t)place * kPackChunkGroups * most_bits;
+    uint4* chunk_out = reinterpret_cast<uint4*>(out.bytes + at);
+    PackHeader* header = out.headers + place;
+    for (uint32_t i = threadIdx.x; i < words; i += kPackThreads) {
+      const uint4 v = reinterpret_cast<const uint4*>(s_packed)[i];
+      if (kStaged) chunk_out[i] = v;
+      else store_past_caches(chunk_out + i, v);
     }
-    __syncthreads();  // the next chunk overwrites what has just been read
+    constexpr uint32_t kLiveWords = kPackChunkGroups / 64;
+    if (threadIdx.x < kLiveWords + 3) {
+      const uint64_t v = threadIdx.x < kLiveWords ? s_live[threadIdx.x % kLiveWords] : threadIdx.x == kLiveWords ? (uint64_t)overflow
+                         : threadIdx.x == kLiveWords + 1 ? (uint64_t)at : (uint64_t)bits | (uint64_t)base << 32;
+      uint64_t* to = reinterpret_cast<uint64_t*>(header) + threadIdx.x;
+      if (kStaged) *to = v;
+      else __hip_atomic_store(to, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    if (!kStaged) asm volatile("s_waitcnt vmcnt(0)" : : : "memory");  // this wavefront's part of the chunk is in host memory
+    __syncthreads();  // ... and the others'; the next chunk overwrites what has just been read
+    if (!kStaged && threadIdx.x == 0) __hip_atomic_store(&header->stamp, out.stamp + chunk, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
   if (kStaged && threadIdx.x == 0 && atomicAdd(out.finished, 1u) == gridDim.x - 1) {
     // the last workgroup: the others' claims were answered before they counted themselves
@@ -510,14 +561,23 @@ struct UnpackPlan {
       shift[i] = (int32_t)(bit & 7u);
     }
   }
+  static const UnpackPlan& of(uint32_t bits) {
+    static const std::vector<UnpackPlan> plans = [] {
+      std::vector<UnpackPlan> made;
+      for (uint32_t b = 0; b <= kPackMostBits + 1; ++b) made.emplace_back(b <= kPackMostBits ? b : 32u);
+      return made;
+    }();
+    return plans[std::min(bits, kPackMostBits + 1)];
+  }
 };
 
 // Bytes the unpacking may read past the last group of a chunk.
 constexpr size_t kUnpackOverread = 32;
 
 // One chunk to dst (kPackChunk ids).
-inline void unpack_chunk_plain(const UnpackPlan& plan, const PackHeader& header, const uint8_t* src, int32_t fill,
-                               int32_t* dst) {
+inline void unpack_chunk_plain(const PackHeader& header, const uint8_t* src, int32_t fill, int32_t* dst) {
+  const UnpackPlan& plan = UnpackPlan::of(header.bits);
+  const bool whole = plan.bits > kPackMostBits;
   for (uint32_t g = 0; g < kPackChunkGroups; ++g, dst += kPackGroup) {
     if (!(header.live[g / 64] >> (g % 64) & 1u)) {
       std::fill_n(dst, kPackGroup, fill);
@@ -525,28 +585,38 @@ inline void unpack_chunk_plain(const UnpackPlan& plan, const PackHeader& header,
     }
     for (uint32_t i = 0; i < kPackGroup; ++i) {
       uint64_t word = 0;
-      memcpy(&word, src + ((i * plan.bits) >> 3), plan.bits > kPackMostBits ? sizeof(uint32_t) : sizeof(word));
-      dst[i] = (int32_t)((uint32_t)(word >> ((i * plan.bits) & 7u)) & plan.mask);
+      memcpy(&word, src + ((i * plan.bits) >> 3), whole ? sizeof(uint32_t) : sizeof(word));
+      const uint32_t code = (uint32_t)(word >> ((i * plan.bits) & 7u)) & plan.mask;
+      dst[i] = whole ? (int32_t)code : code == plan.mask ? fill : (int32_t)(code + header.base);
     }
     src += plan.bits;
   }
 }
 
 #if defined(__x86_64__) && !defined(__HIP_DEVICE_COMPILE__)
-// The same with dst a multiple of 32 bytes.  Streaming stores: the result is written once and read by nobody here, and
+// The same.  kStreaming (dst a multiple of 32 bytes), for results larger than the caches: the result is written once and read by nobody here, and
 // a line that is not fetched before it is overwritten is half the memory traffic.  Words of 64 live groups, and of 64
 // dead ones, have loops of their own; in a mixed word every group is unpacked from where the next live one
 // starts and replaced by `fill` if it is not live itself - no branch to mispredict where walks end at random.
 // Eight threads: 200 GB/s of ids (76-100 with a call for every run of groups of one kind).
-__attribute__((target("avx2"))) inline void unpack_chunk_avx2(const UnpackPlan& plan, const PackHeader& header,
-                                                              const uint8_t* src, int32_t fill, int32_t* dst) {
+template <bool kStreaming>
+__attribute__((target("avx2"))) inline void unpack_chunk_avx2(const PackHeader& header, const uint8_t* src, int32_t fill,
+                                                              int32_t* dst) {
+  const UnpackPlan& plan = UnpackPlan::of(header.bits);
   const bool whole = plan.bits > kPackMostBits;
   const size_t bits = plan.bits;
   const __m256i shuffle = _mm256_loadu_si256((const __m256i*)plan.shuffle);
   const __m256i shift = _mm256_loadu_si256((const __m256i*)plan.shift);
   const __m256i mask = _mm256_set1_epi32((int)plan.mask), dead = _mm256_set1_epi32(fill);
+  const __m256i base = _mm256_set1_epi32((int)header.base);
   const size_t high_at = plan.high_at;
-#define ND_UNPACKED_GROUP                                                                                          \
+#define ND_STORE_GROUP(group)                                        \
+  do {                                                               \
+    const __m256i stored = (group);                                  \
+    if (kStreaming) _mm256_stream_si256((__m256i*)dst, stored);      \
+    else _mm256_storeu_si256((__m256i*)dst, stored);                 \
+  } while (0)
+#define ND_UNPACKED_CODES                                                                                          \
   _mm256_and_si256(                                                                                                \
       _mm256_srlv_epi32(_mm256_shuffle_epi8(_mm256_inserti128_si256(                                               \
                                                 _mm256_castsi128_si256(_mm_loadu_si128((const __m128i*)src)),      \
@@ -557,43 +627,48 @@ __attribute__((target("avx2"))) inline void unpack_chunk_avx2(const UnpackPlan& 
   for (uint32_t w = 0; w < kPackChunkGroups / 64; ++w) {
     uint64_t live = header.live[w];
     if (live == 0) {
-      for (uint32_t g = 0; g < 64; ++g, dst += kPackGroup) _mm256_stream_si256((__m256i*)dst, dead);
+      for (uint32_t g = 0; g < 64; ++g, dst += kPackGroup) ND_STORE_GROUP(dead);
     } else if (whole) {
       for (uint32_t g = 0; g < 64; ++g, dst += kPackGroup, live >>= 1) {
         const __m256i here = _mm256_set1_epi32(-(int)(live & 1u));
-        _mm256_stream_si256((__m256i*)dst, _mm256_blendv_epi8(dead, _mm256_loadu_si256((const __m256i*)src), here));
+        ND_STORE_GROUP(_mm256_blendv_epi8(dead, _mm256_loadu_si256((const __m256i*)src), here));
         src += bits & (0 - (size_t)(live & 1u));
       }
     } else if (~live == 0) {
-      for (uint32_t g = 0; g < 64; ++g, dst += kPackGroup, src += bits)
-        _mm256_stream_si256((__m256i*)dst, ND_UNPACKED_GROUP);
+      for (uint32_t g = 0; g < 64; ++g, dst += kPackGroup, src += bits) {
+        const __m256i codes = ND_UNPACKED_CODES;
+        ND_STORE_GROUP(_mm256_blendv_epi8(_mm256_add_epi32(codes, base), dead, _mm256_cmpeq_epi32(codes, mask)));
+      }
     } else {
       for (uint32_t g = 0; g < 64; ++g, dst += kPackGroup, live >>= 1) {
-        const __m256i here = _mm256_set1_epi32(-(int)(live & 1u));
-        _mm256_stream_si256((__m256i*)dst, _mm256_blendv_epi8(dead, ND_UNPACKED_GROUP, here));
+        const __m256i codes = ND_UNPACKED_CODES, gone = _mm256_set1_epi32((int)(live & 1u) - 1);
+        ND_STORE_GROUP(_mm256_blendv_epi8(_mm256_add_epi32(codes, base), dead,
+                                          _mm256_or_si256(gone, _mm256_cmpeq_epi32(codes, mask))));
         src += bits & (0 - (size_t)(live & 1u));
       }
     }
   }
-#undef ND_UNPACKED_GROUP
+#undef ND_UNPACKED_CODES
+#undef ND_STORE_GROUP
 }
 inline bool unpack_has_avx2() { return __builtin_cpu_supports("avx2"); }
 inline void unpack_fence() { _mm_sfence(); }
 inline void spin_pause() { _mm_pause(); }
 #else
-inline void unpack_chunk_avx2(const UnpackPlan&, const PackHeader&, const uint8_t*, int32_t, int32_t*) {}
+template <bool kStreaming>
+inline void unpack_chunk_avx2(const PackHeader&, const uint8_t*, int32_t, int32_t*) {}
 inline bool unpack_has_avx2() { return false; }
 inline void unpack_fence() {}
 inline void spin_pause() {}
 #endif
 
-// The first count ids (at most kPackChunk) of a chunk to dst.
-inline void unpack_chunk(const UnpackPlan& plan, const PackHeader& header, const uint8_t* src, int32_t fill,
-                         int32_t* dst, size_t count) {
+// The first count ids (at most kPackChunk) of a chunk to dst; streaming: past the caches.
+inline void unpack_chunk(const PackHeader& header, const uint8_t* src, int32_t fill, int32_t* dst, size_t count, bool streaming) {
   alignas(32) int32_t part[kPackChunk];
   int32_t* at = count == kPackChunk ? dst : part;
-  if (((uintptr_t)at & 31u) == 0 && unpack_has_avx2()) unpack_chunk_avx2(plan, header, src, fill, at);
-  else unpack_chunk_plain(plan, header, src, fill, at);
+  if (!unpack_has_avx2()) unpack_chunk_plain(header, src, fill, at);
+  else if (streaming && at != part && ((uintptr_t)at & 31u) == 0) unpack_chunk_avx2<true>(header, src, fill, at);
+  else unpack_chunk_avx2<false>(header, src, fill, at);
   if (at == part) memcpy(dst, part, count * sizeof(int32_t));
 }
 
@@ -621,9 +696,10 @@ inline hipError_t device_of(hipStream_t stream, int* device) {
   return stream ? hipStreamGetDevice(stream, device) : hipGetDevice(device);
 }
 
-// The streams results cross the bus on while something else is computed: two or three per device (which has to be the current one) and process, each on
+// The streams results cross the bus on while something else is computed: two per device (which has to be the current one) and process, each on
 // a hardware queue of its own, which a stream with a mask of compute units (here: all) gets.  (Ordinary streams share
-// four; where the computation's lands on the same one, nothing overlaps.)  What each is for: StreamUse.  They are destroyed when the process ends, while
+// four; where the computation's lands on the same one, nothing overlaps.)  All the samplers of the process share them, so nothing on
+// them ever waits for a computation: what others put there would wait as well.  They are destroyed when the process ends, while
 // the runtime and whatever watches it are still there: left to the runtime, their queues outlive a profiler's
 // bookkeeping of them, and a profiled process ended in a segmentation fault.
 inline std::vector<hipStream_t>& transfer_streams() {
@@ -638,7 +714,7 @@ inline std::vector<hipStream_t>& transfer_streams() {
   }();
   return *streams;
 }
-constexpr size_t kTransferStreams = 3;  // of a device, at most
+constexpr size_t kTransferStreams = 2;  // of a device
 inline hipStream_t transfer_stream(int device, size_t which) {
   static std::mutex mutex;
   std::vector<hipStream_t>* streams = &transfer_streams();
@@ -661,52 +737,6 @@ inline hipStream_t transfer_stream(int device, size_t which) {
 
 // ---- the stream ----------------------------------------------------------------------------
 
-// What a transfer may use besides the first of its device's streams, on which nothing ever waits for a computation: all the
-// samplers of the process share it, and what others put there would wait as well.  The second is either one transfer's that
-// has it wait for its computation, or packs pieces for any number that do not; who wants to pack while somebody waits
-// there does so on a third.  (Not a stream for each from the start: uniform walks 57 K, whose rows wait for them, 0.35 ms, 0.40
-// on the third such stream of a process.)
-class StreamUse {
- public:
-  StreamUse() = default;
-  StreamUse(const StreamUse&) = delete;
-  StreamUse& operator=(const StreamUse&) = delete;
-  ~StreamUse() { give_back(); }
-
-  // the second one, for waiting: false if it is in use
-  bool wait(int device) {
-    give_back();
-    int nobody = 0;
-    if ((unsigned)device >= kDevices || !users(device).compare_exchange_strong(nobody, -1)) return false;
-    device_ = device, held_ = -1;
-    return true;
-  }
-  // the one to pack on
-  size_t pack(int device) {
-    give_back();
-    if ((unsigned)device >= kDevices) return 1;  // nobody waits there
-    for (int now = users(device).load();;) {
-      if (now < 0) return 2;
-      if (users(device).compare_exchange_weak(now, now + 1)) break;
-    }
-    device_ = device, held_ = 1;
-    return 1;
-  }
-  // nothing of the transfer is on it any more
-  void give_back() {
-    if (held_ != 0) users(device_).fetch_sub(held_);
-    held_ = 0;
-  }
-
- private:
-  static constexpr unsigned kDevices = 64;
-  static std::atomic<int>& users(int device) {  // of the second stream; -1: one that waits
-    static std::atomic<int> all[kDevices] = {};
-    return all[device];
-  }
-  int device_ = 0, held_ = 0;
-};
-
 // Brings words of device memory to the host, packed on the way.  One caller at a time.  Everything happens on the device of the
 // stream that is given, whatever the calling thread's current device is, and leaves that as it was.
 class ResultStream {
@@ -726,23 +756,20 @@ class ResultStream {
     uint32_t value = 0;
   };
 
-  // Takes, on the current device and ahead of the first, what a copy() or a fetch() of n words needs.
+  // Takes, on the current device and ahead of the first, what a fetch() of n words needs.
   hipError_t reserve(size_t n, uint32_t bits) {
     hipError_t e = finish();
     if (e == hipSuccess) e = come_to_device_of(nullptr);
-    if (e != hipSuccess) return e;
-    if (n * sizeof(int32_t) <= kDirectResultBytes) {
-      e = make_ring(kDirectResultBytes);
-    } else {
-      if (!transfer_) transfer_.reset(new Transfer);
-      transfer_->set(nullptr, n, bits > kPackMostBits ? 32 : bits, 0, nullptr, {});
-      e = prepare(transfer_->slot_bytes);
-    }
-    if (e == hipSuccess) memset(ring_, 0, ring_bytes_);  // its pages are mapped when they are first touched: 0.8 ms of 2 MB
+    if (e != hipSuccess || n == 0) return e;
+    if (!transfer_) transfer_.reset(new Transfer);
+    transfer_->set(nullptr, n, bits > kPackMostBits ? 32 : bits, 0, nullptr, {});
+    e = prepare(*transfer_);
+    // its pages are mapped when they are first touched: 0.8 ms of 2 MB
+    if (e == hipSuccess) memset(ring_, 0, transfer_->chunk_bytes * transfer_->ring_chunks);
     return e;
   }
 
-  // bytes at src to dst as they are, in stream order, complete on return.  For few of them, and for what is not words.
+  // bytes at src to dst as they are, in stream order, complete on return.  For what is not words.
   hipError_t copy(const void* src, size_t bytes, void* dst, hipStream_t stream) {
     hipError_t e = finish();  // an earlier one that nobody waited for
     if (e == hipSuccess) e = come_to_device_of(stream);
@@ -760,7 +787,7 @@ class ResultStream {
 
   // n words at src (aligned to 16 bytes) to dst, in stream order.  Words that are `fill` in groups of eight cost
   // nothing; words are expected to fit `bits` bits (one that does not makes the whole transfer start again with
-  // 32).  Large transfers only: it pays from a few megabytes on.
+  // 32).
   hipError_t fetch(const int32_t* src, size_t n, uint32_t bits, int32_t fill, int32_t* dst, hipStream_t stream) {
     const hipError_t e = begin(src, n, bits, fill, dst, stream, {});
     return e == hipSuccess ? finish() : e;
@@ -768,11 +795,12 @@ class ResultStream {
 
   // The same as a begin() that returns at once, other threads taking it from there, and a finish() that takes part
   // and returns when the words are at dst.  `ready` (words ascending, the last n): what has to have
-  // happened before words may be read, while other work of the caller's is still going on; empty: stream order.  What is given has to stay until finish().
+  // happened before words may be read, while other work of the caller's is still going on; empty: stream order, and `computed`, if there is
+  // one, an event recorded on the stream before, that the threads need not look for words until it has happened.  What is given has
+  // to stay until finish().
   hipError_t begin(const int32_t* src, size_t n, uint32_t bits, int32_t fill, int32_t* dst, hipStream_t stream,
-                   std::vector<Ready> ready) {
+                   std::vector<Ready> ready, hipEvent_t computed = nullptr) {
     hipError_t e = finish();  // an earlier one that nobody waited for
-    use_.give_back();
     if (e != hipSuccess || n == 0) return e;
     if (!transfer_) transfer_.reset(new Transfer);
     Transfer& t = *transfer_;
@@ -782,25 +810,36 @@ class ResultStream {
     const OnDevice on(t.device);
     if (on.error != hipSuccess) return on.error;
     t.set(src, n, bits > kPackMostBits ? 32 : bits, fill, dst, std::move(ready));
-    e = prepare(t.slot_bytes);
+    e = prepare(t);
     if (e == hipSuccess && t.staged) e = prepare_staging(t.slot_bytes);
     if (e != hipSuccess) return e;
+    t.number = ++transfers_;
     t.streams[0] = t.streams[1] = transfer_stream(t.device, 0);
-    // all words at once: the device waits for them, without a way over a thread, if it can
-    t.device_waits = t.ready.size() == 1 && !t.staged && use_.wait(t.device);
-    if (t.device_waits) t.streams[0] = t.streams[1] = transfer_stream(t.device, 1);
-    if (t.staged) t.streams[0] = transfer_stream(t.device, use_.pack(t.device));
-    if (t.ready.empty()) {
-      // pieces alternate between two streams, so that the bus is not idle between two of them
-      t.streams[0] = stream;
-      e = hipEventRecord(begun_, stream);
-      if (e == hipSuccess) e = hipStreamWaitEvent(t.streams[1], begun_, 0);
-      if (e != hipSuccess) return e;
-    }
+    if (t.staged || !t.ready.empty()) t.streams[t.staged ? 0 : 1] = transfer_stream(t.device, 1);
     if (!t.ready.empty()) ahead_.store(0, std::memory_order_relaxed);
+    size_t helpers = HostWorkers::kMost;
+    if (t.ready.empty()) {
+      t.streams[0] = stream;
+      t.computed_event = computed;
+      if (t.chunks <= t.ring_chunks) t.streams[1] = stream;
+      // two streams, so that the bus is not idle between two launches
+      if (t.chunks > t.ring_chunks) {
+        e = hipEventRecord(begun_, stream);
+        if (e == hipSuccess) e = hipStreamWaitEvent(t.streams[1], begun_, 0);
+      }
+      if (e == hipSuccess) e = launch(std::min(t.chunks, t.ring_chunks), bus_blocks());
+      if (e != hipSuccess) return e;
+      // few chunks are unpacked before a thread is awake, unless it is woken while they are computed
+      if (t.chunks <= kFewChunks) helpers = computed ? t.chunks / kChunksAHelper : 0;
+      if (!computed) t.announce(t.sent, false);
+    }
     job_.body = [this] { take_part(); };
-    HostWorkers::get().start(job_, HostWorkers::kMost);
-    under_way_ = true;  // (not if start() throws: nobody has begun on it then)
+    under_way_ = true;
+    helped_ = false;
+    try {
+      if (helpers) HostWorkers::get().start(job_, (unsigned)helpers), helped_ = true;
+    } catch (const std::bad_alloc&) {  // nobody has begun on it: finish() does all of it
+    }
     return hipSuccess;
   }
 
@@ -808,14 +847,13 @@ class ResultStream {
     if (!under_way_) return hipSuccess;
     Transfer& t = *transfer_;
     take_part();
-    HostWorkers::get().join(job_);
+    if (helped_) HostWorkers::get().join(job_);
     under_way_ = false;
     if (t.error != hipSuccess) {
       const OnDevice on(t.device);
       for (hipStream_t s : t.streams) (void)hipStreamSynchronize(s);  // nothing writes to the ring after this
+      return t.error;
     }
-    use_.give_back();
-    if (t.error != hipSuccess) return t.error;
     if (!t.overflow.load()) return hipSuccess;
     misfit_ = true;
     const OnDevice on(t.device);  // the stream may be the default one
@@ -824,12 +862,12 @@ class ResultStream {
 
   // whether a word has ever not fitted
   bool misfit() const { return misfit_; }
-  // pieces of the last begin() that was given a `ready` which set out before all of that had happened
+  // launches of the last begin() that was given a `ready` which set out before all of that had happened
   size_t parts_ahead() const { return ahead_.load(std::memory_order_relaxed); }
   // of what it owns through a pointer (nd::engine_abi)
   static constexpr size_t transfer_bytes() { return sizeof(Transfer); }
   // page-locked memory it holds until release()
-  size_t page_locked_bytes() const { return ring_bytes_; }
+  size_t page_locked_bytes() const { return ring_bytes_ + headers_held_ * sizeof(PackHeader); }
 
   void release() {
     (void)finish();
@@ -846,18 +884,34 @@ class ResultStream {
     if (ring_) (void)hipHostFree(ring_);
     ring_ = nullptr;
     ring_bytes_ = 0;
+    if (headers_) (void)hipHostFree(headers_);
+    headers_ = nullptr;
+    headers_held_ = 0;
   }
 
-  static constexpr size_t kSlots = 8;
-  // Chunks of a piece: at most 8 MB of results (0.1 ms on the bus, long against a launch and an event; with pieces of
-  // 16 MB the ring no longer stays in the last-level cache between the bus and the threads: 1.68 GB in 16 instead of 14
-  // ms; the copy engine, which rests 8 us between two copies, gets 16 MB all the same).  The first one is 1 MB and each of the next twice as long, so that the threads have something to do soon, and
-  // none is more than a third of what is left, so that little is left to do when the last one arrives.
-  static constexpr size_t kMostChunks = 512, kMostStagedChunks = 1024, kLeastChunks = 64;
-  static constexpr size_t kChunksAtOnce = 4;  // what a thread takes; kLeastChunks is a multiple
+  // Straight to the host: a ring of as many chunks as there are, or of kRingChunks (64 MB of ids; with twice that the ring no longer stays in the
+  // last-level cache between the bus and the threads: 1.68 GB in 16 instead of 14 ms), into which launches of up to
+  // kMostChunks go as the threads make room.
+  static constexpr size_t kRingChunks = 4096, kMostChunks = 512;
+  // Packed in device memory first: pieces in slots; the copy engine rests 8 us between two.  The first one is 1 MB and each of the
+  // next twice as long, so that the threads have something to do soon, and none is more than a third of what is left, so that
+  // little is left to do when the last one arrives.
+  static constexpr size_t kSlots = 8, kMostStagedChunks = 1024;
+  static constexpr size_t kBlock = 64;          // chunks that are counted, as they are unpacked, together
+  static constexpr size_t kChunksAtOnce = 4;    // what a thread takes; kBlock is a multiple
+  static constexpr size_t kFewChunks = kDirectResultBytes / (kPackChunk * sizeof(int32_t)), kChunksAHelper = 32;
   // Workgroups of a launch of pack_results that goes straight to the ring, and launches under way, while something else is
   // computed: stores that wait for the bus stand in the way of that something's own.
   static constexpr uint32_t kGentleBlocks = 32;
+  // ... and of one that has the device to itself: enough to keep the bus busy, and no more, so that chunks arrive in about the order the
+  // threads look for them in, and not all of them at the end; for more chunks than the ring holds that matters less, and the
+  // gaps between launches more.  Passes with their rows by workgroups, ms (a workgroup a chunk: walks 0.47, distinct 1.11):
+  //                                     32     64     96    128    256
+  //     uniform walks 57 K           0.348  0.302  0.341  0.344  0.369
+  //     KHop 60 K, distinct          0.974  0.832  0.897  0.926  0.990
+  //     MVS 150 K                    2.24   2.20   2.22   2.20   2.27
+  //     KHop R-MAT 20 (19 rings)    11.00  10.87  10.55  10.53  10.63
+  static constexpr uint32_t kBusBlocks = 64, kBusBlocksOfMany = 128;
   static constexpr size_t kGentleAhead = 2;
   static constexpr size_t kPackedAhead = 3;     // pieces packed before the copy engine has come to them
   static constexpr int kSignsPerQuery = 1024;   // looks at a sign for one at the event beside it: some 20 us
@@ -882,7 +936,21 @@ class ResultStream {
     return e;
   }
 
-  hipError_t prepare(size_t slot_bytes) {
+  // Headers have memory of their own: nothing but a stamp is ever where a stamp is looked for.
+  hipError_t make_headers(size_t chunks) {
+    if (headers_held_ >= chunks) return hipSuccess;
+    if (headers_) (void)hipHostFree(headers_);
+    headers_ = nullptr;
+    headers_held_ = 0;
+    const hipError_t e = hipHostMalloc((void**)&headers_, chunks * sizeof(PackHeader), hipHostMallocDefault);
+    if (e != hipSuccess) return e;
+    memset((void*)headers_, 0, chunks * sizeof(PackHeader));  // the number of no transfer
+    headers_held_ = chunks;
+    return hipSuccess;
+  }
+
+  struct Transfer;
+  hipError_t prepare(const Transfer& t) {
     for (hipEvent_t& ev : packed_)
       if (!ev) {
         const hipError_t e = hipEventCreateWithFlags(&ev, hipEventDisableTiming | hipEventReleaseToSystem);
@@ -892,7 +960,13 @@ class ResultStream {
       const hipError_t e = hipEventCreateWithFlags(&begun_, hipEventDisableTiming);
       if (e != hipSuccess) return e;
     }
-    return make_ring(slot_bytes * kSlots);
+    if (t.staged) return make_ring(t.slot_bytes * kSlots);
+    // Room for a few chunks more, or for more bits, so that a sampler's other results do not need another ring: to touch one for the
+    // first time takes 0.4 ms a MB (MultiRW, rows of 2,442 chunks and states of 2,466: a first pass of 9.5 ms instead of 3.5).
+    size_t held = 16;
+    while (held < t.ring_chunks) held *= 2;
+    const hipError_t e = make_headers(held);
+    return e != hipSuccess ? e : make_ring((size_t)kPackChunkGroups * std::max(t.bits, kPackMostBits) * held + kUnpackOverread);
   }
 
   // What pieces that are packed in device memory take.
@@ -941,91 +1015,120 @@ class ResultStream {
     int32_t* dst;
     hipStream_t streams[2];
     std::vector<Ready> ready;
+    hipEvent_t computed_event = nullptr;
     bool staged = false;  // pieces are packed in device memory, for the copy engine, while something else is computed
-    bool device_waits = false;
     int device = 0;
 
-    size_t chunks, pieces, chunk_bytes, packed_at, slot_bytes;
-    std::vector<size_t> begins;        // first chunk of every piece, and the end of the last
-    std::vector<uint32_t> piece_of;    // of every kLeastChunks chunks
+    size_t chunks, chunk_bytes;
     size_t happened;                   // of `ready`
     bool computed;                     // all of it
-    UnpackPlan plan{32};
+    // straight
+    size_t ring_chunks = 0;
+    uint64_t number = 0;
+    size_t sent = 0, launches = 0;     // chunks, and what they were sent with
+    size_t unpacked_to = 0;            // blocks
+    // staged
+    size_t pieces = 0, packed_at = 0, slot_bytes = 0;
+    std::vector<size_t> begins;        // first chunk of every piece, and the end of the last
+    std::vector<uint32_t> piece_of;    // of every block
+
     std::atomic<bool> driven{false};   // a thread has taken the launching on
     std::atomic<size_t> next{0};       // chunk to take
-    std::atomic<size_t> arrived{0};    // pieces whose bytes are here
+    std::atomic<size_t> there{0};      // chunks that have been sent (straight), or whose bytes are here (staged)
     std::atomic<bool> stop{false}, overflow{false};
-    hipError_t error = hipSuccess;     // the driving thread's
+    hipError_t error = hipSuccess;     // the first one
     std::mutex mutex;
     std::condition_variable more;
     unsigned sleepers = 0;
-    std::vector<std::atomic<size_t>> left;  // chunks of a piece that are not unpacked yet
+    std::vector<std::atomic<size_t>> left;  // chunks of a block that are not unpacked yet
 
     void set(const int32_t* src_, size_t n_, uint32_t bits_, int32_t fill_, int32_t* dst_, std::vector<Ready> ready_) {
       src = src_, n = n_, bits = bits_, fill = fill_, dst = dst_, ready = std::move(ready_);
       staged = !ready.empty() && ready.front().sign != nullptr;
+      computed_event = nullptr;
       happened = 0;
       computed = false;
       chunks = (n + kPackChunk - 1) / kPackChunk;
+      chunk_bytes = (size_t)kPackChunkGroups * bits;
+      ring_chunks = std::min(chunks, kRingChunks);
+      sent = launches = unpacked_to = 0;
       begins.clear();
       piece_of.clear();
-      size_t most = kLeastChunks, longest = 0;
-      for (size_t at = 0; at < chunks; most = std::min(staged ? kMostStagedChunks : kMostChunks, most * 2)) {
-        const size_t third = ((chunks - at) / 3 + kLeastChunks - 1) / kLeastChunks * kLeastChunks;
-        const size_t here = std::max(kLeastChunks, std::min(most, third));
-        piece_of.insert(piece_of.end(), here / kLeastChunks, (uint32_t)begins.size());
-        begins.push_back(at);
-        longest = std::max(longest, here);
-        at += here;
+      if (staged) {
+        size_t most = kBlock, longest = 0;
+        for (size_t at = 0; at < chunks; most = std::min(kMostStagedChunks, most * 2)) {
+          const size_t third = ((chunks - at) / 3 + kBlock - 1) / kBlock * kBlock;
+          const size_t here = std::max(kBlock, std::min(most, third));
+          piece_of.insert(piece_of.end(), here / kBlock, (uint32_t)begins.size());
+          begins.push_back(at);
+          longest = std::max(longest, here);
+          at += here;
+        }
+        pieces = begins.size();
+        begins.push_back(chunks);
+        packed_at = sizeof(PackHeader) * longest;
+        slot_bytes = (packed_at + chunk_bytes * longest + kUnpackOverread + 255) / 256 * 256;
       }
-      pieces = begins.size();
-      begins.push_back(chunks);
-      chunk_bytes = (size_t)kPackChunkGroups * bits;
-      packed_at = sizeof(PackHeader) * longest;
-      slot_bytes = (packed_at + chunk_bytes * longest + kUnpackOverread + 255) / 256 * 256;
-      plan = UnpackPlan(bits);
-      driven = false, next = 0, arrived = 0, stop = false, overflow = false, error = hipSuccess;
-      left = std::vector<std::atomic<size_t>>(pieces);
-      for (size_t p = 0; p < pieces; ++p) left[p].store(begins[p + 1] - begins[p]);
+      driven = false, next = 0, there = 0, stop = false, overflow = false, error = hipSuccess;
+      const size_t blocks = (chunks + kBlock - 1) / kBlock;
+      left = std::vector<std::atomic<size_t>>(blocks);
+      for (size_t b = 0; b < blocks; ++b) left[b].store(std::min(kBlock, chunks - b * kBlock));
     }
 
-    // A piece comes every 20-200 us: worth a short wait awake (a thread that sleeps is back 50 us later, and
+    // (no other chunk's that was or will be where this one is)
+    uint64_t stamp(size_t chunk) const { return (number << 32) + chunk; }
+
+    // Words come every 20-200 us: worth a short wait awake (a thread that sleeps is back 50 us later, and
     // waking all of them costs the driving thread as much), but not more than that.
-    void await(size_t piece) {
+    void await(size_t chunk) {
       for (int spin = 0; spin < kSpins; ++spin) {
-        if (arrived.load(std::memory_order_acquire) > piece || stop.load()) return;
+        if (there.load(std::memory_order_acquire) > chunk || stop.load()) return;
         spin_pause();
       }
       std::unique_lock<std::mutex> lock(mutex);
       sleepers++;
-      more.wait(lock, [&] { return arrived.load(std::memory_order_acquire) > piece || stop.load(); });
+      more.wait(lock, [&] { return there.load(std::memory_order_acquire) > chunk || stop.load(); });
       sleepers--;
     }
-    void announce(size_t pieces_here, bool stops) {
+    void announce(size_t chunks_there, bool stops) {
       bool asleep;
       {
         std::lock_guard<std::mutex> lock(mutex);
         if (stops) stop.store(true);
-        else arrived.store(pieces_here, std::memory_order_release);
+        else there.store(chunks_there, std::memory_order_release);
         asleep = sleepers > 0;
       }
       if (asleep) more.notify_all();
     }
+    void fail(hipError_t e) {
+      {
+        std::lock_guard<std::mutex> lock(mutex);
+        if (error == hipSuccess) error = e;
+      }
+      (void)hipGetLastError();  // reported by finish(), not to this thread's next launch
+      announce(0, true);
+    }
   };
 
   uint8_t* slot(size_t piece) const { return ring_ + (piece % kSlots) * transfer_->slot_bytes; }
-  size_t piece_end(size_t piece) const {
-    return std::min(transfer_->n, transfer_->begins[piece + 1] * kPackChunk);
+  size_t words_to(size_t chunk) const { return std::min(transfer_->n, chunk * kPackChunk); }
+
+  // (hipEventSynchronize() keeps whoever uses the event's stream otherwise, another transfer's begin() for one, until it has happened.)
+  static hipError_t wait_for(hipEvent_t event) {
+    hipError_t e;
+    while ((e = hipEventQuery(event)) == hipErrorNotReady)
+      for (int pause = 0; pause < 32; ++pause) spin_pause();
+    return e;
   }
 
-  // Whether piece may be read, or, with `waits`, until it may.
-  bool readable(size_t piece, bool waits, hipError_t* error) {
+  // Whether words may be read, or, with `waits`, until they may.
+  bool readable(size_t words, bool waits, hipError_t* error) {
     Transfer& t = *transfer_;
-    while (t.happened < t.ready.size() && (t.happened == 0 || t.ready[t.happened - 1].words < piece_end(piece))) {
+    while (t.happened < t.ready.size() && (t.happened == 0 || t.ready[t.happened - 1].words < words)) {
       const Ready& next = t.ready[t.happened];
       hipError_t e = hipErrorNotReady;
       if (!next.sign) {
-        e = waits ? hipEventSynchronize(next.event) : hipEventQuery(next.event);
+        e = waits ? wait_for(next.event) : hipEventQuery(next.event);
       } else {
         for (;;) {
           if (__atomic_load_n(next.sign, __ATOMIC_ACQUIRE) == next.value) e = hipSuccess;
@@ -1051,24 +1154,39 @@ class ResultStream {
     return t.computed;
   }
 
-  hipError_t launch(size_t piece, uint32_t most_blocks = UINT32_MAX) {
+  uint32_t bus_blocks() const { return transfer_->chunks > transfer_->ring_chunks ? kBusBlocksOfMany : kBusBlocks; }
+
+  // Straight: the chunks from t.sent on, up to `end`.
+  hipError_t launch(size_t end, uint32_t most_blocks) {
+    Transfer& t = *transfer_;
+    const size_t first = t.sent * kPackChunk, here = words_to(end) - first;
+    const uint32_t n_chunks = (uint32_t)(end - t.sent);
+    PackedOut out{ring_, headers_};
+    out.first = (uint32_t)(t.sent % t.ring_chunks);
+    out.ring_mask = t.chunks > t.ring_chunks ? (uint32_t)t.ring_chunks - 1u : UINT32_MAX;
+    static_assert((kRingChunks & (kRingChunks - 1)) == 0, "a ring that is gone round");
+    out.stamp = t.stamp(t.sent);
+    pack_results<false><<<dim3(std::min(n_chunks, most_blocks)), dim3(kPackThreads), 0, t.streams[t.launches % 2]>>>(
+        t.src + first, here, t.bits, t.fill, out, n_chunks);
+    t.launches++;
+    t.sent = end;
+    return hipGetLastError();
+  }
+
+  // Staged: a piece.
+  hipError_t launch_piece(size_t piece) {
     const Transfer& t = *transfer_;
     const size_t first = t.begins[piece] * kPackChunk;
-    const size_t here = piece_end(piece) - first, slot_of = piece % kSlots;
-    uint8_t* at = t.staged ? staging_ + slot_of * t.slot_bytes : slot(piece);
+    const size_t here = words_to(t.begins[piece + 1]) - first, slot_of = piece % kSlots;
+    uint8_t* at = staging_ + slot_of * t.slot_bytes;
     const uint32_t n_chunks = (uint32_t)((here + kPackChunk - 1) / kPackChunk);
-    const hipStream_t stream = t.streams[t.staged ? 0 : piece % 2];  // (a copy on it would be waited for)
     PackedOut out{at + t.packed_at, (PackHeader*)at};
-    if (t.staged) {
-      out.cursor = counts_ + 2 * slot_of * kWordsPerLine;
-      out.finished = out.cursor + kWordsPerLine;
-      out.total = totals_ + slot_of;
-    }
-    const dim3 grid(std::min(n_chunks, most_blocks)), block(kPackThreads);
-    if (t.staged) pack_results<true><<<grid, block, 0, stream>>>(t.src + first, here, t.bits, t.fill, out, n_chunks);
-    else pack_results<false><<<grid, block, 0, stream>>>(t.src + first, here, t.bits, t.fill, out, n_chunks);
+    out.cursor = counts_ + 2 * slot_of * kWordsPerLine;
+    out.finished = out.cursor + kWordsPerLine;
+    out.total = totals_ + slot_of;
+    pack_results<true><<<dim3(n_chunks), dim3(kPackThreads), 0, t.streams[0]>>>(t.src + first, here, t.bits, t.fill, out, n_chunks);
     const hipError_t e = hipGetLastError();
-    return e != hipSuccess ? e : hipEventRecord(packed_[slot_of], stream);
+    return e != hipSuccess ? e : hipEventRecord(packed_[slot_of], t.streams[0]);
   }
 
   // Sends a piece that is packed in device memory on its way.
@@ -1081,23 +1199,53 @@ class ResultStream {
     return e != hipSuccess ? e : hipEventRecord(copied_[slot_of], stream);
   }
 
-  // unpacks the chunks [c, end) of a piece that is here
+  // Straight: waits for a chunk that has been sent.  False: it does not come, or the transfer has failed otherwise.
+  bool await_stamp(const PackHeader& header, size_t chunk) {
+    Transfer& t = *transfer_;
+    const uint64_t stamp = t.stamp(chunk);
+    for (int spin = 1;; ++spin) {
+      if (__atomic_load_n(&header.stamp, __ATOMIC_ACQUIRE) == stamp) return true;
+      if (t.stop.load(std::memory_order_relaxed)) return false;
+      if (spin < kSpins) {
+        spin_pause();
+        continue;
+      }
+      // long in coming: others are before it on its stream, or the kernel has failed
+      const OnDevice on(t.device);
+      hipError_t e = on.error;
+      for (hipStream_t s : t.streams)
+        if (e == hipSuccess) e = hipStreamQuery(s);
+      if (e == hipSuccess && __atomic_load_n(&header.stamp, __ATOMIC_ACQUIRE) != stamp) e = hipErrorUnknown;
+      if (e != hipSuccess && e != hipErrorNotReady) {
+        t.fail(e);
+        return false;
+      }
+      std::this_thread::sleep_for(std::chrono::microseconds(20));
+    }
+  }
+
+  // Unpacks the chunks [c, end) of a block, which have been sent, or (staged) are here.
   void unpack(size_t c, size_t end) {
     Transfer& t = *transfer_;
-    const size_t piece = t.piece_of[c / kLeastChunks];
-    const uint8_t* at = slot(piece);
-    const PackHeader* headers = (const PackHeader*)at + (c - t.begins[piece]);
+    const size_t piece = t.staged ? t.piece_of[c / kBlock] : 0;
+    const PackHeader* headers = t.staged ? (const PackHeader*)slot(piece) + (c - t.begins[piece]) : headers_ + c % t.ring_chunks;
+    const uint8_t* bytes = t.staged ? slot(piece) + t.packed_at : ring_ + (c % t.ring_chunks) * t.chunk_bytes;
+    const bool streaming = t.n * sizeof(int32_t) > kDirectResultBytes;
     // Where a chunk's bytes are is read for all of them first, and only if it has to be: to wait for a header that has just
     // crossed the bus before every chunk cost 4 % of KHop's rows over R-MAT 20.
     size_t bytes_at[kChunksAtOnce];
-    for (size_t i = 0; i < end - c; ++i) bytes_at[i] = t.staged ? headers[i].at : (c - t.begins[piece] + i) * t.chunk_bytes;
+    for (size_t i = 0; i < end - c; ++i) bytes_at[i] = t.staged ? headers[i].at : i * t.chunk_bytes;
     for (size_t i = 0; i < end - c; ++i) {
-      if (headers[i].overflow) t.overflow.store(true, std::memory_order_relaxed);
+      if (!t.staged && !await_stamp(headers[i], c + i)) return;
+      if (headers[i].overflow) {
+        t.overflow.store(true, std::memory_order_relaxed);
+        continue;
+      }
       const size_t first = (c + i) * kPackChunk;
-      unpack_chunk(t.plan, headers[i], at + t.packed_at + bytes_at[i], t.fill, t.dst + first, std::min<size_t>(kPackChunk, t.n - first));
+      unpack_chunk(headers[i], bytes + bytes_at[i], t.fill, t.dst + first, std::min<size_t>(kPackChunk, t.n - first), streaming);
     }
     unpack_fence();
-    t.left[piece].fetch_sub(end - c, std::memory_order_release);
+    t.left[c / kBlock].fetch_sub(end - c, std::memory_order_release);
   }
 
   void take_part() {
@@ -1106,57 +1254,65 @@ class ResultStream {
     for (;;) {
       const size_t c = t.next.fetch_add(kChunksAtOnce);
       if (c >= t.chunks) return;
-      const size_t piece = t.piece_of[c / kLeastChunks];
-      t.await(piece);
+      const size_t end = std::min(c + kChunksAtOnce, t.chunks);
+      t.await(end - 1);
       if (t.stop.load()) return;
-      unpack(c, std::min(c + kChunksAtOnce, t.chunks));
+      unpack(c, end);
     }
   }
 
-  // Whether a piece's slot is free: the piece before it there is unpacked.  If not, does some of that (of pieces that are here).
-  bool slot_is_free(size_t piece, size_t here) {
+  // The driving thread: some of what is there for it to unpack, if anything is.
+  bool unpack_some() {
     Transfer& t = *transfer_;
-    if (piece < kSlots || t.left[piece - kSlots].load(std::memory_order_acquire) == 0) return true;
     size_t c = t.next.load();
-    if (c < t.begins[here] && t.next.compare_exchange_strong(c, c + kChunksAtOnce)) unpack(c, std::min(c + kChunksAtOnce, t.chunks));
-    else std::this_thread::yield();
-    return false;
+    const size_t end = std::min(c + kChunksAtOnce, t.chunks);
+    if (c >= t.chunks || t.there.load(std::memory_order_relaxed) < end || !t.next.compare_exchange_strong(c, c + kChunksAtOnce)) return false;
+    unpack(c, end);
+    return true;
   }
 
-  // Has all pieces packed and announces them as they arrive.
+  // Has all of it packed and announces it as it sets out, or arrives.
   void drive() {
     Transfer& t = *transfer_;
     const OnDevice on(t.device);
     hipError_t error = on.error;
     if (error == hipSuccess) error = t.staged ? drive_staged() : drive_straight();
-    if (error != hipSuccess) {
-      t.error = error;
-      (void)hipGetLastError();  // reported by finish(), not to this thread's next launch
-      t.announce(0, true);
-    }
+    if (error != hipSuccess) t.fail(error);
   }
 
-  // Up to kSlots pieces under way at a time, straight to the ring; few, and of few workgroups, while something is computed.
+  // Launches one after another as words become readable and the threads make room in the ring; few, and of few workgroups, while
+  // something is computed.
   hipError_t drive_straight() {
     Transfer& t = *transfer_;
     hipError_t error = hipSuccess;
-    size_t launched = 0;
+    if (t.computed_event && (error = wait_for(t.computed_event)) == hipSuccess) t.announce(t.sent, false);
     bool gently = !t.ready.empty();
-    if (t.device_waits) {
-      error = hipStreamWaitEvent(t.streams[0], t.ready[0].event, 0);
-      t.happened = 1;
-      gently = false;
-    }
-    for (size_t p = 0; p < t.pieces && error == hipSuccess; ++p) {
-      while (launched < t.pieces && error == hipSuccess && readable(launched, /*waits=*/launched == p, &error)) {
-        gently = gently && !computed();
-        if (launched >= p + (gently ? kGentleAhead : kSlots)) break;
-        while (!slot_is_free(launched, p)) {}
-        if (gently) ahead_.fetch_add(1, std::memory_order_relaxed);
-        error = launch(launched++, gently ? kGentleBlocks : UINT32_MAX);
+    size_t gentle = 0, gone = 0;  // launches of those, and how many of them have ended
+    while (t.sent < t.chunks && error == hipSuccess && !t.stop.load(std::memory_order_relaxed)) {
+      gently = gently && !computed();
+      while (gone < gentle && (error = hipEventQuery(packed_[gone % kSlots])) == hipSuccess) gone++;
+      if (error == hipErrorNotReady) error = hipSuccess;
+      if (error != hipSuccess) break;
+      while (t.unpacked_to < t.left.size() && t.left[t.unpacked_to].load(std::memory_order_acquire) == 0) t.unpacked_to++;
+      const size_t room = t.unpacked_to == t.left.size() ? t.chunks : t.unpacked_to * kBlock + t.ring_chunks;
+      // up to the end of what may be read, if that is known, else a piece at a time
+      size_t end = std::min(t.chunks, t.sent + kMostChunks);
+      if (!t.ready.empty()) {
+        if (!readable(words_to(t.sent + 1), /*waits=*/t.next.load() >= t.sent && gone == gentle, &error)) {
+          if (error == hipSuccess && !unpack_some()) spin_pause();
+          continue;
+        }
+        const size_t words = t.ready[t.happened - 1].words, whole = words == t.n ? t.chunks : words / kPackChunk;
+        end = std::min(whole, gently || t.chunks > t.ring_chunks ? t.sent + kMostChunks : t.chunks);
       }
-      if (error == hipSuccess) error = hipEventSynchronize(packed_[p % kSlots]);
-      if (error == hipSuccess) t.announce(p + 1, false);
+      if (end > room || (gently && gentle - gone >= kGentleAhead)) {
+        if (!unpack_some()) std::this_thread::yield();
+        continue;
+      }
+      if (gently) ahead_.fetch_add(1, std::memory_order_relaxed);
+      error = launch(end, gently ? kGentleBlocks : bus_blocks());
+      if (error == hipSuccess && gently) error = hipEventRecord(packed_[gentle++ % kSlots], t.streams[(t.launches - 1) % 2]);
+      if (error == hipSuccess) t.announce(t.sent, false);
     }
     return error;
   }
@@ -1168,10 +1324,10 @@ class ResultStream {
     while (here < t.pieces) {
       hipError_t e = hipSuccess;
       bool moved = false;
-      if (launched < t.pieces && launched < sent + kPackedAhead && readable(launched, /*waits=*/here == launched, &e) &&
-          slot_is_free(launched, here)) {
+      if (launched < t.pieces && launched < sent + kPackedAhead && readable(words_to(t.begins[launched + 1]), /*waits=*/here == launched, &e) &&
+          slot_is_free(launched)) {
         if (!computed()) ahead_.fetch_add(1, std::memory_order_relaxed);
-        e = launch(launched++);
+        e = launch_piece(launched++);
         moved = true;
       }
       if (e != hipSuccess) return e;
@@ -1182,7 +1338,7 @@ class ResultStream {
       }
       if (here < sent && (e = hipEventQuery(copied_[here % kSlots])) != hipErrorNotReady) {
         if (e != hipSuccess) return e;
-        t.announce(++here, false);
+        t.announce(t.begins[++here], false);
         moved = true;
       }
       if (!moved) spin_pause();
@@ -1190,15 +1346,29 @@ class ResultStream {
     return hipSuccess;
   }
 
+  // Whether a piece's slot is free: the piece before it there is unpacked.  If not, does some of that.
+  bool slot_is_free(size_t piece) {
+    Transfer& t = *transfer_;
+    if (piece < kSlots) return true;
+    for (size_t b = t.begins[piece - kSlots] / kBlock; b * kBlock < t.begins[piece - kSlots + 1]; ++b)
+      if (t.left[b].load(std::memory_order_acquire) != 0) {
+        if (!unpack_some()) std::this_thread::yield();
+        return false;
+      }
+    return true;
+  }
+
   std::unique_ptr<Transfer> transfer_;
   HostWorkers::Job job_;
-  StreamUse use_;
-  bool under_way_ = false, misfit_ = false;
+  bool under_way_ = false, helped_ = false, misfit_ = false;
   int device_ = -1;  // of the events and the ring
   uint32_t looks_ = 0;
   std::atomic<size_t> ahead_{0};  // parts_ahead()
+  uint64_t transfers_ = 0;
   uint8_t* ring_ = nullptr;
   size_t ring_bytes_ = 0;
+  PackHeader* headers_ = nullptr;  // straight
+  size_t headers_held_ = 0;
   hipEvent_t packed_[kSlots] = {}, begun_ = nullptr;
   // of pieces that are packed in device memory
   static constexpr size_t kWordsPerLine = 32;

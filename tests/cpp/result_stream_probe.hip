@@ -1,6 +1,6 @@
 // Results brought to the host by ResultStream (nd_host_results.hpp), against the words that were put on the device:
-// every width, sizes around a group, a chunk and a piece, dead groups, ids that do not fit their width, targets that
-// are no multiple of 32 bytes; straight to the host, and packed on the device as words that come while others are still
+// every width, sizes around a group, a chunk, a piece and the ring, dead groups, chunks of few different ids, ids that do not fit
+// their width, targets that are no multiple of 32 bytes; straight to the host, and packed on the device as words that come while others are still
 // computed are, with a sign that is there and with one that never comes.  Prints the case before it runs, "all equal" at the end.
 #include "../../nextdoor_amd/csrc/nd_host_results.hpp"
 
@@ -135,7 +135,8 @@ int main() {
   if (on_other_devices() != 0) return 1;
   if (beside_one_that_waits() != 0) return 1;
   const size_t piece = (size_t)64 * nd::kPackChunk;  // the smallest piece
-  const size_t sizes[] = {1, 7, 8, 9, nd::kPackChunk - 1, nd::kPackChunk, nd::kPackChunk + 1, piece, piece + 9, 13 * piece + 4097};
+  const size_t sizes[] = {1, 7, 8, 9, nd::kPackChunk - 1, nd::kPackChunk, nd::kPackChunk + 1, piece, piece + 9, 13 * piece + 4097,
+                          (size_t)4200 * nd::kPackChunk + 5};
   nd::ResultStream stream;
   uint32_t* sign = nullptr;  // what has arrived, and what never does
   hipEvent_t done;
@@ -147,6 +148,7 @@ int main() {
     TRY(hipMalloc(&d, n * sizeof(int32_t)));
     for (uint32_t bits : {1u, 2u, 7u, 8u, 9u, 12u, 16u, 17u, 23u, 24u, 25u, 26u, 31u, 32u}) {
       if (n > piece + 9 && bits != 12 && bits != 23 && bits != 32) continue;
+      if (n > 14 * piece && bits == 23) continue;
       for (int misfit = 0; misfit < 2; ++misfit) {
         printf("n %zu bits %u misfit %d\n", n, bits, misfit);
         fflush(stdout);
@@ -155,6 +157,8 @@ int main() {
         std::vector<int32_t> want(n), got(n + 2, 77);
         for (size_t i = 0; i < n; ++i)
           want[i] = (i / 11) % 3 == 0 || (i / 700) % 4 == 1 ? fill : (int32_t)(((uint32_t)i * 2654435761u) & mask);
+        for (size_t i = 0; i < n; ++i)  // every third chunk: ids next to each other, one of them the largest there is
+          if (i / nd::kPackChunk % 3 == 1 && want[i] != fill) want[i] = (int32_t)(mask - 1u - ((uint32_t)want[i] & mask & 9u));
         if (misfit) want[n / 2] = -5;
         TRY(hipMemcpy(d, want.data(), n * sizeof(int32_t), hipMemcpyHostToDevice));
         for (int shift = 0; shift < 2; ++shift) {
