@@ -134,10 +134,12 @@ class EngineBase {
   // Sample states: what an App's struct holds is its own, but mostly it is vertices (and small numbers), which
   // fit the ids' bits.  Where they do not once, no later transfer tries (100 K samples of MultiRW, 40 MB: 0.88 -> 0.52 ms).
   int states_to_host(void* dst, const void* src, size_t bytes, hipStream_t stream) {
-    const int rc = fetch_to_host(dst, src, bytes, states_fit_ids_ ? (uint32_t)max_bits() : 32u, -1, stream);
+    const int rc = fetch_to_host(dst, src, bytes, state_bits(), kNoState, stream);
     if (result_stream->misfit()) states_fit_ids_ = false;
     return rc;
   }
+  static constexpr int32_t kNoState = -1;
+  uint32_t state_bits() const { return states_fit_ids_ && !result_stream->misfit() ? (uint32_t)max_bits() : 32u; }
 
   HostArray<VertexID_t> hFinalSamples{host_pool};  // as NextDoorData::hFinalSamples (libNextDoor.hpp:17)
   HostArray<unsigned char> hSampleStates{host_pool};
@@ -2132,7 +2134,7 @@ class Engine : public EngineBase {
   // the only host wait is at the end.
   int sample(int mode) override {
     if (!allocated_) { last_error = "sample before alloc"; return -1; }
-    (void)finish_rows_ahead();  // nobody asked for them
+    drop_rows_ahead();  // nobody asked for them
     if ((inverts(mode) ? alloc_inversion() : build_walk_tables()) != 0) return -1;  // what an earlier pass has not
     times = PhaseTimes();
     sent_ahead_ = rows_follow_ = false;
@@ -2153,7 +2155,7 @@ class Engine : public EngineBase {
     const int rc = wants_launch_graph() ? replay_pass(mode) : enqueue_pass(mode);
     if (rc != 0) return rc;
     ND_HIP_TRY(hipEventRecord(ev_end_, stream_));
-    if (rows_follow_) send_rows({}, ev_end_);
+    if (rows_follow_) send_rows({}, {}, ev_end_);
     ND_HIP_TRY(hipEventSynchronize(ev_end_));
     ND_HIP_TRY(hipEventElapsedTime(&times.end_to_end, ev_begin_, ev_end_));
     schedule_counts_.passes++;
@@ -2215,40 +2217,64 @@ class Engine : public EngineBase {
     const uint32_t ranges = form == kRowsByRange ? walk_ranges() : 1;
     const size_t F = (size_t)final_sample_size();
     std::vector<ResultStream::Ready> ready;
+    std::vector<size_t> ends;  // samples
     rows_follow_ = form == kRowsFollow;
-    while (form != kRowsStay && form != kRowsFollow && range_ends_.size() < ranges) {
-      hipEvent_t ev = nullptr;
-      ND_HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-      range_ends_.push_back(ev);
-    }
+    if (form != kRowsStay && form != kRowsFollow && make_range_ends(ranges) != 0) return -1;
     uint32_t first = 0;
     for (uint32_t r = 0; r < ranges; ++r) {
       const uint32_t end = r + 1 == ranges ? (uint32_t)n_samples_ : (uint32_t)((uint64_t)n_samples_ * (r + 1) / ranges / kWave * kWave);
       if (launch_walks(first, end - first, d_walk_queue_ + 2 * r, early) != 0) return -1;
       if (form == kRowsStay || form == kRowsFollow) return 0;
       ND_HIP_TRY(hipEventRecord(range_ends_[r], stream_));
-      ready.push_back({end * F, range_ends_[r]});
+      ends.push_back(end);
       first = end;
     }
     if (form == kRowsByStretch) {
-      ready.clear();
+      ends.clear();
       for (uint64_t at = 0; at < (uint64_t)n_samples_; at += 1ull << early.shift)
         ready.push_back({(size_t)std::min<uint64_t>((uint64_t)n_samples_, at + (1ull << early.shift)) * F, range_ends_[0],
                          h_arrived_ + (at >> early.shift), early.pass});
     }
-    send_rows(std::move(ready), nullptr);
+    send_rows(ends, std::move(ready), nullptr);
     sent_ahead_ = ahead_;
     return 0;
   }
+  int make_range_ends(uint32_t ranges) {
+    while (range_ends_.size() < ranges) {
+      hipEvent_t ev = nullptr;
+      ND_HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+      range_ends_.push_back(ev);
+    }
+    return 0;
+  }
 
-  // Has the rows leave for rows_ahead; those that cannot be sent now are fetched when they are asked for.
-  void send_rows(std::vector<ResultStream::Ready> ready, hipEvent_t computed) {
+  // Has the rows leave for rows_ahead, and the states for states_ahead; those that cannot be sent now are fetched when they are asked
+  // for.  ends: of the ranges of samples whose results are there at one of range_ends_ each; none: as `ready` has it, or in
+  // stream order.
+  void send_rows(const std::vector<size_t>& ends, std::vector<ResultStream::Ready> ready, hipEvent_t computed) {
+    const size_t F = (size_t)final_sample_size(), state_words = sizeof(SampleType) / sizeof(int32_t);
+    const bool states = states_ahead && ready.empty();
     try {
-      ahead_ = result_stream->begin(d_final_, (size_t)n_samples_ * (size_t)final_sample_size(), (uint32_t)max_bits_, invalid_,
-                                   rows_ahead, stream_, std::move(ready), computed) == hipSuccess;
+      std::vector<ResultStream::Part> parts;
+      size_t words = 0;
+      for (size_t r = 0, at = 0; r < std::max<size_t>(1, ends.size()); ++r) {
+        const size_t end = ends.empty() ? (size_t)n_samples_ : ends[r];
+        if (r == 0 || states) parts.push_back({d_final_ + at * F, 0, (uint32_t)max_bits_, invalid_, rows_ahead + at * F});
+        parts.back().n += (end - at) * F;
+        words += (end - at) * F;
+        if (states) {
+          parts.push_back({(const int32_t*)d_samples_ + at * state_words, (end - at) * state_words, state_bits(), kNoState,
+                           states_ahead + at * state_words});
+          words += (end - at) * state_words;
+        }
+        if (!ends.empty()) ready.push_back({words, range_ends_[r]});
+        at = end;
+      }
+      ahead_ = result_stream->begin(std::move(parts), stream_, std::move(ready), computed) == hipSuccess;
     } catch (const std::bad_alloc&) {
       ahead_ = false;
     }
+    states_sent_ = ahead_ && states;
     if (!ahead_) (void)hipGetLastError();
   }
 
@@ -2403,8 +2429,6 @@ class Engine : public EngineBase {
   int enqueue_pass(int mode) {
     App app;
     const int n_steps = app.steps();
-    const size_t F = (size_t)final_sample_size();
-    const bool sample_parallel = mode == kSampleParallel;
     if (!inverts(mode)) return enqueue_walks();
     // A pass whose classifications found nothing at all for the workgroup kernel is followed by
     // passes that do not classify (nor launch the workgroup kernel); every kIdleLookEvery-th
@@ -2433,28 +2457,73 @@ class Engine : public EngineBase {
     balanced_this_pass_ = balance;
     if (balance)
       fill_i32<<<dim3((kBalanceWords + 255) / 256), dim3(256), 0, stream_>>>((int32_t*)d_balance_, kBalanceWords, 0);
+    const bool sends = rows_ahead && !profiling && !wants_launch_graph();
+    const uint32_t early = sends ? early_samples() : 0u;
+    if (early == 0) {
+      rows_follow_ = sends;
+      return enqueue_steps(mode, balance, 0, (uint32_t)n_samples_);
+    }
+    if (make_range_ends(2) != 0) return -1;
+    const std::vector<size_t> ends{early, (size_t)n_samples_};
+    for (size_t r = 0, at = 0; r < ends.size(); at = ends[r++]) {
+      if (enqueue_steps(mode, balance, (uint32_t)at, (uint32_t)(ends[r] - at)) != 0) return -1;
+      ND_HIP_TRY(hipEventRecord(range_ends_[r], stream_));
+    }
+    send_rows(ends, {}, nullptr);
+    sent_ahead_ = ahead_;
+    return 0;
+  }
+
+  // Samples that are sampled before the others, so that their rows leave while those are: 0, all at once.  The bus, and the threads that
+  // unpack beside it, take some five times as long as the sampling, so a quarter is enough to keep them busy meanwhile; and
+  // as the launches of the others take a tenth of a millisecond at the least, rows have to be many.  Passes with their rows, ms, by that share:
+  //                     0    15 %   25 %   35 %
+  //    KHop    60 K   0.93   0.95   0.94   0.94    (66 MB)
+  //            90 K   1.35   1.40   1.32   1.36
+  //           200 K   2.90   2.76   2.71   2.73
+  //       R-MAT 20   10.42   9.60   9.67   9.80
+  //    Layer   50 K   0.83   0.98   0.94   0.94
+  //           100 K   1.55   1.65   1.55   1.57    (104 MB)
+  //           150 K   2.31   2.35   2.22   2.11
+  //           300 K   4.80   4.60   4.24   4.17
+  static constexpr uint64_t kEarlyRowsFromBytes = 96u << 20;
+  uint32_t early_samples() const {
+    const uint64_t n = (uint64_t)n_samples_;
+    if (walk_mode_ || sizeof(VertexID_t) * n * (uint64_t)final_sample_size() < kEarlyRowsFromBytes) return 0;
+    return (uint32_t)(n / 4u) / 64u * 64u;
+  }
+  // Rows that the step kernels write with all that is INVALID in them (StepParams::fill_levels).
+  bool kernels_fill() const { return rows_direct_ && !explicit_map_ && !walk_mode_ && App().steps() <= kMaxFillLevels; }
+
+  // The steps of the samples [first_sample, first_sample + count); of walks, all of them.
+  int enqueue_steps(int mode, bool balance, uint32_t first_sample, uint32_t count) {
+    App app;
+    const int n_steps = app.steps();
+    const size_t F = (size_t)final_sample_size();
+    const bool sample_parallel = mode == kSampleParallel, placed = small_placed_;
+    VertexID_t* const final_rows = d_final_ + (size_t)first_sample * F;
     // pairs whose transit is INVALID are dropped by the inversion and never reach a step
     // kernel: their outputs keep this fill - unless the step kernels write the rows themselves
     // and, with every INVALID, what descends from it (StepParams::fill_levels)
-    const bool kernels_fill = rows_direct_ && !explicit_map_ && !walk_mode_ && n_steps <= kMaxFillLevels;
+    const bool kernels_fill = this->kernels_fill();
     // walks whose results go into cells of two steps: the regrouping reads only the cells a walk
     // has written (StepParams::walk_cells)
     const bool no_fill = kernels_fill || paired_results();
     if (!no_fill || mark_unwritten_) {
       const int32_t value = no_fill ? invalid_ + 1 : invalid_;
-      const size_t n_out = (size_t)n_samples_ * (paired_results() ? (F + 1) / 2 * 2 : F);
+      const size_t n_out = (size_t)count * (paired_results() ? (F + 1) / 2 * 2 : F);
       fill_i32<<<dim3((unsigned)((n_out + 1023) / 1024)), dim3(1024), 0, stream_>>>(
-          rows_direct_ ? d_final_ : d_step_out_, n_out, value);
+          rows_direct_ ? final_rows : d_step_out_, n_out, value);
     }
 
     uint32_t transits_per_sample = (uint32_t)init_size_;
     const uint32_t* live_last = nullptr;  // pairs the last inversion kept (device count)
     int sorts_done = 0;
-    const int32_t* transits = d_initial_;  // (sample -> transit) map entering the step
+    const int32_t* transits = d_initial_ + (size_t)first_sample * init_size_;  // (sample -> transit) map entering the step
     KeyLayout transits_layout;             // and how it is laid out
     for (int step = 0; step < n_steps; ++step) {
       const uint32_t m = (uint32_t)app.stepSize(step);
-      const uint32_t n_pairs = (uint32_t)((uint64_t)n_samples_ * transits_per_sample);
+      const uint32_t n_pairs = (uint32_t)((uint64_t)count * transits_per_sample);
       StepParams P;
       P.csr = view_;
       P.step = step;
@@ -2465,21 +2534,21 @@ class Engine : public EngineBase {
       P.invalid = invalid_;
       P.is_last = step == n_steps - 1;
       P.seed = seed_;
-      P.first_slot = (uint64_t)first_sample_ * transits_per_sample * m;  // outputs of the samples before ours
-      P.first_sample = (uint32_t)first_sample_;
+      P.first_slot = ((uint64_t)first_sample_ + first_sample) * transits_per_sample * m;  // outputs of the samples before these
+      P.first_sample = (uint32_t)first_sample_ + first_sample;
       P.n_pairs = n_pairs;
       P.live_pairs = nullptr;
       if (rows_direct_) {
-        P.step_out = d_final_ + layout_.seg_base[step];
+        P.step_out = final_rows + layout_.seg_base[step];
         P.out_pitch = (uint32_t)F;
       } else {
-        P.step_out = d_step_out_ + (size_t)n_samples_ * layout_.seg_base[step];
+        P.step_out = d_step_out_ + (size_t)count * layout_.seg_base[step];
         P.out_pitch = layout_.seg_len[step];
       }
       P.pair_cells = paired_results() ? d_step_out_ : nullptr;
       P.pair_cell_samples = (uint32_t)n_samples_;
       P.walk_cells = paired_results() ? d_walk_cells_ : nullptr;
-      P.samples = d_samples_;
+      P.samples = d_samples_ ? d_samples_ + first_sample : nullptr;
       P.explicit_out = explicit_map_ && step + 1 < n_steps ? d_explicit_ : nullptr;
       P.fill_levels = 0;
       if (kernels_fill) {
@@ -2666,22 +2735,22 @@ class Engine : public EngineBase {
     if (rows_direct_) {
       // the step kernels wrote the rows themselves
     } else if (walk_mode_ && rows_per_block_ > 0) {
-      const unsigned blocks = (unsigned)((n_samples_ + rows_per_block_ - 1) / rows_per_block_);
+      const unsigned blocks = (unsigned)((count + rows_per_block_ - 1) / rows_per_block_);
       const size_t lds = (size_t)rows_per_block_ * row_pitch_ * sizeof(int32_t);
-      assemble_walk_rows<<<dim3(blocks), dim3(256), lds, stream_>>>(d_step_out_, d_final_, (uint32_t)n_samples_,
+      assemble_walk_rows<<<dim3(blocks), dim3(256), lds, stream_>>>(d_step_out_, final_rows, count,
                                                                     (uint32_t)n_steps, row_pitch_, rows_per_block_,
                                                                     paired_results() ? 1u : 0u,
                                                                     paired_results() ? d_walk_cells_ : nullptr, invalid_);
     } else if (rows_per_block_ > 0) {
-      const unsigned blocks = (unsigned)((n_samples_ + rows_per_block_ - 1) / rows_per_block_);
+      const unsigned blocks = (unsigned)((count + rows_per_block_ - 1) / rows_per_block_);
       const size_t lds = (size_t)rows_per_block_ * row_pitch_ * sizeof(int32_t);
-      assemble_final_rows<<<dim3(blocks), dim3(256), lds, stream_>>>(d_step_out_, d_final_, (uint32_t)n_samples_,
+      assemble_final_rows<<<dim3(blocks), dim3(256), lds, stream_>>>(d_step_out_, final_rows, count,
                                                                      (uint32_t)F, row_pitch_, rows_per_block_, layout_);
     } else {
       for (int k = 0; k < n_steps; ++k) {
-        const size_t n = (size_t)n_samples_ * layout_.seg_len[k];
+        const size_t n = (size_t)count * layout_.seg_len[k];
         assemble_final_step<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream_>>>(
-            d_step_out_ + (size_t)n_samples_ * layout_.seg_base[k], d_final_, n, layout_.seg_len[k], (uint32_t)F,
+            d_step_out_ + (size_t)count * layout_.seg_base[k], final_rows, n, layout_.seg_len[k], (uint32_t)F,
             layout_.seg_base[k]);
       }
     }
@@ -2773,6 +2842,8 @@ class Engine : public EngineBase {
   // cross the bus while later walks are still under way; sample() returns when the sampling is done, as
   // always, and the rest of the rows arrives until finish_rows_ahead().  Any pass may leave it be.
   VertexID_t* rows_ahead = nullptr;
+  // ... and its states (whole words), with rows only.
+  int32_t* states_ahead = nullptr;
   // Waits for rows on their way; whether they are at rows_ahead.  Where not (no pass sent them, the transfer failed) they
   // are to be fetched like any others.
   bool finish_rows_ahead() {
@@ -2782,20 +2853,20 @@ class Engine : public EngineBase {
     return there;
   }
 
-  bool is_walk() const { return walk_mode_; }
-
   int fetch_sample_states(void* dst, size_t bytes) override {
     if (!allocated_ || std::is_empty<SampleType>::value) { last_error = "no sample state"; return -1; }
     if (bytes != sample_state_bytes()) { last_error = "sample state size mismatch"; return -1; }
     settle_rows_ahead();
-    return states_to_host(dst, d_samples_, bytes, stream_);
+    const bool there = states_sent_ && dst == states_ahead;
+    states_sent_ = false;
+    return there ? 0 : states_to_host(dst, d_samples_, bytes, stream_);
   }
 
   // Distinct post-pass over the device-resident result rows (see nd_distinct.hpp): every
   // hop segment of every sample becomes its ascending unique valid ids, INVALID-padded.
   int distinct() override {
     if (!allocated_) { last_error = "distinct before alloc"; return -1; }
-    (void)finish_rows_ahead();  // they are about to change
+    drop_rows_ahead();  // they are about to change
     App app;
     if (app.outputFormat() != SampledVertices) { last_error = "distinct needs SampledVertices output"; return -2; }
     const int n_steps = app.steps();
@@ -2973,7 +3044,11 @@ class Engine : public EngineBase {
   // The result stream carries one transfer at a time, and whoever begins another waits for the one before: rows on their way
   // are waited for here first, where it is known whose they are and what has become of them.
   void settle_rows_ahead() {
-    if (ahead_ && result_stream->finish() != hipSuccess) ahead_ = sent_ahead_ = false;
+    if ((ahead_ || states_sent_) && result_stream->finish() != hipSuccess) ahead_ = sent_ahead_ = states_sent_ = false;
+  }
+  void drop_rows_ahead() {
+    if (ahead_ || states_sent_) result_stream->abandon();
+    ahead_ = states_sent_ = false;
   }
 
   void launch_workgroup(const StepParams& P, unsigned grid, const RunsMeta* meta) {
@@ -3132,8 +3207,9 @@ class Engine : public EngineBase {
   }
 
   void free_run_buffers() {
-    (void)finish_rows_ahead();
+    drop_rows_ahead();
     rows_ahead = nullptr;
+    states_ahead = nullptr;
     for (hipEvent_t ev : range_ends_) (void)hipEventDestroy(ev);
     range_ends_.clear();
     free_early_rows();
@@ -3214,6 +3290,7 @@ class Engine : public EngineBase {
   uint32_t walk_waves_at_once_ = 1, cus_ = 1;  // wavefronts of walk_rows_kernel the device holds, compute units
   bool ahead_ = false;                    // rows are on their way to rows_ahead
   bool sent_ahead_ = false;               // ... or have been, in the last pass, while its walks were under way
+  bool states_sent_ = false;              // states are on their way to states_ahead, or there
   bool rows_follow_ = false;              // the pass under way sends them directly behind its last launch
   std::vector<hipEvent_t> range_ends_;    // ends of the launches of such a pass
   // of such a pass: EarlyRows::arrived and walked, and the number of the last

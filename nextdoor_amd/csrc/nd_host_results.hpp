@@ -746,7 +746,17 @@ class ResultStream {
   ResultStream& operator=(const ResultStream&) = delete;
   ~ResultStream() { release(); }
 
-  // The first `words` words of a result are on the device once `event` has happened, or, if there is a `sign` (all of a
+  // Words of device memory that go together.  Those that are `fill` in groups of eight cost nothing; they are expected to fit `bits`
+  // bits (one that does not makes the whole transfer start again with 32).  src is aligned to 16 bytes.
+  struct Part {
+    const int32_t* src;
+    size_t n;
+    uint32_t bits;
+    int32_t fill;
+    int32_t* dst;
+  };
+
+  // The first `words` words of a transfer's parts are on the device once `event` has happened, or, if there is a `sign` (all of a
   // transfer's have one or none has; page-locked memory a kernel that is still running writes to, after the words), once that is
   // `value`.
   struct Ready {
@@ -762,7 +772,7 @@ class ResultStream {
     if (e == hipSuccess) e = come_to_device_of(nullptr);
     if (e != hipSuccess || n == 0) return e;
     if (!transfer_) transfer_.reset(new Transfer);
-    transfer_->set(nullptr, n, bits > kPackMostBits ? 32 : bits, 0, nullptr, {});
+    transfer_->set({{nullptr, n, bits, 0, nullptr}}, {});
     e = prepare(*transfer_);
     // its pages are mapped when they are first touched: 0.8 ms of 2 MB
     if (e == hipSuccess) memset(ring_, 0, transfer_->chunk_bytes * transfer_->ring_chunks);
@@ -785,23 +795,28 @@ class ResultStream {
     return e;
   }
 
-  // n words at src (aligned to 16 bytes) to dst, in stream order.  Words that are `fill` in groups of eight cost
-  // nothing; words are expected to fit `bits` bits (one that does not makes the whole transfer start again with
-  // 32).
-  hipError_t fetch(const int32_t* src, size_t n, uint32_t bits, int32_t fill, int32_t* dst, hipStream_t stream) {
-    const hipError_t e = begin(src, n, bits, fill, dst, stream, {});
+  // Parts to where they belong, in stream order.
+  hipError_t fetch(std::vector<Part> parts, hipStream_t stream) {
+    const hipError_t e = begin(std::move(parts), stream, {});
     return e == hipSuccess ? finish() : e;
+  }
+  hipError_t fetch(const int32_t* src, size_t n, uint32_t bits, int32_t fill, int32_t* dst, hipStream_t stream) {
+    return fetch({{src, n, bits, fill, dst}}, stream);
+  }
+  hipError_t begin(const int32_t* src, size_t n, uint32_t bits, int32_t fill, int32_t* dst, hipStream_t stream,
+                   std::vector<Ready> ready, hipEvent_t computed = nullptr) {
+    return begin({{src, n, bits, fill, dst}}, stream, std::move(ready), computed);
   }
 
   // The same as a begin() that returns at once, other threads taking it from there, and a finish() that takes part
-  // and returns when the words are at dst.  `ready` (words ascending, the last n): what has to have
+  // and returns when the words are at dst.  `ready` (words ascending, the last all of them; with a sign, of a single part): what has to have
   // happened before words may be read, while other work of the caller's is still going on; empty: stream order, and `computed`, if there is
   // one, an event recorded on the stream before, that the threads need not look for words until it has happened.  What is given has
   // to stay until finish().
-  hipError_t begin(const int32_t* src, size_t n, uint32_t bits, int32_t fill, int32_t* dst, hipStream_t stream,
-                   std::vector<Ready> ready, hipEvent_t computed = nullptr) {
+  hipError_t begin(std::vector<Part> parts, hipStream_t stream, std::vector<Ready> ready, hipEvent_t computed = nullptr) {
     hipError_t e = finish();  // an earlier one that nobody waited for
-    if (e != hipSuccess || n == 0) return e;
+    parts.erase(std::remove_if(parts.begin(), parts.end(), [](const Part& p) { return p.n == 0; }), parts.end());
+    if (e != hipSuccess || parts.empty()) return e;
     if (!transfer_) transfer_.reset(new Transfer);
     Transfer& t = *transfer_;
     e = come_to_device_of(stream);
@@ -809,7 +824,7 @@ class ResultStream {
     t.device = device_;
     const OnDevice on(t.device);
     if (on.error != hipSuccess) return on.error;
-    t.set(src, n, bits > kPackMostBits ? 32 : bits, fill, dst, std::move(ready));
+    t.set(std::move(parts), std::move(ready));
     e = prepare(t);
     if (e == hipSuccess && t.staged) e = prepare_staging(t.slot_bytes);
     if (e != hipSuccess) return e;
@@ -827,8 +842,11 @@ class ResultStream {
         e = hipEventRecord(begun_, stream);
         if (e == hipSuccess) e = hipStreamWaitEvent(t.streams[1], begun_, 0);
       }
-      if (e == hipSuccess) e = launch(std::min(t.chunks, t.ring_chunks), bus_blocks());
-      if (e != hipSuccess) return e;
+      while (e == hipSuccess && t.sent < t.ring_chunks) e = launch(std::min(t.part_ends[t.part_of(t.sent)], t.ring_chunks), bus_blocks());
+      if (e != hipSuccess) {
+        for (hipStream_t s : t.streams) (void)hipStreamSynchronize(s);  // nothing writes to the ring after this
+        return e;
+      }
       // few chunks are unpacked before a thread is awake, unless it is woken while they are computed
       if (t.chunks <= kFewChunks) helpers = computed ? t.chunks / kChunksAHelper : 0;
       if (!computed) t.announce(t.sent, false);
@@ -857,7 +875,15 @@ class ResultStream {
     if (!t.overflow.load()) return hipSuccess;
     misfit_ = true;
     const OnDevice on(t.device);  // the stream may be the default one
-    return fetch(t.src, t.n, 32, t.fill, t.dst, t.ready.empty() ? t.streams[0] : transfer_stream(t.device, 0));
+    std::vector<Part> parts = t.parts;
+    for (Part& p : parts) p.bits = 32;
+    return fetch(std::move(parts), t.ready.empty() ? t.streams[0] : transfer_stream(t.device, 0));
+  }
+
+  // Nobody wants the words any more.
+  void abandon() {
+    if (under_way_) transfer_->fail(hipErrorUnknown);
+    (void)finish();
   }
 
   // whether a word has ever not fitted
@@ -1008,13 +1034,13 @@ class ResultStream {
   }
 
   struct Transfer {
-    const int32_t* src;
-    size_t n;
-    uint32_t bits;
-    int32_t fill;
-    int32_t* dst;
+    std::vector<Part> parts;
+    std::vector<size_t> part_ends;     // chunks; a chunk is of one part
+    uint32_t bits = 0;                 // the most of any part
+    bool streaming = false;            // results larger than the caches
     hipStream_t streams[2];
     std::vector<Ready> ready;
+    std::vector<size_t> ready_chunks;  // that are there once a `ready` has happened
     hipEvent_t computed_event = nullptr;
     bool staged = false;  // pieces are packed in device memory, for the copy engine, while something else is computed
     int device = 0;
@@ -1042,13 +1068,24 @@ class ResultStream {
     unsigned sleepers = 0;
     std::vector<std::atomic<size_t>> left;  // chunks of a block that are not unpacked yet
 
-    void set(const int32_t* src_, size_t n_, uint32_t bits_, int32_t fill_, int32_t* dst_, std::vector<Ready> ready_) {
-      src = src_, n = n_, bits = bits_, fill = fill_, dst = dst_, ready = std::move(ready_);
+    void set(std::vector<Part> parts_, std::vector<Ready> ready_) {
+      parts = std::move(parts_), ready = std::move(ready_);
       staged = !ready.empty() && ready.front().sign != nullptr;
       computed_event = nullptr;
       happened = 0;
       computed = false;
-      chunks = (n + kPackChunk - 1) / kPackChunk;
+      chunks = 0;
+      bits = 0;
+      part_ends.clear();
+      size_t words = 0;
+      for (const Part& p : parts) {
+        words += p.n;
+        part_ends.push_back(chunks += (p.n + kPackChunk - 1) / kPackChunk);
+        bits = std::max(bits, p.bits > kPackMostBits ? 32 : p.bits);
+      }
+      streaming = words * sizeof(int32_t) > kDirectResultBytes;
+      ready_chunks.clear();
+      for (const Ready& r : ready) ready_chunks.push_back(chunks_of(r.words));
       chunk_bytes = (size_t)kPackChunkGroups * bits;
       ring_chunks = std::min(chunks, kRingChunks);
       sent = launches = unpacked_to = 0;
@@ -1073,6 +1110,21 @@ class ResultStream {
       const size_t blocks = (chunks + kBlock - 1) / kBlock;
       left = std::vector<std::atomic<size_t>>(blocks);
       for (size_t b = 0; b < blocks; ++b) left[b].store(std::min(kBlock, chunks - b * kBlock));
+    }
+
+    // whole chunks among the first words
+    size_t chunks_of(size_t words) const {
+      for (size_t p = 0; p < parts.size(); ++p) {
+        if (words < parts[p].n) return part_begin(p) + words / kPackChunk;
+        words -= parts[p].n;
+      }
+      return chunks;
+    }
+    size_t part_begin(size_t p) const { return p == 0 ? 0 : part_ends[p - 1]; }
+    size_t part_of(size_t chunk) const {
+      size_t p = 0;
+      while (part_ends[p] <= chunk) p++;
+      return p;
     }
 
     // (no other chunk's that was or will be where this one is)
@@ -1111,7 +1163,6 @@ class ResultStream {
   };
 
   uint8_t* slot(size_t piece) const { return ring_ + (piece % kSlots) * transfer_->slot_bytes; }
-  size_t words_to(size_t chunk) const { return std::min(transfer_->n, chunk * kPackChunk); }
 
   // (hipEventSynchronize() keeps whoever uses the event's stream otherwise, another transfer's begin() for one, until it has happened.)
   static hipError_t wait_for(hipEvent_t event) {
@@ -1121,10 +1172,10 @@ class ResultStream {
     return e;
   }
 
-  // Whether words may be read, or, with `waits`, until they may.
-  bool readable(size_t words, bool waits, hipError_t* error) {
+  // Whether the first chunks may be read, or, with `waits`, until they may.
+  bool readable(size_t chunks, bool waits, hipError_t* error) {
     Transfer& t = *transfer_;
-    while (t.happened < t.ready.size() && (t.happened == 0 || t.ready[t.happened - 1].words < words)) {
+    while (t.happened < t.ready.size() && (t.happened == 0 || t.ready_chunks[t.happened - 1] < chunks)) {
       const Ready& next = t.ready[t.happened];
       hipError_t e = hipErrorNotReady;
       if (!next.sign) {
@@ -1156,18 +1207,20 @@ class ResultStream {
 
   uint32_t bus_blocks() const { return transfer_->chunks > transfer_->ring_chunks ? kBusBlocksOfMany : kBusBlocks; }
 
-  // Straight: the chunks from t.sent on, up to `end`.
+  // Straight: the chunks from t.sent on, up to `end`, all of one part.
   hipError_t launch(size_t end, uint32_t most_blocks) {
     Transfer& t = *transfer_;
-    const size_t first = t.sent * kPackChunk, here = words_to(end) - first;
+    const size_t part = t.part_of(t.sent), first = (t.sent - t.part_begin(part)) * kPackChunk;
+    const Part& p = t.parts[part];
     const uint32_t n_chunks = (uint32_t)(end - t.sent);
+    const size_t here = std::min(p.n - first, n_chunks * (size_t)kPackChunk);
     PackedOut out{ring_, headers_};
     out.first = (uint32_t)(t.sent % t.ring_chunks);
     out.ring_mask = t.chunks > t.ring_chunks ? (uint32_t)t.ring_chunks - 1u : UINT32_MAX;
     static_assert((kRingChunks & (kRingChunks - 1)) == 0, "a ring that is gone round");
     out.stamp = t.stamp(t.sent);
     pack_results<false><<<dim3(std::min(n_chunks, most_blocks)), dim3(kPackThreads), 0, t.streams[t.launches % 2]>>>(
-        t.src + first, here, t.bits, t.fill, out, n_chunks);
+        p.src + first, here, t.bits, p.fill, out, n_chunks);
     t.launches++;
     t.sent = end;
     return hipGetLastError();
@@ -1176,15 +1229,16 @@ class ResultStream {
   // Staged: a piece.
   hipError_t launch_piece(size_t piece) {
     const Transfer& t = *transfer_;
+    const Part& p = t.parts[0];
     const size_t first = t.begins[piece] * kPackChunk;
-    const size_t here = words_to(t.begins[piece + 1]) - first, slot_of = piece % kSlots;
+    const size_t here = std::min(p.n, t.begins[piece + 1] * kPackChunk) - first, slot_of = piece % kSlots;
     uint8_t* at = staging_ + slot_of * t.slot_bytes;
     const uint32_t n_chunks = (uint32_t)((here + kPackChunk - 1) / kPackChunk);
     PackedOut out{at + t.packed_at, (PackHeader*)at};
     out.cursor = counts_ + 2 * slot_of * kWordsPerLine;
     out.finished = out.cursor + kWordsPerLine;
     out.total = totals_ + slot_of;
-    pack_results<true><<<dim3(n_chunks), dim3(kPackThreads), 0, t.streams[0]>>>(t.src + first, here, t.bits, t.fill, out, n_chunks);
+    pack_results<true><<<dim3(n_chunks), dim3(kPackThreads), 0, t.streams[0]>>>(p.src + first, here, t.bits, p.fill, out, n_chunks);
     const hipError_t e = hipGetLastError();
     return e != hipSuccess ? e : hipEventRecord(packed_[slot_of], t.streams[0]);
   }
@@ -1230,7 +1284,6 @@ class ResultStream {
     const size_t piece = t.staged ? t.piece_of[c / kBlock] : 0;
     const PackHeader* headers = t.staged ? (const PackHeader*)slot(piece) + (c - t.begins[piece]) : headers_ + c % t.ring_chunks;
     const uint8_t* bytes = t.staged ? slot(piece) + t.packed_at : ring_ + (c % t.ring_chunks) * t.chunk_bytes;
-    const bool streaming = t.n * sizeof(int32_t) > kDirectResultBytes;
     // Where a chunk's bytes are is read for all of them first, and only if it has to be: to wait for a header that has just
     // crossed the bus before every chunk cost 4 % of KHop's rows over R-MAT 20.
     size_t bytes_at[kChunksAtOnce];
@@ -1241,8 +1294,9 @@ class ResultStream {
         t.overflow.store(true, std::memory_order_relaxed);
         continue;
       }
-      const size_t first = (c + i) * kPackChunk;
-      unpack_chunk(headers[i], bytes + bytes_at[i], t.fill, t.dst + first, std::min<size_t>(kPackChunk, t.n - first), streaming);
+      const size_t part = t.part_of(c + i), first = (c + i - t.part_begin(part)) * kPackChunk;
+      const Part& p = t.parts[part];
+      unpack_chunk(headers[i], bytes + bytes_at[i], p.fill, p.dst + first, std::min<size_t>(kPackChunk, p.n - first), t.streaming);
     }
     unpack_fence();
     t.left[c / kBlock].fetch_sub(end - c, std::memory_order_release);
@@ -1298,13 +1352,13 @@ class ResultStream {
       // up to the end of what may be read, if that is known, else a piece at a time
       size_t end = std::min(t.chunks, t.sent + kMostChunks);
       if (!t.ready.empty()) {
-        if (!readable(words_to(t.sent + 1), /*waits=*/t.next.load() >= t.sent && gone == gentle, &error)) {
+        if (!readable(t.sent + 1, /*waits=*/t.next.load() >= t.sent && gone == gentle, &error)) {
           if (error == hipSuccess && !unpack_some()) spin_pause();
           continue;
         }
-        const size_t words = t.ready[t.happened - 1].words, whole = words == t.n ? t.chunks : words / kPackChunk;
-        end = std::min(whole, gently || t.chunks > t.ring_chunks ? t.sent + kMostChunks : t.chunks);
+        end = std::min(t.ready_chunks[t.happened - 1], gently || t.chunks > t.ring_chunks ? t.sent + kMostChunks : t.chunks);
       }
+      end = std::min(end, t.part_ends[t.part_of(t.sent)]);
       if (end > room || (gently && gentle - gone >= kGentleAhead)) {
         if (!unpack_some()) std::this_thread::yield();
         continue;
@@ -1321,10 +1375,10 @@ class ResultStream {
   hipError_t drive_staged() {
     Transfer& t = *transfer_;
     size_t launched = 0, sent = 0, here = 0;
-    while (here < t.pieces) {
+    while (here < t.pieces && !t.stop.load(std::memory_order_relaxed)) {
       hipError_t e = hipSuccess;
       bool moved = false;
-      if (launched < t.pieces && launched < sent + kPackedAhead && readable(words_to(t.begins[launched + 1]), /*waits=*/here == launched, &e) &&
+      if (launched < t.pieces && launched < sent + kPackedAhead && readable(t.begins[launched + 1], /*waits=*/here == launched, &e) &&
           slot_is_free(launched)) {
         if (!computed()) ahead_.fetch_add(1, std::memory_order_relaxed);
         e = launch_piece(launched++);

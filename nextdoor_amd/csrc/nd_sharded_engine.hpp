@@ -93,10 +93,14 @@ class ShardedEngine : public EngineBase {
     // A caller who took the last pass's rows, array and all, is expected to take this one's as well.  The pass does
     // without where that fails, whatever it is.
     parts_[0]->rows_ahead = nullptr;
-    if (parts_.size() == 1 && parts_[0]->is_walk() && rows_fetched_ && hFinalSamples.taken() &&
-        rows_ahead_.try_resize(hFinalSamples.size()))
+    parts_[0]->states_ahead = nullptr;
+    if (parts_.size() == 1 && rows_fetched_ && hFinalSamples.taken() && rows_ahead_.try_resize(hFinalSamples.size())) {
       parts_[0]->rows_ahead = rows_ahead_.data();
-    rows_fetched_ = false;
+      const size_t bytes = sample_state_bytes();
+      if (states_fetched_ && hSampleStates.taken() && bytes % sizeof(int32_t) == 0 && hSampleStates.try_resize(bytes))
+        parts_[0]->states_ahead = (int32_t*)hSampleStates.data();
+    }
+    rows_fetched_ = states_fetched_ = rows_changed_ = false;
     times = PhaseTimes();
     const auto t0 = std::chrono::steady_clock::now();
     std::vector<int> rc(parts_.size(), 0);
@@ -130,7 +134,8 @@ class ShardedEngine : public EngineBase {
 
   int fetch_final_samples() override {
     size_t at = 0;
-    rows_fetched_ = true;
+    rows_fetched_ = !rows_changed_;  // those of a pass whose rows are changed first are not expected as they are
+    rows_changed_ = false;
     const bool there = parts_.size() == 1 && parts_[0]->finish_rows_ahead();
     if (!rows_ahead_.empty()) {  // of a pass that sent its rows, or that did without
       hFinalSamples.swap(rows_ahead_);
@@ -147,6 +152,7 @@ class ShardedEngine : public EngineBase {
 
   int fetch_sample_states(void* dst, size_t bytes) override {
     if (bytes != sample_state_bytes() || bytes == 0) { last_error = "sample state size mismatch"; return -1; }
+    states_fetched_ = dst == hSampleStates.data();
     char* out = (char*)dst;
     for (size_t i = 0; i < parts_.size(); ++i) {
       const size_t n = parts_[i]->sample_state_bytes();
@@ -158,6 +164,7 @@ class ShardedEngine : public EngineBase {
 
   int distinct() override {
     hDistinctCounts.clear();
+    rows_changed_ = true;
     times.distinct = 0;
     for (size_t i = 0; i < parts_.size(); ++i) {
       const int rc = parts_[i]->distinct();
@@ -193,7 +200,7 @@ class ShardedEngine : public EngineBase {
   const char* name_;
   const CSR* graph_ = nullptr;
   HostArray<VertexID_t> rows_ahead_{host_pool};  // of a pass whose rows are on their way while it runs
-  bool rows_fetched_ = false;                    // since the last pass
+  bool rows_fetched_ = false, states_fetched_ = false, rows_changed_ = false;  // since the last pass
   std::vector<std::unique_ptr<Part>> parts_;
 };
 

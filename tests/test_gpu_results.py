@@ -234,3 +234,78 @@ def test_rows_that_are_stored_by_lines(oracle, app, kind, n, isolated_every):
             assert np.array_equal(s.final_samples(), want)
     finally:
         s.close()
+
+
+# rows enough for a quarter of the samples to be sampled first (96 MB), in the rows themselves and regrouped at the end
+@pytest.mark.parametrize("app,n", [("KHop", 92003), ("Layer", 97001)])
+def test_rows_of_hops_that_leave_before_the_pass_is_over(oracle, app, n):
+    g = graphs.random_graph(n=n, mean_degree=5, seed=n, isolated_every=7)
+    s = nd.Sampler(app, g, seed=42)
+    steps = [s.step_size(k) for k in range(s.steps)]
+    want, _ = oracle.sample_individual(graphs.oracle_view(g), oracle.app_desc(oracle.KHOP, 2, steps), 42, s.initial_contents)
+    counts = None
+    for turn in range(6):  # from the second pass on the rows are expected, but after one whose rows were made distinct first
+        print("n", n, "turn", turn, flush=True)
+        s.do_transit_parallel(load_balancing=turn % 2 == 0)
+        if turn == 3:
+            counts = s.distinct()  # with the rows as they were on their way
+            changed = s.final_samples()
+            assert changed.shape == want.shape and not np.array_equal(changed, want)
+            continue
+        rows = s.final_samples()
+        assert np.array_equal(rows, want)
+        del rows
+    assert np.array_equal(s.distinct(), counts)
+    s.do_sample_parallel()
+    assert np.array_equal(s.final_samples(), want)
+    s.do_transit_parallel()
+    s.close()  # with rows on their way
+
+
+# walks whose rows follow their one launch, and leave by range, with states; weighted walks with a state that travels
+@pytest.mark.parametrize("app,n", [("MultiRW4x6", 3001), ("MultiRW4x6", 90001), ("WeightedNode2Vec8", 300007)])
+def test_states_that_leave_with_the_rows(app, n):
+    g = graphs.random_graph(n=n, mean_degree=5, seed=n, isolated_every=7)
+    s = nd.Sampler(app, g, seed=42)
+    s.do_transit_parallel()
+    want, states = s.final_samples(), s.sample_states()  # fetched after the pass
+    for turn in range(8):
+        print("app", app, "n", n, "turn", turn, flush=True)
+        s.do_transit_parallel()
+        if turn == 2:
+            assert np.array_equal(s.sample_states(), states)  # asked for first
+            assert np.array_equal(s.final_samples(), want)
+        elif turn == 3:
+            assert np.array_equal(s.final_samples(), want)  # and not asked for
+        elif turn == 5:
+            continue  # nor the rows
+        else:
+            assert np.array_equal(s.final_samples(), want)
+            assert np.array_equal(s.sample_states(), states)
+    s.close()
+
+
+# lists that follow the pass, and that leave as they are written (64 MB of rows and columns)
+@pytest.mark.parametrize("n,degree", [(4004, 6), (60004, 24)])
+def test_edge_lists_that_leave_with_the_pass(n, degree):
+    g = graphs.random_graph(n=n, mean_degree=degree, seed=n, isolated_every=7)
+    s = nd.Sampler("MVS", g, seed=42)
+    s.do_transit_parallel()
+    want = s.adjacency()  # fetched after the pass
+    assert n < 5000 or want[0].nbytes + want[1].nbytes > 64 << 20
+    held = []
+    for turn in range(6):
+        print("n", n, "turn", turn, flush=True)
+        s.do_transit_parallel()
+        if turn == 1:
+            continue
+        if turn == 3:
+            assert s.final_samples().shape[0] == s.num_samples  # asked for while the lists are on their way
+        held.append(s.adjacency())
+        if turn == 4:
+            again = s.adjacency()
+            assert all(np.array_equal(a, b) for a, b in zip(want, again))
+    for lists in held:
+        assert all(np.array_equal(a, b) for a, b in zip(want, lists))
+    s.do_transit_parallel()
+    s.close()  # with lists on their way
