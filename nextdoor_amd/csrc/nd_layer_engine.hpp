@@ -508,6 +508,77 @@ struct Keeper {
   }
 };
 
+// The best `wanted` of a sample's keys (those each(f) hands to f, as for nth_smallest), and mostly a few more, in order: an edge
+// between counts of their upper bits first; where more are at or below it than there is room for (many equal keys), the
+// wanted ones are picked out exactly.  Returns how many; their vertices are in `ids`.  For a workgroup of kBinThreads; begins and ends
+// with a barrier.
+constexpr uint32_t kBestEntries = 2048;
+struct BestRoom {
+  uint64_t best[kBestEntries];
+  int32_t ids[kBestEntries];
+};
+struct BestScratch {
+  uint32_t counts[kBoundBins];
+  uint32_t wave_total[kBinWaves];
+  uint64_t last;
+  uint32_t through, n;
+  PickScratch pick;
+};
+template <class Each>
+__device__ __forceinline__ uint32_t best_in_order(Each each, uint32_t wanted, BestRoom& room, BestScratch& scratch) {
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  static_assert(kBoundBins == kBinThreads, "a lane per count");
+  scratch.counts[threadIdx.x] = 0;
+  if (threadIdx.x == 0) scratch.n = 0;
+  __syncthreads();
+  each([&](uint64_t value) { atomicAdd(&scratch.counts[bin_of_key((uint32_t)(value >> 32))], 1u); });
+  __syncthreads();
+  const uint32_t own = scratch.counts[threadIdx.x], through_wave = wave_inclusive_scan(own);
+  if (lane == 63) scratch.wave_total[wave] = through_wave;
+  __syncthreads();
+  uint32_t through = through_wave;
+  for (uint32_t w = 0; w < wave; ++w) through += scratch.wave_total[w];
+  if (threadIdx.x == kBinThreads - 1 && through < wanted) {  // all of them
+    scratch.last = ~0ull;
+    scratch.through = through;
+  }
+  if (through - own < wanted && through >= wanted) {  // else one lane
+    scratch.last = (uint64_t)last_key_of_bin(threadIdx.x) << 32 | 0xFFFFFFFFu;
+    scratch.through = through;
+  }
+  __syncthreads();
+  uint64_t last = scratch.last;
+  uint32_t n = scratch.through;
+  if (n > kBestEntries) {
+    last = nth_smallest(each, wanted, scratch.pick);
+    n = wanted;
+  }
+  each([&](uint64_t value) {
+    if (value <= last) room.best[atomicAdd(&scratch.n, 1u)] = value;
+  });
+  uint32_t padded = 64;
+  while (padded < n) padded *= 2u;
+  __syncthreads();
+  for (uint32_t i = n + threadIdx.x; i < padded; i += kBinThreads) room.best[i] = ~0ull;
+  __syncthreads();
+  for (uint32_t size = 2; size <= padded; size *= 2u) {
+    for (uint32_t stride = size / 2u; stride != 0; stride /= 2u) {
+      for (uint32_t i = threadIdx.x; i < padded / 2u; i += kBinThreads) {
+        const uint32_t a = (i / stride) * 2u * stride + i % stride, b = a + stride;
+        const uint64_t x = room.best[a], y = room.best[b];
+        if ((x > y) == ((a & size) == 0)) {
+          room.best[a] = y;
+          room.best[b] = x;
+        }
+      }
+      __syncthreads();
+    }
+  }
+  for (uint32_t i = threadIdx.x; i < n; i += kBinThreads) room.ids[i] = (int32_t)(uint32_t)room.best[i];
+  __syncthreads();
+  return n;
+}
+
 // A sample without hubs among its transits and with at most this many entries in a workgroup's stretches (a layer whose
 // transits are drawn uniformly) adds them all up at once, in an LDS table of twice as many slots.
 constexpr uint32_t kSparseGroupEntries = 2048;
@@ -835,37 +906,35 @@ __global__ __launch_bounds__(kSortOutThreads) void sort_out_ranked(CSRPartition 
   }
 }
 
-// A workgroup per sample: fetches the entries, sorts them by vertex, adds their terms up, forms the keys and sorts the
-// vertices by them (equal keys by vertex, as the sorts are stable).  Marked stretch by stretch, a layer of 1024 such samples
+// A workgroup per sample: fetches the pairs, adds their terms up in an LDS table hashed by vertex, forms the keys of the vertices
+// there and puts the best of them in order (equal keys by vertex).  Marked stretch by stretch, a layer of 1024 such samples
 // over 500 K vertices wrote and read 4 GB of keys, most of them absent.
+// Bound by round trips to LDS, of which one workgroup fills a compute unit.  806 samples of the first layer over 500 K vertices
+// 0.140 ms, 1024 over 114 K 0.084; by two sorts in LDS, of the pairs by vertex and of the vertices by key, and with the terms fetched
+// in the first one's order, 0.317 and 0.190.
 template <class Draw>
 __device__ __forceinline__ void ranked_layer(const MergedEdges& merged, uint32_t n_vertices, const int32_t* transits,
                                              uint32_t n_transits, int32_t invalid, uint32_t size, uint64_t sample,
-                                             uint32_t step, uint64_t seed, uint32_t* __restrict__ distinct_out, Draw draw) {
+                                             uint32_t step, uint64_t seed, uint32_t wanted, uint32_t* __restrict__ distinct_out,
+                                             Draw draw) {
   constexpr uint32_t kEach = kRankedEntries / kRankedThreads;
-  // two buffers of ids with one for the kept ids between them: next to whichever the sort leaves free it makes the sums' room
-  __shared__ __align__(16) uint32_t s_words[3 * kRankedEntries];
-  __shared__ uint16_t s_payload[2][kRankedEntries];
+  constexpr uint32_t kSlots = kRankedEntries + kRankedEntries / 2;  // at most two thirds of them are ever taken
+  constexpr uint32_t kNobody = 0xFFFFFFFFu;
+  __shared__ __align__(16) unsigned long long s_sum[kSlots];  // then key and vertex, all ones where there is none
+  __shared__ union { uint32_t vertex[kSlots]; BestRoom best; } s_table;
   __shared__ uint32_t s_start[kMaxLayerTransits];
   __shared__ EdgePos_t s_edge[kMaxLayerTransits];
-  __shared__ uint32_t s_count[kRankedThreads / 64][kSortedDigits];
-  __shared__ uint32_t s_wave_count[kRankedThreads / 64];
-  static_assert(kMaxLayerTransits <= kRankedThreads && kRankedEntries <= 65536, "a lane a transit; 16 bits an entry");
-  uint32_t* const kept = s_words + kRankedEntries;
+  __shared__ BestScratch s_scratch;
+  __shared__ uint32_t s_distinct;
+  static_assert(kMaxLayerTransits <= kRankedThreads && kRankedThreads == kBinThreads, "a lane a transit");
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-  auto before_wave = [&](uint32_t through, uint32_t* all) {  // exclusive prefix of a wavefront's total
-    if (lane == 63) s_wave_count[wave] = through;
-    __syncthreads();
-    uint32_t before = 0, total = 0;
-    for (uint32_t w = 0; w < kRankedThreads / 64; ++w) {
-      if (w < wave) before += s_wave_count[w];
-      total += s_wave_count[w];
-    }
-    __syncthreads();
-    *all = total;
-    return before;
-  };
-  uint32_t total;
+  const uint32_t slots = (size + size / 2u + 63u) & ~63u;  // of them in use: fewer to clear and to look through
+  static_assert(kSlots % 64 == 0, "as many as there are");
+  for (uint32_t i = threadIdx.x; i < slots; i += kRankedThreads) {
+    s_sum[i] = 0;
+    s_table.vertex[i] = kNobody;
+  }
+  if (threadIdx.x == 0) s_distinct = 0;
   {
     const int32_t t = threadIdx.x < n_transits ? transits[threadIdx.x] : -1;
     EdgePos_t begin = 0;
@@ -875,75 +944,63 @@ __device__ __forceinline__ void ranked_layer(const MergedEdges& merged, uint32_t
       degree = (uint32_t)(merged.row_ptr[t + 1] - begin);
     }
     const uint32_t through = wave_inclusive_scan(degree);
-    const uint32_t before = before_wave(through, &total);
+    if (lane == 63) s_scratch.wave_total[wave] = through;
+    __syncthreads();
+    uint32_t before = 0;
+    for (uint32_t w = 0; w < wave; ++w) before += s_scratch.wave_total[w];
     if (threadIdx.x < n_transits) {
       s_start[threadIdx.x] = before + through - degree;
       s_edge[threadIdx.x] = begin;
     }
     __syncthreads();
   }
-  auto edge_of = [&](uint32_t e) {
+  uint32_t id[kEach];
+  unsigned long long term[kEach];
+#pragma unroll
+  for (uint32_t k = 0; k < kEach; ++k) {
+    const uint32_t e = k * kRankedThreads + threadIdx.x;
+    id[k] = kNobody;
+    term[k] = 0;
+    if (e >= size) continue;
     uint32_t lo = 0, hi = n_transits;  // the last transit that starts at e or before (empty ones start where the next does)
     while (hi - lo > 1) {
       const uint32_t mid = lo + (hi - lo) / 2;
       if (s_start[mid] <= e) lo = mid; else hi = mid;
     }
-    return s_edge[lo] + (EdgePos_t)(e - s_start[lo]);
-  };
-  for (uint32_t e = threadIdx.x; e < size; e += kRankedThreads) {
-    s_words[e] = (uint32_t)merged.ids[edge_of(e)];
-    s_payload[0][e] = (uint16_t)e;
+    const EdgePos_t at = s_edge[lo] + (EdgePos_t)(e - s_start[lo]);
+    id[k] = (uint32_t)merged.ids[at];
+    term[k] = merged.terms[at];
   }
-  __syncthreads();
-  SortedIds sorted{s_words, s_words + 2 * kRankedEntries, s_payload[0], s_payload[1]};
-  sorted = sort_ids<kRankedThreads, true>(sorted, s_count, s_wave_count, size, 32u - (uint32_t)__clz((int)n_vertices));
-  // which of a lane's entries are a vertex's first, and how many vertices come before
-  unsigned long long* sums = (unsigned long long*)(sorted.other == s_words ? s_words : kept);
-  for (uint32_t i = threadIdx.x; i < kRankedEntries; i += kRankedThreads) sums[i] = 0;
-  uint32_t id[kEach], firsts = 0;
-  uint32_t last = threadIdx.x != 0 && threadIdx.x * kEach <= size ? sorted.ids[threadIdx.x * kEach - 1] : 0xFFFFFFFFu;
 #pragma unroll
   for (uint32_t k = 0; k < kEach; ++k) {
-    const uint32_t i = threadIdx.x * kEach + k;
-    id[k] = i < size ? sorted.ids[i] : 0xFFFFFFFFu;
-    if (i < size && id[k] != last) firsts |= 1u << k;
-    last = id[k];
-  }
-  const uint32_t through = wave_inclusive_scan((uint32_t)__popc(firsts));
-  uint32_t distinct;
-  const uint32_t rank0 = before_wave(through, &distinct) + through - (uint32_t)__popc(firsts);  // the sums are clear now
-#pragma unroll
-  for (uint32_t k = 0; k < kEach; ++k) {
-    const uint32_t i = threadIdx.x * kEach + k;
-    if (i >= size) continue;
-    const uint32_t rank = rank0 + (uint32_t)__popc(firsts & ((2u << k) - 1u)) - 1u;
-    atomicAdd(&sums[rank], merged.terms[edge_of(sorted.payload[i])]);
+    if (id[k] == kNobody) continue;
+    uint32_t slot = __umulhi(id[k] * 2654435761u, slots);
+    for (;;) {
+      const uint32_t before = atomicCAS(&s_table.vertex[slot], kNobody, id[k]);
+      if (before == kNobody || before == id[k]) break;
+      slot = slot + 1u == slots ? 0u : slot + 1u;
+    }
+    atomicAdd(&s_sum[slot], term[k]);
   }
   __syncthreads();
-  uint32_t key[kEach];
-#pragma unroll
-  for (uint32_t k = 0; k < kEach; ++k) {
-    key[k] = 0;
-    if (firsts >> k & 1u)
-      key[k] = ladies_key_bits(sums[rank0 + (uint32_t)__popc(firsts & ((1u << k) - 1u))], ladies_pair_index(sample, n_vertices, id[k]),
-                               step, seed);
+  uint32_t distinct = 0;  // of the wavefront
+  for (uint32_t i = threadIdx.x; i < slots; i += kRankedThreads) {  // whole wavefronts
+    const uint32_t v = s_table.vertex[i];
+    distinct += (uint32_t)__popcll(__ballot(v != kNobody));
+    unsigned long long value = ~0ull;
+    if (v != kNobody) value = rank_value(make_uint2(ladies_key_bits(s_sum[i], ladies_pair_index(sample, n_vertices, v), step, seed), v));
+    s_sum[i] = value;
   }
-  __syncthreads();
-#pragma unroll
-  for (uint32_t k = 0; k < kEach; ++k) {
-    if (!(firsts >> k & 1u)) continue;
-    const uint32_t rank = rank0 + (uint32_t)__popc(firsts & ((1u << k) - 1u));
-    s_words[rank] = key[k];
-    kept[rank] = id[k];
-    s_payload[0][rank] = (uint16_t)rank;
-  }
-  __syncthreads();
-  sorted = SortedIds{s_words, s_words + 2 * kRankedEntries, s_payload[0], s_payload[1]};
-  sorted = sort_ids<kRankedThreads, true>(sorted, s_count, s_wave_count, distinct, 32);
-  for (uint32_t i = threadIdx.x; i < distinct; i += kRankedThreads) sorted.other[i] = kept[sorted.payload[i]];
-  __syncthreads();
-  if (threadIdx.x == 0) *distinct_out = distinct;
-  draw((const CSR::Edge*)sorted.other, distinct);
+  if (lane == 0 && distinct != 0) atomicAdd(&s_distinct, distinct);
+  // (the barrier it begins with: nobody needs s_table.vertex any more)
+  const uint32_t n = best_in_order(
+      [&](auto f) {
+        for (uint32_t i = threadIdx.x; i < slots; i += kRankedThreads)
+          if (s_sum[i] != ~0ull) f(s_sum[i]);
+      },
+      wanted, s_table.best, s_scratch);
+  if (threadIdx.x == 0) *distinct_out = s_distinct;
+  draw((const CSR::Edge*)s_table.best.ids, n);
 }
 
 // item_count[s] = work items of sample s (at least one, so that row offsets get written)
@@ -1042,33 +1099,24 @@ __global__ __launch_bounds__(kRankedThreads) void ranked_layer_kernel(LayerParam
   const uint32_t ls = blockIdx.x, size = merged_sizes[ls];
   if (size > kRankedEntries) return;
   ranked_layer(merged, (uint32_t)P.csr.n_vertices, P.transits.base + (size_t)ls * P.transits.stride, P.transits.count, P.invalid,
-               size, P.first_sample + P.sample_begin + ls, (uint32_t)P.step, P.seed, distinct + ls,
-               [&](const CSR::Edge* ranked, uint32_t n_distinct) {
-                 const uint32_t n_first = n_distinct < P.step_size ? n_distinct : P.step_size;
+               size, P.first_sample + P.sample_begin + ls, (uint32_t)P.step, P.seed, P.step_size, distinct + ls,
+               [&](const CSR::Edge* ranked, uint32_t n) {
+                 const uint32_t n_first = n < P.step_size ? n : P.step_size;
                  for (uint32_t nbr = threadIdx.x; nbr < P.step_size; nbr += kRankedThreads)
                    draw_from<SampleType, App>(P, ls, nbr, ranked, n_first);
                });
 }
 
 // A workgroup per marked sample: the best of what the workgroups of collective_mark_binned have kept of it, in order, and the
-// draws.  An edge between counts first, as there, over all of them together; where more are at or below it than there is room
-// for (many equal keys), the wanted ones are picked out exactly.  1024 samples of 512, five workgroups' keys each (500 K
-// vertices): 0.044 ms; 27 workgroups' (3.07 M vertices): 0.08.
-constexpr uint32_t kBestEntries = 2048;
+// draws.  1024 samples of 512, five workgroups' keys each (500 K vertices): 0.044 ms; 27 workgroups' (3.07 M vertices): 0.08.
 template <class SampleType, class App>
 __global__ __launch_bounds__(kBinThreads) void kept_layer_kernel(LayerParams P, const uint32_t* __restrict__ n_marked,
                                                                  const uint32_t* __restrict__ marked, uint32_t groups,
                                                                  KeptKeys in) {
-  __shared__ uint64_t s_best[kBestEntries];
-  __shared__ int32_t s_ids[kBestEntries];
-  __shared__ uint32_t s_counts[kBoundBins];
-  __shared__ uint32_t s_wave_total[kBinWaves];
-  __shared__ uint64_t s_last;
-  __shared__ uint32_t s_through, s_n;
-  __shared__ PickScratch s_pick;
+  __shared__ BestRoom s_best;
+  __shared__ BestScratch s_scratch;
   const uint32_t at = blockIdx.x;
   if (at >= *n_marked) return;
-  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
   const uint32_t bound = in.bound[at];
   auto each = [&](auto f) {
     for (uint32_t g = 0; g < groups; ++g) {
@@ -1080,55 +1128,8 @@ __global__ __launch_bounds__(kBinThreads) void kept_layer_kernel(LayerParams P, 
       }
     }
   };
-  s_counts[threadIdx.x] = 0;
-  if (threadIdx.x == 0) s_n = 0;
-  __syncthreads();
-  each([&](uint64_t value) { atomicAdd(&s_counts[bin_of_key((uint32_t)(value >> 32))], 1u); });
-  __syncthreads();
-  const uint32_t own = s_counts[threadIdx.x], through_wave = wave_inclusive_scan(own);
-  if (lane == 63) s_wave_total[wave] = through_wave;
-  __syncthreads();
-  uint32_t through = through_wave;
-  for (uint32_t w = 0; w < wave; ++w) through += s_wave_total[w];
-  if (threadIdx.x == kBinThreads - 1 && through < in.wanted) {  // all of them
-    s_last = ~0ull;
-    s_through = through;
-  }
-  if (through - own < in.wanted && through >= in.wanted) {  // else one lane
-    s_last = (uint64_t)last_key_of_bin(threadIdx.x) << 32 | 0xFFFFFFFFu;
-    s_through = through;
-  }
-  __syncthreads();
-  uint64_t last = s_last;
-  uint32_t n = s_through;
-  if (n > kBestEntries) {
-    last = nth_smallest(each, in.wanted, s_pick);
-    n = in.wanted;
-  }
-  each([&](uint64_t value) {
-    if (value <= last) s_best[atomicAdd(&s_n, 1u)] = value;
-  });
-  uint32_t padded = 64;
-  while (padded < n) padded *= 2u;
-  __syncthreads();
-  for (uint32_t i = n + threadIdx.x; i < padded; i += kBinThreads) s_best[i] = ~0ull;
-  __syncthreads();
-  for (uint32_t size = 2; size <= padded; size *= 2u) {
-    for (uint32_t stride = size / 2u; stride != 0; stride /= 2u) {
-      for (uint32_t i = threadIdx.x; i < padded / 2u; i += kBinThreads) {
-        const uint32_t a = (i / stride) * 2u * stride + i % stride, b = a + stride;
-        const uint64_t x = s_best[a], y = s_best[b];
-        if ((x > y) == ((a & size) == 0)) {
-          s_best[a] = y;
-          s_best[b] = x;
-        }
-      }
-      __syncthreads();
-    }
-  }
-  for (uint32_t i = threadIdx.x; i < n; i += kBinThreads) s_ids[i] = (int32_t)(uint32_t)s_best[i];
-  __syncthreads();
-  const CSR::Edge* ranked = (const CSR::Edge*)s_ids;
+  const uint32_t n = best_in_order(each, in.wanted, s_best, s_scratch);
+  const CSR::Edge* ranked = (const CSR::Edge*)s_best.ids;
   // (how many more there are here depends on what the workgroups knew of each other's bounds)
   const uint32_t n_first = n < P.step_size ? n : P.step_size;
   for (uint32_t nbr = threadIdx.x; nbr < P.step_size; nbr += kBinThreads) draw_from<SampleType, App>(P, marked[at], nbr, ranked, n_first);

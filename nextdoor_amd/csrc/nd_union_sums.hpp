@@ -392,27 +392,20 @@ struct SortedByDegreeSquared {
   }
 };
 
-// The n ids at `at.ids` in ascending order, equal ones as they were, by passes over 7 bits, least significant first; the
-// result is where the returned `ids` points.  A wavefront takes a stretch of the ids, 64 at a time: lanes with equal digits find each other by
+// The n ids at `ids` in ascending order, by passes over 7 bits, least significant first; returns where they are, there or in `other`.  A wavefront takes a stretch of the ids, 64 at a time: lanes with equal digits find each other by
 // ballots, and what came before them is in the wavefront's counters.  (A bitonic sort, 78 stages of LDS reads and writes for
 // 4096 ids, took 0.36 ms for the 4096 samples of R-MAT 20's first layer.)
-// With a payload, 16 bits go where the ids go.
 constexpr uint32_t kSortedDigitBits = 7, kSortedDigits = 1u << kSortedDigitBits;
-struct SortedIds {
-  uint32_t *ids, *other;
-  uint16_t *payload, *other_payload;
-};
-template <uint32_t kThreads, bool kPayload>
-__device__ __forceinline__ SortedIds sort_ids(SortedIds at, uint32_t (*s_count)[kSortedDigits], uint32_t* s_wave_count,
-                                              uint32_t n, uint32_t bits) {
-  constexpr uint32_t kWaves = kThreads / 64;
+__device__ __forceinline__ uint32_t* sort_ids(uint32_t* ids, uint32_t* other, uint32_t (*s_count)[kSortedDigits],
+                                              uint32_t* s_wave_count, uint32_t n, uint32_t bits) {
+  constexpr uint32_t kThreads = kSortedThreads, kWaves = kSortedWaves;
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
   const uint32_t stretch = ((n + kWaves - 1) / kWaves + 63u) & ~63u;
   const uint32_t begin = wave * stretch, end = begin + stretch < n ? begin + stretch : n;
   for (uint32_t shift = 0; shift < bits; shift += kSortedDigitBits) {
     for (uint32_t i = threadIdx.x; i < kWaves * kSortedDigits; i += kThreads) (&s_count[0][0])[i] = 0;
     __syncthreads();
-    for (uint32_t i = begin + lane; i < end; i += 64u) atomicAdd(&s_count[wave][at.ids[i] >> shift & (kSortedDigits - 1u)], 1u);
+    for (uint32_t i = begin + lane; i < end; i += 64u) atomicAdd(&s_count[wave][ids[i] >> shift & (kSortedDigits - 1u)], 1u);
     __syncthreads();
     // starts: by digit, then by wavefront; lane t has two counters that follow each other in that order
     const uint32_t digit = threadIdx.x / (kWaves / 2u), of = threadIdx.x % (kWaves / 2u) * 2u;
@@ -427,7 +420,7 @@ __device__ __forceinline__ SortedIds sort_ids(SortedIds at, uint32_t (*s_count)[
     __syncthreads();
     for (uint32_t i0 = begin; i0 < end; i0 += 64u) {
       const bool here = i0 + lane < end;
-      const uint32_t id = here ? at.ids[i0 + lane] : 0u, d = id >> shift & (kSortedDigits - 1u);
+      const uint32_t id = here ? ids[i0 + lane] : 0u, d = id >> shift & (kSortedDigits - 1u);
       uint64_t same = __ballot(here);
 #pragma unroll
       for (uint32_t bit = 0; bit < kSortedDigitBits; ++bit) {
@@ -438,16 +431,17 @@ __device__ __forceinline__ SortedIds sort_ids(SortedIds at, uint32_t (*s_count)[
       if (here) {
         const uint32_t rank = (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
         const uint32_t to = s_count[wave][d] + rank;
-        at.other[to] = id;
-        if (kPayload) at.other_payload[to] = at.payload[i0 + lane];
+        other[to] = id;
         if (rank == 0) s_count[wave][d] = to + (uint32_t)__popcll(same);
       }
       __builtin_amdgcn_wave_barrier();
     }
     __syncthreads();
-    at = SortedIds{at.other, at.ids, at.other_payload, at.payload};
+    uint32_t* const sorted = other;
+    other = ids;
+    ids = sorted;
   }
-  return at;
+  return ids;
 }
 
 // A workgroup per sample: fetches the entries, sorts them, adds degree^2 up over the distinct ones and draws.
@@ -496,8 +490,7 @@ __device__ __forceinline__ void sorted_layer(const CSRPartition& csr, const int3
     s_buffers[0][e] = (uint32_t)csr.edges[s_edge[lo] + (EdgePos_t)(e - s_start[lo])];
   }
   __syncthreads();
-  uint32_t* s_ids = sort_ids<kSortedThreads, false>(SortedIds{s_buffers[0], s_buffers[1], nullptr, nullptr}, s_count, s_wave_count,
-                                                    size, 32u - (uint32_t)__clz(csr.n_vertices)).ids;
+  uint32_t* s_ids = sort_ids(s_buffers[0], s_buffers[1], s_count, s_wave_count, size, 32u - (uint32_t)__clz(csr.n_vertices));
   const uint32_t chunks = size ? (size + kSortedChunk - 1) / kSortedChunk : 1u;
   if (size + threadIdx.x < chunks * kSortedChunk) s_ids[size + threadIdx.x] = 0xFFFFFFFFu;
   __syncthreads();

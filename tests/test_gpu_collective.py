@@ -292,3 +292,26 @@ def test_neighbourhoods_that_are_too_long_are_worked_on_by_nobody():
     assert os.path.exists(LONG_NEIGHBOURHOOD_PROBE), "tests/cpp/long_neighbourhood_probe is built by __graft_entry__.build()"
     out = subprocess.run([LONG_NEIGHBOURHOOD_PROBE], capture_output=True, text=True, timeout=100)
     assert out.returncode == 0 and out.stdout.endswith("all as they should be\n"), out.stdout[-300:] + out.stderr[-300:]
+
+
+# eight transits of this many neighbours each: up to 8192 pairs are ranked in LDS, whose table is fullest then
+@pytest.mark.parametrize("degree", [1, 8, 9, 257, 1023, 1024, 1025])
+@pytest.mark.parametrize("weights", ["random", "equal_keys", "few_vertices"])
+def test_ladies_neighbourhoods_at_the_edge_of_what_is_ranked_in_lds(oracle, degree, weights):
+    """All neighbours different; nearly all keys equal (more than there is room for in order); and many pairs on few vertices."""
+    n = 9001
+    rng = np.random.default_rng(degree)
+    v = np.repeat(np.arange(n), degree)
+    i = np.tile(np.arange(degree), n)
+    dst = (v * 1024 + i * (7 if weights == "few_vertices" else 1)) % (1100 if weights == "few_vertices" else n)
+    w = (rng.random(len(v)) * 4 + 1).astype(np.float32)
+    if weights == "equal_keys":
+        w[i != 0] = 1e-9  # the terms of all but one are below 2^-53
+    g = nd.Graph.from_edges(v, dst, w, n_vertices=n)
+    s = nd.Sampler("LADIESImportance2x8", g, seed=SEED)
+    want = oracle.sample_ladies_importance(graphs.oracle_view(g), layer_desc(oracle, s, oracle.LADIES_IMPORTANCE), SEED,
+                                           s.initial_contents)
+    for _ in range(2):
+        s.do_transit_parallel(True)
+        assert np.array_equal(s.final_samples(), want)
+    s.close()
