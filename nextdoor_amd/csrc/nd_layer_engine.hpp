@@ -1327,6 +1327,10 @@ class LayerEngine : public EngineBase {
       ND_HIP_TRY(hipMemcpyAsync(d_samples_, d_samples_init_, sizeof(SampleType) * (size_t)n_samples_,
                                 hipMemcpyDeviceToDevice, stream_));
     }
+    drop_rows_ahead();  // nobody asked for them
+    // a caller who took the last pass's rows, array and all, is expected to take this one's as well
+    const bool rows_expected = rows_fetched_ && hFinalSamples.taken() && !profiling;
+    rows_fetched_ = false;
     ND_HIP_TRY(hipStreamSynchronize(stream_));
     ND_HIP_TRY(hipEventRecord(ev_begin_, stream_));
     const uint32_t S = (uint32_t)n_samples_;
@@ -1376,15 +1380,26 @@ class LayerEngine : public EngineBase {
       }
     }
     ND_HIP_TRY(hipEventRecord(ev_end_, stream_));
-    ND_HIP_TRY(hipStreamSynchronize(stream_));
+    if (rows_expected) send_rows();
+    ND_HIP_TRY(hipEventSynchronize(ev_end_));
     ND_HIP_TRY(hipEventElapsedTime(&times.end_to_end, ev_begin_, ev_end_));
-    if (h_too_long_ && *h_too_long_) { last_error = kTooLong; return -2; }
+    if (h_too_long_ && *h_too_long_) {
+      drop_rows_ahead();
+      last_error = kTooLong;
+      return -2;
+    }
     counted_ = apps::neighborhood_form_of<App>::value == apps::kConcatenated;
     return 0;
   }
 
   int fetch_final_samples() override {
     if (!allocated_) { last_error = "no device data"; return -1; }
+    rows_fetched_ = true;
+    settle_rows_ahead();
+    if (rows_ahead_) {
+      rows_ahead_ = false;
+      return 0;
+    }
     hFinalSamples.resize((size_t)n_samples_ * (size_t)final_sample_size());
     return fetch_to_host(hFinalSamples.data(), d_final_, sizeof(VertexID_t) * hFinalSamples.size(), (uint32_t)max_bits(),
                          invalid_, stream_);
@@ -1393,6 +1408,7 @@ class LayerEngine : public EngineBase {
   int fetch_sample_states(void* dst, size_t bytes) override {
     if (!allocated_ || std::is_empty<SampleType>::value) { last_error = "no sample state"; return -1; }
     if (bytes != sample_state_bytes()) { last_error = "sample state size mismatch"; return -1; }
+    settle_rows_ahead();
     return states_to_host(dst, d_samples_, bytes, stream_);
   }
 
@@ -1773,7 +1789,29 @@ class LayerEngine : public EngineBase {
     bitmap_samples_ = 0;
   }
 
+  // The rows of the pass that is enqueued, directly behind it; fetched when they are asked for if they cannot be sent now.
+  void send_rows() {
+    try {
+      hFinalSamples.resize((size_t)n_samples_ * (size_t)final_sample_size());
+      rows_ahead_ = result_stream->begin(d_final_, hFinalSamples.size(), (uint32_t)max_bits(), invalid_, hFinalSamples.data(),
+                                         stream_, {}, ev_end_) == hipSuccess;
+    } catch (const std::bad_alloc&) {
+      rows_ahead_ = false;
+    }
+    if (!rows_ahead_) (void)hipGetLastError();
+  }
+  // The result stream carries one transfer at a time: rows on their way are waited for where it is known whose they are.
+  void settle_rows_ahead() {
+    if (rows_ahead_ && result_stream->finish() != hipSuccess) rows_ahead_ = false;
+  }
+  void drop_rows_ahead() {
+    if (rows_ahead_) result_stream->abandon();
+    rows_ahead_ = false;
+  }
+
   void free_run_buffers() {
+    drop_rows_ahead();
+    rows_fetched_ = false;
     release(d_initial_); release(d_samples_); release(d_samples_init_); release(d_final_);
     release(d_sizes_); release(d_offsets_); release(d_row_offsets_); release(d_small_scratch_);
     release(d_item_count_); release(d_item_start_);
@@ -1808,6 +1846,8 @@ class LayerEngine : public EngineBase {
   int32_t invalid_ = 0;
   int max_bits_ = 0;
   uint64_t seed_ = 0;
+  bool rows_fetched_ = false;  // since the last pass
+  bool rows_ahead_ = false;    // rows are on their way to hFinalSamples
   bool allocated_ = false;
   size_t capacity_ = 0;
   uint32_t bitmap_words_ = 0;          // 32-bit words of one sample's presence map (a multiple of kBitmapTileWords)

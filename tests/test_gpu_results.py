@@ -309,3 +309,20 @@ def test_edge_lists_that_leave_with_the_pass(n, degree):
         assert all(np.array_equal(a, b) for a, b in zip(want, lists))
     s.do_transit_parallel()
     s.close()  # with lists on their way
+
+
+@pytest.mark.parametrize("app", ["FastGCNImportance3x16", "LADIESImportance3x16"])
+def test_layer_rows_that_follow_the_pass(app):
+    s = nd.Sampler(app, graphs.random_graph(n=4000, mean_degree=9, seed=5, isolated_every=7, hub=3), seed=42)
+    s.do_transit_parallel()
+    want = s.final_samples()  # fetched after the pass
+    for turn in range(6):
+        s.do_transit_parallel()
+        if turn == 2:
+            continue  # nobody asks
+        got = s.final_samples()
+        assert np.array_equal(got, want)
+        if turn == 4:
+            assert np.array_equal(s.final_samples(), want)
+    s.do_transit_parallel()
+    s.close()  # with rows on their way
