@@ -1140,14 +1140,14 @@ template <class SampleType, class App>
 __global__ __launch_bounds__(256) void marked_layer_kernel(LayerParams P, MarkedSamples marked,
                                                            const uint32_t* __restrict__ distinct,
                                                            const uint32_t* __restrict__ bitmap, uint32_t words_per_sample,
-                                                           const uint64_t* __restrict__ part_before,
-                                                           const uint64_t* __restrict__ group_through, uint32_t parts) {
+                                                           const uint64_t* __restrict__ half_before,
+                                                           const uint64_t* __restrict__ group_through, uint32_t halves) {
   const uint64_t draws = (uint64_t)*marked.count * P.step_size;
   for (uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x; i < draws; i += gridDim.x * 256ull) {
     const uint32_t at = (uint32_t)(i / P.step_size), nbr = (uint32_t)(i - (uint64_t)at * P.step_size);
     const uint32_t ls = marked.sample[at];
-    MarkedByDegreeSquared mine{bitmap + (size_t)at * words_per_sample, part_before + (size_t)at * (parts + 1),
-                               group_through + (size_t)at * parts * kGroupsPerPart, P.csr.row_ptr, parts};
+    MarkedByDegreeSquared mine{bitmap + (size_t)at * words_per_sample, half_before + (size_t)at * (halves + 1),
+                               group_through + (size_t)at * halves * kGroupsPerHalf, P.csr.row_ptr, halves};
     draw_from<SampleType, App>(P, ls, nbr, mine, distinct[ls]);
   }
 }
@@ -1695,14 +1695,13 @@ class LayerEngine : public EngineBase {
 
   // kDistinctByDegreeSquared: the samples of the chunk by the size of their neighbourhoods, and their draws.
   int run_by_degree(const LayerParams& P, int step) {
-    const uint32_t n = P.chunk_samples, parts = union_.parts;
-    const size_t n_parts = (size_t)n * parts;
+    const uint32_t n = P.chunk_samples, parts = union_.parts, halves = parts * kHalvesOfPart;
     if (n > bitmap_samples_) {
-      release(d_bitmap_); release(d_group_through_); release(d_part_total_); release(d_part_before_);
+      release(d_bitmap_); release(d_group_through_); release(d_half_total_); release(d_half_before_);
       ND_HIP_TRY(hipMalloc(&d_bitmap_, sizeof(uint32_t) * (size_t)n * bitmap_words_));
-      ND_HIP_TRY(hipMalloc(&d_group_through_, sizeof(uint64_t) * n_parts * kGroupsPerPart));
-      ND_HIP_TRY(hipMalloc(&d_part_total_, sizeof(uint64_t) * n_parts));
-      ND_HIP_TRY(hipMalloc(&d_part_before_, sizeof(uint64_t) * (size_t)n * (parts + 1)));
+      ND_HIP_TRY(hipMalloc(&d_group_through_, sizeof(uint64_t) * (size_t)n * parts * kGroupsPerPart));
+      ND_HIP_TRY(hipMalloc(&d_half_total_, sizeof(uint64_t) * (size_t)n * halves));
+      ND_HIP_TRY(hipMalloc(&d_half_before_, sizeof(uint64_t) * (size_t)n * (halves + 1)));
       bitmap_samples_ = n;
     }
     const size_t S = (size_t)n_samples_;
@@ -1716,12 +1715,12 @@ class LayerEngine : public EngineBase {
     const uint32_t turns = (parts + kXcdCount - 1) / kXcdCount * kUnionSlices;
     union_parts<<<dim3(turns * kXcdCount), dim3(kUnionThreads), 0, stream_>>>(P.csr, union_.hubs, parts, marked_, bitmap_words_,
                                                                               d_bitmap_);
-    union_sums<<<dim3(parts * kSumSlices), dim3(kSumThreads), 0, stream_>>>(
-        union_.squares, union_.square_rows, parts, marked_, bitmap_words_, d_bitmap_, d_group_through_, d_part_total_, distinct);
+    union_sums<<<dim3(halves * kSumSlices), dim3(kSumThreads), 0, stream_>>>(
+        union_.squares, union_.square_rows, halves, marked_, bitmap_words_, d_bitmap_, d_group_through_, d_half_total_, distinct);
     tock();
-    sample_part_sums<<<dim3(n), dim3(64), 0, stream_>>>(d_part_total_, parts, marked_.count, d_part_before_);
+    sample_half_sums<<<dim3(n), dim3(64), 0, stream_>>>(d_half_total_, halves, marked_.count, d_half_before_);
     marked_layer_kernel<SampleType, App><<<dim3(kDrawBlocks), dim3(256), 0, stream_>>>(
-        P, marked_, distinct, d_bitmap_, bitmap_words_, d_part_before_, d_group_through_, parts);
+        P, marked_, distinct, d_bitmap_, bitmap_words_, d_half_before_, d_group_through_, halves);
     ND_HIP_TRY(hipGetLastError());
     return 0;
   }
@@ -1784,7 +1783,7 @@ class LayerEngine : public EngineBase {
   void release_neighborhood_buffers() {
     release(d_nbr_cols_); release(d_nbr_weights_);
     release(d_bitmap_); release(d_kept_); release(d_n_kept_); release(d_bound_);
-    release(d_group_through_); release(d_part_total_); release(d_part_before_);
+    release(d_group_through_); release(d_half_total_); release(d_half_before_);
     capacity_ = 0;
     bitmap_samples_ = 0;
   }
@@ -1882,7 +1881,7 @@ class LayerEngine : public EngineBase {
   int32_t* d_nbr_cols_ = nullptr;
   float* d_nbr_weights_ = nullptr;
   // FastGCN form: degree^2 of the marked vertices, by group inside a part, by part, by sample
-  uint64_t *d_group_through_ = nullptr, *d_part_total_ = nullptr, *d_part_before_ = nullptr;
+  uint64_t *d_group_through_ = nullptr, *d_half_total_ = nullptr, *d_half_before_ = nullptr;
   UnionTables union_;                  // of the graph
   MarkedSamples marked_{};
   uint32_t* d_layer_counts_ = nullptr;  // entries of every layer and sample's neighbourhood, then its distinct vertices

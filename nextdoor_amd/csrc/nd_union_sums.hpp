@@ -536,11 +536,14 @@ __device__ __forceinline__ void sorted_layer(const CSRPartition& csr, const int3
 constexpr uint32_t kXcdCount = 8;
 constexpr uint32_t kUnionThreads = 256, kUnionWaves = kUnionThreads / 64;
 constexpr uint32_t kUnionSlices = 256;                   // workgroups that share the samples of a part
-constexpr uint32_t kSumThreads = 1024, kSumWaves = kSumThreads / 64;
+// degree^2 is summed over halves of parts, so that two workgroups are on a compute unit and one works while the other waits at a barrier.
+constexpr uint32_t kHalvesOfPart = 2, kGroupsPerHalf = kGroupsPerPart / kHalvesOfPart, kHalfWords = kPartWords / kHalvesOfPart;
+constexpr uint32_t kSumThreads = 512, kSumWaves = kSumThreads / 64;
 constexpr uint32_t kSumSamples = 16;                     // the columns of a matrix product
-constexpr uint32_t kSumGroups = kGroupsPerPart / kSumWaves;  // of a wavefront
-constexpr uint32_t kSumPitch = kPartWords + 8;           // words between samples in LDS: spreads them over the banks
-constexpr uint32_t kSumSlices = 16;                      // workgroups that share the samples of a part
+constexpr uint32_t kSumGroups = kGroupsPerHalf / kSumWaves;  // of a wavefront
+constexpr uint32_t kSumPitch = kHalfWords + 8;           // words between samples in LDS: spreads them over the banks
+constexpr uint32_t kSumSlices = 16;                      // workgroups that share the samples of a half
+static_assert(kSumSamples == 2 * kSumWaves && kHalfWords == 4 * 64 && kGroupsPerHalf == 32, "two samples a wavefront");
 
 typedef int32_t IntVector4 __attribute__((ext_vector_type(4)));
 
@@ -683,25 +686,27 @@ __global__ __launch_bounds__(kUnionThreads, 6) void union_parts(CSRPartition csr
   }
 }
 
-// degree^2 over the bits: a workgroup has one part, a wavefront four of its 64 groups, whose operands stay in its registers
+// degree^2 over the bits: a workgroup has half of a part, a wavefront four of its 32 groups, whose operands stay in its registers
 // while the samples go past them, 16 at a time.
-//   group_through[(at * parts + part) * 64 + g]          degree^2 of the marked vertices of groups 0..g of the part
-//   part_total[at * parts + part]                        of the whole part
+//   group_through[(at * halves + half) * 32 + g]         degree^2 of the marked vertices of groups 0..g of the half
+//   half_total[at * halves + half]                       of the whole half
 //   distinct[sample] += marked vertices
-// Bound by reading the bits once (0.5 GB a layer of R-MAT 20's 4096 samples).
+// Bound by instructions (taking the bits apart is half of them) and the two barriers of a block of samples: second layer of 4096
+// samples over R-MAT 20 (0.5 GB of bits) 0.196 ms, over 0.9 M vertices 0.182; with a whole part a workgroup of 1024, one to a
+// compute unit, 0.244 and 0.243.
 __global__ __launch_bounds__(kSumThreads, 4) void union_sums(const uint32_t* __restrict__ squares, uint32_t square_rows,
-                                                             uint32_t parts, MarkedSamples marked,
+                                                             uint32_t halves, MarkedSamples marked,
                                                              uint32_t words_per_sample,
                                                              const uint32_t* __restrict__ bitmap,
                                                              uint64_t* __restrict__ group_through,
-                                                             uint64_t* __restrict__ part_total,
+                                                             uint64_t* __restrict__ half_total,
                                                              uint32_t* __restrict__ distinct) {
   __shared__ __align__(16) uint32_t s_bits[2][kSumSamples * kSumPitch];
-  __shared__ uint64_t s_sums[2][2][kSumSamples * (kGroupsPerPart + 1)];
-  __shared__ uint32_t s_top[2][kSumSamples * (kGroupsPerPart + 1)];
+  __shared__ uint64_t s_sums[2][2][kSumSamples * (kGroupsPerHalf + 1)];
+  __shared__ uint32_t s_top[2][kSumSamples * (kGroupsPerHalf + 1)];
   __shared__ uint32_t s_marked[2][kSumSamples];
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-  const uint32_t part = blockIdx.x / kSumSlices, slice = blockIdx.x % kSumSlices;
+  const uint32_t half = blockIdx.x / kSumSlices, slice = blockIdx.x % kSumSlices;
   const uint32_t n = *marked.count;
   const uint32_t blocks = (n + kSumSamples - 1) / kSumSamples;
   const uint32_t column = lane & 15u, q = lane >> 4;
@@ -713,32 +718,31 @@ __global__ __launch_bounds__(kSumThreads, 4) void union_sums(const uint32_t* __r
       limbs[g][k] = IntVector4{0, 0, 0, 0};
       if (column < square_rows && slice < blocks)
         limbs[g][k] = *((const IntVector4*)squares +
-                        ((size_t)(part * kGroupsPerPart + wave * kSumGroups + g) * 16u + 4u * k + q) * square_rows + column);
+                        ((size_t)(half * kGroupsPerHalf + wave * kSumGroups + g) * 16u + 4u * k + q) * square_rows + column);
     }
   if (threadIdx.x < 2 * kSumSamples) (&s_marked[0][0])[threadIdx.x] = 0;
   __syncthreads();
-  // A wavefront brings the 2 KB of one sample into LDS; those of the next two blocks are on their way while one is worked
-  // on (one: 0.24 ms, 3.8 us a block).
-  const uint4* lines = (const uint4*)(bitmap + (size_t)part * kPartWords) + 2u * lane;
+  // A wavefront brings the bits of two samples into LDS, 1 KB each; those of the next two blocks are on their way while one is worked
+  // on.
+  const uint4* lines = (const uint4*)(bitmap + (size_t)half * kHalfWords) + lane;
   const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
-  uint4 low[2] = {zero, zero}, high[2] = {zero, zero};
-  auto fetch = [&](uint32_t block, uint4& l, uint4& h) {
-    const uint32_t at = block * kSumSamples + wave;
-    if (at >= n) return;  // what the lane had is no less of a sample: nobody reads its sums
-    l = lines[(size_t)at * (words_per_sample / 4u)];
-    h = lines[(size_t)at * (words_per_sample / 4u) + 1u];
+  uint4 one[2] = {zero, zero}, two[2] = {zero, zero};
+  auto fetch = [&](uint32_t block, uint4& a, uint4& b) {
+    const uint32_t at = block * kSumSamples + 2u * wave;
+    // what the lane had is no less of a sample: nobody reads its sums
+    if (at < n) a = lines[(size_t)at * (words_per_sample / 4u)];
+    if (at + 1u < n) b = lines[(size_t)(at + 1u) * (words_per_sample / 4u)];
   };
-  fetch(slice, low[0], high[0]);
-  fetch(slice + kSumSlices, low[1], high[1]);
+  fetch(slice, one[0], two[0]);
+  fetch(slice + kSumSlices, one[1], two[1]);
   for (uint32_t block0 = slice; block0 < blocks; block0 += 2u * kSumSlices)
 #pragma unroll
   for (uint32_t turn = 0; turn < 2; ++turn) {
     const uint32_t block = block0 + turn * kSumSlices;
     if (block >= blocks) break;
-    uint4* mine = (uint4*)(s_bits[turn] + wave * kSumPitch) + 2u * lane;
-    mine[0] = low[turn];
-    mine[1] = high[turn];
-    fetch(block + 2u * kSumSlices, low[turn], high[turn]);
+    ((uint4*)(s_bits[turn] + 2u * wave * kSumPitch))[lane] = one[turn];
+    ((uint4*)(s_bits[turn] + (2u * wave + 1u) * kSumPitch))[lane] = two[turn];
+    fetch(block + 2u * kSumSlices, one[turn], two[turn]);
     __syncthreads();
     uint2 now[kSumGroups];
 #pragma unroll
@@ -760,74 +764,78 @@ __global__ __launch_bounds__(kSumThreads, 4) void union_sums(const uint32_t* __r
       const uint32_t first = q == 0 ? 0u : (uint32_t)sums[0];
       count += (uint32_t)sums[0];
       const uint64_t share = (uint64_t)(uint32_t)sums[3] * (1u << 21) + (first + ((uint32_t)sums[1] << 7) + ((uint32_t)sums[2] << 14));
-      const uint32_t to = column * (kGroupsPerPart + 1) + wave * kSumGroups + g;
+      const uint32_t to = column * (kGroupsPerHalf + 1) + wave * kSumGroups + g;
       if (q < 2) s_sums[turn][q][to] = share;
       if (q == 2 && square_rows > 8) s_top[turn][to] = (uint32_t)sums[0] + ((uint32_t)sums[1] << 7);
     }
     if (q == 0 && count) atomicAdd(&s_marked[turn][column], count);
     __syncthreads();
-    const uint32_t at = block * kSumSamples + wave;
+    // half of the wavefront has one sample, half the other
+    const uint32_t sample = 2u * wave + (lane >> 5), group = lane & 31u, at = block * kSumSamples + sample;
+    const uint32_t of = sample * (kGroupsPerHalf + 1) + group;
+    uint64_t sum = (s_sums[turn][0][of] >> 7) + (s_sums[turn][1][of] << 21);
+    if (square_rows > 8) sum += (uint64_t)s_top[turn][of] << 49;
+    uint64_t through = wave_inclusive_scan_u64(sum);
+    const uint64_t others = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(through >> 32), 31) << 32 |
+                            (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)through, 31);
+    if (lane >= 32) through -= others;
     if (at < n) {
-      const uint32_t of = wave * (kGroupsPerPart + 1) + lane;
-      uint64_t sum = (s_sums[turn][0][of] >> 7) + (s_sums[turn][1][of] << 21);
-      if (square_rows > 8) sum += (uint64_t)s_top[turn][of] << 49;
-      const uint64_t through = wave_inclusive_scan_u64(sum);
-      const size_t place = (size_t)at * parts + part;
-      group_through[place * kGroupsPerPart + lane] = through;
-      if (lane == 63) part_total[place] = through;
-      if (lane == 0 && s_marked[turn][wave]) atomicAdd(&distinct[marked.sample[at]], s_marked[turn][wave]);
+      const size_t place = (size_t)at * halves + half;
+      group_through[place * kGroupsPerHalf + group] = through;
+      if (group == kGroupsPerHalf - 1u) half_total[place] = through;
+      if (group == 0 && s_marked[turn][sample]) atomicAdd(&distinct[marked.sample[at]], s_marked[turn][sample]);
     }
-    if (lane == 0) s_marked[turn][wave] = 0;
+    if (group == 0) s_marked[turn][sample] = 0;
   }
 }
 
-// One wavefront per marked sample: part_before[at * (parts + 1) + p] = degree^2 of the marked vertices
-// of the sample's parts before p; entry `parts` is the sample's total.
-__global__ __launch_bounds__(64) void sample_part_sums(const uint64_t* __restrict__ part_total, uint32_t parts,
+// One wavefront per marked sample: half_before[at * (halves + 1) + p] = degree^2 of the marked vertices
+// of the sample's halves before p; entry `halves` is the sample's total.
+__global__ __launch_bounds__(64) void sample_half_sums(const uint64_t* __restrict__ half_total, uint32_t halves,
                                                        const uint32_t* __restrict__ n_marked,
-                                                       uint64_t* __restrict__ part_before) {
+                                                       uint64_t* __restrict__ half_before) {
   const uint32_t s = blockIdx.x, lane = threadIdx.x;
   if (s >= *n_marked) return;
   uint64_t carry = 0;
-  for (uint32_t p0 = 0; p0 < parts; p0 += 64) {
+  for (uint32_t p0 = 0; p0 < halves; p0 += 64) {
     const uint32_t p = p0 + lane;
-    const uint64_t mine = p < parts ? part_total[(size_t)s * parts + p] : 0ull;
+    const uint64_t mine = p < halves ? half_total[(size_t)s * halves + p] : 0ull;
     const uint64_t through = wave_inclusive_scan_u64(mine);
-    if (p < parts) part_before[(size_t)s * (parts + 1) + p] = carry + through - mine;
+    if (p < halves) half_before[(size_t)s * (halves + 1) + p] = carry + through - mine;
     const uint32_t lo = __shfl((uint32_t)through, 63, kWave), hi = __shfl((uint32_t)(through >> 32), 63, kWave);
     carry += ((uint64_t)hi << 32) | lo;
   }
-  if (lane == 0) part_before[(size_t)s * (parts + 1) + parts] = carry;
+  if (lane == 0) half_before[(size_t)s * (halves + 1) + halves] = carry;
 }
 
 // What next() receives as transitEdges for a marked sample.  A lane searches for itself: 64 draws' misses are then under
 // way in a wavefront (R-MAT 20, 262 K draws: 0.058 ms; a wavefront to a draw, its lanes searching together: 0.198).
 struct MarkedByDegreeSquared {
   const uint32_t* bits;           // the sample's bitmap
-  const uint64_t* part_before;    // the sample's parts + 1 entries
-  const uint64_t* group_through;  // the sample's parts * 64 entries
+  const uint64_t* half_before;    // the sample's halves + 1 entries
+  const uint64_t* group_through;  // the sample's halves * 32 entries
   const EdgePos_t* row_ptr;
-  uint32_t parts;
+  uint32_t halves;
 
-  __device__ __forceinline__ uint64_t total() const { return part_before[parts]; }
+  __device__ __forceinline__ uint64_t total() const { return half_before[halves]; }
 
   // the smallest marked vertex whose running sum of degree^2 (marked vertices ascending) exceeds target;
   // target < total()
   __device__ inline VertexID first_exceeding(uint64_t target) const {
-    uint32_t part = 0, end = parts;  // the last part whose sum-before is <= target
-    while (end - part > 1) {
-      const uint32_t mid = part + (end - part) / 2;
-      if (part_before[mid] <= target) part = mid; else end = mid;
+    uint32_t half = 0, end = halves;  // the last half whose sum-before is <= target
+    while (end - half > 1) {
+      const uint32_t mid = half + (end - half) / 2;
+      if (half_before[mid] <= target) half = mid; else end = mid;
     }
-    target -= part_before[part];
-    const uint64_t* through = group_through + (size_t)part * kGroupsPerPart;
-    uint32_t group = 0, last = kGroupsPerPart - 1;  // the first group whose sum-through exceeds it
+    target -= half_before[half];
+    const uint64_t* through = group_through + (size_t)half * kGroupsPerHalf;
+    uint32_t group = 0, last = kGroupsPerHalf - 1;  // the first group whose sum-through exceeds it
     while (group < last) {
       const uint32_t mid = group + (last - group) / 2;
       if (through[mid] > target) last = mid; else group = mid + 1;
     }
     if (group) target -= through[group - 1];
-    const uint32_t first_word = part * kPartWords + group * kGroupWords;
+    const uint32_t first_word = half * kHalfWords + group * kGroupWords;
     uint64_t running = 0;
     for (uint32_t k = 0; k < kGroupWords; ++k)
       for (uint32_t word = bits[first_word + k]; word; word &= word - 1u) {
