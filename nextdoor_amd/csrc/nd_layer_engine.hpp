@@ -760,30 +760,37 @@ __global__ __launch_bounds__(kBinThreads, 8) __attribute__((amdgpu_num_vgpr(56))
       if (falls_here && start != e0) atomicOr(&s_starts_here[wave][(start - e0 - 1u) >> 5], 1u << ((start - e0 - 1u) & 31u));
       __builtin_amdgcn_wave_barrier();
       // (nothing may be worked out from an id before the last is asked for: the compiler waits for it where that is done)
-      uint32_t ids[kBinAhead];
-      unsigned long long terms[kBinAhead];
-      uint32_t of = before + ((uint32_t)__builtin_amdgcn_readfirstlane((int)start) == e0 ? 1u : 0u);  // only the first can
+      // all: every lane has an entry every time, as in most rounds, so that none is masked out (500 K vertices: 3.18 -> 3.12 ms a pass)
+      auto add_up = [&](auto all) {
+        constexpr bool kAll = decltype(all)::value;
+        uint32_t ids[kBinAhead];
+        unsigned long long terms[kBinAhead];
+        uint32_t of = before + ((uint32_t)__builtin_amdgcn_readfirstlane((int)start) == e0 ? 1u : 0u);  // only the first can
 #pragma unroll
-      for (uint32_t a = 0; a < kBinAhead; ++a) {
-        const uint32_t low = s_starts_here[wave][2u * a], high = s_starts_here[wave][2u * a + 1u];
-        const uint32_t e = e0 + a * 64u + lane;
-        const uint32_t mine = __builtin_amdgcn_mbcnt_hi(high, __builtin_amdgcn_mbcnt_lo(low, of));
-        of += (uint32_t)__popc(low) + (uint32_t)__popc(high);
-        ids[a] = 0;
-        terms[a] = 0;
-        if (e < end) {
-          const EdgePos_t src = (EdgePos_t)e + s_shift[mine];
+        for (uint32_t a = 0; a < kBinAhead; ++a) {
+          const uint32_t low = s_starts_here[wave][2u * a], high = s_starts_here[wave][2u * a + 1u];
+          const uint32_t e = e0 + a * 64u + lane;
+          const uint32_t mine = __builtin_amdgcn_mbcnt_hi(high, __builtin_amdgcn_mbcnt_lo(low, of));
+          of += (uint32_t)__popc(low) + (uint32_t)__popc(high);
+          if (!kAll) {
+            ids[a] = 0;
+            terms[a] = 0;
+            if (e >= end) continue;
+          }
+          const uint32_t src = e + (uint32_t)s_shift[mine];  // an edge: not negative
           ids[a] = (uint32_t)merged.ids[src];
           terms[a] = merged.terms[src];
         }
-      }
 #pragma unroll
-      for (uint32_t a = 0; a < kBinAhead; ++a) {
-        if (e0 + a * 64u + lane >= end) continue;
-        const uint32_t local = ids[a] - v_lo;
-        atomicAdd(&s_acc[local], terms[a]);
-        if (merged.zero_terms) atomicOr(&s_bits[local >> 5], 1u << (local & 31u));
-      }
+        for (uint32_t a = 0; a < kBinAhead; ++a) {
+          if (!kAll && e0 + a * 64u + lane >= end) continue;
+          const uint32_t local = ids[a] - v_lo;
+          atomicAdd(&s_acc[local], terms[a]);
+          if (merged.zero_terms) atomicOr(&s_bits[local >> 5], 1u << (local & 31u));
+        }
+      };
+      if (end - e0 == kRound) add_up(std::true_type());
+      else add_up(std::false_type());
       before += (uint32_t)__popcll(__ballot(falls_here));
       e0 = end;
     }
