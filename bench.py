@@ -47,10 +47,10 @@ MEASURED = {
                     "bytes_per_pass": 7.45e9},
     # the kernels of a layer, average over a pass's 2 layers
     "fastgcn_importance_rmat22": {
-        "kernels": {"nd::sorted_layer_kernel": 8.169e7, "nd::union_parts": 2.063e9, "nd::union_sums": 1.737e9},
-        "bytes_per_pass": 7.88e9},
+        "kernels": {"nd::sorted_layer_kernel": 8.166e7, "nd::union_parts": 2.061e9, "nd::union_sums": 1.745e9},
+        "bytes_per_pass": 7.90e9},
     "ladies_importance_chunglu3m": {
-        "kernels": {"nd::ranked_layer_kernel": 6.243e7, "nd::collective_mark_binned": 6.172e10}, "bytes_per_pass": 123.74e9},
+        "kernels": {"nd::ranked_layer_kernel": 6.221e7, "nd::collective_mark_binned": 5.905e10}, "bytes_per_pass": 118.40e9},
 }
 
 
@@ -418,7 +418,7 @@ def measure(args, workload, steps, warmup, cpu_seconds, graphs, engine_choice=Tr
         recorded = MEASURED_TRAFFIC_BYTES_PER_LAUNCH.get(workload)
         traffic_gbps = recorded / (prof["neighbourhood_ms"] / launches / 1000.0) / 1e9 if recorded else None
         # (LADIES: 5.8 TB/s, and 52 % of the vector issue slots; FastGCN: union_parts takes its pieces and entries from L2, at
-        # 2.2 TB/s from memory, union_sums reads the bitmaps at 3.1 TB/s)
+        # 2.2 TB/s from memory, union_sums reads the bitmaps at 4.0 TB/s)
         bound = "hbm" if ladies else "L2 (pieces and entries of union_parts), hbm (bitmaps of union_sums)"
         result["roofline"] = {
             "bound": bound, "kernel": kernels, "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",

@@ -586,11 +586,12 @@ constexpr uint32_t kSparseGroupEntries = 2048;
 // The samples that are not ranked in LDS (ranked_layer).
 // Two workgroups of 16 wavefronts share a compute unit only at 8 wavefronts per SIMD, which the kernel's attributes ask
 // the compiler for.
-// 500 K vertices, 12 M edges, second layer of 1024 samples of 512 (1.5 M pairs and 136 pieces a sample): 2.52 ms.  Writing a
+// 500 K vertices, 12 M edges, second layer of 1024 samples of 512 (1.5 M pairs and 136 pieces a sample): 2.42 ms.  Writing a
 // key for every vertex it took 3.42, and the selection, the collecting and the sorts 1.1 more, where kept_layer_kernel takes
 // 0.04; forming only keys that may be within the bound 3.17, the ids of all of a round's entries under way before the first
-// is used 2.86, starts as bits 2.59.  What bounds it now: vector instructions take 69 % of the issue slots (1.08 G of them at four
-// clocks), the rest is the phases of a stretch waiting for each other, and registers that do not fit.
+// is used 2.86, starts as bits 2.59 (2.52 when it was last measured before the next two), those counted by mbcnt and full rounds without
+// masks 2.42.  What bounds it now: vector instructions take 63 % of the issue slots (0.94 G of them at four clocks; 1.08 G before those
+// two), the rest is the phases of a stretch waiting for each other, and registers that do not fit.
 __global__ __launch_bounds__(kBinThreads, 8) __attribute__((amdgpu_num_vgpr(56))) void collective_mark_binned(
     MergedEdges merged, TransitView tv, int32_t invalid, uint32_t n_samples, const uint32_t* __restrict__ n_marked,
     const uint32_t* __restrict__ marked, uint32_t bins_per_sample, DensePieces dense, KeptKeys out) {
