@@ -315,3 +315,23 @@ def test_ladies_neighbourhoods_at_the_edge_of_what_is_ranked_in_lds(oracle, degr
         s.do_transit_parallel(True)
         assert np.array_equal(s.final_samples(), want)
     s.close()
+
+
+# Neighbourhoods too large to be ranked in LDS (8192 pairs), so that they are marked by stretches of 7168 vertices: every transit has `low`
+# neighbours in the first stretch and `high` in the second.  Wavefronts take 256 pairs a round: transits that start with a
+# round, one before it and one behind, rounds of one transit, and of more than the 63 starts that a round takes.
+@pytest.mark.parametrize("app,low,high", [("LADIESImportance2x8", low, high) for low in (255, 256, 257, 512) for high in (900, 1024)] +
+                         [("LADIESImportanceB8", low, high) for low, high in ((1, 17), (2, 15), (4, 16), (5, 64))])
+def test_ladies_transits_that_start_at_the_edges_of_a_round(oracle, app, low, high):
+    n = 9001
+    v = np.repeat(np.arange(n), low + high)
+    i = np.tile(np.arange(low + high), n)
+    dst = np.where(i < low, (v * 37 + i * 11) % 7168, 7168 + (v * 41 + i * 7) % (n - 7168))  # all of a transit's are different
+    w = (np.random.default_rng(low).random(len(v)) * 4 + 1).astype(np.float32)
+    g = nd.Graph.from_edges(v, dst, w, n_vertices=n)
+    s = nd.Sampler(app, g, seed=SEED)
+    want = oracle.sample_ladies_importance(graphs.oracle_view(g), layer_desc(oracle, s, oracle.LADIES_IMPORTANCE), SEED,
+                                           s.initial_contents)
+    s.do_transit_parallel(True)
+    assert np.array_equal(s.final_samples(), want)
+    s.close()
