@@ -2253,7 +2253,7 @@ class Engine : public EngineBase {
   // stream order.
   void send_rows(const std::vector<size_t>& ends, std::vector<ResultStream::Ready> ready, hipEvent_t computed) {
     const size_t F = (size_t)final_sample_size(), state_words = sizeof(SampleType) / sizeof(int32_t);
-    const bool states = states_ahead && ready.empty();
+    const bool states = kStatesAreWords && states_ahead && ready.empty();
     try {
       std::vector<ResultStream::Part> parts;
       size_t words = 0;
@@ -2842,7 +2842,8 @@ class Engine : public EngineBase {
   // cross the bus while later walks are still under way; sample() returns when the sampling is done, as
   // always, and the rest of the rows arrives until finish_rows_ahead().  Any pass may leave it be.
   VertexID_t* rows_ahead = nullptr;
-  // ... and its states (whole words), with rows only.
+  // ... and its states, with rows only, of apps whose samples' states are whole words each: ranges of samples are then ranges of words.
+  static constexpr bool kStatesAreWords = !std::is_empty<SampleType>::value && sizeof(SampleType) % sizeof(int32_t) == 0;
   int32_t* states_ahead = nullptr;
   // Waits for rows on their way; whether they are at rows_ahead.  Where not (no pass sent them, the transfer failed) they
   // are to be fetched like any others.

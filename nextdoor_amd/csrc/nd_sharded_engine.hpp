@@ -96,8 +96,7 @@ class ShardedEngine : public EngineBase {
     parts_[0]->states_ahead = nullptr;
     if (parts_.size() == 1 && rows_fetched_ && hFinalSamples.taken() && rows_ahead_.try_resize(hFinalSamples.size())) {
       parts_[0]->rows_ahead = rows_ahead_.data();
-      const size_t bytes = sample_state_bytes();
-      if (states_fetched_ && hSampleStates.taken() && bytes % sizeof(int32_t) == 0 && hSampleStates.try_resize(bytes))
+      if (Part::kStatesAreWords && states_fetched_ && hSampleStates.taken() && hSampleStates.try_resize(sample_state_bytes()))
         parts_[0]->states_ahead = (int32_t*)hSampleStates.data();
     }
     rows_fetched_ = states_fetched_ = rows_changed_ = false;

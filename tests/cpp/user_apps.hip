@@ -3,6 +3,7 @@
 // that are NOT compiled into libnextdoor_amd.so.  This file is built by hipcc into a shared
 // object of its own (tests/cpp/libuser_apps.so); loading it registers them with the library.
 #include "../../nextdoor_amd/csrc/nd_app_registry.hpp"
+#include "../../nextdoor_amd/csrc/nd_apps_walks.hpp"
 
 class UserHopSample {};
 
@@ -165,6 +166,33 @@ struct UserRankedCountApp : LadiesImportanceAppT<1, 16, 60> {
   }
 };
 
+// States of 2 and 6 bytes: no whole number of words a sample
+struct UserSumSample {
+  uint16_t sum;
+  __device__ void note(VertexID v) { sum = (uint16_t)(sum + v); }
+};
+struct UserTallySample {
+  uint16_t sum, last, steps;
+  __device__ void note(VertexID v) {
+    sum = (uint16_t)(sum + v);
+    last = (uint16_t)v;
+    steps++;
+  }
+};
+
+// Uniform walks that note in their state where they were
+struct UserNotingWalkApp : UniformRandomWalkAppT<8> {
+  template <typename SampleType, typename EdgeArray, typename WeightArray>
+  __device__ inline VertexID next(int step, CSRPartition* csr, const VertexID* transit, const VertexID sampleIdx,
+                                  SampleType* sample, const float max_weight, EdgeArray& transitEdges,
+                                  WeightArray& transitEdgeWeights, const EdgePos_t numEdges,
+                                  const VertexID_t neighbrID, curandState* state) {
+    const VertexID v = transitEdges[RandNumGen::rand_int(state, numEdges)];
+    sample->note(v);
+    return v;
+  }
+};
+
 // The sizes this object was built with, for the test of what the library compares.
 extern "C" int user_apps_shared_layouts(uint64_t* out, int room) {
   const uint64_t sizes[] = {sizeof(nd::EngineBase), sizeof(nd::PhaseTimes), sizeof(nd::ResultStream), nd::ResultStream::transfer_bytes(),
@@ -179,3 +207,5 @@ ND_REGISTER_APP("UserRankedCount", UserRankedSample, UserRankedCountApp)
 ND_REGISTER_APP("UserAnchorHop", UserAnchorSample, UserAnchorHopApp)
 ND_REGISTER_APP("UserThreeHop", UserHopSample, UserThreeHopApp)
 ND_REGISTER_APP("UserShortDeepWalk", UserWalkSample, UserShortDeepWalkApp)
+ND_REGISTER_APP("UserSumWalk", UserSumSample, UserNotingWalkApp)
+ND_REGISTER_APP("UserTallyWalk", UserTallySample, UserNotingWalkApp)

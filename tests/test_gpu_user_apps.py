@@ -103,6 +103,34 @@ def test_a_ranked_layer_hands_over_as_many_vertices_as_it_takes(n, mean_degree, 
         s.close()
 
 
+# rows that follow their one launch and rows that leave by range, all states together a whole number of words and not
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [3002, 3001, 90002])
+@pytest.mark.parametrize("app,fields", [("UserSumWalk", 1), ("UserTallyWalk", 3)])
+def test_states_of_no_whole_number_of_words(oracle, app, fields, n):
+    """States of 2 and 6 bytes are those of the pass, also where rows and states were taken after the passes before."""
+    nd.load_app_library(USER_APPS_LIB)
+    g = graphs.random_graph(n=n, mean_degree=5, seed=n, isolated_every=7)
+    s = nd.Sampler(app, g, seed=SEED)
+    d = ob.app_desc(ob.UNIFORM_WALK, s.steps, [1] * s.steps)
+    want, _ = ob.sample_individual(graphs.oracle_view(g), d, SEED, s.initial_contents)
+    visited = want != s.invalid_vertex
+    steps = visited.sum(axis=1)
+    notes = [np.where(visited, want, 0).sum(axis=1), want[np.arange(n), np.maximum(steps, 1) - 1] * (steps > 0), steps]
+    notes = np.stack(notes[:fields], axis=1).astype(np.uint16)
+    try:
+        for turn in range(6):
+            print("app", app, "n", n, "turn", turn, flush=True)
+            s.set_inversion_period(1 if turn == 4 else 0)
+            s.do_transit_parallel()
+            assert np.array_equal(s.final_samples(), want)
+            states = s.sample_states()
+            assert states.size == 2 * n * fields
+            assert np.array_equal(np.frombuffer(states.tobytes(), np.uint16).reshape(n, fields), notes)
+    finally:
+        s.close()
+
+
 def write_binary_edge_list(path, src, dst, weight):
     """The reference's binary edge list: 12-byte records (int32 src, int32 dst, float32 weight),
     src/graph.hpp:42-75."""
