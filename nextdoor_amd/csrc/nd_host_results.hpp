@@ -837,14 +837,12 @@ class ResultStream {
       t.streams[0] = stream;
       t.computed_event = computed;
       if (t.chunks <= t.ring_chunks) t.streams[1] = stream;
-      // two streams, so that the bus is not idle between two launches
-      if (t.chunks > t.ring_chunks) {
-        e = hipEventRecord(begun_, stream);
-        if (e == hipSuccess) e = hipStreamWaitEvent(t.streams[1], begun_, 0);
-      }
-      while (e == hipSuccess && t.sent < t.ring_chunks) e = launch(std::min(t.part_ends[t.part_of(t.sent)], t.ring_chunks), bus_blocks());
+      else e = hipEventRecord(begun_, stream);
+      // (all on the given stream: the other one is not only ours, and what is computed before this may take long)
+      while (e == hipSuccess && t.sent < t.ring_chunks)
+        e = launch(std::min(t.part_ends[t.part_of(t.sent)], t.ring_chunks), bus_blocks(), stream);
       if (e != hipSuccess) {
-        for (hipStream_t s : t.streams) (void)hipStreamSynchronize(s);  // nothing writes to the ring after this
+        (void)hipStreamSynchronize(stream);  // nothing writes to the ring after this
         return e;
       }
       // few chunks are unpacked before a thread is awake, unless it is woken while they are computed
@@ -1208,7 +1206,7 @@ class ResultStream {
   uint32_t bus_blocks() const { return transfer_->chunks > transfer_->ring_chunks ? kBusBlocksOfMany : kBusBlocks; }
 
   // Straight: the chunks from t.sent on, up to `end`, all of one part.
-  hipError_t launch(size_t end, uint32_t most_blocks) {
+  hipError_t launch(size_t end, uint32_t most_blocks, hipStream_t on) {
     Transfer& t = *transfer_;
     const size_t part = t.part_of(t.sent), first = (t.sent - t.part_begin(part)) * kPackChunk;
     const Part& p = t.parts[part];
@@ -1219,7 +1217,7 @@ class ResultStream {
     out.ring_mask = t.chunks > t.ring_chunks ? (uint32_t)t.ring_chunks - 1u : UINT32_MAX;
     static_assert((kRingChunks & (kRingChunks - 1)) == 0, "a ring that is gone round");
     out.stamp = t.stamp(t.sent);
-    pack_results<false><<<dim3(std::min(n_chunks, most_blocks)), dim3(kPackThreads), 0, t.streams[t.launches % 2]>>>(
+    pack_results<false><<<dim3(std::min(n_chunks, most_blocks)), dim3(kPackThreads), 0, on>>>(
         p.src + first, here, t.bits, p.fill, out, n_chunks);
     t.launches++;
     t.sent = end;
@@ -1340,7 +1338,7 @@ class ResultStream {
     Transfer& t = *transfer_;
     hipError_t error = hipSuccess;
     if (t.computed_event && (error = wait_for(t.computed_event)) == hipSuccess) t.announce(t.sent, false);
-    bool gently = !t.ready.empty();
+    bool gently = !t.ready.empty(), ordered = gently;
     size_t gentle = 0, gone = 0;  // launches of those, and how many of them have ended
     while (t.sent < t.chunks && error == hipSuccess && !t.stop.load(std::memory_order_relaxed)) {
       gently = gently && !computed();
@@ -1363,9 +1361,14 @@ class ResultStream {
         if (!unpack_some()) std::this_thread::yield();
         continue;
       }
+      // Two streams, so that the bus is not idle between two launches.  Words in stream order are there by now, as chunks behind them
+      // have arrived: nobody waits for that event.
+      if (!ordered && (error = hipStreamWaitEvent(t.streams[1], begun_, 0)) != hipSuccess) break;
+      ordered = true;
       if (gently) ahead_.fetch_add(1, std::memory_order_relaxed);
-      error = launch(end, gently ? kGentleBlocks : bus_blocks());
-      if (error == hipSuccess && gently) error = hipEventRecord(packed_[gentle++ % kSlots], t.streams[(t.launches - 1) % 2]);
+      const hipStream_t stream = t.streams[t.launches % 2];
+      error = launch(end, gently ? kGentleBlocks : bus_blocks(), stream);
+      if (error == hipSuccess && gently) error = hipEventRecord(packed_[gentle++ % kSlots], stream);
       if (error == hipSuccess) t.announce(t.sent, false);
     }
     return error;

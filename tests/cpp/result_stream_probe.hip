@@ -131,9 +131,71 @@ static int beside_one_that_waits() {
   return 0;
 }
 
+// One in stream order behind a long computation, of more chunks than the ring holds, and others whose words are there: those do not wait
+// for it.
+static int beside_one_that_follows() {
+  const size_t many = (size_t)4200 * nd::kPackChunk, n = (size_t)300 * nd::kPackChunk;
+  std::vector<int32_t> want(many), late(many), got(n);
+  for (size_t i = 0; i < many; ++i) want[i] = (int32_t)(i & 0xfff);
+  int32_t *d = nullptr, *d_late = nullptr;
+  uint32_t* sign = nullptr;
+  hipStream_t busy, stream;
+  hipEvent_t there, computed;
+  TRY(hipMalloc(&d, n * sizeof(int32_t)));
+  TRY(hipMalloc(&d_late, many * sizeof(int32_t)));
+  TRY(hipHostMalloc((void**)&sign, sizeof(uint32_t), hipHostMallocDefault));
+  *sign = 7;
+  TRY(hipStreamCreate(&stream));
+  TRY(hipStreamCreate(&busy));
+  TRY(hipEventCreateWithFlags(&there, hipEventDisableTiming));
+  TRY(hipEventCreateWithFlags(&computed, hipEventDisableTiming));
+  TRY(hipMemcpyAsync(d, want.data(), n * sizeof(int32_t), hipMemcpyHostToDevice, stream));
+  TRY(hipEventRecord(there, stream));
+  TRY(hipStreamSynchronize(stream));
+  nd::ResultStream first, other;
+  for (int turn = 0; turn < 3; ++turn) {  // the first one takes the memory
+    TRY(hipMemset(d_late, 0, many * sizeof(int32_t)));
+    TRY(hipDeviceSynchronize());
+    if (turn) take_a_while<<<dim3(1), dim3(64), 0, busy>>>();
+    write_words<<<dim3((unsigned)((many + 255) / 256)), dim3(256), 0, busy>>>(d_late, many);
+    TRY(hipGetLastError());
+    TRY(hipEventRecord(computed, busy));
+    std::fill(late.begin(), late.end(), -1);
+    TRY(first.begin(d_late, many, 12, 0, late.data(), busy, {}, turn < 2 ? computed : nullptr));
+    std::this_thread::sleep_for(std::chrono::milliseconds(5));  // other threads take it on
+    for (int form = 0; form < 3; ++form) {
+      printf("beside one that follows: turn %d form %d\n", turn, form);
+      fflush(stdout);
+      std::vector<nd::ResultStream::Ready> ready{{n, there}};
+      if (form == 1) ready.insert(ready.begin(), {n / 2, there});
+      if (form == 2) ready = {{n / 3, there, sign, 7u}, {n, there, sign, 7u}};
+      std::fill(got.begin(), got.end(), -1);
+      TRY(other.begin(d, n, 12, 0, got.data(), stream, ready));
+      TRY(other.finish());
+      const bool before = hipEventQuery(computed) == hipErrorNotReady;
+      (void)hipGetLastError();
+      if (!std::equal(got.begin(), got.end(), want.begin())) { printf("other words\n"); return 1; }
+      if (turn && !before) { printf("held up until the other computation was over\n"); return 1; }
+    }
+    TRY(first.finish());
+    if (late != want) { printf("words from before they were there\n"); return 1; }
+  }
+  first.release();
+  other.release();
+  TRY(hipEventDestroy(there));
+  TRY(hipEventDestroy(computed));
+  TRY(hipStreamDestroy(stream));
+  TRY(hipStreamDestroy(busy));
+  TRY(hipHostFree(sign));
+  TRY(hipFree(d));
+  TRY(hipFree(d_late));
+  return 0;
+}
+
 int main() {
   if (on_other_devices() != 0) return 1;
   if (beside_one_that_waits() != 0) return 1;
+  if (beside_one_that_follows() != 0) return 1;
   const size_t piece = (size_t)64 * nd::kPackChunk;  // the smallest piece
   const size_t sizes[] = {1, 7, 8, 9, nd::kPackChunk - 1, nd::kPackChunk, nd::kPackChunk + 1, piece, piece + 9, 13 * piece + 4097,
                           (size_t)4200 * nd::kPackChunk + 5};
