@@ -2155,8 +2155,9 @@ class Engine : public EngineBase {
     const int rc = wants_launch_graph() ? replay_pass(mode) : enqueue_pass(mode);
     if (rc != 0) return rc;
     ND_HIP_TRY(hipEventRecord(ev_end_, stream_));
-    if (rows_follow_) send_rows({}, {}, ev_end_);
+    if (rows_follow_) send_rows({}, {});
     ND_HIP_TRY(hipEventSynchronize(ev_end_));
+    if (rows_follow_) result_stream->words_are_there();
     ND_HIP_TRY(hipEventElapsedTime(&times.end_to_end, ev_begin_, ev_end_));
     schedule_counts_.passes++;
     if (balanced_this_pass_) {
@@ -2235,7 +2236,7 @@ class Engine : public EngineBase {
         ready.push_back({(size_t)std::min<uint64_t>((uint64_t)n_samples_, at + (1ull << early.shift)) * F, range_ends_[0],
                          h_arrived_ + (at >> early.shift), early.pass});
     }
-    send_rows(ends, std::move(ready), nullptr);
+    send_rows(ends, std::move(ready));
     sent_ahead_ = ahead_;
     return 0;
   }
@@ -2249,9 +2250,9 @@ class Engine : public EngineBase {
   }
 
   // Has the rows leave for rows_ahead, and the states for states_ahead; those that cannot be sent now are fetched when they are asked
-  // for.  ends: of the ranges of samples whose results are there at one of range_ends_ each; none: as `ready` has it, or in
-  // stream order.
-  void send_rows(const std::vector<size_t>& ends, std::vector<ResultStream::Ready> ready, hipEvent_t computed) {
+  // for.  ends: of the ranges of samples whose results are there at one of range_ends_ each; none: as `ready` has it, or behind
+  // the pass.
+  void send_rows(const std::vector<size_t>& ends, std::vector<ResultStream::Ready> ready) {
     const size_t F = (size_t)final_sample_size(), state_words = sizeof(SampleType) / sizeof(int32_t);
     const bool states = kStatesAreWords && states_ahead && ready.empty();
     try {
@@ -2270,7 +2271,8 @@ class Engine : public EngineBase {
         if (!ends.empty()) ready.push_back({words, range_ends_[r]});
         at = end;
       }
-      ahead_ = result_stream->begin(std::move(parts), stream_, std::move(ready), computed) == hipSuccess;
+      const bool follow = ready.empty();
+      ahead_ = result_stream->begin(std::move(parts), stream_, std::move(ready), follow) == hipSuccess;
     } catch (const std::bad_alloc&) {
       ahead_ = false;
     }
@@ -2469,7 +2471,7 @@ class Engine : public EngineBase {
       if (enqueue_steps(mode, balance, (uint32_t)at, (uint32_t)(ends[r] - at)) != 0) return -1;
       ND_HIP_TRY(hipEventRecord(range_ends_[r], stream_));
     }
-    send_rows(ends, {}, nullptr);
+    send_rows(ends, {});
     sent_ahead_ = ahead_;
     return 0;
   }

@@ -804,16 +804,17 @@ class ResultStream {
     return fetch({{src, n, bits, fill, dst}}, stream);
   }
   hipError_t begin(const int32_t* src, size_t n, uint32_t bits, int32_t fill, int32_t* dst, hipStream_t stream,
-                   std::vector<Ready> ready, hipEvent_t computed = nullptr) {
-    return begin({{src, n, bits, fill, dst}}, stream, std::move(ready), computed);
+                   std::vector<Ready> ready, bool follows = false) {
+    return begin({{src, n, bits, fill, dst}}, stream, std::move(ready), follows);
   }
 
   // The same as a begin() that returns at once, other threads taking it from there, and a finish() that takes part
   // and returns when the words are at dst.  `ready` (words ascending, the last all of them; with a sign, of a single part): what has to have
-  // happened before words may be read, while other work of the caller's is still going on; empty: stream order, and `computed`, if there is
-  // one, an event recorded on the stream before, that the threads need not look for words until it has happened.  What is given has
-  // to stay until finish().
-  hipError_t begin(std::vector<Part> parts, hipStream_t stream, std::vector<Ready> ready, hipEvent_t computed = nullptr) {
+  // happened before words may be read, while other work of the caller's is still going on; empty: stream order, and `follows` where what the
+  // words follow there takes a while: the threads then look for none until the caller, who waits for that anyway, says words_are_there().
+  // (A thread that asked for the event meanwhile would get no answer: hipEventSynchronize() holds the event until it returns, and a
+  // query of 13.9 ms was over 13 to 36 us after that.)  What is given has to stay until finish().
+  hipError_t begin(std::vector<Part> parts, hipStream_t stream, std::vector<Ready> ready, bool follows = false) {
     hipError_t e = finish();  // an earlier one that nobody waited for
     parts.erase(std::remove_if(parts.begin(), parts.end(), [](const Part& p) { return p.n == 0; }), parts.end());
     if (e != hipSuccess || parts.empty()) return e;
@@ -835,7 +836,7 @@ class ResultStream {
     size_t helpers = HostWorkers::kMost;
     if (t.ready.empty()) {
       t.streams[0] = stream;
-      t.computed_event = computed;
+      t.follows = follows;
       if (t.chunks <= t.ring_chunks) t.streams[1] = stream;
       else e = hipEventRecord(begun_, stream);
       // (all on the given stream: the other one is not only ours, and what is computed before this may take long)
@@ -846,8 +847,8 @@ class ResultStream {
         return e;
       }
       // few chunks are unpacked before a thread is awake, unless it is woken while they are computed
-      if (t.chunks <= kFewChunks) helpers = computed ? t.chunks / kChunksAHelper : 0;
-      if (!computed) t.announce(t.sent, false);
+      if (t.chunks <= kFewChunks) helpers = follows ? t.chunks / kChunksAHelper : 0;
+      if (!follows) t.announce(t.sent, false);
     }
     job_.body = [this] { take_part(); };
     under_way_ = true;
@@ -859,9 +860,17 @@ class ResultStream {
     return hipSuccess;
   }
 
+  // What the words of the last begin() follow is done.
+  void words_are_there() {
+    if (!under_way_ || !transfer_->follows) return;
+    transfer_->follows = false;
+    transfer_->announce(transfer_->sent, false);  // (nobody sends more before that)
+  }
+
   hipError_t finish() {
     if (!under_way_) return hipSuccess;
     Transfer& t = *transfer_;
+    words_are_there();  // or will be: who looks for a chunk waits until it comes
     take_part();
     if (helped_) HostWorkers::get().join(job_);
     under_way_ = false;
@@ -1039,7 +1048,7 @@ class ResultStream {
     hipStream_t streams[2];
     std::vector<Ready> ready;
     std::vector<size_t> ready_chunks;  // that are there once a `ready` has happened
-    hipEvent_t computed_event = nullptr;
+    bool follows = false;  // and the caller has not said that they are there
     bool staged = false;  // pieces are packed in device memory, for the copy engine, while something else is computed
     int device = 0;
 
@@ -1069,7 +1078,7 @@ class ResultStream {
     void set(std::vector<Part> parts_, std::vector<Ready> ready_) {
       parts = std::move(parts_), ready = std::move(ready_);
       staged = !ready.empty() && ready.front().sign != nullptr;
-      computed_event = nullptr;
+      follows = false;
       happened = 0;
       computed = false;
       chunks = 0;
@@ -1337,7 +1346,7 @@ class ResultStream {
   hipError_t drive_straight() {
     Transfer& t = *transfer_;
     hipError_t error = hipSuccess;
-    if (t.computed_event && (error = wait_for(t.computed_event)) == hipSuccess) t.announce(t.sent, false);
+    if (t.ready.empty()) t.await(0);  // those that follow something are announced by the caller
     bool gently = !t.ready.empty(), ordered = gently;
     size_t gentle = 0, gone = 0;  // launches of those, and how many of them have ended
     while (t.sent < t.chunks && error == hipSuccess && !t.stop.load(std::memory_order_relaxed)) {

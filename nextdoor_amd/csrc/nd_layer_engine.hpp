@@ -1388,6 +1388,7 @@ class LayerEngine : public EngineBase {
     ND_HIP_TRY(hipEventRecord(ev_end_, stream_));
     if (rows_expected) send_rows();
     ND_HIP_TRY(hipEventSynchronize(ev_end_));
+    if (rows_ahead_) result_stream->words_are_there();
     ND_HIP_TRY(hipEventElapsedTime(&times.end_to_end, ev_begin_, ev_end_));
     if (h_too_long_ && *h_too_long_) {
       drop_rows_ahead();
@@ -1799,7 +1800,7 @@ class LayerEngine : public EngineBase {
     try {
       hFinalSamples.resize((size_t)n_samples_ * (size_t)final_sample_size());
       rows_ahead_ = result_stream->begin(d_final_, hFinalSamples.size(), (uint32_t)max_bits(), invalid_, hFinalSamples.data(),
-                                         stream_, {}, ev_end_) == hipSuccess;
+                                         stream_, {}, /*follows=*/true) == hipSuccess;
     } catch (const std::bad_alloc&) {
       rows_ahead_ = false;
     }

@@ -466,6 +466,7 @@ class SubgraphEngine : public EngineBase {
     }
     if (expected && total > 0) send_lists(cut);
     ND_HIP_TRY(hipEventSynchronize(ev_end_));
+    if (lists_ahead_) result_stream->words_are_there();
     ND_HIP_TRY(hipEventElapsedTime(&times.end_to_end, ev_begin_, ev_end_));
     times.flat_kernel = times.end_to_end;
     return 0;
@@ -566,8 +567,8 @@ class SubgraphEngine : public EngineBase {
       }
       parts.push_back(list_part(d_rows_, hListRows, first, edges));
       parts.push_back(list_part(d_cols_, hListCols, first, edges));
-      const hipEvent_t computed = ready.empty() ? ev_written_ : nullptr;
-      lists_ahead_ = result_stream->begin(std::move(parts), stream_, std::move(ready), computed) == hipSuccess;
+      const bool follow = ready.empty();
+      lists_ahead_ = result_stream->begin(std::move(parts), stream_, std::move(ready), follow) == hipSuccess;
     } catch (const std::bad_alloc&) {
       lists_ahead_ = false;
     }

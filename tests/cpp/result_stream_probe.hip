@@ -161,7 +161,7 @@ static int beside_one_that_follows() {
     TRY(hipGetLastError());
     TRY(hipEventRecord(computed, busy));
     std::fill(late.begin(), late.end(), -1);
-    TRY(first.begin(d_late, many, 12, 0, late.data(), busy, {}, turn < 2 ? computed : nullptr));
+    TRY(first.begin(d_late, many, 12, 0, late.data(), busy, {}, /*follows=*/turn < 2));
     std::this_thread::sleep_for(std::chrono::milliseconds(5));  // other threads take it on
     for (int form = 0; form < 3; ++form) {
       printf("beside one that follows: turn %d form %d\n", turn, form);
@@ -176,6 +176,10 @@ static int beside_one_that_follows() {
       (void)hipGetLastError();
       if (!std::equal(got.begin(), got.end(), want.begin())) { printf("other words\n"); return 1; }
       if (turn && !before) { printf("held up until the other computation was over\n"); return 1; }
+    }
+    if (turn == 1) {  // else finish() goes on without
+      TRY(hipEventSynchronize(computed));
+      first.words_are_there();
     }
     TRY(first.finish());
     if (late != want) { printf("words from before they were there\n"); return 1; }
