@@ -70,8 +70,8 @@ class HostWorkers {
     return *workers;
   }
 
-  // Work that several threads may take part in: each calls body() once, and every body() has to be able to
-  // do all of it alone, and must not throw.  A Job stays where it is from start() to join().
+  // Work that several threads may take part in: each calls body() once, and the body() of whoever calls join() has to be able to
+  // do all of it alone.  It must not throw.  A Job stays where it is from start() to join().
   struct Job {
     std::function<void()> body;
     unsigned wanted = 0, running = 0;
@@ -86,6 +86,15 @@ class HostWorkers {
       std::lock_guard<std::mutex> lock(mutex_);
       grow(job.wanted);
       jobs_.push_back(&job);
+    }
+    wake_.notify_all();
+  }
+
+  // The same again, for a job that has been started: for threads whose body() returned because there was nothing to do yet.
+  void more(Job& job, unsigned helpers) {
+    {
+      std::lock_guard<std::mutex> lock(mutex_);
+      job.wanted += helpers;
     }
     wake_.notify_all();
   }
@@ -848,9 +857,9 @@ class ResultStream {
       }
       // few chunks are unpacked before a thread is awake, unless it is woken while they are computed
       if (t.chunks <= kFewChunks) helpers = follows ? t.chunks / kChunksAHelper : 0;
-      if (!follows) t.announce(t.sent, false);
+      if (!follows) announce(t.sent);
     }
-    job_.body = [this] { take_part(); };
+    job_.body = [this] { take_part(/*stays=*/false); };
     under_way_ = true;
     helped_ = false;
     try {
@@ -864,14 +873,14 @@ class ResultStream {
   void words_are_there() {
     if (!under_way_ || !transfer_->follows) return;
     transfer_->follows = false;
-    transfer_->announce(transfer_->sent, false);  // (nobody sends more before that)
+    announce(transfer_->sent);  // (nobody sends more before that)
   }
 
   hipError_t finish() {
     if (!under_way_) return hipSuccess;
     Transfer& t = *transfer_;
     words_are_there();  // or will be: who looks for a chunk waits until it comes
-    take_part();
+    take_part(/*stays=*/true);
     if (helped_) HostWorkers::get().join(job_);
     under_way_ = false;
     if (t.error != hipSuccess) {
@@ -1072,7 +1081,7 @@ class ResultStream {
     hipError_t error = hipSuccess;     // the first one
     std::mutex mutex;
     std::condition_variable more;
-    unsigned sleepers = 0;
+    unsigned sleepers = 0, gone = 0;   // threads that wait for chunks, and that went back for want of them
     std::vector<std::atomic<size_t>> left;  // chunks of a block that are not unpacked yet
 
     void set(std::vector<Part> parts_, std::vector<Ready> ready_) {
@@ -1113,7 +1122,7 @@ class ResultStream {
         packed_at = sizeof(PackHeader) * longest;
         slot_bytes = (packed_at + chunk_bytes * longest + kUnpackOverread + 255) / 256 * 256;
       }
-      driven = false, next = 0, there = 0, stop = false, overflow = false, error = hipSuccess;
+      driven = false, next = 0, there = 0, stop = false, overflow = false, error = hipSuccess, gone = 0;
       const size_t blocks = (chunks + kBlock - 1) / kBlock;
       left = std::vector<std::atomic<size_t>>(blocks);
       for (size_t b = 0; b < blocks; ++b) left[b].store(std::min(kBlock, chunks - b * kBlock));
@@ -1137,37 +1146,59 @@ class ResultStream {
     // (no other chunk's that was or will be where this one is)
     uint64_t stamp(size_t chunk) const { return (number << 32) + chunk; }
 
+    bool here(size_t chunk) const { return there.load(std::memory_order_acquire) > chunk || stop.load(); }
     // Words come every 20-200 us: worth a short wait awake (a thread that sleeps is back 50 us later, and
     // waking all of them costs the driving thread as much), but not more than that.
-    void await(size_t chunk) {
+    bool comes_soon(size_t chunk) const {
       for (int spin = 0; spin < kSpins; ++spin) {
-        if (there.load(std::memory_order_acquire) > chunk || stop.load()) return;
+        if (here(chunk)) return true;
         spin_pause();
       }
+      return false;
+    }
+    void await(size_t chunk) {
+      if (comes_soon(chunk)) return;
       std::unique_lock<std::mutex> lock(mutex);
       sleepers++;
-      more.wait(lock, [&] { return there.load(std::memory_order_acquire) > chunk || stop.load(); });
+      more.wait(lock, [&] { return here(chunk); });
       sleepers--;
     }
-    void announce(size_t chunks_there, bool stops) {
+    // False: it is not here, and who announces the next ones calls a thread back for this one.
+    bool here_or_gone(size_t chunk) {
+      if (comes_soon(chunk)) return true;
+      std::lock_guard<std::mutex> lock(mutex);
+      if (here(chunk)) return true;
+      gone++;
+      return false;
+    }
+    // Returns how many threads to call back.
+    unsigned announce(size_t chunks_there) {
       bool asleep;
+      unsigned back;
       {
         std::lock_guard<std::mutex> lock(mutex);
-        if (stops) stop.store(true);
-        else there.store(chunks_there, std::memory_order_release);
+        there.store(chunks_there, std::memory_order_release);
         asleep = sleepers > 0;
+        back = gone;
+        gone = 0;
       }
       if (asleep) more.notify_all();
+      return back;
     }
     void fail(hipError_t e) {
       {
         std::lock_guard<std::mutex> lock(mutex);
         if (error == hipSuccess) error = e;
+        stop.store(true);
       }
       (void)hipGetLastError();  // reported by finish(), not to this thread's next launch
-      announce(0, true);
+      more.notify_all();
     }
   };
+
+  void announce(size_t chunks_there) {
+    if (const unsigned back = transfer_->announce(chunks_there)) HostWorkers::get().more(job_, back);
+  }
 
   uint8_t* slot(size_t piece) const { return ring_ + (piece % kSlots) * transfer_->slot_bytes; }
 
@@ -1309,25 +1340,30 @@ class ResultStream {
     t.left[c / kBlock].fetch_sub(end - c, std::memory_order_release);
   }
 
-  void take_part() {
+  // Has all of it packed, if nobody does yet, and unpacks what is there.  A thread that does not stay holds no chunk that is not, and is
+  // free for other transfers until there are some: a pass may take long, and there are no more than kMost threads for all samplers.
+  void take_part(bool stays) {
     Transfer& t = *transfer_;
-    if (!t.driven.exchange(true)) drive();
     for (;;) {
-      const size_t c = t.next.fetch_add(kChunksAtOnce);
-      if (c >= t.chunks) return;
-      const size_t end = std::min(c + kChunksAtOnce, t.chunks);
-      t.await(end - 1);
-      if (t.stop.load()) return;
-      unpack(c, end);
+      // (what follows something has nothing to be driven before it is there)
+      if (!t.driven.load(std::memory_order_relaxed) && (!t.ready.empty() || t.there.load() != 0) && !t.driven.exchange(true)) drive();
+      const size_t c = t.next.load();
+      if (c >= t.chunks || t.stop.load()) return;
+      if (unpack_some()) continue;
+      const size_t last = std::min(c + kChunksAtOnce, t.chunks) - 1;
+      if (stays) t.await(last);
+      else if (!t.here_or_gone(last)) return;
     }
   }
 
-  // The driving thread: some of what is there for it to unpack, if anything is.
+  // Some of what is there, if anything is that nobody has taken.
   bool unpack_some() {
     Transfer& t = *transfer_;
-    size_t c = t.next.load();
-    const size_t end = std::min(c + kChunksAtOnce, t.chunks);
-    if (c >= t.chunks || t.there.load(std::memory_order_relaxed) < end || !t.next.compare_exchange_strong(c, c + kChunksAtOnce)) return false;
+    size_t c = t.next.load(), end;
+    do {
+      end = std::min(c + kChunksAtOnce, t.chunks);
+      if (c >= t.chunks || t.there.load(std::memory_order_acquire) < end) return false;
+    } while (!t.next.compare_exchange_weak(c, c + kChunksAtOnce));
     unpack(c, end);
     return true;
   }
@@ -1346,7 +1382,6 @@ class ResultStream {
   hipError_t drive_straight() {
     Transfer& t = *transfer_;
     hipError_t error = hipSuccess;
-    if (t.ready.empty()) t.await(0);  // those that follow something are announced by the caller
     bool gently = !t.ready.empty(), ordered = gently;
     size_t gentle = 0, gone = 0;  // launches of those, and how many of them have ended
     while (t.sent < t.chunks && error == hipSuccess && !t.stop.load(std::memory_order_relaxed)) {
@@ -1378,7 +1413,7 @@ class ResultStream {
       const hipStream_t stream = t.streams[t.launches % 2];
       error = launch(end, gently ? kGentleBlocks : bus_blocks(), stream);
       if (error == hipSuccess && gently) error = hipEventRecord(packed_[gentle++ % kSlots], stream);
-      if (error == hipSuccess) t.announce(t.sent, false);
+      if (error == hipSuccess) announce(t.sent);
     }
     return error;
   }
@@ -1404,7 +1439,7 @@ class ResultStream {
       }
       if (here < sent && (e = hipEventQuery(copied_[here % kSlots])) != hipErrorNotReady) {
         if (e != hipSuccess) return e;
-        t.announce(t.begins[++here], false);
+        announce(t.begins[++here]);
         moved = true;
       }
       if (!moved) spin_pause();

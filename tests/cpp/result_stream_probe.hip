@@ -196,10 +196,70 @@ static int beside_one_that_follows() {
   return 0;
 }
 
+// Threads that take part in work that is asked for now.
+static unsigned threads_that_are_free() {
+  std::atomic<unsigned> here{0};
+  const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(10);
+  nd::HostWorkers::get().run(nd::HostWorkers::kMost, [&] {
+    if (std::chrono::steady_clock::now() < until) here++;  // else one of them comes again
+    while (std::chrono::steady_clock::now() < until) std::this_thread::yield();
+  });
+  return here.load();
+}
+
+// While a transfer waits for its words, at most one thread does: one that asks for them, unless they follow a computation.
+static int threads_beside_one_that_waits() {
+  const size_t n = (size_t)300 * nd::kPackChunk;
+  std::vector<int32_t> want(n), late(n);
+  for (size_t i = 0; i < n; ++i) want[i] = (int32_t)(i & 0xfff);
+  int32_t* d_late = nullptr;
+  uint32_t* sign = nullptr;
+  hipStream_t busy;
+  hipEvent_t computed;
+  TRY(hipMalloc(&d_late, n * sizeof(int32_t)));
+  TRY(hipHostMalloc((void**)&sign, sizeof(uint32_t), hipHostMallocDefault));
+  *sign = 0;
+  TRY(hipStreamCreate(&busy));
+  TRY(hipEventCreateWithFlags(&computed, hipEventDisableTiming));
+  nd::ResultStream first;
+  const unsigned all = threads_that_are_free();
+  for (int turn = 0; turn < 2; ++turn)  // the first one takes the memory
+    for (int form = 0; form < 3; ++form) {
+      TRY(hipMemset(d_late, 0, n * sizeof(int32_t)));
+      TRY(hipDeviceSynchronize());
+      if (turn) take_a_while<<<dim3(1), dim3(64), 0, busy>>>();
+      write_words<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, busy>>>(d_late, n);
+      TRY(hipGetLastError());
+      TRY(hipEventRecord(computed, busy));
+      std::vector<nd::ResultStream::Ready> ready{{n, computed}};
+      if (form == 0) ready.clear();
+      if (form == 2) ready = {{n / 3, computed, sign, 7u}, {n, computed, sign, 7u}};
+      std::fill(late.begin(), late.end(), -1);
+      TRY(first.begin(d_late, n, 12, 0, late.data(), busy, ready, /*follows=*/form == 0));
+      std::this_thread::sleep_for(std::chrono::milliseconds(5));  // other threads take it on
+      const unsigned now = threads_that_are_free();
+      const bool before = hipEventQuery(computed) == hipErrorNotReady;
+      (void)hipGetLastError();
+      printf("threads beside one that waits: turn %d form %d: %u of %u\n", turn, form, now, all);
+      fflush(stdout);
+      if (turn && !before) { printf("the computation was over\n"); return 1; }
+      if (turn && now + (form == 0 ? 0 : 1) < all) { printf("threads are kept\n"); return 1; }
+      TRY(first.finish());
+      if (late != want) { printf("words from before they were there\n"); return 1; }
+    }
+  first.release();
+  TRY(hipEventDestroy(computed));
+  TRY(hipStreamDestroy(busy));
+  TRY(hipHostFree(sign));
+  TRY(hipFree(d_late));
+  return 0;
+}
+
 int main() {
   if (on_other_devices() != 0) return 1;
   if (beside_one_that_waits() != 0) return 1;
   if (beside_one_that_follows() != 0) return 1;
+  if (threads_beside_one_that_waits() != 0) return 1;
   const size_t piece = (size_t)64 * nd::kPackChunk;  // the smallest piece
   const size_t sizes[] = {1, 7, 8, 9, nd::kPackChunk - 1, nd::kPackChunk, nd::kPackChunk + 1, piece, piece + 9, 13 * piece + 4097,
                           (size_t)4200 * nd::kPackChunk + 5};
