@@ -40,7 +40,7 @@ const char* nd_app_name(int index);
  * with every change of the engine's interface, combined with the sizes of the structs the two
  * sides share, so that a forgotten raise is caught as well.  nd_engine_abi() is the library's own
  * value.  Returns 0, or a negative value (-2 ABI mismatch, -3 name taken). */
-#define ND_ENGINE_ABI 7
+#define ND_ENGINE_ABI 8
 int nd_engine_abi(void);
 int nd_register_app(const char* name, void* (*make)(const char* name), int engine_abi);
 

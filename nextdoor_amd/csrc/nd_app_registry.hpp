@@ -60,9 +60,9 @@ void* make_app_engine(const char* name) {
 // What nd_register_app compares: the hand-raised ND_ENGINE_ABI and the sizes of what a shared object of apps and the library
 // both lay out: the engine's base class with all that it owns through a pointer (an engine made by one side brings its results
 // home with the other's code), the graph, the kernel parameters, the per-step bookkeeping.
-constexpr size_t kSharedLayouts[] = {sizeof(EngineBase),   sizeof(PhaseTimes), sizeof(ResultStream), ResultStream::transfer_bytes(),
-                                     sizeof(HostPool),     sizeof(HostLease),  sizeof(HostWorkers),  sizeof(HostWorkers::Job),
-                                     sizeof(CSR),          sizeof(StepParams), sizeof(RunsMeta)};
+constexpr size_t kSharedLayouts[] = {sizeof(EngineBase), sizeof(PhaseTimes), sizeof(ResultStream), ResultStream::transfer_bytes(),
+                                     sizeof(ResultStream::Part), sizeof(HostPool), sizeof(HostLease), sizeof(HostWorkers),
+                                     sizeof(HostWorkers::Job), sizeof(CSR), sizeof(StepParams), sizeof(RunsMeta)};
 constexpr int engine_abi() {
   uint32_t sizes = 0;
   for (size_t bytes : kSharedLayouts) sizes = sizes * 31u + (uint32_t)bytes;  // two that change do not make up for each other

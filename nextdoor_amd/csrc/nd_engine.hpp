@@ -118,11 +118,11 @@ class EngineBase {
   const std::shared_ptr<HostPool> host_pool = std::make_shared<HostPool>();
   // (engines that are parts of another one use that one's, so that there is one ring a sampler, and one to give back)
   std::shared_ptr<ResultStream> result_stream = std::make_shared<ResultStream>();
-  // Device memory to the host, complete on return.  bits, fill: what is known of its words (ResultStream::fetch).
-  int fetch_to_host(void* dst, const void* src, size_t bytes, uint32_t bits, int32_t fill, hipStream_t stream) {
+  // Device memory to the host, complete on return.  bits, fill, sparse: what is known of its words (ResultStream::Part).
+  int fetch_to_host(void* dst, const void* src, size_t bytes, uint32_t bits, int32_t fill, hipStream_t stream, bool sparse = false) {
     hipError_t e;
     if (bytes % sizeof(int32_t) == 0) {
-      e = result_stream->fetch((const int32_t*)src, bytes / sizeof(int32_t), bits, fill, (int32_t*)dst, stream);
+      e = result_stream->fetch({{(const int32_t*)src, bytes / sizeof(int32_t), bits, fill, (int32_t*)dst, sparse}}, stream);
     } else {
       e = result_stream->copy(src, bytes, dst, stream);
     }
@@ -2260,7 +2260,7 @@ class Engine : public EngineBase {
       size_t words = 0;
       for (size_t r = 0, at = 0; r < std::max<size_t>(1, ends.size()); ++r) {
         const size_t end = ends.empty() ? (size_t)n_samples_ : ends[r];
-        if (r == 0 || states) parts.push_back({d_final_ + at * F, 0, (uint32_t)max_bits_, invalid_, rows_ahead + at * F});
+        if (r == 0 || states) parts.push_back({d_final_ + at * F, 0, (uint32_t)max_bits_, invalid_, rows_ahead + at * F, walk_mode_});
         parts.back().n += (end - at) * F;
         words += (end - at) * F;
         if (states) {
@@ -2837,7 +2837,7 @@ class Engine : public EngineBase {
     if (!allocated_) { last_error = "no device data"; return -1; }
     settle_rows_ahead();
     return fetch_to_host(dst, d_final_, sizeof(VertexID_t) * (size_t)n_samples_ * (size_t)final_sample_size(),
-                         (uint32_t)max_bits_, invalid_, stream_);
+                         (uint32_t)max_bits_, invalid_, stream_, walk_mode_);
   }
 
   // Walks: where the next pass's rows shall go, if the caller expects to fetch them.  Rows of the first walks then

@@ -763,6 +763,7 @@ class ResultStream {
     uint32_t bits;
     int32_t fill;
     int32_t* dst;
+    bool sparse = false;  // such groups are to be expected anywhere (rows of walks, which end)
   };
 
   // The first `words` words of a transfer's parts are on the device once `event` has happened, or, if there is a `sign` (all of a
@@ -850,7 +851,7 @@ class ResultStream {
       else e = hipEventRecord(begun_, stream);
       // (all on the given stream: the other one is not only ours, and what is computed before this may take long)
       while (e == hipSuccess && t.sent < t.ring_chunks)
-        e = launch(std::min(t.part_ends[t.part_of(t.sent)], t.ring_chunks), bus_blocks(), stream);
+        e = launch(std::min(t.part_ends[t.part_of(t.sent)], t.ring_chunks), blocks_in_order(), stream);
       if (e != hipSuccess) {
         (void)hipStreamSynchronize(stream);  // nothing writes to the ring after this
         return e;
@@ -954,6 +955,26 @@ class ResultStream {
   //     MVS 150 K                    2.24   2.20   2.22   2.20   2.27
   //     KHop R-MAT 20 (19 rings)    11.00  10.87  10.55  10.53  10.63
   static constexpr uint32_t kBusBlocks = 64, kBusBlocksOfMany = 128;
+  // More chunks in stream order than the ring holds: the ring is filled by one launch, and what is launched beside that takes its part of
+  // the bus for chunks that nobody looks for yet.  So the next launch sets out when no more than kChunksAhead are on their way.  Rows
+  // of walks keep to kBusBlocks: where many groups are left out it is the threads that take the time, and they want chunks in their
+  // order.  Passes with their rows, and (fetch) rows alone, ms, by workgroups (Chung-Lu graphs, a third of the walks' groups left out); with
+  // 128 and launches as far ahead as the ring has room; in pieces on two streams, an event for each, as it was before chunks had stamps:
+  //                                     64     80     96    128    far ahead   in pieces
+  //     uniform walks 170 K          0.762  0.828  0.846  0.872        0.894       0.785
+  //                   190 K          0.842  0.908  0.931  0.954        0.963       0.867
+  //     DeepWalk 180 K               1.024  1.089  1.102  1.122        1.151       1.043
+  //     weighted node2vec 170 K      1.481  1.556  1.558  1.583        1.609       1.480
+  //                       230 K      1.788  1.849  1.866  1.891        1.915       1.814
+  //     KHop 65 K                    0.959  0.942  0.945  0.972        0.978
+  //          85 K                    1.286  1.261  1.244  1.249        1.235       1.327
+  //     Layer 85 K                   1.373  1.339  1.325  1.330        1.319       1.410
+  //     fetch: KHop 62 K             0.758  0.753  0.759  0.799        0.805       0.770
+  //                300 K             3.629  3.599  3.625  3.673        3.768       3.664
+  //            MVS 90 K              0.788  0.778  0.787  0.783        0.860
+  //            PPR 262 K             0.694  0.698  0.728  0.789        0.826       0.903
+  static constexpr uint32_t kBusBlocksInOrder = 96;
+  static constexpr size_t kChunksAhead = 1024;
   static constexpr size_t kGentleAhead = 2;
   static constexpr size_t kPackedAhead = 3;     // pieces packed before the copy engine has come to them
   static constexpr int kSignsPerQuery = 1024;   // looks at a sign for one at the event beside it: some 20 us
@@ -1054,6 +1075,7 @@ class ResultStream {
     std::vector<size_t> part_ends;     // chunks; a chunk is of one part
     uint32_t bits = 0;                 // the most of any part
     bool streaming = false;            // results larger than the caches
+    bool sparse = false;               // a part is
     hipStream_t streams[2];
     std::vector<Ready> ready;
     std::vector<size_t> ready_chunks;  // that are there once a `ready` has happened
@@ -1092,10 +1114,12 @@ class ResultStream {
       computed = false;
       chunks = 0;
       bits = 0;
+      sparse = false;
       part_ends.clear();
       size_t words = 0;
       for (const Part& p : parts) {
         words += p.n;
+        sparse = sparse || p.sparse;
         part_ends.push_back(chunks += (p.n + kPackChunk - 1) / kPackChunk);
         bits = std::max(bits, p.bits > kPackMostBits ? 32 : p.bits);
       }
@@ -1244,6 +1268,9 @@ class ResultStream {
   }
 
   uint32_t bus_blocks() const { return transfer_->chunks > transfer_->ring_chunks ? kBusBlocksOfMany : kBusBlocks; }
+  uint32_t blocks_in_order() const {
+    return transfer_->chunks > transfer_->ring_chunks && !transfer_->sparse ? kBusBlocksInOrder : kBusBlocks;
+  }
 
   // Straight: the chunks from t.sent on, up to `end`, all of one part.
   hipError_t launch(size_t end, uint32_t most_blocks, hipStream_t on) {
@@ -1390,10 +1417,11 @@ class ResultStream {
       if (error == hipErrorNotReady) error = hipSuccess;
       if (error != hipSuccess) break;
       while (t.unpacked_to < t.left.size() && t.left[t.unpacked_to].load(std::memory_order_acquire) == 0) t.unpacked_to++;
-      const size_t room = t.unpacked_to == t.left.size() ? t.chunks : t.unpacked_to * kBlock + t.ring_chunks;
+      const bool in_order = t.ready.empty();
+      const size_t unpacked = std::min(t.chunks, t.unpacked_to * kBlock), room = std::min(t.chunks, unpacked + t.ring_chunks);
       // up to the end of what may be read, if that is known, else a piece at a time
       size_t end = std::min(t.chunks, t.sent + kMostChunks);
-      if (!t.ready.empty()) {
+      if (!in_order) {
         if (!readable(t.sent + 1, /*waits=*/t.next.load() >= t.sent && gone == gentle, &error)) {
           if (error == hipSuccess && !unpack_some()) spin_pause();
           continue;
@@ -1401,7 +1429,7 @@ class ResultStream {
         end = std::min(t.ready_chunks[t.happened - 1], gently || t.chunks > t.ring_chunks ? t.sent + kMostChunks : t.chunks);
       }
       end = std::min(end, t.part_ends[t.part_of(t.sent)]);
-      if (end > room || (gently && gentle - gone >= kGentleAhead)) {
+      if (end > room || (gently && gentle - gone >= kGentleAhead) || (in_order && t.sent > unpacked + kChunksAhead)) {
         if (!unpack_some()) std::this_thread::yield();
         continue;
       }
@@ -1411,7 +1439,7 @@ class ResultStream {
       ordered = true;
       if (gently) ahead_.fetch_add(1, std::memory_order_relaxed);
       const hipStream_t stream = t.streams[t.launches % 2];
-      error = launch(end, gently ? kGentleBlocks : bus_blocks(), stream);
+      error = launch(end, gently ? kGentleBlocks : in_order ? blocks_in_order() : bus_blocks(), stream);
       if (error == hipSuccess && gently) error = hipEventRecord(packed_[gentle++ % kSlots], stream);
       if (error == hipSuccess) announce(t.sent);
     }

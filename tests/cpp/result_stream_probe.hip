@@ -262,7 +262,7 @@ int main() {
   if (threads_beside_one_that_waits() != 0) return 1;
   const size_t piece = (size_t)64 * nd::kPackChunk;  // the smallest piece
   const size_t sizes[] = {1, 7, 8, 9, nd::kPackChunk - 1, nd::kPackChunk, nd::kPackChunk + 1, piece, piece + 9, 13 * piece + 4097,
-                          (size_t)4200 * nd::kPackChunk + 5};
+                          (size_t)4200 * nd::kPackChunk + 5, (size_t)9000 * nd::kPackChunk + 5};
   nd::ResultStream stream;
   uint32_t* sign = nullptr;  // what has arrived, and what never does
   hipEvent_t done;
@@ -275,6 +275,7 @@ int main() {
     for (uint32_t bits : {1u, 2u, 7u, 8u, 9u, 12u, 16u, 17u, 23u, 24u, 25u, 26u, 31u, 32u}) {
       if (n > piece + 9 && bits != 12 && bits != 23 && bits != 32) continue;
       if (n > 14 * piece && bits == 23) continue;
+      if (n > 70 * piece && bits != 12) continue;
       for (int misfit = 0; misfit < 2; ++misfit) {
         printf("n %zu bits %u misfit %d\n", n, bits, misfit);
         fflush(stdout);
@@ -293,7 +294,7 @@ int main() {
             TRY(stream.copy(d, bytes, got.data() + shift, nullptr));
             if (memcmp(got.data() + shift, want.data(), bytes) != 0) { printf("bytes differ\n"); return 1; }
           }
-          TRY(stream.fetch(d, n, bits, fill, got.data() + shift, nullptr));
+          TRY(stream.fetch({{d, n, bits, fill, got.data() + shift, /*sparse=*/shift == 1}}, nullptr));
           if (memcmp(got.data() + shift, want.data(), n * sizeof(int32_t)) != 0 || got[n + 1] != 77) {
             printf("differs at shift %d\n", shift);
             return 1;

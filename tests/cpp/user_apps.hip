@@ -196,6 +196,7 @@ struct UserNotingWalkApp : UniformRandomWalkAppT<8> {
 // The sizes this object was built with, for the test of what the library compares.
 extern "C" int user_apps_shared_layouts(uint64_t* out, int room) {
   const uint64_t sizes[] = {sizeof(nd::EngineBase), sizeof(nd::PhaseTimes), sizeof(nd::ResultStream), nd::ResultStream::transfer_bytes(),
+                            sizeof(nd::ResultStream::Part),
                             sizeof(nd::HostPool), sizeof(nd::HostLease), sizeof(nd::HostWorkers), sizeof(nd::HostWorkers::Job),
                             sizeof(CSR), sizeof(nd::StepParams), sizeof(nd::RunsMeta)};
   const int n = (int)(sizeof(sizes) / sizeof(sizes[0]));

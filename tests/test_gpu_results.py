@@ -106,6 +106,21 @@ def test_rows_that_leave_before_the_pass_is_over(oracle, n):
     assert all(np.array_equal(r, want) for r in rows)
 
 
+# rows of one launch: as many as the ring of what is on its way holds (64 MB of ids), a few more, and more than that by a whole launch
+@pytest.mark.parametrize("n", [167772, 167801, 190003])
+def test_rows_behind_a_pass_around_what_the_ring_holds(oracle, n):
+    g = graphs.random_graph(n=n, mean_degree=4, seed=n, isolated_every=3)
+    s = nd.Sampler("UniformRandomWalk", g, seed=42)
+    d = oracle.app_desc(oracle.UNIFORM_WALK, s.steps, [s.step_size(k) for k in range(s.steps)])
+    want, _ = oracle.sample_individual(graphs.oracle_view(g), d, 42, s.initial_contents)
+    for turn in range(4):  # fetched after the first pass, behind the others
+        print("n", n, "turn", turn, flush=True)
+        s.do_transit_parallel()
+        assert np.array_equal(s.final_samples(), want)
+    s.do_transit_parallel()
+    s.close()  # with rows on their way
+
+
 def device_memory_left():
     hip = ctypes.CDLL("libamdhip64.so")
     left, total = ctypes.c_size_t(), ctypes.c_size_t()
