@@ -435,8 +435,9 @@ class SubgraphEngine : public EngineBase {
     ND_HIP_TRY(exclusive_scan_u32(d_lengths_, d_list_start_, (size_t)n_samples_ + 1, d_scan_scratch_, stream_));
     sum_lengths<<<dim3(256), dim3(256), 0, stream_>>>(d_lengths_, (size_t)n_samples_, d_total_);
     ND_HIP_TRY(hipGetLastError());
-    // Lists that are expected leave as they are written: those of a quarter of the samples while the others' are (20.8 M edges
-    // of 37,501 samples: 2.20 -> 1.83 ms a pass with its lists; the bus and the threads that unpack take four times as long as the writing).
+    // Lists that are expected leave as they are written: those of a quarter of the samples while the others' are; the bus and the
+    // threads that unpack take four times as long as the writing.  A pass with its lists, ms, all at once / so: 9.7 M edges (78 MB) 0.94 / 0.98,
+    // 13.9 M 1.25 / 1.25, 20.8 M 1.89 / 1.77, 30.5 M 2.72 / 2.53, 41.6 M 3.77 / 3.41.
     const bool early = expected && 2 * sizeof(VertexID_t) * list_capacity_ >= kEarlyListBytes;
     const int64_t cut = early ? n_samples_ / 4 : 0;
     ND_HIP_TRY(hipMemcpyAsync(&h_known_->total, d_total_, sizeof(unsigned long long), hipMemcpyDeviceToHost, stream_));
@@ -553,7 +554,9 @@ class SubgraphEngine : public EngineBase {
   // Has the lists leave; those that cannot be sent now are fetched when they are asked for.
   void send_lists(int64_t cut) {
     try {
-      const size_t edges = (size_t)n_edges_listed_, first = cut > 0 ? h_known_->cut / 4 * 4 : 0;  // (parts are aligned to 16 bytes)
+      const size_t edges = (size_t)n_edges_listed_, first = cut > 0 ? h_known_->cut / kPackGroup * kPackGroup : 0;
+      // (parts are aligned to 16 bytes on the device, and where they are to be to 32: elsewhere rows and columns do not pass the caches,
+      // and 20.8 M edges took 2.05 ms instead of 1.77 where the first list of the others was at an odd multiple of 16)
       start_ahead_.resize((size_t)n_samples_ + 1);
       hListRows.resize(edges);
       hListCols.resize(edges);

@@ -301,13 +301,14 @@ def test_states_that_leave_with_the_rows(app, n):
 
 
 # lists that follow the pass, and that leave as they are written (64 MB of rows and columns)
-@pytest.mark.parametrize("n,degree", [(4004, 6), (60004, 24)])
+@pytest.mark.parametrize("n,degree", [(4004, 6), (60004, 24), (60020, 24)])
 def test_edge_lists_that_leave_with_the_pass(n, degree):
     g = graphs.random_graph(n=n, mean_degree=degree, seed=n, isolated_every=7)
     s = nd.Sampler("MVS", g, seed=42)
     s.do_transit_parallel()
     want = s.adjacency()  # fetched after the pass
     assert n < 5000 or want[0].nbytes + want[1].nbytes > 64 << 20
+    print("edges of the first quarter, from a group of eight on", want[2][s.num_samples // 4] % 8, flush=True)
     held = []
     for turn in range(6):
         print("n", n, "turn", turn, flush=True)
