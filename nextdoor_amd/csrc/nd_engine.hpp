@@ -2188,7 +2188,7 @@ class Engine : public EngineBase {
   // pass after one that found nothing for the workgroup class is not), 7 = load-balanced steps
   // whose two classes ran as one launch, 8 = as two launches side by side on two streams,
   // 9 = one after the other.
-  // Walks: 10 = parts of the last pass's rows that were on their way to the host before its walks were done.
+  // 10 = parts of the last pass's rows that were on their way to the host before its samples were done.
   int64_t counter(int which) const override {
     switch (which) {
       case 0: return (int64_t)class_counters_.sorted_pairs;
@@ -2282,46 +2282,54 @@ class Engine : public EngineBase {
 
   // How rows leave before the pass is over.  kRowsByStretch: one launch, whose wavefronts count the walks that are done by
   // stretch (EarlyRows); rows leave as fast as they come, packed for the copy engine, and the walks are not slowed down.
-  // kRowsByRange: a few launches, one range of walks after another; rows leave from the end of the first on (one launch:
-  // when it has ended).  Every launch ends with its longest walks alone on the device (0.07 ms of uniform walks, 0.2 of
+  // kRowsByRange: a few launches, one range of walks after another; rows leave from the end of the first on.  Every launch ends with
+  // its longest walks alone on the device (0.07 ms of uniform walks, 0.2 of
   // DeepWalk and PPR, 0.6 of second-order walks), but all of a range's rows are there at once, and their way straight to
-  // the ring has no 8 us between two pieces.  Passes with their rows, ms, by launches and by stretch, over Chung-Lu graphs
-  // (exponent 2.2) of the mean degree that is named:
+  // the ring has no 8 us between two pieces.  kRowsFollow: one launch, and the rows' packing directly behind it.  Passes with their
+  // rows (MultiRW: and states), ms, by launches (1: kRowsFollow) and by stretch, over Chung-Lu graphs (exponent 2.2) of the mean degree
+  // that is named:
   //                     launches   1     2     3     4     6   stretch
-  //    uniform     11   400 K         1.86  1.73  1.66          1.76      of 8 steps   8   300 K  0.21  0.21        0.22        0.29
-  //                     500 K         2.33  2.19  2.08          2.12                       500 K  0.31  0.32        0.30        0.38
-  //                     600 K         2.90  2.75  2.64          2.52                       800 K                    0.45  0.45  0.53
-  //                     800 K         3.83  3.64  3.54          3.15                       1.2 M                    0.68  0.66  0.69
-  //                 5   500 K               1.64  1.62          1.61                       1.6 M                    0.88  0.84  0.86
-  //                18   500 K               2.95  2.82          2.62                       2 M    1.30  1.24        1.09        1.02
-  //    DeepWalk    11   350 K         1.76  1.73  1.79          1.85
-  //                     450 K         2.29  2.15  2.10          2.18
-  //                     550 K         2.86  2.63  2.57          2.58
-  //                18   500 K                     3.08          2.81
-  //    PPR         11   250 K         1.24  1.26  1.41          1.34
-  //                     450 K         2.08  2.02  1.98          2.02
-  //                     550 K         2.55  2.40  2.44          2.36
-  //    weighted    11   100 K   1.13  1.53                      1.17      of 8 steps   8   120 K  0.22  0.28        0.43        0.26
-  //    node2vec         150 K   1.38  1.77                      1.46                       300 K  0.38  0.36        0.50        0.43
-  //                     200 K   1.64  1.87                      1.69                       500 K  0.57  0.48  0.51  0.59        0.58
-  //                     240 K   1.94  2.02  2.54                1.95                       900 K  0.92  0.95  0.80  0.83        0.85
-  //                     300 K   2.85  2.21                      2.34                       1.2 M  1.18  1.13  1.16  1.02        1.05
-  //                     400 K   3.54  2.74  2.98                2.93
-  //                 6   300 K   1.92  1.69  2.10                1.64
-  //                     400 K         2.22  2.30                2.09
-  //                20   300 K   4.04  3.07  3.45                2.98
-  //                     400 K         4.10  4.22                3.70
-  //       R-MAT 17 x 16         1.33  1.73                      1.39
-  //       R-MAT 18 x 12         2.10  2.06                      2.23
-  //       R-MAT 19 x 16               3.85  3.91                3.73
-  //    MultiRW     11   100 K         1.42  1.45  1.54          1.57      of 6 steps   8   200 K  0.15  0.16        0.17        0.20
-  //                     135 K         1.97  1.84                1.93                       500 K  0.39  0.29        0.29        0.33
-  //                     190 K         2.74  2.53  2.50          2.48                       850 K        0.51        0.46        0.46
-  //                                                                                        1 M    0.68  0.69        0.55        0.51
-  // Where the two meet moves with the graph (second-order walks of 400 K from 10 % for stretches to 6 % against them, by its
-  // degree), and with the walks' length as if a walk were 24 results longer.  Longer walks are not taken from fewer on: a pass whose
-  // walks are all under way at once has no first ones.
-  // kRowsFollow: one launch, and the rows' packing directly behind it.
+  //    uniform     11   160 K   0.73  0.72  0.73  0.76  0.88  0.93     of 8 steps   8   300 K  0.20  0.20  0.21  0.23  0.25  0.31
+  //                     192 K   0.84  0.83  0.88  0.85  1.00  1.04                      500 K  0.31  0.31  0.29  0.30  0.32  0.40
+  //                     250 K   1.07  1.01  1.04  1.03  1.16  1.24                      800 K  0.61  0.45  0.49  0.44  0.43  0.54
+  //                     400 K   1.83  1.65  1.58  1.60  1.67  1.77                      1.2 M  0.86  0.74  0.71  0.66  0.58  0.71
+  //                     500 K   2.23  2.09  1.98  1.91  1.92  2.09                      2 M    1.36  1.19  1.15  1.09  1.01  1.03
+  //                     800 K   3.62  3.57  3.33  3.19  2.98  3.17                      3 M    1.91  1.69  1.71  1.65  1.50  1.45
+  //                     1.1 M   5.03  4.64  4.84  4.62  4.23  4.27
+  //                     1.6 M   7.16  6.58  6.33  6.95  6.38  5.96
+  //                 5   500 K   1.44  1.36  1.37  1.34  1.35  1.51
+  //                18   500 K   3.06  2.85  2.69  2.55  2.51  2.64
+  //    DeepWalk    11   150 K   0.91  0.92  1.18  1.36  1.75  1.02     PPR         11   150 K  0.79  0.84  1.11  1.30  1.78  1.02
+  //                     200 K   1.10  1.04  1.23  1.47  1.91  1.26                      262 K  1.17  1.14  1.31  1.46  1.95  1.32
+  //                     350 K   2.10  1.69  1.70  1.80  2.22  1.82                      450 K  2.01  1.74  1.72  1.72  2.11  1.97
+  //                     450 K   2.41  2.10  2.01  2.04  2.41  2.12                      550 K  2.39  2.26  2.09  2.05  2.26  2.28
+  //                     550 K   2.97  2.61  2.44  2.40  2.68  2.52                      800 K  3.43  3.20  3.02  2.94  2.85  3.06
+  //                     1.1 M   5.90  5.26  5.34  4.83  4.60  4.57                      1.1 M  4.63  4.21  4.56  4.00  3.79  4.02
+  //                18   500 K   3.68  3.23  2.86  2.76  3.43  2.81
+  //    weighted    11   100 K   1.08  1.48  1.97  2.47  3.47  1.18     of 8 steps   8   120 K  0.19  0.25  0.34  0.41  0.56  0.26
+  //    node2vec         200 K   1.62  1.84  2.28  2.84  3.90  1.70                      300 K  0.36  0.33  0.40  0.47  0.62  0.44
+  //                     262 K   2.04  2.05  2.56  3.01  4.13  2.10                      500 K  0.55  0.46  0.49  0.56  0.71  0.60
+  //                     300 K   2.84  2.26  2.67  3.25  4.29  2.33                      900 K  0.92  0.88  0.75  0.75  0.87  0.86
+  //                     400 K   3.45  2.71  3.01  3.52  4.62  2.89                      1.2 M  1.20  1.09  1.16  0.97  1.01  1.05
+  //                     500 K   4.16  3.36  3.37  3.82  5.03  3.49                      2 M    1.93  1.72  1.73  1.74  1.88  1.57
+  //                     700 K   5.73  5.25  4.60  4.64  5.74  4.49
+  //                 6   400 K   1.95  1.80  2.17  2.55  3.44  1.99
+  //                20   200 K   2.24  2.18  2.70  3.28  4.39  2.22
+  //                     300 K   4.00  2.96  3.26  3.92  5.03  2.99
+  //                     400 K   4.85  4.05  3.94  4.39  5.58  3.76
+  //       R-MAT 17 x 16         1.31  1.71  2.22  2.74  3.78  1.40
+  //       R-MAT 18 x 12         2.44  2.27  2.73  3.30  4.45  2.49
+  //       R-MAT 19 x 16         4.91  4.39  4.21  4.61  5.82  4.09
+  //    MultiRW     11    40 K   0.56  0.64  0.71  0.80  1.01  0.70     of 6 steps   8   200 K  0.18  0.20  0.21  0.23  0.26  0.30
+  //                      60 K   0.81  0.79  0.88  0.98  1.20  0.91                      500 K  0.49  0.40  0.39  0.40  0.43  0.49
+  //                     100 K   1.55  1.18  1.23  1.23  1.53  1.51                      850 K  0.78  0.66  0.63  0.64  0.64  0.73
+  //                     135 K   2.20  1.73  1.59  1.65  1.67  1.93                      1 M    0.90  0.83  0.74  0.73  0.73  0.81
+  //                     190 K   3.14  2.46  2.28  2.11  2.24  2.45                      2 M    1.75  1.59  1.54  1.62  1.45  1.44
+  //                     400 K   6.83  6.43  5.59  4.90  4.76  4.81
+  // Where stretches begin was drawn when a launch more cost an event and several launches of the transfer: some of what is just above that
+  // line would now leave by ranges in up to 15 % less (uniform 500 K, PPR 550 K, node2vec 400 K, MultiRW of 6 steps 1 M), and short walks
+  // with a state of their own in one launch (200 K).  Where the two meet moves with the graph, and with the walks' length as if a walk were
+  // 24 results longer.  Longer walks are not taken from fewer on: a pass whose walks are all under way at once has no first ones.
   enum EarlyForm { kRowsStay, kRowsFollow, kRowsByRange, kRowsByStretch };
   EarlyForm early_form(EarlyRows* early) {
     if (!rows_ahead || profiling || wants_launch_graph()) return kRowsStay;
@@ -2840,9 +2848,9 @@ class Engine : public EngineBase {
                          (uint32_t)max_bits_, invalid_, stream_, walk_mode_);
   }
 
-  // Walks: where the next pass's rows shall go, if the caller expects to fetch them.  Rows of the first walks then
-  // cross the bus while later walks are still under way; sample() returns when the sampling is done, as
-  // always, and the rest of the rows arrives until finish_rows_ahead().  Any pass may leave it be.
+  // Where the next pass's rows shall go, if the caller expects to fetch them.  Those of the first samples then
+  // cross the bus while later ones are still sampled, or all of them directly behind the pass; sample() returns when the sampling is
+  // done, as always, and the rest of the rows arrives until finish_rows_ahead().  Any pass may leave it be.
   VertexID_t* rows_ahead = nullptr;
   // ... and its states, with rows only, of apps whose samples' states are whole words each: ranges of samples are then ranges of words.
   static constexpr bool kStatesAreWords = !std::is_empty<SampleType>::value && sizeof(SampleType) % sizeof(int32_t) == 0;
@@ -3292,7 +3300,7 @@ class Engine : public EngineBase {
   const walk_record<App>* walk_records_ = nullptr;  // dgraph_'s, where they pay
   uint32_t walk_waves_at_once_ = 1, cus_ = 1;  // wavefronts of walk_rows_kernel the device holds, compute units
   bool ahead_ = false;                    // rows are on their way to rows_ahead
-  bool sent_ahead_ = false;               // ... or have been, in the last pass, while its walks were under way
+  bool sent_ahead_ = false;               // ... or have been, in the last pass, while it was under way
   bool states_sent_ = false;              // states are on their way to states_ahead, or there
   bool rows_follow_ = false;              // the pass under way sends them directly behind its last launch
   std::vector<hipEvent_t> range_ends_;    // ends of the launches of such a pass

@@ -1887,7 +1887,7 @@ class LayerEngine : public EngineBase {
   MergedEdges merged_{};
   int32_t* d_nbr_cols_ = nullptr;
   float* d_nbr_weights_ = nullptr;
-  // FastGCN form: degree^2 of the marked vertices, by group inside a part, by part, by sample
+  // FastGCN form: degree^2 of the marked vertices, by group inside half a part, by half, by sample
   uint64_t *d_group_through_ = nullptr, *d_half_total_ = nullptr, *d_half_before_ = nullptr;
   UnionTables union_;                  // of the graph
   MarkedSamples marked_{};
