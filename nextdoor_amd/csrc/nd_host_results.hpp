@@ -947,13 +947,15 @@ class ResultStream {
   // computed: stores that wait for the bus stand in the way of that something's own.
   static constexpr uint32_t kGentleBlocks = 32;
   // ... and of one that has the device to itself: enough to keep the bus busy, and no more, so that chunks arrive in about the order the
-  // threads look for them in, and not all of them at the end; for more chunks than the ring holds that matters less, and the
-  // gaps between launches more.  Passes with their rows by workgroups, ms (a workgroup a chunk: walks 0.47, distinct 1.11):
+  // threads look for them in, and not all of them at the end; of more chunks than the ring holds that leave while others are computed
+  // (OfMany: the last three) the gaps between launches matter more.  Passes with their rows by workgroups, ms (a workgroup a chunk: walks
+  // 0.47, distinct 1.11):
   //                                     32     64     96    128    256
-  //     uniform walks 57 K           0.348  0.302  0.341  0.344  0.369
-  //     KHop 60 K, distinct          0.974  0.832  0.897  0.926  0.990
-  //     MVS 150 K                    2.24   2.20   2.22   2.20   2.27
-  //     KHop R-MAT 20 (19 rings)    11.00  10.87  10.55  10.53  10.63
+  //     uniform walks 57 K           0.347  0.302  0.336  0.350  0.391
+  //     KHop 60 K, distinct          0.951  0.798  0.876  0.913  0.950
+  //     MVS 150 K                    1.774  1.739  1.728  1.730  1.785
+  //     uniform walks 250 K          1.020  0.984  0.992  1.009  1.048
+  //     KHop R-MAT 20 (17 rings)     9.96   9.71   9.65   9.60   9.72
   static constexpr uint32_t kBusBlocks = 64, kBusBlocksOfMany = 128;
   // More chunks in stream order than the ring holds: the ring is filled by one launch, and what is launched beside that takes its part of
   // the bus for chunks that nobody looks for yet.  So the next launch sets out when no more than kChunksAhead are on their way.  Rows
