@@ -172,8 +172,8 @@ int nd_sampler_get_distinct_counts(const nd_sampler* s, const int32_t** data, in
  * transits the workgroup kernel served as one work item, 2 = pairs on transits split over several
  * work items (grid-wide), 3 = pairs in runs long enough for the workgroup kernel that stayed with
  * the flat kernel because of the transit's degree, 4 = work items; the flat kernel served
- * 0 minus 1 minus 2.  Walks: 10 = parts of the last pass's rows that were on their way to the host
- * before its walks were done (0 where the caller is not expected to take the rows, and where they are
+ * 0 minus 1 minus 2.  10 = parts of the last pass's rows that were on their way to the host
+ * before its samples were done (0 where the caller is not expected to take the rows, and where they are
  * few).  Edge-list apps: 0 = edges listed. */
 int64_t nd_sampler_counter(const nd_sampler* s, int which);
 /* The validators the reference's apps pass to nextdoor() as checkResultsFunc
